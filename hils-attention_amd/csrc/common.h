@@ -105,6 +105,22 @@ __device__ __forceinline__ unsigned rows_bcast0(unsigned x) {
   return b.x;
 }
 
+// Value of lane (lane ^ O), O a power of two: DPP moves inside a row of 16 lanes, a shuffle for 16 and 32.
+// Every lane of the wavefront takes part.
+template <int O>
+__device__ __forceinline__ float lane_xor(float x) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one lane bit");
+  const int v = __float_as_int(x);
+  if (O == 1) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
+  if (O == 2) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // quad_perm 2,3,0,1
+  if (O == 4) {  // row_shl:4 for the lanes with bit 2 clear, row_shr:4 for the others
+    const int a = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);
+    return __int_as_float(__builtin_amdgcn_update_dpp(a, v, 0x114, 0xf, 0xa, false));
+  }
+  if (O == 8) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false));  // row_ror:8
+  return __shfl_xor(x, O, 64);
+}
+
 // block-wide reductions for blockDim.x a multiple of 64, <= 1024; `red` holds >= 17 floats
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);

@@ -44,6 +44,8 @@ SIGNATURES = {
     "hils_rope": [_P] * 4 + [_I] * 7 + [_F, _P],
     "hils_norm_rope_pool_fwd": [_P] * 6 + [_I] * 6 + [_F, _P],
     "hils_norm_rope_pool_bwd": [_P] * 8 + [_I] * 6 + [_F, _P],
+    "hils_norm_rope_pool_bwd_ws": [_P] * 8 + [_I, _P, _Z] + [_I] * 6 + [_F, _P],
+    "hils_norm_rope_pool_bwd_workspace": [_I] * 5,
     "hils_swa_fwd": [_P] * 5 + [_I] * 12 + [_F, _P],
     "hils_swa_bwd": [_P] * 11 + [_I] * 10 + [_F, _P],
 }
@@ -83,7 +85,7 @@ def load():
     lib.hils_sparse_attn_bwd_workspace.argtypes = [_I] * 11 + [_F]
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)
-        fn.restype = c_int
+        fn.restype = ctypes.c_size_t if name.endswith("_workspace") else c_int
         fn.argtypes = argtypes
     _lib = lib
     return lib

@@ -53,10 +53,19 @@ class _NormRopePoolFn(torch.autograd.Function):
         if g_out is None and g_lmk is None:
             return None, None, None, None, None, None, None
         dx = torch.empty_like(x_in)
-        dw = torch.zeros(D, dtype=torch.float32, device=x_in.device) if w_in is not None else None
-        _cabi.call("hils_norm_rope_pool_bwd", _cabi.ptr(x_in), _cabi.ptr(w_in), _cabi.ptr(cos_in), _cabi.ptr(sin_in),
-                   _cabi.ptr(g_out), _cabi.ptr(g_lmk), _cabi.ptr(dx), _cabi.ptr(dw), B, L, H, D, S, per_batch, eps)
-        return dx, (None if dw is None else dw.to(ctx.w_dtype)), None, None, None, None, None
+        args = (_cabi.ptr(x_in), _cabi.ptr(w_in), _cabi.ptr(cos_in), _cabi.ptr(sin_in), _cabi.ptr(g_out),
+                _cabi.ptr(g_lmk), _cabi.ptr(dx))
+        dims = (B, L, H, D, S, per_batch, eps)
+        if w_in is None:
+            _cabi.call("hils_norm_rope_pool_bwd", *args, None, *dims)
+            return dx, None, None, None, None, None, None
+        bf16 = ctx.w_dtype == torch.bfloat16
+        dw = torch.empty(D, dtype=torch.bfloat16 if bf16 else torch.float32, device=x_in.device)
+        ws = torch.empty(_cabi.load().hils_norm_rope_pool_bwd_workspace(B, L, H, D, S), dtype=torch.uint8,
+                         device=x_in.device)
+        _cabi.call("hils_norm_rope_pool_bwd_ws", *args, _cabi.ptr(dw), int(bf16), _cabi.ptr(ws), _cabi.nbytes(ws),
+                   *dims)
+        return dx, dw.to(ctx.w_dtype), None, None, None, None, None
 
 
 def norm_rope_pool(x, norm_weight=None, cos=None, sin=None, chunk_size=64, eps=1e-6, pool=True):
