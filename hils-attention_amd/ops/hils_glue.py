@@ -187,8 +187,13 @@ def decode_step(q, lmks, k, v, lse_swa, topk, block_size, window_size, q_offset=
             pb = prior_b.float().contiguous()
         else:
             pb = _prior_bias(prior_b, B, N, h_q)
-    if not (lib.hils_decode_step_covers(B, L, N, h_q, h_kv, D, int(topk), int(block_size), int(pb is not None))
-            and Lkv >= N * block_size):
+    # Many queries per sequence (a prompt's next slice on a cache): the prefill kernels read a chunk once for all
+    # queries of a block that selected it, after one pass that repacks K and V; the one-launch kernel reads topk
+    # chunks per query.  Repacking moves 8 bytes per cache element at about 5 TB/s, the one-launch kernel 256 * topk
+    # bytes per query and feature pair at about 7.5 TB/s, which meet near L = Lkv / (20 * topk).
+    many = L >= 64 and 16 * L * int(topk) >= Lkv
+    if many or not (lib.hils_decode_step_covers(B, L, N, h_q, h_kv, D, int(topk), int(block_size),
+                                                int(pb is not None)) and Lkv >= N * block_size):
         if lmk_head_major:  # the two-call kernels read the reference's layout
             lmks = lmks[:, :, :N].permute(0, 2, 1, 3).contiguous()
             if pb is not None:
