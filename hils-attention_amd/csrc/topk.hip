@@ -2036,9 +2036,14 @@ static bool topk_use_row(long rows, int N, int G, int D, int per_qhead, bool pla
                          bool paged = false) {
   int inplace;
   if ((D == 64 || D == 128) && !topk_row_fits(N, G, D, paged, with_bias, 8, &inplace)) return false;
-  (void)per_qhead;  // shared chunk keys or one per query head: the same kernel
-  return plain && G <= 8 && (D == 64 || D == 128) && N >= 256 && N <= TOPK_R_MAXN &&
-         rows >= 96 && rows <= 2147483647L;
+  // Few rows: a workgroup streams its row's keys at about 40 GB/s whatever the others do, so the two-kernel path,
+  // which spreads a row's keys over the chip, is ahead only where those keys take longer than its extra launches
+  // and its slower selection (measured with a key per query head at 2048 chunks: 2 MiB of keys a row 82 us against
+  // 66 with 2 rows, 83 against 88 with 16; 1 MiB a row and less: the row kernel from one row on, 18 against 26 us
+  // at 4 rows of 512 chunks).
+  const long key_bytes = (long)N * (per_qhead ? G : 1) * D * 2;
+  if (rows < 16 && key_bytes > (3L << 19)) return false;
+  return plain && G <= 8 && (D == 64 || D == 128) && N >= 1 && N <= TOPK_R_MAXN && rows <= 2147483647L;
 }
 
 static int topk_fwd_row(const void* q, const void* lmks, const float* lse_swa, const float* bias, int32_t* indices,
@@ -2125,7 +2130,7 @@ static int decode_step_launch(const void* q, const void* lmks, const void* k, co
   a.q = (const bf16_t*)q; a.lmks = (const bf16_t*)lmks; a.k = (const bf16_t*)k; a.v = (const bf16_t*)v;
   a.lse_swa = lse_swa; a.bias = bias; a.indices = indices;
   a.lmk_hm = lmk_hm; a.lmk_cap = lmk_cap; a.perq = perq; a.bias_inplace = bias_inplace;
-  a.stagger_ticks = rows <= topk_cus() ? 800 : 0;  // one round of rows: they would run in step
+  a.stagger_ticks = rows <= topk_cus() && 4 * rows > 3 * topk_cus() ? 800 : 0;  // one full round of rows: they would run in step
   a.scores = (bf16_t*)scores; a.weights = (bf16_t*)weights; a.o = (bf16_t*)o;
   a.lse_total = lse_total; a.sel_logits = sel_logits;
   a.L = L; a.N = N; a.NP = NP; a.h_kv = H; a.G = G; a.topk = topk; a.block_size = block_size;

@@ -192,6 +192,9 @@ def decode_step(q, lmks, k, v, lse_swa, topk, block_size, window_size, q_offset=
     # chunks per query.  Repacking moves 8 bytes per cache element at about 5 TB/s, the one-launch kernel 256 * topk
     # bytes per query and feature pair at about 7.5 TB/s, which meet near L = Lkv / (20 * topk).
     many = L >= 64 and 16 * L * int(topk) >= Lkv
+    # Few rows with a key per query head on a long cache: a row's workgroup would stream its keys at about 40 GB/s
+    # while the rest of the chip idles (2 MiB a row: 82 us against 66 at two rows, 83 against 88 at sixteen); topk_use_row has the same line.
+    many = many or (per_qhead and B * L * h_kv < 16 and 2 * N * G * D > 3 << 19)
     if many or not (lib.hils_decode_step_covers(B, L, N, h_q, h_kv, D, int(topk), int(block_size),
                                                 int(pb is not None)) and Lkv >= N * block_size):
         if lmk_head_major:  # the two-call kernels read the reference's layout
