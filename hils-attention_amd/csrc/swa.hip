@@ -9,12 +9,7 @@
 // plus one row-swap reduction) and the probabilities are already the A operand of the second product.
 #include <type_traits>
 #include "stream_tiles.h"
-#include "../../include/hils_amd.h"
-
-struct SwaDims {
-  int Lq, Lk, HQ, H, window, chunk, mask_lmk, expand, kv_start, chunk_pow2;
-  float sm_scale;
-};
+#include "swa_dims.h"
 
 // Workgroup order.  Neighbouring blocks of a head read the same key / value (or query) tiles, and the
 // hardware hands consecutive workgroup ids to the 8 XCDs in turn: with the block index in the grid's
@@ -299,14 +294,14 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
         const int pc = tid + NT * i;
         int tok = (tile0 + ti) * 64 + pc / KSEG;
         tok = tok < dm.Lk ? tok : dm.Lk - 1;
-        kd[i] = *(const swa_u32x4*)(k + ((b * dm.Lk + tok) * (long)dm.H + hk) * D + (pc % KSEG) * 8);
+        kd[i] = *(const swa_u32x4*)(k + b * dm.k_batch + ((long)tok * dm.H + hk) * D + (pc % KSEG) * 8);
       }
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
         const int pc = tid + NT * i;
         int tok = (tile0 + ti) * 64 + pc / VSEG;
         tok = tok < dm.Lk ? tok : dm.Lk - 1;
-        vd[i] = *(const swa_u32x4*)(v + ((b * dm.Lk + tok) * (long)dm.H + hk) * DV + (pc % VSEG) * 8);
+        vd[i] = *(const swa_u32x4*)(v + b * dm.v_batch + ((long)tok * dm.H + hk) * DV + (pc % VSEG) * 8);
       }
     };
     auto stash = [&](int ti, const swa_u32x4 (&kd)[KPT], const swa_u32x4 (&vd)[VPT]) __attribute__((always_inline)) {
@@ -860,10 +855,10 @@ static int swa_launch_g(int G, int B, hipStream_t st, const bf16_t* q, const bf1
   }
 }
 
-extern "C" int hils_swa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B,
-                            int Lq, int Lk, int HQ, int H, int D, int Dv, int window, int chunk,
-                            int mask_lmk, int expand_to_chunk, int kv_start, float sm_scale,
-                            void* stream) {
+extern "C" int hils_swa_fwd_strided(const void* q, const void* k, const void* v, size_t k_batch_stride,
+                                    size_t v_batch_stride, void* o, float* lse, int B, int Lq, int Lk, int HQ,
+                                    int H, int D, int Dv, int window, int chunk, int mask_lmk, int expand_to_chunk,
+                                    int kv_start, float sm_scale, void* stream) {
   HILS_REQUIRE(q && k && v && o && lse, "hils_swa_fwd: null pointer");
   HILS_REQUIRE(B > 0 && Lq > 0 && Lk > 0 && HQ > 0 && H > 0, "hils_swa_fwd: sizes must be positive");
   HILS_REQUIRE(Lq <= Lk, "hils_swa_fwd: Lq (%d) must not exceed Lk (%d)", Lq, Lk);
@@ -877,18 +872,31 @@ extern "C" int hils_swa_fwd(const void* q, const void* k, const void* v, void* o
                "hils_swa_fwd: group size %d must be 1, 2, 4, 8 or 16", G);
   HILS_REQUIRE(((long)Lq / 8 + 1) * H * B < (1L << 31) - 8, "hils_swa_fwd: B * H * Lq too large for the grid");
   HILS_REQUIRE((long)kv_start + Lk < 2147483647L / 2, "hils_swa_fwd: positions overflow 32 bits");
+  HILS_REQUIRE(B == 1 || (k_batch_stride >= (size_t)Lk * H * D && v_batch_stride >= (size_t)Lk * H * Dv &&
+                          k_batch_stride % 8 == 0 && v_batch_stride % 8 == 0),
+               "hils_swa_fwd: a batch stride is shorter than a sequence or no multiple of 8 elements");
   SwaDims dm{Lq, Lk, HQ, H, window, chunk, mask_lmk, expand_to_chunk, kv_start,
-             (chunk & (chunk - 1)) == 0, sm_scale};
+             (chunk & (chunk - 1)) == 0, sm_scale, (long)k_batch_stride, (long)v_batch_stride};
   hipStream_t st = (hipStream_t)stream;
   const bf16_t *qq = (const bf16_t*)q, *kk = (const bf16_t*)k, *vv = (const bf16_t*)v;
   int rc;
-  if (D == 64 && Dv == 64) rc = swa_launch_g<64, 64>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
+  if (hils_swa_rows_better(B, dm)) rc = hils_swa_fwd_rows(B, st, q, k, v, o, lse, D, Dv, dm);
+  else if (D == 64 && Dv == 64) rc = swa_launch_g<64, 64>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   else if (D == 128 && Dv == 128) rc = swa_launch_g<128, 128>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   else if (D == 64) rc = swa_launch_g<64, 128>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   else rc = swa_launch_g<128, 64>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   if (rc) return rc;
   HILS_CHECK_LAUNCH("hils_swa_fwd");
   return HILS_OK;
+}
+
+extern "C" int hils_swa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B,
+                            int Lq, int Lk, int HQ, int H, int D, int Dv, int window, int chunk,
+                            int mask_lmk, int expand_to_chunk, int kv_start, float sm_scale,
+                            void* stream) {
+  const size_t row = (size_t)(Lk > 0 ? Lk : 0) * (size_t)(H > 0 ? H : 0);
+  return hils_swa_fwd_strided(q, k, v, row * (size_t)(D > 0 ? D : 0), row * (size_t)(Dv > 0 ? Dv : 0), o, lse, B, Lq,
+                              Lk, HQ, H, D, Dv, window, chunk, mask_lmk, expand_to_chunk, kv_start, sm_scale, stream);
 }
 
 template <int D, int DV, int G>

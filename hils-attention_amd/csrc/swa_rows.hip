@@ -1,0 +1,241 @@
+// Sliding-window attention for few query rows (a decode step, a short slice on a cache).
+//
+// The tile kernel (swa.hip) gives a workgroup 128 or 256 score rows and walks the window tile by tile:
+// with a single query per sequence most of those rows are padding and the walk over a window of 512 is a
+// serial chain of phases (19 us for one sequence, 33 us for 64 (sequence, KV head) pairs of heads of 128).
+// Here a workgroup owns 16 score rows (16/G queries times the G heads of a KV head: the 16 columns of the
+// matrix instructions) and its eight wavefronts share the WINDOW: units of 32 tokens go round-robin, the
+// next unit's K and V loads are in flight while one is worked on, and the eight partial results
+// (running maximum, sum, output) meet once in LDS.  The chain is two or three units long.
+//
+// S^T = K q^T takes the K rows straight from memory as A operands (a lane reads 16 bytes of its token's
+// row); V is staged row-major in the wavefront's own LDS area and read by the transposing LDS load as the
+// A operand of O^T += V^T P, in the token order in which the S^T accumulators hold P.  Rows are matrix
+// columns in both products, so maxima, sums and the rescaling of the accumulators stay in their lanes.
+#include "stream_tiles.h"
+#include "swa_dims.h"
+
+#define SR_WAVES 8
+#define SR_UNIT 32  // tokens a wavefront works on at a time
+
+template <int D, int DV>
+__global__ void __launch_bounds__(SR_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
+swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
+             bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int G, int n_rb) {
+  constexpr int KS = D / 32, MT = DV / 16;
+  constexpr int VL = DV / 8, TPI = 64 / VL, VI = SR_UNIT / TPI;  // lanes per V row, rows per load, loads per unit
+  constexpr int VP = 2 * DV + 16;                                // bytes of a staged V row
+  constexpr int OP = DV + 4;                                     // floats of a parked output row
+  constexpr int AREA = SR_UNIT * VP > 16 * OP * 4 ? SR_UNIT * VP : 16 * OP * 4;
+  typedef unsigned sr_u4 __attribute__((ext_vector_type(4)));
+  typedef short sr_s4 __attribute__((ext_vector_type(4)));
+  typedef short sr_s8 __attribute__((ext_vector_type(8)));
+  __shared__ __align__(16) unsigned char area_s[SR_WAVES * AREA];
+  __shared__ float m_s[SR_WAVES][16], l_s[SR_WAVES][16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, j = lane >> 4;
+  const int rb = blockIdx.x % n_rb;
+  const int hk = (blockIdx.x / n_rb) % dm.H;
+  const long b = blockIdx.x / n_rb / dm.H;
+  const int QB = 16 / G;
+  const int tq0 = rb * QB;
+  const int q_off = dm.kv_start + dm.Lk - dm.Lq;  // absolute position of query 0
+
+  // this lane's row and the key positions it sees, [vlo, vlo + vspan] (a start no position reaches: none)
+  const int t = tq0 + col / G, g = col % G;
+  const bool live = t < dm.Lq;
+  const int tc = live ? t : dm.Lq - 1;
+  bf16x8_t qb[KS];
+  {
+    const bf16_t* qp = q + ((b * dm.Lq + tc) * (long)dm.HQ + hk * G + g) * D + j * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qb[ks] = *(const bf16x8_t*)(qp + ks * 32);
+  }
+  auto win_start = [&](int tt) -> int {  // first absolute position query tt sees
+    const int left = q_off + tt - dm.window + 1;
+    return dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left;
+  };
+  int vlo;
+  unsigned vspan;
+  {
+    const int c0 = win_start(tc), hi = q_off + tc;
+    const bool some = live && hi >= c0;
+    vlo = some ? c0 : 0x7fffffff;
+    vspan = some ? (unsigned)(hi - c0) : 0u;
+  }
+  // key range of the workgroup (raw indices into k / v), in units
+  int lo = win_start(tq0) - dm.kv_start;
+  lo = lo < 0 ? 0 : lo;
+  int tq1 = tq0 + QB - 1;
+  tq1 = tq1 < dm.Lq ? tq1 : dm.Lq - 1;
+  int hi = q_off + tq1 - dm.kv_start + 1;
+  hi = hi < dm.Lk ? hi : dm.Lk;
+  const int n_units = hi > lo ? (hi - lo + SR_UNIT - 1) / SR_UNIT : 0;
+  const float c2 = dm.sm_scale * HILS_LOG2E;
+
+  const bf16_t* kb = k + b * dm.k_batch + (long)hk * D + j * 8;
+  const bf16_t* vb = v + b * dm.v_batch + (long)hk * DV + (lane % VL) * 8;
+  auto issue = [&](sr_u4 (&kd)[2][KS], sr_u4 (&vd)[VI], int u) __attribute__((always_inline)) {
+    const int t0 = lo + u * SR_UNIT;  // tokens past the end read the last row: their scores are masked
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      int tok = t0 + tt * 16 + col;
+      tok = tok < dm.Lk ? tok : dm.Lk - 1;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kd[tt][ks] = *(const sr_u4*)(kb + (long)tok * dm.H * D + ks * 32);
+    }
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      int tok = t0 + i * TPI + lane / VL;
+      tok = tok < dm.Lk ? tok : dm.Lk - 1;
+      vd[i] = *(const sr_u4*)(vb + (long)tok * dm.H * DV);
+    }
+  };
+
+  unsigned char* area = area_s + wave * AREA;
+  unsigned char* const w_addr = area + (lane / VL) * VP + (lane % VL) * 16;
+  const unsigned char* const t_addr = area + (4 * j + (col >> 2)) * VP + (col & 3) * 8;
+  f32x4_t O[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) O[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = HILS_NEG_INF, l_run = 0.f;  // of this lane's row over the units seen (l_run: this lane's tokens)
+
+  auto unit = [&](const sr_u4 (&kd)[2][KS], const sr_u4 (&vd)[VI], int u) __attribute__((always_inline)) {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < VI; ++i) *(sr_u4*)(w_addr + i * TPI * VP) = vd[i];
+    __builtin_amdgcn_wave_barrier();
+    f32x4_t S[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      S[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        S[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kd[tt][ks]), qb[ks], S[tt], 0, 0, 0);
+    }
+    const int tok_raw0 = lo + u * SR_UNIT + 4 * j;
+    const unsigned base = (unsigned)(dm.kv_start + tok_raw0 - vlo);
+    float mx = HILS_NEG_INF;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bool see = base + (unsigned)(tt * 16 + i) <= vspan && tok_raw0 + tt * 16 + i < dm.Lk;
+        if (dm.mask_lmk) {  // uniform
+          const int ta = dm.kv_start + tok_raw0 + tt * 16 + i + 1;
+          see = see && (dm.chunk_pow2 ? (ta & (dm.chunk - 1)) : ta % dm.chunk) != 0;
+        }
+        S[tt][i] = see ? S[tt][i] : HILS_NEG_INF;
+        mx = fmaxf(mx, S[tt][i]);
+      }
+    mx = rows_max(mx);
+    const float m_new = fmaxf(m_run, mx);
+    const bool any = m_new > HILS_NEG_INF;
+    const float mc = any ? m_new * c2 : 0.f;
+    const float corr = any ? __builtin_amdgcn_exp2f(fmaf(m_run, c2, -mc)) : 1.f;  // exp2(-inf) = 0: nothing yet
+    m_run = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(S[tt][i], c2, -mc));
+        S[tt][i] = e;
+        sum += e;
+      }
+    l_run = l_run * corr + sum;
+    sr_u4 pk;
+    pk.x = pack_bf2(S[0][0], S[0][1]);
+    pk.y = pack_bf2(S[0][2], S[0][3]);
+    pk.z = pack_bf2(S[1][0], S[1][1]);
+    pk.w = pack_bf2(S[1][2], S[1][3]);
+    const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, pk);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const sr_s4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) sr_s4*)(t_addr + mt * 32));
+      const sr_s4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) sr_s4*)(t_addr + mt * 32 + 16 * VP));
+      const sr_s8 a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) O[mt][i] *= corr;
+      O[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), pb, O[mt], 0, 0, 0);
+    }
+  };
+  {
+    // two units' loads in flight; an index past the end reads the last unit again and is not worked on
+    sr_u4 ka[2][KS], va[VI], kc[2][KS], vc[VI];
+    const int last = n_units - 1;
+    if (wave < n_units) {
+      issue(ka, va, wave);
+      for (int u = wave; u < n_units; u += 2 * SR_WAVES) {
+        const int u1 = u + SR_WAVES, u2 = u + 2 * SR_WAVES;
+        issue(kc, vc, u1 < last ? u1 : last);
+        unit(ka, va, u);
+        if (u1 >= n_units) break;
+        issue(ka, va, u2 < last ? u2 : last);
+        unit(kc, vc, u1);
+      }
+    }
+  }
+  // park the partial results: accumulator register i of tile mt in lane (row = col, j) is feature mt*16 + 4j + i
+  __builtin_amdgcn_wave_barrier();
+  float* o_s = (float*)area;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) *(f32x4_t*)&o_s[col * OP + mt * 16 + 4 * j] = O[mt];
+  const float l_row = rows_sum(l_run);
+  if (j == 0) {
+    m_s[wave][col] = m_run;
+    l_s[wave][col] = l_row;
+  }
+  __syncthreads();
+  // 16 rows x DV/4 pieces of four features over the workgroup
+  for (int p = tid; p < 16 * (DV / 4); p += SR_WAVES * 64) {
+    const int row = p / (DV / 4), d4 = p % (DV / 4);
+    const int tr = tq0 + row / G;
+    if (tr >= dm.Lq) continue;
+    float M = HILS_NEG_INF;
+#pragma unroll
+    for (int w = 0; w < SR_WAVES; ++w) M = fmaxf(M, m_s[w][row]);
+    float L = 0.f;
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    if (M > HILS_NEG_INF) {
+#pragma unroll
+      for (int w = 0; w < SR_WAVES; ++w) {
+        const float f = __builtin_amdgcn_exp2f((m_s[w][row] - M) * c2);
+        const f32x4_t ow = *(const f32x4_t*)((const float*)(area_s + w * AREA) + row * OP + d4 * 4);
+        L = fmaf(f, l_s[w][row], L);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = fmaf(f, ow[i], x[i]);
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    const long rix = (b * dm.Lq + tr) * (long)dm.HQ + hk * G + row % G;
+    uint2 pk;
+    pk.x = pack_bf2(x[0] * inv, x[1] * inv);
+    pk.y = pack_bf2(x[2] * inv, x[3] * inv);
+    *(uint2*)(o + rix * DV + d4 * 4) = pk;
+    if (d4 == 0) lse[rix] = L > 0.f ? (M * c2 + __builtin_amdgcn_logf(L)) * HILS_LN2 : HILS_NEG_INF;
+  }
+}
+
+// Score rows the tile kernel would spread over too few workgroups.
+bool hils_swa_rows_better(int B, const SwaDims& dm) {
+  const long rows = (long)B * dm.Lq * dm.HQ;
+  return rows <= SWA_ROWS_MAX;
+}
+
+int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int D,
+                      int Dv, const SwaDims& dm) {
+  const int G = dm.HQ / dm.H;
+  const int n_rb = (dm.Lq + 16 / G - 1) / (16 / G);
+  const dim3 grid((unsigned)((long)n_rb * dm.H * B)), wg(SR_WAVES * 64);
+#define SR_CALL(D_, V_)                                                                                     \
+  hipLaunchKernelGGL((swa_fwd_rows<D_, V_>), grid, wg, 0, st, (const bf16_t*)q, (const bf16_t*)k,            \
+                     (const bf16_t*)v, (bf16_t*)o, lse, dm, G, n_rb)
+  if (D == 64 && Dv == 64) SR_CALL(64, 64);
+  else if (D == 128 && Dv == 128) SR_CALL(128, 128);
+  else if (D == 64) SR_CALL(64, 128);
+  else SR_CALL(128, 64);
+#undef SR_CALL
+  return HILS_OK;
+}

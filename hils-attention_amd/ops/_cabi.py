@@ -6,6 +6,7 @@ fails, a RuntimeError is raised.  There is no Triton/TileLang/PyTorch fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_float, c_int, c_void_p
 
@@ -13,6 +14,7 @@ import torch
 
 _PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG_DIR, "libhils_amd.so")
+HOST_PATH = os.path.join(_PKG_DIR, "_hils_host.so")
 
 _P, _I, _F, _Z = c_void_p, c_int, c_float, ctypes.c_size_t
 
@@ -47,10 +49,12 @@ SIGNATURES = {
     "hils_norm_rope_pool_bwd_ws": [_P] * 8 + [_I, _P, _Z] + [_I] * 6 + [_F, _P],
     "hils_norm_rope_pool_bwd_workspace": [_I] * 5,
     "hils_swa_fwd": [_P] * 5 + [_I] * 12 + [_F, _P],
+    "hils_swa_fwd_strided": [_P] * 3 + [_Z, _Z] + [_P] * 2 + [_I] * 12 + [_F, _P],
     "hils_swa_bwd": [_P] * 11 + [_I] * 10 + [_F, _P],
 }
 
 _lib = None
+_host = None
 
 
 def load():
@@ -89,6 +93,22 @@ def load():
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def host():
+    """The native host path (csrc/host_ops.cpp), loaded once; raise if it has not been built."""
+    global _host
+    if _host is None:
+        load()  # the library whose entry points the module calls
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(
+                f"{HOST_PATH} is missing: build it with `python __graft_entry__.py build`. "
+                "This package has no fallback path.")
+        spec = importlib.util.spec_from_file_location("_hils_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _host = mod
+    return _host
 
 
 def ptr(t):

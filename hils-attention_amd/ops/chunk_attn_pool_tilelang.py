@@ -12,56 +12,15 @@ import torch
 from . import _cabi
 
 
-class ChunkAttnPoolFunction(torch.autograd.Function):
-    """Mirrors ChunkAttnPoolFunction (ops/chunk_attn_pool_tilelang.py:540-602); k_chunked may carry
-    fewer heads than mu_q (grouped query heads: head h reads K head h // (H // h_kv)), which the
-    reference reaches by repeating K's heads in memory first
+class ChunkAttnPoolFunction:
+    """Mirrors ChunkAttnPoolFunction (ops/chunk_attn_pool_tilelang.py:540-602): the autograd node is
+    native (csrc/host_ops.cpp).  k_chunked may carry fewer heads than mu_q (grouped query heads: head h
+    reads K head h // (H // h_kv)), which the reference reaches by repeating K's heads in memory first
     (models/FlashHiLS/hils_attention.py:20-50, :391)."""
 
     @staticmethod
-    def forward(ctx, mu_q, k_chunked, sm_scale, compact_lmk_k=False, shared_k=False):
-        _cabi.require_gpu_bf16("chunk_attn_pool", mu_q, k_chunked)
-        B, N, H, D = mu_q.shape
-        S, HK = k_chunked.shape[2], k_chunked.shape[3]
-        assert k_chunked.shape == (B, N, S, HK, D) and H % HK == 0, (
-            f"k_chunked shape {tuple(k_chunked.shape)} does not go with mu_q {tuple(mu_q.shape)}")
-        assert not shared_k or HK == H
-        BN = B * N
-        mu_flat = mu_q.reshape(BN, H, D).contiguous()
-        k_flat = k_chunked.reshape(BN, S, HK, D).contiguous()
-        compact = bool(compact_lmk_k)
-        lmk_k = torch.empty((BN, H, D), dtype=mu_q.dtype, device=mu_q.device)
-        lmk_b = torch.empty((BN, H), dtype=torch.float32, device=mu_q.device)
-        p_saved = torch.empty((BN, S, H), dtype=torch.float32, device=mu_q.device)
-        _cabi.call("hils_attn_pool_fwd", _cabi.ptr(mu_flat), _cabi.ptr(k_flat), _cabi.ptr(lmk_k),
-                   _cabi.ptr(lmk_b), _cabi.ptr(p_saved), BN, S, H, HK, D, float(sm_scale),
-                   int(compact), int(bool(shared_k)))
-        ctx.save_for_backward(mu_flat, k_flat, p_saved, lmk_b)
-        ctx.sm_scale = float(sm_scale)
-        ctx.orig_shape = (B, N, H, HK, D, S)
-        ctx.compact = compact
-        ctx.shared_k = bool(shared_k)
-        return lmk_k.reshape(B, N, H, D), lmk_b.reshape(B, N, H)
-
-    @staticmethod
-    def backward(ctx, grad_lmk_k, grad_lmk_b):
-        mu_flat, k_flat, p_saved, lmk_b = ctx.saved_tensors
-        B, N, H, HK, D, S = ctx.orig_shape
-        BN = B * N
-        if grad_lmk_k is None or ctx.compact:
-            grad_lmk_k = torch.zeros((BN, H, D), dtype=mu_flat.dtype, device=mu_flat.device)
-        else:
-            grad_lmk_k = grad_lmk_k.reshape(BN, H, D).to(mu_flat.dtype).contiguous()
-        if grad_lmk_b is None:
-            grad_lmk_b = torch.zeros((BN, H), dtype=torch.float32, device=mu_flat.device)
-        else:
-            grad_lmk_b = grad_lmk_b.reshape(BN, H).float().contiguous()
-        d_mu = torch.empty_like(mu_flat)
-        d_k = torch.empty_like(k_flat)
-        _cabi.call("hils_attn_pool_bwd", _cabi.ptr(mu_flat), _cabi.ptr(k_flat), _cabi.ptr(p_saved),
-                   _cabi.ptr(lmk_b), _cabi.ptr(grad_lmk_k), _cabi.ptr(grad_lmk_b), _cabi.ptr(d_mu),
-                   _cabi.ptr(d_k), BN, S, H, HK, D, ctx.sm_scale, int(ctx.compact), int(ctx.shared_k))
-        return d_mu.reshape(B, N, H, D), d_k.reshape(B, N, S, HK, D), None, None, None
+    def apply(mu_q, k_chunked, sm_scale, compact_lmk_k=False, shared_k=False):
+        return _cabi.host().attn_pool(mu_q, k_chunked, float(sm_scale), bool(compact_lmk_k), bool(shared_k))
 
 
 def chunk_attn_pool(mu_q, k_chunked, sm_scale=None):

@@ -17,95 +17,21 @@ def _check_kv_workspace(ws, need_bytes, device, what):
             "with prepare_kv_workspace for this shape.")
 
 
-class _hils_block_M_attention_inverse(torch.autograd.Function):
-    """Mirrors _hils_block_M_attention_inverse (ops/hils_fwd_bwd_head.py:771-913)."""
+class _hils_block_M_attention_inverse:
+    """Mirrors _hils_block_M_attention_inverse (ops/hils_fwd_bwd_head.py:771-913): the autograd node is
+    native (csrc/host_ops.cpp)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, weights, indices, block_size, sm_scale, mask_last_token,
-                is_training, slope=None, kv_workspace=None, swa_o=None, swa_weight_index=None):
-        assert q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
-        assert weights.is_contiguous() and indices.is_contiguous()
-        _cabi.require_gpu_bf16("HiLS_block_M_head", q)
-        # inference may read K and V of an offloaded cache in place (pinned host memory)
-        _cabi.require_gpu_bf16("HiLS_block_M_head", k, v, pinned_ok=not is_training)
-        B, L, HQ, D = q.shape
-        L_kv, H, Dk = k.shape[1], k.shape[2], k.shape[-1]
-        Dv = v.shape[-1]
-        K = indices.shape[-1]
-        num_weights = weights.shape[-1]
-        assert HQ % H == 0, f"HQ={HQ} must be divisible by H={H}"
-        assert Dk == D, f"Q head_dim ({D}) must equal K head_dim ({Dk})"
-        assert indices.shape == (B, L, H, K), f"indices shape {tuple(indices.shape)} != {(B, L, H, K)}"
-        assert weights.shape[:3] == (B, L, HQ) and num_weights >= K, (
-            f"weights shape {tuple(weights.shape)} must be ({B}, {L}, {HQ}, >= {K})")
-        if sm_scale is None:
-            sm_scale = 1.0 / math.sqrt(D)
-        slope_dev = None
-        if slope is not None:
-            assert slope.shape == (HQ,), f"slope must be 1-D with shape ({HQ},), got {tuple(slope.shape)}"
-            slope_dev = slope.to(dtype=torch.float32, device=q.device).contiguous()
-        w_in = weights.to(q.dtype).contiguous()
-        idx_in = indices.to(torch.int32).contiguous()
-        swa_in, merge_col = None, 0
-        if swa_o is not None:
-            assert swa_o.shape == (B, L, HQ, Dv), f"swa_o shape {tuple(swa_o.shape)} != {(B, L, HQ, Dv)}"
-            merge_col = int(K if swa_weight_index is None else swa_weight_index) % num_weights
-            assert merge_col >= K, f"the local branch's weight column ({merge_col}) lies among the {K} chunk slots"
-            _cabi.require_gpu_bf16("HiLS_block_M_head", swa_o)
-            swa_in = swa_o.contiguous()
-        o = torch.empty((B, L, HQ, Dv), dtype=q.dtype, device=q.device)
-        lse = None
-        if is_training:
-            lse = torch.empty((B, L, HQ, K), dtype=torch.float32, device=q.device)
-        ws_ready = 0
+    def apply(q, k, v, weights, indices, block_size, sm_scale, mask_last_token, is_training, slope=None,
+              kv_workspace=None, swa_o=None, swa_weight_index=None):
         if kv_workspace is not None:
-            need = _cabi.sparse_attn_fwd_workspace_bytes(B, L, L_kv, HQ, H, D, Dv, K, HQ, 1,
-                                                         int(block_size), 0.0)
+            B, L, HQ, D = q.shape
+            L_kv, H, Dv, K = k.shape[1], k.shape[2], v.shape[-1], indices.shape[-1]
+            need = _cabi.sparse_attn_fwd_workspace_bytes(B, L, L_kv, HQ, H, D, Dv, K, HQ, 1, int(block_size), 0.0)
             _check_kv_workspace(kv_workspace, need, q.device,
                                 f"q_len {L}, kv_len {L_kv}, {HQ}/{H} heads, D {D}, Dv {Dv}, top-{K}")
-            ws, ws_ready = kv_workspace, 1
-        else:
-            ws = _cabi.sparse_attn_fwd_workspace(q.device, B, L, L_kv, HQ, H, D, Dv, K, HQ, 1,
-                                                 int(block_size), 0.0)
-        _cabi.call("hils_sparse_attn_fwd", _cabi.ptr(q), _cabi.ptr(k), _cabi.ptr(v), _cabi.ptr(w_in),
-                   _cabi.ptr(idx_in), _cabi.ptr(slope_dev), _cabi.ptr(swa_in), _cabi.ptr(o), _cabi.ptr(lse),
-                   _cabi.ptr(ws), _cabi.nbytes(ws), ws_ready, B, L, L_kv, HQ, H, D, Dv, K, num_weights, HQ, 1, int(block_size),
-                   float(sm_scale), int(bool(mask_last_token)), 0.0, merge_col)
-        ctx.is_training = bool(is_training)
-        if is_training:
-            ctx.save_for_backward(q, k, v, w_in, idx_in, lse, slope_dev, swa_in)
-            ctx.cfg = (B, L, L_kv, HQ, H, D, Dv, K, num_weights, int(block_size), float(sm_scale),
-                       int(bool(mask_last_token)), merge_col)
-            ctx.w_dtype = weights.dtype
-        return o
-
-    @staticmethod
-    def backward(ctx, do):
-        if not getattr(ctx, "is_training", True):
-            raise RuntimeError(
-                "[_hils_block_M_attention_inverse] forward ran with is_training=False: the "
-                "per-chunk LSE needed by the backward was not saved.")
-        q, k, v, w_in, idx_in, lse, slope_dev, swa_in = ctx.saved_tensors
-        B, L, L_kv, HQ, H, D, Dv, K, NW, S, sm_scale, mask_last, merge_col = ctx.cfg
-        d_swa = torch.empty_like(swa_in) if swa_in is not None else None
-        do = do.to(q.dtype).contiguous()
-        dq = torch.empty_like(q)
-        dw = torch.zeros((B, L, HQ, NW), dtype=torch.float32, device=q.device)
-        ws = _cabi.sparse_attn_bwd_workspace(q.device, B, L, L_kv, HQ, H, D, Dv, K, HQ, 1, S, 0.0)
-        # the workspace kernels write dk / dv once, as bf16; the shape-generic one adds into fp32
-        kv16 = ws is not None and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16
-        if kv16:
-            dk, dv = torch.empty_like(k), torch.empty_like(v)
-        else:
-            dk = torch.zeros(k.shape, dtype=torch.float32, device=k.device)
-            dv = torch.zeros(v.shape, dtype=torch.float32, device=v.device)
-        _cabi.call("hils_sparse_attn_bwd", _cabi.ptr(q), _cabi.ptr(k), _cabi.ptr(v), _cabi.ptr(w_in),
-                   _cabi.ptr(idx_in), _cabi.ptr(slope_dev), _cabi.ptr(lse), _cabi.ptr(do),
-                   _cabi.ptr(dq), _cabi.ptr(dk), _cabi.ptr(dv), _cabi.ptr(dw), _cabi.ptr(ws), _cabi.nbytes(ws),
-                   B, L, L_kv, HQ, H, D, Dv, K, NW, HQ, 1, S, sm_scale, mask_last, 0.0,
-                   _cabi.ptr(swa_in), _cabi.ptr(d_swa), merge_col, int(kv16))
-        return (dq, dk.to(k.dtype), dv.to(v.dtype), dw.to(ctx.w_dtype), None,
-                None, None, None, None, None, None, d_swa, None)
+        return _cabi.host().sparse_attn(q, k, v, weights, indices, int(block_size), sm_scale, bool(mask_last_token),
+                                        bool(is_training), slope, kv_workspace, swa_o, swa_weight_index)
 
 
 class _hils_block_M_attention_f32(torch.autograd.Function):

@@ -6,71 +6,30 @@ sequence; the backward of the returned scores is sparse (no dense (L x N) scatte
 Selection order: score descending, lower chunk index wins a tie; indices come back sorted
 ascending with -1 padding.
 """
-import math
-
 import torch
 
 from . import _cabi
 
 
-class SoftmaxTopKMaxPoolingFusedFn(torch.autograd.Function):
-    """Mirrors SoftmaxTopKMaxPoolingFusedFn (ops/topk_head_softmax.py:975-1092)."""
+class SoftmaxTopKMaxPoolingFusedFn:
+    """Mirrors SoftmaxTopKMaxPoolingFusedFn (ops/topk_head_softmax.py:975-1092): the autograd node is
+    native (csrc/host_ops.cpp).  Returns indices (B,L,h_kv,topk) and scores (B,L,h_kv,G,topk)."""
 
     @staticmethod
-    def forward(ctx, q, lmks, lse_swa, topk, block_size, window_size, is_causal, q_offset,
-                drop_mask, sm_scale, bias, gumbel_noise, per_qhead_lmks, debug):
-        B, L, h_kv, G, D = q.shape
-        B2, N, lmks_h, D2 = lmks.shape
-        assert B == B2 and D == D2
-        if per_qhead_lmks:
-            assert lmks_h == h_kv * G, (
-                f"per_qhead_lmks expects lmks h dim = h_kv*G ({h_kv * G}), got {lmks_h}")
-        else:
-            assert lmks_h == h_kv, f"default mode expects lmks h dim = h_kv ({h_kv}), got {lmks_h}"
-        _cabi.require_gpu_bf16("online_softmax_topk_head", q, lmks)
-        q_in = q.contiguous()
-        k_in = lmks.contiguous()
-        lse_in = lse_swa.reshape(B, L, h_kv, G).float().contiguous()
-        dev = q.device
-        scale = float(sm_scale) if sm_scale is not None else 1.0 / math.sqrt(D)
-        indices = torch.empty((B, L, h_kv, topk), dtype=torch.int32, device=dev)
-        scores = torch.empty((B, L, h_kv, G, topk), dtype=q.dtype, device=dev)
-        lse_total = sel_logits = None
+    def apply(q, lmks, lse_swa, topk, block_size, window_size, is_causal, q_offset,
+              drop_mask, sm_scale, bias, gumbel_noise, per_qhead_lmks, debug):
+        dbg, no_ws = [], False
         if debug is not None:
-            lse_total = torch.empty((B, L, h_kv, G), dtype=torch.float32, device=dev)
-            sel_logits = torch.full((B, L, h_kv, G, N), float("-inf"), dtype=torch.float32, device=dev)
-        if drop_mask is not None:
-            assert drop_mask.shape == (B, L, N), f"drop_mask shape {tuple(drop_mask.shape)} != {(B, L, N)}"
-            drop_mask = drop_mask.to(torch.int32).contiguous()
-        ws = None
-        if debug is None or not debug.get("no_workspace"):  # test hook: keep the one-kernel path
-            ws = _cabi.topk_fwd_workspace(dev, B, L, N, h_kv, G)
-        _cabi.call("hils_topk_fwd", _cabi.ptr(q_in), _cabi.ptr(k_in), _cabi.ptr(lse_in),
-                   _cabi.ptr(bias), _cabi.ptr(gumbel_noise), _cabi.ptr(drop_mask),
-                   _cabi.ptr(indices), _cabi.ptr(scores), _cabi.ptr(lse_total),
-                   _cabi.ptr(sel_logits), _cabi.ptr(ws), _cabi.nbytes(ws), B, L, N, h_kv, G, D, int(topk), int(block_size),
-                   int(window_size), int(bool(is_causal)), int(q_offset), int(bool(per_qhead_lmks)),
-                   scale)
+            B, L, h_kv, G, _ = q.shape
+            dbg = [torch.empty((B, L, h_kv, G), dtype=torch.float32, device=q.device),
+                   torch.full((B, L, h_kv, G, lmks.shape[1]), float("-inf"), dtype=torch.float32, device=q.device)]
+            no_ws = bool(debug.get("no_workspace"))  # test hook: keep the one-kernel path
+        indices, scores = _cabi.host().topk_select(
+            q, lmks, lse_swa, int(topk), int(block_size), int(window_size), bool(is_causal), int(q_offset),
+            drop_mask, sm_scale, bias, gumbel_noise, bool(per_qhead_lmks), dbg, no_ws)
         if debug is not None:
-            debug["lse_total"] = lse_total
-            debug["sel_logits"] = sel_logits
-        ctx.save_for_backward(q_in, k_in, indices)
-        ctx.cfg = (B, L, N, h_kv, G, D, int(topk), bool(per_qhead_lmks), scale)
-        ctx.mark_non_differentiable(indices)
-        return indices, scores
-
-    @staticmethod
-    def backward(ctx, grad_indices_unused, grad_scores):
-        q_in, k_in, indices = ctx.saved_tensors
-        B, L, N, h_kv, G, D, topk, per_qhead, scale = ctx.cfg
-        gs = grad_scores.to(q_in.dtype).contiguous()
-        dq = torch.empty_like(q_in)
-        dlmk = torch.zeros(k_in.shape, dtype=torch.float32, device=k_in.device)
-        ws = _cabi.topk_bwd_workspace(q_in.device, B, L, N, h_kv, G, D, topk)
-        _cabi.call("hils_topk_bwd", _cabi.ptr(gs), _cabi.ptr(q_in), _cabi.ptr(k_in),
-                   _cabi.ptr(indices), _cabi.ptr(dq), _cabi.ptr(dlmk), _cabi.ptr(ws), _cabi.nbytes(ws), B, L, N, h_kv, G, D, topk,
-                   int(per_qhead), scale)
-        return (dq, dlmk.to(k_in.dtype)) + (None,) * 12
+            debug["lse_total"], debug["sel_logits"] = dbg
+        return indices, scores.view(*q.shape[:4], -1)
 
 
 def _bias_per_group(bias, B, N, h_kv, G, device):

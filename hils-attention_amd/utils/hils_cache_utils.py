@@ -354,80 +354,5 @@ def paged_hils_attend(q, k_pages, v_pages, lmk_pages, page_table, lse_swa, seq_l
     head-major (``lmk_dense`` (B,H,cap,D), prior bias ``prior_dense`` (B,H,cap,G)); either may carry h_q
     heads in place of H (one chunk key per query head); the prior bias, when given, is the selection
     bias and the bias of the inter-chunk softmax (models/FlashHiLS/hils_attention.py:568-602)."""
-    dense = lmk_dense is not None
-    _cabi.require_gpu_bf16("paged_hils_attend", q, k_pages, v_pages, lmk_dense if dense else lmk_pages)
-    B, Lq, HQ, D = q.shape
-    num_pages, H, S, Dk = k_pages.shape
-    assert S == 64 and Dk == D and v_pages.shape == k_pages.shape
-    assert page_table.dtype == torch.int32 and page_table.shape[0] == B and page_table.is_contiguous()
-    assert HQ % H == 0
-    G = HQ // H
-    max_pages = page_table.shape[1]
-    N = seq_len // S  # chunks with a pooled key
-    assert 0 < N <= max_pages
-    cap = 0
-    h_lmk = lmk_dense.shape[1] if dense else lmk_pages.shape[1]
-    assert h_lmk in (H, HQ), f"the chunk keys carry {h_lmk} heads: neither the {H} KV heads nor the {HQ} query heads"
-    per_qhead = int(h_lmk != H)
-    if dense:
-        cap = lmk_dense.shape[2]
-        assert lmk_dense.shape == (B, h_lmk, cap, D) and lmk_dense.is_contiguous() and cap >= N
-        bias = None
-        if prior_dense is not None:
-            assert prior_dense.shape == (B, H, cap, G) and prior_dense.dtype == torch.float32
-            bias = prior_dense.contiguous()
-        lmk_arg = lmk_dense
-    else:
-        assert lmk_pages.shape == (num_pages, h_lmk, D) and lmk_pages.is_contiguous()
-        bias = None
-        if prior_pages is not None:
-            assert prior_pages.shape == (num_pages, HQ) and prior_pages.dtype == torch.float32
-            bias = prior_pages.contiguous()
-        lmk_arg = lmk_pages
-    if sm_scale is None:
-        sm_scale = 1.0 / math.sqrt(D)
-    dev = q.device
-    lse = lse_swa.reshape(B, Lq, HQ).float().contiguous()
-    indices = torch.empty((B, Lq, H, topk), dtype=torch.int32, device=dev)
-    scores = torch.empty((B, Lq, HQ, topk), dtype=q.dtype, device=dev)
-    weights = torch.empty((B, Lq, HQ, topk + 1), dtype=q.dtype, device=dev)
-    lse_total = sel_logits = None
-    if _debug is not None:
-        lse_total = torch.empty((B, Lq, H, G), dtype=torch.float32, device=dev)
-        sel_logits = torch.full((B, Lq, H, G, N), float("-inf"), dtype=torch.float32, device=dev)
-    qc = q.contiguous()
-    if _cabi.load().hils_decode_step_covers(B, Lq, N, HQ, H, D, int(topk), S, int(bias is not None)):
-        # selection and attention of a row by one workgroup, one launch
-        o = torch.empty((B, Lq, HQ, D), dtype=q.dtype, device=dev)
-        _cabi.call("hils_decode_step_paged", _cabi.ptr(qc), _cabi.ptr(lmk_arg), _cabi.ptr(k_pages),
-                   _cabi.ptr(v_pages), _cabi.ptr(page_table), _cabi.ptr(lse), _cabi.ptr(bias), _cabi.ptr(indices),
-                   _cabi.ptr(scores), _cabi.ptr(weights), _cabi.ptr(o), _cabi.ptr(lse_total), _cabi.ptr(sel_logits),
-                   B, Lq, N, HQ, H, D, int(topk), S, int(window_size), seq_len - Lq, max_pages, num_pages,
-                   float(sm_scale), float(sm_scale), 1, int(dense), int(dense), cap, per_qhead)
-        if _debug is not None:
-            _debug.update(lse_total=lse_total, sel_logits=sel_logits, scores=scores)
-        return o, weights, indices
-    if dense:
-        # shapes outside the one-launch kernel: selection and softmax on the reference's dense layout,
-        # attention on the pages
-        lmk_tm = lmk_dense[:, :, :N].permute(0, 2, 1, 3).contiguous()
-        pb = None if bias is None else bias[:, :, :N].permute(0, 2, 1, 3).reshape(B, N, HQ).contiguous()
-        indices, scores, weights = topk_chunk_weights(qc, lmk_tm, lse, topk, S, window_size,
-                                                      q_offset=seq_len - Lq, sm_scale=sm_scale, prior_b=pb,
-                                                      num_kv_heads=H)
-        if _debug is not None:
-            _debug.update(scores=scores)
-    else:
-        _cabi.call("hils_topk_fwd_weights_paged", _cabi.ptr(qc), _cabi.ptr(lmk_pages), _cabi.ptr(page_table),
-                   _cabi.ptr(lse), _cabi.ptr(bias), _cabi.ptr(indices), _cabi.ptr(scores), _cabi.ptr(weights),
-                   _cabi.ptr(lse_total), _cabi.ptr(sel_logits), B, Lq, N, H, G, D, int(topk), S, int(window_size),
-                   seq_len - Lq, max_pages, num_pages, float(sm_scale), per_qhead)
-        if _debug is not None:
-            _debug.update(lse_total=lse_total, sel_logits=sel_logits, scores=scores)
-    o = torch.empty((B, Lq, HQ, D), dtype=q.dtype, device=dev)
-    n_ws = _cabi.load().hils_sparse_attn_decode_paged_workspace(B, Lq, HQ, H, D, int(topk))
-    ws = torch.empty(n_ws, dtype=torch.uint8, device=dev) if n_ws else None
-    _cabi.call("hils_sparse_attn_decode_paged", _cabi.ptr(qc), _cabi.ptr(k_pages), _cabi.ptr(v_pages),
-               _cabi.ptr(page_table), _cabi.ptr(weights), _cabi.ptr(indices), _cabi.ptr(o), _cabi.ptr(ws), _cabi.nbytes(ws),
-               B, Lq, HQ, H, D, int(topk), topk + 1, max_pages, num_pages, float(sm_scale), 1)
-    return o, weights, indices
+    return _cabi.host().paged_step(q, k_pages, v_pages, lmk_pages, page_table, lse_swa, int(seq_len), int(topk),
+                                   int(window_size), sm_scale, _debug, prior_pages, lmk_dense, prior_dense)

@@ -349,6 +349,12 @@ int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float* log_z, con
 int hils_swa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int B, int Lq,
                  int Lk, int HQ, int H, int D, int Dv, int window, int chunk, int mask_lmk,
                  int expand_to_chunk, int kv_start, float sm_scale, void* stream);
+/* The same with the elements from a sequence's keys / values to the next one's given (multiples of 8): the
+ * last Lk tokens of a longer cache buffer are read in place. */
+int hils_swa_fwd_strided(const void* q, const void* k, const void* v, size_t k_batch_stride, size_t v_batch_stride,
+                         void* o, float* lse, int B, int Lq, int Lk, int HQ, int H, int D, int Dv, int window,
+                         int chunk, int mask_lmk, int expand_to_chunk, int kv_start, float sm_scale, void* stream);
+
 
 /* Backward (training: Lq == Lk = L, kv_start = 0).  Replaces flex_attn_bwd_preprocess,
  * flex_attn_bwd_dq and flex_attn_bwd_dkdv (ops/flex_attn_tilelang.py:270-1153) as driven by
