@@ -40,10 +40,13 @@ struct DrDims {
   int max_pages, num_pages;
 };
 
-static inline size_t dr_smem_bytes(int D, int G, int nwave) {
+__host__ __device__ static inline size_t dr_work_bytes(int D, int G, int nwave) {
   return (size_t)nwave * 32 * (2 * D + 16)             // staging areas: 32 padded token rows
-         + (size_t)nwave * G * D * sizeof(float)       // partial outputs
-         + (size_t)nwave * DR_MAXSLOT * (sizeof(long) + sizeof(int))  // slot lists
+         + (size_t)nwave * G * D * sizeof(float);      // partial outputs
+}
+static inline size_t dr_list_bytes(int nwave) { return (size_t)nwave * DR_MAXSLOT * (sizeof(long) + sizeof(int)); }
+static inline size_t dr_smem_bytes(int D, int G, int nwave) {
+  return dr_work_bytes(D, G, nwave) + dr_list_bytes(nwave)
          + (size_t)nwave * DR_MAXSLOT * DR_NH * sizeof(bf16_t);       // slot weights
 }
 
@@ -52,17 +55,18 @@ struct DrNoHook {
 };
 
 // One (query, KV head) row by a workgroup of NWAVE wavefronts: `split` of dm.nsplit shares of the
-// slots, KV head hk, query bt = b * L + t; dr_smem = dr_smem_bytes(D, G, NWAVE) bytes of LDS.
-// weights and indices may point into LDS (the one-launch decode step hands the row's selection over
-// there: generic loads reach either memory).  `hook` runs once in every wavefront after its first
-// chunk's loads have been issued and before it writes the staging areas of dr_smem (that kernel puts
-// the barrier there that ends the selection's use of the same LDS).
-template <int D, int NWAVE, class Hook = DrNoHook>
+// slots, KV head hk, query bt = b * L + t; dr_smem = dr_work_bytes(D, G, NWAVE) bytes of LDS, slots =
+// dr_list_bytes(NWAVE) more (and the slot weights behind them).
+// WLDS (the decode step's kernels): weights and indices point into LDS, where the row's selection leaves
+// them.  `hook` runs once in every wavefront after its first chunk's loads have been issued and before it
+// writes dr_smem or reads the weights: those kernels work the weights out there, and the hook ends with the
+// barrier that ends the selection's use of the same LDS.
+template <int D, int NWAVE, bool WLDS = false, class Hook = DrNoHook>
 __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                  const bf16_t* __restrict__ v, const bf16_t* __restrict__ weights,
                                                  const int32_t* __restrict__ indices, bf16_t* __restrict__ o,
                                                  float* __restrict__ partial, const DrDims& dm, char* dr_smem,
-                                                 int split, int hk, long bt, Hook hook = Hook{}) {
+                                                 int split, int hk, long bt, char* slots, Hook hook = Hook{}) {
   constexpr int LR = D / 8;          // lanes per token row
   constexpr int TPI = 64 / LR;       // token rows per load instruction
   constexpr int GL = DR_QT / TPI;    // load instructions per group
@@ -79,7 +83,7 @@ __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, c
 
   char* stage_w = dr_smem + (size_t)wave * STAGE_B;
   float* o_s = (float*)(dr_smem + (size_t)NWAVE * STAGE_B);  // [wave][G][D]
-  long* sl_off_all = (long*)(o_s + (size_t)NWAVE * G * D);
+  long* sl_off_all = (long*)slots;
   int* sl_id_all = (int*)(sl_off_all + NWAVE * DR_MAXSLOT);
   bf16_t* sl_w_all = (bf16_t*)(sl_id_all + NWAVE * DR_MAXSLOT);
   long* sl_off = sl_off_all + wave * DR_MAXSLOT;
@@ -110,7 +114,7 @@ __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, c
 #pragma unroll
     for (int p4 = 0; p4 < DR_MAXSLOT / 4; ++p4) {
       wv[p4] = 0;
-      if (p4 * 4 < nmine) {  // uniform
+      if (!WLDS && p4 * 4 < nmine) {  // uniform
         const int i = p4 * 4 + j;
         if (i < nmine && col < G)
           wv[p4] = weights[(bt * dm.HQ + hk * G + col) * (long)dm.NW + s_begin + wave + i * NWAVE];
@@ -139,7 +143,7 @@ __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, c
     }
 #pragma unroll
     for (int p4 = 0; p4 < DR_MAXSLOT / 4; ++p4)
-      if (p4 * 4 < nmine) sl_w[(p4 * 4 + j) * DR_NH + col] = wv[p4];
+      if (!WLDS && p4 * 4 < nmine) sl_w[(p4 * 4 + j) * DR_NH + col] = wv[p4];
   }
   __builtin_amdgcn_wave_barrier();
 
@@ -225,7 +229,10 @@ __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, c
         l += S[t][i];
       }
     l = rows_sum(l);
-    const float wr = (col < G) ? bf2f(sl_w[sl_id[si] * DR_NH + col]) : 0.f;
+    float wr = 0.f;
+    if (col < G)
+      wr = bf2f(WLDS ? weights[(bt * dm.HQ + hk * G + col) * (long)dm.NW + s_begin + wave + sl_id[si] * NWAVE]
+                     : sl_w[sl_id[si] * DR_NH + col]);
     const float f = (l > 0.f) ? wr / l : 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -282,7 +289,9 @@ __device__ __forceinline__ void decode_rows_body(const bf16_t* __restrict__ q, c
 #pragma unroll
     for (int w2 = 0; w2 < NWAVE; ++w2) x += o_s[((size_t)w2 * G + g) * D + dv];
     if (dm.nsplit == 1) o[(bt * dm.HQ + hk * G + g) * (long)D + dv] = f2bf(x);
-    else partial[((bt * dm.HQ + hk * G + g) * (long)dm.nsplit + split) * D + dv] = x;
+    else  // (through to memory: another workgroup of the same launch may be the one to add the shares up)
+      __hip_atomic_store(&partial[((bt * dm.HQ + hk * G + g) * (long)dm.nsplit + split) * D + dv], x, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 

@@ -665,10 +665,6 @@ Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v,
   // chunks per query.  Repacking moves 8 bytes per cache element at about 5 TB/s, the one-launch kernel 256 * topk
   // bytes per query and feature pair at about 7.5 TB/s, which meet near L = Lkv / (20 * topk).
   bool two_calls = L >= 64 && 16 * L * topk >= Lkv;
-  // Few rows with a key per query head on a long cache: a row's workgroup would stream its keys at about 40 GB/s
-  // while the rest of the chip idles (2 MiB a row: 82 us against 66 at two rows, 83 against 88 at sixteen);
-  // topk_use_row has the same line.
-  two_calls = two_calls || (per_qhead && B * L * hkv < 16 && 2 * N * G * D > (3 << 19));
   two_calls = two_calls || Lkv < N * block ||
               !hils_decode_step_covers(i32(B), i32(L), i32(N), i32(hq), i32(hkv), i32(D), i32(topk), i32(block),
                                        (int)pb.defined());
@@ -693,10 +689,12 @@ Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v,
     lse_total = new_tensor({B, L, hkv, G}, q, at::kFloat);
     sel = at::full({B, L, hkv, G, N}, -INFINITY, q.options().dtype(at::kFloat));
   }
-  HILS_CALL(hils_decode_step, cptr(qc), cptr(lm), cptr(kc), cptr(vc), fptr(lse), fptr(pb), miptr(idx), mptr(sc), mptr(w),
+  const Tensor ws = workspace(hils_decode_step_workspace(i32(B), i32(L), i32(N), i32(hq), i32(hkv), i32(D), i32(topk),
+                                                         per_qhead, 0), q);
+  HILS_CALL(hils_decode_step_ws, cptr(qc), cptr(lm), cptr(kc), cptr(vc), fptr(lse), fptr(pb), miptr(idx), mptr(sc), mptr(w),
             mptr(o), mfptr(lse_total), mfptr(sel), i32(B), i32(L), i32(Lkv), i32(N), i32(hq), i32(hkv), i32(D),
             i32(topk), i32(block), i32(window), i32(q_offset), (float)scale, (float)scale, (int)mask_last,
-            (int)head_major, i32(cap), per_qhead);
+            (int)head_major, i32(cap), per_qhead, mptr(ws), bytes(ws));
   if (!debug.is_none()) {
     debug["lse_total"] = lse_total;
     debug["sel_logits"] = sel;
@@ -764,10 +762,11 @@ std::tuple<Tensor, Tensor, Tensor> paged_step(const Tensor& q, const Tensor& k_p
   }
   Tensor o = new_tensor({B, Lq, HQ, D}, q, q.scalar_type());
   if (one) {  // selection and attention of a row by one workgroup, one launch
-    HILS_CALL(hils_decode_step_paged, cptr(qc), cptr(lmk), cptr(kp), cptr(vp), iptr(table), fptr(lse), fptr(bias),
+    const Tensor ws = workspace(hils_decode_step_workspace(b, lq, n, hq, h, d, tk, per_qhead, (int)!dense), q);
+    HILS_CALL(hils_decode_step_paged_ws, cptr(qc), cptr(lmk), cptr(kp), cptr(vp), iptr(table), fptr(lse), fptr(bias),
               miptr(idx), mptr(sc), mptr(w), mptr(o), mfptr(lse_total), mfptr(sel), b, lq, n, hq, h, d, tk, 64,
               i32(window), off, i32(max_pages), i32(pages), scale, scale, 1, (int)dense, (int)dense, i32(cap),
-              per_qhead);
+              per_qhead, mptr(ws), bytes(ws));
   } else if (dense) {
     // shapes outside the one-launch kernel: selection and softmax on the reference's dense layout, attention on the pages
     const Tensor lm = lmk.slice(2, 0, N).permute({0, 2, 1, 3}).contiguous();

@@ -10,7 +10,7 @@ sparse_attn_decode_rows_kernel(const bf16_t* __restrict__ q, const bf16_t* __res
                                float* __restrict__ partial, DrDims dm) {
   extern __shared__ __align__(16) char dr_dyn[];
   decode_rows_body<D, NWAVE>(q, k, v, weights, indices, o, partial, dm, dr_dyn, (int)blockIdx.x, (int)blockIdx.y,
-                             (long)blockIdx.z);
+                             (long)blockIdx.z, dr_dyn + dr_work_bytes(D, dm.G, NWAVE));
 }
 
 // A workgroup of 8 (no split) or 4 wavefronts, DR_MAXSLOT slots per wavefront: K <= 128 covers

@@ -880,7 +880,7 @@ extern "C" int hils_swa_fwd_strided(const void* q, const void* k, const void* v,
   hipStream_t st = (hipStream_t)stream;
   const bf16_t *qq = (const bf16_t*)q, *kk = (const bf16_t*)k, *vv = (const bf16_t*)v;
   int rc;
-  if (hils_swa_rows_better(B, dm)) rc = hils_swa_fwd_rows(B, st, q, k, v, o, lse, D, Dv, dm);
+  if (hils_swa_rows_better(B, D, Dv, dm)) rc = hils_swa_fwd_rows(B, st, q, k, v, o, lse, D, Dv, dm);
   else if (D == 64 && Dv == 64) rc = swa_launch_g<64, 64>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   else if (D == 128 && Dv == 128) rc = swa_launch_g<128, 128>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);
   else if (D == 64) rc = swa_launch_g<64, 128>(G, B, st, qq, kk, vv, (bf16_t*)o, lse, dm);

@@ -9,7 +9,7 @@ struct SwaDims {
   long k_batch, v_batch;  // elements from a sequence's keys / values to the next one's
 };
 
-#define SWA_ROWS_MAX 4096
-bool hils_swa_rows_better(int B, const SwaDims& dm);
+// Is the row kernel the faster one for this shape?
+bool hils_swa_rows_better(int B, int D, int Dv, const SwaDims& dm);
 int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int D,
                       int Dv, const SwaDims& dm);

@@ -218,10 +218,14 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   }
 }
 
-// Score rows the tile kernel would spread over too few workgroups.
-bool hils_swa_rows_better(int B, const SwaDims& dm) {
-  const long rows = (long)B * dm.Lq * dm.HQ;
-  return rows <= SWA_ROWS_MAX;
+// While the row kernel's workgroups fit two rounds of the chip it is ahead of the tile kernel, whose few
+// workgroups walk the window in series (window 512, row / tile kernel: heads of 64 7 / 19 us with one
+// workgroup, 8 / 25 us at 256, 12 / 25 at 512, 20 / 25 at 1024, 36 / 26 at 2048; heads of 128 10 / 24,
+// 12 / 31, 22 / 32, 41 / 32).  Window 64: 7 / 9 up to 512 workgroups, about even at 1024 with heads of 64.
+bool hils_swa_rows_better(int B, int D, int Dv, const SwaDims& dm) {
+  const int QB = 16 / (dm.HQ / dm.H);
+  const long wgs = (long)((dm.Lq + QB - 1) / QB) * dm.H * B;
+  return wgs <= 512 || (wgs <= 1024 && D <= 64 && Dv <= 64 && dm.window >= 256);
 }
 
 int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int D,

@@ -1393,18 +1393,24 @@ struct TopkRowSharedT {
   int rank[64];                            // one-launch decode step: candidates ahead of each candidate
   int win_i[TOPK_MAXK];                    // ... the winners' chunks, ascending, -1 padded
   bf16_t win_w[GM * (TOPK_MAXK + 1) + 2];   // ... and the heads' inter-chunk weights, [head][topk + 1]
+  float swa[GM];               // ... and the heads' local-branch log-sum-exp
   uint32_t thr;                // the candidate bound
   int next_group;
+};
+struct TopkWinners {
+  int widx, nc;  // lane kk (kk < nc) of every wavefront: chunk of winner kk
 };
 #define TOPK_R_CAND 256  // candidates the single-wavefront final selection takes
 
 // One (query, KV head) row (row = (b*L + t)*h_kv + hk) by a workgroup of NW wavefronts; dyn = the
 // workgroup's dynamic LDS (topk_row_smem bytes).
-// FUSED (the one-launch decode step): the row's attention follows in the same workgroup.  Every
-// wavefront then works out the winners itself and leaves the row's indices and inter-chunk weights in
-// LDS (sh.win_i, sh.win_w: the same values from every wavefront), where the attention reads them
-// without waiting for anybody; wavefront 0 writes the selection's global outputs on the way.
-template <int D, int GMAX, int NW, bool PAGED, bool FUSED = false, int GI = 8>  // GI: load instructions per register buffer
+// FUSED (the decode step): the row's attention follows in the same workgroup.  Every wavefront works out
+// the winners itself, leaves them in sh.win_i and in *win, and goes on to load the chunks it has to attend
+// over; the weights (topk_step_weights) are worked out under those loads.  write_out: this workgroup
+// writes the selection's debugging outputs (one of a row's workgroups does).
+// PRE: the logits and the key groups' partial sums come from decode_logits_kernel (pre_logits: the row's
+// [GMAX][NP], pre_m / pre_l: the row's [key group][GMAX]) instead of phase 1.
+template <int D, int GMAX, int NW, bool PAGED, bool FUSED = false, int GI = 8, bool PRE = false>  // GI: load instructions per register buffer
 __device__ __forceinline__ void
 topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
               const float* __restrict__ lse_swa, const float* __restrict__ bias, int32_t* __restrict__ indices,
@@ -1413,7 +1419,9 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
               int NP, int h_kv, int G, int topk, int block_size, int window_size, int causal, int q_offset,
               float sm_scale, const int32_t* __restrict__ page_table, int max_pages, int num_pages,
               int lmk_hm, int lmk_cap, int perq, int bias_inplace, float* dyn, const long row,
-              TopkRowSharedT<GMAX>* sh_p = nullptr) {
+              TopkRowSharedT<GMAX>* sh_p = nullptr, const float* __restrict__ pre_logits = nullptr,
+              const float* __restrict__ pre_m = nullptr, const float* __restrict__ pre_l = nullptr,
+              const bool write_out = true, TopkWinners* win = nullptr) {
   // bias_inplace (with a bias only): the staged bias and the logits share one array, a slot holding the
   // bias until the chunk's logit is added to it; a winner's bias is then read again from global memory
   // and its raw score is the biased logit minus that bias (one rounding of the sum away from the raw
@@ -1449,7 +1457,13 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   float swa[GMAX];
 #pragma unroll
   for (int g = 0; g < GMAX; ++g) swa[g] = (g < G) ? lse_swa[row * G + g] : 0.f;
-  if (tid == 0) sh.next_group = 2 * NW;
+  if (tid == 0) {
+    sh.next_group = 2 * NW;
+    if (FUSED) {
+#pragma unroll
+      for (int g = 0; g < GMAX; ++g) sh.swa[g] = swa[g];
+    }
+  }
   if (bias) {
     // chunk c of this row: the G biases are contiguous in all three layouts
     for (int c = tid; c < NP; c += THREADS) {
@@ -1466,14 +1480,45 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
         } else {
           e0 = ((b * N + c) * (long)h_kv + hk) * G;
         }
+        if (G == GMAX) {  // whole 16-byte pieces
 #pragma unroll
-        for (int g = 0; g < GMAX; ++g)
-          if (g < G) bv[g] = bias[e0 + g];
+          for (int g = 0; g < GMAX; g += 4) {
+            const f32x4_t b4 = *(const f32x4_t*)&bias[e0 + g];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bv[g + i] = b4[i];
+          }
+        } else {
+#pragma unroll
+          for (int g = 0; g < GMAX; ++g)
+            if (g < G) bv[g] = bias[e0 + g];
+        }
       }
 #pragma unroll
       for (int g = 0; g < GMAX; ++g) bias_s[g * NP + c] = bv[g];
     }
   }
+  if constexpr (PRE) {
+    if (inplace) __syncthreads();  // the bias is in the logits' places
+    const int ngroups = (lim + KG - 1) / KG;
+    const int q4 = (lim + 3) / 4;
+    for (int i = tid; i < GMAX * q4; i += THREADS) {
+      const int g = i / q4, c = (i - g * q4) * 4;
+      f32x4_t x = {HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF};
+      if (g < G) {
+        x = *(const f32x4_t*)&pre_logits[g * NP + c];
+        if (inplace) {
+          const f32x4_t bb = *(const f32x4_t*)&bias_s[g * NP + c];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = __fadd_rn(x[e], bb[e]);
+        }
+      }
+      *(f32x4_t*)&logit_s[g * NP + c] = x;
+    }
+    for (int i = tid; i < ngroups * GMAX; i += THREADS) {
+      sh.grp_m[i / GMAX][i % GMAX] = pre_m[i];
+      sh.grp_l[i / GMAX][i % GMAX] = pre_l[i];
+    }
+  } else {
   // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
   // features ks*32 + 8j ..; loaded here so that the barrier below has waited for them
   typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
@@ -1618,6 +1663,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       fetch(kb, gb < last ? gb : last);
     }
   }
+  }
   __syncthreads();
 
   // ---- phase 2: LSE per head from the key groups' partial sums.  Work every wavefront would do
@@ -1645,7 +1691,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     const float t = (lo == HILS_NEG_INF) ? hi : hi + __logf(1.f + __expf(lo - hi));
     if (lane == 0) {
       sh.tot[g] = t;
-      if (lse_total_out && g < G) lse_total_out[row * G + g] = t;
+      if (lse_total_out && write_out && g < G) lse_total_out[row * G + g] = t;
     }
   }
   __syncthreads();
@@ -1682,7 +1728,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     }
   };
   if (bias && !inplace) form_keys(std::true_type{}); else form_keys(std::false_type{});
-  if (sel_logits_out) {  // the exported selection logits (a debugging output)
+  if (sel_logits_out && write_out) {  // the exported selection logits (a debugging output)
     for (int i = tid; i < G * N; i += THREADS) {
       const int g = i / N, c = i - g * N;
       float xv = c < lim ? logit_s[g * NP + c] : HILS_NEG_INF;
@@ -1754,58 +1800,11 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     }
     return bias[e0 + g];
   };
-  // ---- FUSED: what every wavefront does once lane kk (kk < nc) holds winner kk's chunk (ascending) ----
-  auto fused_tail = [&](int widx, int nc) __attribute__((always_inline)) {
-    const bool has = lane < nc;
-    float xs[GMAX], wgt[GMAX], wloc[GMAX], bws[GMAX];
-    // (the winner's biases first, all heads' loads in flight together: read from global memory when the
-    // bias shares the logits' array)
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g) bws[g] = (bias && has && g < G) ? bias_at(widx, g) : 0.f;
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-      xs[g] = (has && g < G) ? logit_s[g * NP + widx] : HILS_NEG_INF;  // raw scaled score
-      const float bw = bws[g];
-      if (inplace && has && g < G) xs[g] = __fsub_rn(xs[g], bw);
-      // the layer's inter-chunk softmax over [scores as bf16 (+ bias as bf16, summed in bf16), lse_swa]
-      float x = HILS_NEG_INF;
-      if (has && g < G) {
-        x = bf2f(f2bf(xs[g]));
-        if (bias) x = bf2f(f2bf(x + bf2f(f2bf(bw))));
-      }
-      const float m = fmaxf(wave_max_f(x), swa[g]);
-      if (m == HILS_NEG_INF) {  // every logit -inf: NaN row, as a softmax gives
-        wgt[g] = wloc[g] = __uint_as_float(0x7fc00000u);
-      } else {
-        const float e = (x == HILS_NEG_INF) ? 0.f : __expf(x - m);
-        const float el = __expf(swa[g] - m);
-        const float inv = 1.f / (wave_sum_f(e) + el);
-        wgt[g] = e * inv;
-        wloc[g] = el * inv;
-      }
-    }
-    if (wave == 0) {  // the selection's outputs
-      if (lane < topk) indices[row * topk + lane] = has ? widx : -1;
-#pragma unroll
-      for (int g = 0; g < GMAX; ++g)
-        if (g < G) {
-          if (lane < topk) scores[(row * G + g) * (long)topk + lane] = f2bf(xs[g]);
-          if (weights_out) {
-            bf16_t* wrow = weights_out + (row * G + g) * (long)(topk + 1);
-            if (lane < topk) wrow[lane] = f2bf(wgt[g]);
-            if (lane == 0) wrow[topk] = f2bf(wloc[g]);
-          }
-        }
-    }
-    // the row's indices and weights for the attention, in the layout of the global tensors
-    if (lane < topk) sh.win_i[lane] = has ? widx : -1;
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g)
-      if (g < G) {
-        if (lane < topk) sh.win_w[g * (topk + 1) + lane] = f2bf(wgt[g]);
-        if (lane == 0) sh.win_w[g * (topk + 1) + topk] = f2bf(wloc[g]);
-      }
+  // FUSED: lane kk (kk < nc) of every wavefront holds winner kk's chunk (ascending)
+  auto fused_winners = [&](int widx, int nc) __attribute__((always_inline)) {
+    if (lane < topk) sh.win_i[lane] = lane < nc ? widx : -1;  // (the same values from every wavefront)
     __builtin_amdgcn_wave_barrier();
+    *win = {widx, nc};
   };
   if (cand_total <= TOPK_R_CAND) {
     uint32_t* ck = (uint32_t*)sh.merge_s;  // NW * TOPK_MAXK >= 512 entries
@@ -1851,7 +1850,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
         if (win) sh.cand_i[wave][__popcll(wm & lt)] = ci;
         __builtin_amdgcn_wave_barrier();
         const int nc = __popcll(wm);
-        fused_tail(lane < nc ? sh.cand_i[wave][lane] : -1, nc);
+        fused_winners(lane < nc ? sh.cand_i[wave][lane] : -1, nc);
         return;
       }
     }
@@ -1893,7 +1892,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   __syncthreads();
   if constexpr (FUSED) {  // the selections that did not fit one lane per candidate: winners from LDS
     const int nc = sh.ncand[0];
-    fused_tail(lane < nc ? sh.cand_i[0][lane] : -1, nc);
+    fused_winners(lane < nc ? sh.cand_i[0][lane] : -1, nc);
     return;
   }
   // ---- phase 4: indices (ascending) and the raw scaled scores of the winners ----
@@ -1966,11 +1965,100 @@ struct DsArgs {
   float sm_scale_sel;
   const int32_t* page_table;
   int max_pages, num_pages, lmk_hm, lmk_cap, perq, bias_inplace;
+  // the step over several workgroups per row (decode_logits_kernel, decode_attend_kernel)
+  float *pre_logits, *pre_m, *pre_l, *partial;
+  int* arrived;    // [row] workgroups that have left their partial outputs
+  int pre_groups;  // key groups of a row
+  int slot_off;    // bytes of LDS before the attention's slot lists: past the selection's and the attention's other arrays
   int stagger_ticks;  // 100 MHz ticks by which every other row of an XCD starts late (0: none)
   DrDims dr;
 };
+// Wavefront g works out head g's inter-chunk weights (all heads in every wavefront took 5 us with eight of
+// them) and leaves them in sh.win_w in the layout of the global tensor; write_out: the selection's global
+// outputs are written on the way.  dyn: the LDS of topk_row_body, which still holds logits and bias.
+template <int D, int GMAX, bool PAGED>
+__device__ __forceinline__ void topk_step_weights(const DsArgs& a, TopkRowSharedT<GMAX>& sh, const float* dyn,
+                                                  const long row, const TopkWinners& win, const bool write_out) {
+  static_assert(DS_WAVES >= GMAX, "one wavefront per head");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int G = a.G, NP = a.NP, topk = a.topk, widx = win.widx;
+  const bool has = lane < win.nc;
+  if (wave == DS_WAVES - 1 && write_out && lane < topk) a.indices[row * topk + lane] = has ? widx : -1;
+  if (wave >= G) return;
+  const int g = wave, hk = (int)(row % a.h_kv);
+  const long b = row / a.h_kv / a.L;
+  const float* logit_s = dyn;
+  const int* page_s = (const int*)(dyn + (size_t)(GMAX + 1) * NP);
+  float bw = 0.f;
+  if (a.bias && has) {
+    if (!a.bias_inplace) {
+      bw = ((const float*)page_s)[(PAGED ? NP : 0) + g * NP + widx];
+    } else {  // the staged bias has become the biased logit: read it again
+      long e0;
+      if (PAGED) {
+        const int pg = page_s[widx];
+        e0 = ((long)(pg < 0 ? 0 : pg) * a.h_kv + hk) * G;
+      } else if (a.lmk_hm) {
+        e0 = ((b * a.h_kv + hk) * (long)a.lmk_cap + widx) * G;
+      } else {
+        e0 = ((b * a.N + widx) * (long)a.h_kv + hk) * G;
+      }
+      bw = a.bias[e0 + g];
+    }
+  }
+  float xs = has ? logit_s[g * NP + widx] : HILS_NEG_INF;  // raw scaled score
+  if (a.bias && a.bias_inplace && has) xs = __fsub_rn(xs, bw);
+  // the layer's inter-chunk softmax over [scores as bf16 (+ bias as bf16, summed in bf16), lse_swa]
+  float x = HILS_NEG_INF;
+  if (has) {
+    x = bf2f(f2bf(xs));
+    if (a.bias) x = bf2f(f2bf(x + bf2f(f2bf(bw))));
+  }
+  const float swg = sh.swa[g];
+  const float m = fmaxf(wave_max_f(x), swg);
+  float wgt, wloc;
+  if (m == HILS_NEG_INF) {  // every logit -inf: NaN row, as a softmax gives
+    wgt = wloc = __uint_as_float(0x7fc00000u);
+  } else {
+    const float e = (x == HILS_NEG_INF) ? 0.f : __expf(x - m);
+    const float el = __expf(swg - m);
+    const float inv = 1.f / (wave_sum_f(e) + el);
+    wgt = e * inv;
+    wloc = el * inv;
+  }
+  if (lane < topk) sh.win_w[g * (topk + 1) + lane] = f2bf(wgt);
+  if (lane == 0) sh.win_w[g * (topk + 1) + topk] = f2bf(wloc);
+  if (write_out) {
+    bf16_t* wrow = a.weights + (row * G + g) * (long)(topk + 1);
+    if (lane < topk) {
+      a.scores[(row * G + g) * (long)topk + lane] = f2bf(xs);
+      wrow[lane] = f2bf(wgt);
+    }
+    if (lane == 0) wrow[topk] = f2bf(wloc);
+  }
+}
+
 // PAGED: the chunk keys (and the bias) are addressed through the page table; the attention reads
 // K and V through it whenever a.dr.page_table is set.
+// The attention reads the row's indices and weights where the selection leaves them in LDS: the pointers are
+// offset so that the row's entries of the (B, L, heads, ...) tensors fall there.  Its staging areas lie over
+// the selection's logits: in every wavefront, once its first chunk's loads are in flight, the weights are
+// worked out and the barrier runs that separates the two uses.
+template <int D, bool PAGED, int GMAX>
+__device__ __forceinline__ void decode_step_attend(const DsArgs& a, TopkRowSharedT<GMAX>& sh, float* dyn,
+                                                   const long row, const TopkWinners& win, int split,
+                                                   const bool write_out) {
+  const int hk = (int)(row % a.h_kv);
+  const long bt = row / a.h_kv;
+  const bf16_t* w_row = sh.win_w - (bt * a.dr.HQ + hk * a.G) * (long)a.dr.NW;
+  const int32_t* i_row = sh.win_i - (bt * a.dr.H + hk) * (long)a.dr.K;
+  decode_rows_body<D, DS_WAVES, true>(a.q, a.k, a.v, w_row, i_row, a.o, a.partial, a.dr, (char*)dyn, split, hk, bt,
+                                      (char*)dyn + a.slot_off, [&]() __attribute__((always_inline)) {
+                                        topk_step_weights<D, GMAX, PAGED>(a, sh, dyn, row, win, write_out);
+                                        lds_barrier();  // (no wait for the loads in flight)
+                                      });
+}
+
 template <int D, bool PAGED, int GMAX>
 __global__ void __launch_bounds__(DS_WAVES * 64) decode_step_kernel(DsArgs a) {
   extern __shared__ __align__(16) float ds_dyn[];
@@ -1979,27 +2067,162 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_step_kernel(DsArgs a) {
   // With at most one row per compute unit all rows run in step: every compute unit streams keys, then
   // every one sits in the selection's tail with the memory system idle, then every one streams K and V.
   // Half of the rows (every other one of an XCD's) start a little late, so that one half's tail falls
-  // into the other half's streaming (75.5 -> 72.2 us at 256 rows of 2048 keys with 8 us; 5 us: 75.0,
-  // 12 us: 74.2; thirds or a continuous spread of the start times did less).
+  // into the other half's streaming (256 rows of 2048 keys and 32 chunks at D = 128: 79 us without, 72.0 with
+  // 3 us, 70.2 with 6, 70.4 with 8; 1024 keys: 62.4, 57.5, 57.7, 59.6).
   if (a.stagger_ticks > 0 && ((blockIdx.x >> 3) & 1)) {
     const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
     while (__builtin_amdgcn_s_memrealtime() - t0 < (unsigned long long)a.stagger_ticks) __builtin_amdgcn_s_sleep(8);
   }
+  TopkWinners win;
   topk_row_body<D, GMAX, DS_WAVES, PAGED, true>(a.q, a.lmks, a.lse_swa, a.bias, a.indices, a.scores, a.lse_total,
                                              a.sel_logits, a.weights, a.L, a.N, a.NP, a.h_kv, a.G, a.topk,
                                              a.block_size, a.window_size, 1, a.q_offset, a.sm_scale_sel,
                                              a.page_table, a.max_pages, a.num_pages, a.lmk_hm, a.lmk_cap, a.perq,
-                                             a.bias_inplace, ds_dyn, row, &ds_sh);
-  // The attention reads the row's indices and weights where the selection left them in LDS: the
-  // pointers are offset so that the row's entries of the (B, L, heads, ...) tensors fall there.  Its
-  // staging areas lie over the selection's logits: the barrier that separates the two uses runs in
-  // every wavefront once its first chunk's loads are in flight.
+                                             a.bias_inplace, ds_dyn, row, &ds_sh, nullptr, nullptr, nullptr, true, &win);
+  decode_step_attend<D, PAGED, GMAX>(a, ds_sh, ds_dyn, row, win, 0, true);
+}
+
+// ---- the decode step over several workgroups per row ------------------------------------------------
+// A compute unit streams 30 to 40 GB/s whatever the others do (its loads in flight over the latency of
+// memory), so with few rows the one-launch step leaves the chip idle: 16 rows of 468 chunks with a key per
+// query head (480 KB a row) 16 us of logits and 10 us of attention, 64 rows of 1563 chunks at D = 128 13 us
+// and 28 us.  Here the logits come from a first kernel, one wavefront per group of keys, and in a second
+// one `nsplit` workgroups of a row each repeat the selection on those logits (a few microseconds that cost
+// nothing while compute units are idle), attend over their share of the selected chunks and leave partial
+// outputs; the last of them to arrive adds these up in a fixed order (no workgroup ever waits for another).
+
+// One wavefront per group of KG keys: raw scaled logits of the visible chunks and the group's (max, sum of
+// exponentials) per head, as phase 1 of topk_row_body forms them.
+template <int D, int GMAX>
+__global__ void __launch_bounds__(256) decode_logits_kernel(DsArgs a) {
+  constexpr int LR = D / 8, TPI = 64 / LR, GI = 8, KG = GI * TPI, KS = D / 32, ROWB = 2 * D + 16, LPT = 16 / TPI;
+  __shared__ __align__(16) char stage_s[4][16 * ROWB];
+  typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, j = lane >> 4, piece = lane % LR, tsub = lane / LR;
+  const long row = blockIdx.y;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.arrived[row] = 0;
   const int hk = (int)(row % a.h_kv);
-  const long bt = row / a.h_kv;
-  const bf16_t* w_row = ds_sh.win_w - (bt * a.dr.HQ + hk * a.G) * (long)a.dr.NW;
-  const int32_t* i_row = ds_sh.win_i - (bt * a.dr.H + hk) * (long)a.dr.K;
-  decode_rows_body<D, DS_WAVES>(a.q, a.k, a.v, w_row, i_row, a.o, nullptr, a.dr, (char*)ds_dyn, 0, hk, bt,
-                                [] __device__() { lds_barrier(); });  // (no wait for the loads in flight)
+  const long bt = row / a.h_kv, b = bt / a.L;
+  const int t = (int)(bt % a.L), G = a.G, N = a.N, NP = a.NP;
+  int lim = visible_limit(t + a.q_offset, a.window_size, a.block_size);
+  lim = lim < 0 ? 0 : (lim > N ? N : lim);
+  const int GK = a.perq ? G : 1, h_lmk = a.h_kv * GK;
+  const int vg = blockIdx.x * 4 + wave;
+  if (vg >= ((lim + KG - 1) / KG) * GK) return;
+  const int grp = vg / GK, gh = a.perq ? vg - grp * GK : -1;
+  bf16x8_t qb[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    tr_u4 x = {0u, 0u, 0u, 0u};
+    if (col < G) x = *(const tr_u4*)(a.q + (row * (long)G + col) * D + ks * 32 + j * 8);
+    qb[ks] = __builtin_bit_cast(bf16x8_t, x);
+  }
+  const long cstride = a.lmk_hm ? (long)D : (long)h_lmk * D;
+  const bf16_t* base = a.lmks + piece * 8 +
+                       (a.lmk_hm ? (b * h_lmk + hk * GK + (gh > 0 ? gh : 0)) * (long)a.lmk_cap * D
+                                 : (b * N * (long)h_lmk + hk * GK + (gh > 0 ? gh : 0)) * D);
+  tr_u4 kr[GI];
+#pragma unroll
+  for (int it = 0; it < GI; ++it) {
+    int c = grp * KG + it * TPI + tsub;
+    c = c < N ? c : N - 1;
+    kr[it] = *(const tr_u4*)(base + c * cstride);
+  }
+  char* stage_w = stage_s[wave];
+  char* const w_addr = stage_w + tsub * ROWB + piece * 16;
+  const char* const k_addr = stage_w + col * ROWB + j * 16;
+  float* logits = a.pre_logits + row * (long)GMAX * NP;
+  const bool mine = col < G && (gh < 0 || col == gh);
+  float m_run = HILS_NEG_INF, l_run = 0.f;
+#pragma unroll
+  for (int tt = 0; tt < GI / LPT; ++tt) {
+    const int c0 = grp * KG + tt * 16 + 4 * j;
+    f32x4_t bb = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias && mine) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c0 + i < lim)
+          bb[i] = a.bias[(a.lmk_hm ? ((b * a.h_kv + hk) * (long)a.lmk_cap + c0 + i) : ((b * N + c0 + i) * (long)a.h_kv + hk)) * G + col];
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int ii = 0; ii < LPT; ++ii) *(tr_u4*)(w_addr + ii * TPI * ROWB) = kr[tt * LPT + ii];
+    __builtin_amdgcn_wave_barrier();
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const tr_u4 x = *(const tr_u4*)(k_addr + ks * 64);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x), qb[ks], acc, 0, 0, 0);
+    }
+    if (mine) {
+      f32x4_t out;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[i] = (c0 + i < lim) ? __fmul_rn(acc[i], a.sm_scale_sel) : HILS_NEG_INF;
+      *(f32x4_t*)&logits[col * NP + c0] = out;
+      if (a.bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = __fadd_rn(out[i], bb[i]);
+      }
+      const float mn = fmaxf(fmaxf(m_run, fmaxf(out[0], out[1])), fmaxf(out[2], out[3]));
+      const float ms = (mn == HILS_NEG_INF) ? 0.f : mn * HILS_LOG2E;
+      float add = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add += __builtin_amdgcn_exp2f(fmaf(out[i], HILS_LOG2E, -ms));
+      l_run = fmaf(l_run, __builtin_amdgcn_exp2f(fmaf(m_run, HILS_LOG2E, -ms)), add);
+      m_run = mn;
+    }
+  }
+  const float M = rows_max(m_run);
+  const float Ms = (M == HILS_NEG_INF) ? 0.f : M * HILS_LOG2E;
+  const float Lg = rows_sum(l_run * __builtin_amdgcn_exp2f(fmaf(m_run, HILS_LOG2E, -Ms)));
+  // (the entries of the heads past G are read as (-inf, 0))
+  const bool past = col >= G && col < GMAX && (gh < 0 || gh == G - 1);
+  if (j == 0 && (mine || past)) {
+    const long e = (row * a.pre_groups + grp) * GMAX + col;
+    a.pre_m[e] = mine ? M : HILS_NEG_INF;
+    a.pre_l[e] = mine ? Lg : 0.f;
+  }
+}
+
+// grid: nsplit shares of every row, a row's shares a whole number of rows apart
+template <int D, int GMAX>
+__global__ void __launch_bounds__(DS_WAVES * 64) decode_attend_kernel(DsArgs a, long rows) {
+  extern __shared__ __align__(16) float da_dyn[];
+  __shared__ TopkRowSharedT<GMAX> ds_sh;
+  __shared__ int last_s;
+  const long row = blockIdx.x % rows;
+  const int split = (int)(blockIdx.x / rows);
+  TopkWinners win;
+  topk_row_body<D, GMAX, DS_WAVES, false, true, 8, true>(
+      a.q, a.lmks, a.lse_swa, a.bias, a.indices, a.scores, a.lse_total, a.sel_logits, a.weights, a.L, a.N, a.NP, a.h_kv,
+      a.G, a.topk, a.block_size, a.window_size, 1, a.q_offset, a.sm_scale_sel, nullptr, 0, 0, a.lmk_hm, a.lmk_cap,
+      a.perq, a.bias_inplace, da_dyn, row, &ds_sh, a.pre_logits + row * (long)GMAX * a.NP,
+      a.pre_m + row * a.pre_groups * (long)GMAX, a.pre_l + row * a.pre_groups * (long)GMAX, split == 0, &win);
+  decode_step_attend<D, false, GMAX>(a, ds_sh, da_dyn, row, win, split, split == 0);
+  if (a.dr.nsplit == 1) return;
+  // The partial outputs were written through to memory (agent-scope atomic stores): once every wavefront's
+  // are acknowledged, the workgroup says that it has arrived.  (A device-wide fence here writes the whole
+  // L2 back, once per wavefront: 0.2 us for every workgroup of the launch, one after the other.)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) last_s = atomicAdd(&a.arrived[row], 1) == a.dr.nsplit - 1;
+  __syncthreads();
+  if (!last_s) return;
+  float* p = a.partial + row * a.G * (long)a.dr.nsplit * D;
+  for (int i = threadIdx.x; i < a.G * (D / 4); i += DS_WAVES * 64) {
+    const int g = i / (D / 4), d4 = i % (D / 4);
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    for (int sp = 0; sp < a.dr.nsplit; ++sp) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[e] += __hip_atomic_load(&p[(g * (long)a.dr.nsplit + sp) * D + d4 * 4 + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    uint2 pk;
+    pk.x = pack_bf2(x[0], x[1]);
+    pk.y = pack_bf2(x[2], x[3]);
+    *(uint2*)(a.o + (row * a.G + g) * (long)D + d4 * 4) = pk;
+  }
 }
 
 static int topk_cus() { return hils_device_cus(); }
@@ -2109,14 +2332,43 @@ extern "C" int hils_decode_step_covers(int B, int L, int N, int HQ, int H, int D
   return topk_use_row((long)B * L * H, N, G, D, 0, true, with_bias != 0, true) && hils_decode_rows_covers(D, D, G, topk) ? 1 : 0;
 }
 
+// Workgroups per row of the decode step, 1: the one-launch kernel.  The second launch, the repeated selection and
+// the final sum cost about 6 us, what a workgroup streams of the row's keys and selected chunks in 256 KB, and the
+// more rows there are the more of the chip one workgroup per row already uses (one launch / split, 4 rows of 468
+// keys of 128 and 32 chunks, 0.9 MB saved: 25 / 20 us; 64 rows of them: 28 / 27; 16 rows of 468 keys per query head,
+// 0.9 MB: 32 / 21; 64 rows of 468 shared keys of 64, 0.4 MB: 20 / 22; 2 rows of 128 keys and 8 chunks: 13 / 16).
+static int decode_step_nsplit(long rows, int N, int G, int D, int topk, int per_qhead, int lmk_paged) {
+  if (lmk_paged || rows > topk_cus() / 4) return 1;
+  long s = (topk + DS_WAVES - 1) / DS_WAVES;  // no fewer than a chunk per wavefront
+  if (s > topk_cus() / rows) s = topk_cus() / rows;
+  if (s < 2) s = 2;  // (short selections: the logits alone are worth the split)
+  const long keys = (long)N * (per_qhead ? G : 1) * D * 2, kv = (long)topk * DR_S * D * 4;
+  const long saved = keys + (kv - kv / s);
+  return saved >= (256 + 8 * rows) * 1024 ? (int)s : 1;
+}
+static size_t decode_step_ws_bytes(long rows, int nsplit, int N, int G, int D) {
+  const size_t gm = G <= 4 ? 4 : 8, NP = (N + 63) & ~63, groups = NP / (D == 64 ? 64 : 32);
+  return rows * (gm * NP + 2 * groups * gm + (size_t)G * nsplit * D + 1) * sizeof(float) + 64;
+}
+extern "C" size_t hils_decode_step_workspace(int B, int L, int N, int HQ, int H, int D, int topk, int lmk_per_qhead,
+                                             int lmk_paged) {
+  if (B <= 0 || L <= 0 || N <= 0 || H <= 0 || HQ <= 0 || topk <= 0) return 0;
+  const long rows = (long)B * L * H;
+  const int s = decode_step_nsplit(rows, N, HQ / H, D, topk, lmk_per_qhead, lmk_paged);
+  return s > 1 ? decode_step_ws_bytes(rows, s, N, HQ / H, D) : 0;
+}
+
 static int decode_step_launch(const void* q, const void* lmks, const void* k, const void* v, const float* lse_swa,
                               const float* bias, int lmk_paged, int lmk_hm, int lmk_cap, int perq, int32_t* indices, void* scores, void* weights, void* o, float* lse_total,
                               float* sel_logits, int B, int L, int Lkv, int N, int HQ, int H, int D, int topk,
                               int block_size, int window_size, int q_offset, float sm_scale_sel,
                               float sm_scale_attn, int mask_last, const int32_t* page_table, int max_pages,
-                              int num_pages, hipStream_t st) {
+                              int num_pages, void* workspace, size_t workspace_bytes, hipStream_t st) {
   const int G = HQ / H;
   const long rows = (long)B * L * H;
+  const int nsplit = workspace ? decode_step_nsplit(rows, N, G, D, topk, perq, lmk_paged) : 1;
+  HILS_REQUIRE(nsplit == 1 || workspace_bytes >= decode_step_ws_bytes(rows, nsplit, N, G, D),
+               "hils_decode_step: the workspace is too short (%zu bytes)", workspace_bytes);
   const int NP = (N + 63) & ~63;
   int bias_inplace = 0;
   const bool sel_fits = topk_row_fits(N, G, D, lmk_paged != 0, bias != nullptr, DS_WAVES, &bias_inplace);
@@ -2124,20 +2376,48 @@ static int decode_step_launch(const void* q, const void* lmks, const void* k, co
                        (size_t)DS_WAVES * 16 * (2 * D + 16);
   HILS_REQUIRE(sel_fits,
                "hils_decode_step: too many chunks (%d) for the logits (and the bias) of the row's heads in LDS", N);
-  const size_t att_b = dr_smem_bytes(D, G, DS_WAVES);
-  const size_t smem = sel_b > att_b ? sel_b : att_b;
+  const size_t att_b = dr_work_bytes(D, G, DS_WAVES);
+  const size_t slot_off = ((sel_b > att_b ? sel_b : att_b) + 15) & ~(size_t)15;
+  const size_t smem = slot_off + dr_list_bytes(DS_WAVES);
   DsArgs a;
+  a.slot_off = (int)slot_off;
   a.q = (const bf16_t*)q; a.lmks = (const bf16_t*)lmks; a.k = (const bf16_t*)k; a.v = (const bf16_t*)v;
   a.lse_swa = lse_swa; a.bias = bias; a.indices = indices;
   a.lmk_hm = lmk_hm; a.lmk_cap = lmk_cap; a.perq = perq; a.bias_inplace = bias_inplace;
-  a.stagger_ticks = rows <= topk_cus() && 4 * rows > 3 * topk_cus() ? 800 : 0;  // one full round of rows: they would run in step
+  a.stagger_ticks = rows <= topk_cus() && 4 * rows > 3 * topk_cus() ? 600 : 0;  // one full round of rows: they would run in step
   a.scores = (bf16_t*)scores; a.weights = (bf16_t*)weights; a.o = (bf16_t*)o;
   a.lse_total = lse_total; a.sel_logits = sel_logits;
   a.L = L; a.N = N; a.NP = NP; a.h_kv = H; a.G = G; a.topk = topk; a.block_size = block_size;
   a.window_size = window_size; a.q_offset = q_offset; a.sm_scale_sel = sm_scale_sel;
   a.page_table = page_table; a.max_pages = max_pages; a.num_pages = num_pages;
-  a.dr = DrDims{L, Lkv, HQ, H, G, topk, topk + 1, page_table ? max_pages : Lkv / DR_S, 1, mask_last,
+  a.dr = DrDims{L, Lkv, HQ, H, G, topk, topk + 1, page_table ? max_pages : Lkv / DR_S, nsplit, mask_last,
                 sm_scale_attn, page_table, max_pages, num_pages};
+  if (nsplit > 1) {
+    const int gm = G <= 4 ? 4 : 8;
+    a.stagger_ticks = 0;
+    a.pre_groups = NP / (D == 64 ? 64 : 32);
+    a.pre_logits = (float*)workspace;
+    a.pre_m = a.pre_logits + rows * gm * NP;
+    a.pre_l = a.pre_m + rows * (long)a.pre_groups * gm;
+    a.partial = a.pre_l + rows * (long)a.pre_groups * gm;
+    a.arrived = (int*)(a.partial + rows * (long)G * nsplit * D);
+    const unsigned wgs = (unsigned)((a.pre_groups * (perq ? G : 1) + 3) / 4);
+#define DS_SPLIT_CALL(D_, G_)                                                                          \
+  do {                                                                                                 \
+    auto kern = decode_attend_kernel<D_, G_>;                                                          \
+    static HilsLdsReserve reserved;                                                                    \
+    if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_decode_step")) return rc;  \
+    hipLaunchKernelGGL((decode_logits_kernel<D_, G_>), dim3(wgs, (unsigned)rows), dim3(256), 0, st, a); \
+    hipLaunchKernelGGL(kern, dim3((unsigned)(rows * nsplit)), dim3(DS_WAVES * 64), smem, st, a, rows);  \
+  } while (0)
+    if (D == 64) {
+      if (G <= 4) DS_SPLIT_CALL(64, 4); else DS_SPLIT_CALL(64, 8);
+    } else {
+      if (G <= 4) DS_SPLIT_CALL(128, 4); else DS_SPLIT_CALL(128, 8);
+    }
+#undef DS_SPLIT_CALL
+    return HILS_OK;
+  }
 #define DS_CALL_G(D_, P_, G_)                                                                      \
   do {                                                                                             \
     auto kern = decode_step_kernel<D_, P_, G_>;                                                    \
@@ -2159,12 +2439,13 @@ static int decode_step_launch(const void* q, const void* lmks, const void* k, co
   return HILS_OK;
 }
 
-extern "C" int hils_decode_step(const void* q, const void* lmks, const void* k, const void* v,
+extern "C" int hils_decode_step_ws(const void* q, const void* lmks, const void* k, const void* v,
                                 const float* lse_swa, const float* bias, int32_t* indices, void* scores,
                                 void* weights, void* o, float* lse_total, float* sel_logits, int B, int L, int Lkv,
                                 int N, int HQ, int H, int D, int topk, int block_size, int window_size,
                                 int q_offset, float sm_scale_sel, float sm_scale_attn, int mask_last,
-                                int lmk_head_major, int lmk_cap, int lmk_per_qhead, void* stream) {
+                                int lmk_head_major, int lmk_cap, int lmk_per_qhead, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
   HILS_REQUIRE(q && lmks && k && v && lse_swa && indices && scores && weights && o, "hils_decode_step: null pointer");
   HILS_REQUIRE(B > 0 && L > 0 && N > 0 && H > 0 && HQ > 0 && HQ % H == 0, "hils_decode_step: bad sizes");
   HILS_REQUIRE(!lmk_head_major || lmk_cap >= N, "hils_decode_step: lmk_cap (%d) must be at least N (%d)", lmk_cap, N);
@@ -2174,21 +2455,32 @@ extern "C" int hils_decode_step(const void* q, const void* lmks, const void* k, 
   HILS_REQUIRE((long)B * L * H <= 2147483647L, "hils_decode_step: grid too large");
   if (int rc = decode_step_launch(q, lmks, k, v, lse_swa, bias, 0, lmk_head_major, lmk_cap, lmk_per_qhead, indices, scores, weights, o,
                                   lse_total, sel_logits, B, L, Lkv, N, HQ, H, D, topk, block_size, window_size,
-                                  q_offset, sm_scale_sel, sm_scale_attn, mask_last, nullptr, 0, 0,
-                                  (hipStream_t)stream))
+                                  q_offset, sm_scale_sel, sm_scale_attn, mask_last, nullptr, 0, 0, workspace,
+                                  workspace_bytes, (hipStream_t)stream))
     return rc;
   HILS_CHECK_LAUNCH("hils_decode_step");
   return HILS_OK;
 }
 
-extern "C" int hils_decode_step_paged(const void* q, const void* lmk_pages, const void* k_pages,
+extern "C" int hils_decode_step(const void* q, const void* lmks, const void* k, const void* v,
+                                const float* lse_swa, const float* bias, int32_t* indices, void* scores,
+                                void* weights, void* o, float* lse_total, float* sel_logits, int B, int L, int Lkv,
+                                int N, int HQ, int H, int D, int topk, int block_size, int window_size,
+                                int q_offset, float sm_scale_sel, float sm_scale_attn, int mask_last,
+                                int lmk_head_major, int lmk_cap, int lmk_per_qhead, void* stream) {
+  return hils_decode_step_ws(q, lmks, k, v, lse_swa, bias, indices, scores, weights, o, lse_total, sel_logits, B, L,
+                             Lkv, N, HQ, H, D, topk, block_size, window_size, q_offset, sm_scale_sel, sm_scale_attn,
+                             mask_last, lmk_head_major, lmk_cap, lmk_per_qhead, nullptr, 0, stream);
+}
+
+extern "C" int hils_decode_step_paged_ws(const void* q, const void* lmk_pages, const void* k_pages,
                                       const void* v_pages, const int32_t* page_table, const float* lse_swa,
                                       const float* bias, int32_t* indices, void* scores, void* weights, void* o,
                                       float* lse_total, float* sel_logits, int B, int L, int N, int HQ, int H,
                                       int D, int topk, int block_size, int window_size, int q_offset,
                                       int max_pages, int num_pages, float sm_scale_sel, float sm_scale_attn,
                                       int mask_last, int lmk_dense, int lmk_head_major, int lmk_cap,
-                                      int lmk_per_qhead, void* stream) {
+                                      int lmk_per_qhead, void* workspace, size_t workspace_bytes, void* stream) {
   HILS_REQUIRE(!lmk_dense || !lmk_head_major || lmk_cap >= N,
                "hils_decode_step_paged: lmk_cap (%d) must be at least N (%d)", lmk_cap, N);
   HILS_REQUIRE(q && lmk_pages && k_pages && v_pages && page_table && lse_swa && indices && scores && weights && o,
@@ -2202,10 +2494,24 @@ extern "C" int hils_decode_step_paged(const void* q, const void* lmk_pages, cons
                                   lmk_dense ? lmk_head_major : 0, lmk_cap, lmk_per_qhead, indices, scores, weights, o, lse_total,
                                   sel_logits, B, L, 0, N, HQ, H, D, topk, block_size, window_size, q_offset,
                                   sm_scale_sel, sm_scale_attn, mask_last, page_table, max_pages, num_pages,
-                                  (hipStream_t)stream))
+                                  workspace, workspace_bytes, (hipStream_t)stream))
     return rc;
   HILS_CHECK_LAUNCH("hils_decode_step_paged");
   return HILS_OK;
+}
+
+extern "C" int hils_decode_step_paged(const void* q, const void* lmk_pages, const void* k_pages,
+                                      const void* v_pages, const int32_t* page_table, const float* lse_swa,
+                                      const float* bias, int32_t* indices, void* scores, void* weights, void* o,
+                                      float* lse_total, float* sel_logits, int B, int L, int N, int HQ, int H,
+                                      int D, int topk, int block_size, int window_size, int q_offset,
+                                      int max_pages, int num_pages, float sm_scale_sel, float sm_scale_attn,
+                                      int mask_last, int lmk_dense, int lmk_head_major, int lmk_cap,
+                                      int lmk_per_qhead, void* stream) {
+  return hils_decode_step_paged_ws(q, lmk_pages, k_pages, v_pages, page_table, lse_swa, bias, indices, scores, weights,
+                                   o, lse_total, sel_logits, B, L, N, HQ, H, D, topk, block_size, window_size, q_offset,
+                                   max_pages, num_pages, sm_scale_sel, sm_scale_attn, mask_last, lmk_dense,
+                                   lmk_head_major, lmk_cap, lmk_per_qhead, nullptr, 0, stream);
 }
 
 static bool topk_use_split(int B, int L, int N, int h_kv) {

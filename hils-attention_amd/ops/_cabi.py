@@ -32,6 +32,9 @@ SIGNATURES = {
     "hils_sparse_attn_decode_paged": [_P] * 8 + [_Z] + [_I] * 9 + [_F, _I, _P],
     "hils_decode_step": [_P] * 12 + [_I] * 11 + [_F, _F, _I, _I, _I, _I, _P],
     "hils_decode_step_paged": [_P] * 13 + [_I] * 12 + [_F, _F, _I, _I, _I, _I, _I, _P],
+    "hils_decode_step_workspace": [_I] * 9,
+    "hils_decode_step_ws": [_P] * 12 + [_I] * 11 + [_F, _F, _I, _I, _I, _I, _P, _Z, _P],
+    "hils_decode_step_paged_ws": [_P] * 13 + [_I] * 12 + [_F, _F, _I, _I, _I, _I, _I, _P, _Z, _P],
     "hils_topk_bwd": [_P] * 7 + [_Z] + [_I] * 8 + [_F, _P],
     "hils_sparse_attn_fwd": [_P] * 10 + [_Z] + [_I] * 13 + [_F, _I, _F, _I, _P],
     "hils_pack_kv_chunks": [_P, _P, _P, _Z, _I, _I, _I, _I, _I, _P],

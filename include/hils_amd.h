@@ -318,6 +318,25 @@ int hils_decode_step_paged(const void* q, const void* lmk_pages, const void* k_p
                            int q_offset, int max_pages, int num_pages, float sm_scale_sel, float sm_scale_attn,
                            int mask_last, int lmk_dense, int lmk_head_major, int lmk_cap, int lmk_per_qhead,
                            void* stream);
+/* The same with a workspace of hils_decode_step_workspace(...) bytes (0: none is of use; lmk_paged: the chunk
+ * keys are addressed through the page table).  With it, and few rows for the chip, several workgroups share
+ * a row: the logits come from a first kernel, the attention of a row is split over workgroups. */
+size_t hils_decode_step_workspace(int B, int L, int N, int HQ, int H, int D, int topk, int lmk_per_qhead,
+                                  int lmk_paged);
+int hils_decode_step_ws(const void* q, const void* lmks, const void* k, const void* v, const float* lse_swa,
+                        const float* bias, int32_t* indices, void* scores, void* weights, void* o,
+                        float* lse_total, float* sel_logits, int B, int L, int Lkv, int N, int HQ, int H, int D,
+                        int topk, int block_size, int window_size, int q_offset, float sm_scale_sel,
+                        float sm_scale_attn, int mask_last, int lmk_head_major, int lmk_cap, int lmk_per_qhead,
+                        void* workspace, size_t workspace_bytes, void* stream);
+int hils_decode_step_paged_ws(const void* q, const void* lmk_pages, const void* k_pages, const void* v_pages,
+                              const int32_t* page_table, const float* lse_swa, const float* bias, int32_t* indices,
+                              void* scores, void* weights, void* o, float* lse_total, float* sel_logits, int B,
+                              int L, int N, int HQ, int H, int D, int topk, int block_size, int window_size,
+                              int q_offset, int max_pages, int num_pages, float sm_scale_sel, float sm_scale_attn,
+                              int mask_last, int lmk_dense, int lmk_head_major, int lmk_cap, int lmk_per_qhead,
+                              void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* ---- exact per-chunk log Z ---------------------------------------------------- */
 
