@@ -742,8 +742,13 @@ static size_t ga_vmax_bytes(int B, int H, int nchunk) {
 // such that the fixed-point output tile, the chunk histogram, the pair list and the add counts
 // fit in the LDS of a compute unit, with at most GA_MAXP pairs per thread.  The more rows share a
 // visit, the fewer bytes of K and V the block pulls per row.  Returns 0 when nothing fits.
+// A call too small for that gets more, smaller blocks: one round of the compute units (or two, when it
+// would otherwise end in a partly filled second one), down to four queries.  units: (batch, KV head)
+// pairs.  (56 blocks of 72 queries -> 250 of 8 at B1 L2000 16/2 heads of 64: 57 -> 22 us; 16 blocks of 64
+// -> 256 of 4 at 128 queries on 64K tokens, 32/8 heads of 128: 329 -> 65; 420 of 72 -> 474 of 64 at B3
+// L5000 16/2: 150 -> 137; twice as many blocks as compute units were slower again, 31 us in the first.)
 #define GA_SMEM_MAX (160 * 1024 - 512)  // dynamic LDS beside the kernel's static arrays
-static int ga_pick_T(int L, int G, int Dv, int K, int nchunk, int q_block, size_t* smem_out) {
+static int ga_pick_T(int L, long units, int G, int Dv, int K, int nchunk, int q_block, size_t* smem_out) {
   // per query: G output rows, K pairs, G add counts, G row scales
   const size_t per_q = (size_t)G * Dv * 4 + (size_t)K * 4 + (size_t)G * 4 + (size_t)G * 4;
   const size_t fixed = (size_t)nchunk * 4;
@@ -751,6 +756,19 @@ static int ga_pick_T(int L, int G, int Dv, int K, int nchunk, int q_block, size_
   long T = (long)((GA_SMEM_MAX - fixed) / per_q);
   if (T * K > GA_MAXP * GA_THREADS) T = (GA_MAXP * GA_THREADS) / K;
   if (T > L) T = L;
+  {
+    const long cus = hils_device_cus(), wgs = units * ((L + T - 1) / T);
+    const long rounds = wgs <= cus ? 1 : 2;
+    if (wgs <= cus || (4 * wgs > 5 * cus && wgs < 2 * cus)) {
+      const long per_unit = cus * rounds / units;  // blocks a (batch, KV head) gets
+      if (per_unit > 0) {
+        long t = (L + per_unit - 1) / per_unit;
+        t = t <= 4 ? 4 : (t + 7) & ~7L;
+        t = (t + q_block - 1) / q_block * q_block;
+        if (t < T) T = t;
+      }
+    }
+  }
   if (T >= 8 && q_block <= 8 && 8 % q_block == 0) T &= ~7L;
   else T -= T % q_block;
   if (T < 1) return 0;
@@ -770,7 +788,7 @@ size_t hils_ga_workspace_bytes(int B, int L, int Lkv, int HQ, int H, int D, int 
                   K >= 1 && K <= 256 && (long)L * q_block < (1L << 31);  // hils_udiv by q_block stays exact
   if (!ok) return 0;
   size_t smem;
-  const int T = ga_pick_T(L, G, Dv, K, Lkv / S, q_block, &smem);
+  const int T = ga_pick_T(L, (long)B * H, G, Dv, K, Lkv / S, q_block, &smem);
   if (T == 0 || T % q_block != 0) return 0;  // a query block holds whole index-sharing groups
   const int nchunk = Lkv / S;
   return ga_vt_bytes(B, H, nchunk, Dv) + ga_vt_bytes(B, H, nchunk, D) + ga_vmax_bytes(B, H, nchunk) +
@@ -789,7 +807,7 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
   const int nchunk = Lkv / S;
   hipStream_t st = (hipStream_t)stream;
   size_t smem;
-  const int T = ga_pick_T(L, G, Dv, K, nchunk, q_block, &smem);
+  const int T = ga_pick_T(L, (long)B * H, G, Dv, K, nchunk, q_block, &smem);
   if (T == 0 || T % q_block != 0 || H > 65535 || B > 65535) return HILS_OK;
   const int nblk = (L + T - 1) / T;
   const long total = (long)nblk * H * B;
