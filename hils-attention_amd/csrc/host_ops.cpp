@@ -130,9 +130,10 @@ struct SwaFn : torch::autograd::Function<SwaFn> {
     const Tensor d_lse = g[1].defined() ? as_f32(g[1]) : Tensor();
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     Tensor delta = new_tensor({B, L, HQ}, q, at::kFloat);
-    HILS_CALL(hils_swa_bwd, cptr(q), cptr(k), cptr(v), cptr(o), fptr(lse), cptr(d_o), fptr(d_lse), mptr(dq), mptr(dk),
+    const Tensor ws = workspace(hils_swa_bwd_workspace(i32(B), i32(L), i32(HQ), i32(H), i32(D), i32(Dv), i32(cfg[0])), q);
+    HILS_CALL(hils_swa_bwd_ws, cptr(q), cptr(k), cptr(v), cptr(o), fptr(lse), cptr(d_o), fptr(d_lse), mptr(dq), mptr(dk),
               mptr(dv), mfptr(delta), i32(B), i32(L), i32(HQ), i32(H), i32(D), i32(Dv), i32(cfg[0]), i32(cfg[1]),
-              i32(cfg[2]), i32(cfg[3]), (float)ctx->saved_data["scale"].toDouble());
+              i32(cfg[2]), i32(cfg[3]), (float)ctx->saved_data["scale"].toDouble(), mptr(ws), bytes(ws));
     return {dq, dk, dv, Tensor()};
   }
 };

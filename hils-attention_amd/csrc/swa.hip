@@ -612,7 +612,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                   const bf16_t* __restrict__ v, const float* __restrict__ lse,
                   const bf16_t* __restrict__ d_o, const float* __restrict__ delta_in,
-                  bf16_t* __restrict__ dk, bf16_t* __restrict__ dv, SwaDims dm, int n_kb, int n_b) {
+                  bf16_t* __restrict__ dk, bf16_t* __restrict__ dv, SwaDims dm, int n_kb, int n_b, int n_split,
+                  float* __restrict__ part) {
   constexpr int TT = swa_dq_rt(D, DV);
   constexpr int KS = D / 32, VS = DV / 32, DT = D / 16, DVT = DV / 16;
   constexpr int QT = 64 / G;
@@ -631,7 +632,9 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   const int col = lane & 15, j = lane >> 4;
   int kb, hk;
   long b;
-  if (!swa_xcd_unit(n_kb, dm.H, n_b, kb, hk, b)) return;
+  if (!swa_xcd_unit(n_kb * n_split, dm.H, n_b, kb, hk, b)) return;
+  const int split = kb % n_split;
+  kb /= n_split;
   const int L = dm.Lq;
   const int j0 = kb * (64 * TT);
   const int tok_w = j0 + wave * (16 * TT);  // first owned token of the wavefront
@@ -661,8 +664,13 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   if (j1 > L - 1) j1 = L - 1;
   long t_hi = dm.expand ? ((long)(j1 / dm.chunk) + 1) * dm.chunk + dm.window - 2 : (long)j1 + dm.window - 1;
   if (t_hi > L - 1) t_hi = L - 1;
-  const int tile0 = j0 / QT;
-  const int n_tiles = (int)(t_hi / QT) + 1;
+  // this workgroup's share of the row tiles
+  int tile0 = j0 / QT, n_tiles = (int)(t_hi / QT) + 1;
+  {
+    const int n = n_tiles - tile0;
+    n_tiles = tile0 + (int)((long)n * (split + 1) / n_split);
+    tile0 += (int)((long)n * split / n_split);
+  }
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
   uint4 qr[QPASS][2], dor[OPASS][2];
@@ -719,8 +727,10 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 #pragma unroll
     for (int dt = 0; dt < DVT; ++dt) accv[tt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  fetch(tile0);
-  stash();
+  if (tile0 < n_tiles) {
+    fetch(tile0);
+    stash();
+  }
   __syncthreads();
   for (int tile = tile0; tile < n_tiles; ++tile) {
     fetch(tile + 1 < n_tiles ? tile + 1 : tile);
@@ -781,6 +791,20 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     stash();
     __syncthreads();
   }
+  if (n_split > 1) {
+    float* out = part + (((b * dm.H + hk) * n_kb + kb) * (long)n_split + split) * (64 * TT * (D + DV));
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* row = out + (wave * (16 * TT) + tt * 16 + 4 * j + i) * (D + DV) + col;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) row[dt * 16] = acck[tt][dt][i];
+#pragma unroll
+        for (int dt = 0; dt < DVT; ++dt) row[D + dt * 16] = accv[tt][dt][i];
+      }
+    return;
+  }
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
@@ -794,6 +818,49 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 #pragma unroll
       for (int dt = 0; dt < DVT; ++dt) outv[dt * 16] = f2bf(accv[tt][dt][i]);
     }
+}
+
+// Sum of the shares of swa_bwd_dkdv_mfma, in order; four features per thread.
+template <int D, int DV>
+__global__ void __launch_bounds__(256)
+swa_bwd_dkdv_sum(const float* __restrict__ part, bf16_t* __restrict__ dk, bf16_t* __restrict__ dv, int L, int H, int n_kb,
+                 int n_split) {
+  constexpr int F4 = (D + DV) / 4, NTOK = 64 * swa_dq_rt(D, DV), N = NTOK * F4;
+  const int cell = blockIdx.x, kb = cell % n_kb, unit = cell / n_kb;
+  const int hk = unit % H;
+  const long b = unit / H;
+  const f32x4_t* src = (const f32x4_t*)part + (long)cell * n_split * N;
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < N; i += gridDim.y * 256) {
+    const int t = i / F4, f = (i - t * F4) * 4, tok = kb * NTOK + t;
+    if (tok >= L) break;
+    f32x4_t x = src[i];
+    for (int s = 1; s < n_split; ++s) {
+      const f32x4_t y = src[(long)s * N + i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += y[e];
+    }
+    uint2 pk;
+    pk.x = pack_bf2(x[0], x[1]);
+    pk.y = pack_bf2(x[2], x[3]);
+    const long row = (b * L + tok) * H + hk;
+    *(uint2*)(f < D ? dk + row * D + f : dv + row * DV + f - D) = pk;
+  }
+}
+
+// Shares of a token block's rows: with fewer than two workgroups per compute unit (what registers allow) the
+// row tiles of a block (88 of them at window 512 and eight heads, 2 us each) are split, four tiles or more each.
+static int swa_bwd_nsplit(int B, int L, int HQ, int H, int D, int Dv, int window) {
+  const int nt = 64 * swa_dq_rt(D, Dv);
+  const long cells = (long)((L + nt - 1) / nt) * H * B;
+  const long tiles = ((long)(window < L ? window : L) + nt + 63) * (HQ / H) / 64;
+  long s = 2L * hils_device_cus() / cells;
+  if (s > tiles / 4) s = tiles / 4;
+  return s < 2 ? 1 : (int)s;
+}
+extern "C" size_t hils_swa_bwd_workspace(int B, int L, int HQ, int H, int D, int Dv, int window) {
+  if (B <= 0 || L <= 0 || H <= 0 || HQ <= 0) return 0;
+  const int s = swa_bwd_nsplit(B, L, HQ, H, D, Dv, window), nt = 64 * swa_dq_rt(D, Dv);
+  return s == 1 ? 0 : (size_t)((L + nt - 1) / nt) * H * B * s * nt * (D + Dv) * sizeof(float);
 }
 
 template <int D, int DV, int G, int NWV, int RES>
@@ -902,7 +969,7 @@ extern "C" int hils_swa_fwd(const void* q, const void* k, const void* v, void* o
 template <int D, int DV, int G>
 static int swa_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, const bf16_t* o,
                           const float* lse, const bf16_t* d_o, const float* d_lse, bf16_t* dq, bf16_t* dk,
-                          bf16_t* dv, float* delta, int B, const SwaDims& dm, hipStream_t st) {
+                          bf16_t* dv, float* delta, int B, const SwaDims& dm, int n_split, float* part, hipStream_t st) {
   const int QB = 4 * 16 * swa_dq_rt(D, DV) / G;
   const int n_qt = (dm.Lq + QB - 1) / QB;
   hipLaunchKernelGGL((swa_bwd_dq_mfma<D, DV, G>), swa_xcd_grid(n_qt, dm.H, B),
@@ -913,28 +980,32 @@ static int swa_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, con
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_swa_bwd")) return rc;
   const int n_kb = (dm.Lq + 64 * swa_dq_rt(D, DV) - 1) / (64 * swa_dq_rt(D, DV));
-  hipLaunchKernelGGL(kern, swa_xcd_grid(n_kb, dm.H, B), dim3(256), smem, st, q, k, v, lse, d_o, delta, dk, dv, dm,
-                     n_kb, B);
+  hipLaunchKernelGGL(kern, swa_xcd_grid(n_kb * n_split, dm.H, B), dim3(256), smem, st, q, k, v, lse, d_o, delta, dk, dv,
+                     dm, n_kb, B, n_split, part);
+  if (n_split > 1)
+    hipLaunchKernelGGL((swa_bwd_dkdv_sum<D, DV>), dim3((unsigned)((long)n_kb * dm.H * B), 8), dim3(256), 0, st, part, dk,
+                       dv, dm.Lq, dm.H, n_kb, n_split);
   return HILS_OK;
 }
 
 template <int D, int DV>
 static int swa_bwd_launch_g(int G, const bf16_t* q, const bf16_t* k, const bf16_t* v, const bf16_t* o,
                             const float* lse, const bf16_t* d_o, const float* d_lse, bf16_t* dq,
-                            bf16_t* dk, bf16_t* dv, float* delta, int B, const SwaDims& dm, hipStream_t st) {
+                            bf16_t* dk, bf16_t* dv, float* delta, int B, const SwaDims& dm, int n_split, float* part, hipStream_t st) {
   switch (G) {
-    case 1: return swa_bwd_launch<D, DV, 1>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, st);
-    case 2: return swa_bwd_launch<D, DV, 2>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, st);
-    case 4: return swa_bwd_launch<D, DV, 4>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, st);
-    case 8: return swa_bwd_launch<D, DV, 8>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, st);
-    default: return swa_bwd_launch<D, DV, 16>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, st);
+    case 1: return swa_bwd_launch<D, DV, 1>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, n_split, part, st);
+    case 2: return swa_bwd_launch<D, DV, 2>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, n_split, part, st);
+    case 4: return swa_bwd_launch<D, DV, 4>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, n_split, part, st);
+    case 8: return swa_bwd_launch<D, DV, 8>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, n_split, part, st);
+    default: return swa_bwd_launch<D, DV, 16>(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, dm, n_split, part, st);
   }
 }
 
-extern "C" int hils_swa_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
+extern "C" int hils_swa_bwd_ws(const void* q, const void* k, const void* v, const void* o, const float* lse,
                             const void* d_o, const float* d_lse, void* dq, void* dk, void* dv,
                             float* delta, int B, int L, int HQ, int H, int D, int Dv, int window,
-                            int chunk, int mask_lmk, int expand_to_chunk, float sm_scale, void* stream) {
+                            int chunk, int mask_lmk, int expand_to_chunk, float sm_scale, void* workspace,
+                               size_t workspace_bytes, void* stream) {
   HILS_REQUIRE(q && k && v && o && lse && d_o && dq && dk && dv && delta, "hils_swa_bwd: null pointer");
   HILS_REQUIRE(B > 0 && L > 0 && HQ > 0 && H > 0, "hils_swa_bwd: sizes must be positive");
   HILS_REQUIRE(HQ % H == 0, "hils_swa_bwd: HQ (%d) must be a multiple of H (%d)", HQ, H);
@@ -947,19 +1018,31 @@ extern "C" int hils_swa_bwd(const void* q, const void* k, const void* v, const v
   HILS_REQUIRE(((long)L / 8 + 1) * H * B < (1L << 31) - 8, "hils_swa_bwd: B * H * L too large for the grid");
   HILS_REQUIRE((long)L + window < 2147483647L / 2, "hils_swa_bwd: positions overflow 32 bits");
   SwaDims dm{L, L, HQ, H, window, chunk, mask_lmk, expand_to_chunk, 0, (chunk & (chunk - 1)) == 0, sm_scale};
+  const int n_split = workspace ? swa_bwd_nsplit(B, L, HQ, H, D, Dv, window) : 1;
+  HILS_REQUIRE(n_split == 1 || workspace_bytes >= hils_swa_bwd_workspace(B, L, HQ, H, D, Dv, window),
+               "hils_swa_bwd: the workspace is too short (%zu bytes)", workspace_bytes);
+  float* part = (float*)workspace;
   hipStream_t st = (hipStream_t)stream;
   const bf16_t *qq = (const bf16_t*)q, *kk = (const bf16_t*)k, *vv = (const bf16_t*)v,
                *oo = (const bf16_t*)o, *dd = (const bf16_t*)d_o;
   int rc;
   if (D == 64 && Dv == 64)
-    rc = swa_bwd_launch_g<64, 64>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, st);
+    rc = swa_bwd_launch_g<64, 64>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, n_split, part, st);
   else if (D == 128 && Dv == 128)
-    rc = swa_bwd_launch_g<128, 128>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, st);
+    rc = swa_bwd_launch_g<128, 128>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, n_split, part, st);
   else if (D == 64)
-    rc = swa_bwd_launch_g<64, 128>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, st);
+    rc = swa_bwd_launch_g<64, 128>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, n_split, part, st);
   else
-    rc = swa_bwd_launch_g<128, 64>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, st);
+    rc = swa_bwd_launch_g<128, 64>(G, qq, kk, vv, oo, lse, dd, d_lse, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, delta, B, dm, n_split, part, st);
   if (rc) return rc;
   HILS_CHECK_LAUNCH("hils_swa_bwd");
   return HILS_OK;
+}
+
+extern "C" int hils_swa_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                            const void* d_o, const float* d_lse, void* dq, void* dk, void* dv,
+                            float* delta, int B, int L, int HQ, int H, int D, int Dv, int window,
+                            int chunk, int mask_lmk, int expand_to_chunk, float sm_scale, void* stream) {
+  return hils_swa_bwd_ws(q, k, v, o, lse, d_o, d_lse, dq, dk, dv, delta, B, L, HQ, H, D, Dv, window, chunk, mask_lmk,
+                         expand_to_chunk, sm_scale, nullptr, 0, stream);
 }

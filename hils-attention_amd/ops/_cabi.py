@@ -53,6 +53,8 @@ SIGNATURES = {
     "hils_norm_rope_pool_bwd_workspace": [_I] * 5,
     "hils_swa_fwd": [_P] * 5 + [_I] * 12 + [_F, _P],
     "hils_swa_fwd_strided": [_P] * 3 + [_Z, _Z] + [_P] * 2 + [_I] * 12 + [_F, _P],
+    "hils_swa_bwd_workspace": [_I] * 7,
+    "hils_swa_bwd_ws": [_P] * 11 + [_I] * 10 + [_F, _P, _Z, _P],
     "hils_swa_bwd": [_P] * 11 + [_I] * 10 + [_F, _P],
 }
 

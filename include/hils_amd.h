@@ -385,6 +385,14 @@ int hils_swa_bwd(const void* q, const void* k, const void* v, const void* o, con
                  const void* d_o, const float* d_lse, void* dq, void* dk, void* dv, float* delta,
                  int B, int L, int HQ, int H, int D, int Dv, int window, int chunk, int mask_lmk,
                  int expand_to_chunk, float sm_scale, void* stream);
+/* The same with a workspace of hils_swa_bwd_workspace(...) bytes (0: none is of use): few tokens for the chip have
+ * the rows that see a token block split over workgroups, whose shares are added up there. */
+size_t hils_swa_bwd_workspace(int B, int L, int HQ, int H, int D, int Dv, int window);
+int hils_swa_bwd_ws(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                    const void* d_o, const float* d_lse, void* dq, void* dk, void* dv, float* delta,
+                    int B, int L, int HQ, int H, int D, int Dv, int window, int chunk, int mask_lmk,
+                    int expand_to_chunk, float sm_scale, void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* ---- rotary position embedding ---------------------------------------------------- */
 
