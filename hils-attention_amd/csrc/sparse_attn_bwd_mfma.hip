@@ -86,36 +86,94 @@ bw_count_kernel(const int32_t* __restrict__ indices, int* __restrict__ counts, i
     if (hist[i]) atomicAdd(&out[i], hist[i]);
 }
 
-// exclusive scan of n counts into offsets[0..n] (offsets[n] = total); one workgroup
+// Work items of the dK/dV kernel (null: none wanted): every cell (batch, KV head, chunk) is cut into
+// segments of at most seg_pairs pairs, an empty one is one item (its gradients are zeroed).
+struct BwItems {
+  int2* list;     // (cell, segment)
+  int* total;     // number of items
+  int* part_off;  // [cell] first partial result of a cell of several segments
+  int seg_pairs;
+};
+
+// exclusive scan of n counts into offsets[0..n] (offsets[n] = total) and the item list; one workgroup, four
+// counts per thread and step.  The arrays are 16-byte aligned and padded to a multiple of four entries.
 __global__ void __launch_bounds__(1024)
-bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* __restrict__ cursor, long n) {
-  __shared__ int wsum[16];
-  __shared__ int carry_s;
+bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* __restrict__ cursor, int n, BwItems it) {
+  __shared__ int wsum[3][16];
+  __shared__ int carry_s[3];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) carry_s = 0;
+  auto segs = [&](int x) -> int { return x > it.seg_pairs ? (x + it.seg_pairs - 1) / it.seg_pairs : 1; };
+  if (tid < 3) carry_s[tid] = 0;
   __syncthreads();
-  for (long base = 0; base < n; base += 1024) {
-    const long i = base + tid;
-    const int x = (i < n) ? counts[i] : 0;
-    int incl = x;
+  for (int base = 0; base < n; base += 4096) {
+    const int i0 = base + tid * 4;  // (the arrays are padded to whole groups of four)
+    int x[4] = {0, 0, 0, 0};
+    if (i0 < n) {
+      const int4 c4 = *(const int4*)&counts[i0];
+      x[0] = c4.x;
+      x[1] = i0 + 1 < n ? c4.y : 0;
+      x[2] = i0 + 2 < n ? c4.z : 0;
+      x[3] = i0 + 3 < n ? c4.w : 0;
+    }
+    int s[3] = {0, 0, 0};  // pairs, items, partial results
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += y;
+    for (int e = 0; e < 4; ++e) {
+      s[0] += x[e];
+      if (it.list && i0 + e < n) {
+        const int ns = segs(x[e]);
+        s[1] += ns;
+        s[2] += ns > 1 ? ns : 0;
+      }
     }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int pre = carry_s;
-    for (int w = 0; w < wave; ++w) pre += wsum[w];
-    if (i < n) {
-      offsets[i] = pre + incl - x;
-      cursor[i] = pre + incl - x;
+    int pos[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      int incl = s[e];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) wsum[e][wave] = incl;
+      pos[e] = incl - s[e];
     }
     __syncthreads();
-    if (tid == 1023) carry_s = pre + incl;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      pos[e] += carry_s[e];
+      for (int w = 0; w < wave; ++w) pos[e] += wsum[e][w];
+    }
+    __syncthreads();
+    if (tid == 1023) {
+#pragma unroll
+      for (int e = 0; e < 3; ++e) carry_s[e] = pos[e] + s[e];
+    }
+    if (i0 < n) {
+      int4 o4, p4;
+      int* op = (int*)&o4;
+      int* pp = (int*)&p4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        op[e] = pos[0];
+        pos[0] += x[e];
+        pp[e] = pos[2];
+        if (it.list && i0 + e < n) {
+          const int ns = segs(x[e]);
+          for (int k = 0; k < ns; ++k) it.list[pos[1] + k] = make_int2(i0 + e, k);
+          pos[1] += ns;
+          pos[2] += ns > 1 ? ns : 0;
+        }
+      }
+      *(int4*)&offsets[i0] = o4;  // (offsets[n], when it lies in the group, is written below)
+      *(int4*)&cursor[i0] = o4;
+      if (it.list) *(int4*)&it.part_off[i0] = p4;
+    }
     __syncthreads();
   }
-  if (tid == 0) offsets[n] = carry_s;
+  if (tid == 0) {
+    offsets[n] = carry_s[0];
+    if (it.list) *it.total = carry_s[1];
+  }
 }
 
 // pairs grouped by (b,h,c): a workgroup histograms its segment of queries in LDS, reserves one
@@ -147,7 +205,11 @@ bw_scatter_kernel(const int32_t* __restrict__ indices, int* __restrict__ cursor,
 }
 
 // ---------------------------------------------------------------------------
-// dK, dV: one workgroup of four wavefronts per (batch, KV head, chunk)
+// dK, dV: one workgroup of four wavefronts per work item, a segment of the pairs of a (batch, KV head,
+// chunk).  A chunk near the start of the sequence is selected two to three times as often as the average
+// one, and with one workgroup per chunk and all of them resident at once the kernel ran as long as its
+// fullest chunk (B2 L8192 32/4 heads of 64, top-32: 1300 us; in segments 1035).  The segments of
+// a cut chunk leave fp32 partial results that bw_dkdv_sum_kernel adds up.
 // ---------------------------------------------------------------------------
 struct BwDims {
   int L, Lkv, HQ, H, K, NW, nchunk, mask_last;
@@ -155,12 +217,21 @@ struct BwDims {
   int out16;  // dk, dv are bf16 tensors that this kernel overwrites (else fp32, added to)
   int B;
   const float* slope;  // per query head, or null: scores lose slope * max(0, 62 - token) before the softmax
+  BwItems items;
+  float* part;  // [partial result][64 tokens][D + DV]
 };
 
+// Tokens of a wavefront.  Every staged row is read (row-wise and column-wise) by each wavefront that has
+// other tokens, and those LDS reads are what bounds the kernel: 144 KiB a round of 64 rows at D = 64 with
+// 16 tokens per wavefront.  Narrow heads have the registers for 32: two wavefronts share the tokens, each
+// takes half of the rows and the two add up at the end (80 KiB a round; two wavefronts per SIMD instead of
+// four: held to 168 registers the kernel spills 63 and takes twice the time).  With one multiply-add per
+// row address, delta as the start of the dP accumulators and the mask left to the output: 1527 -> 1439 us
+// at B8 L8192 16/16 heads of 64, top-32, 1035 -> 930 at B2 L8192 32/4.
+constexpr int bw_tt(int D, int DV) { return (D <= 64 && DV <= 64) ? 2 : 1; }
+
 template <int D, int DV, int G>
-// (64-wide heads fit the register budget of four wavefronts per SIMD: four workgroups per compute
-// unit, whose two 19 KiB staging buffers each just fit the LDS)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D <= 64 && DV <= 64) ? 4 : 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                const bf16_t* __restrict__ weights, const float* __restrict__ lse,
                const float* __restrict__ delta, const bf16_t* __restrict__ d_o,
@@ -169,9 +240,8 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   // delta (B,L,HQ,NW) fp32: sum_tokens P dP of every (row, slot), written by the dQ kernel
   constexpr int KS = D / 32, VS = DV / 32;    // k-steps of the two 16x16x32 products
   constexpr int DT = D / 16, VT = DV / 16;    // 16-wide column tiles of dK, dV
-  constexpr int DMAX = D > DV ? D : DV;
-  constexpr int NSUB = 256 / DMAX;            // 16-row tiles staged per round (4 or 2)
-  constexpr int ROWS = 16 * NSUB;             // rows per round
+  constexpr int TT = bw_tt(D, DV);            // 16-token tiles of a wavefront
+  constexpr int ROWS = 32 * TT;               // rows staged per round: 32 for each wavefront with the same tokens
   constexpr int PPR = ROWS / G;               // pairs per round
   constexpr int QROW = D * 2 + 16;            // staging: padded row (bytes)
   constexpr int OROW = DV * 2 + 16;
@@ -180,16 +250,19 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   // XCD-aware order: hardware hands consecutive workgroup ids to the 8 XCDs in turn; an XCD works
-  // through the chunks of one (batch, KV head) at a time, so the query and dO rows that its
-  // workgroups gather (the same L rows for every chunk of the head) stay in its L2.
-  const int units = dm.H * dm.B;
-  const int slot = (int)(blockIdx.x / 8);
-  const int unit = (slot / dm.nchunk) * 8 + (int)(blockIdx.x % 8);
-  if (unit >= units) return;
-  const int c = slot % dm.nchunk, hk = unit % dm.H;
+  // through one contiguous share of the items, i.e. of the (batch, KV head) pairs, so the query and dO
+  // rows that its workgroups gather (the same L rows for every chunk of the head) stay in its L2.
+  const int n_items = *dm.items.total;
+  const int vid = (int)(blockIdx.x % 8) * ((n_items + 7) / 8) + (int)(blockIdx.x / 8);
+  if ((int)(blockIdx.x / 8) >= (n_items + 7) / 8 || vid >= n_items) return;
+  const int2 item = dm.items.list[vid];
+  const int cell = item.x, c = cell % dm.nchunk, unit = cell / dm.nchunk;
+  const int hk = unit % dm.H;
   const long b = unit / dm.H;
-  const long cell = (b * dm.H + hk) * (long)dm.nchunk + c;
-  const int p_lo = offsets[cell], p_hi = offsets[cell + 1];
+  const int c_lo = offsets[cell], c_hi = offsets[cell + 1];  // the chunk's pairs
+  const bool whole = c_hi - c_lo <= dm.items.seg_pairs;
+  const int p_lo = c_lo + item.y * dm.items.seg_pairs;
+  const int p_hi = c_hi - p_lo <= dm.items.seg_pairs ? c_hi : p_lo + dm.items.seg_pairs;
   if (p_lo == p_hi) {
     if (dm.out16) {  // nobody selected the chunk: its gradients are zero
       bf16_t* dk16 = (bf16_t*)dk_out + ((b * dm.Lkv + (long)c * BW_S) * dm.H + hk) * D;
@@ -202,30 +275,28 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     return;
   }
 
-  // this wavefront's 16 tokens of the chunk as B operands (k = feature, n = token)
-  const long tok = (long)c * BW_S + wave * 16 + col;
-  uint4 kb[KS], vb[VS];
+  // this wavefront's 16 * TT tokens of the chunk as B operands (k = feature, n = token), and its rows
+  const int tw = TT == 2 ? (wave & 1) : wave, rw = TT == 2 ? (wave >> 1) : 0;
+  uint4 kb[TT][KS], vb[TT][VS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-    kb[ks] = *(const uint4*)(k + ((b * dm.Lkv + tok) * dm.H + hk) * D + ks * 32 + j * 8);
+  for (int tt = 0; tt < TT; ++tt) {
+    const long tok = (long)c * BW_S + tw * (16 * TT) + tt * 16 + col;
 #pragma unroll
-  for (int ks = 0; ks < VS; ++ks)
-    vb[ks] = *(const uint4*)(v + ((b * dm.Lkv + tok) * dm.H + hk) * DV + ks * 32 + j * 8);
-  const bool masked_col = dm.mask_last && wave == 3 && col == 15;  // token 63 of the chunk
-  // distance penalty of this lane's token for its four accumulator rows (16 % G == 0: the head of
-  // row 4j + i is the same in every 16-row tile)
-  float pen[4] = {0.f, 0.f, 0.f, 0.f};
-  if (dm.slope) {
-    const int dist = BW_S - 2 - (wave * 16 + col);
+    for (int ks = 0; ks < KS; ++ks)
+      kb[tt][ks] = *(const uint4*)(k + ((b * dm.Lkv + tok) * dm.H + hk) * D + ks * 32 + j * 8);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pen[i] = dm.slope[hk * G + (4 * j + i) % G] * (float)(dist > 0 ? dist : 0);
+    for (int ks = 0; ks < VS; ++ks)
+      vb[tt][ks] = *(const uint4*)(v + ((b * dm.Lkv + tok) * dm.H + hk) * DV + ks * 32 + j * 8);
   }
 
-  f32x4_t acc_k[DT], acc_v[VT];
+  f32x4_t acc_k[TT][DT], acc_v[TT][VT];
 #pragma unroll
-  for (int t = 0; t < DT; ++t) acc_k[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  for (int tt = 0; tt < TT; ++tt) {
 #pragma unroll
-  for (int t = 0; t < VT; ++t) acc_v[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < DT; ++t) acc_k[tt][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < VT; ++t) acc_v[tt][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
   // Staging roles: thread -> (row, 16-byte piece), NQ (NO) items per thread and round.
@@ -259,25 +330,39 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     for (int u = 0; u < NO; ++u) pk_o[u] = pair_of(round, o_row0 + u * ORS);
     pk_r = pair_of(round, tid);
   };
+  // Row addresses are this lane's base plus query * stride, one 32 x 32 + 64 multiply-add each (the row
+  // steps of a thread are multiples of 16: its head is the same for all its rows).
+  static_assert(QRS % 16 == 0 && ORS % 16 == 0, "a thread stages rows of one head");
+  const char* q_lane = (const char*)(q + (b * dm.L * (long)dm.HQ + hk * G + q_row0 % G) * D + q_pc * 8);
+  const char* o_lane = (const char*)(d_o + (b * dm.L * (long)dm.HQ + hk * G + o_row0 % G) * DV + o_pc * 8);
+  const long row_lane = b * dm.L * (long)dm.HQ + hk * G + tid % G;
+  const float* l_lane = lse + row_lane * dm.K;
+  const bf16_t* w_lane = weights + row_lane * dm.NW;
+  const float* d_lane = delta + row_lane * dm.NW;
+  const unsigned q_step = (unsigned)dm.HQ * D * 2u, o_step = (unsigned)dm.HQ * DV * 2u;
+  const unsigned l_step = (unsigned)(dm.HQ * dm.K), w_step = (unsigned)(dm.HQ * dm.NW);
+  auto mad64 = [](unsigned a, unsigned b2, unsigned long c3) __attribute__((always_inline)) -> unsigned long {
+    return (unsigned long)a * b2 + c3;
+  };
   auto fetch = [&](int round) __attribute__((always_inline)) {  // gathers of `round`, whose pairs load_pairs(round) fetched
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
       // padding rows read the row of the chunk's first pair (finite values): their P is 0, so they add nothing
-      xq[u] = *(const bw_u4*)(q + ((b * dm.L + (pk_q[u] >> 8)) * (long)dm.HQ + hk * G + (q_row0 + u * QRS) % G) * D + q_pc * 8);
+      xq[u] = *(const bw_u4*)mad64(pk_q[u] >> 8, q_step, (unsigned long)q_lane);
     }
 #pragma unroll
     for (int u = 0; u < NO; ++u) {
-      xo[u] = *(const bw_u4*)(d_o + ((b * dm.L + (pk_o[u] >> 8)) * (long)dm.HQ + hk * G + (o_row0 + u * ORS) % G) * DV + o_pc * 8);
+      xo[u] = *(const bw_u4*)mad64(pk_o[u] >> 8, o_step, (unsigned long)o_lane);
     }
     {
       // raw values; what a padding row gets instead is decided where they are staged, so that
       // nothing here has to wait for a load
       r_ok = pair_ok(round, tid);
       const uint32_t pk = pk_r;
-      const long rowi = (b * dm.L + (pk >> 8)) * (long)dm.HQ + hk * G + tid % G;
-      r_l2 = lse[rowi * dm.K + (pk & 255)];
-      r_wb = weights[rowi * dm.NW + (pk & 255)];
-      r_dl = delta[rowi * dm.NW + (pk & 255)];
+      const unsigned long le = mad64(pk >> 8, l_step, pk & 255), we = mad64(pk >> 8, w_step, pk & 255);
+      r_l2 = l_lane[le];
+      r_wb = w_lane[we];
+      r_dl = d_lane[we];
     }
   };
   // staging of the gathered rows of a round (in registers since fetch(round)) into buffer `buf`
@@ -294,7 +379,7 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     if (tid < ROWS) {  // padding rows and empty slots: P = 0
       row_lse[tid] = (r_ok && r_l2 != HILS_NEG_INF) ? r_l2 : INFINITY;
       row_w[tid] = r_ok ? bf2f(r_wb) : 0.f;
-      row_delta[tid] = r_ok ? r_dl : 0.f;
+      row_delta[tid] = r_ok ? -r_dl : 0.f;  // negated: the accumulators of dP start from it
     }
   };
   // one column-read of a staged tile: rows r0 + 4j .. r0 + 4j + 3 of columns c0 .. c0 + 15, this
@@ -323,60 +408,89 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     const float* row_w = row_lse + ROWS;
     const float* row_delta = row_w + ROWS;
     const int rows_here = ((npair - round * PPR < PPR) ? npair - round * PPR : PPR) * G;
-    // two 16-row tiles at a time: their P and dS, side by side, are the A operands (m = token,
-    // k = 32 rows) of one 16x16x32 product per column tile; k index 8j + e stands for row
+    // This wavefront's two 16-row tiles: their P and dS, side by side, are the A operands (m = token,
+    // k = 32 rows) of one 16x16x32 product per column tile and token tile; k index 8j + e stands for row
     // 4j + e of the first tile (e < 4) or row 4j + e - 4 of the second
+    const int r0 = rw * 32;
+    if (r0 < rows_here) {
+      uint2 xp[TT][2], xds[TT][2];  // [token tile][row tile]
 #pragma unroll
-    for (int sub = 0; sub < NSUB; sub += 2) {
-      if (sub * 16 < rows_here) {
-        uint2 xp[2], xds[2];
+      for (int h2 = 0; h2 < 2; ++h2) {
+        // ---- S and dP of 16 rows x this wavefront's tokens
+        const int r = r0 + h2 * 16 + 4 * j;
+        const f32x4_t l4 = *(const f32x4_t*)&row_lse[r], w4 = *(const f32x4_t*)&row_w[r], d4 = *(const f32x4_t*)&row_delta[r];
+        f32x4_t s[TT], dp[TT];
 #pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
-          const int sb = sub + h2;
-          // ---- S and dP of 16 rows x this wavefront's 16 tokens
-          f32x4_t s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+        for (int tt = 0; tt < TT; ++tt) {
+          s[tt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+          dp[tt] = d4;  // dP - delta
+        }
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks) {
-            const uint4 a = *(const uint4*)(q_rm + (sb * 16 + col) * QROW + (ks * 32 + j * 8) * 2);
-            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&kb[ks], s, 0, 0, 0);
-          }
+        for (int ks = 0; ks < KS; ++ks) {
+          const uint4 a = *(const uint4*)(q_rm + (r0 + h2 * 16 + col) * QROW + (ks * 32 + j * 8) * 2);
 #pragma unroll
-          for (int ks = 0; ks < VS; ++ks) {
-            const uint4 a = *(const uint4*)(o_rm + (sb * 16 + col) * OROW + (ks * 32 + j * 8) * 2);
-            dp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&vb[ks], dp, 0, 0, 0);
-          }
-          // accumulator layout: column = token `col`, registers = rows 4j..4j+3
-          float pw[4], ds[4];
+          for (int tt = 0; tt < TT; ++tt)
+            s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&kb[tt][ks], s[tt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int ks = 0; ks < VS; ++ks) {
+          const uint4 a = *(const uint4*)(o_rm + (r0 + h2 * 16 + col) * OROW + (ks * 32 + j * 8) * 2);
+#pragma unroll
+          for (int tt = 0; tt < TT; ++tt)
+            dp[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&vb[tt][ks], dp[tt], 0, 0, 0);
+        }
+        if (dm.slope) {  // distance penalty (16 % G == 0: row 4j + i is the same head in every 16-row tile)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int r = sb * 16 + 4 * j + i;
-            float pv = __builtin_amdgcn_exp2f((s[i] - pen[i]) * c2 - row_lse[r]);
-            if (masked_col) pv = 0.f;
-            pw[i] = row_w[r] * pv;
-            ds[i] = pw[i] * (dp[i] - row_delta[r]);
+            const float sl = dm.slope[hk * G + (4 * j + i) % G];
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+              const int dist = BW_S - 2 - (tw * (16 * TT) + tt * 16 + col);
+              s[tt][i] -= sl * (float)(dist > 0 ? dist : 0);
+            }
           }
-          xp[h2].x = pack_bf2(pw[0], pw[1]);
-          xp[h2].y = pack_bf2(pw[2], pw[3]);
-          xds[h2].x = pack_bf2(ds[0], ds[1]);
-          xds[h2].y = pack_bf2(ds[2], ds[3]);
         }
-        const uint4 a_p = make_uint4(xp[0].x, xp[0].y, xp[1].x, xp[1].y);
-        const uint4 a_ds = make_uint4(xds[0].x, xds[0].y, xds[1].x, xds[1].y);
-        // ---- dK += dS^T Q, dV += (wP)^T dO: contraction over the 32 rows
+        // accumulator layout: column = token `col`, registers = rows 4j..4j+3
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-          const uint2 b0 = col_read(q_rm, QROW, sub * 16, t * 16);
-          const uint2 b1 = col_read(q_rm, QROW, (sub + 1) * 16, t * 16);
-          const uint4 bq = make_uint4(b0.x, b0.y, b1.x, b1.y);
-          acc_k[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_ds, *(const bf16x8_t*)&bq, acc_k[t], 0, 0, 0);
-        }
+        for (int tt = 0; tt < TT; ++tt) {
+          float pv[4], ds[4];
 #pragma unroll
-        for (int t = 0; t < VT; ++t) {
-          const uint2 b0 = col_read(o_rm, OROW, sub * 16, t * 16);
-          const uint2 b1 = col_read(o_rm, OROW, (sub + 1) * 16, t * 16);
-          const uint4 bo = make_uint4(b0.x, b0.y, b1.x, b1.y);
-          acc_v[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_p, *(const bf16x8_t*)&bo, acc_v[t], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) pv[i] = __builtin_amdgcn_exp2f(fmaf(s[tt][i], c2, -l4[i]));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            pv[i] *= w4[i];
+            ds[i] = pv[i] * dp[tt][i];
+          }
+          xp[tt][h2].x = pack_bf2(pv[0], pv[1]);
+          xp[tt][h2].y = pack_bf2(pv[2], pv[3]);
+          xds[tt][h2].x = pack_bf2(ds[0], ds[1]);
+          xds[tt][h2].y = pack_bf2(ds[2], ds[3]);
         }
+      }
+      uint4 a_p[TT], a_ds[TT];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        a_p[tt] = make_uint4(xp[tt][0].x, xp[tt][0].y, xp[tt][1].x, xp[tt][1].y);
+        a_ds[tt] = make_uint4(xds[tt][0].x, xds[tt][0].y, xds[tt][1].x, xds[tt][1].y);
+      }
+      // ---- dK += dS^T Q, dV += (wP)^T dO: contraction over the 32 rows
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const uint2 b0 = col_read(q_rm, QROW, r0, t * 16);
+        const uint2 b1 = col_read(q_rm, QROW, r0 + 16, t * 16);
+        const uint4 bq = make_uint4(b0.x, b0.y, b1.x, b1.y);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+          acc_k[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_ds[tt], *(const bf16x8_t*)&bq, acc_k[tt][t], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < VT; ++t) {
+        const uint2 b0 = col_read(o_rm, OROW, r0, t * 16);
+        const uint2 b1 = col_read(o_rm, OROW, r0 + 16, t * 16);
+        const uint4 bo = make_uint4(b0.x, b0.y, b1.x, b1.y);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+          acc_v[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_p[tt], *(const bf16x8_t*)&bo, acc_v[tt][t], 0, 0, 0);
       }
     }
     // the next round's rows (gathered while this round computed) go to the other buffer, which
@@ -390,25 +504,114 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     }
     lds_barrier();
   }
-  // accumulators: column = feature t*16 + col, rows = tokens wave*16 + 4j + i
+  // The two wavefronts with the same tokens add up their row halves: each hands the token tile that the
+  // other keeps over through LDS (the last round's barrier is behind the staging buffers' last use).
+  constexpr int NT = DT + VT;
+  static_assert(TT == 1 || 4 * NT * 64 * 16 <= 2 * BUF, "the exchange fits the staging buffers");
+  f32x4_t* xch = (f32x4_t*)bw_smem;  // [wavefront][column tile][lane]
+  auto give = [&](const f32x4_t (&ak)[DT], const f32x4_t (&av)[VT]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long tk = (long)c * BW_S + wave * 16 + 4 * j + i;
-    const long rk = ((b * dm.Lkv + tk) * dm.H + hk) * D, rv = ((b * dm.Lkv + tk) * dm.H + hk) * DV;
+    for (int t = 0; t < DT; ++t) xch[(wave * NT + t) * 64 + lane] = ak[t];
+#pragma unroll
+    for (int t = 0; t < VT; ++t) xch[(wave * NT + DT + t) * 64 + lane] = av[t];
+  };
+  // accumulators: column = feature t*16 + col, rows = tokens 4j + i of the tile
+  auto finish = [&](f32x4_t (&ak)[DT], f32x4_t (&av)[VT], int tok0) __attribute__((always_inline)) {
+    if constexpr (TT == 2) {
+      const int other = wave ^ 2;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const f32x4_t x = xch[(other * NT + t) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (t < DT) ak[t < DT ? t : 0][i] += x[i];
+          else av[t < DT ? 0 : t - DT][i] += x[i];
+        }
+      }
+    }
+    // a masked last token's own row of sums is the only place its probabilities went: it becomes 0 here
+    if (dm.mask_last && tok0 == BW_S - 16 && j == 3) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t) ak[t][3] = 0.f;
+#pragma unroll
+      for (int t = 0; t < VT; ++t) av[t][3] = 0.f;
+    }
+    if (!whole) {
+      float* out = dm.part + (long)(dm.items.part_off[cell] + item.y) * (BW_S * (D + DV));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* row = out + (tok0 + 4 * j + i) * (D + DV) + col;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) row[t * 16] = ak[t][i];
+#pragma unroll
+        for (int t = 0; t < VT; ++t) row[D + t * 16] = av[t][i];
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const long tk = (long)c * BW_S + tok0 + 4 * j + i;
+      const long rk = ((b * dm.Lkv + tk) * dm.H + hk) * D, rv = ((b * dm.Lkv + tk) * dm.H + hk) * DV;
+      if (dm.out16) {
+        bf16_t* dkr = (bf16_t*)dk_out + rk;
+        bf16_t* dvr = (bf16_t*)dv_out + rv;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) dkr[t * 16 + col] = f2bf(ak[t][i] * dm.sm_scale);
+#pragma unroll
+        for (int t = 0; t < VT; ++t) dvr[t * 16 + col] = f2bf(av[t][i]);
+      } else {
+        float* dkr = (float*)dk_out + rk;
+        float* dvr = (float*)dv_out + rv;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) dkr[t * 16 + col] += ak[t][i] * dm.sm_scale;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) dvr[t * 16 + col] += av[t][i];
+      }
+    }
+  };
+  if constexpr (TT == 2) {
+    if (rw == 0) give(acc_k[1], acc_v[1]); else give(acc_k[0], acc_v[0]);
+    lds_barrier();
+    if (rw == 0) finish(acc_k[0], acc_v[0], tw * 32); else finish(acc_k[1], acc_v[1], tw * 32 + 16);
+  } else {
+    finish(acc_k[0], acc_v[0], tw * 16);
+  }
+}
+
+// the segments of the cut chunks, four features per thread, segments in order
+template <int D, int DV>
+__global__ void __launch_bounds__(256)
+bw_dkdv_sum_kernel(const int* __restrict__ offsets, void* __restrict__ dk_out, void* __restrict__ dv_out, BwDims dm) {
+  const int cell = blockIdx.x;
+  const int cnt = offsets[cell + 1] - offsets[cell];
+  if (cnt <= dm.items.seg_pairs) return;
+  const int ns = (cnt + dm.items.seg_pairs - 1) / dm.items.seg_pairs;
+  const int c = cell % dm.nchunk, unit = cell / dm.nchunk;
+  const int hk = unit % dm.H;
+  const long b = unit / dm.H;
+  constexpr int F4 = (D + DV) / 4, N = BW_S * F4;
+  const f32x4_t* src = (const f32x4_t*)(dm.part + (long)dm.items.part_off[cell] * (BW_S * (D + DV)));
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < N; i += gridDim.y * 256) {
+    f32x4_t x = src[i];
+    for (int k = 1; k < ns; ++k) {
+      const f32x4_t y = src[(long)k * N + i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += y[e];
+    }
+    const int t = i / F4, f = (i - t * F4) * 4;
+    const long row = (b * dm.Lkv + (long)c * BW_S + t) * dm.H + hk;
+    const bool is_k = f < D;
+    const float sc = is_k ? dm.sm_scale : 1.f;
+    const long o = is_k ? row * D + f : row * DV + f - D;
+    void* out = is_k ? dk_out : dv_out;
     if (dm.out16) {
-      bf16_t* dkr = (bf16_t*)dk_out + rk;
-      bf16_t* dvr = (bf16_t*)dv_out + rv;
-#pragma unroll
-      for (int t = 0; t < DT; ++t) dkr[t * 16 + col] = f2bf(acc_k[t][i] * dm.sm_scale);
-#pragma unroll
-      for (int t = 0; t < VT; ++t) dvr[t * 16 + col] = f2bf(acc_v[t][i]);
+      uint2 pk;
+      pk.x = pack_bf2(x[0] * sc, x[1] * sc);
+      pk.y = pack_bf2(x[2] * sc, x[3] * sc);
+      *(uint2*)((bf16_t*)out + o) = pk;
     } else {
-      float* dkr = (float*)dk_out + rk;
-      float* dvr = (float*)dv_out + rv;
 #pragma unroll
-      for (int t = 0; t < DT; ++t) dkr[t * 16 + col] += acc_k[t][i] * dm.sm_scale;
-#pragma unroll
-      for (int t = 0; t < VT; ++t) dvr[t * 16 + col] += acc_v[t][i];
+      for (int e = 0; e < 4; ++e) ((float*)out)[o + e] += x[e] * sc;
     }
   }
 }
@@ -591,9 +794,17 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   const float fx_inv = 1.f / fx_scale;
   const float c2 = dm.sm_scale * HILS_LOG2E;
   const float out_scale = dm.sm_scale * fx_scale;
+  // rows of lse, weights and dw from the block's first query on, with 32-bit element offsets (hils_bw_run)
+  const float* lse_blk = lse + (b * dm.L + t0) * (long)dm.HQ * K;
+  const bf16_t* w_blk = weights + (b * dm.L + t0) * (long)dm.HQ * dm.NW;
+  float* dw_blk = dw + (b * dm.L + t0) * (long)dm.HQ * dm.NW;
+  const bf16_t* q_blk = q + (b * dm.L + t0) * (long)dm.HQ * D;
+  const bf16_t* do_blk = d_o + (b * dm.L + t0) * (long)dm.HQ * DV;
   const int qs = r / G, g = r - qs * G;  // this lane's row of a tile: query slot, head
   const int hq = hk * G + g;
   const float sl = dm.slope ? dm.slope[hq] : 0.f;
+  const unsigned l_row = (unsigned)(hq * K), w_row0 = (unsigned)(hq * dm.NW);  // ... of query 0 and this lane's head
+  const unsigned l_step = (unsigned)(dm.HQ * K), w_step = (unsigned)(dm.HQ * dm.NW);
   const int npair_valid = cur[dm.nchunk - 1];
 
   for (;;) {
@@ -631,7 +842,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
                          __attribute__((always_inline)) {
       const int last = ((ve - p < QT) ? ve - p : QT) - 1;  // padding rows repeat the tile's last pair
       pk_r = pairs[p + (qs < last ? qs : last)];
-      const long rowi = (b * dm.L + t0 + (pk_r >> 8)) * (long)dm.HQ + hq;
+      const unsigned ql_r = (unsigned)pk_r >> 8, slot_r = (unsigned)pk_r & 255u;
       if (STAGE) {
         const int row_l = (pk_r >> 8) * G + g;
 #pragma unroll
@@ -640,12 +851,14 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         for (int ks = 0; ks < VS; ++ks) o_r[ks] = *(const bw_u4*)(rows_o + row_l * OROWB + (ks * 32 + j * 8) * 2);
       } else {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) q_r[ks] = *(const bw_u4*)(q + rowi * D + ks * 32 + j * 8);
+        for (int ks = 0; ks < KS; ++ks)
+          q_r[ks] = *(const bw_u4*)(q_blk + (__umul24(ql_r, (unsigned)(dm.HQ * D)) + (unsigned)(hq * D + ks * 32 + j * 8)));
 #pragma unroll
-        for (int ks = 0; ks < VS; ++ks) o_r[ks] = *(const bw_u4*)(d_o + rowi * DV + ks * 32 + j * 8);
+        for (int ks = 0; ks < VS; ++ks)
+          o_r[ks] = *(const bw_u4*)(do_blk + (__umul24(ql_r, (unsigned)(dm.HQ * DV)) + (unsigned)(hq * DV + ks * 32 + j * 8)));
       }
-      l_r = lse[rowi * K + (pk_r & 255)];
-      w_r = weights[rowi * dm.NW + (pk_r & 255)];
+      l_r = lse_blk[__umul24(ql_r, l_step) + l_row + slot_r];
+      w_r = w_blk[__umul24(ql_r, w_step) + w_row0 + slot_r];
     };
     if (KEEP) load_rows(vs, bq, bdo, l2, wb, pk);
     for (int p = vs; p < ve; p += QT) {
@@ -665,8 +878,6 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         const int qsl = (4 * j + i) / G;
         pk_o[i] = pairs[p + (qsl < last ? qsl : last)];
       }
-      const int ql = pk >> 8, slot = pk & 255;
-      const long rowi = (b * dm.L + t0 + ql) * (long)dm.HQ + hq;
       if (l2 == HILS_NEG_INF) l2 = INFINITY;
       const float w_row = bf2f(wb);
       int orow[4];
@@ -701,6 +912,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         for (int u = 0; u < 2 * DT; ++u) xa[u] = *(const bw_u4*)(kt_c + u * 512);
       }
       if (dm.slope) {
+        asm volatile("" ::: "memory");  // (a branch, not sixteen subtractions of zero in every tile)
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -724,16 +936,17 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         st[3][3] = 0.f;
       }
       delta = rows_sum(delta);
-      if (j == 0 && qs <= last) dw[rowi * dm.NW + slot] = delta;
-      const float f = w_row * out_scale;
+      if (j == 0 && qs <= last) dw_blk[__umul24((unsigned)pk >> 8, w_step) + w_row0 + ((unsigned)pk & 255u)] = delta;
+      const float f = w_row * out_scale, fd = -f * delta;
       bf16x8_t ap[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
+        auto ds = [&](int mt, int i) __attribute__((always_inline)) { return st[mt][i] * fmaf(dpt[mt][i], f, fd); };
         uint4 x;
-        x.x = pack_bf2(f * st[2 * s2][0] * (dpt[2 * s2][0] - delta), f * st[2 * s2][1] * (dpt[2 * s2][1] - delta));
-        x.y = pack_bf2(f * st[2 * s2][2] * (dpt[2 * s2][2] - delta), f * st[2 * s2][3] * (dpt[2 * s2][3] - delta));
-        x.z = pack_bf2(f * st[2 * s2 + 1][0] * (dpt[2 * s2 + 1][0] - delta), f * st[2 * s2 + 1][1] * (dpt[2 * s2 + 1][1] - delta));
-        x.w = pack_bf2(f * st[2 * s2 + 1][2] * (dpt[2 * s2 + 1][2] - delta), f * st[2 * s2 + 1][3] * (dpt[2 * s2 + 1][3] - delta));
+        x.x = pack_bf2(ds(2 * s2, 0), ds(2 * s2, 1));
+        x.y = pack_bf2(ds(2 * s2, 2), ds(2 * s2, 3));
+        x.z = pack_bf2(ds(2 * s2 + 1, 0), ds(2 * s2 + 1, 1));
+        x.w = pack_bf2(ds(2 * s2 + 1, 2), ds(2 * s2 + 1, 3));
         ap[s2] = __builtin_bit_cast(bf16x8_t, x);
       }
       // ---- dQ tile += dS K: four column tiles at a time
@@ -827,10 +1040,18 @@ static int bq_pick_T(int L, int G, int D, int Dv, int K, int nchunk, bool stage,
 }
 
 struct BwLayout {
-  size_t counts, offsets, cursor, pairs, ka, va, kt, vmax, kmax, total;
+  size_t counts, offsets, cursor, pairs, ka, va, kt, vmax, kmax, items, n_items, part_off, part, total;
+  int seg_pairs;
+  size_t max_items;
 };
-static BwLayout bw_layout(int B, int L, int Lkv, int H, int D, int Dv, int K) {
+// Pairs per work item of the dK/dV kernel: about 2048 items of equal size in all (some four rounds of the
+// workgroups that fit the chip), but no less than 512 rows, whose gathers are four times the partial result's bytes.
+static BwLayout bw_layout(int B, int L, int Lkv, int G, int H, int D, int Dv, int K) {
   const size_t cells = (size_t)B * H * (Lkv / BW_S);
+  const size_t pairs = (size_t)B * L * H * K;
+  size_t seg = (pairs + 2047) / 2048;
+  const size_t least = G < 8 ? 512 / G : 64;
+  seg = ((seg > least ? seg : least) + 63) & ~(size_t)63;
   BwLayout lo;
   size_t o = 0;
   lo.counts = o; o += bw_round((cells + 1) * 4);
@@ -842,6 +1063,14 @@ static BwLayout bw_layout(int B, int L, int Lkv, int H, int D, int Dv, int K) {
   lo.kt = o; o += bw_round(cells * BW_S * D * 2);
   lo.vmax = o; o += bw_round(cells * 4);
   lo.kmax = o; o += bw_round(cells * 4);
+  const bool cut = (size_t)L > seg;  // (no chunk has more than L pairs unless a query names it twice)
+  lo.seg_pairs = cut ? (int)seg : 0x7fffffff;
+  lo.max_items = cells + (cut ? pairs / seg : 0);
+  lo.items = o; o += bw_round(lo.max_items * sizeof(int2));
+  lo.n_items = o; o += bw_round(4);
+  lo.part_off = o; o += bw_round((cells + 1) * 4);
+  // a cell of n > seg pairs has ceil(n / seg) <= 2 n / seg partial results
+  lo.part = o; o += cut ? bw_round(2 * (pairs / seg + 1) * BW_S * (size_t)(D + Dv) * 4) : 0;
   lo.total = o;
   return lo;
 }
@@ -851,7 +1080,7 @@ size_t hils_bw_workspace_bytes(int B, int L, int Lkv, int HQ, int H, int D, int 
   if (!hils_bw_covers(L, Lkv, HQ, H, D, Dv, K, S, q_block, WH, sm_n, nullptr)) return 0;
   size_t smem;
   if (bq_pick_T(L, HQ / H, D, Dv, K, Lkv / S, false, &smem) == 0) return 0;
-  return bw_layout(B, L, Lkv, H, D, Dv, K).total;
+  return bw_layout(B, L, Lkv, HQ / H, H, D, Dv, K).total;
 }
 
 template <int D, int DV>
@@ -859,13 +1088,15 @@ static int bw_launch_dkdv(int G, dim3 grid, hipStream_t st, const bf16_t* q, con
                           const bf16_t* v, const bf16_t* w, const float* lse, const float* delta,
                           const bf16_t* d_o, const int* offsets, const uint32_t* pairs, void* dk, void* dv,
                           const BwDims& dm) {
-#define BW_CALL(G_)                                                                                 \
-  hipLaunchKernelGGL((bw_dkdv_kernel<D, DV, G_>), grid, dim3(256), smem, st, q, k, v, w, lse, delta, d_o, \
-                     offsets, pairs, dk, dv, dm)
-  constexpr int DMAX = D > DV ? D : DV;
-  constexpr int NSUB = 256 / DMAX;
-  const size_t smem = 2 * ((size_t)16 * NSUB * (D * 2 + 16) + (size_t)16 * NSUB * (DV * 2 + 16) +
-                           (size_t)3 * 16 * NSUB * sizeof(float));  // two staging buffers
+#define BW_CALL(G_)                                                                                         \
+  do {                                                                                                      \
+    auto kern = bw_dkdv_kernel<D, DV, G_>;                                                                  \
+    static HilsLdsReserve reserved;                                                                         \
+    if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_sparse_attn_bwd")) return rc;   \
+    hipLaunchKernelGGL(kern, grid, dim3(256), smem, st, q, k, v, w, lse, delta, d_o, offsets, pairs, dk, dv, dm); \
+  } while (0)
+  constexpr size_t ROWS = 32 * bw_tt(D, DV);
+  const size_t smem = 2 * (ROWS * (D * 2 + 16) + ROWS * (DV * 2 + 16) + 3 * ROWS * sizeof(float));  // two staging buffers
   switch (G) {
     case 1: BW_CALL(1); break;
     case 2: BW_CALL(2); break;
@@ -875,6 +1106,9 @@ static int bw_launch_dkdv(int G, dim3 grid, hipStream_t st, const bf16_t* q, con
     default: return -1;
   }
 #undef BW_CALL
+  if (dm.items.seg_pairs != 0x7fffffff)  // some chunk may have been cut
+    hipLaunchKernelGGL((bw_dkdv_sum_kernel<D, DV>), dim3((unsigned)((long)dm.B * dm.H * dm.nchunk), 4), dim3(256), 0, st,
+                       offsets, dk, dv, dm);
   return HILS_OK;
 }
 
@@ -920,8 +1154,8 @@ static bool bq_stage_pays(int L, int G, int D, int Dv, int K, int nchunk) {
 // Inverse index of an index tensor (B, L, H, K) with values in [0, nchunk) or < 0: counts,
 // offsets (cells + 1 ints, cells = B*H*nchunk), cursor (scratch) and the pairs (t << 8 | slot)
 // grouped by (b, h, chunk).  Also used by the top-k backward.
-void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
-                            int B, int L, int H, int K, int nchunk, void* stream) {
+static void bw_build_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
+                           const BwItems& items, int B, int L, int H, int K, int nchunk, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const long cells = (long)B * H * nchunk;
   {
@@ -935,8 +1169,14 @@ void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, i
   while ((long)B * H * ((L + seg_len - 1) / seg_len) < 4096 && seg_len > 128) seg_len = (seg_len + 1) / 2;
   dim3 gs((L + seg_len - 1) / seg_len, H, B);
   hipLaunchKernelGGL(bw_count_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, counts, L, H, K, nchunk, seg_len);
-  hipLaunchKernelGGL(bw_scan_kernel, dim3(1), dim3(1024), 0, st, counts, offsets, cursor, cells);
+  hipLaunchKernelGGL(bw_scan_kernel, dim3(1), dim3(1024), 0, st, counts, offsets, cursor, (int)cells, items);
   hipLaunchKernelGGL(bw_scatter_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, cursor, pairs, L, H, K, nchunk, seg_len);
+}
+
+void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
+                            int B, int L, int H, int K, int nchunk, void* stream) {
+  bw_build_index(indices, counts, offsets, cursor, pairs, BwItems{nullptr, nullptr, nullptr, 0}, B, L, H, K, nchunk,
+                 stream);
 }
 
 // Whole backward on the MFMA kernels: dq (bf16, written), dw (fp32, written at the valid slots),
@@ -948,7 +1188,7 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   hipStream_t st = (hipStream_t)stream;
   const int nchunk = Lkv / BW_S;
   const size_t cells = (size_t)B * H * nchunk;
-  const BwLayout lo = bw_layout(B, L, Lkv, H, D, Dv, K);
+  const BwLayout lo = bw_layout(B, L, Lkv, HQ / H, H, D, Dv, K);
   char* ws = (char*)workspace;
   int* counts = (int*)(ws + lo.counts);
   int* offsets = (int*)(ws + lo.offsets);
@@ -960,7 +1200,9 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   float* vmax = (float*)(ws + lo.vmax);
   float* kmax = (float*)(ws + lo.kmax);
   const int G = HQ / H;
-  if (H > 65535 || B > 65535) return -1;
+  if (H > 65535 || B > 65535 || cells > (1u << 30)) return -1;
+  // (24-bit row strides and 32-bit offsets inside a block of up to 256 queries)
+  if ((long)HQ * (D > Dv ? D : Dv) >= (1 << 23) || (long)HQ * NW >= (1 << 22) || (long)HQ * K >= (1 << 22)) return -1;
   // ---- operand packing: K as A operand (+ max|V|), V as A operand + K transposed (+ max|K|)
   hils_ga_pack_launch(k, v, ka, nullptr, vmax, B, Lkv, H, D, Dv, stream);
   hils_ga_pack_launch(v, k, va, kt, kmax, B, Lkv, H, Dv, D, stream);
@@ -970,9 +1212,12 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
     const bool stage = bq_stage_pays(L, G, D, Dv, K, nchunk);
     int T = bq_pick_T(L, G, D, Dv, K, nchunk, stage, &smem);
     if (T == 0) return -1;
-    // small problems: rather every compute unit busy than the largest blocks
-    while (T >= 72 && (long)((L + T - 1) / T) * H * B < 256) {
-      T -= 8;
+    // small problems: rather a block for every compute unit than the largest blocks (64 blocks of 64 queries ->
+    // 256 of 16 at B2 L1024 16/2 heads of 64: 63 -> 26 us)
+    const long cus = hils_device_cus(), units = (long)B * H, per_unit = cus / units;
+    if (units * ((L + T - 1) / T) < cus && per_unit > 0) {
+      const long t = ((L + per_unit - 1) / per_unit + 7) & ~7L;
+      if (t < T) T = (int)t;
       smem = bq_smem_bytes(T, G, D, Dv, K, nchunk, stage);
     }
     const int nblk = (L + T - 1) / T;
@@ -992,8 +1237,9 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
     if (rc != HILS_OK) return rc;
   }
   // ---- inverse index, then dK, dV
-  hils_build_chunk_index(indices, counts, offsets, cursor, pairs, B, L, H, K, nchunk, stream);
-  BwDims dm{L, Lkv, HQ, H, K, NW, nchunk, mask_last, sm_scale, kv16, B, slope};
+  const BwItems items{(int2*)(ws + lo.items), (int*)(ws + lo.n_items), (int*)(ws + lo.part_off), lo.seg_pairs};
+  bw_build_index(indices, counts, offsets, cursor, pairs, items, B, L, H, K, nchunk, stream);
+  BwDims dm{L, Lkv, HQ, H, K, NW, nchunk, mask_last, sm_scale, kv16, B, slope, items, (float*)(ws + lo.part)};
   if (kv16 && Lkv > nchunk * BW_S) {  // tokens behind the last whole chunk are never attended
     for (int b2 = 0; b2 < B; ++b2) {
       const long nk = (long)(Lkv - nchunk * BW_S) * H * D / 2, nv = (long)(Lkv - nchunk * BW_S) * H * Dv / 2;
@@ -1003,9 +1249,9 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
       hipLaunchKernelGGL(bw_fill_int_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, pv, 0, nv);
     }
   }
-  const long unit_rounds = ((long)H * B + 7) / 8;
-  if (unit_rounds * nchunk * 8 > 2147483647L) return -1;
-  dim3 grid((unsigned)(unit_rounds * nchunk * 8));
+  const long grid_n = ((long)lo.max_items + 7) / 8 * 8;
+  if (grid_n > 2147483647L) return -1;
+  dim3 grid((unsigned)grid_n);
   int rc = -1;
 #define BW_D(D_, DV_)                                                                              \
   rc = bw_launch_dkdv<D_, DV_>(G, grid, st, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v,   \

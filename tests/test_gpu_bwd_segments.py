@@ -1,0 +1,100 @@
+"""Backward kernels that share a result between workgroups: chunks whose (query, slot) pairs are cut into segments, token
+blocks of the local branch whose rows are split, and the small query blocks of short calls; against autograd in fp32."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _selected(B, L, H, K, dev, gen, crowd):
+    """Ascending chunk indices, -1 padded; `crowd`: every query takes the first chunks it can see."""
+    N = L // 64
+    vis = ((torch.arange(L, device=dev) - 63) // 64).clamp(0, N).view(1, L, 1, 1)
+    r = torch.rand(B, L, H, N, device=dev, generator=gen)
+    if crowd:
+        r = -torch.arange(N, device=dev, dtype=torch.float32).expand(B, L, H, N)
+    r = r.masked_fill(torch.arange(N, device=dev) >= vis, -1e9)
+    val, idx = r.topk(min(K, N), -1)
+    idx = torch.where(val < -1e8, N, idx).sort(-1).values
+    idx = torch.where(idx == N, -1, idx)
+    return torch.nn.functional.pad(idx, (0, K - idx.shape[-1]), value=-1).int().contiguous()
+
+
+def _reference(q, k, v, w, idx, scale, mask_last):
+    B, L, HQ, D = q.shape
+    H, K, N = k.shape[2], idx.shape[-1], k.shape[1] // 64
+    G = HQ // H
+    out = []
+    for b in range(B):
+        for h in range(H):
+            qq = q[b, :, h * G:(h + 1) * G]                                      # (L, G, D)
+            kk = k[b, : N * 64, h].view(N, 64, D)
+            vv = v[b, : N * 64, h].view(N, 64, -1)
+            s = torch.matmul(qq.reshape(-1, D), kk.reshape(-1, D).t().contiguous()).view(L, G, N, 64) * scale
+            if mask_last:
+                s = torch.cat([s[..., :63], torch.full_like(s[..., :1], float("-inf"))], -1)
+            p = torch.softmax(s, -1)
+            ci = idx[b, :, h].long()
+            wf = torch.zeros(L, G, N + 1, device=q.device)
+            wf = wf.scatter_add(2, torch.where(ci < 0, N, ci).unsqueeze(1).expand(L, G, K), w[b, :, h * G:(h + 1) * G, :K])
+            pw = (p * wf[..., :N].unsqueeze(-1)).view(L * G, N * 64)
+            out.append(torch.matmul(pw, vv.reshape(N * 64, -1)).view(L, G, -1))
+    return torch.stack(out).view(B, H, L, G, -1).permute(0, 2, 1, 3, 4).reshape(B, L, HQ, -1)
+
+
+@pytest.mark.parametrize("B,L,HQ,H,D,Dv,K,crowd,mask_last", [
+    (1, 1024, 8, 1, 64, 64, 8, True, True),     # 64-pair segments, the first chunks cut many times
+    (2, 1000, 16, 2, 64, 64, 16, False, True),  # a ragged last chunk
+    (1, 777, 4, 1, 128, 128, 8, True, False),
+    (1, 2048, 4, 4, 64, 64, 32, True, True),    # one head per KV head
+    (1, 640, 2, 1, 64, 128, 4, True, True),
+    (1, 640, 16, 1, 128, 64, 10, False, True),  # all chunks selected
+    (1, 192, 8, 2, 64, 64, 3, False, True),     # nothing is cut
+])
+def test_sparse_attn_backward(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mask_last):
+    gen = torch.Generator(device=dev).manual_seed(L + D)
+    scale = 1 / math.sqrt(D)
+    q, k, v, w = (torch.randn(*s, device=dev, generator=gen).bfloat16() for s in
+                  ((B, L, HQ, D), (B, L, H, D), (B, L, H, Dv), (B, L, HQ, K + 1)))
+    d_o = torch.randn(B, L, HQ, Dv, device=dev, generator=gen).bfloat16()
+    idx = _selected(B, L, H, K, dev, gen, crowd)
+    xs = [x.clone().requires_grad_() for x in (q, k, v, w)]
+    o = pkg.HiLS_block_M_head(*xs, idx, block_size=64, mask_last_token=mask_last)
+    got = torch.autograd.grad(o, xs, d_o)
+    fs = [x.float().requires_grad_() for x in (q, k, v, w)]
+    ref_o = _reference(*fs, idx, scale, mask_last)
+    ref = torch.autograd.grad(ref_o, fs, d_o.float())
+    for name, a, b in zip(("o", "dq", "dk", "dv", "dw"), (o, *got), (ref_o, *ref)):
+        err = (a.float() - b).norm() / b.norm().clamp_min(1e-20)
+        assert err < 1.5e-2, (name, err.item())
+    if mask_last and L >= 128:  # no query attends to a chunk's last token
+        assert not got[1][:, 63].any() and not got[2][:, 63].any()
+
+
+@pytest.mark.parametrize("B,L,HQ,H,D,W", [(1, 700, 8, 1, 64, 512), (2, 1024, 16, 2, 64, 512), (1, 513, 4, 1, 128, 300),
+                                          (1, 2000, 4, 4, 64, 512)])
+def test_swa_backward_split(pkg, dev, B, L, HQ, H, D, W):
+    from hils_attention_amd.ops import _cabi
+    assert _cabi.load().hils_swa_bwd_workspace(B, L, HQ, H, D, D, W) > 0, "the case must be split"
+    gen = torch.Generator(device=dev).manual_seed(W)
+    q, k, v = (torch.randn(B, L, h, D, device=dev, generator=gen).bfloat16() for h in (HQ, H, H))
+    d_o = torch.randn(B, L, HQ, D, device=dev, generator=gen).bfloat16()
+    d_lse = torch.randn(B, L, HQ, device=dev, generator=gen)
+    xs = [x.clone().requires_grad_() for x in (q, k, v)]
+    o, lse = pkg.flex_attn_tl(*xs, W, 64)
+    got = torch.autograd.grad((o, lse), xs, (d_o, d_lse))
+    fs = [x.float().requires_grad_() for x in (q, k, v)]
+    G = HQ // H
+    t = torch.arange(L, device=dev)
+    see = (t >= (torch.div(t.view(-1, 1) - W + 1, 64, rounding_mode="floor") * 64)) & (t <= t.view(-1, 1)) & ((t + 1) % 64 != 0)
+    s = torch.matmul(fs[0].permute(0, 2, 1, 3).contiguous(),
+                     fs[1].repeat_interleave(G, 2).permute(0, 2, 3, 1).contiguous()) / math.sqrt(D)
+    s = s.masked_fill(~see, float("-inf"))
+    ro = torch.matmul(torch.softmax(s, -1), fs[2].repeat_interleave(G, 2).permute(0, 2, 1, 3).contiguous()).permute(0, 2, 1, 3)
+    rl = torch.logsumexp(s, -1).permute(0, 2, 1)
+    ref = torch.autograd.grad((ro, rl), fs, (d_o.float(), d_lse))
+    for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), (o, lse, *got), (ro, rl, *ref)):
+        err = (a.float() - b).norm() / b.norm()
+        assert err < 1.5e-2, (name, err.item())
