@@ -2519,6 +2519,20 @@ static bool topk_use_split(int B, int L, int N, int h_kv) {
   return fused_wgs < 2L * topk_cus() && N >= 256 && N <= 16384;
 }
 
+// Is the one-pass prefill kernel ahead of one workgroup per row?  The row kernel streams a row's keys for every row:
+// 19 ns a row (its serial chain, two rows per compute unit at a time) or the keys at 9.5 TB/s, whichever is longer.  The
+// one-pass kernel reads the keys once per 4 to 16 queries; up to some thousand rows it takes one wavefront's time,
+// which grows with the chunks.  (us, row / one-pass, at 500 chunks: 1024 rows of 4 heads of 128 28 / 25, 4096 rows 85 / 30,
+// with a key for each of 8 heads 4096 rows of 128 470 / 52; at 1023 chunks 256 rows of 128 14 / 39, 4096 rows 107 / 49, with
+// a key for each of 8 heads 256 rows 54 / 104, 4096 rows 830 / 135.)
+static bool topk_group_ahead(long rows, int N, int G, int D, int per_qhead) {
+  const double key_bytes = (double)N * (per_qhead ? G : 1) * D * 2;
+  const double row_us = 8.0 + rows * (key_bytes > 180e3 ? key_bytes / 9.5e6 : 0.019);
+  const double group_us = per_qhead ? (G > 4 && N > 512 ? 20.0 + N / 14.0 : 20.0 + N / 28.0)
+                                    : (G == 1 ? 16.0 + N / 15.0 : 12.0 + N / 40.0);
+  return group_us < row_us;
+}
+
 // Shapes that hils_topk_fwd_weights hands to the one-pass prefill kernel, the only one that reads
 // lse_swa in bf16 (mirrors the dispatch of topk_fwd_impl; the workspace must be given).
 extern "C" int hils_topk_lse16_covers(int B, int L, int N, int h_kv, int G, int D, int topk) {
@@ -2542,13 +2556,21 @@ static const float* topk_pack_bias(const float* bias, void* workspace, int B, in
   return out;
 }
 
+// many queries: room for the chunk keys repacked into MFMA operand order (head dim up to 128; a key
+// per query head when the caller's keys are per query head)
+// and behind them for an additive bias in blocks of 16 chunks per head
+static size_t topk_ws_packed(int B, int N, int h_kv, int G) {
+  return G <= 8 ? topk_ws_key_bytes(B, N, h_kv, G) + (size_t)B * h_kv * G * ((N + 15) / 16) * 16 * sizeof(float) : 0;
+}
+// what a call cannot do without: few queries may park their logits there
+static size_t topk_ws_least(int B, int L, int N, int h_kv, int G) {
+  return topk_use_split(B, L, N, h_kv) ? (size_t)B * L * h_kv * G * N * sizeof(float) : topk_ws_packed(B, N, h_kv, G);
+}
+
 extern "C" size_t hils_topk_fwd_workspace(int B, int L, int N, int h_kv, int G) {
-  // many queries: room for the chunk keys repacked into MFMA operand order (head dim up to 128; a key
-  // per query head when the caller's keys are per query head)
-  // and behind them for an additive bias in blocks of 16 chunks per head
-  if (!topk_use_split(B, L, N, h_kv))
-    return G <= 8 ? topk_ws_key_bytes(B, N, h_kv, G) + (size_t)B * h_kv * G * ((N + 15) / 16) * 16 * sizeof(float) : 0;
-  return (size_t)B * L * h_kv * G * N * sizeof(float);
+  // (few queries: the dispatch may still come to the one-pass kernel, when the repacked keys fit too)
+  const size_t least = topk_ws_least(B, L, N, h_kv, G), packed = topk_ws_packed(B, N, h_kv, G);
+  return L > 4 && N <= 1024 && packed > least ? packed : least;
 }
 
 static int topk_fwd_split(const void* q, const void* lmks, const float* lse_swa, const float* bias,
@@ -2603,9 +2625,9 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
   HILS_REQUIRE(G <= 16, "hils_topk_fwd: group size %d not supported (max 16)", G);
   HILS_REQUIRE(block_size > 0, "hils_topk_fwd: block_size must be positive");
   HILS_REQUIRE(h_kv <= 65535 && B <= 65535, "hils_topk_fwd: h_kv/B too large for the grid");
-  HILS_REQUIRE(!workspace || workspace_bytes >= hils_topk_fwd_workspace(B, L, N, h_kv, G),
-               "hils_topk_fwd: workspace of %zu bytes is shorter than the %zu bytes hils_topk_fwd_workspace "
-               "returns for this shape", workspace_bytes, hils_topk_fwd_workspace(B, L, N, h_kv, G));
+  HILS_REQUIRE(!workspace || workspace_bytes >= topk_ws_least(B, L, N, h_kv, G),
+               "hils_topk_fwd: workspace of %zu bytes is shorter than the %zu bytes this shape takes at least "
+               "(hils_topk_fwd_workspace)", workspace_bytes, topk_ws_least(B, L, N, h_kv, G));
   hipStream_t st = (hipStream_t)stream;
   HILS_REQUIRE(!lse_bf16 || hils_topk_lse16_covers(B, L, N, h_kv, G, D, topk),
                "hils_topk_fwd_weights_lse16: shape not taken by the one-pass prefill kernel "
@@ -2614,7 +2636,10 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
   // there are enough rows to occupy the machine, however many more there are
   // (with a bias the row kernel's inter-chunk softmax adds that same bias to the winners' scores:
   // it writes the weights only when the caller's prior bias is this bias)
-  if ((topk_use_split(B, L, N, h_kv) || L <= 4) &&
+  const bool group = L > 4 && workspace && workspace_bytes >= topk_ws_packed(B, N, h_kv, G) &&
+                     hils_topk_group_covers(N, G, D, topk, per_qhead, !gumbel && !drop_mask) &&
+                     topk_group_ahead((long)B * L * h_kv, N, G, D, per_qhead);
+  if (!group && (topk_use_split(B, L, N, h_kv) || L <= 4) &&
       topk_use_row((long)B * L * h_kv, N, G, D, per_qhead, !gumbel && !drop_mask, bias != nullptr)) {
     const bool w_here = weights != nullptr && prior_b == bias;
     *weights_fused = w_here;
@@ -2625,7 +2650,7 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
     HILS_CHECK_LAUNCH("hils_topk_fwd");
     return HILS_OK;
   }
-  if (workspace && (D == 64 || D == 128) && topk_use_split(B, L, N, h_kv) &&
+  if (!group && workspace && (D == 64 || D == 128) && topk_use_split(B, L, N, h_kv) &&
       (long)B * L <= 2147483647L / h_kv) {
     if (int rc2 = topk_fwd_split(q, lmks, lse_swa, bias, gumbel, drop_mask, indices, scores, lse_total,
                                  sel_logits, (float*)workspace, B, L, N, h_kv, G, D, topk, block_size,
@@ -2872,7 +2897,7 @@ extern "C" int hils_topk_fwd_noalloc(const void* q, const void* lmks, const floa
                                      int block_size, int window_size, int causal, int q_offset,
                                      int per_qhead, float sm_scale, void* stream) {
   HILS_REQUIRE(B > 0 && L > 0 && N > 0 && h_kv > 0 && G > 0, "hils_topk_fwd_noalloc: sizes must be positive");
-  const size_t need = hils_topk_fwd_workspace(B, L, N, h_kv, G);
+  const size_t need = topk_ws_least(B, L, N, h_kv, G);
   HILS_REQUIRE(need <= HILS_TOPK_SCRATCH_BYTES,
                "hils_topk_fwd_noalloc: this shape needs %zu bytes of scratch, the built-in buffer holds %zu; "
                "use hils_topk_fwd with a caller-allocated workspace",

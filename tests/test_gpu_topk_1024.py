@@ -1,0 +1,57 @@
+"""One-pass selection kernel with 513 to 1024 chunks, and the dispatch between it and one workgroup per row."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,N,h_kv,G,D,topk,perq,bias", [
+    (300, 513, 2, 1, 64, 32, False, False), (700, 1024, 2, 4, 128, 32, False, False), (400, 1000, 1, 2, 64, 7, False, True),
+    (260, 777, 2, 8, 64, 16, False, True), (520, 1023, 1, 6, 128, 32, True, True), (300, 600, 2, 3, 64, 32, True, False),
+    (900, 1024, 4, 8, 64, 32, True, True), (1500, 900, 3, 1, 128, 32, False, True),
+])
+def test_topk_many_chunks(pkg, orc, dev, L, N, h_kv, G, D, topk, perq, bias):
+    gen = torch.Generator(device=dev).manual_seed(N)
+    h_q, S, W = h_kv * G, 64, 512
+    off = N * S - L  # the last queries see all but the window's chunks, the first ones some fewer
+    q = torch.randn(1, L, h_q, D, device=dev, generator=gen).bfloat16()
+    lmk = torch.randn(1, N, h_q if perq else h_kv, D, device=dev, generator=gen).bfloat16()
+    lse = torch.randn(1, L, h_q, device=dev, generator=gen) + 3
+    pb = torch.randn(1, N, h_q, device=dev, generator=gen) if bias else None
+    idx, sc, w = pkg.topk_chunk_weights(q, lmk, lse, topk, S, W, q_offset=off, prior_b=pb, num_kv_heads=h_kv)
+    scale = 1 / math.sqrt(D)
+    kf = (lmk if perq else lmk.repeat_interleave(G, 2)).float()[0].permute(1, 2, 0).contiguous()       # (h_q, D, N)
+    s = torch.matmul(q.float()[0].permute(1, 0, 2).contiguous(), kf) * scale                            # (h_q, L, N)
+    sel = s if pb is None else s + pb[0].t().unsqueeze(1)
+    lim = torch.div(torch.arange(L, device=dev) + off - W + 1, S, rounding_mode="floor").clamp(0, N)
+    vis = torch.arange(N, device=dev) < lim.view(L, 1)
+    sel = sel.masked_fill(~vis, float("-inf"))
+    tot = torch.logaddexp(torch.logsumexp(sel, -1), lse[0].t())                                         # (h_q, L)
+    pooled = (sel - tot.unsqueeze(-1)).view(h_kv, G, L, N).amax(1)                                      # (h_kv, L, N)
+    ref = pooled.topk(topk, -1)
+    assert ((idx[0, :, :, 1:] > idx[0, :, :, :-1]) | (idx[0, :, :, 1:] < 0)).all(), "ascending"
+    got = idx[0].permute(1, 0, 2).long()
+    assert (got >= 0).all() and (got < lim.view(1, L, 1)).all()
+    # the same scores up to rounding: every winner is at least as good as the reference's last, less a rounding
+    worst = pooled.gather(-1, got).amin(-1)
+    assert (worst >= ref.values[..., -1] - 2e-4).all()
+    raw = s.view(h_kv, G, L, N).gather(-1, got.unsqueeze(1).expand(-1, G, -1, -1)).permute(2, 0, 1, 3).reshape(L, h_q, topk)
+    torch.testing.assert_close(sc[0].float(), raw, atol=2e-2, rtol=1e-2)
+    x = sc[0].float()
+    if pb is not None:
+        bw = pb[0].t().view(h_kv, G, 1, N).expand(-1, -1, L, -1).gather(-1, got.unsqueeze(1).expand(-1, G, -1, -1))
+        x = (x + bw.permute(2, 0, 1, 3).reshape(L, h_q, topk).bfloat16().float()).bfloat16().float()
+    wr = torch.softmax(torch.cat([x, lse[0].unsqueeze(-1)], -1), -1)
+    torch.testing.assert_close(w[0].float(), wr, atol=1e-2, rtol=2e-2)
+
+
+def test_equal_scores_past_512_chunks(pkg, dev):
+    """All scores equal: the lowest chunks win, also through the search over all scores."""
+    L, N, D = 600, 1024, 64
+    q = torch.zeros(1, L, 4, D, device=dev).bfloat16()
+    lmk = torch.randn(1, N, 1, D, device=dev).bfloat16()
+    lse = torch.zeros(1, L, 4, device=dev)
+    idx, _, _ = pkg.topk_chunk_weights(q, lmk, lse, 32, 64, 1, q_offset=N * 64 - L)
+    assert torch.equal(idx, torch.arange(32, device=dev, dtype=torch.int32).expand_as(idx))
