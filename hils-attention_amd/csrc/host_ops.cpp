@@ -838,8 +838,9 @@ struct LogzFn : torch::autograd::Function<LogzFn> {
     const float scale = (float)ctx->saved_data["scale"].toDouble();
     HILS_CALL(hils_chunk_logz_bwd_dq, cptr(q), cptr(k), fptr(z), fptr(dz), mptr(dq), B, L, HQ, H, D, i32(cfg[0]),
               i32(cfg[1]), scale);
-    HILS_CALL(hils_chunk_logz_bwd_dk, cptr(q), cptr(k), fptr(z), fptr(dz), mptr(dk), B, L, HQ, H, D, i32(cfg[0]),
-              i32(cfg[1]), scale);
+    const Tensor ws = workspace(hils_chunk_logz_bwd_dk_workspace(B, L, HQ, H, D, i32(cfg[0]), i32(cfg[1])), q);
+    HILS_CALL(hils_chunk_logz_bwd_dk_ws, cptr(q), cptr(k), fptr(z), fptr(dz), mptr(dk), B, L, HQ, H, D, i32(cfg[0]),
+              i32(cfg[1]), scale, mptr(ws), bytes(ws));
     return {dq, dk, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };

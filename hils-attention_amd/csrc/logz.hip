@@ -72,18 +72,26 @@ logz_fwd_simple(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 // in-lane reduction plus one row-swap reduction.
 #define LZM_RT 2  // 16-row tiles per wavefront
 
-// Workgroup order of the matrix-core kernels: one-dimensional grids in which all blocks of a
+// Workgroup order of the matrix-core kernels: one-dimensional grids in which the blocks of a
 // (batch, KV head) unit run on one XCD (the hardware hands consecutive workgroup ids to the 8 XCDs in
-// turn: id -> (xcd, slot); unit = 8 * (slot / n_blk) + xcd), so that the keys (or query rows) the
-// unit's workgroups stream are fetched into one L2 once instead of into all eight.  False for the
-// padding ids of a unit count that is not a multiple of 8.
-__device__ __forceinline__ bool lz_xcd_unit(int n_blk, int n_unit, int& unit, int& blk) {
-  const int xcd = (int)(blockIdx.x % 8), slot = (int)(blockIdx.x / 8);
-  unit = (slot / n_blk) * 8 + xcd;
-  blk = slot % n_blk;
-  return unit < n_unit;
+// turn: id -> (xcd, slot)), so that the keys (or query rows) the unit's workgroups stream are fetched into
+// one L2 once instead of into all eight.  A unit count that is no multiple of 8 has its blocks dealt out to
+// 2, 4 or 8 XCDs in turn, so that all of them work (two units on two XCDs left three quarters of the chip
+// idle).  False for padding ids.
+__host__ __device__ __forceinline__ int lz_units_apart(int n_unit) {  // units that run side by side
+  return (n_unit & 7) == 0 ? 8 : (n_unit & 3) == 0 ? 4 : (n_unit & 1) == 0 ? 2 : 1;
 }
-static dim3 lz_xcd_grid(int n_blk, int n_unit) { return dim3((unsigned)(8 * ((n_unit + 7) / 8) * n_blk)); }
+__device__ __forceinline__ bool lz_xcd_unit(int n_blk, int n_unit, int& unit, int& blk) {
+  const int g = lz_units_apart(n_unit), m = 8 / g, per = (n_blk + m - 1) / m;
+  const int xcd = (int)(blockIdx.x % 8), slot = (int)(blockIdx.x / 8);
+  unit = (slot / per) * g + xcd / m;
+  blk = (slot % per) * m + xcd % m;
+  return blk < n_blk;
+}
+static dim3 lz_xcd_grid(int n_blk, int n_unit) {
+  const int g = lz_units_apart(n_unit), m = 8 / g;
+  return dim3((unsigned)(8l * (n_unit / g) * ((n_blk + m - 1) / m)));
+}
 // (the occupancy hint also keeps the score accumulators in ordinary registers: without it the
 // compiler, free to use 512 registers at this workgroup size, parks them in accumulation registers
 // and copies every score back for the softmax)
@@ -352,12 +360,28 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 }
 
 // dK: a workgroup owns two chunks (wavefront: 32 tokens of one chunk), the score rows of the
-// queries behind them stream in tiles of 64 rows (64/G queries x G heads).
+// queries behind them stream in tiles of 64 rows (64/G queries x G heads).  The first chunks have the whole
+// sequence behind them, the last ones nothing: walks are cut into segments of about equal length whose fp32
+// sums logz_bwd_dk_sum adds up.  With one workgroup per pair of chunks the kernel ran as long as the first
+// pair's walk: L 8192, 32/8 heads of 128: 1010 us, in segments 880 us; forward and both gradients at L 3532,
+// 16/2 heads of 64: 707 us, in segments and with the units dealt out to all XCDs 202 us.
+struct LzSeg {
+  int target;   // tiles of a segment, about
+  int max_seg;  // segments of the longest walk (1: no walk is cut)
+};
+__host__ __device__ __forceinline__ int lz_tile0(int pair, int W, int QT) {  // first tile behind a pair's first chunk
+  const int t = (2 * pair + 1) * 64 + W - 1;
+  return t < 0 ? 0 : t / QT;
+}
+__host__ __device__ __forceinline__ int lz_nseg(int len, const LzSeg& sg) {
+  int n = len > 0 ? (len + sg.target / 2) / sg.target : 1;
+  return n < 1 ? 1 : (n > sg.max_seg ? sg.max_seg : n);
+}
 template <int D, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  const float* __restrict__ log_z, const float* __restrict__ d_log_z,
-                 bf16_t* __restrict__ dk, LzDims dm, int n_pair, int n_unit) {
+                 bf16_t* __restrict__ dk, LzDims dm, int n_pair, int n_unit, LzSeg sg, float* __restrict__ part) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int QT = 64 / G;  // queries per streamed tile
   constexpr int PITCH = D * 2 + 16;
@@ -374,9 +398,12 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   // (the hardware hands consecutive workgroup ids to the 8 XCDs in turn: id -> (xcd, slot)), whose L2
   // then serves all but the first reader of a tile.  Walking forward from different starting points
   // in the hardware's order, every read of a tile missed (L2 hit rate 2 %, the kernel waiting on
-  // HBM latency at one wavefront per SIMD).  The chunk pairs of a unit come longest walk first.
+  // HBM latency at one wavefront per SIMD).  The chunk pairs of a unit come longest walk first; of the
+  // segments the last ones (which only long walks have) start first, so that the short walks fill the end.
   int unit, pair;
-  if (!lz_xcd_unit(n_pair, n_unit, unit, pair)) return;
+  if (!lz_xcd_unit(n_pair * sg.max_seg, n_unit, unit, pair)) return;
+  const int seg_i = sg.max_seg - 1 - pair / n_pair;
+  pair %= n_pair;
   const int c0 = 2 * pair, ch = wave >> 1;
   const int hk = unit % dm.H;
   const long b = unit / dm.H;
@@ -392,10 +419,15 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     for (int ks = 0; ks < KS; ++ks) ka[tt][ks] = *(const bf16x8_t*)(kp + ks * 32);
   }
   // first query with chunk c0 fully behind its window, rounded down to a tile
-  int t_first = (c0 + 1) * 64 + dm.W - 1;
-  if (t_first < 0) t_first = 0;
-  const int tile0 = t_first / QT;
-  const int n_tiles = (dm.L + QT - 1) / QT;
+  int tile0 = lz_tile0(pair, dm.W, QT);
+  int n_tiles = (dm.L + QT - 1) / QT;
+  const int n_seg = lz_nseg(n_tiles - tile0, sg);
+  if (seg_i >= n_seg) return;
+  if (n_seg > 1) {  // segment 0 has the last tiles
+    const int len = n_tiles - tile0, hi = n_tiles;
+    n_tiles = hi - (int)((long)len * seg_i / n_seg);
+    tile0 = hi - (int)((long)len * (seg_i + 1) / n_seg);
+  }
   const float sc2 = dm.sm_scale * HILS_LOG2E;
 
   const int seg = tid % SEGS, rp0 = tid / SEGS;
@@ -480,6 +512,16 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     stash();
     __syncthreads();
   }
+  if (n_seg > 1) {
+    float* out = part + (((long)unit * n_pair + pair) * sg.max_seg + seg_i) * (128 * D);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) out[(wave * 32 + tt * 16 + 4 * j + i) * D + dt * 16 + col] = acc[tt][dt][i];
+    return;
+  }
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -490,6 +532,32 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) out[dt * 16] = f2bf(acc[tt][dt][i]);
     }
+}
+
+// the segments of the cut walks, in order; four features per thread
+__global__ void __launch_bounds__(256)
+logz_bwd_dk_sum(const float* __restrict__ part, bf16_t* __restrict__ dk, LzDims dm, int n_pair, LzSeg sg) {
+  const int pair = blockIdx.x % n_pair, unit = blockIdx.x / n_pair, QT = 64 / dm.G, D = dm.D;
+  const int n_seg = lz_nseg((dm.L + QT - 1) / QT - lz_tile0(pair, dm.W, QT), sg);
+  if (n_seg == 1) return;
+  const int hk = unit % dm.H;
+  const long b = unit / dm.H;
+  const f32x4_t* src = (const f32x4_t*)(part + ((long)unit * n_pair + pair) * sg.max_seg * (128 * D));
+  const int n = 128 * D / 4;
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < n; i += gridDim.y * 256) {
+    const int t = i / (D / 4), f = (i - t * (D / 4)) * 4, tok = pair * 128 + t;
+    if (tok >= dm.L) break;
+    f32x4_t x = src[i];
+    for (int s = 1; s < n_seg; ++s) {
+      const f32x4_t y = src[(long)s * n + i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] += y[e];
+    }
+    uint2 pk;
+    pk.x = pack_bf2(x[0], x[1]);
+    pk.y = pack_bf2(x[2], x[3]);
+    *(uint2*)(dk + ((b * dm.L + tok) * (long)dm.H + hk) * D + f) = pk;
+  }
 }
 
 // dq[b,t,hq,:] = sum_c sum_j dlz[c] * exp(s_j - lz[c]) * scale * k_j
@@ -652,7 +720,7 @@ extern "C" int hils_chunk_logz_fwd(const void* q, const void* k, float* log_z, i
   if (lz_mfma_covers(G, D, S, H, B)) {
     const int QB = 4 * 16 * LZM_RT / G;
     const int n_qt = (L + QB - 1) / QB;
-    HILS_REQUIRE(((long)B * H + 7) / 8 * 8 * n_qt < (1L << 31), "hils_chunk_logz_fwd: B * H * L too large for the grid");
+    HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_fwd: B * H * L too large for the grid");
     const dim3 grid = lz_xcd_grid(n_qt, B * H);
 #define LZ_LAUNCH(DD, GG)                                                                      \
   hipLaunchKernelGGL((logz_fwd_mfma<DD, GG>), grid, dim3(256), 0, (hipStream_t)stream,         \
@@ -680,7 +748,7 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
     const int G = HQ / H;
     const int QB = 4 * 16 * LZM_RT / G;
     const int n_qt = (L + QB - 1) / QB;
-    HILS_REQUIRE(((long)B * H + 7) / 8 * 8 * n_qt < (1L << 31), "hils_chunk_logz_bwd_dq: B * H * L too large for the grid");
+    HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_bwd_dq: B * H * L too large for the grid");
     const dim3 grid = lz_xcd_grid(n_qt, B * H);
 #define LZ_LAUNCH(DD, GG)                                                                      \
   hipLaunchKernelGGL((logz_bwd_dq_mfma<DD, GG>), grid, dim3(256), 0, (hipStream_t)stream,      \
@@ -697,9 +765,34 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   return HILS_OK;
 }
 
-extern "C" int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float* log_z,
-                                      const float* d_log_z, void* dk, int B, int L, int HQ, int H,
-                                      int D, int S, int window, float sm_scale, void* stream) {
+// Segments of the dK walks: with two workgroups per compute unit (what registers allow) about 1.6 times as
+// many items as fit at once, in segments no shorter than eight tiles (a partial result is as many bytes as four).
+static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
+  const int n_pair = (N + 1) / 2, QT = 64 / G, n_tiles = (L + QT - 1) / QT;
+  long total = 0;
+  for (int p = 0; p < n_pair; ++p) {
+    const int len = n_tiles - lz_tile0(p, W, QT);
+    if (len <= 0) break;
+    total += len;
+  }
+  const int longest = n_tiles - lz_tile0(0, W, QT);
+  long target = total * B * H / (3L * hils_device_cus());
+  if (target < 8) target = 8;
+  LzSeg sg{(int)(target < (1 << 30) ? target : (1 << 30)), 1 << 30};
+  sg.max_seg = lz_nseg(longest, sg);
+  return sg;
+}
+extern "C" size_t hils_chunk_logz_bwd_dk_workspace(int B, int L, int HQ, int H, int D, int S, int window) {
+  if (B <= 0 || L <= 0 || H <= 0 || HQ <= 0 || HQ % H != 0 || !lz_mfma_covers(HQ / H, D, S, H, B)) return 0;
+  const int N = (L + S - 1) / S;
+  const LzSeg sg = lz_segments(B, L, HQ / H, H, N, window);
+  return sg.max_seg == 1 ? 0 : (size_t)B * H * ((N + 1) / 2) * sg.max_seg * 128 * D * sizeof(float);
+}
+
+extern "C" int hils_chunk_logz_bwd_dk_ws(const void* q, const void* k, const float* log_z,
+                                         const float* d_log_z, void* dk, int B, int L, int HQ, int H,
+                                         int D, int S, int window, float sm_scale, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
   HILS_REQUIRE(q && k && log_z && d_log_z && dk, "hils_chunk_logz_bwd_dk: null pointer");
   if (int rc = lz_check("hils_chunk_logz_bwd_dk", B, L, HQ, H, D, S)) return rc;
   const int G = HQ / H;
@@ -707,14 +800,21 @@ extern "C" int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float*
   LzDims dm{L, HQ, H, G, D, S, window, (L + S - 1) / S, 0, sm_scale};
   if (lz_mfma_covers(G, D, S, H, B)) {
     const int n_pair = (dm.N + 1) / 2;
-    HILS_REQUIRE(((long)B * H + 7) / 8 * 8 * n_pair < (1L << 31), "hils_chunk_logz_bwd_dk: B * H * N too large for the grid");
+    HILS_REQUIRE(((long)B * H + 8) * (n_pair + 8) * 8 < (1L << 31), "hils_chunk_logz_bwd_dk: B * H * N too large for the grid");
     const int n_unit = B * H;
-    const dim3 grid = lz_xcd_grid(n_pair, n_unit);
+    const LzSeg sg = workspace ? lz_segments(B, L, G, H, dm.N, window) : LzSeg{1 << 30, 1};
+    HILS_REQUIRE(sg.max_seg == 1 || workspace_bytes >= (size_t)n_unit * n_pair * sg.max_seg * 128 * D * sizeof(float),
+                 "hils_chunk_logz_bwd_dk: the workspace is too short (%zu bytes)", workspace_bytes);
+    const dim3 grid = lz_xcd_grid(n_pair * sg.max_seg, n_unit);
 #define LZ_LAUNCH(DD, GG)                                                                      \
   hipLaunchKernelGGL((logz_bwd_dk_mfma<DD, GG>), grid, dim3(256), 0, (hipStream_t)stream,      \
-                     (const bf16_t*)q, (const bf16_t*)k, log_z, d_log_z, (bf16_t*)dk, dm, n_pair, n_unit)
+                     (const bf16_t*)q, (const bf16_t*)k, log_z, d_log_z, (bf16_t*)dk, dm, n_pair, n_unit, sg, \
+                     (float*)workspace)
     LZ_DISPATCH(D, G);
 #undef LZ_LAUNCH
+    if (sg.max_seg > 1)
+      hipLaunchKernelGGL(logz_bwd_dk_sum, dim3((unsigned)(n_pair * n_unit), 4), dim3(256), 0, (hipStream_t)stream,
+                         (const float*)workspace, (bf16_t*)dk, dm, n_pair, sg);
     HILS_CHECK_LAUNCH("hils_chunk_logz_bwd_dk");
     return HILS_OK;
   }
@@ -729,4 +829,10 @@ extern "C" int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float*
                      (bf16_t*)dk, dm);
   HILS_CHECK_LAUNCH("hils_chunk_logz_bwd_dk");
   return HILS_OK;
+}
+
+extern "C" int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float* log_z,
+                                      const float* d_log_z, void* dk, int B, int L, int HQ, int H,
+                                      int D, int S, int window, float sm_scale, void* stream) {
+  return hils_chunk_logz_bwd_dk_ws(q, k, log_z, d_log_z, dk, B, L, HQ, H, D, S, window, sm_scale, nullptr, 0, stream);
 }

@@ -46,6 +46,8 @@ SIGNATURES = {
     "hils_chunk_logz_fwd": [_P, _P, _P] + [_I] * 7 + [_F, _I, _P],
     "hils_chunk_logz_bwd_dq": [_P] * 5 + [_I] * 7 + [_F, _P],
     "hils_chunk_logz_bwd_dk": [_P] * 5 + [_I] * 7 + [_F, _P],
+    "hils_chunk_logz_bwd_dk_workspace": [_I] * 7,
+    "hils_chunk_logz_bwd_dk_ws": [_P] * 5 + [_I] * 7 + [_F, _P, _Z, _P],
     "hils_rope": [_P] * 4 + [_I] * 7 + [_F, _P],
     "hils_norm_rope_pool_fwd": [_P] * 6 + [_I] * 6 + [_F, _P],
     "hils_norm_rope_pool_bwd": [_P] * 8 + [_I] * 6 + [_F, _P],

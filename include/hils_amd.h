@@ -354,6 +354,12 @@ int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float* log_z, con
 int hils_chunk_logz_bwd_dk(const void* q, const void* k, const float* log_z, const float* d_log_z,
                            void* dk, int B, int L, int HQ, int H, int D, int S, int window,
                            float sm_scale, void* stream);
+/* The same with a workspace of hils_chunk_logz_bwd_dk_workspace(...) bytes (0: none is of use): the queries behind
+ * the first chunks are split over workgroups whose sums meet there. */
+size_t hils_chunk_logz_bwd_dk_workspace(int B, int L, int HQ, int H, int D, int S, int window);
+int hils_chunk_logz_bwd_dk_ws(const void* q, const void* k, const float* log_z, const float* d_log_z,
+                              void* dk, int B, int L, int HQ, int H, int D, int S, int window,
+                              float sm_scale, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- sliding-window attention of the local branch ------------------------------- */
 
