@@ -94,9 +94,12 @@ static dim3 lz_xcd_grid(int n_blk, int n_unit) {
 }
 // (the occupancy hint also keeps the score accumulators in ordinary registers: without it the
 // compiler, free to use 512 registers at this workgroup size, parks them in accumulation registers
-// and copies every score back for the softmax)
+// and copies every score back for the softmax; its upper bound keeps the scheduler from saving registers for
+// wavefronts that do not fit anyway, one LDS read and its wait behind the other)
+// Bound by vector-ALU issue: 207 vector instructions per 32 x 64 scores with a maximum per chunk and addresses worked
+// out per load, about 115 now; L 8192, 32/8 heads of 128: 390 -> 341 us.
 template <int D, int G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
               float* __restrict__ log_z, LzDims dm, int n_qt, int n_unit) {
   constexpr int KS = D / 32;
@@ -139,13 +142,16 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   // is kept in scratch memory by the compiler)
   typedef unsigned lz_u32x4 __attribute__((ext_vector_type(4)));
   lz_u32x4 kr[NP];
-  auto fetch = [&](int c) {
+  // uniform base per chunk, lane offsets fixed: no address arithmetic per chunk (a quarter of the vector
+  // instructions of a chunk when it was worked out each time)
+  const bf16_t* const k_unit = k + (b * dm.L * (long)dm.H + hk) * D;
+  unsigned k_off[NP];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int p = tid + 256 * i;
-      const int tok = p / (D / 8), seg = p % (D / 8);
-      kr[i] = *(const lz_u32x4*)(k + ((b * dm.L + c * 64 + tok) * (long)dm.H + hk) * D + seg * 8);
-    }
+  for (int i = 0; i < NP; ++i) k_off[i] = (unsigned)((tid + 256 * i) / (D / 8) * (dm.H * D) + (tid + 256 * i) % (D / 8) * 8);
+  auto fetch = [&](int c) {
+    const bf16_t* kc = k_unit + (long)c * 64 * dm.H * D;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) kr[i] = *(const lz_u32x4*)(kc + k_off[i]);
   };
   auto stash = [&](int buf) {
 #pragma unroll
@@ -161,8 +167,12 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
   __syncthreads();
   float keep[LZM_RT];
+  float ref[LZM_RT];  // reference point of the exponentials: the last chunk's log sum (log2 units)
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt) keep[rt] = HILS_NEG_INF;
+  for (int rt = 0; rt < LZM_RT; ++rt) {
+    keep[rt] = HILS_NEG_INF;
+    ref[rt] = 0.f;
+  }
   for (int c = 0; c < nc; ++c) {
     fetch(c + 1 < nc ? c + 1 : c);
     const unsigned char* kb = k_s[c & 1];
@@ -182,23 +192,34 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       }
 #pragma unroll
     for (int rt = 0; rt < LZM_RT; ++rt) {
-      // the maximum is taken over the raw products (the scale is positive) and the scale is applied
-      // inside the exponent's fused multiply-add: no separate scaling pass
+      // The reference point need not be the maximum: fp32 keeps its relative precision as long as the sum
+      // neither overflows nor sinks so low that terms near its own size are flushed.  The previous chunk's log sum
+      // serves nearly always; a sum out of [2^-60, 2^60] anywhere in the wavefront takes the maximum instead
+      // (the maximum of every chunk was a sixth of the vector instructions).  The scale is applied inside the
+      // exponent's fused multiply-add.
       float x[16];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[tt * 4 + i] = acc[rt][tt][i];
       if (dm.mask_lmk && j == 3) x[15] = HILS_NEG_INF;  // token 63 = tile 3, lane row 3, register 3
-      float m = fmaxf(x[0], x[1]);
-#pragma unroll
-      for (int i = 2; i < 16; i += 2) m = fmaxf(fmaxf(m, x[i]), x[i + 1]);
-      m = rows_max(m) * sc2;  // in log2 units, as the sum below
-      float s = 0.f;
+      float s = 0.f, m = ref[rt];
 #pragma unroll
       for (int i = 0; i < 16; ++i) s += __builtin_amdgcn_exp2f(fmaf(x[i], sc2, -m));
       s = rows_sum(s);
-      const float val = (c < lim[rt]) ? (m + __builtin_amdgcn_logf(s)) * HILS_LN2 : HILS_NEG_INF;
+      if (__any(!(s > 0x1p-60f && s < 0x1p60f))) {
+        m = fmaxf(x[0], x[1]);
+#pragma unroll
+        for (int i = 2; i < 16; i += 2) m = fmaxf(fmaxf(m, x[i]), x[i + 1]);
+        m = rows_max(m) * sc2;  // in log2 units, as the sum below
+        s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s += __builtin_amdgcn_exp2f(fmaf(x[i], sc2, -m));
+        s = rows_sum(s);
+      }
+      const float lse2 = m + __builtin_amdgcn_logf(s);
+      ref[rt] = lse2;
+      const float val = (c < lim[rt]) ? lse2 * HILS_LN2 : HILS_NEG_INF;
       if (j == (c & 3)) keep[rt] = val;
     }
     if ((c & 3) == 3 || c == nc - 1) {
@@ -225,24 +246,25 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 //   dQ = dS K,   dK = dS^T Q.
 // One side of the product is OWNED by a wavefront (32 rows, held in registers as matrix operands,
 // with the fp32 gradient accumulators), the other side STREAMS through LDS in 64-row tiles, stored
-// twice: row-major (operand of the score product) and transposed (operand of the gradient
-// product, whose contraction runs over the streamed rows).  The scores are computed with the
+// row-major and double-buffered: the operand of the score product is a row read, that of the gradient product
+// (whose contraction runs over the streamed rows) comes through the transposing LDS load.  With a second, transposed
+// copy in LDS a tile took 16 lane permutations, 8 more stores and two barriers; L 8192, 32/8 heads of 128: dQ
+// 715 -> 530 us, dK 840 -> 635 us; what is left is vector-ALU and matrix
+// issue, 128 .. 150 vector instructions beside 64 matrix ones per tile.
+// The scores are computed with the
 // owned side as matrix columns, so their accumulator registers are already the left operand of
 // the gradient product.
 // dQ: a wavefront owns 32 score rows (query x head), the chunks' keys stream.
 template <int D, int G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  const float* __restrict__ log_z, const float* __restrict__ d_log_z,
                  bf16_t* __restrict__ dq, LzDims dm, int n_qt, int n_unit) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int QW = 16 * LZM_RT / G, QB = 4 * QW;
   constexpr int PITCH = D * 2 + 16;
-  constexpr int SEGS = D / 8;            // 16-byte pieces per row
-  constexpr int PPP = 256 / SEGS;        // row pairs per pass of the workgroup
-  constexpr int NPASS = 32 / PPP;
-  __shared__ __align__(16) unsigned char k_s[64 * PITCH];
-  __shared__ __align__(16) unsigned char kt_s[D * LZM_PT];
+  constexpr int NP = D / 32;  // 16-byte pieces of a chunk per thread
+  __shared__ __align__(16) unsigned char k_s[2][64 * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   int unit, qt;
@@ -271,21 +293,21 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   const int nc = lz_limit(dm, t_last);
   const float sc2 = dm.sm_scale * HILS_LOG2E;
 
-  const int seg = tid % SEGS, rp0 = tid / SEGS;
-  uint4 kr[NPASS][2];
+  typedef unsigned lz_u32x4 __attribute__((ext_vector_type(4)));
+  lz_u32x4 kr[NP];
+  const bf16_t* const k_unit = k + (b * dm.L * (long)dm.H + hk) * D;
+  unsigned k_off[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) k_off[i] = (unsigned)((tid + 256 * i) / (D / 8) * (dm.H * D) + (tid + 256 * i) % (D / 8) * 8);
   auto fetch = [&](int c) {
+    const bf16_t* kc = k_unit + (long)c * 64 * dm.H * D;
 #pragma unroll
-    for (int i = 0; i < NPASS; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int tok = 2 * (rp0 + PPP * i) + h;
-        kr[i][h] = *(const uint4*)(k + ((b * dm.L + c * 64 + tok) * (long)dm.H + hk) * D + seg * 8);
-      }
+    for (int i = 0; i < NP; ++i) kr[i] = *(const lz_u32x4*)(kc + k_off[i]);
   };
-  auto stash = [&]() {
+  auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NPASS; ++i)
-      lzm_stash_pair<PITCH>(k_s, kt_s, 2 * (rp0 + PPP * i), seg, kr[i][0], kr[i][1]);
+    for (int i = 0; i < NP; ++i)
+      *(lz_u32x4*)(&k_s[buf][(tid + 256 * i) / (D / 8) * PITCH + (tid + 256 * i) % (D / 8) * 16]) = kr[i];
   };
   f32x4_t acc[LZM_RT][DT];
 #pragma unroll
@@ -293,20 +315,26 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float lzn[LZM_RT], dln[LZM_RT];
+  unsigned z_off[LZM_RT];  // of the lane's row behind the first row of the workgroup's first query
+  const long z_first = (b * dm.L + qt * QB) * (long)dm.HQ * dm.N;
+#pragma unroll
+  for (int rt = 0; rt < LZM_RT; ++rt) z_off[rt] = (unsigned)(orow[rt] * dm.N - z_first);
   auto fetch_z = [&](int c) {
+    const float *zc = log_z + z_first + c, *dc = d_log_z + z_first + c;
 #pragma unroll
     for (int rt = 0; rt < LZM_RT; ++rt) {
-      lzn[rt] = log_z[orow[rt] * dm.N + c];
-      dln[rt] = d_log_z[orow[rt] * dm.N + c];
+      lzn[rt] = zc[z_off[rt]];
+      dln[rt] = dc[z_off[rt]];
     }
   };
   if (nc > 0) {
     fetch(0);
     fetch_z(0);
-    stash();
+    stash(0);
   }
   __syncthreads();
   for (int c = 0; c < nc; ++c) {
+    const unsigned char* kb = k_s[c & 1];
     float off[LZM_RT], coef[LZM_RT];
 #pragma unroll
     for (int rt = 0; rt < LZM_RT; ++rt) {
@@ -317,6 +345,7 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     const int cn = c + 1 < nc ? c + 1 : c;
     fetch(cn);
     fetch_z(cn);
+    __builtin_amdgcn_sched_barrier(0);  // (the loads would sink to their stores into LDS)
     float p[LZM_RT][4][4];
     {
       f32x4_t st[LZM_RT][4];
@@ -328,7 +357,7 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(k_s + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(kb + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
 #pragma unroll
           for (int rt = 0; rt < LZM_RT; ++rt)
             st[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], st[rt][tt], 0, 0, 0);
@@ -341,9 +370,8 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
           for (int i = 0; i < 4; ++i)
             p[rt][tt][i] = __builtin_amdgcn_exp2f(st[rt][tt][i] * sc2 - off[rt]) * coef[rt];
     }
-    lzm_grad_product<D, LZM_RT>(kt_s, p, acc, col, j);
-    __syncthreads();
-    stash();
+    lzm_grad_product_rows<D, LZM_RT, PITCH>(kb, p, acc, col, j);
+    stash((c + 1) & 1);
     __syncthreads();
   }
 #pragma unroll
@@ -378,18 +406,17 @@ __host__ __device__ __forceinline__ int lz_nseg(int len, const LzSeg& sg) {
   return n < 1 ? 1 : (n > sg.max_seg ? sg.max_seg : n);
 }
 template <int D, int G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
 logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  const float* __restrict__ log_z, const float* __restrict__ d_log_z,
                  bf16_t* __restrict__ dk, LzDims dm, int n_pair, int n_unit, LzSeg sg, float* __restrict__ part) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int QT = 64 / G;  // queries per streamed tile
   constexpr int PITCH = D * 2 + 16;
-  constexpr int SEGS = D / 8, PPP = 256 / SEGS, NPASS = 32 / PPP;
-  __shared__ __align__(16) unsigned char q_s[64 * PITCH];
-  __shared__ __align__(16) unsigned char qt_s[D * LZM_PT];
-  __shared__ __align__(16) float off_s[2][64];
-  __shared__ __align__(16) float coef_s[2][64];
+  constexpr int NP = D / 32;  // 16-byte pieces of a tile per thread
+  __shared__ __align__(16) unsigned char q_s[2][64 * PITCH];
+  __shared__ __align__(16) float off_s[2][2][64];
+  __shared__ __align__(16) float coef_s[2][2][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   // Workgroup order.  The workgroups of one (batch, KV head) stream the same query rows, each from the
@@ -430,41 +457,46 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
   const float sc2 = dm.sm_scale * HILS_LOG2E;
 
-  const int seg = tid % SEGS, rp0 = tid / SEGS;
-  uint4 qr[NPASS][2];
+  // staging: a uniform base per tile and fixed lane offsets; only the sequence's last tile may reach past its end,
+  // and its rows there read the last query again (their coefficients are 0)
+  typedef unsigned lz_u32x4 __attribute__((ext_vector_type(4)));
+  lz_u32x4 qr[NP];
   float zo = 0.f, zc = 0.f;  // raw log_z and d_log_z of this thread's (row, chunk); zin: inside the limits
   bool zin = false;
-  auto fetch = [&](int tile) {
+  const long q_row = (long)dm.HQ * D, z_row = (long)dm.HQ * dm.N;  // of one query
+  const bf16_t* const q_unit = q + b * dm.L * q_row + hk * G * D;
+  const float* const z_unit = log_z + b * dm.L * z_row + (long)hk * G * dm.N;
+  const float* const dz_unit = d_log_z + b * dm.L * z_row + (long)hk * G * dm.N;
+  const int z_r = tid & 63, z_c = c0 + (tid >> 6 & 1);  // row and chunk of this thread's coefficient (the first 128)
+  const int z_cc = z_c < dm.N ? z_c : dm.N - 1;
+  const int z_t0 = z_c < dm.N ? (z_c + 1) * 64 + dm.W - 1 : 0x7fffffff;  // first query with the chunk behind its window
+  auto fetch = [&](int tile) __attribute__((always_inline)) {
+    const int last = dm.L - 1 - tile * QT;  // last query of the sequence, counted from the tile's first
+    const bf16_t* qc = q_unit + (long)tile * QT * q_row;
 #pragma unroll
-    for (int i = 0; i < NPASS; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 2 * (rp0 + PPP * i) + h;
-        int t = tile * QT + row / G;
-        if (t > dm.L - 1) t = dm.L - 1;
-        qr[i][h] = *(const uint4*)(q + ((b * dm.L + t) * (long)dm.HQ + hk * G + row % G) * D + seg * 8);
-      }
+    for (int i = 0; i < NP; ++i) {
+      const int row = (tid + 256 * i) / (D / 8);
+      const int t = row / G < last ? row / G : last;
+      qr[i] = *(const lz_u32x4*)(qc + (unsigned)((t * dm.HQ + row % G) * D + (tid + 256 * i) % (D / 8) * 8));
+    }
     if (tid < 128) {
-      const int row = tid & 63, cc = c0 + (tid >> 6);
-      const int t = tile * QT + row / G;
-      const bool in = t < dm.L && cc < dm.N && cc < lz_limit(dm, t < dm.L ? t : 0);
-      const long zi = ((b * dm.L + (t < dm.L ? t : dm.L - 1)) * (long)dm.HQ + hk * G + row % G) * dm.N +
-                      (cc < dm.N ? cc : dm.N - 1);
       // raw values: what a row outside the limits gets is decided in stash(), so that nothing
       // here waits for a load (which would also wait for the query rows issued before it)
-      zo = log_z[zi];
-      zc = d_log_z[zi];
-      zin = in;
+      const int tr = z_r / G, t = tr < last ? tr : last;
+      const unsigned zi = (unsigned)((t * dm.HQ + z_r % G) * dm.N + z_cc);
+      zo = (z_unit + (long)tile * QT * z_row)[zi];
+      zc = (dz_unit + (long)tile * QT * z_row)[zi];
+      zin = tr <= last && tile * QT + tr >= z_t0;
     }
   };
-  auto stash = [&]() {
+  auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NPASS; ++i)
-      lzm_stash_pair<PITCH>(q_s, qt_s, 2 * (rp0 + PPP * i), seg, qr[i][0], qr[i][1]);
+    for (int i = 0; i < NP; ++i)
+      *(lz_u32x4*)(&q_s[buf][(tid + 256 * i) / (D / 8) * PITCH + (tid + 256 * i) % (D / 8) * 16]) = qr[i];
     if (tid < 128) {
       const bool ok = zin && zo > -1e30f;
-      off_s[tid >> 6][tid & 63] = ok ? zo * HILS_LOG2E : 0.f;
-      coef_s[tid >> 6][tid & 63] = ok ? zc * dm.sm_scale : 0.f;
+      off_s[buf][tid >> 6][tid & 63] = ok ? zo * HILS_LOG2E : 0.f;
+      coef_s[buf][tid >> 6][tid & 63] = ok ? zc * dm.sm_scale : 0.f;
     }
   };
   f32x4_t acc[2][DT];
@@ -474,11 +506,13 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     for (int dt = 0; dt < DT; ++dt) acc[tt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if (tile0 < n_tiles) {
     fetch(n_tiles - 1);
-    stash();
+    stash(0);
   }
   __syncthreads();
-  for (int tile = n_tiles - 1; tile >= tile0; --tile) {
+  for (int tile = n_tiles - 1, buf = 0; tile >= tile0; --tile, buf ^= 1) {
     fetch(tile > tile0 ? tile - 1 : tile);
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* qb = q_s[buf];
     float p[2][4][4];  // [owned token tile][streamed row tile][row 4j+i]
     {
       f32x4_t st[2][4];
@@ -490,15 +524,15 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       for (int rr = 0; rr < 4; ++rr)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(q_s + (rr * 16 + col) * PITCH + ks * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(qb + (rr * 16 + col) * PITCH + ks * 64 + j * 16);
 #pragma unroll
           for (int tt = 0; tt < 2; ++tt)
             st[tt][rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ka[tt][ks], st[tt][rr], 0, 0, 0);
         }
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float4 o4 = *(const float4*)&off_s[ch][rr * 16 + 4 * j];
-        const float4 c4 = *(const float4*)&coef_s[ch][rr * 16 + 4 * j];
+        const float4 o4 = *(const float4*)&off_s[buf][ch][rr * 16 + 4 * j];
+        const float4 c4 = *(const float4*)&coef_s[buf][ch][rr * 16 + 4 * j];
         const float o[4] = {o4.x, o4.y, o4.z, o4.w}, cf[4] = {c4.x, c4.y, c4.z, c4.w};
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
@@ -507,9 +541,8 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
             p[tt][rr][i] = __builtin_amdgcn_exp2f(st[tt][rr][i] * sc2 - o[i]) * cf[i];
       }
     }
-    lzm_grad_product<D, 2>(qt_s, p, acc, col, j);
-    __syncthreads();
-    stash();
+    lzm_grad_product_rows<D, 2, PITCH>(qb, p, acc, col, j);
+    stash(buf ^ 1);
     __syncthreads();
   }
   if (n_seg > 1) {

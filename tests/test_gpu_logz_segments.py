@@ -48,3 +48,19 @@ def test_logz_gradients(pkg, dev, B, L, HQ, H, D, W):
         assert err.item() < 1.5e-2, (name, err.item())
     cut = pkg.ops._cabi.load().hils_chunk_logz_bwd_dk_workspace(B, L, HQ, H, D, 64, W)
     assert (cut > 0) == (L > 800)
+
+
+@pytest.mark.parametrize("D,scale,step", [(64, 6.0, 1.0), (128, 12.0, 1.0), (64, 1.0, 40.0)])
+def test_logz_far_from_the_last_chunk(pkg, dev, D, scale, step):
+    """Scores in the hundreds, and chunks whose log sums jump by hundreds from one to the next: the last chunk's log sum
+    is no reference point for the next one's exponentials there."""
+    gen = torch.Generator(device=dev).manual_seed(D)
+    q = (torch.randn(1, 700, 8, D, device=dev, generator=gen) * scale).bfloat16()
+    k = torch.randn(1, 700, 2, D, device=dev, generator=gen) * scale
+    k[:, :, :, :] *= 1 + (step - 1) * (torch.arange(700, device=dev) // 64 % 2).view(1, -1, 1, 1)
+    k = k.bfloat16()
+    out = pkg.exact_chunk_log_z_tl(q, k, chunk_size=64, window_size=64)
+    ref = _reference(q.float(), k.float(), 64)
+    seen = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(out), seen)
+    assert (out[seen] - ref[seen]).abs().max().item() < 1e-5 * ref[seen].abs().max().item() + 2e-3
