@@ -1969,7 +1969,7 @@ struct DsArgs {
   float *pre_logits, *pre_m, *pre_l, *partial;
   int* arrived;    // [row] workgroups that have left their partial outputs
   int pre_groups;  // key groups of a row
-  int slot_off;    // bytes of LDS before the attention's slot lists: past the selection's and the attention's other arrays
+  int slot_off;    // bytes of LDS before the attention's slot lists (decode_step_lds)
   int stagger_ticks;  // 100 MHz ticks by which every other row of an XCD starts late (0: none)
   DrDims dr;
 };
@@ -2358,6 +2358,33 @@ extern "C" size_t hils_decode_step_workspace(int B, int L, int N, int HQ, int H,
   return s > 1 ? decode_step_ws_bytes(rows, s, N, HQ / H, D) : 0;
 }
 
+// LDS of a row's workgroup in the decode step's kernels.  The selection holds logits, pooled scores, page ids and bias
+// (sel_base bytes) and, behind them, the wavefronts' key staging; the attention's slot lists are written while the
+// logits are still read (the weights are worked out under the first loads), but the staging is done with by then, so
+// they lie over it and the step takes no more than the selection alone, which is what topk_row_fits counts.  (Behind
+// the staging they made the 3 KB that refused 1409 .. 1472 chunks of a 32/4 x 128 model with the prior bias.)  The
+// attention's other areas lie over the logits, from the start.
+struct DecodeStepLds {
+  size_t slot_off, dyn;
+  int fits, bias_inplace;
+};
+static DecodeStepLds decode_step_lds(int N, int G, int D, bool lmk_paged, bool with_bias) {
+  DecodeStepLds s;
+  s.fits = topk_row_fits(N, G, D, lmk_paged, with_bias, DS_WAVES, &s.bias_inplace);
+  const size_t base = topk_row_smem_base(N, G, lmk_paged, with_bias, s.bias_inplace != 0);
+  const size_t att_b = dr_work_bytes(D, G, DS_WAVES), sel_b = base + (size_t)DS_WAVES * 16 * (2 * D + 16);
+  s.slot_off = ((base > att_b ? base : att_b) + 15) & ~(size_t)15;
+  s.dyn = s.slot_off + dr_list_bytes(DS_WAVES);
+  if (s.dyn < sel_b) s.dyn = sel_b;
+  return s;
+}
+// bytes of LDS (static and dynamic) a row's workgroup of the decode step takes; 0: the selection does not fit
+extern "C" int hils_decode_step_lds(int N, int HQ, int H, int D, int with_bias, int lmk_paged) {
+  if (N <= 0 || H <= 0 || HQ <= 0 || HQ % H != 0 || HQ / H > 8 || (D != 64 && D != 128)) return 0;
+  const DecodeStepLds s = decode_step_lds(N, HQ / H, D, lmk_paged != 0, with_bias != 0);
+  return s.fits ? (int)(s.dyn + topk_row_shared_bytes(HQ / H) + 16) : 0;  // (16: decode_attend_kernel's flag)
+}
+
 static int decode_step_launch(const void* q, const void* lmks, const void* k, const void* v, const float* lse_swa,
                               const float* bias, int lmk_paged, int lmk_hm, int lmk_cap, int perq, int32_t* indices, void* scores, void* weights, void* o, float* lse_total,
                               float* sel_logits, int B, int L, int Lkv, int N, int HQ, int H, int D, int topk,
@@ -2370,17 +2397,13 @@ static int decode_step_launch(const void* q, const void* lmks, const void* k, co
   HILS_REQUIRE(nsplit == 1 || workspace_bytes >= decode_step_ws_bytes(rows, nsplit, N, G, D),
                "hils_decode_step: the workspace is too short (%zu bytes)", workspace_bytes);
   const int NP = (N + 63) & ~63;
-  int bias_inplace = 0;
-  const bool sel_fits = topk_row_fits(N, G, D, lmk_paged != 0, bias != nullptr, DS_WAVES, &bias_inplace);
-  const size_t sel_b = topk_row_smem_base(N, G, lmk_paged != 0, bias != nullptr, bias_inplace != 0) +
-                       (size_t)DS_WAVES * 16 * (2 * D + 16);
-  HILS_REQUIRE(sel_fits,
+  const DecodeStepLds lds = decode_step_lds(N, G, D, lmk_paged != 0, bias != nullptr);
+  const int bias_inplace = lds.bias_inplace;
+  HILS_REQUIRE(lds.fits,
                "hils_decode_step: too many chunks (%d) for the logits (and the bias) of the row's heads in LDS", N);
-  const size_t att_b = dr_work_bytes(D, G, DS_WAVES);
-  const size_t slot_off = ((sel_b > att_b ? sel_b : att_b) + 15) & ~(size_t)15;
-  const size_t smem = slot_off + dr_list_bytes(DS_WAVES);
+  const size_t smem = lds.dyn;
   DsArgs a;
-  a.slot_off = (int)slot_off;
+  a.slot_off = (int)lds.slot_off;
   a.q = (const bf16_t*)q; a.lmks = (const bf16_t*)lmks; a.k = (const bf16_t*)k; a.v = (const bf16_t*)v;
   a.lse_swa = lse_swa; a.bias = bias; a.indices = indices;
   a.lmk_hm = lmk_hm; a.lmk_cap = lmk_cap; a.perq = perq; a.bias_inplace = bias_inplace;

@@ -305,6 +305,10 @@ int hils_sparse_attn_decode_paged(const void* q, const void* k_pages, const void
  * that with eight head rows) it shares the logits' array and a winner's raw score is its biased logit
  * minus the bias (one fp32 rounding away from the product, far inside the bf16 it is returned in). */
 int hils_decode_step_covers(int B, int L, int N, int HQ, int H, int D, int topk, int block_size, int with_bias);
+/* Bytes of LDS the workgroup of a (query, KV head) row takes in the decode step's kernels (lmk_paged: the chunk keys
+ * are addressed through the page table), 0 if the selection of N chunks does not fit; at most 160 KiB for every
+ * shape that hils_decode_step_covers accepts. */
+int hils_decode_step_lds(int N, int HQ, int H, int D, int with_bias, int lmk_paged);
 int hils_decode_step(const void* q, const void* lmks, const void* k, const void* v, const float* lse_swa,
                      const float* bias, int32_t* indices, void* scores, void* weights, void* o,
                      float* lse_total, float* sel_logits, int B, int L, int Lkv, int N, int HQ, int H, int D,
