@@ -10,17 +10,22 @@ import math
 import torch
 
 from . import _cabi
+from ._native_op import NativeOp
 
 
-class ChunkAttnPoolFunction:
+class ChunkAttnPoolFunction(NativeOp):
     """Mirrors ChunkAttnPoolFunction (ops/chunk_attn_pool_tilelang.py:540-602): the autograd node is
     native (csrc/host_ops.cpp).  k_chunked may carry fewer heads than mu_q (grouped query heads: head h
     reads K head h // (H // h_kv)), which the reference reaches by repeating K's heads in memory first
     (models/FlashHiLS/hils_attention.py:20-50, :391)."""
 
     @staticmethod
-    def apply(mu_q, k_chunked, sm_scale, compact_lmk_k=False, shared_k=False):
+    def native(mu_q, k_chunked, sm_scale, compact_lmk_k=False, shared_k=False):
         return _cabi.host().attn_pool(mu_q, k_chunked, float(sm_scale), bool(compact_lmk_k), bool(shared_k))
+
+    @staticmethod
+    def forward(ctx, *args):
+        return NativeOp.record(ctx, ChunkAttnPoolFunction.native, args)
 
 
 def chunk_attn_pool(mu_q, k_chunked, sm_scale=None):

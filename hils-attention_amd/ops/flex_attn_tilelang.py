@@ -1,17 +1,22 @@
 """Sliding-window attention of the local branch (drop-in for flex_attn_tl of the reference's
 ops/flex_attn_tilelang.py)."""
 from . import _cabi
+from ._native_op import NativeOp
 
 
-class _FlexAttnTL:
+class _FlexAttnTL(NativeOp):
     """Mirrors _FlexAttnTL (ops/flex_attn_tilelang.py:1156-1255; kernels :26-267 forward,
     :270-1153 backward): the autograd node is native (csrc/host_ops.cpp).  lse is kept in natural-log
     units throughout."""
 
     @staticmethod
-    def apply(q, k, v, window_size, chunk_size, mask_lmk, expand_to_chunk, use_cache, sm_scale, kv_start):
+    def native(q, k, v, window_size, chunk_size, mask_lmk, expand_to_chunk, use_cache, sm_scale, kv_start):
         return _cabi.host().flex_attn(q, k, v, int(window_size), int(chunk_size), bool(mask_lmk),
                                       bool(expand_to_chunk), bool(use_cache), sm_scale, int(kv_start))
+
+    @staticmethod
+    def forward(ctx, *args):
+        return NativeOp.record(ctx, _FlexAttnTL.native, args)
 
 
 def flex_attn_tl(q, k, v, window_size: int, chunk_size: int, training: bool = True,
@@ -24,8 +29,7 @@ def flex_attn_tl(q, k, v, window_size: int, chunk_size: int, training: bool = Tr
     and a cache truncated at ``kv_start``."""
     if training and int(kv_start) != 0:
         raise ValueError("flex_attn_tl only supports non-zero kv_start in inference (training=False)")
-    return _FlexAttnTL.apply(q, k, v, int(window_size), int(chunk_size), bool(mask_lmk),
-                             bool(expand_to_chunk), not training, sm_scale, int(kv_start))
+    return _FlexAttnTL.apply(q, k, v, window_size, chunk_size, mask_lmk, expand_to_chunk, not training, sm_scale, kv_start)
 
 
 def flex_attn_tl_two_phase(q, k, v, window_size: int, chunk_size: int, training: bool = True,

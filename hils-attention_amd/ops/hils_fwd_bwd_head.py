@@ -4,6 +4,7 @@ import math
 import torch
 
 from . import _cabi
+from ._native_op import NativeOp
 
 
 def _check_kv_workspace(ws, need_bytes, device, what):
@@ -17,12 +18,12 @@ def _check_kv_workspace(ws, need_bytes, device, what):
             "with prepare_kv_workspace for this shape.")
 
 
-class _hils_block_M_attention_inverse:
+class _hils_block_M_attention_inverse(NativeOp):
     """Mirrors _hils_block_M_attention_inverse (ops/hils_fwd_bwd_head.py:771-913): the autograd node is
     native (csrc/host_ops.cpp)."""
 
     @staticmethod
-    def apply(q, k, v, weights, indices, block_size, sm_scale, mask_last_token, is_training, slope=None,
+    def native(q, k, v, weights, indices, block_size, sm_scale, mask_last_token, is_training, slope=None,
               kv_workspace=None, swa_o=None, swa_weight_index=None):
         if kv_workspace is not None:
             B, L, HQ, D = q.shape
@@ -32,6 +33,10 @@ class _hils_block_M_attention_inverse:
                                 f"q_len {L}, kv_len {L_kv}, {HQ}/{H} heads, D {D}, Dv {Dv}, top-{K}")
         return _cabi.host().sparse_attn(q, k, v, weights, indices, int(block_size), sm_scale, bool(mask_last_token),
                                         bool(is_training), slope, kv_workspace, swa_o, swa_weight_index)
+
+    @staticmethod
+    def forward(ctx, *args):
+        return NativeOp.record(ctx, _hils_block_M_attention_inverse.native, args)
 
 
 class _hils_block_M_attention_f32(torch.autograd.Function):

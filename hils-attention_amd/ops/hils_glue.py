@@ -9,13 +9,24 @@ kernel; column K is the weight of the local (sliding-window) branch.
 import torch
 
 from . import _cabi
+from ._native_op import NativeOp
+
+
+class _ChunkWeights(NativeOp):
+    @staticmethod
+    def native(scores, lse_swa, prior_b, indices, enable_softmax1):
+        return _cabi.host().chunk_weights(scores, lse_swa, prior_b, indices, bool(enable_softmax1))
+
+    @staticmethod
+    def forward(ctx, *args):
+        return NativeOp.record(ctx, _ChunkWeights.native, args)
 
 
 def chunk_weights(scores, lse_swa, prior_b=None, indices=None, enable_softmax1=False):
     """scores (B,L,HQ,K) bf16, lse_swa (B,L,HQ) -> weights (B,L,HQ,K+1(+1)) bf16.
     ``prior_b`` (B,N,HQ) with ``indices`` (B,L,H,K) adds the gathered prior bias first.
     Differentiable in scores, lse_swa and prior_b."""
-    return _cabi.host().chunk_weights(scores, lse_swa, prior_b, indices, bool(enable_softmax1))
+    return _ChunkWeights.apply(scores, lse_swa, prior_b, indices, enable_softmax1)
 
 
 def topk_chunk_weights(q, lmks, lse_swa, topk, block_size, window_size, is_causal=True, q_offset=0,

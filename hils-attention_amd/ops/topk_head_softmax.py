@@ -9,14 +9,15 @@ ascending with -1 padding.
 import torch
 
 from . import _cabi
+from ._native_op import NativeOp
 
 
-class SoftmaxTopKMaxPoolingFusedFn:
+class SoftmaxTopKMaxPoolingFusedFn(NativeOp):
     """Mirrors SoftmaxTopKMaxPoolingFusedFn (ops/topk_head_softmax.py:975-1092): the autograd node is
     native (csrc/host_ops.cpp).  Returns indices (B,L,h_kv,topk) and scores (B,L,h_kv,G,topk)."""
 
     @staticmethod
-    def apply(q, lmks, lse_swa, topk, block_size, window_size, is_causal, q_offset,
+    def native(q, lmks, lse_swa, topk, block_size, window_size, is_causal, q_offset,
               drop_mask, sm_scale, bias, gumbel_noise, per_qhead_lmks, debug):
         dbg, no_ws = [], False
         if debug is not None:
@@ -30,6 +31,10 @@ class SoftmaxTopKMaxPoolingFusedFn:
         if debug is not None:
             debug["lse_total"], debug["sel_logits"] = dbg
         return indices, scores.view(*q.shape[:4], -1)
+
+    @staticmethod
+    def forward(ctx, *args):
+        return NativeOp.record(ctx, SoftmaxTopKMaxPoolingFusedFn.native, args)
 
 
 def _bias_per_group(bias, B, N, h_kv, G, device):
