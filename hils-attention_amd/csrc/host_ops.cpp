@@ -683,37 +683,47 @@ Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v,
   two_calls = two_calls || Lkv < N * block ||
               !hils_decode_step_covers(i32(B), i32(L), i32(N), i32(hq), i32(hkv), i32(D), i32(topk), i32(block),
                                        (int)pb.defined());
+  // (views of any strides, such as the slices of a cache buffer)
+  const Tensor qc = q.contiguous(), kc = gpu_readable(k, q.device()), vc = gpu_readable(v, q.device());
+  Tensor lse_total, sel;
+  if (!debug.is_none()) {
+    lse_total = new_tensor({B, L, hkv, G}, q, at::kFloat);
+    sel = at::full({B, L, hkv, G, N}, -INFINITY, q.options().dtype(at::kFloat));
+    debug["lse_total"] = lse_total;
+    debug["sel_logits"] = sel;
+  }
   if (two_calls) {
     if (head_major) {  // the two-call kernels read the reference's layout
       lmks = lmks.slice(2, 0, N).permute({0, 2, 1, 3}).contiguous();
       if (pb.defined()) pb = pb.slice(2, 0, N).permute({0, 2, 1, 3}).reshape({B, N, hq}).contiguous();
     }
-    const Selection s = topk_weights(q, lmks, lse_swa, topk, block, window, true, q_offset, scale, pb, hkv);
-    const Tensor o = sparse_attn(q, k, v, s.weights, s.idx, block, scale, mask_last, false, {}, {}, {}, {});
+    Selection s;
+    if (debug.is_none()) {
+      s = topk_weights(qc, lmks, lse_swa, topk, block, window, true, q_offset, scale, pb, hkv);
+    } else {  // the selection's logits are wanted: the entry point that exports them, then the softmax
+      const Tensor lse = as_f32(lse_swa.reshape({B, L, hq}));
+      const TopkCfg c{topk, block, window, 1, q_offset, per_qhead, scale};
+      const variable_list r = TopkFn::forward(nullptr, qc.view({B, L, hkv, G, D}), lmks.contiguous(), lse, maybe(pb), {},
+                                              {}, c, {lse_total, sel}, false);
+      s.idx = r[0];
+      s.scores = r[1];
+      s.weights = weights_forward(s.scores, lse, pb, s.idx, hkv, N, 0);
+    }
+    const Tensor o = sparse_attn(qc, kc, vc, s.weights, s.idx, block, scale, mask_last, false, {}, {}, {}, {});
     return {o, s.weights, s.idx, s.scores};
   }
-  const Tensor qc = q.contiguous(), kc = gpu_readable(k, q.device()), vc = gpu_readable(v, q.device());
   const Tensor lse = as_f32(lse_swa.reshape({B, L, hq}));
   const Tensor lm = lmks.contiguous();
   Tensor idx = new_tensor({B, L, hkv, topk}, q, at::kInt);
   Tensor sc = new_tensor({B, L, hq, topk}, q, q.scalar_type());
   Tensor w = new_tensor({B, L, hq, topk + 1}, q, q.scalar_type());
   Tensor o = new_tensor({B, L, hq, D}, q, q.scalar_type());
-  Tensor lse_total, sel;
-  if (!debug.is_none()) {
-    lse_total = new_tensor({B, L, hkv, G}, q, at::kFloat);
-    sel = at::full({B, L, hkv, G, N}, -INFINITY, q.options().dtype(at::kFloat));
-  }
   const Tensor ws = workspace(hils_decode_step_workspace(i32(B), i32(L), i32(N), i32(hq), i32(hkv), i32(D), i32(topk),
                                                          per_qhead, 0), q);
   HILS_CALL(hils_decode_step_ws, cptr(qc), cptr(lm), cptr(kc), cptr(vc), fptr(lse), fptr(pb), miptr(idx), mptr(sc), mptr(w),
             mptr(o), mfptr(lse_total), mfptr(sel), i32(B), i32(L), i32(Lkv), i32(N), i32(hq), i32(hkv), i32(D),
             i32(topk), i32(block), i32(window), i32(q_offset), (float)scale, (float)scale, (int)mask_last,
             (int)head_major, i32(cap), per_qhead, mptr(ws), bytes(ws));
-  if (!debug.is_none()) {
-    debug["lse_total"] = lse_total;
-    debug["sel_logits"] = sel;
-  }
   return {o, w, idx, sc};
 }
 
