@@ -709,7 +709,13 @@ Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v,
       s.scores = r[1];
       s.weights = weights_forward(s.scores, lse, pb, s.idx, hkv, N, 0);
     }
-    const Tensor o = sparse_attn(qc, kc, vc, s.weights, s.idx, block, scale, mask_last, false, {}, {}, {}, {});
+    // (the sums as exact as the one-launch kernel's)
+    Tensor o = new_tensor({B, L, hq, D}, q, q.scalar_type());
+    const Tensor ws = workspace(hils_sparse_attn_fwd_workspace(i32(B), i32(L), i32(Lkv), i32(hq), i32(hkv), i32(D), i32(D),
+                                                               i32(topk), i32(hq), 1, i32(block), 0.f), q);
+    HILS_CALL(hils_sparse_attn_fwd_fine, cptr(qc), cptr(kc), cptr(vc), cptr(s.weights), iptr(s.idx), mptr(o), mptr(ws),
+              bytes(ws), i32(B), i32(L), i32(Lkv), i32(hq), i32(hkv), i32(D), i32(D), i32(topk), i32(topk + 1), i32(block),
+              (float)scale, (int)mask_last);
     return {o, s.weights, s.idx, s.scores};
   }
   const Tensor lse = as_f32(lse_swa.reshape({B, L, hq}));

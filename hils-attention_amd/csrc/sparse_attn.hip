@@ -17,7 +17,7 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
                               const int32_t* indices, const float* slope, const void* swa_o, int merge_col,
                               void* o, float* lse, void* workspace, int workspace_ready, int B, int L,
                               int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int S, float sm_scale,
-                              int mask_last, int q_block, int WH, float sm_n, void* stream,
+                              int mask_last, int q_block, int WH, float sm_n, bool fine, void* stream,
                               int* handled);
 
 bool hils_decode_covers(int L, int HQ, int H, int D, int Dv, int S, int q_block, int WH, float sm_n,
@@ -335,13 +335,10 @@ static int sa_merge_local(void* o, const void* swa_o, const void* weights, int B
   return HILS_OK;
 }
 
-extern "C" int hils_sparse_attn_fwd(const void* q, const void* k, const void* v,
-                                    const void* weights, const int32_t* indices,
-                                    const float* slope, const void* swa_o, void* o, float* lse,
-                                    void* workspace, size_t workspace_bytes, int workspace_ready, int B, int L,
-                                    int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int WH, int q_block,
-                                    int S, float sm_scale, int mask_last, float sm_n, int merge_col,
-                                    void* stream) {
+static int sa_fwd(const void* q, const void* k, const void* v, const void* weights, const int32_t* indices,
+                  const float* slope, const void* swa_o, void* o, float* lse, void* workspace, size_t workspace_bytes,
+                  int workspace_ready, int B, int L, int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int WH,
+                  int q_block, int S, float sm_scale, int mask_last, float sm_n, int merge_col, bool fine, void* stream) {
   HILS_REQUIRE(q && k && v && weights && indices && o, "hils_sparse_attn_fwd: null pointer");
   if (int rc = sa_check("hils_sparse_attn_fwd", B, L, Lkv, HQ, H, D, Dv, K, NW, WH, q_block, S)) return rc;
   {
@@ -366,7 +363,7 @@ extern "C" int hils_sparse_attn_fwd(const void* q, const void* k, const void* v,
     int handled = 0;
     if (int rc = hils_sparse_attn_fwd_mfma(q, k, v, weights, indices, slope, swa_o, merge_col, o, lse,
                                            workspace, workspace_ready, B, L, Lkv, HQ, H, D, Dv, K, NW, S,
-                                           sm_scale, mask_last, q_block, WH, sm_n, stream, &handled))
+                                           sm_scale, mask_last, q_block, WH, sm_n, fine, stream, &handled))
       return rc;
     if (handled) {
       HILS_CHECK_LAUNCH("hils_sparse_attn_fwd");
@@ -383,6 +380,24 @@ extern "C" int hils_sparse_attn_fwd(const void* q, const void* k, const void* v,
     if (int rc = sa_merge_local(o, swa_o, weights, B, L, HQ, H, Dv, NW, WH, q_block, merge_col, stream)) return rc;
   HILS_CHECK_LAUNCH("hils_sparse_attn_fwd");
   return HILS_OK;
+}
+
+extern "C" int hils_sparse_attn_fwd(const void* q, const void* k, const void* v, const void* weights,
+                                    const int32_t* indices, const float* slope, const void* swa_o, void* o, float* lse,
+                                    void* workspace, size_t workspace_bytes, int workspace_ready, int B, int L,
+                                    int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int WH, int q_block,
+                                    int S, float sm_scale, int mask_last, float sm_n, int merge_col,
+                                    void* stream) {
+  return sa_fwd(q, k, v, weights, indices, slope, swa_o, o, lse, workspace, workspace_bytes, workspace_ready, B, L, Lkv,
+                HQ, H, D, Dv, K, NW, WH, q_block, S, sm_scale, mask_last, sm_n, merge_col, false, stream);
+}
+
+extern "C" int hils_sparse_attn_fwd_fine(const void* q, const void* k, const void* v, const void* weights,
+                                         const int32_t* indices, void* o, void* workspace, size_t workspace_bytes, int B,
+                                         int L, int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int S,
+                                         float sm_scale, int mask_last, void* stream) {
+  return sa_fwd(q, k, v, weights, indices, nullptr, nullptr, o, nullptr, workspace, workspace_bytes, 0, B, L, Lkv, HQ, H,
+                D, Dv, K, NW, HQ, 1, S, sm_scale, mask_last, 0.f, 0, true, stream);
 }
 
 bool hils_bw_covers(int L, int Lkv, int HQ, int H, int D, int Dv, int K, int S, int q_block, int WH,

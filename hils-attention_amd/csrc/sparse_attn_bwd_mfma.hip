@@ -757,8 +757,9 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   for (int c = c_lo; c < c_lo + per_thr && c < dm.nchunk; ++c) {
     const int h = cur[c];
     if (h > 0) {
-      vm = fmaxf(vm, vmax[(b * dm.H + hk) * (long)dm.nchunk + c]);
-      km = fmaxf(km, kmax[(b * dm.H + hk) * (long)dm.nchunk + c]);
+      // (the sign marks a chunk with a NaN or an infinity)
+      vm = fmaxf(vm, fabsf(vmax[(b * dm.H + hk) * (long)dm.nchunk + c]));
+      km = fmaxf(km, fabsf(kmax[(b * dm.H + hk) * (long)dm.nchunk + c]));
     }
     local += h;
   }

@@ -11,8 +11,12 @@
 // the accumulator layout; V is pre-transposed per chunk in the same order).  The
 // (rows x Dv) partial outputs are summed into a fixed-point output tile in LDS with integer
 // LDS atomics, which is what lets rows of different visits be arbitrary subsets of the block.
+// What fixed point cannot hold is kept out of it: a block that visits a chunk with a NaN or an
+// infinity in V (or meets such a weight) sums in floating point instead, and a row whose softmax
+// is not a number comes out as NaN.
 #include "common.h"
 #include "../../include/hils_amd.h"
+#include <type_traits>
 
 #define GA_THREADS 512
 #ifndef GA_THREADS_NARROW
@@ -33,7 +37,8 @@
 //   vp[chunk][dt][s][lane][8]  = V[token tok(s, lane>>4, e)][dv = dt*16 + (lane&15)]
 // with tok(s, j, e) = 32*s + 16*(e/4) + 4*j + e%4, the order in which an accumulator-layout
 // P supplies tokens when it is fed back as the A operand of O = P V.
-// Also records max|V| of every chunk (it bounds the fixed-point output accumulation).
+// Also records max|V| of every chunk (it bounds the fixed-point output accumulation), NaNs left out,
+// with the sign bit set when the chunk holds a NaN or an infinity.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256)
 pack_kv_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, bf16_t* __restrict__ kp,
@@ -61,7 +66,8 @@ pack_kv_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, bf16_
   // ---- V: transposed through LDS
   const int DP = Dv + 2;
   const int d8n = Dv / 8;
-  float mx = 0.f;
+  uint32_t mx = 0;  // bf16 bits: the order of the magnitudes
+  int odd = 0;
   for (int i = threadIdx.x; i < GA_S * d8n; i += 256) {
     const int s = i / d8n, d8 = i - s * d8n;
     uint4 x = *(const uint4*)(v + ((b * Lkv + (long)c * GA_S + s) * H + h) * Dv + d8 * 8);
@@ -69,11 +75,14 @@ pack_kv_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, bf16_
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       tile[s * DP + d8 * 8 + e] = xs[e];
-      mx = fmaxf(mx, fabsf(bf2f(xs[e])));
+      const uint32_t mag = xs[e] & 0x7fffu;
+      if (mag >= 0x7f80u) odd = 1;
+      if (mag <= 0x7f80u && mag > mx) mx = mag;
     }
   }
-  mx = block_max(mx, red);  // contains the barrier that orders the tile writes
-  if (threadIdx.x == 0) vmax[chunk] = mx;
+  odd = __syncthreads_or(odd);  // (the barrier orders the tile writes)
+  const float top = block_max(__uint_as_float(mx << 16), red);
+  if (threadIdx.x == 0) vmax[chunk] = odd ? -top : top;
   if (!vp) return;  // only max|V| wanted
   bf16_t* out = vp + chunk * (long)GA_S * Dv;
   for (int i = threadIdx.x; i < Dv * 8; i += 256) {
@@ -98,6 +107,12 @@ pack_kv_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, bf16_
 #define GA_FX_BIAS 12582912.0f
 #define GA_FX_BIAS_BITS 0x4B400000
 #define GA_FX_LOG2_MAX 21  // sums are scaled below 2^21: one bit of head room for the rounding of P
+// The fine variant converts the products to integers instead: 29 bits below the bound for an instruction per
+// accumulator element (32K prefill, 32/8 heads of 128: 2126 -> 2210 us; B4 L8192, 16/16 of 64: 645 -> 662).
+#define GA_FX_LOG2_MAX_FINE 30
+// Entries of nadd[]: adds of the row (at most a tile's 16 a slot) and, above them, rows that are not numbers
+#define GA_ODD_ROW (1 << 16)
+#define GA_FX_LIMIT 1.0e18f  // row weight sums and |V| past this go the floating-point way
 
 struct GaDims {
   int L, Lkv, HQ, H, B, K, NW, T, nblk, nchunk, mask_last;
@@ -110,10 +125,18 @@ struct GaDims {
   uint32_t k_magic, qb_magic;  // hils_udiv_magic of K and q_block (pair index < 2^16, query index < 2^24)
 };
 
-// Power-of-two fixed-point scale for sums bounded by `bound`: bound * scale < 2^GA_FX_LOG2_MAX.
-__device__ __forceinline__ float ga_fx_scale(float bound) {
-  if (!(bound > 0.f && bound < 3.0e38f)) return 1.f;
-  int e2 = GA_FX_LOG2_MAX - 1 - ilogbf(bound);
+// The bits of a value that may be a NaN.  This file is compiled without NaN handling: the compiler would reason a test of
+// the bits of a float it has computed back into one that no NaN passes, so they come through an empty asm statement.
+__device__ __forceinline__ unsigned ga_bits(float x) {
+  unsigned u = __float_as_uint(x);
+  asm("" : "+v"(u));
+  return u;
+}
+
+// Power-of-two fixed-point scale for sums bounded by `bound`: bound * scale < 2^log2_max.
+__device__ __forceinline__ float ga_fx_scale(float bound, int log2_max) {
+  if (bound == 0.f) return 1.f;
+  int e2 = log2_max - 1 - ilogbf(bound);
   e2 = e2 > 90 ? 90 : (e2 < -90 ? -90 : e2);
   return ldexpf(1.f, e2);
 }
@@ -163,7 +186,9 @@ struct GaTile {
 // The scale is chosen per output row from bound = sum_k |w_row,k| * max_visited|V|, which
 // bounds every element of the row because each P row is a convex combination: a row keeps
 // 20 bits below its own bound however small its weights are beside its neighbours'.
-template <int D, int DV, int G, bool SLOPE, int NT>
+// FINE: 29 bits, which a column whose V is small beside the largest keeps its precision with: for the calls
+// that would otherwise run on the decode kernels, whose sums are fp32.
+template <int D, int DV, int G, bool SLOPE, int NT, bool FINE>
 __global__ void __launch_bounds__(NT)
 sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* __restrict__ kp,
                        const bf16_t* __restrict__ vp, const float* __restrict__ vmax,
@@ -180,7 +205,7 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
   int* o_acc = smem_i;                       // R x DV fixed point
   int* cur = o_acc + (size_t)R * DV;         // nchunk: histogram -> running ends
   int* pairs = cur + dm.nchunk;              // T*K pairs (query << 8 | slot) grouped by chunk
-  int* nadd = pairs + dm.T * dm.K;           // R: tiles added to each output row
+  int* nadd = pairs + dm.T * dm.K;           // R: tiles added to each output row, and how many were not numbers
   float* rscale = (float*)(nadd + R);        // R: sum_k |w| of the row, then its fixed-point scale
   __shared__ float red[32];
   __shared__ int scan_s[NT / 64];
@@ -246,6 +271,7 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
   }
   // (2) weight rows, for the bound of the fixed-point scale: a row's sum of |w| over the K slots
   // (aligned dword loads, all in flight together)
+  bool no_fx = false;  // something fixed point cannot hold (told by the bits: NaNs compare as the largest)
   for (int row = tid; row < R; row += NT) {
     const int ql = row / G, g = row - ql * G;
     float a = 0.f;
@@ -254,6 +280,7 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
                       dm.NW;  // first element
       a = hils_abs_row_sum_bf16(weights, e0, K, (long)dm.B * LB * dm.WH * dm.NW);
     }
+    no_fx = no_fx || ga_bits(a) > __float_as_uint(GA_FX_LIMIT);
     rscale[row] = a;  // only this thread touches the entry until the barrier behind the scan
   }
   // The packed copy goes through LDS (the output tile is not in use yet): pieces arrive in the
@@ -315,7 +342,11 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
   int local = 0;
   for (int c = c_lo; c < c_lo + per_thr && c < dm.nchunk; ++c) {
     const int h = cur[c];
-    if (h > 0) vm = fmaxf(vm, vmax[(b * dm.H + hk) * (long)dm.nchunk + c]);
+    if (h > 0) {
+      const float cm = vmax[(b * dm.H + hk) * (long)dm.nchunk + c];
+      no_fx = no_fx || ga_bits(cm) > __float_as_uint(GA_FX_LIMIT);  // (a set sign bit too)
+      vm = fmaxf(vm, cm);
+    }
     local += h;
   }
   int incl = local;
@@ -325,7 +356,8 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
     if (lane >= o2) incl += x;
   }
   if (lane == 63) scan_s[wave] = incl;
-  vm = block_max_lds(vm, red);  // barrier: scan_s visible, all histogram reads done
+  vm = block_max_lds(no_fx ? INFINITY : vm, red);  // barrier: scan_s visible, all histogram reads done
+  const bool flt = __builtin_amdgcn_readfirstlane((int)(vm > GA_FX_LIMIT)) != 0;  // of the whole block
   int base = incl - local;
   for (int w2 = 0; w2 < wave; ++w2) base += scan_s[w2];
   for (int c = c_lo; c < c_lo + per_thr && c < dm.nchunk; ++c) {
@@ -333,7 +365,7 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
     cur[c] = base;
     base += h;
   }
-  for (int row = tid; row < R; row += NT) rscale[row] = ga_fx_scale(rscale[row] * vm);
+  for (int row = tid; row < R; row += NT) rscale[row] = flt ? 1.f : ga_fx_scale(rscale[row] * vm, FINE ? GA_FX_LOG2_MAX_FINE : GA_FX_LOG2_MAX);
   lds_barrier();
 #pragma unroll
   for (int e = 0; e < MAXP; ++e)
@@ -468,7 +500,7 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
     ga_pin(t.wbits);
   };
   // output rows 4j .. 4j+3 of a tile starting at pair p (element offsets of this lane's column)
-  auto tile_rows = [&](Tile& t, int p) {
+  auto tile_rows = [&](Tile& t, int p, auto flt_c) __attribute__((always_inline)) {
     const int last = t.n - 1;
     if constexpr (G >= 4) {  // the four rows are consecutive heads of one query
       const int qsl = (4 * j) / G;
@@ -488,6 +520,11 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
         const int rr = 4 * j + i;
         t.orow[i] = ((pk_o[i] >> 8) * G + rr % G) * DV + r;
       }
+    }
+    if constexpr (decltype(flt_c)::value) {  // a padding row's zero times an infinity is no zero: it is left out
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if ((4 * j + i) / G > last) t.orow[i] = -1;
     }
   };
   bf16x8_t ap[2];   // P of the previous tile (A operand of O = P V)
@@ -539,9 +576,10 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
       const int ql = t.pk >> 8, slot = t.pk & 255;
       lse_blk[(ql * dm.HQ + hq) * K + slot] = mc + __builtin_amdgcn_logf(sum);
     }
-    if (j == 0) atomicAdd(&nadd[(t.pk >> 8) * G + g], 1);  // padding rows count on the row they are added to
     const float w_row = qs < t.n ? __uint_as_float(t.wbits << 16) : 0.f;
     const float f = w_row * t.rs * __builtin_amdgcn_rcpf(sum);  // fixed-point scale (a power of two) folded into P
+    // (padding rows count on the row they are added to)
+    if (j == 0) atomicAdd(&nadd[(t.pk >> 8) * G + g], (ga_bits(f) & 0x7f800000u) == 0x7f800000u ? GA_ODD_ROW + 1 : 1);
     // P as the A operand of O = P V: k-step s takes tokens of accumulator tiles 2s, 2s+1
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -554,8 +592,11 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
     }
   };
   // O += P V for the tile whose rows are `orow` (V has landed); V(c_next) replaces V when asked
-  const f32x4_t fx_bias = {GA_FX_BIAS, GA_FX_BIAS, GA_FX_BIAS, GA_FX_BIAS};
-  auto output_stage = [&](const int* orow, bool reload, int c_next) {
+  auto add = [&](int* at, float x) __attribute__((always_inline)) { atomicAdd(at, FINE ? (int)x : __float_as_int(x)); };
+  auto output_stage = [&](const int* orow, bool reload, int c_next, auto flt_c) __attribute__((always_inline)) {
+    constexpr bool FLT = decltype(flt_c)::value;
+    constexpr float acc0 = FINE || FLT ? 0.f : GA_FX_BIAS;
+    const f32x4_t fx_bias = {acc0, acc0, acc0, acc0};
     // four column tiles at a time: their eight MFMAs interleaved (two-deep chains), then the
     // operand reload, then the fixed-point adds
 #pragma unroll
@@ -569,20 +610,25 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
         for (int u = 0; u < 4; ++u)
           acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[s2], ga_bf(vb[d0 + u][s2]), acc[u], 0, 0, 0);
       if (reload) load_v_half(c_next, d0, 4);
-      if constexpr (G >= 4) {
+      if constexpr (FLT) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (orow[i] >= 0) unsafeAtomicAdd((float*)&o_acc[orow[i] + (d0 + u) * 16], acc[u][i]);
+      } else if constexpr (G >= 4) {
         // the lane's four rows are consecutive heads of one query: one address, the rest are offsets
         // the instruction carries
         int* o0 = o_acc + orow[0];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) atomicAdd(o0 + i * DV + (d0 + u) * 16, __float_as_int(acc[u][i]));
+          for (int i = 0; i < 4; ++i) add(o0 + i * DV + (d0 + u) * 16, acc[u][i]);
       } else {
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            atomicAdd(&o_acc[orow[i] + (d0 + u) * 16], __float_as_int(acc[u][i]));
+          for (int i = 0; i < 4; ++i) add(&o_acc[orow[i] + (d0 + u) * 16], acc[u][i]);
       }
     }
   };
@@ -594,70 +640,74 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
   // O += P(i-1) V needs B_{i-1}: the loads behind it are C_{i-1} (NK when x_i) and A_i;
   // S(i) needs C_{i-1} and A_{i-1}: the loads behind C_{i-1} are A_i and B_i (NV when x_i).
   // Without a tile i+1 there is no A_i and the step simply waits for everything.
-  int c_cur, p_cur = 0, ve_cur = 0;
-  c_cur = grab(p_cur, ve_cur);
-  if (c_cur >= 0) {
-    Tile ta, tb;
+  auto stream = [&](auto flt_c) __attribute__((always_inline)) {
+    int c_cur, p_cur = 0, ve_cur = 0;
+    c_cur = grab(p_cur, ve_cur);
+    if (c_cur >= 0) {
+      Tile ta, tb;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) { ta.bq[ks] = (ga_u32x4){0, 0, 0, 0}; tb.bq[ks] = (ga_u32x4){0, 0, 0, 0}; }
-    ta.wbits = tb.wbits = 0;
+      for (int ks = 0; ks < KS; ++ks) { ta.bq[ks] = (ga_u32x4){0, 0, 0, 0}; tb.bq[ks] = (ga_u32x4){0, 0, 0, 0}; }
+      ta.wbits = tb.wbits = 0;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) ka[mt][ks] = (ga_u32x4){0, 0, 0, 0};
+        for (int ks = 0; ks < KS; ++ks) ka[mt][ks] = (ga_u32x4){0, 0, 0, 0};
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) vb[dt][0] = vb[dt][1] = (ga_u32x4){0, 0, 0, 0};
-    // step 0 (no previous tile): A_{-1} = tile 0, C_{-1} = K(c_0), then A_0, B_0 = V(c_0)
-    issue_tile(ta, p_cur, ve_cur);
-    tile_rows(ta, p_cur);
-    load_k_all(c_cur);
-    int c_nxt = c_cur, p_nxt = p_cur, ve_nxt = ve_cur;
-    advance(c_nxt, p_nxt, ve_nxt);
-    if (c_nxt >= 0) {
-      issue_tile(tb, p_nxt, ve_nxt);
-      tile_rows(tb, p_nxt);
-    }
-    load_v_half(c_cur, 0, DT);
-    if (c_nxt >= 0) ga_vmwait<NA + NV>(); else ga_vmwait<NV>();
-    pin_k();
-    pin_tile(ta);
-    score_stage(ta, c_nxt >= 0 && c_nxt != c_cur, c_nxt);
-    int c_prev = c_cur;
-    // one step: `cu` is the tile whose scores are due (its loads were issued a step ago), `nx`
-    // holds the previous tile's output rows until the output stage is through, then the tile
-    // after `cu`.
-    auto step = [&](Tile& cu, Tile& nx) {
-      c_cur = c_nxt; p_cur = p_nxt; ve_cur = ve_nxt;
+      for (int dt = 0; dt < DT; ++dt) vb[dt][0] = vb[dt][1] = (ga_u32x4){0, 0, 0, 0};
+      // step 0 (no previous tile): A_{-1} = tile 0, C_{-1} = K(c_0), then A_0, B_0 = V(c_0)
+      issue_tile(ta, p_cur, ve_cur);
+      tile_rows(ta, p_cur, flt_c);
+      load_k_all(c_cur);
+      int c_nxt = c_cur, p_nxt = p_cur, ve_nxt = ve_cur;
       advance(c_nxt, p_nxt, ve_nxt);
-      const bool more = c_nxt >= 0;
-      const bool x = c_cur != c_prev;
-      if (more) issue_tile(nx, p_nxt, ve_nxt);  // A_i; leaves nx.orow alone
-      if (!more) ga_vmwait<0>(); else if (x) ga_vmwait<NA + NK>(); else ga_vmwait<NA>();
-      pin_v();
-      output_stage(nx.orow, x, c_cur);          // B_i
-      if (more) tile_rows(nx, p_nxt);
-      if (!more) ga_vmwait<0>(); else if (x) ga_vmwait<NA + NV>(); else ga_vmwait<NA>();
+      if (c_nxt >= 0) {
+        issue_tile(tb, p_nxt, ve_nxt);
+        tile_rows(tb, p_nxt, flt_c);
+      }
+      load_v_half(c_cur, 0, DT);
+      if (c_nxt >= 0) ga_vmwait<NA + NV>(); else ga_vmwait<NV>();
       pin_k();
-      pin_tile(cu);
-      score_stage(cu, more && c_nxt != c_cur, c_nxt);  // C_i
-      c_prev = c_cur;
-    };
-    // the stream: tile 0 = ta (scored above), tile 1 = tb, tile 2 -> ta, ...
-    bool last_is_a = true;
-    while (c_nxt >= 0) {
-      step(tb, ta);
-      last_is_a = false;
-      if (c_nxt < 0) break;
-      step(ta, tb);
-      last_is_a = true;
-    }
-    int orow_last[4];
+      pin_tile(ta);
+      score_stage(ta, c_nxt >= 0 && c_nxt != c_cur, c_nxt);
+      int c_prev = c_cur;
+      // one step: `cu` is the tile whose scores are due (its loads were issued a step ago), `nx`
+      // holds the previous tile's output rows until the output stage is through, then the tile
+      // after `cu`.
+      auto step = [&](Tile& cu, Tile& nx) {
+        c_cur = c_nxt; p_cur = p_nxt; ve_cur = ve_nxt;
+        advance(c_nxt, p_nxt, ve_nxt);
+        const bool more = c_nxt >= 0;
+        const bool x = c_cur != c_prev;
+        if (more) issue_tile(nx, p_nxt, ve_nxt);  // A_i; leaves nx.orow alone
+        if (!more) ga_vmwait<0>(); else if (x) ga_vmwait<NA + NK>(); else ga_vmwait<NA>();
+        pin_v();
+        output_stage(nx.orow, x, c_cur, flt_c);          // B_i
+        if (more) tile_rows(nx, p_nxt, flt_c);
+        if (!more) ga_vmwait<0>(); else if (x) ga_vmwait<NA + NV>(); else ga_vmwait<NA>();
+        pin_k();
+        pin_tile(cu);
+        score_stage(cu, more && c_nxt != c_cur, c_nxt);  // C_i
+        c_prev = c_cur;
+      };
+      // the stream: tile 0 = ta (scored above), tile 1 = tb, tile 2 -> ta, ...
+      bool last_is_a = true;
+      while (c_nxt >= 0) {
+        step(tb, ta);
+        last_is_a = false;
+        if (c_nxt < 0) break;
+        step(ta, tb);
+        last_is_a = true;
+      }
+      int orow_last[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) orow_last[i] = last_is_a ? ta.orow[i] : tb.orow[i];
-    ga_vmwait<0>();
-    pin_v();
-    output_stage(orow_last, false, 0);
-  }
+      for (int i = 0; i < 4; ++i) orow_last[i] = last_is_a ? ta.orow[i] : tb.orow[i];
+      ga_vmwait<0>();
+      pin_v();
+      output_stage(orow_last, false, 0, flt_c);
+    }
+  };
+  // (two copies of the stream: a branch at its adds cost 1.5 % with heads of 128)
+  if (flt) stream(std::true_type{}); else stream(std::false_type{});
   __syncthreads();
   constexpr int C8 = DV / 8;
   const int wcol = dm.merge_col;
@@ -667,11 +717,18 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
     const int t = t0 + ql;
     if (t < dm.L) {
       const int* src = o_acc + (size_t)row * DV + c8 * 8;
-      const unsigned bias = (unsigned)nadd[row] * (unsigned)GA_FX_BIAS_BITS;  // wraps like the sums did
+      const unsigned added = (unsigned)nadd[row];
+      const unsigned bias = FINE ? 0u : (added & (GA_ODD_ROW - 1)) * (unsigned)GA_FX_BIAS_BITS;  // wraps like the sums did
       const float fx_inv = 1.f / rscale[row];  // a power of two: exact
+      const int4 s0 = *(const int4*)src, s1 = *(const int4*)(src + 4);
+      const int sum[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
       float f[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = (float)(int)((unsigned)src[e] - bias) * fx_inv;
+      for (int e = 0; e < 8; ++e) f[e] = (float)(int)((unsigned)sum[e] - bias) * fx_inv;
+      if (flt) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = __int_as_float(sum[e]);
+      }
       const long orow_g = ((b * dm.L + t) * (long)dm.HQ + hk * G + g2) * DV + c8 * 8;
       if (swa_o) {  // o = remote branch + local branch * its inter-chunk weight, rounded once
         const float wl = bf2f(weights[((b * LB + (long)hils_udiv((uint32_t)t, (uint32_t)dm.q_block, dm.qb_magic)) * (long)dm.WH + (w_per_q ? hk * G + g2 : hk)) *
@@ -686,12 +743,13 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
       x.y = pack_bf2(f[2], f[3]);
       x.z = pack_bf2(f[4], f[5]);
       x.w = pack_bf2(f[6], f[7]);
+      if (added >= GA_ODD_ROW) x = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
       *(uint4*)(o + orow_g) = x;
     }
   }
 }
 
-template <int D, int DV, int G, bool SLOPE>
+template <int D, int DV, int G, bool SLOPE, bool FINE>
 static int ga_launch_s(dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, bf16_t* qp, const bf16_t* k,
                        const bf16_t* vt, const float* vmax, const bf16_t* w, const int32_t* idx,
                        const float* slope, const bf16_t* swa_o, bf16_t* o, float* lse, const GaDims& dm) {
@@ -699,7 +757,7 @@ static int ga_launch_s(dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, 
   // Narrow heads leave the wavefronts under 168 registers: twelve of them per workgroup (one workgroup
   // per compute unit, its size is what sets the occupancy) instead of eight.
   constexpr int NT = (D <= 64 && DV <= 64) ? GA_THREADS_NARROW : GA_THREADS;
-  auto kern = sparse_attn_fwd_gather<D, DV, G, SLOPE, NT>;
+  auto kern = sparse_attn_fwd_gather<D, DV, G, SLOPE, NT, FINE>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_sparse_attn_fwd")) return rc;
   hipLaunchKernelGGL(kern, grid, dim3(NT), smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
@@ -709,22 +767,24 @@ static int ga_launch_s(dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, 
 template <int D, int DV, int G>
 static int ga_launch(dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, bf16_t* qp, const bf16_t* k,
                      const bf16_t* vt, const float* vmax, const bf16_t* w, const int32_t* idx,
-                     const float* slope, const bf16_t* swa_o, bf16_t* o, float* lse, const GaDims& dm) {
-  if (slope) return ga_launch_s<D, DV, G, true>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
-  return ga_launch_s<D, DV, G, false>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
+                     const float* slope, const bf16_t* swa_o, bf16_t* o, float* lse, bool fine, const GaDims& dm) {
+  if constexpr (D == DV && G <= 8)  // (what decode_step takes)
+    if (fine && !slope) return ga_launch_s<D, DV, G, false, true>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
+  if (slope) return ga_launch_s<D, DV, G, true, false>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
+  return ga_launch_s<D, DV, G, false, false>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
 }
 
 template <int D, int DV>
 static int ga_dispatch_g(int G, dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, bf16_t* qp,
                          const bf16_t* k, const bf16_t* vt, const float* vmax, const bf16_t* w,
                          const int32_t* idx, const float* slope, const bf16_t* swa_o, bf16_t* o, float* lse,
-                         const GaDims& dm) {
+                         bool fine, const GaDims& dm) {
   switch (G) {
-    case 1: return ga_launch<D, DV, 1>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
-    case 2: return ga_launch<D, DV, 2>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
-    case 4: return ga_launch<D, DV, 4>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
-    case 8: return ga_launch<D, DV, 8>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
-    case 16: return ga_launch<D, DV, 16>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, dm);
+    case 1: return ga_launch<D, DV, 1>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, fine, dm);
+    case 2: return ga_launch<D, DV, 2>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, fine, dm);
+    case 4: return ga_launch<D, DV, 4>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, fine, dm);
+    case 8: return ga_launch<D, DV, 8>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, fine, dm);
+    case 16: return ga_launch<D, DV, 16>(grid, smem, st, q, qp, k, vt, vmax, w, idx, slope, swa_o, o, lse, fine, dm);
   }
   return -1;
 }
@@ -800,7 +860,7 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
                               const int32_t* indices, const float* slope, const void* swa_o, int merge_col,
                               void* o, float* lse, void* workspace, int workspace_ready, int B, int L,
                               int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int S, float sm_scale,
-                              int mask_last, int q_block, int WH, float sm_n, void* stream,
+                              int mask_last, int q_block, int WH, float sm_n, bool fine, void* stream,
                               int* handled) {
   *handled = 0;
   const int G = HQ / H;
@@ -829,7 +889,7 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
   int rc = -1;
 #define GA_CALL(D_, DV_)                                                                       \
   rc = ga_dispatch_g<D_, DV_>(G, grid, smem, st, (const bf16_t*)q, qpk, kpk, vpk, vmax,        \
-                              (const bf16_t*)weights, indices, slope, (const bf16_t*)swa_o, (bf16_t*)o, lse, dm)
+                              (const bf16_t*)weights, indices, slope, (const bf16_t*)swa_o, (bf16_t*)o, lse, fine, dm)
   if (D == 64 && Dv == 64) GA_CALL(64, 64);
   else if (D == 128 && Dv == 128) GA_CALL(128, 128);
   else if (D == 64 && Dv == 128) GA_CALL(64, 128);

@@ -38,6 +38,7 @@ SIGNATURES = {
     "hils_decode_step_paged_ws": [_P] * 13 + [_I] * 12 + [_F, _F, _I, _I, _I, _I, _I, _P, _Z, _P],
     "hils_topk_bwd": [_P] * 7 + [_Z] + [_I] * 8 + [_F, _P],
     "hils_sparse_attn_fwd": [_P] * 10 + [_Z] + [_I] * 13 + [_F, _I, _F, _I, _P],
+    "hils_sparse_attn_fwd_fine": [_P] * 7 + [_Z] + [_I] * 10 + [_F, _I, _P],
     "hils_pack_kv_chunks": [_P, _P, _P, _Z, _I, _I, _I, _I, _I, _P],
     "hils_sparse_attn_bwd": [_P] * 13 + [_Z] + [_I] * 12 + [_F, _I, _F, _P, _P, _I, _I, _P],
     "hils_sparse_attn_fwd_f32": [_P] * 8 + [_I] * 12 + [_F, _I, _F, _P],

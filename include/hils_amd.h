@@ -194,11 +194,17 @@ int hils_sparse_attn_fwd(const void* q, const void* k, const void* v, const void
                          float* lse, void* workspace, size_t workspace_bytes, int workspace_ready, int B,
                          int L, int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int WH, int q_block,
                          int S, float sm_scale, int mask_last, float sm_n, int merge_col, void* stream);
+/* The same without the options, for the calls that would otherwise run on the decode kernels: the prefill kernel's
+ * output sums keep 29 instead of 20 bits below a row's bound sum|w| max|V| (the decode kernels sum in fp32). */
+int hils_sparse_attn_fwd_fine(const void* q, const void* k, const void* v, const void* weights,
+                              const int32_t* indices, void* o, void* workspace, size_t workspace_bytes, int B,
+                              int L, int Lkv, int HQ, int H, int D, int Dv, int K, int NW, int S, float sm_scale,
+                              int mask_last, void* stream);
 /* Fills a workspace of hils_sparse_attn_fwd_workspace(...) bytes on its own: per 64-token
  * chunk of a (batch, KV head), K and V rewritten in the register order of the MFMA operands
  * the prefill kernel loads (every operand load becomes one contiguous 1 KiB burst), followed
- * by max|V| of every chunk (fp32).  No counterpart in the reference (TileLang stages K/V
- * through shared memory on every use). */
+ * by max|V| of every chunk (fp32, NaNs left out, the sign bit set when the chunk holds a NaN or an
+ * infinity).  No counterpart in the reference (TileLang stages K/V through shared memory on every use). */
 int hils_pack_kv_chunks(const void* k, const void* v, void* workspace, size_t workspace_bytes, int B,
                         int Lkv, int H, int D, int Dv, void* stream);
 
