@@ -938,11 +938,12 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
       }
       delta = rows_sum(delta);
       if (j == 0 && qs <= last) dw_blk[__umul24((unsigned)pk >> 8, w_step) + w_row0 + ((unsigned)pk & 255u)] = delta;
-      const float f = w_row * out_scale, fd = -f * delta;
+      const float f = w_row * out_scale;
       bf16x8_t ap[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
-        auto ds = [&](int mt, int i) __attribute__((always_inline)) { return st[mt][i] * fmaf(dpt[mt][i], f, fd); };
+        // (the difference first: a product rounded before the cancellation leaves its error behind)
+        auto ds = [&](int mt, int i) __attribute__((always_inline)) { return f * st[mt][i] * (dpt[mt][i] - delta); };
         uint4 x;
         x.x = pack_bf2(ds(2 * s2, 0), ds(2 * s2, 1));
         x.y = pack_bf2(ds(2 * s2, 2), ds(2 * s2, 3));
