@@ -198,15 +198,14 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
     for (int w = 0; w < SR_WAVES; ++w) M = fmaxf(M, m_s[w][row]);
     float L = 0.f;
     f32x4_t x = {0.f, 0.f, 0.f, 0.f};
-    if (M > HILS_NEG_INF) {
+    // (no maximum: nothing was seen, and the sums are zero, or scores that are not numbers, which the sums keep)
 #pragma unroll
-      for (int w = 0; w < SR_WAVES; ++w) {
-        const float f = __builtin_amdgcn_exp2f((m_s[w][row] - M) * c2);
-        const f32x4_t ow = *(const f32x4_t*)((const float*)(area_s + w * AREA) + row * OP + d4 * 4);
-        L = fmaf(f, l_s[w][row], L);
+    for (int w = 0; w < SR_WAVES; ++w) {
+      const float f = M > HILS_NEG_INF ? __builtin_amdgcn_exp2f((m_s[w][row] - M) * c2) : 1.f;
+      const f32x4_t ow = *(const f32x4_t*)((const float*)(area_s + w * AREA) + row * OP + d4 * 4);
+      L = fmaf(f, l_s[w][row], L);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = fmaf(f, ow[i], x[i]);
-      }
+      for (int i = 0; i < 4; ++i) x[i] = fmaf(f, ow[i], x[i]);
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
     const long rix = (b * dm.Lq + tr) * (long)dm.HQ + hk * G + row % G;

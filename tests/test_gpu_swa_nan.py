@@ -1,0 +1,30 @@
+"""A query or key that is not a number shows in the local branch's output, whichever kernel the shape runs on."""
+import pytest
+import torch
+
+from util import note
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("HQ,H,D,Dv", [(4, 4, 64, 64), (16, 2, 128, 128), (8, 1, 64, 128)])
+@pytest.mark.parametrize("B,L,training", [(1, 96, True), (1, 3, False), (2, 3000, True)])  # rows of a few blocks, a step, tiles
+def test_nan_shows(pkg, dev, HQ, H, D, Dv, B, L, training):
+    note(f"local branch with a NaN, B{B} L{L} heads {HQ}/{H} x {D}/{Dv}")
+    gen = torch.Generator(device=dev).manual_seed(L)
+    Lk = L if training else L + 200
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev).bfloat16()
+    q, k, v = r(B, L, HQ, D), r(B, Lk, H, D), r(B, Lk, H, Dv)
+    o0, lse0 = pkg.flex_attn_tl(q, k, v, 64, 64, training=training)
+    bad = q.clone()
+    bad[B - 1, L - 1, 1, 5] = float("nan")
+    o, lse = pkg.flex_attn_tl(bad, k, v, 64, 64, training=training)
+    hit = torch.zeros(B, L, HQ, dtype=torch.bool, device=dev)
+    hit[B - 1, L - 1, 1] = True
+    assert o.isnan().all(-1).equal(hit) and o.isnan().any(-1).equal(hit)
+    assert torch.equal(o[~hit], o0[~hit]) and torch.equal(lse[~hit], lse0[~hit])
+    bad = k.clone()
+    bad[0, Lk - 2, 0, 7] = float("nan")
+    o, _ = pkg.flex_attn_tl(q, bad, v, 64, 64, training=training, mask_lmk=False)
+    G = HQ // H
+    assert o[0, L - 1, :G].isnan().all() and not o[0, L - 1, G:].isnan().any()
