@@ -630,24 +630,6 @@ Tensor sparse_attn(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
 // ---- decode steps ------------------------------------------------------------------------------------
 using Step = std::tuple<Tensor, Tensor, Tensor, Tensor>;  // o, weights, indices, scores
 
-// Many queries per sequence (a prompt's next slice on a cache).  The one-launch kernel reads a row's chunk keys
-// and its topk chunks for every row, at about 10 TB/s out of the caches, and no row faster than every 33 ns.  The
-// prefill kernels repack the whole cache (8 bytes per cache element at 5.9 TB/s), select, and read a chunk once for
-// all queries of a block that selected it, about 80 GB/s per block.  In us, one launch / prefill kernels: 128 queries
-// on 64K tokens, 32/8 heads of 128, top-32: 144 / 209, 256 queries 270 / 258, 512 queries 529 / 312; 163 queries on 35K,
-// 16/2 heads of 64: 23 / 55; 512 queries on 4K, 4/4 heads of 64, top-8: 72 / 49.
-bool prefill_kernels_ahead(int64_t B, int64_t L, int64_t N, int64_t Lkv, int64_t hkv, int64_t G, int64_t D,
-                           int64_t topk, bool per_qhead) {
-  const double rows = (double)B * L * hkv, chunk = 64.0 * D * 4, keys = (double)N * (per_qhead ? G : 1) * D * 2;
-  const double one = 12 + rows * std::max(0.033, (keys + topk * chunk) / 10.5e6);
-  const double by_row = 8 + rows * std::max(0.019, keys / 9.5e6);  // the selection, as hils_topk_fwd chooses
-  const double by_group = per_qhead ? 20 + N / 28.0 : (G == 1 ? 16 + N / 15.0 : 12 + N / 40.0);
-  const double block = std::max(4.0, rows / 256);  // queries of a workgroup
-  const double visits = N * (1 - std::exp(-block * topk / N));
-  const double two = 13 + std::min(by_row, by_group) + (double)B * Lkv * hkv * D * 8 / 5.9e6 + 10 + visits * chunk / 80e3;
-  return two < one;
-}
-
 Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v, const Tensor& lse_swa, int64_t topk,
                  int64_t block, int64_t window, int64_t q_offset, std::optional<double> sm_scale, bool mask_last,
                  const OptTensor& prior_b, bool head_major, std::optional<int64_t> num_chunks, py::object debug) {
@@ -679,7 +661,8 @@ Step decode_step(const Tensor& q, Tensor lmks, const Tensor& k, const Tensor& v,
       pb = prior_bias(pb, B, N, hq);
     }
   }
-  bool two_calls = L >= 64 && prefill_kernels_ahead(B, L, N, Lkv, hkv, G, D, topk, per_qhead);
+  bool two_calls = block == 64 && hils_decode_step_prefill_ahead(i32(B), i32(L), i32(N), i32(Lkv), i32(hq), i32(hkv), i32(D),
+                                                                 i32(topk), per_qhead);
   two_calls = two_calls || Lkv < N * block ||
               !hils_decode_step_covers(i32(B), i32(L), i32(N), i32(hq), i32(hkv), i32(D), i32(topk), i32(block),
                                        (int)pb.defined());

@@ -855,6 +855,13 @@ size_t hils_ga_workspace_bytes(int B, int L, int Lkv, int HQ, int H, int D, int 
          (size_t)B * L * HQ * D * sizeof(bf16_t);  // packed V, packed K, per-chunk max|V|, packed Q
 }
 
+// Queries of a workgroup for a call of one index row per query, 0 if the MFMA path does not take it.
+int hils_ga_block(int B, int L, int Lkv, int HQ, int H, int D, int K) {
+  if (hils_ga_workspace_bytes(B, L, Lkv, HQ, H, D, D, K, GA_S, 1, HQ, 0.f) == 0) return 0;
+  size_t smem;
+  return ga_pick_T(L, (long)B * H, HQ / H, D, K, Lkv / GA_S, 1, &smem);
+}
+
 // Returns HILS_OK and sets *handled = 1 when the MFMA path ran.
 int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const void* weights,
                               const int32_t* indices, const float* slope, const void* swa_o, int merge_col,

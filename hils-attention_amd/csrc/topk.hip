@@ -2548,12 +2548,42 @@ static bool topk_use_split(int B, int L, int N, int h_kv) {
 // which grows with the chunks.  (us, row / one-pass, at 500 chunks: 1024 rows of 4 heads of 128 28 / 25, 4096 rows 85 / 30,
 // with a key for each of 8 heads 4096 rows of 128 470 / 52; at 1023 chunks 256 rows of 128 14 / 39, 4096 rows 107 / 49, with
 // a key for each of 8 heads 256 rows 54 / 104, 4096 rows 830 / 135.)
-static bool topk_group_ahead(long rows, int N, int G, int D, int per_qhead) {
+static double topk_row_us(long rows, int N, int G, int D, int per_qhead) {
   const double key_bytes = (double)N * (per_qhead ? G : 1) * D * 2;
-  const double row_us = 8.0 + rows * (key_bytes > 180e3 ? key_bytes / 9.5e6 : 0.019);
-  const double group_us = per_qhead ? (G > 4 && N > 512 ? 20.0 + N / 14.0 : 20.0 + N / 28.0)
-                                    : (G == 1 ? 16.0 + N / 15.0 : 12.0 + N / 40.0);
-  return group_us < row_us;
+  return 8.0 + rows * (key_bytes > 180e3 ? key_bytes / 9.5e6 : 0.019);
+}
+static double topk_group_us(int N, int G, int per_qhead) {
+  return per_qhead ? (G > 4 && N > 512 ? 20.0 + N / 14.0 : 20.0 + N / 28.0) : (G == 1 ? 16.0 + N / 15.0 : 12.0 + N / 40.0);
+}
+static bool topk_group_ahead(long rows, int N, int G, int D, int per_qhead) {
+  return topk_group_us(N, G, per_qhead) < topk_row_us(rows, N, G, D, per_qhead);
+}
+
+// Many queries per sequence on a cache (a prompt's next slice): are selection and prefill attention ahead of the
+// one-launch step?  That reads a row's chunk keys and its topk chunks for every row, at about 10 TB/s out of the caches,
+// and no row faster than every 33 ns.  The prefill kernels repack the cache as it was handed over, all Lkv tokens of it
+// (8 bytes per element of K at 5.9 TB/s), select, and read a chunk once for all queries of a block that selected it, at
+// about 80 GB/s per block and round of the compute units.  In us, one launch / prefill kernels: 128 queries on 64K tokens,
+// 32/8 heads of 128, top-32: 144 / 209, 256 queries 270 / 258, 512 queries 529 / 312; 163 queries on 35K, 16/2 heads of 64:
+// 23 / 55; 512 queries on 4K, 4/4 heads of 64, top-8: 72 / 49.
+int hils_ga_block(int B, int L, int Lkv, int HQ, int H, int D, int K);  // queries of a block, 0: not covered
+extern "C" int hils_decode_step_prefill_ahead(int B, int L, int N, int Lkv, int HQ, int H, int D, int topk,
+                                              int lmk_per_qhead) {
+  if (B <= 0 || L < 64 || N <= 0 || H <= 0 || HQ <= 0 || HQ % H != 0 || topk <= 0) return 0;
+  const int T = hils_ga_block(B, L, Lkv, HQ, H, D, topk);
+  if (T == 0) return 0;  // (three, five, six or seven heads per KV head: the shape-generic kernel)
+  const int G = HQ / H;
+  const long rows = (long)B * L * H;
+  const double chunk = 64.0 * D * 4, keys = (double)N * (lmk_per_qhead ? G : 1) * D * 2;
+  const double one_row = (keys + topk * chunk) / 10.5e6;
+  const double one = 12 + rows * (one_row > 0.033 ? one_row : 0.033);
+  double sel = topk_row_us(rows, N, G, D, lmk_per_qhead);
+  if (hils_topk_group_covers(N, G, D, topk, lmk_per_qhead, true) && topk_group_us(N, G, lmk_per_qhead) < sel)
+    sel = topk_group_us(N, G, lmk_per_qhead);
+  const long wgs = (long)B * H * ((L + T - 1) / T);
+  const double visits = N * (1 - exp(-(double)T * topk / N)), rounds = (double)((wgs + topk_cus() - 1) / topk_cus());
+  const double two = 13 + sel + (double)B * Lkv * H * D * 8 / 5.9e6 + 10 + rounds * visits * chunk / 80e3;
+  return two < one ? 1 : 0;
 }
 
 // Shapes that hils_topk_fwd_weights hands to the one-pass prefill kernel, the only one that reads

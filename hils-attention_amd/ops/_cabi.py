@@ -33,6 +33,7 @@ SIGNATURES = {
     "hils_decode_step": [_P] * 12 + [_I] * 11 + [_F, _F, _I, _I, _I, _I, _P],
     "hils_decode_step_paged": [_P] * 13 + [_I] * 12 + [_F, _F, _I, _I, _I, _I, _I, _P],
     "hils_decode_step_lds": [_I] * 6,
+    "hils_decode_step_prefill_ahead": [_I] * 9,
     "hils_decode_step_workspace": [_I] * 9,
     "hils_decode_step_ws": [_P] * 12 + [_I] * 11 + [_F, _F, _I, _I, _I, _I, _P, _Z, _P],
     "hils_decode_step_paged_ws": [_P] * 13 + [_I] * 12 + [_F, _F, _I, _I, _I, _I, _I, _P, _Z, _P],

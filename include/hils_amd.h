@@ -311,6 +311,9 @@ int hils_sparse_attn_decode_paged(const void* q, const void* k_pages, const void
  * that with eight head rows) it shares the logits' array and a winner's raw score is its biased logit
  * minus the bias (one fp32 rounding away from the product, far inside the bf16 it is returned in). */
 int hils_decode_step_covers(int B, int L, int N, int HQ, int H, int D, int topk, int block_size, int with_bias);
+/* 1 when a step of many queries per sequence (64 and more) is faster as hils_topk_fwd_weights + hils_sparse_attn_fwd_fine
+ * on the prefill kernels than as one launch, by a model of both; Lkv: the tokens K and V are handed over with. */
+int hils_decode_step_prefill_ahead(int B, int L, int N, int Lkv, int HQ, int H, int D, int topk, int lmk_per_qhead);
 /* Bytes of LDS the workgroup of a (query, KV head) row takes in the decode step's kernels (lmk_paged: the chunk keys
  * are addressed through the page table), 0 if the selection of N chunks does not fit; at most 160 KiB for every
  * shape that hils_decode_step_covers accepts. */
