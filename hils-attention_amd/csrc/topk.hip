@@ -2559,6 +2559,41 @@ static bool topk_group_ahead(long rows, int N, int G, int D, int per_qhead) {
   return topk_group_us(N, G, per_qhead) < topk_row_us(rows, N, G, D, per_qhead);
 }
 
+// Past 512 visible chunks a query's logits take 64 registers a lane and leave one wavefront per SIMD, and the one-pass
+// kernel's time no longer depends on how many chunks there are.  With two to four heads on shared keys, and with a key for
+// each of five to eight heads, the two-pass kernel is ahead there once it has queries enough to fill the chip.  us,
+// one-pass / two-pass: whole prompts, 32/8 heads of 128: 577 chunks 647 / 693, 640 chunks 831 / 775, 1024 chunks
+// 2095 / 1577; 16/8 of 64: 596 / 593, 1508 / 1242; a key per head, 32/4 of 64: 1331 / 1469, 3548 / 2934, 40/8 of 64:
+// 2483 / 2019, 6711 / 4140; the last 1024 queries of 768 chunks, 32/8 of 128: 79 / 94, the last 2048: 136 / 110, the last
+// 16384: 849 / 509.  Elsewhere it is not (one head: 3010 / 3823, five to eight on shared keys: 2212 / 3683, a key for each
+// of three or four: 2987 / 4388).  Both times below are fits to such measurements, in us.
+static bool topk_two_pass_ahead(int B, int L, int N, int h_kv, int G, int D, int per_qhead, int block_size, int window_size,
+                                int causal, int q_offset) {
+  if (N <= 512 || (per_qhead ? G < 5 : G < 2 || G > 4)) return false;
+  auto limit = [&](int t) -> int {
+    const int lm = causal ? visible_limit(t + q_offset, window_size, block_size) : N;
+    return lm < 0 ? 0 : (lm > N ? N : lm);
+  };
+  int lo = 0, hi = L;  // first query that sees more than 512 chunks
+  while (lo < hi) {
+    const int mid = lo + (hi - lo) / 2;
+    if (limit(mid) <= 512) lo = mid + 1; else hi = mid;
+  }
+  const double unit = (double)B * h_kv, rows = unit * L, wide = unit * (L - lo), n = 0.5 * (limit(0) + limit(L - 1));
+  double one, two;
+  if (per_qhead) {
+    one = 25 + (rows - wide) * (D == 64 ? 4.6e-3 : 5.3e-3) + (D == 64 ? 46 : 52) * ceil(wide / (8 * topk_cus()));
+    two = (200 + rows * (D == 64 ? 2.5e-3 + 17e-6 * n : 5.0e-3 + 19.5e-6 * n)) * G / 8;
+  } else if (G == 2) {
+    one = 25 + (rows - wide) * 1.3e-3 + 41 * ceil(wide / (32 * topk_cus()));
+    two = 60 + rows * (1.0e-3 + 3.0e-6 * n);
+  } else {
+    one = 25 + (rows - wide) * (D == 64 ? 1.4e-3 : 1.7e-3) + (D == 64 ? 24.5 : 26.6) * ceil(wide / (16 * topk_cus()));
+    two = 70 + rows * (D == 64 ? 1.05e-3 + 3.0e-6 * n : 1.15e-3 + 3.15e-6 * n);
+  }
+  return two < one;
+}
+
 // Many queries per sequence on a cache (a prompt's next slice): are selection and prefill attention ahead of the
 // one-launch step?  That reads a row's chunk keys and its topk chunks for every row, at about 10 TB/s out of the caches,
 // and no row faster than every 33 ns.  The prefill kernels repack the cache as it was handed over, all Lkv tokens of it
@@ -2592,7 +2627,7 @@ extern "C" int hils_topk_lse16_covers(int B, int L, int N, int h_kv, int G, int 
   if (B <= 0 || L <= 0 || N <= 0 || h_kv <= 0 || G <= 0) return 0;
   if (topk_use_split(B, L, N, h_kv)) return 0;
   if (L <= 4 && topk_use_row((long)B * L * h_kv, N, G, D, 0, true)) return 0;
-  return hils_topk_group_covers(N, G, D, topk, 0, true) ? 1 : 0;
+  return N <= 512 && hils_topk_group_covers(N, G, D, topk, 0, true) ? 1 : 0;  // (further: topk_two_pass_ahead may decide)
 }
 
 static size_t topk_ws_key_bytes(int B, int N, int h_kv, int G) {
@@ -2714,7 +2749,9 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
   }
   // the one-pass kernel with one chunk key per query head (a wavefront per head for the logits, G = 3..8),
   // or with more than four query heads on shared keys (two wavefronts per four queries)
-  if ((per_qhead || G > 4) && workspace && hils_topk_group_covers(N, G, D, topk, per_qhead, !gumbel && !drop_mask)) {  // (G = 2..8 / 5..8)
+  const bool two_pass = topk_two_pass_ahead(B, L, N, h_kv, G, D, per_qhead, block_size, window_size, causal, q_offset);
+  if ((per_qhead || G > 4) && workspace && !two_pass &&
+      hils_topk_group_covers(N, G, D, topk, per_qhead, !gumbel && !drop_mask)) {  // (G = 2..8 / 5..8)
     const int nblk16 = (N + 15) / 16;
     const int h_lmk = per_qhead ? h_kv * G : h_kv;
     const long total = (long)B * h_lmk * nblk16 * (D / 32) * 64;
@@ -2727,9 +2764,9 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
     HILS_CHECK_LAUNCH("hils_topk_fwd");
     return HILS_OK;
   }
-  // one chunk key per query head outside that kernel's envelope (more than 512 chunks, more than 32
-  // winners, noise, a drop mask), or five to eight query heads on shared keys: the two-pass MFMA kernel,
-  // 16 queries a wavefront, head by head
+  // one chunk key per query head outside that kernel's envelope (more than 1024 chunks or 32 winners, noise, a drop mask)
+  // or behind its line, or five to eight query heads on shared keys: the two-pass MFMA kernel, 16 queries a
+  // wavefront, head by head
   if ((per_qhead || G > 4) && workspace && G <= 8 && (D == 64 || D == 128)) {
     const int nblk16 = (N + 15) / 16;
     const int h_lmk = per_qhead ? h_kv * G : h_kv;
@@ -2778,8 +2815,8 @@ static int topk_fwd_impl(const void* q, const void* lmks, const float* lse_swa,
       hipLaunchKernelGGL(topk_pack_lmk_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
                          (const bf16_t*)lmks, (uint4*)workspace, N, h_kv, D, nblk16, total);
       packed = (const uint4*)workspace;
-      // up to 512 chunks and 32 winners, nothing added to the logits: the one-pass kernel
-      if (hils_topk_group_covers(N, G, D, topk, per_qhead, !gumbel && !drop_mask)) {
+      // up to 1024 chunks and 32 winners, no noise, no drop mask: the one-pass kernel
+      if (!two_pass && hils_topk_group_covers(N, G, D, topk, per_qhead, !gumbel && !drop_mask)) {
         if (int rc2 = hils_topk_group_launch(q, packed, lse_swa, bias, indices, scores, lse_total, sel_logits, B, L, N,
                                              h_kv, G, D, topk, block_size, window_size, causal, q_offset,
                                              sm_scale, lse_bf16, 0, stream))
