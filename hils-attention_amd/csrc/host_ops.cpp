@@ -477,7 +477,8 @@ struct WeightsFn : torch::autograd::Function<WeightsFn> {
       ctx->set_materialize_grads(false);
       ctx->save_for_backward({sc, lse, pb, idx});
       ctx->saved_data["cfg"] = std::vector<int64_t>{H, N, sm1, (int64_t)lse_swa.scalar_type(),
-                                                    prior_b.defined() ? (int64_t)prior_b.scalar_type() : -1};
+                                                    prior_b.defined() ? (int64_t)prior_b.scalar_type() : -1,
+                                                    lse_swa.requires_grad(), prior_b.defined() && prior_b.requires_grad()};
       ctx->saved_data["lse_shape"] = lse_swa.sizes().vec();
     }
     return out;
@@ -490,13 +491,14 @@ struct WeightsFn : torch::autograd::Function<WeightsFn> {
     const Tensor &sc = s[0], &lse = s[1], &pb = s[2], &idx = s[3];
     const int64_t B = sc.size(0), L = sc.size(1), HQ = sc.size(2), K = sc.size(3), N = cfg[1];
     const Tensor dw = g[0].to(sc.scalar_type()).contiguous();
-    Tensor d_sc = at::empty_like(sc), d_lse = new_tensor({B, L, HQ}, sc, at::kFloat);
-    Tensor d_pb = pb.defined() ? at::zeros({B, N, HQ}, sc.options().dtype(at::kFloat)) : Tensor();
+    // (what nobody asked for is neither filled nor written)
+    Tensor d_sc = at::empty_like(sc), d_lse = cfg[5] ? new_tensor({B, L, HQ}, sc, at::kFloat) : Tensor();
+    Tensor d_pb = cfg[6] ? at::zeros({B, N, HQ}, sc.options().dtype(at::kFloat)) : Tensor();
     HILS_CALL(hils_chunk_weights_bwd, cptr(sc), cptr(lse), (int)(lse.scalar_type() == at::kBFloat16), fptr(pb),
               iptr(idx), cptr(dw), mptr(d_sc), mfptr(d_lse), mfptr(d_pb), i32(B), i32(L), i32(HQ), i32(cfg[0]), i32(N),
               i32(K), i32(cfg[2]));
     out[0] = d_sc;
-    out[1] = d_lse.reshape(ctx->saved_data["lse_shape"].toIntVector()).to((at::ScalarType)cfg[3]);
+    if (d_lse.defined()) out[1] = d_lse.reshape(ctx->saved_data["lse_shape"].toIntVector()).to((at::ScalarType)cfg[3]);
     if (d_pb.defined()) out[2] = d_pb.to((at::ScalarType)cfg[4]);
     return out;
   }

@@ -1,0 +1,40 @@
+"""chunk_weights backward with every combination of inputs that want a gradient."""
+import itertools
+
+import pytest
+import torch
+
+from util import assert_close_bf16, note
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("want", [w for w in itertools.product((False, True), repeat=3) if any(w)])
+def test_only_what_is_asked_for(pkg, dev, want):
+    note(f"chunk_weights gradients of scores, lse, prior: {want}")
+    gen = torch.Generator(device=dev).manual_seed(23)
+    B, L, HQ, H, K, N = 1, 64, 16, 4, 8, 100000
+    sc = torch.randn(B, L, HQ, K, device=dev, generator=gen).bfloat16()
+    lse = torch.randn(B, L, HQ, device=dev, generator=gen) + 1
+    pb = torch.randn(B, N, HQ, device=dev, generator=gen).bfloat16()
+    idx = torch.randint(0, N, (B, L, H, K), device=dev, generator=gen, dtype=torch.int32)
+    g = torch.randn(B, L, HQ, K + 1, device=dev, generator=gen).bfloat16()
+    ins = [x.clone().requires_grad_(w) for x, w in zip((sc, lse, pb), want)]
+    ref_in = [x.float().clone().requires_grad_() for x in (sc, lse, pb)]
+    at = idx.long().repeat_interleave(HQ // H, 2)                                            # (B, L, HQ, K)
+    bias = ref_in[2][0].t()[torch.arange(HQ, device=dev).view(1, 1, HQ, 1), at]
+    ref = torch.softmax(torch.cat([ref_in[0] + bias, ref_in[1].unsqueeze(-1)], -1), -1)
+    ref_g = torch.autograd.grad(ref, ref_in, g.float())
+    out = pkg.chunk_weights(ins[0], ins[1], ins[2], idx)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out.backward(g)
+    torch.cuda.synchronize()
+    used = torch.cuda.max_memory_allocated() - before
+    if not want[2]:
+        assert used < 4 * N * HQ, "the prior's gradient was not asked for: nothing of its size is allocated"
+    for name, x, w, r in zip(("scores", "lse", "prior"), ins, want, ref_g):
+        assert (x.grad is not None) == w
+        if w:
+            assert_close_bf16(x.grad, r, name)
