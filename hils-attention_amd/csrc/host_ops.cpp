@@ -739,7 +739,7 @@ std::tuple<Tensor, Tensor, Tensor> paged_step(const Tensor& q, const Tensor& k_p
   HOST_ASSERT(HQ % H == 0, "HQ=", HQ, " must be divisible by H=", H);
   const int64_t G = HQ / H, N = seq_len / S;  // chunks with a pooled key
   HOST_ASSERT(0 < N && N <= max_pages, "seq_len ", seq_len, " has no whole chunk or more than the page table");
-  const int64_t hl = dense ? lmk.size(1) : lmk.size(1);
+  const int64_t hl = lmk.size(1);
   HOST_ASSERT(hl == H || hl == HQ, "the chunk keys carry ", hl, " heads: neither the ", H, " KV heads nor the ", HQ,
               " query heads");
   const int per_qhead = hl != H;

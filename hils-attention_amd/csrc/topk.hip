@@ -2067,8 +2067,9 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_step_kernel(DsArgs a) {
   // With at most one row per compute unit all rows run in step: every compute unit streams keys, then
   // every one sits in the selection's tail with the memory system idle, then every one streams K and V.
   // Half of the rows (every other one of an XCD's) start a little late, so that one half's tail falls
-  // into the other half's streaming (256 rows of 2048 keys and 32 chunks at D = 128: 79 us without, 72.0 with
-  // 3 us, 70.2 with 6, 70.4 with 8; 1024 keys: 62.4, 57.5, 57.7, 59.6).
+  // into the other half's streaming (256 rows of 2048 keys and 32 chunks at D = 128, kernel time in us back to back /
+  // alone: 75.6 / 73.5 without, 74.8 / 73.0 with 3 us, 72.5 / 71.1 with 6, 73.1 / 70.9 with 8; 1024 keys: 65.0 / 59.7,
+  // 64.7 / 58.3, 63.1 / 57.7, 64.6 / 60.4).
   if (a.stagger_ticks > 0 && ((blockIdx.x >> 3) & 1)) {
     const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
     while (__builtin_amdgcn_s_memrealtime() - t0 < (unsigned long long)a.stagger_ticks) __builtin_amdgcn_s_sleep(8);

@@ -133,17 +133,6 @@ def nbytes(t):
     return 0 if t is None else t.numel() * t.element_size()
 
 
-def gpu_readable(t, device):
-    """A contiguous tensor the kernels can read: ``t`` itself when it is contiguous in device memory
-    or in pinned host memory; otherwise a contiguous copy in device memory (a copy of a pinned
-    tensor made on the host would land in pageable memory, which the GPU cannot address)."""
-    if t.is_contiguous() and (t.is_cuda or t.is_pinned()):
-        return t
-    if t.is_cuda:
-        return t.contiguous()
-    return t.to(device, non_blocking=True).contiguous()
-
-
 def stream():
     return c_void_p(torch.cuda.current_stream().cuda_stream)
 
@@ -173,14 +162,6 @@ def sparse_attn_fwd_workspace_bytes(B, L, Lkv, HQ, H, D, Dv, K, WH, q_block, S, 
 def sparse_attn_fwd_workspace(device, B, L, Lkv, HQ, H, D, Dv, K, WH, q_block, S, sm_n):
     """Scratch tensor for hils_sparse_attn_fwd (None when the shape needs none)."""
     n = sparse_attn_fwd_workspace_bytes(B, L, Lkv, HQ, H, D, Dv, K, WH, q_block, S, sm_n)
-    if n == 0:
-        return None
-    return torch.empty(n, dtype=torch.uint8, device=device)
-
-
-def topk_bwd_workspace(device, B, L, N, h_kv, G, D, topk):
-    """Scratch tensor for hils_topk_bwd (None when the shape needs none)."""
-    n = load().hils_topk_bwd_workspace(B, L, N, h_kv, G, D, topk)
     if n == 0:
         return None
     return torch.empty(n, dtype=torch.uint8, device=device)

@@ -65,16 +65,20 @@ def head_major_chunk_keys(lmks, prior_b=None, capacity=None, num_kv_heads=None):
 def decode_step(q, lmks, k, v, lse_swa, topk, block_size, window_size, q_offset=0, sm_scale=None,
                 mask_last_token=True, _debug=None, prior_b=None, lmk_head_major=False, num_chunks=None):
     """Inference: the remote branch of a decode step, ``topk_chunk_weights`` followed by
-    ``HiLS_block_M_head(..., is_training=False)`` on the selected chunks, in one kernel launch (one
-    workgroup per (query, KV head) selects and then attends).  q (B,L,h_q,D), lmks (B,N,h_kv,D), k, v
+    ``HiLS_block_M_head(..., is_training=False)`` on the selected chunks, as one kernel (one workgroup per
+    (query, KV head) selects and then attends) or, with few rows for the chip, two that split a row over
+    workgroups.  q (B,L,h_q,D), lmks (B,N,h_kv,D), k, v
     (B,Lkv,h_kv,D) bf16 (k, v may live in pinned host memory), lse_swa (B,L,h_q) -> o (B,L,h_q,D),
     weights (B,L,h_q,topk+1), indices (B,L,h_kv,topk), scores (B,L,h_q,topk).  ``prior_b`` (B,N,h_q):
     the layer's prior bias (selection bias and the bias of the inter-chunk softmax).
     ``lmk_head_major``: lmks is (B,h_kv,cap,D) and prior_b (B,h_kv,cap,G) (``head_major_chunk_keys``),
     of which the first ``num_chunks`` (default cap) chunks are looked at.  lmks may carry h_q heads
     instead of h_kv (one chunk key per query head, the layer's attention-pooled keys): (B,N,h_q,D) or,
-    head-major, (B,h_q,cap,D).  Shapes the fused kernel does not take (few rows, short caches, more
-    than eight query heads per KV head, ...) run as the two calls."""
+    head-major, (B,h_q,cap,D).  What the fused kernels do not take (more than eight query heads per KV head,
+    more chunks than fit the LDS, K and V shorter than the chunks) runs as the two calls, and so do 64 queries
+    per sequence and more where the prefill kernels are ahead.
+    q, k and v may have any strides (what is not contiguous is copied).  ``_debug`` (a dict) receives the fp32
+    ``sel_logits`` and ``lse_total`` of the selection."""
     return _cabi.host().decode_step(q, lmks, k, v, lse_swa, int(topk), int(block_size), int(window_size),
                                     int(q_offset), sm_scale, bool(mask_last_token), prior_b, bool(lmk_head_major),
                                     num_chunks, _debug)

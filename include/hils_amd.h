@@ -286,9 +286,9 @@ int hils_sparse_attn_decode_paged(const void* q, const void* k_pages, const void
  * hils_topk_fwd_weights_paged followed by hils_sparse_attn_decode_paged (paged cache), fused: what
  * the layer runs per generated token between the local branch and the merge
  * (models/FlashHiLS/hils_attention.py:568-623 on the cached keys of utils/hils_cache_utils.py:34-62).
- * One workgroup per (query, KV head) row selects the row's chunks, writes indices / scores / weights
- * and then attends over the chunks it has selected: one launch instead of two, and the rows'
- * selection tails overlap other rows' memory streams.  Outputs as the two calls give them; o
+ * One workgroup per (query, KV head) row (several, with a workspace and few rows) selects the row's chunks, writes
+ * indices / scores / weights and then attends over the chunks it has selected: one launch instead of two,
+ * and the rows' selection tails overlap other rows' memory streams.  Outputs as the two calls give them; o
  * (B,L,HQ,D) bf16 is the remote branch's output (the caller adds swa_o * weights[..., topk]).
  * lse_total / sel_logits optional as in hils_topk_fwd.  q (B,L,HQ,D); k, v (B,Lkv,H,D) with
  * Lkv >= N * 64 or k_pages, v_pages (num_pages,H,64,D).
@@ -304,9 +304,8 @@ int hils_sparse_attn_decode_paged(const void* q, const void* k_pages, const void
  * and the bias gathered into the inter-chunk softmax), fp32, NULL for none; laid out like the chunk
  * keys with the G heads of a KV head in place of D: (B,N,H*G), (B,H,lmk_cap,G) or (num_pages,H*G).
  * Covered shapes (hils_decode_step_covers returns 1): causal, block_size 64,
- * D = Dv in {64, 128}, HQ/H <= 8, 256 <= N <= 4096 (with more than four query heads per KV head, whose
- * logits take eight rows of LDS: 2752 chunks at D = 128 and 3200 at D = 64, 2496 / 2880 with chunk keys
- * per page; the covers function knows), topk <= 64, at least 96 rows B*L*H.  A bias is staged in LDS
+ * D = Dv in {64, 128}, HQ/H <= 8, topk <= 64, 1 <= N <= 4096 (with more than four query heads per KV
+ * head, whose logits take eight rows of LDS: 2496 chunks at D = 128 and 2880 at D = 64).  A bias is staged in LDS
  * beside the logits; where the two do not fit side by side (from about 2900 chunks at D = 128, half of
  * that with eight head rows) it shares the logits' array and a winner's raw score is its biased logit
  * minus the bias (one fp32 rounding away from the product, far inside the bf16 it is returned in). */
