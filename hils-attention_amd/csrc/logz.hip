@@ -96,8 +96,9 @@ static dim3 lz_xcd_grid(int n_blk, int n_unit) {
 // compiler, free to use 512 registers at this workgroup size, parks them in accumulation registers
 // and copies every score back for the softmax; its upper bound keeps the scheduler from saving registers for
 // wavefronts that do not fit anyway, one LDS read and its wait behind the other)
-// Bound by vector-ALU issue: 207 vector instructions per 32 x 64 scores with a maximum per chunk and addresses worked
-// out per load, about 115 now; L 8192, 32/8 heads of 128: 390 -> 341 us.
+// Bound by vector-ALU issue: 222 vector instructions (counted, beside 32 matrix ones) per 32 x 64 scores with a maximum
+// per chunk and addresses worked out per load, 197 with fixed addresses, 174 where the maximum is not taken; L 8192,
+// 32/8 heads of 128: 390, 366 and 350 us.
 template <int D, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
@@ -198,8 +199,7 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       // the sum are rounded at the size of their distance from it.  The previous chunk's log sum serves while the
       // sums of the whole wavefront stay within [1/8, 8] of it, which scores of a standard deviation of 1 do (the error
       // against 64 bits is then a tenth below the maximum's; within 2^60 it was up to 1.2 times it with peaked
-      // scores); else the maximum is taken, a sixth of the vector instructions of a chunk.  The scale is applied inside
-      // the exponent's fused multiply-add.
+      // scores); else the maximum is taken.  The scale is applied inside the exponent's fused multiply-add.
       float x[16];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
@@ -259,7 +259,7 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 // (whose contraction runs over the streamed rows) comes through the transposing LDS load.  With a second, transposed
 // copy in LDS a tile took 16 lane permutations, 8 more stores and two barriers; L 8192, 32/8 heads of 128: dQ
 // 715 -> 530 us, dK 840 -> 635 us; what is left is vector-ALU and matrix
-// issue, 128 .. 150 vector instructions beside 64 matrix ones per tile.
+// issue, 150 to 160 vector instructions beside 64 matrix ones per tile.
 // The scores are computed with the
 // owned side as matrix columns, so their accumulator registers are already the left operand of
 // the gradient product.
