@@ -2,22 +2,22 @@
 //
 // dK and dV of a chunk are sums over every (query, head) row that selected the chunk, so
 // that side is computed chunk-major: an inverse index (for each (batch, KV head, chunk) the
-// list of (query, slot) pairs that hold it) is built by a counting sort, then one workgroup
-// per chunk streams its rows in tiles of 16, recomputes P and dS with the scores in the
+// list of (query, slot) pairs that hold it) is built by a counting sort, then a workgroup per
+// segment of a chunk's pairs streams its rows in rounds of 64, recomputes P and dS with the scores in the
 // orientation rows x tokens, and keeps dK, dV of the chunk in MFMA accumulators: no atomics,
-// one write per element.
+// one write per element (a chunk cut into several segments: one per segment, added up afterwards).
 //
-//   S  = Q K^T            (16 rows x 16 tokens per wavefront, 16x16x32 MFMA over d)
-//   dP = dO V^T           (same shape, 16x16x32 MFMA over dv)
+//   S  = Q K^T            (16x16x32 MFMA over d)
+//   dP = dO V^T           (16x16x32 MFMA over dv)
 //   P  = exp2(S c2 - lse2),  delta = sum_tokens P dP,  dS = w P (dP - delta)
-//   dV += (w P)^T dO      (16 tokens x Dv, 16x16x16 MFMA over the 16 rows)
-//   dK += scale dS^T Q    (16 tokens x D,  16x16x16 MFMA over the 16 rows)
+//   dV += (w P)^T dO      (tokens x Dv, 16x16x32 MFMA over 32 rows)
+//   dK += scale dS^T Q    (tokens x D,  16x16x32 MFMA over 32 rows)
 //
 // An accumulator-layout tile (lane: column = token, registers = rows 4j..4j+3) is, two row tiles
 // side by side, exactly the A operand of the 16x16x32 MFMA with the roles (row m = token, k = 32
 // rows), so P and dS feed the second pair of products without leaving registers.  Their B operands
 // (k = rows, n = feature) are columns of the gathered Q and dO rows: the workgroup stages the rows
-// row-major in LDS once per round for all four wavefronts (16 tokens each), and the column reads
+// row-major in LDS once per round for all four wavefronts, and the column reads
 // are the hardware's transposing LDS loads (a 16-lane group fetches a 4 x 16 block and every lane
 // receives one column of it).
 #include "decode_rows.h"
