@@ -654,11 +654,11 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   constexpr int DT = D / 16;
   constexpr int QT = 16 / G;
   constexpr int MAXP = BQ_MAXP;
-  extern __shared__ int smem_i[];
+  extern __shared__ __align__(16) int smem_i[];  // (16-byte row pieces are read from it)
   const int R = dm.T * G;
   int* q_acc = smem_i;                       // (R + 1) x D fixed point; row R takes padding rows
   int* cur = q_acc + (size_t)(R + 1) * D;    // nchunk: histogram -> running ends
-  unsigned short* pairs = (unsigned short*)(cur + dm.nchunk);  // T*K pairs (query << 8 | slot) grouped by chunk (T, K <= 256)
+  unsigned short* pairs = (unsigned short*)(cur + ((dm.nchunk + 3) & ~3));  // T*K pairs (query << 8 | slot) grouped by chunk (T, K <= 256)
   constexpr int QROWB = D * 2 + 16, OROWB = DV * 2 + 16;       // staged rows, padded (bytes)
   char* rows_q = (char*)pairs + (((size_t)dm.T * dm.K * 2 + 15) & ~(size_t)15);  // STAGE: R x QROWB
   char* rows_o = rows_q + (size_t)R * QROWB;                                     //        R x OROWB
@@ -1021,7 +1021,7 @@ void hils_ga_pack_launch(const void* a, const void* b, void* ap, void* bp, float
 // and the pair list (and, with `stage`, the block's own query and dO rows) fit in LDS; 0 when the
 // shape does not fit.
 static size_t bq_smem_bytes(int T, int G, int D, int Dv, int K, int nchunk, bool stage) {
-  size_t n = (size_t)(T * G + 1) * D * 4 + (size_t)nchunk * 4 + (((size_t)T * K * 2 + 15) & ~(size_t)15);
+  size_t n = (size_t)(T * G + 1) * D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + (((size_t)T * K * 2 + 15) & ~(size_t)15);
   if (stage) n += (size_t)T * G * ((size_t)D * 2 + 16 + (size_t)Dv * 2 + 16);
   return n;
 }
@@ -1029,7 +1029,7 @@ static int bq_pick_T(int L, int G, int D, int Dv, int K, int nchunk, bool stage,
   // the largest block that fits: the more rows share a visit, the fewer K/V bytes per row
   const size_t limit = 156 * 1024;
   const size_t per_q = (size_t)G * D * 4 + (size_t)K * 2 + (stage ? (size_t)G * ((size_t)(D + Dv) * 2 + 32) : 0);
-  const size_t fixed = (size_t)D * 4 + (size_t)nchunk * 4 + 16;  // spare row, histogram, alignment
+  const size_t fixed = (size_t)D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + 16;  // spare row, histogram, alignment
   if (fixed + per_q > limit) return 0;
   long T = (long)((limit - fixed) / per_q);
   if (T > 256) T = 256;  // a pair is (query << 8 | slot) in 16 bits
