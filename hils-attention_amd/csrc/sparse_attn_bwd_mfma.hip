@@ -629,8 +629,8 @@ bw_dkdv_sum_kernel(const int* __restrict__ offsets, void* __restrict__ dk_out, v
 // scaled by a power of two from the bound  scale * 2 * max_row(sum_k|w| * |dO|_1) * max|V| * max|K|.
 // ---------------------------------------------------------------------------
 #define BQ_THREADS 512
+#define BQ_STAGE_THREADS 768
 #define BQ_MAXP 16  // (query, slot) pairs of a block per thread
-#define BQ_WAVES (BQ_THREADS / 64)
 
 struct BqDims {
   int L, Lkv, HQ, H, B, K, NW, T, nblk, nchunk, mask_last;
@@ -639,12 +639,43 @@ struct BqDims {
   uint32_t k_magic;    // hils_udiv_magic(K)
 };
 
+typedef __attribute__((address_space(3))) int bq_lds_int;
+
+// Rows behind the output tile that padding rows add to: as many as one address serves (the heads of a query among the
+// four rows of a lane group).
+constexpr int bq_spare(int G) { return G < 4 ? G : 4; }
+
+// floor(x + 0.5) as an integer, one instruction (__float2int_rn is two).  The compiler counts no wait states between a
+// matrix product and inline assembly that reads its result: bq_settle waits out the 12 behind the last one.
+__device__ __forceinline__ void bq_settle(f32x4_t (&a)[4]) {
+  asm volatile("s_nop 11" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+}
+__device__ __forceinline__ int bq_round(float x) {
+  int i;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(i) : "v"(x));
+  return i;
+}
+
+// a tile's rows, this lane's: pair (query of the block << 8 | slot), pieces of its q and dO, lse, weight
+template <int KS, int VS>
+struct BqRows {
+  bw_u4 q[KS], o[VS];
+  float l2;
+  bf16_t wb;
+  unsigned pk;
+};
+
 // STAGE: the block's own query and dO rows are copied into LDS once (coalesced) and every tile
 // takes its row operands from there instead of gathering them from global memory once per (row,
-// slot) pair; chosen by the launcher when those rows fit beside the output tile without shrinking
-// the block much (narrow heads without grouping).
-template <int D, int DV, int G, bool STAGE>
-__global__ void __launch_bounds__(BQ_THREADS)
+// slot) pair (narrow heads; bq_stage_pays has the rule).  A tile is vector-ALU and LDS work with a matrix product at
+// either end, one wavefront's pieces hardly overlap, so the rows' short way from the LDS buys a third wavefront per
+// SIMD: their registers are loaded at their use, S before dP, and 12 wavefronts of at most 168 registers run instead of
+// 8.  B8 L8192 16/16 heads of 64, top-32, dQ: 1800 us with the rows off their 16-byte boundaries (a ds_read_b128 then
+// takes three times as long), 1550 on them, 1530 with 200 vector instructions a tile for 259 (row addresses without
+// clamps in full tiles, one-instruction rounding, nothing copied between tiles), 1480 with 12 wavefronts; 280 of it are
+// the block's set-up and end.
+template <int D, int DV, int G, bool STAGE, int NT>
+__global__ void __launch_bounds__(NT)
 bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const bf16_t* __restrict__ ka,
              const bf16_t* __restrict__ va, const bf16_t* __restrict__ kt, const float* __restrict__ vmax,
              const float* __restrict__ kmax, const bf16_t* __restrict__ weights,
@@ -656,14 +687,15 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   constexpr int MAXP = BQ_MAXP;
   extern __shared__ __align__(16) int smem_i[];  // (16-byte row pieces are read from it)
   const int R = dm.T * G;
-  int* q_acc = smem_i;                       // (R + 1) x D fixed point; row R takes padding rows
-  int* cur = q_acc + (size_t)(R + 1) * D;    // nchunk: histogram -> running ends
+  constexpr int SPARE = bq_spare(G);
+  int* q_acc = smem_i;                       // (R + SPARE) x D fixed point; padding rows add to the last SPARE
+  int* cur = q_acc + (size_t)(R + SPARE) * D;  // nchunk: histogram -> running ends
   unsigned short* pairs = (unsigned short*)(cur + ((dm.nchunk + 3) & ~3));  // T*K pairs (query << 8 | slot) grouped by chunk (T, K <= 256)
   constexpr int QROWB = D * 2 + 16, OROWB = DV * 2 + 16;       // staged rows, padded (bytes)
   char* rows_q = (char*)pairs + (((size_t)dm.T * dm.K * 2 + 15) & ~(size_t)15);  // STAGE: R x QROWB
   char* rows_o = rows_q + (size_t)R * QROWB;                                     //        R x OROWB
   __shared__ float red[32];
-  __shared__ int scan_s[BQ_WAVES];
+  __shared__ int scan_s[NT / 64];
   __shared__ int next_s;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -684,7 +716,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   int creg[MAXP], preg[MAXP];
 #pragma unroll
   for (int e = 0; e < MAXP; ++e) {
-    const int i = tid + e * BQ_THREADS;
+    const int i = tid + e * NT;
     int c = -1;
     preg[e] = 0;
     if (i < npair) {
@@ -697,7 +729,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   }
   // row bound: sum_k |w| * |dO|_1
   float rb = 0.f;
-  for (int row = tid; row < R; row += BQ_THREADS) {
+  for (int row = tid; row < R; row += NT) {
     const int ql = row / G, g = row - ql * G;
     if (t0 + ql < dm.L) {
       const long rowi = (b * dm.L + t0 + ql) * (long)dm.HQ + hk * G + g;
@@ -713,19 +745,19 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
       rb = fmaxf(rb, a * l1);
     }
   }
-  for (int i = tid; i < (R + 1) * D; i += BQ_THREADS) q_acc[i] = 0;
-  for (int i = tid; i < dm.nchunk; i += BQ_THREADS) cur[i] = 0;
+  for (int i = tid; i < (R + SPARE) * D; i += NT) q_acc[i] = 0;
+  for (int i = tid; i < dm.nchunk; i += NT) cur[i] = 0;
   if (tid == 0) next_s = 0;
   if (STAGE) {
     // rows beyond the sequence end are never addressed by a pair: they re-read the last row.  Four
     // loads in flight per thread and none inside a branch (a load inside a branch is waited for there).
     auto stage_rows = [&](const bf16_t* src, char* dst, int rowb, int npc) __attribute__((always_inline)) {
       const int n = R * npc;
-      for (int i0 = 0; i0 < n; i0 += 4 * BQ_THREADS) {
+      for (int i0 = 0; i0 < n; i0 += 4 * NT) {
         bw_u4 t[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int i = i0 + u * BQ_THREADS + tid;
+          const int i = i0 + u * NT + tid;
           const int ic = i < n ? i : n - 1;
           const int row = ic / npc, pc = ic - row * npc;
           int tq = t0 + row / G;
@@ -734,7 +766,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int i = i0 + u * BQ_THREADS + tid;
+          const int i = i0 + u * NT + tid;
           if (i < n) {
             const int row = i / npc, pc = i - row * npc;
             *(bw_u4*)(dst + row * rowb + pc * 16) = t[u];
@@ -751,7 +783,7 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
     if (creg[e] >= 0) atomicAdd(&cur[creg[e]], 1);
   rb = block_max(rb, red);  // barrier: histogram complete
   float vm = 0.f, km = 0.f;
-  const int per_thr = (dm.nchunk + BQ_THREADS - 1) / BQ_THREADS;
+  const int per_thr = (dm.nchunk + NT - 1) / NT;
   const int c_lo = tid * per_thr;
   int local = 0;
   for (int c = c_lo; c < c_lo + per_thr && c < dm.nchunk; ++c) {
@@ -796,8 +828,8 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   const float c2 = dm.sm_scale * HILS_LOG2E;
   const float out_scale = dm.sm_scale * fx_scale;
   // rows of lse, weights and dw from the block's first query on, with 32-bit element offsets (hils_bw_run)
-  const float* lse_blk = lse + (b * dm.L + t0) * (long)dm.HQ * K;
-  const bf16_t* w_blk = weights + (b * dm.L + t0) * (long)dm.HQ * dm.NW;
+  const char* lse_blk = (const char*)(lse + (b * dm.L + t0) * (long)dm.HQ * K);
+  const char* w_blk = (const char*)(weights + (b * dm.L + t0) * (long)dm.HQ * dm.NW);
   float* dw_blk = dw + (b * dm.L + t0) * (long)dm.HQ * dm.NW;
   const bf16_t* q_blk = q + (b * dm.L + t0) * (long)dm.HQ * D;
   const bf16_t* do_blk = d_o + (b * dm.L + t0) * (long)dm.HQ * DV;
@@ -807,6 +839,11 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
   const unsigned l_row = (unsigned)(hq * K), w_row0 = (unsigned)(hq * dm.NW);  // ... of query 0 and this lane's head
   const unsigned l_step = (unsigned)(dm.HQ * K), w_step = (unsigned)(dm.HQ * dm.NW);
   const int npair_valid = cur[dm.nchunk - 1];
+  // LDS addresses of this lane's column r in the four output rows of its lane group, for query 0 of the block (rows of
+  // one query are consecutive heads: one address, up to SPARE rows from it), and in the spare rows
+  unsigned acc_lane = (unsigned)(size_t)(bq_lds_int*)(q_acc + ((4 * j) % G) * D + r);
+  unsigned spare_lane = (unsigned)(size_t)(bq_lds_int*)(q_acc + R * D + r);
+  asm volatile("" : "+v"(acc_lane), "+v"(spare_lane));  // (kept as registers: or the constant parts are added per use)
 
   for (;;) {
     int c = 0;
@@ -834,61 +871,54 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
 #pragma unroll
       for (int u = 0; u < 2 * DT; ++u) xt[u] = *(const bw_u4*)(kt_c + u * 512);
     }
-    // rows of a tile starting at pair p: this lane's row (pair, gathered q and dO pieces, lse, weight)
-    bw_u4 bq[KS], bdo[VS], bq_n[KEEP ? KS : 1], bdo_n[KEEP ? VS : 1];
-    float l2 = 0.f, l2_n = 0.f;
-    bf16_t wb = 0, wb_n = 0;
-    int pk = 0, pk_n = 0;
-    auto load_rows = [&](int p, bw_u4* q_r, bw_u4* o_r, float& l_r, bf16_t& w_r, int& pk_r)
-                         __attribute__((always_inline)) {
+    auto load_rows = [&](int p, BqRows<KS, VS>& x) __attribute__((always_inline)) {
       const int last = ((ve - p < QT) ? ve - p : QT) - 1;  // padding rows repeat the tile's last pair
-      pk_r = pairs[p + (qs < last ? qs : last)];
-      const unsigned ql_r = (unsigned)pk_r >> 8, slot_r = (unsigned)pk_r & 255u;
-      if (STAGE) {
-        const int row_l = (pk_r >> 8) * G + g;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) q_r[ks] = *(const bw_u4*)(rows_q + row_l * QROWB + (ks * 32 + j * 8) * 2);
-#pragma unroll
-        for (int ks = 0; ks < VS; ++ks) o_r[ks] = *(const bw_u4*)(rows_o + row_l * OROWB + (ks * 32 + j * 8) * 2);
-      } else {
+      x.pk = pairs[p + (qs < last ? qs : last)];
+      const unsigned ql_r = x.pk >> 8, slot_r = x.pk & 255u;
+      if (!STAGE) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-          q_r[ks] = *(const bw_u4*)(q_blk + (__umul24(ql_r, (unsigned)(dm.HQ * D)) + (unsigned)(hq * D + ks * 32 + j * 8)));
+          x.q[ks] = *(const bw_u4*)(q_blk + (__umul24(ql_r, (unsigned)(dm.HQ * D)) + (unsigned)(hq * D + ks * 32 + j * 8)));
 #pragma unroll
         for (int ks = 0; ks < VS; ++ks)
-          o_r[ks] = *(const bw_u4*)(do_blk + (__umul24(ql_r, (unsigned)(dm.HQ * DV)) + (unsigned)(hq * DV + ks * 32 + j * 8)));
+          x.o[ks] = *(const bw_u4*)(do_blk + (__umul24(ql_r, (unsigned)(dm.HQ * DV)) + (unsigned)(hq * DV + ks * 32 + j * 8)));
       }
-      l_r = lse_blk[__umul24(ql_r, l_step) + l_row + slot_r];
-      w_r = w_blk[__umul24(ql_r, w_step) + w_row0 + slot_r];
+      // (byte offsets below 2^32: a uniform base and one register)
+      x.l2 = *(const float*)(lse_blk + (__umul24(ql_r, l_step) + l_row + slot_r) * 4u);
+      x.wb = *(const bf16_t*)(w_blk + (__umul24(ql_r, w_step) + w_row0 + slot_r) * 2u);
     };
-    if (KEEP) load_rows(vs, bq, bdo, l2, wb, pk);
-    for (int p = vs; p < ve; p += QT) {
-      const int last = ((ve - p < QT) ? ve - p : QT) - 1;
+    // one tile, its rows in x; the next tile's rows, if there is one, are loaded into nx behind its arithmetic
+    auto tile = [&](int p, BqRows<KS, VS>& x, BqRows<KS, VS>& nx) __attribute__((always_inline)) {
+      const int n = (ve - p < QT) ? ve - p : QT;  // pairs of the tile
       if (!KEEP) {
-        load_rows(p, bq, bdo, l2, wb, pk);
+        load_rows(p, x);
 #pragma unroll
         for (int u = 0; u < 4 * KS; ++u) xa[u] = *(const bw_u4*)(ka_c + u * 512);
 #pragma unroll
         for (int u = 0; u < 4 * VS; ++u) ya[u] = *(const bw_u4*)(va_c + u * 512);
       }
-      const bool more = KEEP && p + QT < ve;
-      if (more) load_rows(p + QT, bq_n, bdo_n, l2_n, wb_n, pk_n);  // in flight behind this tile's arithmetic
-      int pk_o[4];
+      if (KEEP && p + QT < ve) load_rows(p + QT, nx);
+      if (STAGE) {
+        const unsigned row_l = (x.pk >> 8) * G + g;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int qsl = (4 * j + i) / G;
-        pk_o[i] = pairs[p + (qsl < last ? qsl : last)];
+        for (int ks = 0; ks < KS; ++ks) x.q[ks] = *(const bw_u4*)(rows_q + row_l * QROWB + (ks * 32 + j * 8) * 2);
       }
-      if (l2 == HILS_NEG_INF) l2 = INFINITY;
-      const float w_row = bf2f(wb);
-      int orow[4];
+      // LDS addresses of the output rows 4j .. 4j + 3, this lane's column
+      constexpr int NP = G >= 4 ? 1 : 4 / G;  // pairs they belong to
+      const unsigned short* op = pairs + p + (4 * j) / G;
+      unsigned at[NP];
+      if (n == QT) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = 4 * j + i;
-        const int qsl = rr / G;
-        const int row = (qsl <= last) ? (pk_o[i] >> 8) * G + (rr - qsl * G) : R;
-        orow[i] = row * D + r;
+        for (int u = 0; u < NP; ++u) at[u] = __umul24((unsigned)op[u] >> 8, (unsigned)(G * D * 4)) + acc_lane;
+      } else {  // padding rows add to the spare rows
+        const int last = n - 1 - (4 * j) / G;
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+          const unsigned real = __umul24((unsigned)op[u <= last ? u : last] >> 8, (unsigned)(G * D * 4)) + acc_lane;
+          at[u] = u <= last ? real : spare_lane;
+        }
       }
+      const float l2 = x.l2 == HILS_NEG_INF ? INFINITY : x.l2;
       // ---- S^T and dP^T: tokens x rows, four token tiles each
       f32x4_t st[4], dpt[4];
 #pragma unroll
@@ -901,25 +931,33 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
           st[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[mt * KS + ks]),
-                                                           __builtin_bit_cast(bf16x8_t, bq[ks]), st[mt], 0, 0, 0);
+                                                           __builtin_bit_cast(bf16x8_t, x.q[ks]), st[mt], 0, 0, 0);
+      if (STAGE) {
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned row_l = (x.pk >> 8) * G + g;
+#pragma unroll
+        for (int ks = 0; ks < VS; ++ks) x.o[ks] = *(const bw_u4*)(rows_o + row_l * OROWB + (ks * 32 + j * 8) * 2);
+      }
 #pragma unroll
       for (int ks = 0; ks < VS; ++ks)
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
           dpt[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ya[mt * VS + ks]),
-                                                            __builtin_bit_cast(bf16x8_t, bdo[ks]), dpt[mt], 0, 0, 0);
+                                                            __builtin_bit_cast(bf16x8_t, x.o[ks]), dpt[mt], 0, 0, 0);
       if (!KEEP) {  // K of the chunk as B operand of dQ = dS K replaces the first operand set
 #pragma unroll
         for (int u = 0; u < 2 * DT; ++u) xa[u] = *(const bw_u4*)(kt_c + u * 512);
       }
       if (dm.slope) {
-        asm volatile("" ::: "memory");  // (a branch, not sixteen subtractions of zero in every tile)
+        float sl_v = sl;
+        int j_v = j;
+        asm volatile("" : "+v"(sl_v), "+v"(j_v) : : "memory");  // (a branch that keeps no registers between tiles)
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int dist = BW_S - 2 - (mt * 16 + j * 4 + i);
-            st[mt][i] -= sl * (float)(dist > 0 ? dist : 0);
+            const int dist = BW_S - 2 - (mt * 16 + j_v * 4 + i);
+            st[mt][i] -= sl_v * (float)(dist > 0 ? dist : 0);
           }
       }
       // ---- P, delta, dS (this lane: row r of the tile, tokens mt*16 + 4j + i)
@@ -937,19 +975,19 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
         st[3][3] = 0.f;
       }
       delta = rows_sum(delta);
-      if (j == 0 && qs <= last) dw_blk[__umul24((unsigned)pk >> 8, w_step) + w_row0 + ((unsigned)pk & 255u)] = delta;
-      const float f = w_row * out_scale;
+      if (j == 0 && qs < n) dw_blk[__umul24(x.pk >> 8, w_step) + w_row0 + (x.pk & 255u)] = delta;
+      const float f = __uint_as_float((unsigned)x.wb << 16) * out_scale;
       bf16x8_t ap[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
         // (the difference first: a product rounded before the cancellation leaves its error behind)
         auto ds = [&](int mt, int i) __attribute__((always_inline)) { return f * st[mt][i] * (dpt[mt][i] - delta); };
-        uint4 x;
-        x.x = pack_bf2(ds(2 * s2, 0), ds(2 * s2, 1));
-        x.y = pack_bf2(ds(2 * s2, 2), ds(2 * s2, 3));
-        x.z = pack_bf2(ds(2 * s2 + 1, 0), ds(2 * s2 + 1, 1));
-        x.w = pack_bf2(ds(2 * s2 + 1, 2), ds(2 * s2 + 1, 3));
-        ap[s2] = __builtin_bit_cast(bf16x8_t, x);
+        uint4 y;
+        y.x = pack_bf2(ds(2 * s2, 0), ds(2 * s2, 1));
+        y.y = pack_bf2(ds(2 * s2, 2), ds(2 * s2, 3));
+        y.z = pack_bf2(ds(2 * s2 + 1, 0), ds(2 * s2 + 1, 1));
+        y.w = pack_bf2(ds(2 * s2 + 1, 2), ds(2 * s2 + 1, 3));
+        ap[s2] = __builtin_bit_cast(bf16x8_t, y);
       }
       // ---- dQ tile += dS K: four column tiles at a time
 #pragma unroll
@@ -964,25 +1002,29 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
             const bw_u4 kb2 = KEEP ? xt[KEEP ? (d0 + u) * 2 + s2 : 0] : xa[(d0 + u) * 2 + s2];
             acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[s2], __builtin_bit_cast(bf16x8_t, kb2), acc[u], 0, 0, 0);
           }
+        bq_settle(acc);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) atomicAdd(&q_acc[orow[i] + (d0 + u) * 16], __float2int_rn(acc[u][i]));
+          for (int i = 0; i < 4; ++i)
+            __hip_atomic_fetch_add((bq_lds_int*)(at[i * NP / 4] + (unsigned)((i % (4 / NP)) * D + (d0 + u) * 16) * 4u),
+                                   bq_round(acc[u][i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      if (more) {  // the next tile's rows become the current ones
-#pragma unroll
-        for (int ks = 0; ks < (KEEP ? KS : 1); ++ks) bq[ks] = bq_n[ks];
-#pragma unroll
-        for (int ks = 0; ks < (KEEP ? VS : 1); ++ks) bdo[ks] = bdo_n[ks];
-        l2 = l2_n;
-        wb = wb_n;
-        pk = pk_n;
-      }
+    };
+    BqRows<KS, VS> xa_r, xb_r;
+    if (KEEP) load_rows(vs, xa_r);
+    for (int p = vs;;) {  // two row sets in turn: nothing is copied from one to the other
+      tile(p, xa_r, xb_r);
+      p += QT;
+      if (p >= ve) break;
+      tile(p, xb_r, xa_r);
+      p += QT;
+      if (p >= ve) break;
     }
   }
   __syncthreads();
   constexpr int C8 = D / 8;
-  for (int i = tid; i < R * C8; i += BQ_THREADS) {
+  for (int i = tid; i < R * C8; i += NT) {
     const int row = i / C8, c8 = i - row * C8;
     const int ql = row / G, g2 = row - ql * G;
     const int t = t0 + ql;
@@ -1021,7 +1063,7 @@ void hils_ga_pack_launch(const void* a, const void* b, void* ap, void* bp, float
 // and the pair list (and, with `stage`, the block's own query and dO rows) fit in LDS; 0 when the
 // shape does not fit.
 static size_t bq_smem_bytes(int T, int G, int D, int Dv, int K, int nchunk, bool stage) {
-  size_t n = (size_t)(T * G + 1) * D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + (((size_t)T * K * 2 + 15) & ~(size_t)15);
+  size_t n = (size_t)(T * G + bq_spare(G)) * D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + (((size_t)T * K * 2 + 15) & ~(size_t)15);
   if (stage) n += (size_t)T * G * ((size_t)D * 2 + 16 + (size_t)Dv * 2 + 16);
   return n;
 }
@@ -1029,7 +1071,7 @@ static int bq_pick_T(int L, int G, int D, int Dv, int K, int nchunk, bool stage,
   // the largest block that fits: the more rows share a visit, the fewer K/V bytes per row
   const size_t limit = 156 * 1024;
   const size_t per_q = (size_t)G * D * 4 + (size_t)K * 2 + (stage ? (size_t)G * ((size_t)(D + Dv) * 2 + 32) : 0);
-  const size_t fixed = (size_t)D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + 16;  // spare row, histogram, alignment
+  const size_t fixed = (size_t)bq_spare(G) * D * 4 + (size_t)((nchunk + 3) & ~3) * 4 + 16;  // spare rows, histogram, alignment
   if (fixed + per_q > limit) return 0;
   long T = (long)((limit - fixed) / per_q);
   if (T > 256) T = 256;  // a pair is (query << 8 | slot) in 16 bits
@@ -1114,15 +1156,15 @@ static int bw_launch_dkdv(int G, dim3 grid, hipStream_t st, const bf16_t* q, con
   return HILS_OK;
 }
 
-template <int D, int DV, int G, bool STAGE>
+template <int D, int DV, int G, bool STAGE, int NT>
 static int bq_launch(dim3 grid, size_t smem, hipStream_t st, const bf16_t* q, const bf16_t* d_o,
                      const bf16_t* ka, const bf16_t* va, const bf16_t* kt, const float* vmax,
                      const float* kmax, const bf16_t* w, const int32_t* idx, const float* lse, bf16_t* dq,
                      float* dw, const BqDims& dm) {
-  auto kern = bw_dq_kernel<D, DV, G, STAGE>;
+  auto kern = bw_dq_kernel<D, DV, G, STAGE, NT>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_sparse_attn_bwd")) return rc;
-  hipLaunchKernelGGL(kern, grid, dim3(BQ_THREADS), smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+  hipLaunchKernelGGL(kern, grid, dim3(NT), smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
   return HILS_OK;
 }
 
@@ -1131,26 +1173,38 @@ static int bq_dispatch_g(int G, bool stage, dim3 grid, size_t smem, hipStream_t 
                          const bf16_t* d_o, const bf16_t* ka, const bf16_t* va, const bf16_t* kt,
                          const float* vmax, const float* kmax, const bf16_t* w, const int32_t* idx,
                          const float* lse, bf16_t* dq, float* dw, const BqDims& dm) {
-  if (stage)  // only built without head grouping (see bq_stage_pays)
-    return bq_launch<D, DV, 1, true>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+  if constexpr (D <= 64 && DV <= 64) {
+    if (stage) switch (G) {
+      case 1: return bq_launch<D, DV, 1, true, BQ_STAGE_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+      case 2: return bq_launch<D, DV, 2, true, BQ_STAGE_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+      case 4: return bq_launch<D, DV, 4, true, BQ_STAGE_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+      case 8: return bq_launch<D, DV, 8, true, BQ_STAGE_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+      case 16: return bq_launch<D, DV, 16, true, BQ_STAGE_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+      default: return -1;
+    }
+  }
   switch (G) {
-    case 1: return bq_launch<D, DV, 1, false>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
-    case 2: return bq_launch<D, DV, 2, false>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
-    case 4: return bq_launch<D, DV, 4, false>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
-    case 8: return bq_launch<D, DV, 8, false>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
-    case 16: return bq_launch<D, DV, 16, false>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+    case 1: return bq_launch<D, DV, 1, false, BQ_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+    case 2: return bq_launch<D, DV, 2, false, BQ_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+    case 4: return bq_launch<D, DV, 4, false, BQ_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+    case 8: return bq_launch<D, DV, 8, false, BQ_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
+    case 16: return bq_launch<D, DV, 16, false, BQ_THREADS>(grid, smem, st, q, d_o, ka, va, kt, vmax, kmax, w, idx, lse, dq, dw, dm);
   }
   return -1;
 }
 
-// Staging the block's rows in LDS pays when it costs little block size: the block shrinks by the
-// rows' bytes, and a smaller block pulls more K/V bytes per row.
-static bool bq_stage_pays(int L, int G, int D, int Dv, int K, int nchunk) {
-  if (G != 1) return false;
+// Staging the block's rows in LDS halves the block or more (its rows take as much as its output tile), but the rows of
+// all blocks of an XCD together would not stay in its L2 beside the operands, and every (row, slot) pair gathers one:
+// gathered / staged, dQ alone at B2 L8192, 4 KV heads of 64, top-32: 236 / 202 us with 2 query heads per KV head,
+// 514 / 382 with 4, 785 / 650 with 8, 1646 / 1283 with 16.  Calls whose gathering blocks fit one round of the chip keep
+// them (B1 L3001 32/4: 96 / 107 us, B2 L1024 16/2: 24.6 / 26.5).  Wide heads have no registers for a visit's operands
+// and no room for the rows.
+static bool bq_stage_pays(long units, int L, int G, int D, int Dv, int K, int nchunk) {
+  if (D > 64 || Dv > 64) return false;
   size_t a, b2;
   const int t_plain = bq_pick_T(L, G, D, Dv, K, nchunk, false, &a);
   const int t_stage = bq_pick_T(L, G, D, Dv, K, nchunk, true, &b2);
-  return t_stage > 0 && 4 * t_stage >= 3 * t_plain;
+  return t_plain > 0 && t_stage > 0 && units * ((L + t_plain - 1) / t_plain) > hils_device_cus();
 }
 
 // Inverse index of an index tensor (B, L, H, K) with values in [0, nchunk) or < 0: counts,
@@ -1211,7 +1265,7 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   // ---- dQ, dW
   {
     size_t smem;
-    const bool stage = bq_stage_pays(L, G, D, Dv, K, nchunk);
+    const bool stage = bq_stage_pays((long)B * H, L, G, D, Dv, K, nchunk);
     int T = bq_pick_T(L, G, D, Dv, K, nchunk, stage, &smem);
     if (T == 0) return -1;
     // small problems: rather a block for every compute unit than the largest blocks (64 blocks of 64 queries ->

@@ -73,6 +73,15 @@ def test_sparse_attn_backward(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mask_last)
         assert not got[1][:, 63].any() and not got[2][:, 63].any()
 
 
+# blocks for more than one round of the compute units: narrow heads keep their own rows in LDS (short ones gather them),
+# the last block of a sequence and most tiles of a visit are partly filled
+@pytest.mark.parametrize("B,L,HQ,H,K,mask_last", [
+    (6, 527, 16, 16, 5, True), (6, 650, 32, 16, 7, False), (4, 650, 64, 16, 6, True), (2, 650, 128, 16, 9, True),
+    (1, 579, 256, 16, 3, False)])
+def test_sparse_attn_backward_many_blocks(pkg, dev, B, L, HQ, H, K, mask_last):
+    test_sparse_attn_backward(pkg, dev, B, L, HQ, H, 64, 64, K, False, mask_last)
+
+
 @pytest.mark.parametrize("B,L,HQ,H,D,W", [(1, 700, 8, 1, 64, 512), (2, 1024, 16, 2, 64, 512), (1, 513, 4, 1, 128, 300),
                                           (1, 2000, 4, 4, 64, 512)])
 def test_swa_backward_split(pkg, dev, B, L, HQ, H, D, W):
