@@ -64,11 +64,11 @@ __device__ __forceinline__ void bw_walk_indices(const int32_t* __restrict__ seg0
   }
 }
 
-// counts[(b*H + h) * nchunk + c] = number of valid entries equal to c; one workgroup per
-// (batch, KV head, segment of queries), LDS histogram first.
+// counts[((b*H + h) * ranges + t / range) * nchunk + c] = number of valid entries equal to c; one workgroup per
+// (batch, KV head, segment of queries of one range), LDS histogram first.
 __global__ void __launch_bounds__(1024)
 bw_count_kernel(const int32_t* __restrict__ indices, int* __restrict__ counts, int L, int H, int K,
-                int nchunk, int seg_len) {
+                int nchunk, int seg_len, int range, int n_range) {
   extern __shared__ int hist[];
   const int h = blockIdx.y;
   const long b = blockIdx.z;
@@ -81,18 +81,22 @@ bw_count_kernel(const int32_t* __restrict__ indices, int* __restrict__ counts, i
     if (c >= 0 && c < nchunk) atomicAdd(&hist[c], 1);
   });
   __syncthreads();
-  int* out = counts + (b * H + h) * (long)nchunk;
+  int* out = counts + ((b * H + h) * n_range + t_lo / range) * (long)nchunk;
   for (int i = threadIdx.x; i < nchunk; i += 1024)
     if (hist[i]) atomicAdd(&out[i], hist[i]);
 }
 
-// Work items of the dK/dV kernel (null: none wanted): every cell (batch, KV head, chunk) is cut into
-// segments of at most seg_pairs pairs, an empty one is one item (its gradients are zeroed).
+// Work items of the dK/dV kernel (null: none wanted): every cell (batch, KV head, range of queries, chunk) is cut
+// into segments of at most seg_pairs pairs.  With one range a cell is a chunk: one that is not cut is written by its
+// item, which also zeroes the gradients of an empty one.  With several, every item leaves a partial result and an
+// empty cell has none.
 struct BwItems {
   int2* list;     // (cell, segment)
   int* total;     // number of items
-  int* part_off;  // [cell] first partial result of a cell of several segments
+  int* part_off;  // [cell] first partial result of a cell
   int seg_pairs;
+  int n_range;
+  __device__ __forceinline__ int segs(int x) const { return x > seg_pairs ? (x + seg_pairs - 1) / seg_pairs : n_range == 1 || x ? 1 : 0; }
 };
 
 // exclusive scan of n counts into offsets[0..n] (offsets[n] = total) and the item list; one workgroup, four
@@ -102,7 +106,7 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
   __shared__ int wsum[3][16];
   __shared__ int carry_s[3];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  auto segs = [&](int x) -> int { return x > it.seg_pairs ? (x + it.seg_pairs - 1) / it.seg_pairs : 1; };
+  auto parts = [&](int ns) -> int { return ns > 1 || it.n_range > 1 ? ns : 0; };
   if (tid < 3) carry_s[tid] = 0;
   __syncthreads();
   for (int base = 0; base < n; base += 4096) {
@@ -120,9 +124,9 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
     for (int e = 0; e < 4; ++e) {
       s[0] += x[e];
       if (it.list && i0 + e < n) {
-        const int ns = segs(x[e]);
+        const int ns = it.segs(x[e]);
         s[1] += ns;
-        s[2] += ns > 1 ? ns : 0;
+        s[2] += parts(ns);
       }
     }
     int pos[3];
@@ -158,10 +162,10 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
         pos[0] += x[e];
         pp[e] = pos[2];
         if (it.list && i0 + e < n) {
-          const int ns = segs(x[e]);
+          const int ns = it.segs(x[e]);
           for (int k = 0; k < ns; ++k) it.list[pos[1] + k] = make_int2(i0 + e, k);
           pos[1] += ns;
-          pos[2] += ns > 1 ? ns : 0;
+          pos[2] += parts(ns);
         }
       }
       *(int4*)&offsets[i0] = o4;  // (offsets[n], when it lies in the group, is written below)
@@ -180,13 +184,13 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
 // range per chunk with a single global atomic, and scatters (t << 8 | slot) inside its ranges
 __global__ void __launch_bounds__(1024)
 bw_scatter_kernel(const int32_t* __restrict__ indices, int* __restrict__ cursor,
-                  uint32_t* __restrict__ pairs, int L, int H, int K, int nchunk, int seg_len) {
+                  uint32_t* __restrict__ pairs, int L, int H, int K, int nchunk, int seg_len, int range, int n_range) {
   extern __shared__ int pos[];  // nchunk: count -> next free position
   const int h = blockIdx.y;
   const long b = blockIdx.z;
   const int t_lo = blockIdx.x * seg_len;
   const int t_hi = (t_lo + seg_len < L) ? t_lo + seg_len : L;
-  int* cur = cursor + (b * H + h) * (long)nchunk;
+  int* cur = cursor + ((b * H + h) * n_range + t_lo / range) * (long)nchunk;
   for (int i = threadIdx.x; i < nchunk; i += 1024) pos[i] = 0;
   __syncthreads();
   const int32_t* seg0 = indices + ((b * L + t_lo) * H + h) * (long)K;
@@ -210,6 +214,10 @@ bw_scatter_kernel(const int32_t* __restrict__ indices, int* __restrict__ cursor,
 // one, and with one workgroup per chunk and all of them resident at once the kernel ran as long as its
 // fullest chunk (B2 L8192 32/4 heads of 64, top-32: 1300 us; in segments 1035).  The segments of
 // a cut chunk leave fp32 partial results that bw_dkdv_sum_kernel adds up.
+// Rows of many heads (16 MiB for these four KV heads' queries) are fetched again by every chunk: 5.3 GB past the L2.
+// The items then go by ranges of queries (bw_range): 926 -> 735 us.  With the gathers as global instead of flat loads,
+// whose data every wait for the LDS had waited for, and a round's reads ahead of its products: 712 us; B8 L8192 16/16
+// heads of 64: 1435 -> 1400, vector ALU 42 % and matrix cores 29 % busy, LDS 42 %.
 // ---------------------------------------------------------------------------
 struct BwDims {
   int L, Lkv, HQ, H, K, NW, nchunk, mask_last;
@@ -247,7 +255,7 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   constexpr int OROW = DV * 2 + 16;
   constexpr int BUF = ROWS * (QROW + OROW) + 3 * ROWS * 4;  // one staging buffer (bytes)
   extern __shared__ __attribute__((aligned(16))) char bw_smem[];  // two staging buffers
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, j = lane >> 4;
   // XCD-aware order: hardware hands consecutive workgroup ids to the 8 XCDs in turn; an XCD works
   // through one contiguous share of the items, i.e. of the (batch, KV head) pairs, so the query and dO
@@ -256,11 +264,11 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   const int vid = (int)(blockIdx.x % 8) * ((n_items + 7) / 8) + (int)(blockIdx.x / 8);
   if ((int)(blockIdx.x / 8) >= (n_items + 7) / 8 || vid >= n_items) return;
   const int2 item = dm.items.list[vid];
-  const int cell = item.x, c = cell % dm.nchunk, unit = cell / dm.nchunk;
+  const int cell = item.x, c = cell % dm.nchunk, unit = cell / dm.nchunk / dm.items.n_range;
   const int hk = unit % dm.H;
   const long b = unit / dm.H;
-  const int c_lo = offsets[cell], c_hi = offsets[cell + 1];  // the chunk's pairs
-  const bool whole = c_hi - c_lo <= dm.items.seg_pairs;
+  const int c_lo = offsets[cell], c_hi = offsets[cell + 1];  // the cell's pairs
+  const bool whole = dm.items.n_range == 1 && c_hi - c_lo <= dm.items.seg_pairs;
   const int p_lo = c_lo + item.y * dm.items.seg_pairs;
   const int p_hi = c_hi - p_lo <= dm.items.seg_pairs ? c_hi : p_lo + dm.items.seg_pairs;
   if (p_lo == p_hi) {
@@ -327,7 +335,7 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
 #pragma unroll
     for (int u = 0; u < NQ; ++u) pk_q[u] = pair_of(round, q_row0 + u * QRS);
 #pragma unroll
-    for (int u = 0; u < NO; ++u) pk_o[u] = pair_of(round, o_row0 + u * ORS);
+    for (int u = 0; u < NO; ++u) pk_o[u] = D == DV ? pk_q[u < NQ ? u : 0] : pair_of(round, o_row0 + u * ORS);  // (the same rows)
     pk_r = pair_of(round, tid);
   };
   // Row addresses are this lane's base plus query * stride, one 32 x 32 + 64 multiply-add each (the row
@@ -335,12 +343,14 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   static_assert(QRS % 16 == 0 && ORS % 16 == 0, "a thread stages rows of one head");
   const char* q_lane = (const char*)(q + (b * dm.L * (long)dm.HQ + hk * G + q_row0 % G) * D + q_pc * 8);
   const char* o_lane = (const char*)(d_o + (b * dm.L * (long)dm.HQ + hk * G + o_row0 % G) * DV + o_pc * 8);
-  const long row_lane = b * dm.L * (long)dm.HQ + hk * G + tid % G;
+  const long row_lane = b * dm.L * (long)dm.HQ + hk * G + (tid < ROWS ? tid % G : 0);  // (one address for the threads without a row)
   const float* l_lane = lse + row_lane * dm.K;
   const bf16_t* w_lane = weights + row_lane * dm.NW;
   const float* d_lane = delta + row_lane * dm.NW;
   const unsigned q_step = (unsigned)dm.HQ * D * 2u, o_step = (unsigned)dm.HQ * DV * 2u;
   const unsigned l_step = (unsigned)(dm.HQ * dm.K), w_step = (unsigned)(dm.HQ * dm.NW);
+  // (as global pointers: an integer made a generic pointer is read by flat loads, which every wait for the LDS waits for)
+  typedef const __attribute__((address_space(1))) bw_u4* bw_gptr;
   auto mad64 = [](unsigned a, unsigned b2, unsigned long c3) __attribute__((always_inline)) -> unsigned long {
     return (unsigned long)a * b2 + c3;
   };
@@ -348,11 +358,11 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
       // padding rows read the row of the chunk's first pair (finite values): their P is 0, so they add nothing
-      xq[u] = *(const bw_u4*)mad64(pk_q[u] >> 8, q_step, (unsigned long)q_lane);
+      xq[u] = *(bw_gptr)mad64(pk_q[u] >> 8, q_step, (unsigned long)q_lane);
     }
 #pragma unroll
     for (int u = 0; u < NO; ++u) {
-      xo[u] = *(const bw_u4*)mad64(pk_o[u] >> 8, o_step, (unsigned long)o_lane);
+      xo[u] = *(bw_gptr)mad64(pk_o[u] >> 8, o_step, (unsigned long)o_lane);
     }
     {
       // raw values; what a padding row gets instead is decided where they are staged, so that
@@ -382,14 +392,15 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
       row_delta[tid] = r_ok ? -r_dl : 0.f;  // negated: the accumulators of dP start from it
     }
   };
-  // one column-read of a staged tile: rows r0 + 4j .. r0 + 4j + 3 of columns c0 .. c0 + 15, this
-  // lane's column.  (Transposing load: lane l of a 16-lane group addresses row l/4, columns
-  // 4*(l%4) .. +3 of the 4 x 16 block and receives column l of it.)
+  // column reads of a staged tile: rows r0 + 4j .. r0 + 4j + 3 of columns c0 .. c0 + 15, this
+  // lane's column, and the same of the 16 rows behind.  (Transposing load: lane l of a 16-lane group addresses row l/4,
+  // columns 4*(l%4) .. +3 of the 4 x 16 block and receives column l of it.)
   typedef short bw_tr4 __attribute__((ext_vector_type(4)));
-  auto col_read = [&](const char* base, int rowb, int r0, int c0) __attribute__((always_inline)) -> uint2 {
+  auto col_pair = [&](const char* base, int rowb, int r0, int c0) __attribute__((always_inline)) -> bw_u4 {
     const char* p = base + (r0 + 4 * j + (col >> 2)) * rowb + (c0 + 4 * (col & 3)) * 2;
-    const bw_tr4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bw_tr4*)p);
-    return __builtin_bit_cast(uint2, v);
+    const uint2 a = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bw_tr4*)p));
+    const uint2 b2 = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bw_tr4*)(p + 16 * rowb)));
+    return (bw_u4){a.x, a.y, b2.x, b2.y};
   };
   load_pairs(0);
   fetch(0);
@@ -410,88 +421,104 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
     const int rows_here = ((npair - round * PPR < PPR) ? npair - round * PPR : PPR) * G;
     // This wavefront's two 16-row tiles: their P and dS, side by side, are the A operands (m = token,
     // k = 32 rows) of one 16x16x32 product per column tile and token tile; k index 8j + e stands for row
-    // 4j + e of the first tile (e < 4) or row 4j + e - 4 of the second
+    // 4j + e of the first tile (e < 4) or row 4j + e - 4 of the second.
+    // A SIMD holds two wavefronts and a round is a chain (rows, scores, exponentials, column reads, products): the
+    // reads of a link are issued ahead of the link before it, fenced so that the scheduler does not sink them.
     const int r0 = rw * 32;
     if (r0 < rows_here) {
-      uint2 xp[TT][2], xds[TT][2];  // [token tile][row tile]
+      bw_u4 qa[2][KS], oa[2][VS];
+      f32x4_t l4[2], w4[2], d4[2];
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2) {
-        // ---- S and dP of 16 rows x this wavefront's tokens
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qa[h2][ks] = *(const bw_u4*)(q_rm + (r0 + h2 * 16 + col) * QROW + (ks * 32 + j * 8) * 2);
+      }
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
         const int r = r0 + h2 * 16 + 4 * j;
-        const f32x4_t l4 = *(const f32x4_t*)&row_lse[r], w4 = *(const f32x4_t*)&row_w[r], d4 = *(const f32x4_t*)&row_delta[r];
-        f32x4_t s[TT], dp[TT];
+        d4[h2] = *(const f32x4_t*)&row_delta[r];
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-          s[tt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-          dp[tt] = d4;  // dP - delta
-        }
+        for (int ks = 0; ks < VS; ++ks) oa[h2][ks] = *(const bw_u4*)(o_rm + (r0 + h2 * 16 + col) * OROW + (ks * 32 + j * 8) * 2);
+        l4[h2] = *(const f32x4_t*)&row_lse[r];
+        w4[h2] = *(const f32x4_t*)&row_w[r];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- S and dP of 32 rows x this wavefront's tokens
+      f32x4_t s[2][TT], dp[2][TT];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const uint4 a = *(const uint4*)(q_rm + (r0 + h2 * 16 + col) * QROW + (ks * 32 + j * 8) * 2);
+      for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) s[h2][tt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
           for (int tt = 0; tt < TT; ++tt)
-            s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&kb[tt][ks], s[tt], 0, 0, 0);
-        }
+            s[h2][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, qa[h2][ks]), *(const bf16x8_t*)&kb[tt][ks], s[h2][tt], 0, 0, 0);
 #pragma unroll
-        for (int ks = 0; ks < VS; ++ks) {
-          const uint4 a = *(const uint4*)(o_rm + (r0 + h2 * 16 + col) * OROW + (ks * 32 + j * 8) * 2);
+      for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) dp[h2][tt] = d4[h2];  // dP - delta
+#pragma unroll
+      for (int ks = 0; ks < VS; ++ks)
+#pragma unroll
+        for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
           for (int tt = 0; tt < TT; ++tt)
-            dp[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&vb[tt][ks], dp[tt], 0, 0, 0);
-        }
-        if (dm.slope) {  // distance penalty (16 % G == 0: row 4j + i is the same head in every 16-row tile)
+            dp[h2][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, oa[h2][ks]), *(const bf16x8_t*)&vb[tt][ks], dp[h2][tt], 0, 0, 0);
+      if (dm.slope) {  // distance penalty (16 % G == 0: row 4j + i is the same head in every 16-row tile)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float sl = dm.slope[hk * G + (4 * j + i) % G];
+        for (int i = 0; i < 4; ++i) {
+          const float sl = dm.slope[hk * G + (4 * j + i) % G];
 #pragma unroll
-            for (int tt = 0; tt < TT; ++tt) {
-              const int dist = BW_S - 2 - (tw * (16 * TT) + tt * 16 + col);
-              s[tt][i] -= sl * (float)(dist > 0 ? dist : 0);
-            }
+          for (int tt = 0; tt < TT; ++tt) {
+            const int dist = BW_S - 2 - (tw * (16 * TT) + tt * 16 + col);
+            s[0][tt][i] -= sl * (float)(dist > 0 ? dist : 0);
+            s[1][tt][i] -= sl * (float)(dist > 0 ? dist : 0);
           }
-        }
-        // accumulator layout: column = token `col`, registers = rows 4j..4j+3
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-          float pv[4], ds[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pv[i] = __builtin_amdgcn_exp2f(fmaf(s[tt][i], c2, -l4[i]));
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            pv[i] *= w4[i];
-            ds[i] = pv[i] * dp[tt][i];
-          }
-          xp[tt][h2].x = pack_bf2(pv[0], pv[1]);
-          xp[tt][h2].y = pack_bf2(pv[2], pv[3]);
-          xds[tt][h2].x = pack_bf2(ds[0], ds[1]);
-          xds[tt][h2].y = pack_bf2(ds[2], ds[3]);
         }
       }
+      bw_u4 bo[VT], bq[DT];
+#pragma unroll
+      for (int t = 0; t < VT; ++t) bo[t] = col_pair(o_rm, OROW, r0, t * 16);
+      __builtin_amdgcn_sched_barrier(0);
       uint4 a_p[TT], a_ds[TT];
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
-        a_p[tt] = make_uint4(xp[tt][0].x, xp[tt][0].y, xp[tt][1].x, xp[tt][1].y);
-        a_ds[tt] = make_uint4(xds[tt][0].x, xds[tt][0].y, xds[tt][1].x, xds[tt][1].y);
-      }
-      // ---- dK += dS^T Q, dV += (wP)^T dO: contraction over the 32 rows
+        // accumulator layout: column = token `col`, registers = rows 4j..4j+3
+        uint2 xp[2], xds[2];
 #pragma unroll
-      for (int t = 0; t < DT; ++t) {
-        const uint2 b0 = col_read(q_rm, QROW, r0, t * 16);
-        const uint2 b1 = col_read(q_rm, QROW, r0 + 16, t * 16);
-        const uint4 bq = make_uint4(b0.x, b0.y, b1.x, b1.y);
+        for (int h2 = 0; h2 < 2; ++h2) {
+          float pv[4], ds[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pv[i] = __builtin_amdgcn_exp2f(fmaf(s[h2][tt][i], c2, -l4[h2][i]));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            pv[i] *= w4[h2][i];
+            ds[i] = pv[i] * dp[h2][tt][i];
+          }
+          xp[h2].x = pack_bf2(pv[0], pv[1]);
+          xp[h2].y = pack_bf2(pv[2], pv[3]);
+          xds[h2].x = pack_bf2(ds[0], ds[1]);
+          xds[h2].y = pack_bf2(ds[2], ds[3]);
+        }
+        a_p[tt] = make_uint4(xp[0].x, xp[0].y, xp[1].x, xp[1].y);
+        a_ds[tt] = make_uint4(xds[0].x, xds[0].y, xds[1].x, xds[1].y);
+      }
+      // ---- dV += (wP)^T dO, dK += dS^T Q: contraction over the 32 rows
+#pragma unroll
+      for (int t = 0; t < DT; ++t) bq[t] = col_pair(q_rm, QROW, r0, t * 16);
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
-          acc_k[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_ds[tt], *(const bf16x8_t*)&bq, acc_k[tt][t], 0, 0, 0);
-      }
+          acc_v[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_p[tt], __builtin_bit_cast(bf16x8_t, bo[t]), acc_v[tt][t], 0, 0, 0);
 #pragma unroll
-      for (int t = 0; t < VT; ++t) {
-        const uint2 b0 = col_read(o_rm, OROW, r0, t * 16);
-        const uint2 b1 = col_read(o_rm, OROW, r0 + 16, t * 16);
-        const uint4 bo = make_uint4(b0.x, b0.y, b1.x, b1.y);
+      for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
-          acc_v[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_p[tt], *(const bf16x8_t*)&bo, acc_v[tt][t], 0, 0, 0);
-      }
+          acc_k[tt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a_ds[tt], __builtin_bit_cast(bf16x8_t, bq[t]), acc_k[tt][t], 0, 0, 0);
     }
     // the next round's rows (gathered while this round computed) go to the other buffer, which
     // was last read a round ago (before the previous barrier); its gathers follow
@@ -578,25 +605,28 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   }
 }
 
-// the segments of the cut chunks, four features per thread, segments in order
+// the partial results of the cut chunks, four features per thread, ranges and their segments in order
 template <int D, int DV>
 __global__ void __launch_bounds__(256)
 bw_dkdv_sum_kernel(const int* __restrict__ offsets, void* __restrict__ dk_out, void* __restrict__ dv_out, BwDims dm) {
-  const int cell = blockIdx.x;
-  const int cnt = offsets[cell + 1] - offsets[cell];
-  if (cnt <= dm.items.seg_pairs) return;
-  const int ns = (cnt + dm.items.seg_pairs - 1) / dm.items.seg_pairs;
-  const int c = cell % dm.nchunk, unit = cell / dm.nchunk;
+  const int c = blockIdx.x % dm.nchunk, unit = blockIdx.x / dm.nchunk;
+  const int nr = dm.items.n_range;
+  const int cell0 = unit * nr * dm.nchunk + c;  // of the first range
+  if (nr == 1 && offsets[cell0 + 1] - offsets[cell0] <= dm.items.seg_pairs) return;
   const int hk = unit % dm.H;
   const long b = unit / dm.H;
   constexpr int F4 = (D + DV) / 4, N = BW_S * F4;
-  const f32x4_t* src = (const f32x4_t*)(dm.part + (long)dm.items.part_off[cell] * (BW_S * (D + DV)));
   for (int i = blockIdx.y * 256 + threadIdx.x; i < N; i += gridDim.y * 256) {
-    f32x4_t x = src[i];
-    for (int k = 1; k < ns; ++k) {
-      const f32x4_t y = src[(long)k * N + i];
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < nr; ++r) {
+      const int cell = cell0 + r * dm.nchunk;
+      const int ns = dm.items.segs(offsets[cell + 1] - offsets[cell]);
+      const f32x4_t* src = (const f32x4_t*)(dm.part + (long)dm.items.part_off[cell] * (BW_S * (D + DV)));
+      for (int k = 0; k < ns; ++k) {
+        const f32x4_t y = src[(long)k * N + i];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] += y[e];
+        for (int e = 0; e < 4; ++e) x[e] += y[e];
+      }
     }
     const int t = i / F4, f = (i - t * F4) * 4;
     const long row = (b * dm.Lkv + (long)c * BW_S + t) * dm.H + hk;
@@ -1085,36 +1115,50 @@ static int bq_pick_T(int L, int G, int D, int Dv, int K, int nchunk, bool stage,
 
 struct BwLayout {
   size_t counts, offsets, cursor, pairs, ka, va, kt, vmax, kmax, items, n_items, part_off, part, total;
-  int seg_pairs;
+  int seg_pairs, range, n_range;
   size_t max_items;
 };
+// Queries per range of the dK/dV kernel: the gathered rows of a unit should stay in an XCD's L2 (4 MiB, and the
+// workgroups of one range overlap with those of the next).  Where a unit's rows are more than 3 MiB the items go range
+// by range of 2 MiB, at the price of a partial result per (range, chunk).  B2 L8192 32/4 heads of 64, dK/dV + sum:
+// 942 us in one range, 857 in ranges of 1 MiB, 806 of 2, 912 of 3, 914 of 4; B1 L8192 32/8 of 128: 980, 1016, 960, 1040, 1039.
+static int bw_range(int L, int G, int D, int Dv) {
+  const size_t row = (size_t)G * (D + Dv) * 2;
+  if ((size_t)L * row <= ((size_t)3 << 20)) return L;
+  const int r = (int)(((size_t)2 << 20) / row) & ~255;
+  return r > 256 ? r : 256;
+}
 // Pairs per work item of the dK/dV kernel: about 2048 items of equal size in all (some four rounds of the
 // workgroups that fit the chip), but no less than 512 rows, whose gathers are four times the partial result's bytes.
 static BwLayout bw_layout(int B, int L, int Lkv, int G, int H, int D, int Dv, int K) {
-  const size_t cells = (size_t)B * H * (Lkv / BW_S);
+  const size_t chunks = (size_t)B * H * (Lkv / BW_S);
   const size_t pairs = (size_t)B * L * H * K;
   size_t seg = (pairs + 2047) / 2048;
   const size_t least = G < 8 ? 512 / G : 64;
   seg = ((seg > least ? seg : least) + 63) & ~(size_t)63;
   BwLayout lo;
+  lo.range = bw_range(L, G, D, Dv);
+  lo.n_range = (L + lo.range - 1) / lo.range;
+  const size_t cells = chunks * lo.n_range;
   size_t o = 0;
   lo.counts = o; o += bw_round((cells + 1) * 4);
   lo.offsets = o; o += bw_round((cells + 1) * 4);
   lo.cursor = o; o += bw_round((cells + 1) * 4);
   lo.pairs = o; o += bw_round((size_t)B * L * H * K * 4);
-  lo.ka = o; o += bw_round(cells * BW_S * D * 2);
-  lo.va = o; o += bw_round(cells * BW_S * Dv * 2);
-  lo.kt = o; o += bw_round(cells * BW_S * D * 2);
-  lo.vmax = o; o += bw_round(cells * 4);
-  lo.kmax = o; o += bw_round(cells * 4);
-  const bool cut = (size_t)L > seg;  // (no chunk has more than L pairs unless a query names it twice)
+  lo.ka = o; o += bw_round(chunks * BW_S * D * 2);
+  lo.va = o; o += bw_round(chunks * BW_S * Dv * 2);
+  lo.kt = o; o += bw_round(chunks * BW_S * D * 2);
+  lo.vmax = o; o += bw_round(chunks * 4);
+  lo.kmax = o; o += bw_round(chunks * 4);
+  const bool cut = (size_t)lo.range > seg;  // (no cell has more pairs than its range queries unless one names a chunk twice)
   lo.seg_pairs = cut ? (int)seg : 0x7fffffff;
   lo.max_items = cells + (cut ? pairs / seg : 0);
   lo.items = o; o += bw_round(lo.max_items * sizeof(int2));
   lo.n_items = o; o += bw_round(4);
   lo.part_off = o; o += bw_round((cells + 1) * 4);
-  // a cell of n > seg pairs has ceil(n / seg) <= 2 n / seg partial results
-  lo.part = o; o += cut ? bw_round(2 * (pairs / seg + 1) * BW_S * (size_t)(D + Dv) * 4) : 0;
+  // one range: a cell of n > seg pairs has ceil(n / seg) <= 2 n / seg partial results; several: every item has one
+  const size_t parts = lo.n_range > 1 ? lo.max_items < pairs ? lo.max_items : pairs : cut ? 2 * (pairs / seg + 1) : 0;
+  lo.part = o; o += bw_round(parts * BW_S * (size_t)(D + Dv) * 4);
   lo.total = o;
   return lo;
 }
@@ -1150,7 +1194,7 @@ static int bw_launch_dkdv(int G, dim3 grid, hipStream_t st, const bf16_t* q, con
     default: return -1;
   }
 #undef BW_CALL
-  if (dm.items.seg_pairs != 0x7fffffff)  // some chunk may have been cut
+  if (dm.items.n_range > 1 || dm.items.seg_pairs != 0x7fffffff)  // some chunk may have been cut
     hipLaunchKernelGGL((bw_dkdv_sum_kernel<D, DV>), dim3((unsigned)((long)dm.B * dm.H * dm.nchunk), 4), dim3(256), 0, st,
                        offsets, dk, dv, dm);
   return HILS_OK;
@@ -1211,9 +1255,10 @@ static bool bq_stage_pays(long units, int L, int G, int D, int Dv, int K, int nc
 // offsets (cells + 1 ints, cells = B*H*nchunk), cursor (scratch) and the pairs (t << 8 | slot)
 // grouped by (b, h, chunk).  Also used by the top-k backward.
 static void bw_build_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
-                           const BwItems& items, int B, int L, int H, int K, int nchunk, void* stream) {
+                           const BwItems& items, int B, int L, int H, int K, int nchunk, int range, void* stream) {
   hipStream_t st = (hipStream_t)stream;
-  const long cells = (long)B * H * nchunk;
+  const int n_range = (L + range - 1) / range;
+  const long cells = (long)B * H * nchunk * n_range;
   {
     const long n = cells + 1;
     hipLaunchKernelGGL(bw_fill_int_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, counts, 0, n);
@@ -1221,18 +1266,18 @@ static void bw_build_index(const int32_t* indices, int* counts, int* offsets, in
   // segments of queries per workgroup: short enough for a few thousand workgroups (the LDS atomics of
   // a workgroup on one chunk's counter serialise), long enough that a workgroup's one global atomic per
   // chunk stays cheap
-  int seg_len = L;
+  int seg_len = n_range > 1 ? 256 : L;  // (a segment lies in one range)
   while ((long)B * H * ((L + seg_len - 1) / seg_len) < 4096 && seg_len > 128) seg_len = (seg_len + 1) / 2;
   dim3 gs((L + seg_len - 1) / seg_len, H, B);
-  hipLaunchKernelGGL(bw_count_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, counts, L, H, K, nchunk, seg_len);
+  hipLaunchKernelGGL(bw_count_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, counts, L, H, K, nchunk, seg_len, range, n_range);
   hipLaunchKernelGGL(bw_scan_kernel, dim3(1), dim3(1024), 0, st, counts, offsets, cursor, (int)cells, items);
-  hipLaunchKernelGGL(bw_scatter_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, cursor, pairs, L, H, K, nchunk, seg_len);
+  hipLaunchKernelGGL(bw_scatter_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, cursor, pairs, L, H, K, nchunk, seg_len, range, n_range);
 }
 
 void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
                             int B, int L, int H, int K, int nchunk, void* stream) {
-  bw_build_index(indices, counts, offsets, cursor, pairs, BwItems{nullptr, nullptr, nullptr, 0}, B, L, H, K, nchunk,
-                 stream);
+  bw_build_index(indices, counts, offsets, cursor, pairs, BwItems{nullptr, nullptr, nullptr, 0, 1}, B, L, H, K, nchunk,
+                 L, stream);
 }
 
 // Whole backward on the MFMA kernels: dq (bf16, written), dw (fp32, written at the valid slots),
@@ -1243,7 +1288,6 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
                 float sm_scale, int mask_last, int kv16, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const int nchunk = Lkv / BW_S;
-  const size_t cells = (size_t)B * H * nchunk;
   const BwLayout lo = bw_layout(B, L, Lkv, HQ / H, H, D, Dv, K);
   char* ws = (char*)workspace;
   int* counts = (int*)(ws + lo.counts);
@@ -1256,7 +1300,7 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   float* vmax = (float*)(ws + lo.vmax);
   float* kmax = (float*)(ws + lo.kmax);
   const int G = HQ / H;
-  if (H > 65535 || B > 65535 || cells > (1u << 30)) return -1;
+  if (H > 65535 || B > 65535 || (size_t)B * H * nchunk * lo.n_range > (1u << 30)) return -1;
   // (24-bit row strides and 32-bit offsets inside a block of up to 256 queries)
   if ((long)HQ * (D > Dv ? D : Dv) >= (1 << 23) || (long)HQ * NW >= (1 << 22) || (long)HQ * K >= (1 << 22)) return -1;
   // ---- operand packing: K as A operand (+ max|V|), V as A operand + K transposed (+ max|K|)
@@ -1293,8 +1337,8 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
     if (rc != HILS_OK) return rc;
   }
   // ---- inverse index, then dK, dV
-  const BwItems items{(int2*)(ws + lo.items), (int*)(ws + lo.n_items), (int*)(ws + lo.part_off), lo.seg_pairs};
-  bw_build_index(indices, counts, offsets, cursor, pairs, items, B, L, H, K, nchunk, stream);
+  const BwItems items{(int2*)(ws + lo.items), (int*)(ws + lo.n_items), (int*)(ws + lo.part_off), lo.seg_pairs, lo.n_range};
+  bw_build_index(indices, counts, offsets, cursor, pairs, items, B, L, H, K, nchunk, lo.range, stream);
   BwDims dm{L, Lkv, HQ, H, K, NW, nchunk, mask_last, sm_scale, kv16, B, slope, items, (float*)(ws + lo.part)};
   if (kv16 && Lkv > nchunk * BW_S) {  // tokens behind the last whole chunk are never attended
     for (int b2 = 0; b2 < B; ++b2) {
