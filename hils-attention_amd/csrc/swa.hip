@@ -44,6 +44,11 @@ static dim3 swa_xcd_grid(int n_blk, int H, int B) { return dim3((unsigned)(((lon
 // compute unit, one loading while the other computes; taken when no block of 128/G queries needs more
 // than two tiles (window <= 64 at chunk 64), at the price of every tile being staged by twice as many
 // workgroups (L2 hits).
+// Few blocks (SPLIT): a workgroup walks its window in series, two wavefronts per SIMD whose tiles (235 vector and matrix
+// instructions) take turns, so with fewer workgroups than compute units the walk is the kernel.  Two wavefronts then own
+// the same rows and take every other tile, half the queries per workgroup, twice the workgroups; their sums meet in LDS.
+// L1999, 16/2 heads of 64, window 512: 26.6 -> 19.5 us.  The pipelined phases of this form do nothing for a full chip
+// (B2 L8192 32/4 x 64 206 -> 212 us, L8192 32/8 x 128 153 -> 160): the other workgroups hide the loads there.
 #define SWA_FWD_RT 2   // 16-row tiles per wavefront
 #define SWA_LAZY 6.f   // log2 of the growth of a row's maximum that moves its reference point
 
@@ -54,14 +59,16 @@ static size_t swa_fwd_smem() {
   return (tiles > outs ? tiles : outs) + (size_t)NWV * SWA_FWD_RT * 16 * sizeof(float);
 }
 
-template <int D, int DV, int G, int NWV, int RES>
+template <int D, int DV, int G, int NWV, int RES, int SPLIT>
 __global__ void __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2)))
 swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
             bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int n_qt, int n_b) {
   constexpr int RT = SWA_FWD_RT, NT = NWV * 64;
   constexpr int KS = D / 32, DT = DV / 16;
   constexpr int QW = 16 * RT / G > 0 ? 16 * RT / G : 1;  // queries per wavefront (G <= 16: >= 2)
-  constexpr int QB = NWV * 16 * RT / G;                  // queries per workgroup
+  constexpr int NRG = NWV / SPLIT;                       // wavefronts with rows of their own
+  constexpr int QB = NRG * 16 * RT / G;                  // queries per workgroup
+  static_assert(SPLIT == 1 || (SPLIT == 2 && RES == 4), "a phase's two tiles go to the two wavefronts with the same rows");
   constexpr int KP = D * 2 + 16, VP = DV * 2 + 16;       // bytes per staged row
   constexpr int KSEG = D / 8, VSEG = DV / 8;
   constexpr int KPT = 64 * KSEG / NT, VPT = 64 * VSEG / NT;  // 16-byte pieces per thread and tile
@@ -74,7 +81,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
   typedef short swa_s8 __attribute__((ext_vector_type(8)));
   extern __shared__ __align__(16) unsigned char swa_dyn[];
   constexpr size_t TILES_B = (size_t)RES * TILE_B;
-  constexpr size_t OUTS_B = (size_t)NWV * 16 * RT * OP;
+  constexpr size_t OUTS_B = (size_t)NRG * 16 * RT * OP;
   float* bc_all = (float*)(swa_dyn + (TILES_B > OUTS_B ? TILES_B : OUTS_B));  // [wave][rt][16] row factors
   const int tid = threadIdx.x, lane = tid & 63;
   // in a scalar register: what is derived from it (the wavefront's key range, "does this tile need
@@ -87,7 +94,8 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
   if (!swa_xcd_unit(n_qt, dm.H, n_b, qt, hk, b)) return;
   qt = n_qt - 1 - qt;
   const int tq0 = qt * QB;
-  const int t0 = tq0 + wave * QW;
+  const int rg = wave % NRG, share = wave / NRG;  // its rows, and which of a phase's tiles it takes
+  const int t0 = tq0 + rg * QW;
   const int q_off = dm.kv_start + dm.Lk - dm.Lq;  // absolute position of query 0
 
   bf16x8_t qa[RT][KS];
@@ -283,63 +291,140 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
     }
   };
 
-  // loads of a phase of N resident tiles, two tiles in flight (tokens past the end read the last row:
-  // their scores are masked); one copy of the code per N, so no load is conditional
-  auto phase = [&](int tile0, auto n_const) __attribute__((always_inline)) {
-    constexpr int N = decltype(n_const)::value;
-    swa_u32x4 kr[2][KPT], vr[2][VPT];  // two tiles' loads in flight
-    auto issue = [&](int ti, swa_u32x4 (&kd)[KPT], swa_u32x4 (&vd)[VPT]) __attribute__((always_inline)) {
+  // a tile's loads (tokens past the end read the last row: their scores are masked) and their way into the LDS
+  auto issue = [&](int tile, swa_u32x4 (&kd)[KPT], swa_u32x4 (&vd)[VPT]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < KPT; ++i) {
-        const int pc = tid + NT * i;
-        int tok = (tile0 + ti) * 64 + pc / KSEG;
-        tok = tok < dm.Lk ? tok : dm.Lk - 1;
-        kd[i] = *(const swa_u32x4*)(k + b * dm.k_batch + ((long)tok * dm.H + hk) * D + (pc % KSEG) * 8);
-      }
+    for (int i = 0; i < KPT; ++i) {
+      const int pc = tid + NT * i;
+      int tok = tile * 64 + pc / KSEG;
+      tok = tok < dm.Lk ? tok : dm.Lk - 1;
+      kd[i] = *(const swa_u32x4*)(k + b * dm.k_batch + ((long)tok * dm.H + hk) * D + (pc % KSEG) * 8);
+    }
 #pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        const int pc = tid + NT * i;
-        int tok = (tile0 + ti) * 64 + pc / VSEG;
-        tok = tok < dm.Lk ? tok : dm.Lk - 1;
-        vd[i] = *(const swa_u32x4*)(v + b * dm.v_batch + ((long)tok * dm.H + hk) * DV + (pc % VSEG) * 8);
-      }
-    };
-    auto stash = [&](int ti, const swa_u32x4 (&kd)[KPT], const swa_u32x4 (&vd)[VPT]) __attribute__((always_inline)) {
-      unsigned char* k_s = swa_dyn + (size_t)ti * TILE_B;
-      unsigned char* v_s = k_s + 64 * KP;
-#pragma unroll
-      for (int i = 0; i < KPT; ++i) {
-        const int pc = tid + NT * i;
-        *(swa_u32x4*)(k_s + (pc / KSEG) * KP + (pc % KSEG) * 16) = kd[i];
-      }
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        const int pc = tid + NT * i;
-        *(swa_u32x4*)(v_s + (pc / VSEG) * VP + (pc % VSEG) * 16) = vd[i];
-      }
-    };
-    issue(0, kr[0], vr[0]);
-    if (N > 1) issue(1, kr[1], vr[1]);
-#pragma unroll
-    for (int ti = 0; ti < N; ++ti) {
-      stash(ti, kr[ti & 1], vr[ti & 1]);
-      if (ti + 2 < N) issue(ti + 2, kr[ti & 1], vr[ti & 1]);
+    for (int i = 0; i < VPT; ++i) {
+      const int pc = tid + NT * i;
+      int tok = tile * 64 + pc / VSEG;
+      tok = tok < dm.Lk ? tok : dm.Lk - 1;
+      vd[i] = *(const swa_u32x4*)(v + b * dm.v_batch + ((long)tok * dm.H + hk) * DV + (pc % VSEG) * 8);
     }
   };
-  for (int tile0 = tile_lo; tile0 < tile_hi; tile0 += RES) {
-    if (tile0 != tile_lo) __syncthreads();  // the previous phase's tiles are no longer read
-    const int n = tile_hi - tile0 < RES ? tile_hi - tile0 : RES;
-    if (RES >= 4 && n == 4) phase(tile0, std::integral_constant<int, RES >= 4 ? 4 : 1>{});
-    else if (RES >= 3 && n == 3) phase(tile0, std::integral_constant<int, RES >= 3 ? 3 : 1>{});
-    else if (n == 2) phase(tile0, std::integral_constant<int, 2>{});
-    else phase(tile0, std::integral_constant<int, 1>{});
-    __syncthreads();
-    for (int ti = 0; ti < n; ++ti) {  // one copy of the tile code
-      const int tile = tile0 + ti;
-      if (tile * 64 < w_hi && tile * 64 + 64 > w_lo) {  // uniform: some row of the wavefront sees the tile
-        const unsigned char* k_s = swa_dyn + (size_t)ti * TILE_B;
-        tile_step(tile, k_s, k_s + 64 * KP);
+  auto stash = [&](int slot, const swa_u32x4 (&kd)[KPT], const swa_u32x4 (&vd)[VPT]) __attribute__((always_inline)) {
+    unsigned char* k_s = swa_dyn + (size_t)slot * TILE_B;
+    unsigned char* v_s = k_s + 64 * KP;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+      const int pc = tid + NT * i;
+      *(swa_u32x4*)(k_s + (pc / KSEG) * KP + (pc % KSEG) * 16) = kd[i];
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int pc = tid + NT * i;
+      *(swa_u32x4*)(v_s + (pc / VSEG) * VP + (pc % VSEG) * 16) = vd[i];
+    }
+  };
+  swa_u32x4 kr[2][KPT], vr[2][VPT];  // two tiles' loads in flight
+  auto resident = [&](int tile, int slot) __attribute__((always_inline)) {
+    if (tile * 64 < w_hi && tile * 64 + 64 > w_lo) {  // uniform: some row of the wavefront sees the tile
+      const unsigned char* k_s = swa_dyn + (size_t)slot * TILE_B;
+      tile_step(tile, k_s, k_s + 64 * KP);
+    }
+  };
+  if constexpr (SPLIT == 2) {
+    // phases of two tiles in the two halves of the resident four: the next phase's loads are in flight behind this
+    // one's arithmetic (a tile past the end is loaded and not worked on)
+    if (tile_lo < tile_hi) {
+      issue(tile_lo, kr[0], vr[0]);
+      issue(tile_lo + 1, kr[1], vr[1]);
+      stash(0, kr[0], vr[0]);
+      stash(1, kr[1], vr[1]);
+      lds_barrier();
+    }
+    int half = 0;
+    for (int tile0 = tile_lo; tile0 < tile_hi; tile0 += 2, half ^= 2) {
+      const bool more = tile0 + 2 < tile_hi;
+      if (more) {
+        issue(tile0 + 2, kr[0], vr[0]);
+        issue(tile0 + 3, kr[1], vr[1]);
       }
+      if (tile0 + share < tile_hi) resident(tile0 + share, half + share);
+      if (more) {  // (the other half was last read a phase ago, before the barrier)
+        stash(half ^ 2, kr[0], vr[0]);
+        stash((half ^ 2) + 1, kr[1], vr[1]);
+      }
+      lds_barrier();
+    }
+  } else {
+    // loads of a phase of N resident tiles; one copy of the code per N, so no load is conditional
+    auto phase = [&](int tile0, auto n_const) __attribute__((always_inline)) {
+      constexpr int N = decltype(n_const)::value;
+      issue(tile0, kr[0], vr[0]);
+      if (N > 1) issue(tile0 + 1, kr[1], vr[1]);
+#pragma unroll
+      for (int ti = 0; ti < N; ++ti) {
+        stash(ti, kr[ti & 1], vr[ti & 1]);
+        if (ti + 2 < N) issue(tile0 + ti + 2, kr[ti & 1], vr[ti & 1]);
+      }
+    };
+    for (int tile0 = tile_lo; tile0 < tile_hi; tile0 += RES) {
+      if (tile0 != tile_lo) __syncthreads();  // the previous phase's tiles are no longer read
+      const int n = tile_hi - tile0 < RES ? tile_hi - tile0 : RES;
+      if (RES >= 4 && n == 4) phase(tile0, std::integral_constant<int, RES >= 4 ? 4 : 1>{});
+      else if (RES >= 3 && n == 3) phase(tile0, std::integral_constant<int, RES >= 3 ? 3 : 1>{});
+      else if (n == 2) phase(tile0, std::integral_constant<int, 2>{});
+      else phase(tile0, std::integral_constant<int, 1>{});
+      __syncthreads();
+      for (int ti = 0; ti < n; ++ti) resident(tile0 + ti, ti);  // one copy of the tile code
+    }
+  }
+  if constexpr (SPLIT == 2) {
+    // the second share of every row group hands its sums over, [row group][register][lane], and is done (the last
+    // barrier lies behind the tiles' last use)
+    f32x4_t* xch = (f32x4_t*)swa_dyn;
+    constexpr int XR = RT * DT + 1;
+    static_assert((size_t)NRG * XR * 64 * 16 <= TILES_B, "the exchange fits the tiles");
+    if (share) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) xch[(rg * XR + rt * DT + dt) * 64 + lane] = acc[rt][dt];
+      xch[(rg * XR + RT * DT) * 64 + lane] = f32x4_t{m_run[0], l_run[0], m_run[1], l_run[1]};
+    }
+    lds_barrier();
+    if (!share) {
+      const f32x4_t ml = xch[(rg * XR + RT * DT) * 64 + lane];
+      float fa[RT], fb[RT];  // of this lane's rows
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const float m2 = ml[2 * rt], l2 = ml[2 * rt + 1];
+        // (no maximum: nothing was seen, and the sums are zero, or scores that are not numbers, which the sums keep)
+        const float M = fmaxf(m_run[rt], m2);
+        const bool any = M > HILS_NEG_INF;
+        fa[rt] = any ? __builtin_amdgcn_exp2f((m_run[rt] - M) * c2) : 1.f;
+        fb[rt] = any ? __builtin_amdgcn_exp2f((m2 - M) * c2) : 1.f;
+        m_run[rt] = M;
+        l_run[rt] = l_run[rt] * fa[rt] + l2 * fb[rt];
+        if (j == 0) bc_s[rt * 16 + col] = fa[rt];
+      }
+      __builtin_amdgcn_wave_barrier();
+      f32x4_t ca[RT], cb[RT];  // ... of the accumulators' rows 4j + i
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) ca[rt] = *(const f32x4_t*)&bc_s[rt * 16 + 4 * j];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+        if (j == 0) bc_s[rt * 16 + col] = fb[rt];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) cb[rt] = *(const f32x4_t*)&bc_s[rt * 16 + 4 * j];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const f32x4_t x = xch[(rg * XR + rt * DT + dt) * 64 + lane];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[rt][dt][i] = acc[rt][dt][i] * ca[rt][i] + x[i] * cb[rt][i];
+        }
     }
   }
   // ---- finalize: o = acc / l, lse = ln(l) + max * scale ----
@@ -349,14 +434,15 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
     if (j == 0) bc_s[rt * 16 + col] = inv;
     const int row = rt * 16 + col;
     const int t = t0 + row / G, g = row % G;
-    if (j == 0 && t < dm.Lq)
+    if (j == 0 && t < dm.Lq && share == 0)
       lse[(b * dm.Lq + t) * (long)dm.HQ + hk * G + g] =
           l_run[rt] > 0.f ? (m_run[rt] * c2 + __builtin_amdgcn_logf(l_run[rt])) * HILS_LN2 : HILS_NEG_INF;
   }
   __syncthreads();  // every wavefront is through with the tiles: their LDS becomes the output stage
+  if (share) return;
   // Each wavefront parks its normalised rows as bf16 and writes them out as 16-byte pieces (a query's
   // heads are contiguous).
-  unsigned char* ob = swa_dyn + (size_t)wave * (16 * RT) * OP;
+  unsigned char* ob = swa_dyn + (size_t)rg * (16 * RT) * OP;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const float4 c4 = *(const float4*)&bc_s[rt * 16 + 4 * j];
@@ -863,14 +949,14 @@ extern "C" size_t hils_swa_bwd_workspace(int B, int L, int HQ, int H, int D, int
   return s == 1 ? 0 : (size_t)((L + nt - 1) / nt) * H * B * s * nt * (D + Dv) * sizeof(float);
 }
 
-template <int D, int DV, int G, int NWV, int RES>
+template <int D, int DV, int G, int NWV, int RES, int SPLIT = 1>
 static int swa_fwd_launch_shape(int B, hipStream_t st, const bf16_t* q, const bf16_t* k, const bf16_t* v,
                                 bf16_t* o, float* lse, const SwaDims& dm) {
   const size_t smem = swa_fwd_smem<D, DV, NWV, RES>();
-  auto kern = swa_fwd_blk<D, DV, G, NWV, RES>;
+  auto kern = swa_fwd_blk<D, DV, G, NWV, RES, SPLIT>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_swa_fwd")) return rc;
-  const int QB = NWV * 16 * SWA_FWD_RT / G;  // queries of a workgroup (>= 8: G <= 16)
+  const int QB = NWV / SPLIT * 16 * SWA_FWD_RT / G;  // queries of a workgroup (>= 8: G <= 16)
   const int n_qt = (dm.Lq + QB - 1) / QB;
   hipLaunchKernelGGL(kern, swa_xcd_grid(n_qt, dm.H, B), dim3(NWV * 64), smem, st, q, k, v, o, lse, dm, n_qt, B);
   return HILS_OK;
@@ -907,6 +993,8 @@ static int swa_fwd_launch(int B, hipStream_t st, const bf16_t* q, const bf16_t* 
   // where one 8-wavefront workgroup does (150 registers: three wavefronts per SIMD)
   if constexpr (D <= 64 && DV <= 64)
     if (tiles <= 4) return swa_fwd_launch_shape<D, DV, G, 4, 4>(B, st, q, k, v, o, lse, dm);
+  const long wgs = (long)((dm.Lq + 256 / G - 1) / (256 / G)) * dm.H * B;  // of one share
+  if (wgs < hils_device_cus()) return swa_fwd_launch_shape<D, DV, G, 8, 4, 2>(B, st, q, k, v, o, lse, dm);
   return swa_fwd_launch_shape<D, DV, G, 8, 4>(B, st, q, k, v, o, lse, dm);
 }
 
