@@ -111,13 +111,14 @@ template <int O>
 __device__ __forceinline__ float lane_xor(float x) {
   static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one lane bit");
   const int v = __float_as_int(x);
-  if (O == 1) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
-  if (O == 2) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // quad_perm 2,3,0,1
+  // (every lane has a source: no old value, so that the move folds into the operation that reads it)
+  if (O == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true));   // quad_perm 1,0,3,2
+  if (O == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true));   // quad_perm 2,3,0,1
   if (O == 4) {  // row_shl:4 for the lanes with bit 2 clear, row_shr:4 for the others
     const int a = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);
     return __int_as_float(__builtin_amdgcn_update_dpp(a, v, 0x114, 0xf, 0xa, false));
   }
-  if (O == 8) return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false));  // row_ror:8
+  if (O == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true));  // row_ror:8
   return __shfl_xor(x, O, 64);
 }
 

@@ -92,6 +92,15 @@ extern "C" int hils_rope(const void* x, const void* cos_t, const void* sin_t, vo
 // a head vector stay inside 8, 16 or 32 lanes and run as DPP moves (no LDS traffic).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float np_round_bf16(float x) { return bf2f(f2bf(x)); }
+// a vector rounded to bf16 in pairs (three instructions for two values)
+__device__ __forceinline__ void np_round8(float (&f)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const uint32_t u = pack_bf2(f[e], f[e + 1]);
+    f[e] = __uint_as_float(u << 16);
+    f[e + 1] = __uint_as_float(u & 0xffff0000u);
+  }
+}
 
 struct NpDims {
   int B, L, H, S, hg, hg_log2, nchunk_all, nchunk_full;
@@ -101,12 +110,29 @@ struct NpDims {
 
 constexpr int kNpBatch = 4;  // steps whose loads are in flight together
 
+// The mirrored lane of the eight (one move that folds into its use; the lane with bit 2 flipped takes two and copies).
+__device__ __forceinline__ float np_mirror8(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, true));  // row_half_mirror
+}
+// Piece of the head vector that a row's lane holds, and the value of the lane with the other half's: with eight lanes
+// the upper four hold their pieces in reverse, so that the mirrored lane has the partner.
+template <int LPR>
+__device__ __forceinline__ int np_piece(int lane) {
+  const int p = lane % LPR;
+  return LPR == 8 && p >= 4 ? 11 - p : p;
+}
+template <int LPR>
+__device__ __forceinline__ float np_other(float v) {
+  if (LPR == 8) return np_mirror8(v);
+  return lane_xor<LPR / 2>(v);
+}
+
 // sum over the LPR lanes of a row
 template <int LPR>
 __device__ __forceinline__ float np_row_sum(float v) {
   v += lane_xor<1>(v);
   v += lane_xor<2>(v);
-  v += lane_xor<4>(v);
+  v += np_mirror8(v);  // (four lanes alike by now)
   if (LPR > 8) v += lane_xor<8>(v);
   if (LPR > 16) v += lane_xor<16>(v);
   return v;
@@ -123,7 +149,7 @@ norm_rope_pool_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
   const int hgroups = dm.H >> dm.hg_log2, tps = RPI >> dm.hg_log2;  // tokens per step
   const int bn = blockIdx.x / hgroups, hg0 = (blockIdx.x % hgroups) << dm.hg_log2;
   const int b = bn / dm.nchunk_all, n = bn % dm.nchunk_all;
-  const int p = lane % LPR, r = lane / LPR;
+  const int p = np_piece<LPR>(lane), r = lane / LPR;
   const int h = hg0 + (r & (dm.hg - 1)), tt = r >> dm.hg_log2;
   const long row0 = (long)b * dm.L;
   float wv[8];
@@ -160,25 +186,35 @@ norm_rope_pool_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
         for (int e = 0; e < 8; ++e) ss = fmaf(f[e], f[e], ss);
         const float rr = rsqrtf(np_row_sum<LPR>(ss) * (1.f / D) + dm.eps);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = np_round_bf16(wv[e] * np_round_bf16(f[e] * rr));
+        for (int e = 0; e < 8; ++e) f[e] *= rr;
+        np_round8(f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] *= wv[e];
+        if (cos_t) np_round8(f);  // (else the packed output is that rounding)
       }
       if (cos_t) {
         float c[8], s[8];
         unpack8(cv[u], c);
-        unpack8(sv[u], s);
-        const float sign = p < LPR / 2 ? -1.f : 1.f;  // rotate_half: (-x_hi, x_lo)
+        const uint32_t flip = p < LPR / 2 ? 0x80008000u : 0u;  // rotate_half: (-x_hi, x_lo)
+        unpack8(make_uint4(sv[u].x ^ flip, sv[u].y ^ flip, sv[u].z ^ flip, sv[u].w ^ flip), s);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float other = lane_xor<LPR / 2>(f[e]);
-          f[e] = np_round_bf16(np_round_bf16(f[e] * c[e]) + np_round_bf16(sign * other * s[e]));
-        }
+        for (int e = 0; e < 8; ++e) s[e] *= np_other<LPR>(f[e]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e] *= f[e];
+        np_round8(c);
+        np_round8(s);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = c[e] + s[e];
       }
       if (ok) {
         uint4 o;
         o.x = pack_bf2(f[0], f[1]); o.y = pack_bf2(f[2], f[3]); o.z = pack_bf2(f[4], f[5]); o.w = pack_bf2(f[6], f[7]);
         *(uint4*)(out + ((row0 + t) * dm.H + h) * (long)D + p * 8) = o;
+        if (lmk) {  // of the rounded outputs
+          unpack8(o, f);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += f[e];
+          for (int e = 0; e < 8; ++e) acc[e] += f[e];
+        }
       }
     }
   }
@@ -225,7 +261,7 @@ norm_rope_pool_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
   const int hgroups = dm.H >> dm.hg_log2, tps = RPI >> dm.hg_log2;
   const int bn = blockIdx.x / hgroups, hg0 = (blockIdx.x % hgroups) << dm.hg_log2;
   const int b = bn / dm.nchunk_all, n = bn % dm.nchunk_all;
-  const int p = lane % LPR, r = lane / LPR;
+  const int p = np_piece<LPR>(lane), r = lane / LPR;
   const int h = hg0 + (r & (dm.hg - 1)), tt = r >> dm.hg_log2;
   const long row0 = (long)b * dm.L;
   float wv[8], gl[8], wacc[8];
@@ -272,7 +308,7 @@ norm_rope_pool_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
         const float sign = p < LPR / 2 ? 1.f : -1.f;  // transpose of rotate_half: (u_hi, -u_lo)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float other = lane_xor<LPR / 2>(g[e] * s[e]);
+          const float other = np_other<LPR>(g[e] * s[e]);
           g[e] = fmaf(g[e], c[e], sign * other);
         }
       }
@@ -307,7 +343,7 @@ norm_rope_pool_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict
       for (int o2 = LPR; o2 < 64; o2 <<= 1) wacc[e] += __shfl_xor(wacc[e], o2, 64);
     if (lane < LPR) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) np_red[wave * D + lane * 8 + e] = wacc[e];
+      for (int e = 0; e < 8; ++e) np_red[wave * D + p * 8 + e] = wacc[e];
     }
     lds_barrier();
     for (int c = threadIdx.x; c < D; c += blockDim.x) {
@@ -364,14 +400,25 @@ static int np_heads(int H, int D) {
 
 static long np_blocks(int B, int L, int H, int D, int S) { return (long)B * ((L + S - 1) / S) * (H / np_heads(H, D)); }
 
-// Launch shape: 4 wavefronts per workgroup; up to 16 while the grid has fewer than 16 wavefronts per compute
-// unit and every wavefront still has a token (short sequences: the pass is a chain of a wavefront's loads).
-static NpDims np_dims(int B, int L, int H, int D, int S, int table_per_batch, float eps, int* threads) {
+// Tokens of a workgroup that forms no chunk mean: 64, fewer while the grid leaves compute units idle (a step is 200 to
+// 250 vector instructions of a wavefront: with a chunk per workgroup a short sequence kept 64 of 256 compute units busy,
+// 16 wavefronts each; B2 L1024 16 and 2 heads of 64, forward 9.4 -> 6.3 us, backward 12.5 -> 8.0), down to one step per
+// wavefront.
+static int np_tokens(int B, int L, int H, int D, long least_blocks) {
+  const int tps = 512 / D / np_heads(H, D);
+  int tok = 64;
+  while (tok >= 8 * tps && np_blocks(B, L, H, D, tok) < least_blocks) tok /= 2;
+  return tok;
+}
+
+// Launch shape: 4 wavefronts per workgroup; with a chunk mean up to 16 while the grid has fewer than 16 wavefronts per
+// compute unit and every wavefront still has a token (short sequences: the pass is a chain of a wavefront's loads).
+static NpDims np_dims(int B, int L, int H, int D, int S, bool pool, int table_per_batch, float eps, int* threads) {
   NpDims dm{B, L, H, S, np_heads(H, D), 0, (L + S - 1) / S, L / S, table_per_batch ? (long)L * D : 0, eps};
   while ((1 << dm.hg_log2) < dm.hg) ++dm.hg_log2;
   const int tps = 512 / D / dm.hg, steps = (S + tps - 1) / tps;
   int nw = 4;
-  while (nw < 16 && nw * 2 <= steps && np_blocks(B, L, H, D, S) * nw < 16L * hils_device_cus()) nw *= 2;
+  while (pool && nw < 16 && nw * 2 <= steps && np_blocks(B, L, H, D, S) * nw < 16L * hils_device_cus()) nw *= 2;
   *threads = nw * 64;
   return dm;
 }
@@ -382,7 +429,8 @@ extern "C" int hils_norm_rope_pool_fwd(const void* x, const void* norm_weight, c
   if (int rc = np_check("hils_norm_rope_pool_fwd", x, cos_t, sin_t, B, L, H, D, S)) return rc;
   HILS_REQUIRE(out, "hils_norm_rope_pool_fwd: null output");
   int threads;
-  const NpDims dm = np_dims(B, L, H, D, S, table_per_batch, eps, &threads);
+  if (!lmk) S = np_tokens(B, L, H, D, 4L * hils_device_cus());
+  const NpDims dm = np_dims(B, L, H, D, S, lmk != nullptr, table_per_batch, eps, &threads);
   const dim3 grid((unsigned)np_blocks(B, L, H, D, S));
   const size_t lds = lmk ? (size_t)(threads / 64) * dm.hg * D * sizeof(float) : 0;
 #define NP_FWD(LPR_)                                                                                      \
@@ -395,13 +443,16 @@ extern "C" int hils_norm_rope_pool_fwd(const void* x, const void* norm_weight, c
   return HILS_OK;
 }
 
+// (one block per compute unit: every block is a row of d_weight's sum)
+static int np_bwd_tokens(int B, int L, int H, int D) { return np_tokens(B, L, H, D, hils_device_cus()); }
+
 static int np_bwd(const char* who, const void* x, const void* norm_weight, const void* cos_t, const void* sin_t,
                   const void* d_out, const void* d_lmk, void* dx, float* d_weight, float* part, int B, int L, int H,
                   int D, int S, int table_per_batch, float eps, void* stream) {
   if (int rc = np_check(who, x, cos_t, sin_t, B, L, H, D, S)) return rc;
   HILS_REQUIRE(dx && (d_out || d_lmk), "%s: null pointer", who);
   int threads;
-  const NpDims dm = np_dims(B, L, H, D, S, table_per_batch, eps, &threads);
+  const NpDims dm = np_dims(B, L, H, D, S, d_lmk != nullptr, table_per_batch, eps, &threads);
   const dim3 grid((unsigned)np_blocks(B, L, H, D, S));
   const size_t lds = norm_weight ? (size_t)(threads / 64) * D * sizeof(float) : 0;
 #define NP_BWD(LPR_)                                                                                      \
@@ -419,13 +470,15 @@ extern "C" int hils_norm_rope_pool_bwd(const void* x, const void* norm_weight, c
                                        float* d_weight, int B, int L, int H, int D, int S,
                                        int table_per_batch, float eps, void* stream) {
   HILS_REQUIRE(!norm_weight || d_weight, "hils_norm_rope_pool_bwd: the norm weight needs d_weight");
+  if (!d_lmk && B > 0 && L > 0 && H > 0 && S > 0 && (D == 64 || D == 128 || D == 256)) S = np_bwd_tokens(B, L, H, D);
   return np_bwd("hils_norm_rope_pool_bwd", x, norm_weight, cos_t, sin_t, d_out, d_lmk, dx, d_weight, nullptr, B, L,
                 H, D, S, table_per_batch, eps, stream);
 }
 
 extern "C" size_t hils_norm_rope_pool_bwd_workspace(int B, int L, int H, int D, int S) {
   if (B <= 0 || L <= 0 || H <= 0 || S <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
-  return (size_t)np_blocks(B, L, H, D, S) * D * sizeof(float);
+  const long pooled = np_blocks(B, L, H, D, S), plain = np_blocks(B, L, H, D, np_bwd_tokens(B, L, H, D));
+  return (size_t)(pooled > plain ? pooled : plain) * D * sizeof(float);
 }
 
 extern "C" int hils_norm_rope_pool_bwd_ws(const void* x, const void* norm_weight, const void* cos_t,
@@ -436,6 +489,7 @@ extern "C" int hils_norm_rope_pool_bwd_ws(const void* x, const void* norm_weight
   const char* who = "hils_norm_rope_pool_bwd_ws";
   HILS_REQUIRE(norm_weight && d_weight && workspace, "%s: null pointer", who);
   HILS_REQUIRE(workspace_bytes >= hils_norm_rope_pool_bwd_workspace(B, L, H, D, S), "%s: workspace too small", who);
+  if (!d_lmk && B > 0 && L > 0 && H > 0 && S > 0 && (D == 64 || D == 128 || D == 256)) S = np_bwd_tokens(B, L, H, D);
   if (int rc = np_bwd(who, x, norm_weight, cos_t, sin_t, d_out, d_lmk, dx, nullptr, (float*)workspace, B, L, H, D, S,
                       table_per_batch, eps, stream))
     return rc;

@@ -43,3 +43,24 @@ def test_norm_rope_pool_shapes(pkg, orc, dev, B, L, H, D, S):
     out32, _ = pkg.norm_rope_pool(xd.detach(), w32, cos.to(dev), sin.to(dev), S, pool=False)
     dw32, = torch.autograd.grad(out32, w32, rep(g_o))
     assert dw32.dtype == torch.float32
+
+
+# without the mean a workgroup owns fewer tokens than a chunk: the same arithmetic row by row, so the same bits, and a
+# weight gradient that differs by the order of its fp32 sum (2^-24 times sqrt of the rows added, rounded to bf16)
+@pytest.mark.parametrize("B,L,H,D", [(1, 1999, 16, 64), (2, 1024, 2, 64), (1, 77, 5, 128), (3, 333, 4, 256), (1, 1, 1, 64),
+                                     (16, 4096, 16, 64)])
+def test_norm_rope_without_mean_equals_with(pkg, dev, B, L, H, D):
+    gen = torch.Generator(device=dev).manual_seed(47)
+    x = torch.randn(B, L, H, D, device=dev, generator=gen).bfloat16().requires_grad_()
+    w = (torch.rand(D, device=dev, generator=gen) + 0.5).bfloat16().requires_grad_()
+    ang = torch.rand(L, D // 2, device=dev, generator=gen) * 6.0
+    cos, sin = (torch.cat([f(ang), f(ang)], -1).bfloat16() for f in (torch.cos, torch.sin))
+    g_o = torch.randn(B, L, H, D, device=dev, generator=gen).bfloat16()
+    got = []
+    for pool in (False, True):
+        out, lmk = pkg.norm_rope_pool(x, w, cos, sin, 64, pool=pool)
+        z = [] if lmk is None or not lmk.numel() else [torch.zeros_like(lmk)]
+        got.append([out, *torch.autograd.grad([out, *([lmk] if z else [])], [x, w], [g_o, *z])])
+    (o1, dx1, dw1), (o2, dx2, dw2) = got
+    assert torch.equal(o1, o2) and torch.equal(dx1, dx2)
+    assert (dw1.float() - dw2.float()).abs().max() <= 2.0 ** -7 * dw2.float().abs().max()
