@@ -510,16 +510,19 @@ sparse_attn_fwd_gather(const bf16_t* __restrict__ q, bf16_t* qp, const bf16_t* _
       for (int i = 0; i < 4; ++i) t.orow[i] = base + i * DV;
     } else {
       int pk_o[4];
+      if (t.n == QT) {  // neighbouring entries, no clamps
+        const int* po = pairs + p + (4 * j) / G;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int qsl = (4 * j + i) / G;
-        pk_o[i] = pairs[p + (qsl < last ? qsl : last)];
+        for (int i = 0; i < 4; ++i) pk_o[i] = po[i / G];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int qsl = (4 * j + i) / G;
+          pk_o[i] = pairs[p + (qsl < last ? qsl : last)];
+        }
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = 4 * j + i;
-        t.orow[i] = ((pk_o[i] >> 8) * G + rr % G) * DV + r;
-      }
+      for (int i = 0; i < 4; ++i) t.orow[i] = (int)__umul24((unsigned)pk_o[i] >> 8, (unsigned)(G * DV)) + (i % G) * DV + r;
     }
     if constexpr (decltype(flt_c)::value) {  // a padding row's zero times an infinity is no zero: it is left out
 #pragma unroll
