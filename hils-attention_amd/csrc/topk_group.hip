@@ -26,6 +26,7 @@
 // kernels of topk.hip.  With a bias the registers hold the biased logits (what the log-sum-exp and
 // the selection work on) and a winner's raw score is its logit minus the bias again.
 #include "topk_group_kernel.h"
+#include "topk_cols_kernel.h"
 
 // plain: no Gumbel noise and no drop mask (a bias is fine)
 bool hils_topk_group_covers(int N, int G, int D, int topk, int per_qhead, bool plain) {
@@ -74,14 +75,27 @@ int hils_topk_group_launch(const void* q, const void* lmk_packed, const float* l
     dim3 grid((t_hi - t + NQ * QGROUPS - 1) / (NQ * QGROUPS), h_kv, B);
     const TgArgs a{(const bf16_t*)q, (const uint4*)lmk_packed, lse_swa, bias, indices, (bf16_t*)scores, lse_total,
                    sel_logits, L, N, h_kv, G, topk, block_size, window_size, causal, q_offset, sm_scale, t, t_hi, lse_bf16};
-    if (NB == 64) {
+    if (GM == 1 && NB <= 16 && !exp) {
+      // one head per KV head: queries as columns, 16 at once (B4 L8192 16/16 heads of 64, top-32: 174 -> 98 us; past 256
+      // chunks two copies of the scores do not fit the registers)
+      const int bs_shift = (block_size > 0 && (block_size & (block_size - 1)) == 0) ? __builtin_ctz(block_size) : -1;
+      grid.x = (t_hi - t + 16 * TC_WAVES - 1) / (16 * TC_WAVES);
+      auto cols = [&](auto ks, auto bi) {
+        if (NB == 8) hipLaunchKernelGGL((topk_fwd_cols_kernel<ks.value, 8, bi.value>), grid, dim3(64 * TC_WAVES), 0, st, a, bs_shift);
+        else hipLaunchKernelGGL((topk_fwd_cols_kernel<ks.value, 16, bi.value>), grid, dim3(64 * TC_WAVES), 0, st, a, bs_shift);
+      };
+      auto with_bias = [&](auto ks) {
+        if (bias) cols(ks, std::true_type{}); else cols(ks, std::false_type{});
+      };
+      if (D == 64) with_bias(std::integral_constant<int, 2>{}); else with_bias(std::integral_constant<int, 4>{});
+    } else if (NB == 64) {
       tg_launch_wide(GM, D, per_qhead != 0, halves, exp, grid, st, a);
     } else {
       tg_dispatch(GM, D, bias != nullptr, per_qhead != 0, halves, [&](auto gm, auto ks, auto bi, auto pq, auto hf) {
 #define TG_NBS(NB_, EX_) tg_call<gm.value, ks.value, NB_, EX_, bi.value, pq.value, hf.value>(grid, st, a)
         if (exp) TG_NBS(32, true);
-        else if (NB == 8) TG_NBS(8, false);
-        else if (NB == 16) TG_NBS(16, false);
+        else if (gm.value > 1 && NB == 8) TG_NBS((gm.value > 1 ? 8 : 24), false);  // (one head: above)
+        else if (gm.value > 1 && NB == 16) TG_NBS((gm.value > 1 ? 16 : 24), false);
         else if (NB == 24) TG_NBS(24, false);
         else TG_NBS(32, false);
 #undef TG_NBS
