@@ -807,8 +807,9 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   return HILS_OK;
 }
 
-// Segments of the dK walks: with two workgroups per compute unit (what registers allow) about 1.6 times as
-// many items as fit at once, in segments no shorter than eight tiles (a partial result is as many bytes as four).
+// Segments of the dK walks: with two workgroups per compute unit (what registers allow) about 2.6 times as
+// many items as fit at once, in segments no shorter than eight tiles (a partial result is as many bytes as four).  dK +
+// sum, us, for 1.6 / 2.6 / 4 / 6 times: L8192 32/8 heads of 128 721, 703, 677, 698; L6000 16/16 of 64 124, 119, 122, 131.
 static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
   const int n_pair = (N + 1) / 2, QT = 64 / G, n_tiles = (L + QT - 1) / QT;
   long total = 0;
@@ -818,7 +819,7 @@ static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
     total += len;
   }
   const int longest = n_tiles - lz_tile0(0, W, QT);
-  long target = total * B * H / (3L * hils_device_cus());
+  long target = total * B * H / (5L * hils_device_cus());
   if (target < 8) target = 8;
   LzSeg sg{(int)(target < (1 << 30) ? target : (1 << 30)), 1 << 30};
   sg.max_seg = lz_nseg(longest, sg);
