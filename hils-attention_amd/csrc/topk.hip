@@ -3156,27 +3156,30 @@ topk_bwd_dlmk_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q
 // row: dq = sm_scale * A LMK and dlmk = sm_scale * A^T Q.  A workgroup owns TD_R consecutive rows
 // (queries x the heads that share the chunk keys) of one (batch, chunk-key head), scatters their
 // gradients into a dense bf16 tile of A in LDS (128 chunks at a time), and runs both products on
-// 16x16x32 MFMAs with the chunk keys and the query rows staged transposed beside it: no inverse
-// index, every input read once and coalesced.  dlmk tiles of the query blocks are added with
+// 16x16x32 MFMAs with the chunk keys and the query rows staged beside it, all row-major: what a product needs by
+// columns (A for A^T, chunk keys and query rows as right operands) comes by the transposing LDS load, in whose order of
+// rows the other operand is read too.  No inverse index, every input read once and coalesced.  (With A twice and keys
+// and rows feature-major, two-byte stores to a quarter of the banks were two thirds of the LDS time and 102 KiB allowed one
+// workgroup per compute unit; 71 KiB are two: B8 L8192 16 heads of 64, top-32: 294 -> 172 us.)  dlmk tiles of the query blocks are added with
 // float atomics (the summation order over query blocks is not fixed).  The chunk indices of one
 // row must be distinct (they are when they come from the selection).
 #define TD_R 128        // rows per workgroup
 #define TD_NC 128       // chunks per tile (== TD_R: one thread-to-piece split serves rows and chunk keys)
 #define TD_THREADS 512
-#define TD_STRIDE 136   // elements per LDS row: 128 + 8, so that 16-byte operand reads of 16 rows hit 64 banks
+#define TD_STRIDE 136   // elements per row of A: 128 + 8
 
 template <int D>
 __global__ void __launch_bounds__(TD_THREADS)
 topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q,
                       const bf16_t* __restrict__ lmks, const int32_t* __restrict__ indices,
                       bf16_t* __restrict__ dq, float* __restrict__ dlmk, int L, int N, int h_kv, int G,
-                      int topk, int per_qhead, float sm_scale) {
+                      int topk, int per_qhead, float sm_scale, uint32_t k_magic, int g_sh) {
   constexpr int DT = D / 16, PPR = D / 8;
+  constexpr int RS = D + 8;                   // elements per staged row
   extern __shared__ __align__(16) bf16_t td_sm[];
-  bf16_t* A_s = td_sm;                        // [TD_R][TD_STRIDE]   A, row-major
-  bf16_t* At_s = A_s + TD_R * TD_STRIDE;      // [TD_NC][TD_STRIDE]  A transposed
-  bf16_t* Lt_s = At_s + TD_NC * TD_STRIDE;    // [D][TD_STRIDE]      chunk keys of the tile, feature-major
-  bf16_t* Qt_s = Lt_s + D * TD_STRIDE;        // [D][TD_STRIDE]      query rows, feature-major
+  bf16_t* A_s = td_sm;                        // [TD_R][TD_STRIDE]
+  bf16_t* L_s = A_s + TD_R * TD_STRIDE;       // [TD_NC][RS]  chunk keys of the tile
+  bf16_t* Q_s = L_s + TD_NC * RS;             // [TD_R][RS]   query rows
   __shared__ int cmax_s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
@@ -3186,11 +3189,11 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   const long b = blockIdx.y;
   const int lmk_h = per_qhead ? h_kv * G : h_kv;
   const int hk = per_qhead ? lh / G : lh;
-  const int g_lo = per_qhead ? lh % G : 0, g_n = per_qhead ? 1 : G;
-  const int TQ = TD_R / g_n;
+  const int g_lo = per_qhead ? lh % G : 0, g_n = 1 << g_sh;  // (a divisor of TD_R)
+  const int TQ = TD_R >> g_sh;
   const int t0 = blockIdx.z * TQ;
   auto row_rg = [&](int row) -> long {  // row of gs / q / dq of a block row (valid rows only)
-    return ((b * L + t0 + row / g_n) * h_kv + hk) * (long)G + g_lo + row % g_n;
+    return ((b * L + t0 + (row >> g_sh)) * h_kv + hk) * (long)G + g_lo + (row & (g_n - 1));
   };
   if (tid == 0) cmax_s = -1;
   // Every global load of the first tile is issued before anything waits (clamped addresses, no
@@ -3204,17 +3207,17 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   for (int u = 0; u < NP; ++u) {
     const int i = tid + u * TD_THREADS;
     const int row = i / PPR, pc = i % PPR;     // the pieces of a row sit in neighbouring lanes
-    const int rc = (t0 + row / g_n < L) ? row : 0;  // row 0 of a block always exists
+    const int rc = (t0 + (row >> g_sh) < L) ? row : 0;  // row 0 of a block always exists
     qx[u] = *(const uint4*)(q + row_rg(rc) * D + pc * 8);
     const int cc = row < N ? row : N - 1;      // TD_NC == TD_R: the same split serves the chunk keys
     lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
   }
   auto item_load = [&](int i, int& c, bf16_t& val) {  // entry i of the block (any i: clamped)
     const int ic = i < n_item ? i : 0;
-    const int row = ic / topk, slot = ic - row * topk;
-    const bool ok = i < n_item && t0 + row / g_n < L;
+    const int row = (int)hils_udiv((uint32_t)ic, (uint32_t)topk, k_magic), slot = ic - row * topk;
+    const bool ok = i < n_item && t0 + (row >> g_sh) < L;
     const int rc = ok ? row : 0;
-    c = indices[((b * L + t0 + rc / g_n) * h_kv + hk) * (long)topk + slot];
+    c = indices[((b * L + t0 + (rc >> g_sh)) * h_kv + hk) * (long)topk + slot];
     val = gs[row_rg(rc) * topk + slot];
     if (!ok || c >= N) c = -1;
   };
@@ -3226,19 +3229,25 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   for (int u = 0; u < NP; ++u) {
     const int i = tid + u * TD_THREADS;
     const int row = i / PPR, pc = i % PPR;
-    const bool ok = t0 + row / g_n < L;
-    const bf16_t* xs = (const bf16_t*)&qx[u];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) Qt_s[(pc * 8 + e) * TD_STRIDE + row] = ok ? xs[e] : (bf16_t)0;
+    const bool ok = t0 + (row >> g_sh) < L;
+    *(uint4*)(Q_s + row * RS + pc * 8) = ok ? qx[u] : make_uint4(0, 0, 0, 0);
   }
+  // Operand of columns c0 .. c0 + 15 over the rows r0 .. r0 + 31: a lane's eight values are column c0 + col of the rows
+  // 4j .. 4j + 3 and 16 + 4j .. (transposing load: lane l of a 16-lane group addresses row l/4, columns 4*(l%4) .. +3)
+  typedef short td_s4 __attribute__((ext_vector_type(4)));
+  auto cols = [&](const bf16_t* base, int stride, int r0, int c0) __attribute__((always_inline)) -> uint4 {
+    const bf16_t* p = base + (r0 + 4 * j + (col >> 2)) * stride + c0 + 4 * (col & 3);
+    const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) td_s4*)p));
+    const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) td_s4*)(p + 16 * stride)));
+    return make_uint4(x.x, x.y, y.x, y.y);
+  };
   f32x4_t acc_q[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) acc_q[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   int cmax = 0;
   for (int c0 = 0; c0 <= cmax; c0 += TD_NC) {
-    // clear both copies of A (the rows of At beyond the tile's chunks stay zero)
-    for (int i = tid; i < (TD_R + TD_NC) * TD_STRIDE / 8; i += TD_THREADS) ((uint4*)A_s)[i] = make_uint4(0, 0, 0, 0);
-    // chunk keys of the tile, feature-major
+    for (int i = tid; i < TD_R * TD_STRIDE / 8; i += TD_THREADS) ((uint4*)A_s)[i] = make_uint4(0, 0, 0, 0);
+    // chunk keys of the tile
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
       const int i = tid + u * TD_THREADS;
@@ -3248,9 +3257,7 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
         lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
       }
       const bool ok = c0 + cl < N;
-      const bf16_t* xs = (const bf16_t*)&lx[u];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) Lt_s[(pc * 8 + e) * TD_STRIDE + cl] = ok ? xs[e] : (bf16_t)0;
+      *(uint4*)(L_s + cl * RS + pc * 8) = ok ? lx[u] : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
     int my_max = -1;
@@ -3264,9 +3271,8 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
         const int c = ci[u];
         my_max = c > my_max ? c : my_max;
         if (c >= c0 && c < c0 + TD_NC) {
-          const int row = (i0 + tid + u * TD_THREADS) / topk;
+          const int row = (int)hils_udiv((uint32_t)(i0 + tid + u * TD_THREADS), (uint32_t)topk, k_magic);
           A_s[row * TD_STRIDE + (c - c0)] = gv[u];
-          At_s[(c - c0) * TD_STRIDE + row] = gv[u];
         }
       }
     }
@@ -3284,10 +3290,12 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
       // dq rows of this wavefront's row tile += A LMK
 #pragma unroll
       for (int kc = 0; kc < TD_NC / 32; ++kc) {
-        const uint4 a = *(const uint4*)(A_s + (wave * 16 + col) * TD_STRIDE + kc * 32 + j * 8);
+        const bf16_t* ap = A_s + (wave * 16 + col) * TD_STRIDE + kc * 32 + 4 * j;
+        const uint2 a0 = *(const uint2*)ap, a1 = *(const uint2*)(ap + 16);
+        const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-          const uint4 bb = *(const uint4*)(Lt_s + (t * 16 + col) * TD_STRIDE + kc * 32 + j * 8);
+          const uint4 bb = cols(L_s, RS, kc * 32, t * 16);
           acc_q[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_q[t], 0, 0, 0);
         }
       }
@@ -3299,10 +3307,10 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
         for (int t = 0; t < DT; ++t) acc_l[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kr = 0; kr < TD_R / 32; ++kr) {
-          const uint4 a = *(const uint4*)(At_s + (wave * 16 + col) * TD_STRIDE + kr * 32 + j * 8);
+          const uint4 a = cols(A_s, TD_STRIDE, kr * 32, wave * 16);
 #pragma unroll
           for (int t = 0; t < DT; ++t) {
-            const uint4 bb = *(const uint4*)(Qt_s + (t * 16 + col) * TD_STRIDE + kr * 32 + j * 8);
+            const uint4 bb = cols(Q_s, RS, kr * 32, t * 16);
             acc_l[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_l[t], 0, 0, 0);
           }
         }
@@ -3325,7 +3333,7 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = wave * 16 + 4 * j + i;
-    if (t0 + row / g_n < L) {
+    if (t0 + (row >> g_sh) < L) {
       bf16_t* dst = dq + row_rg(row) * D + col;
 #pragma unroll
       for (int t = 0; t < DT; ++t) dst[t * 16] = f2bf(acc_q[t][i] * sm_scale);
@@ -3342,12 +3350,12 @@ template <int D>
 static int topk_bwd_dense_launch(dim3 grid, hipStream_t st, const bf16_t* gs, const bf16_t* q, const bf16_t* lmks,
                                  const int32_t* indices, bf16_t* dq, float* dlmk, int L, int N, int h_kv, int G,
                                  int topk, int per_qhead, float sm_scale) {
-  const size_t smem = (size_t)(TD_R + TD_NC + 2 * D) * TD_STRIDE * sizeof(bf16_t);
+  const size_t smem = ((size_t)TD_R * TD_STRIDE + (size_t)(TD_R + TD_NC) * (D + 8)) * sizeof(bf16_t);
   auto kern = topk_bwd_dense_kernel<D>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_topk_bwd")) return rc;
   hipLaunchKernelGGL(kern, grid, dim3(TD_THREADS), smem, st, gs, q, lmks, indices, dq, dlmk, L, N, h_kv, G, topk,
-                     per_qhead, sm_scale);
+                     per_qhead, sm_scale, hils_udiv_magic((uint32_t)topk), __builtin_ctz(per_qhead ? 1 : G));
   return HILS_OK;
 }
 
