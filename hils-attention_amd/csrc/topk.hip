@@ -40,8 +40,8 @@ __device__ __forceinline__ float key_score(uint32_t k) {
 // [lo, hi] and at least K lanes hold a non-zero x; the leading bits lo and hi share are
 // skipped.  Counting is one ballot + scalar popcount per bit.  Returns T with
 // count(x >= T) >= K and count(x > T) < K (T need not be one of the values when exactly K
-// values are >= T).
-__device__ __forceinline__ uint32_t lane_kth_largest(uint32_t x, uint32_t lo, uint32_t hi, int K) {
+// values are >= T).  slack: a T with up to that many values too many from it up will do.
+__device__ __forceinline__ uint32_t lane_kth_largest(uint32_t x, uint32_t lo, uint32_t hi, int K, int slack = 0) {
   const uint32_t diff = lo ^ hi;
   if (diff == 0u) return lo;
   const int top = 31 - __clz((int)diff);
@@ -56,7 +56,7 @@ __device__ __forceinline__ uint32_t lane_kth_largest(uint32_t x, uint32_t lo, ui
     if (n3 >= K) { T = c3; cnt = n3; }
     else if (n2 >= K) { T = c2; cnt = n2; }
     else if (n1 >= K) { T = c1; cnt = n1; }
-    if (cnt == K) return T;
+    if (cnt >= K && cnt - K <= slack) return T;
   }
   if (bit == 0) {
     const uint32_t c = T | 1u;
@@ -1394,7 +1394,6 @@ struct TopkRowSharedT {
   int win_i[TOPK_MAXK];                    // ... the winners' chunks, ascending, -1 padded
   bf16_t win_w[GM * (TOPK_MAXK + 1) + 2];   // ... and the heads' inter-chunk weights, [head][topk + 1]
   float swa[GM];               // ... and the heads' local-branch log-sum-exp
-  uint32_t thr;                // the candidate bound
   int next_group;
 };
 struct TopkWinners {
@@ -1464,6 +1463,30 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       for (int g = 0; g < GMAX; ++g) sh.swa[g] = swa[g];
     }
   }
+  // PRE: the wavefronts share out the heads' rows, four pieces a lane in flight at once (of up to NP / 4 a row), issued ahead
+  // of the bias staging (as atomic loads, which the compiler leaves where they are written: one by one in a loop, three or
+  // four latencies of memory were most of 2.7 us)
+  constexpr int PRE_N = 4, WPH = PRE ? NW / GMAX : 1;  // wavefronts of a head's row
+  const int pre_g = wave / WPH, pre_i = (wave % WPH) * 64 + lane, q4 = (lim + 3) / 4;
+  f32x4_t px[PRE_N];
+  float pm = 0.f, pl = 0.f;
+  auto pre_fetch = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PRE_N; ++u) {
+      const int i = i0 + u * 64 * WPH;
+      const unsigned long long* src = (const unsigned long long*)(pre_logits + (pre_g < G ? pre_g : G - 1) * NP + (i < q4 ? i : 0) * 4);
+      const unsigned long long lo = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const unsigned long long hi = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      px[u] = f32x4_t{__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
+                      __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32))};
+    }
+  };
+  if constexpr (PRE) {
+    const int n = ((lim + KG - 1) / KG) * GMAX, e = tid < n ? tid : 0;
+    pm = __hip_atomic_load(pre_m + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    pl = __hip_atomic_load(pre_l + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    pre_fetch(pre_i);
+  }
   if (bias) {
     // chunk c of this row: the G biases are contiguous in all three layouts
     for (int c = tid; c < NP; c += THREADS) {
@@ -1500,23 +1523,27 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   if constexpr (PRE) {
     if (inplace) __syncthreads();  // the bias is in the logits' places
     const int ngroups = (lim + KG - 1) / KG;
-    const int q4 = (lim + 3) / 4;
-    for (int i = tid; i < GMAX * q4; i += THREADS) {
-      const int g = i / q4, c = (i - g * q4) * 4;
-      f32x4_t x = {HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF};
-      if (g < G) {
-        x = *(const f32x4_t*)&pre_logits[g * NP + c];
-        if (inplace) {
-          const f32x4_t bb = *(const f32x4_t*)&bias_s[g * NP + c];
+    for (int i0 = pre_i; i0 < q4; i0 += PRE_N * 64 * WPH) {
+      if (i0 != pre_i) pre_fetch(i0);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = __fadd_rn(x[e], bb[e]);
+      for (int u = 0; u < PRE_N; ++u) {
+        const int c = (i0 + u * 64 * WPH) * 4;
+        if (c >= lim) break;
+        f32x4_t x = {HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF, HILS_NEG_INF};
+        if (pre_g < G) {
+          x = px[u];
+          if (inplace) {
+            const f32x4_t bb = *(const f32x4_t*)&bias_s[pre_g * NP + c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = __fadd_rn(x[e], bb[e]);
+          }
         }
+        *(f32x4_t*)&logit_s[pre_g * NP + c] = x;
       }
-      *(f32x4_t*)&logit_s[g * NP + c] = x;
     }
     for (int i = tid; i < ngroups * GMAX; i += THREADS) {
-      sh.grp_m[i / GMAX][i % GMAX] = pre_m[i];
-      sh.grp_l[i / GMAX][i % GMAX] = pre_l[i];
+      sh.grp_m[i / GMAX][i % GMAX] = i == tid ? pm : pre_m[i];
+      sh.grp_l[i / GMAX][i % GMAX] = i == tid ? pl : pre_l[i];
     }
   } else {
   // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
@@ -1689,6 +1716,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     // logaddexp on the hardware exp2/log2
     const float hi = fmaxf(sw, lse_hils), lo = fminf(sw, lse_hils);
     const float t = (lo == HILS_NEG_INF) ? hi : hi + __logf(1.f + __expf(lo - hi));
+    if (FUSED && wave == 0) sh.rank[lane] = 0;
     if (lane == 0) {
       sh.tot[g] = t;
       if (lse_total_out && write_out && g < G) lse_total_out[row * G + g] = t;
@@ -1697,7 +1725,10 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   __syncthreads();
   float tot[GMAX];
 #pragma unroll
-  for (int g = 0; g < GMAX; ++g) tot[g] = sh.tot[g];
+  for (int g = 0; g < GMAX; ++g) {
+    tot[g] = sh.tot[g];
+    if (tot[g] == HILS_NEG_INF) tot[g] = 0.f;  // (every logit is -inf and stays so: -inf - -inf would be a NaN)
+  }
   // ---- phase 3: selection.  Wavefront w owns the chunks [w*per, (w+1)*per); the selection key of a
   // chunk is max over the heads of (logit - lse_total) as an order-preserving integer ----
   const int per = ((N + NW - 1) / NW + 63) & ~63;  // <= 64 * EPT
@@ -1708,23 +1739,40 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   // per element; the logit rows of the heads past G hold -inf, so every head is read alike)
   auto form_keys = [&](auto with_bias) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      key[e] = 0u;
-      if (e * 64 < per) {  // uniform: the slots past the wavefront's share cost nothing
-        const int c = cbase + e * 64 + lane;
-        const bool mine = c < lim;
-        float best = HILS_NEG_INF;
+    for (int e = 0; e < EPT; ++e) key[e] = 0u;
+    // n slots from e0 on, their logits read together
+    auto batch = [&](auto n, const int e0) __attribute__((always_inline)) {
+      constexpr int EB = decltype(n)::value;
+      float xv[EB][GMAX];
+#pragma unroll
+      for (int u = 0; u < EB; ++u) {
+        int c = cbase + (e0 + u) * 64 + lane;
+        c = c < NP ? c : NP - 1;
 #pragma unroll
         for (int g = 0; g < GMAX; ++g) {
-          float xv = mine ? logit_s[g * NP + c] : HILS_NEG_INF;
-          if (decltype(with_bias)::value) xv = mine ? __fadd_rn(xv, bias_s[g * NP + c]) : xv;  // the sum the log-sum-exp saw
-          const float nrm = (xv == HILS_NEG_INF) ? HILS_NEG_INF : __fsub_rn(xv, tot[g]);
-          best = fmaxf(best, nrm);
+          xv[u][g] = logit_s[g * NP + c];
+          if (decltype(with_bias)::value) xv[u][g] = __fadd_rn(xv[u][g], bias_s[g * NP + c]);  // the sum the log-sum-exp saw
         }
-        if (mine) pooled[c] = best;
-        key[e] = score_key(best);
-        lmax = key[e] > lmax ? key[e] : lmax;
       }
+#pragma unroll
+      for (int u = 0; u < EB; ++u) {
+        const int c = cbase + (e0 + u) * 64 + lane;
+        const bool mine = c < lim && (e0 + u) * 64 < per;
+        float best = __fsub_rn(xv[u][0], tot[0]);
+#pragma unroll
+        for (int g = 1; g < GMAX; ++g) best = fmaxf(best, __fsub_rn(xv[u][g], tot[g]));
+        if (mine) pooled[c] = best;
+        key[e0 + u] = mine ? score_key(best) : 0u;
+        lmax = key[e0 + u] > lmax ? key[e0 + u] : lmax;
+      }
+    };
+    if (per == 64) {
+      batch(std::integral_constant<int, 1>{}, 0);
+    } else {
+      static_assert(EPT % 4 == 0, "slots come in batches of four");
+#pragma unroll
+      for (int e0 = 0; e0 < EPT; e0 += 4)
+        if (e0 * 64 < per) batch(std::integral_constant<int, 4>{}, e0);  // uniform: no cost past the wavefront's share
     }
   };
   if (bias && !inplace) form_keys(std::true_type{}); else form_keys(std::false_type{});
@@ -1757,32 +1805,44 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     }
   }
   __syncthreads();
-  if (wave == 0) {
-    uint32_t t = 1u;  // every valid key is >= 1
+  uint32_t thr = 1u;  // every valid key is >= 1.  (Found by every wavefront alike: a hand-over is a barrier more.)
+  {
     const uint32_t gv = sh.gmax[lane];
     if (__popcll(__ballot(gv != 0u)) >= topk) {
       const uint32_t hi = wave_max_u(gv);
       const uint32_t lo = ~wave_max_u(gv ? ~gv : 0u);  // smallest non-zero group maximum
-      t = lane_kth_largest(gv, lo, hi, topk);
+      thr = lane_kth_largest(gv, lo, hi, topk, topk / 16);  // (a bound: a group or two more are a few candidates more)
     }
-    if (lane == 0) sh.thr = t;
   }
-  __syncthreads();
   const unsigned long long lt = (1ull << lane) - 1ull;
-  const uint32_t thr = sh.thr;
   {
     int cnt = 0;
 #pragma unroll
     for (int e = 0; e < EPT; ++e)
-      if (e * 64 < per) cnt += __popcll(__ballot(key[e] >= thr));
+      if (e * 64 < per) {
+        const bool pred = key[e] >= thr;
+        const unsigned long long m = __ballot(pred);
+        if (FUSED && pred) {  // the wavefront's candidates in chunk order
+          const int o = cnt + __popcll(m & lt);
+          if (o < 64) {
+            sh.cand_s[wave][o] = __uint_as_float(key[e]);
+            sh.cand_i[wave][o] = cbase + e * 64 + lane;
+          }
+        }
+        cnt += __popcll(m);
+      }
     if (lane == 0) sh.wcnt[wave] = cnt;
-    if (FUSED && wave == 0) sh.rank[lane] = 0;
   }
   __syncthreads();
   int cand_base = 0, cand_total = 0;
+  int cand_w = 0, cand_o = lane;  // the candidate of this lane among all: of wavefront cand_w, number cand_o
 #pragma unroll
   for (int w2 = 0; w2 < NW; ++w2) {
     const int v = sh.wcnt[w2];
+    if (lane >= cand_total) {
+      cand_w = w2;
+      cand_o = lane - cand_total;
+    }
     cand_total += v;
     cand_base += (w2 < wave) ? v : 0;
   }
@@ -1806,6 +1866,35 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     __builtin_amdgcn_wave_barrier();
     *win = {widx, nc};
   };
+  if constexpr (FUSED) {
+    if (cand_total <= 64) {
+      // One candidate per lane, in chunk order: its rank among the candidates (keys descending, ties
+      // to the lower chunk) says whether it wins, the winners before it give its slot.  Every
+      // wavefront does this for itself; the 64 x 64 comparisons are shared out: wavefront w compares every candidate with
+      // candidates w * 64 / NW ..., the partial ranks meet in LDS (all of them in every wavefront: 1.8 against 0.7 us).
+      const uint32_t kc = lane < cand_total ? __float_as_uint(sh.cand_s[cand_w][cand_o]) : 0u;  // (valid keys are >= 1)
+      const int ci = lane < cand_total ? sh.cand_i[cand_w][cand_o] : -1;
+      constexpr int JW = 64 / NW;
+      int part = 0;
+#pragma unroll
+      for (int u = 0; u < JW; ++u) {
+        const int jj = wave * JW + u;
+        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)kc, jj);
+        part += ((kj > kc) | ((kj == kc) & (jj < lane))) ? 1 : 0;
+      }
+      if (part) atomicAdd(&sh.rank[lane], part);
+      lds_barrier();
+      const int rank = sh.rank[lane];
+      const bool win = lane < cand_total && rank < topk;
+      const unsigned long long wm = __ballot(win);
+      int* const list = sh.cand_i[wave];  // (the candidates are in registers everywhere)
+      if (win) list[__popcll(wm & lt)] = ci;
+      __builtin_amdgcn_wave_barrier();
+      const int nc = __popcll(wm);
+      fused_winners(lane < nc ? list[lane] : -1, nc);
+      return;
+    }
+  }
   if (cand_total <= TOPK_R_CAND) {
     uint32_t* ck = (uint32_t*)sh.merge_s;  // NW * TOPK_MAXK >= 512 entries
     int pos = cand_base;
@@ -1823,37 +1912,6 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       }
     }
     __syncthreads();
-    if constexpr (FUSED) {
-      if (cand_total <= 64) {
-        // One candidate per lane, in chunk order: its rank among the candidates (keys descending, ties
-        // to the lower chunk) says whether it wins, the winners before it give its slot.  Every
-        // wavefront does this for itself: no hand-over, no barrier before the attention's first loads.
-        // The 64 x 64 comparisons are shared out: wavefront w compares every candidate with candidates
-        // w * 64 / NW ..., the partial ranks meet in LDS.
-        const uint32_t kc = lane < cand_total ? ck[lane] : 0u;  // (valid keys are >= 1)
-        const int ci = lane < cand_total ? sh.merge_i[lane] : -1;
-        {
-          constexpr int JW = 64 / NW;
-          int part = 0;
-#pragma unroll
-          for (int u = 0; u < JW; ++u) {
-            const int jj = wave * JW + u;
-            const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)kc, jj);
-            part += ((kj > kc) | ((kj == kc) & (jj < lane))) ? 1 : 0;
-          }
-          if (part) atomicAdd(&sh.rank[lane], part);
-        }
-        lds_barrier();
-        const int rank = sh.rank[lane];
-        const bool win = lane < cand_total && rank < topk;
-        const unsigned long long wm = __ballot(win);
-        if (win) sh.cand_i[wave][__popcll(wm & lt)] = ci;
-        __builtin_amdgcn_wave_barrier();
-        const int nc = __popcll(wm);
-        fused_winners(lane < nc ? sh.cand_i[wave][lane] : -1, nc);
-        return;
-      }
-    }
     if (wave == 0) {
       // (the usual case, about 1.4 topk candidates, is one key per lane)
       const int nc = cand_total <= 64
