@@ -103,23 +103,23 @@ struct BwItems {
 // counts per thread and step.  The arrays are 16-byte aligned and padded to a multiple of four entries.
 __global__ void __launch_bounds__(1024)
 bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* __restrict__ cursor, int n, BwItems it) {
-  __shared__ int wsum[3][16];
-  __shared__ int carry_s[3];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ __align__(16) int wsum[3][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto parts = [&](int ns) -> int { return ns > 1 || it.n_range > 1 ? ns : 0; };
-  if (tid < 3) carry_s[tid] = 0;
-  __syncthreads();
+  int carry[3] = {0, 0, 0};  // pairs, items, partial results before this step's
+  int4 next = tid * 4 < n ? *(const int4*)&counts[tid * 4] : make_int4(0, 0, 0, 0);
   for (int base = 0; base < n; base += 4096) {
     const int i0 = base + tid * 4;  // (the arrays are padded to whole groups of four)
+    const int4 c4 = next;
+    if (i0 + 4096 < n) next = *(const int4*)&counts[i0 + 4096];
     int x[4] = {0, 0, 0, 0};
     if (i0 < n) {
-      const int4 c4 = *(const int4*)&counts[i0];
       x[0] = c4.x;
       x[1] = i0 + 1 < n ? c4.y : 0;
       x[2] = i0 + 2 < n ? c4.z : 0;
       x[3] = i0 + 3 < n ? c4.w : 0;
     }
-    int s[3] = {0, 0, 0};  // pairs, items, partial results
+    int s[3] = {0, 0, 0};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       s[0] += x[e];
@@ -129,28 +129,34 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
         s[2] += parts(ns);
       }
     }
-    int pos[3];
+    int pos[3], incl[3] = {s[0], s[1], s[2]};
 #pragma unroll
-    for (int e = 0; e < 3; ++e) {
-      int incl = s[e];
+    for (int o = 1; o < 64; o <<= 1) {
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += y;
+      for (int e = 0; e < 3; ++e) {
+        const int y = __shfl_up(incl[e], o, 64);
+        if (lane >= o) incl[e] += y;
       }
-      if (lane == 63) wsum[e][wave] = incl;
-      pos[e] = incl - s[e];
     }
-    __syncthreads();
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
-      pos[e] += carry_s[e];
-      for (int w = 0; w < wave; ++w) pos[e] += wsum[e][w];
+      if (lane == 63) wsum[e][wave] = incl[e];
+      pos[e] = carry[e] + incl[e] - s[e];
     }
     __syncthreads();
-    if (tid == 1023) {
+    // (all sums read at once and kept by every thread: two barriers a step; 18.8 -> 16.7 us for 16384 counts)
 #pragma unroll
-      for (int e = 0; e < 3; ++e) carry_s[e] = pos[e] + s[e];
+    for (int e = 0; e < 3; ++e) {
+#pragma unroll
+      for (int w = 0; w < 16; w += 4) {
+        const int4 y = *(const int4*)&wsum[e][w];
+        const int ys[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          pos[e] += w + u < wave ? ys[u] : 0;
+          carry[e] += ys[u];
+        }
+      }
     }
     if (i0 < n) {
       int4 o4, p4;
@@ -175,37 +181,106 @@ bw_scan_kernel(const int* __restrict__ counts, int* __restrict__ offsets, int* _
     __syncthreads();
   }
   if (tid == 0) {
-    offsets[n] = carry_s[0];
-    if (it.list) *it.total = carry_s[1];
+    offsets[n] = carry[0];
+    if (it.list) *it.total = carry[1];
   }
 }
 
-// pairs grouped by (b,h,c): a workgroup histograms its segment of queries in LDS, reserves one
-// range per chunk with a single global atomic, and scatters (t << 8 | slot) inside its ranges
-__global__ void __launch_bounds__(1024)
+// Pairs grouped by (b, h, c).  A workgroup reads its segment's entries once, at most BW_SCATTER / 1024 per thread, and
+// takes every entry's place among its chunk's with an LDS atomic; one global atomic per chunk reserves the range in the
+// chunk's list.  Written straight from there a wavefront's 64 entries go to 64 lines, and the L2's rate of requests
+// bounds the kernel (33.5 M pairs, B8 L8192 16 KV heads, top-32, 128 chunks: 153 us).  STAGE: the pairs are laid out
+// in LDS by chunk first and leave in runs.  With 8192 entries and 16 wavefronts 117 us; 101 with the workgroups of a
+// unit on one XCD, whose L2 then merges the runs' partial lines; 61 with 4096 entries and 8 wavefronts (four workgroups
+// on a compute unit, whose phases overlap; 71 with 2048 and 4).
+#define BW_SCATTER 4096  // entries per workgroup
+#define BW_SCATTER_NT 512
+template <bool STAGE>
+__global__ void __launch_bounds__(BW_SCATTER_NT)
 bw_scatter_kernel(const int32_t* __restrict__ indices, int* __restrict__ cursor,
-                  uint32_t* __restrict__ pairs, int L, int H, int K, int nchunk, int seg_len, int range, int n_range) {
-  extern __shared__ int pos[];  // nchunk: count -> next free position
-  const int h = blockIdx.y;
-  const long b = blockIdx.z;
-  const int t_lo = blockIdx.x * seg_len;
-  const int t_hi = (t_lo + seg_len < L) ? t_lo + seg_len : L;
+                  uint32_t* __restrict__ pairs, int L, int H, int K, int nchunk, int seg_len, int range, int n_range, int n_wg) {
+  constexpr int NT = BW_SCATTER_NT, E = BW_SCATTER / NT;
+  extern __shared__ __attribute__((aligned(16))) int bs_smem[];
+  int* hist = bs_smem;               // [nchunk] entries of a chunk; then where they go, less their place in LDS (STAGE)
+  int* first = hist + nchunk;        // [nchunk] a chunk's first place in LDS (STAGE)
+  int2* out = (int2*)(bs_smem + ((2 * nchunk + 3) & ~3));  // [entry] pair, where it goes (STAGE)
+  __shared__ int wsum[NT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wg = (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8);  // (an XCD takes whole units)
+  if (wg >= n_wg) return;
+  const int nseg = (L + seg_len - 1) / seg_len;
+  const int seg = wg % nseg, unit = wg / nseg;
+  const int h = unit % H;
+  const long b = unit / H;
+  const int t_lo = seg * seg_len;
+  const int rows = t_lo + seg_len < L ? seg_len : L - t_lo;
   int* cur = cursor + ((b * H + h) * n_range + t_lo / range) * (long)nchunk;
-  for (int i = threadIdx.x; i < nchunk; i += 1024) pos[i] = 0;
-  __syncthreads();
   const int32_t* seg0 = indices + ((b * L + t_lo) * H + h) * (long)K;
-  bw_walk_indices(seg0, t_lo, t_hi - t_lo, H, K, [&](int, int, int c) {
-    if (c >= 0 && c < nchunk) atomicAdd(&pos[c], 1);
-  });
-  __syncthreads();
-  for (int i = threadIdx.x; i < nchunk; i += 1024) {
-    const int cnt = pos[i];
-    pos[i] = cnt ? atomicAdd(&cur[i], cnt) : 0;
+  const long rstride = (long)H * K;
+  const int qK = NT / K, rK = NT % K;
+  int r = tid / K, sl = tid - r * K;
+  int cc[E], rank[E];
+  uint32_t pr[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const bool in = r < rows;
+    const int c = seg0[(long)(in ? r : rows - 1) * rstride + sl];
+    cc[u] = in && c >= 0 && c < nchunk ? c : -1;
+    pr[u] = ((uint32_t)(t_lo + r) << 8) | (uint32_t)sl;
+    sl += rK;
+    r += qK;
+    if (sl >= K) { sl -= K; ++r; }
   }
+  for (int i = tid; i < nchunk; i += NT) hist[i] = 0;
   __syncthreads();
-  bw_walk_indices(seg0, t_lo, t_hi - t_lo, H, K, [&](int t, int slot, int c) {
-    if (c >= 0 && c < nchunk) pairs[atomicAdd(&pos[c], 1)] = ((uint32_t)t << 8) | (uint32_t)slot;
-  });
+#pragma unroll
+  for (int u = 0; u < E; ++u)
+    if (cc[u] >= 0) rank[u] = atomicAdd(&hist[cc[u]], 1);
+  __syncthreads();
+  if constexpr (!STAGE) {
+    for (int i = tid; i < nchunk; i += NT) {
+      const int cnt = hist[i];
+      hist[i] = cnt ? atomicAdd(&cur[i], cnt) : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      if (cc[u] >= 0) pairs[hist[cc[u]] + rank[u]] = pr[u];
+    return;
+  }
+  int total = 0;
+  for (int base = 0; base < nchunk; base += NT) {
+    const int i = base + tid;
+    const int cnt = i < nchunk ? hist[i] : 0;
+    const int dst = cnt ? atomicAdd(&cur[i], cnt) : 0;
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int pos = total + incl - cnt;
+    for (int w = 0; w < NT / 64; ++w) {
+      const int x = wsum[w];
+      pos += w < wave ? x : 0;
+      total += x;
+    }
+    if (i < nchunk) {
+      first[i] = pos;
+      hist[i] = dst - pos;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < E; ++u)
+    if (cc[u] >= 0) {
+      const int pos = first[cc[u]] + rank[u];
+      out[pos] = make_int2((int)pr[u], hist[cc[u]] + pos);
+    }
+  __syncthreads();
+  for (int i = tid; i < total; i += NT) pairs[out[i].y] = (uint32_t)out[i].x;
 }
 
 // ---------------------------------------------------------------------------
@@ -1254,7 +1329,7 @@ static bool bq_stage_pays(long units, int L, int G, int D, int Dv, int K, int nc
 // Inverse index of an index tensor (B, L, H, K) with values in [0, nchunk) or < 0: counts,
 // offsets (cells + 1 ints, cells = B*H*nchunk), cursor (scratch) and the pairs (t << 8 | slot)
 // grouped by (b, h, chunk).  Also used by the top-k backward.
-static void bw_build_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
+static int bw_build_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
                            const BwItems& items, int B, int L, int H, int K, int nchunk, int range, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   const int n_range = (L + range - 1) / range;
@@ -1271,13 +1346,26 @@ static void bw_build_index(const int32_t* indices, int* counts, int* offsets, in
   dim3 gs((L + seg_len - 1) / seg_len, H, B);
   hipLaunchKernelGGL(bw_count_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, counts, L, H, K, nchunk, seg_len, range, n_range);
   hipLaunchKernelGGL(bw_scan_kernel, dim3(1), dim3(1024), 0, st, counts, offsets, cursor, (int)cells, items);
-  hipLaunchKernelGGL(bw_scatter_kernel, gs, dim3(1024), (size_t)nchunk * 4, st, indices, cursor, pairs, L, H, K, nchunk, seg_len, range, n_range);
+  // The scatter keeps a segment's entries in registers.  Staging them pays where a chunk has several of them and where
+  // there are many (direct / staged: 33.5 M pairs 153 / 61 us, 2 M 13.1 / 8.8, 128 K 4.6 / 5.5, 16 K 3.8 / 5.0).
+  while ((long)seg_len * K > BW_SCATTER && seg_len > 1) seg_len = (seg_len + 1) / 2;
+  const long n_wg = (long)B * H * ((L + seg_len - 1) / seg_len);
+  const dim3 gc((unsigned)((n_wg + 7) / 8 * 8));
+  const size_t staged = (size_t)((2 * nchunk + 3) & ~3) * 4 + (size_t)seg_len * K * sizeof(int2);
+  if ((long)B * L * H * K >= 1 << 19 && (long)seg_len * K >= 4L * nchunk && staged <= 80 * 1024) {
+    static HilsLdsReserve reserved;
+    if (int rc = hils_reserve_lds(&reserved, (const void*)bw_scatter_kernel<true>, staged, "hils_sparse_attn_bwd")) return rc;
+    hipLaunchKernelGGL(bw_scatter_kernel<true>, gc, dim3(BW_SCATTER_NT), staged, st, indices, cursor, pairs, L, H, K, nchunk, seg_len, range, n_range, (int)n_wg);
+  } else {
+    hipLaunchKernelGGL(bw_scatter_kernel<false>, gc, dim3(BW_SCATTER_NT), (size_t)nchunk * 4, st, indices, cursor, pairs, L, H, K, nchunk, seg_len, range, n_range, (int)n_wg);
+  }
+  return HILS_OK;
 }
 
-void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
-                            int B, int L, int H, int K, int nchunk, void* stream) {
-  bw_build_index(indices, counts, offsets, cursor, pairs, BwItems{nullptr, nullptr, nullptr, 0, 1}, B, L, H, K, nchunk,
-                 L, stream);
+int hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
+                           int B, int L, int H, int K, int nchunk, void* stream) {
+  return bw_build_index(indices, counts, offsets, cursor, pairs, BwItems{nullptr, nullptr, nullptr, 0, 1}, B, L, H, K,
+                        nchunk, L, stream);
 }
 
 // Whole backward on the MFMA kernels: dq (bf16, written), dw (fp32, written at the valid slots),
@@ -1338,7 +1426,7 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   }
   // ---- inverse index, then dK, dV
   const BwItems items{(int2*)(ws + lo.items), (int*)(ws + lo.n_items), (int*)(ws + lo.part_off), lo.seg_pairs, lo.n_range};
-  bw_build_index(indices, counts, offsets, cursor, pairs, items, B, L, H, K, nchunk, lo.range, stream);
+  if (int rc = bw_build_index(indices, counts, offsets, cursor, pairs, items, B, L, H, K, nchunk, lo.range, stream)) return rc;
   BwDims dm{L, Lkv, HQ, H, K, NW, nchunk, mask_last, sm_scale, kv16, B, slope, items, (float*)(ws + lo.part)};
   if (kv16 && Lkv > nchunk * BW_S) {  // tokens behind the last whole chunk are never attended
     for (int b2 = 0; b2 < B; ++b2) {

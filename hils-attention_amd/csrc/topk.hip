@@ -3417,8 +3417,8 @@ static int topk_bwd_dense_launch(dim3 grid, hipStream_t st, const bf16_t* gs, co
   return HILS_OK;
 }
 
-void hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
-                            int B, int L, int H, int K, int nchunk, void* stream);
+int hils_build_chunk_index(const int32_t* indices, int* counts, int* offsets, int* cursor, uint32_t* pairs,
+                           int B, int L, int H, int K, int nchunk, void* stream);
 
 static size_t topk_bwd_round(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -3469,7 +3469,7 @@ extern "C" int hils_topk_bwd(const void* g_scores, const void* q, const void* lm
     hipLaunchKernelGGL(topk_bwd_dq_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st,
                        (const bf16_t*)g_scores, (const bf16_t*)lmks, indices, (bf16_t*)dq, rows_g, L, N, h_kv,
                        G, D, topk, per_qhead, sm_scale);
-    hils_build_chunk_index(indices, counts, offsets, cursor, pairs, B, L, h_kv, topk, N, stream);
+    if (int rc = hils_build_chunk_index(indices, counts, offsets, cursor, pairs, B, L, h_kv, topk, N, stream)) return rc;
     const int lmk_h = per_qhead ? h_kv * G : h_kv;
     hipLaunchKernelGGL(topk_bwd_dlmk_kernel, dim3(N, lmk_h, B), dim3(256), 0, st, (const bf16_t*)g_scores,
                        (const bf16_t*)q, offsets, pairs, dlmk, L, N, h_kv, G, D, topk, per_qhead, sm_scale);

@@ -90,6 +90,37 @@ def test_sparse_attn_backward_ranges(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mas
     test_sparse_attn_backward(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mask_last)
 
 
+# the inverse index itself, out of the workspace of a score gather that uses it (G = 3), against a sort: pairs placed
+# directly (few, or too few of a chunk per workgroup) and by way of LDS, ragged last segments, more chunks than threads
+@pytest.mark.parametrize("B,L,N,H,K,hole", [(1, 77, 5, 2, 3, 0.3), (2, 300, 64, 1, 200, 0.5), (1, 2100, 12288, 1, 256, 0.),
+                                            (1, 8195, 1024, 1, 64, 0.2), (3, 5003, 130, 2, 37, 0.), (1, 2049, 7, 1, 256, 0.99)])
+def test_inverse_index(dev, B, L, N, H, K, hole):
+    from hils_attention_amd.ops import _cabi
+    lib, G, D = _cabi.load(), 3, 8
+    gen = torch.Generator(device=dev).manual_seed(L)
+    idx = torch.randint(0, N, (B, L, H, K), device=dev, generator=gen, dtype=torch.int32)
+    idx.masked_fill_(torch.rand(B, L, H, K, device=dev, generator=gen) < hole, -1)
+    size = lib.hils_topk_bwd_workspace(B, L, N, H, G, D, K)
+    ws = torch.empty(size, dtype=torch.uint8, device=dev)
+    g, q, lmks = (torch.zeros(*s, dtype=torch.bfloat16, device=dev) for s in ((B, L, H, G, K), (B, L, H, G, D), (B, N, H, D)))
+    dq, dlmk = torch.empty_like(q), torch.zeros(B, N, H, D, device=dev)
+    rc = lib.hils_topk_bwd(_cabi.ptr(g), _cabi.ptr(q), _cabi.ptr(lmks), _cabi.ptr(idx), _cabi.ptr(dq), _cabi.ptr(dlmk),
+                           _cabi.ptr(ws), size, B, L, N, H, G, D, K, 0, 1.0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    cells = B * H * N
+    part = ((cells + 1) * 4 + 255) // 256 * 256
+    offsets = ws[part:part + (cells + 1) * 4].view(torch.int32).long()
+    pairs = ws[3 * part:3 * part + idx.numel() * 4].view(torch.int32).long()
+    b, t, h, s = torch.meshgrid(*(torch.arange(n, device=dev) for n in (B, L, H, K)), indexing="ij")
+    ok = idx >= 0
+    cell = ((b * H + h) * N + idx)[ok]
+    ref = (cell * (1 << 32) + (t * 256 + s)[ok]).sort().values
+    count = torch.bincount(cell, minlength=cells)
+    assert torch.equal(offsets, torch.nn.functional.pad(count.cumsum(0), (1, 0)))
+    got = torch.repeat_interleave(torch.arange(cells, device=dev), count) * (1 << 32) + pairs[:cell.numel()]
+    assert torch.equal(got.sort().values, ref)
+
+
 @pytest.mark.parametrize("B,L,HQ,H,D,W", [(1, 700, 8, 1, 64, 512), (2, 1024, 16, 2, 64, 512), (1, 513, 4, 1, 128, 300),
                                           (1, 2000, 4, 4, 64, 512)])
 def test_swa_backward_split(pkg, dev, B, L, HQ, H, D, W):
