@@ -1161,8 +1161,8 @@ bool hils_bw_covers(int L, int Lkv, int HQ, int H, int D, int Dv, int K, int S, 
          Lkv >= S && K <= 256 && L < (1 << 24) && Lkv / S <= 12288;
 }
 
-void hils_ga_pack_launch(const void* a, const void* b, void* ap, void* bp, float* bmax, int B, int Lkv,
-                         int H, int Da, int Db, void* stream);
+void hils_bw_pack_launch(const void* k, const void* v, bf16_t* ka, bf16_t* va, bf16_t* kt, float* kmax, float* vmax,
+                         int B, int Lkv, int H, int D, int Dv, void* stream);
 
 // T queries per workgroup of the dQ kernel such that the fixed-point tile, the chunk histogram
 // and the pair list (and, with `stage`, the block's own query and dO rows) fit in LDS; 0 when the
@@ -1391,9 +1391,7 @@ int hils_bw_run(const void* q, const void* k, const void* v, const void* weights
   if (H > 65535 || B > 65535 || (size_t)B * H * nchunk * lo.n_range > (1u << 30)) return -1;
   // (24-bit row strides and 32-bit offsets inside a block of up to 256 queries)
   if ((long)HQ * (D > Dv ? D : Dv) >= (1 << 23) || (long)HQ * NW >= (1 << 22) || (long)HQ * K >= (1 << 22)) return -1;
-  // ---- operand packing: K as A operand (+ max|V|), V as A operand + K transposed (+ max|K|)
-  hils_ga_pack_launch(k, v, ka, nullptr, vmax, B, Lkv, H, D, Dv, stream);
-  hils_ga_pack_launch(v, k, va, kt, kmax, B, Lkv, H, Dv, D, stream);
+  hils_bw_pack_launch(k, v, ka, va, kt, kmax, vmax, B, Lkv, H, D, Dv, stream);  // operands of the dQ kernel
   // ---- dQ, dW
   {
     size_t smem;

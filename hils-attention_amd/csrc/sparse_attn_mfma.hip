@@ -39,65 +39,112 @@
 // P supplies tokens when it is fed back as the A operand of O = P V.
 // Also records max|V| of every chunk (it bounds the fixed-point output accumulation), NaNs left out,
 // with the sign bit set when the chunk holds a NaN or an infinity.
+// BWD: what the backward's dQ kernel needs, in one pass over K and V: kp, vp in the order of kp, kt = K
+// in the order that vp has otherwise, and both maxima.
+//
+// Memory-bound.  Every 16-byte piece of the chunk is loaded once, all of a thread's before any is used, in
+// the order of kp; the transposed matrix goes by way of row-major rows in LDS and the transposing load.
+// B8 L8192 16 heads of 64: 89 us (6.0 TB/s; the chunks' bytes one by one through LDS: 90), the backward's arrays
+// 123 us (two passes of 90); B1 L2048 2 heads 5.1 -> 3.7 us.
 // ---------------------------------------------------------------------------
+template <int D, int DV, bool BWD>
 __global__ void __launch_bounds__(256)
 pack_kv_kernel(const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, bf16_t* __restrict__ kp,
-               bf16_t* __restrict__ vp, float* __restrict__ vmax, int Lkv, int H, int D, int Dv,
-               int nchunk) {
-  extern __shared__ bf16_t tile[];  // 64 x (max(D, Dv) + 2)
-  __shared__ float red[32];
+               bf16_t* __restrict__ vp, bf16_t* __restrict__ kt, float* __restrict__ kmax, float* __restrict__ vmax,
+               int Lkv, int H, int nchunk) {
+  typedef short pk_s4 __attribute__((ext_vector_type(4)));
+  typedef short pk_s8 __attribute__((ext_vector_type(8)));
+  constexpr int DT = BWD ? D : DV, PITCH = DT * 2 + 16;  // the transposed matrix
+  constexpr int NK = D / 32, NV = DV / 32;               // pieces of a thread
+  __shared__ __align__(16) unsigned char tile[GA_S * PITCH];
+  __shared__ uint32_t red[2][4];  // largest magnitude, bit 31: not all numbers
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, j = lane >> 4;
   const int c = blockIdx.x, h = blockIdx.y;
   const long b = blockIdx.z;
   const long chunk = (b * H + h) * (long)nchunk + c;
-  // ---- K: rows are already contiguous along d; only the order of 16-byte pieces changes
-  {
-    const int pieces = D / 8;  // 16-byte pieces per token row
-    bf16_t* out = kp + chunk * (long)GA_S * D;
-    for (int i = threadIdx.x; i < GA_S * pieces; i += 256) {
-      // destination order: ((mt * KS + ks) * 64 + lane)
-      const int lane = i & 63, blk = i >> 6;
-      const int KS = D / 32;
-      const int mt = blk / KS, ks = blk - mt * KS;
-      const int tok = mt * 16 + (lane & 15), d = ks * 32 + (lane >> 4) * 8;
-      const uint4 x = *(const uint4*)(k + ((b * Lkv + (long)c * GA_S + tok) * H + h) * D + d);
-      *(uint4*)(out + (long)i * 8) = x;
-    }
-  }
-  // ---- V: transposed through LDS
-  const int DP = Dv + 2;
-  const int d8n = Dv / 8;
-  uint32_t mx = 0;  // bf16 bits: the order of the magnitudes
-  int odd = 0;
-  for (int i = threadIdx.x; i < GA_S * d8n; i += 256) {
-    const int s = i / d8n, d8 = i - s * d8n;
-    uint4 x = *(const uint4*)(v + ((b * Lkv + (long)c * GA_S + s) * H + h) * Dv + d8 * 8);
-    const bf16_t* xs = (const bf16_t*)&x;
+  const long row0 = (b * Lkv + (long)c * GA_S) * H + h;
+  // (piece i of a matrix: ((mt * KS + ks) * 64 + lane), a wavefront's u-th at i = u * 256 + tid)
+  uint4 kx[NK], vx[NV];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      tile[s * DP + d8 * 8 + e] = xs[e];
-      const uint32_t mag = xs[e] & 0x7fffu;
-      if (mag >= 0x7f80u) odd = 1;
-      if (mag <= 0x7f80u && mag > mx) mx = mag;
-    }
+  for (int u = 0; u < NK; ++u) {
+    const int blk = u * 4 + wave;
+    kx[u] = *(const uint4*)(k + (row0 + (long)(blk / (D / 32) * 16 + col) * H) * D + blk % (D / 32) * 32 + j * 8);
   }
-  odd = __syncthreads_or(odd);  // (the barrier orders the tile writes)
-  const float top = block_max(__uint_as_float(mx << 16), red);
-  if (threadIdx.x == 0) vmax[chunk] = odd ? -top : top;
-  if (!vp) return;  // only max|V| wanted
-  bf16_t* out = vp + chunk * (long)GA_S * Dv;
-  for (int i = threadIdx.x; i < Dv * 8; i += 256) {
-    // destination order: ((dt * 2 + s) * 64 + lane)
-    const int lane = i & 63, blk = i >> 6;
-    const int dt = blk >> 1, s = blk & 1;
-    const int dv = dt * 16 + (lane & 15), j = lane >> 4;
-    bf16_t y[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int tok = 32 * s + 16 * (e >> 2) + 4 * j + (e & 3);
-      y[e] = tile[tok * DP + dv];
-    }
-    *(uint4*)(out + (long)i * 8) = *(uint4*)y;
+  for (int u = 0; u < NV; ++u) {
+    const int blk = u * 4 + wave;
+    vx[u] = *(const uint4*)(v + (row0 + (long)(blk / (DV / 32) * 16 + col) * H) * DV + blk % (DV / 32) * 32 + j * 8);
   }
+  const auto& tx = [&]() -> const auto& { if constexpr (BWD) return kx; else return vx; }();
+#pragma unroll
+  for (int u = 0; u < DT / 32; ++u) {
+    const int blk = u * 4 + wave;
+    *(uint4*)(tile + (blk / (DT / 32) * 16 + col) * PITCH + blk % (DT / 32) * 64 + j * 16) = tx[u];
+  }
+#pragma unroll
+  for (int u = 0; u < NK; ++u) *(uint4*)(kp + chunk * (long)GA_S * D + (long)(u * 256 + tid) * 8) = kx[u];
+  if constexpr (BWD) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) *(uint4*)(vp + chunk * (long)GA_S * DV + (long)(u * 256 + tid) * 8) = vx[u];
+  }
+  // ---- maxima (bf16 bits: the order of the magnitudes)
+  auto largest = [&](const auto& x, int m) {
+    uint32_t mx = 0, odd = 0;
+    for (const uint4& y : x) {
+      const uint32_t w[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t mag = (e & 1 ? w[e / 2] >> 16 : w[e / 2]) & 0x7fffu;
+        odd |= mag >= 0x7f80u;
+        mx = mag <= 0x7f80u && mag > mx ? mag : mx;
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t y = __shfl_xor((int)mx, o, 64);
+      mx = y > mx ? y : mx;
+    }
+    const bool any = __ballot(odd != 0) != 0;
+    if (lane == 0) red[m][wave] = mx | (any ? 0x80000000u : 0u);
+  };
+  largest(vx, 0);
+  if constexpr (BWD) largest(kx, 1);
+  __syncthreads();
+  if (tid < (BWD ? 2 : 1)) {
+    uint32_t mx = 0, odd = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t x = red[tid][w], m = x & 0x7fffffffu;
+      odd |= x & 0x80000000u;
+      mx = m > mx ? m : mx;
+    }
+    const float top = __uint_as_float(mx << 16);
+    (tid ? kmax : vmax)[chunk] = odd ? -top : top;
+  }
+  // ---- transposed: piece ((dt * 2 + s) * 64 + lane)
+  bf16_t* out = (BWD ? kt : vp) + chunk * (long)GA_S * DT;
+#pragma unroll
+  for (int u = 0; u < DT / 32; ++u) {
+    const int blk = u * 4 + wave, dt = blk >> 1, s = blk & 1;
+    const unsigned char* p = tile + (32 * s + 4 * j + (col >> 2)) * PITCH + (col & 3) * 8 + dt * 32;
+    const pk_s4 y0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pk_s4*)p);
+    const pk_s4 y1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pk_s4*)(p + 16 * PITCH));
+    *(uint4*)(out + (long)(u * 256 + tid) * 8) = __builtin_bit_cast(uint4, (pk_s8)__builtin_shufflevector(y0, y1, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+}
+
+template <bool BWD>
+static void pack_kv_launch(const void* k, const void* v, bf16_t* kp, bf16_t* vp, bf16_t* kt, float* kmax, float* vmax,
+                           int B, int Lkv, int H, int D, int Dv, hipStream_t st) {
+  const int nchunk = Lkv / GA_S;
+#define PACK(D_, DV_)                                                                                              \
+  hipLaunchKernelGGL((pack_kv_kernel<D_, DV_, BWD>), dim3(nchunk, H, B), dim3(256), 0, st, (const bf16_t*)k,       \
+                     (const bf16_t*)v, kp, vp, kt, kmax, vmax, Lkv, H, nchunk)
+  if (D == 64 && Dv == 64) PACK(64, 64);
+  else if (D == 64) PACK(64, 128);
+  else if (Dv == 64) PACK(128, 64);
+  else PACK(128, 128);
+#undef PACK
 }
 
 // Fixed point by accumulator bias: a product accumulated onto GA_FX_BIAS = 1.5 * 2^23 comes out
@@ -886,12 +933,7 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
   bf16_t* kpk = (bf16_t*)((char*)workspace + ga_vt_bytes(B, H, nchunk, Dv));
   float* vmax = (float*)((char*)kpk + ga_vt_bytes(B, H, nchunk, D));
   bf16_t* qpk = (bf16_t*)((char*)vmax + ga_vmax_bytes(B, H, nchunk));
-  if (!workspace_ready) {
-    const int dmax = D > Dv ? D : Dv;
-    hipLaunchKernelGGL(pack_kv_kernel, dim3(nchunk, H, B), dim3(256),
-                       (size_t)GA_S * (dmax + 2) * sizeof(bf16_t), st, (const bf16_t*)k,
-                       (const bf16_t*)v, kpk, vpk, vmax, Lkv, H, D, Dv, nchunk);
-  }
+  if (!workspace_ready) pack_kv_launch<false>(k, v, kpk, vpk, nullptr, nullptr, vmax, B, Lkv, H, D, Dv, st);
   GaDims dm{L, Lkv, HQ, H, B, K, NW, T, nblk, nchunk, mask_last, sm_scale, q_block, WH, sm_n, merge_col,
             hils_udiv_magic((uint32_t)K), hils_udiv_magic((uint32_t)q_block)};
   const long per_xcd = (total + 7) / 8;
@@ -910,15 +952,10 @@ int hils_sparse_attn_fwd_mfma(const void* q, const void* k, const void* v, const
   return HILS_OK;
 }
 
-// Launches the packing kernel on explicit buffers: ap = a in A-operand order, bp = b in the
-// transposed B-operand order, bmax = max|b| per chunk (also used by the backward kernels).
-void hils_ga_pack_launch(const void* a, const void* b, void* ap, void* bp, float* bmax, int B, int Lkv,
-                         int H, int Da, int Db, void* stream) {
-  const int nchunk = Lkv / GA_S;
-  const int dmax = Da > Db ? Da : Db;
-  hipLaunchKernelGGL(pack_kv_kernel, dim3(nchunk, H, B), dim3(256),
-                     (size_t)GA_S * (dmax + 2) * sizeof(bf16_t), (hipStream_t)stream, (const bf16_t*)a,
-                     (const bf16_t*)b, (bf16_t*)ap, (bf16_t*)bp, bmax, Lkv, H, Da, Db, nchunk);
+// The operands of the backward's dQ kernel.
+void hils_bw_pack_launch(const void* k, const void* v, bf16_t* ka, bf16_t* va, bf16_t* kt, float* kmax, float* vmax,
+                         int B, int Lkv, int H, int D, int Dv, void* stream) {
+  pack_kv_launch<true>(k, v, ka, va, kt, kmax, vmax, B, Lkv, H, D, Dv, (hipStream_t)stream);
 }
 
 extern "C" int hils_pack_kv_chunks(const void* k, const void* v, void* workspace, size_t workspace_bytes,
@@ -937,10 +974,7 @@ extern "C" int hils_pack_kv_chunks(const void* k, const void* v, void* workspace
   bf16_t* vpk = (bf16_t*)workspace;
   bf16_t* kpk = (bf16_t*)((char*)workspace + ga_vt_bytes(B, H, nchunk, Dv));
   float* vmax = (float*)((char*)kpk + ga_vt_bytes(B, H, nchunk, D));
-  const int dmax = D > Dv ? D : Dv;
-  hipLaunchKernelGGL(pack_kv_kernel, dim3(nchunk, H, B), dim3(256),
-                     (size_t)GA_S * (dmax + 2) * sizeof(bf16_t), (hipStream_t)stream,
-                     (const bf16_t*)k, (const bf16_t*)v, kpk, vpk, vmax, Lkv, H, D, Dv, nchunk);
+  pack_kv_launch<false>(k, v, kpk, vpk, nullptr, nullptr, vmax, B, Lkv, H, D, Dv, (hipStream_t)stream);
   HILS_CHECK_LAUNCH("hils_pack_kv_chunks");
   return HILS_OK;
 }

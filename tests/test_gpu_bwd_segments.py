@@ -94,7 +94,7 @@ def test_sparse_attn_backward_ranges(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mas
 # directly (few, or too few of a chunk per workgroup) and by way of LDS, ragged last segments, more chunks than threads
 @pytest.mark.parametrize("B,L,N,H,K,hole", [(1, 77, 5, 2, 3, 0.3), (2, 300, 64, 1, 200, 0.5), (1, 2100, 12288, 1, 256, 0.),
                                             (1, 8195, 1024, 1, 64, 0.2), (3, 5003, 130, 2, 37, 0.), (1, 2049, 7, 1, 256, 0.99)])
-def test_inverse_index(dev, B, L, N, H, K, hole):
+def test_inverse_index(pkg, dev, B, L, N, H, K, hole):
     from hils_attention_amd.ops import _cabi
     lib, G, D = _cabi.load(), 3, 8
     gen = torch.Generator(device=dev).manual_seed(L)
