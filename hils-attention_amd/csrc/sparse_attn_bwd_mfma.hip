@@ -1218,18 +1218,31 @@ struct BwLayout {
   int seg_pairs, range, n_range;
   size_t max_items;
 };
-// Queries per range of the dK/dV kernel: the gathered rows of a unit should stay in an XCD's L2 (4 MiB, and the
-// workgroups of one range overlap with those of the next).  Where a unit's rows are more than 3 MiB the items go range
-// by range of 2 MiB, at the price of a partial result per (range, chunk).  B2 L8192 32/4 heads of 64, dK/dV + sum:
-// 942 us in one range, 857 in ranges of 1 MiB, 806 of 2, 912 of 3, 914 of 4; B1 L8192 32/8 of 128: 980, 1016, 960, 1040, 1039.
-static int bw_range(int L, int G, int D, int Dv) {
+// Queries per range of the dK/dV kernel: the gathered rows of a unit (batch, KV head) should stay in an XCD's L2 (4 MiB,
+// and the workgroups of one range overlap with those of the next).  Where a unit's rows are more than 3 MiB the items go
+// range by range of 2 MiB, at the price of a partial result of 64 (D + Dv) floats per (range, chunk): as many bytes,
+// written and read, as the gathers of 256 rows, and ranges times chunks grow with the square of the length.  Hence only
+// where such a cell has 1024 rows on average (a causal call reaches about half of the cells) and the partial results stay
+// within 1 GiB; with fewer than eight units the XCDs share a unit's items, whose rows are unequal (the first ranges have
+// few chunks and full cells), and it takes 2048.  Rows of one or two heads are bound by requests and gain nothing.
+// Whole backward, us, one range / ranges of 2 MiB (in brackets, rows of a cell): top-32, B2 L8192 32/4 heads of 64 [2048]
+// 1583 / 1449, B1 L8192 32/8 of 128 [1024] 1800 / 1759, B2 L8192 16/4 of 128 [1024] 1783 / 1757, B1 L16384 32/8 of 128
+// [512] 3757 / 3984, L32768 [256] 9314 / 10019; few units: B1 L8192 16/2 of 64 [2048] 526 / 497, B1 L8192 32/4 of 128
+// [1024] 1820 / 1908 (the rule costs here: B1 L16384 32/4 of 64 [1024] 1974 / 1859); top-8: B2 L8192 32/4 of 64 [512] 621 / 649, B1 L8192 32/8 of 128 [256] 726 / 790, B1 L16384 16/2 of 64
+// [256] 396 / 481; one or two heads: B2 L16384 16/16 of 64 [1024] 1863 / 2056, B8 L8192 32/16 of 64 [2048] 5570 / 5965.
+// Ranges of other lengths, dK/dV + sum, B2 L8192 32/4 of 64: 857 in ranges of 1 MiB, 806 of 2, 912 of 3, 914 of 4.
+static int bw_range(size_t units, int L, int nchunk, int G, int D, int Dv, int K) {
   const size_t row = (size_t)G * (D + Dv) * 2;
-  if ((size_t)L * row <= ((size_t)3 << 20)) return L;
-  const int r = (int)(((size_t)2 << 20) / row) & ~255;
-  return r > 256 ? r : 256;
+  if (G < 4 || (size_t)L * row <= ((size_t)3 << 20)) return L;
+  int r = (int)(((size_t)2 << 20) / row) & ~255;
+  r = r > 256 ? r : 256;
+  const size_t rows = (size_t)r * K * G / nchunk;  // of a cell
+  const size_t parts = units * nchunk * ((L + r - 1) / r) * (BW_S * (size_t)(D + Dv) * 4);
+  return rows >= (units >= 8 ? 1024u : 2048u) && parts <= ((size_t)1 << 30) ? r : L;
 }
 // Pairs per work item of the dK/dV kernel: about 2048 items of equal size in all (some four rounds of the
-// workgroups that fit the chip), but no less than 512 rows, whose gathers are four times the partial result's bytes.
+// workgroups that fit the chip), but no less than 512 rows (a cell may have fewer), whose gathers are four times the
+// partial result's bytes.
 static BwLayout bw_layout(int B, int L, int Lkv, int G, int H, int D, int Dv, int K) {
   const size_t chunks = (size_t)B * H * (Lkv / BW_S);
   const size_t pairs = (size_t)B * L * H * K;
@@ -1237,7 +1250,7 @@ static BwLayout bw_layout(int B, int L, int Lkv, int G, int H, int D, int Dv, in
   const size_t least = G < 8 ? 512 / G : 64;
   seg = ((seg > least ? seg : least) + 63) & ~(size_t)63;
   BwLayout lo;
-  lo.range = bw_range(L, G, D, Dv);
+  lo.range = bw_range((size_t)B * H, L, Lkv / BW_S, G, D, Dv, K);
   lo.n_range = (L + lo.range - 1) / lo.range;
   const size_t cells = chunks * lo.n_range;
   size_t o = 0;

@@ -219,8 +219,9 @@ int hils_pack_kv_chunks(const void* k, const void* v, void* workspace, size_t wo
  * atomics when q_block > 1 or WH != HQ, written otherwise: caller zero-fills).
  * workspace: device scratch of hils_sparse_attn_bwd_workspace(...) bytes (0 = shape not covered)
  * for the MFMA kernels: an inverse index (pairs of (query, slot) grouped by chunk) is built there
- * and dK, dV are then computed chunk-major without atomics.  NULL selects the shape-generic
- * kernel for everything.
+ * and dK, dV are then computed chunk-major without atomics, with fp32 partial results in the workspace
+ * where a chunk's pairs are shared between workgroups (its size is linear in L; at most 1 GiB of it is
+ * partial results of ranges of queries).  NULL selects the shape-generic kernel for everything.
  * swa_o / d_swa_o / merge_col: when the forward merged the local branch (swa_o given there), pass
  * the same swa_o and merge_col: d_swa_o (B,L,HQ,Dv) bf16 = d_o * weights[..., merge_col] is written
  * and dw[..., merge_col] = <d_o, swa_o> (q_block = 1, WH = HQ only).  NULL otherwise. */

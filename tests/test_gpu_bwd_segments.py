@@ -82,10 +82,12 @@ def test_sparse_attn_backward_many_blocks(pkg, dev, B, L, HQ, H, K, mask_last):
     test_sparse_attn_backward(pkg, dev, B, L, HQ, H, 64, 64, K, False, mask_last)
 
 
-# rows of more than 3 MiB per (batch, KV head): the items go by ranges of queries (the last one ragged), every chunk is
-# a sum of partial results, and the chunk nobody can see has none
+# rows of more than 3 MiB per (batch, KV head): where a range's cells have rows enough (1024 on average with eight units and
+# more, 2048 with fewer: all but the first two) the items go by ranges of queries (the last one ragged), every chunk is a
+# sum of partial results, and the chunk nobody can see has none
 @pytest.mark.parametrize("B,L,HQ,H,D,Dv,K,crowd,mask_last", [
-    (1, 2111, 16, 2, 64, 128, 6, False, True), (1, 1601, 8, 1, 128, 128, 5, True, False), (2, 1600, 16, 1, 64, 64, 8, True, True)])
+    (1, 2111, 16, 2, 64, 128, 6, False, True), (1, 1601, 8, 1, 128, 128, 5, True, False), (2, 1600, 16, 1, 64, 64, 8, True, True),
+    (1, 2111, 16, 2, 64, 128, 20, False, True), (1, 1601, 8, 1, 128, 128, 13, True, False), (2, 1601, 32, 8, 128, 128, 7, False, True)])
 def test_sparse_attn_backward_ranges(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mask_last):
     test_sparse_attn_backward(pkg, dev, B, L, HQ, H, D, Dv, K, crowd, mask_last)
 
