@@ -47,8 +47,14 @@ static dim3 swa_xcd_grid(int n_blk, int H, int B) { return dim3((unsigned)(((lon
 // Few blocks (SPLIT): a workgroup walks its window in series, two wavefronts per SIMD whose tiles (235 vector and matrix
 // instructions) take turns, so with fewer workgroups than compute units the walk is the kernel.  Two wavefronts then own
 // the same rows and take every other tile, half the queries per workgroup, twice the workgroups; their sums meet in LDS.
-// L1999, 16/2 heads of 64, window 512: 26.6 -> 19.5 us.  The pipelined phases of this form do nothing for a full chip
-// (B2 L8192 32/4 x 64 206 -> 212 us, L8192 32/8 x 128 153 -> 160): the other workgroups hide the loads there.
+// L1999, 16/2 heads of 64, window 512: 26.6 -> 19.5 us.  Either form has one workgroup on a compute unit (registers at 64,
+// LDS at 128), so the halves must fit the chip at once: a second round of them costs as much as the first.  Only where
+// every XCD has the same (batch, head)s of a whole prompt, whose short first blocks come last, may an eighth more follow.
+// us in a graph, whole / in halves, window 512, by workgroups of the halves: 32/8 heads of 128: 256 30.1 / 22.6, 288 30.4 /
+// 22.9, 320 30.5 / 28.7, 376 30.8 / 39.4; 32/4 of 128: 328 31.5 / 41.5; 16/2 of 64: 256 24.1 / 17.4, 276 24.4 / 30.5, 488
+// 25.1 / 31.3; 16/16 of 64: 256 28.2 / 17.8, 288 28.1 / 22.5, 320 28.0 / 29.3; 32/8 of 64: 376 24.6 / 29.0.  The pipelined
+// phases of this form do nothing for a full chip (B2 L8192 32/4 x 64 206 -> 212 us, L8192 32/8 x 128 153 -> 160): the other
+// workgroups hide the loads there.
 #define SWA_FWD_RT 2   // 16-row tiles per wavefront
 #define SWA_LAZY 6.f   // log2 of the growth of a row's maximum that moves its reference point
 
@@ -1001,8 +1007,10 @@ static int swa_fwd_launch(int B, hipStream_t st, const bf16_t* q, const bf16_t* 
   // where one 8-wavefront workgroup does (150 registers: three wavefronts per SIMD)
   if constexpr (D <= 64 && DV <= 64)
     if (tiles <= 4) return swa_fwd_launch_shape<D, DV, G, 4, 4>(B, st, q, k, v, o, lse, dm);
-  const long wgs = (long)((dm.Lq + 256 / G - 1) / (256 / G)) * dm.H * B;  // of one share
-  if (wgs < hils_device_cus()) return swa_fwd_launch_shape<D, DV, G, 8, 4, 2>(B, st, q, k, v, o, lse, dm);
+  const long halves = (long)((dm.Lq + 128 / G - 1) / (128 / G)) * dm.H * B;
+  const bool prompt = dm.Lq == dm.Lk && dm.kv_start == 0, even = (long)dm.H * B % 8 == 0;
+  if (halves <= hils_device_cus() || (prompt && even && 8 * halves <= 9L * hils_device_cus()))
+    return swa_fwd_launch_shape<D, DV, G, 8, 4, 2>(B, st, q, k, v, o, lse, dm);
   return swa_fwd_launch_shape<D, DV, G, 8, 4>(B, st, q, k, v, o, lse, dm);
 }
 

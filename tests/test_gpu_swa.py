@@ -39,7 +39,9 @@ def test_swa_training_shapes(pkg, orc, dev, B, L, HQ, H, D, W, S):
 @pytest.mark.parametrize("B,Lq,Lk,HQ,H,D,Dv,W,S,kw", [
     (1, 1999, 1999, 16, 2, 64, 64, 512, 64, {}), (1, 1100, 1100, 32, 8, 128, 128, 300, 64, {"mask_lmk": True}),
     (1, 1203, 1203, 16, 16, 64, 64, 200, 64, {"expand": False}), (1, 700, 1500, 16, 1, 64, 128, 128, 64, {}),
-    (2, 601, 650, 16, 4, 128, 64, 640, 48, {"mask_lmk": True})])
+    (2, 601, 650, 16, 4, 128, 64, 640, 48, {"mask_lmk": True}), (1, 1024, 1024, 32, 8, 128, 128, 300, 64, {}),
+    (1, 1152, 1152, 32, 8, 128, 128, 300, 64, {}), (1, 1153, 1153, 32, 8, 128, 128, 300, 64, {}),
+    (1, 1025, 1040, 32, 8, 128, 128, 300, 64, {})])  # (the largest that split, each before one that does not)
 def test_swa_few_blocks(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, kw):
     run(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, **kw)
 
