@@ -807,9 +807,13 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   return HILS_OK;
 }
 
-// Segments of the dK walks: with two workgroups per compute unit (what registers allow) about 2.6 times as
-// many items as fit at once, in segments no shorter than eight tiles (a partial result is as many bytes as four).  dK +
-// sum, us, for 1.6 / 2.6 / 4 / 6 times: L8192 32/8 heads of 128 721, 703, 677, 698; L6000 16/16 of 64 124, 119, 122, 131.
+// Segments of the dK walks.  Equal shares fill the chip the better the more of them there are, but each leaves a partial
+// result of as many bytes as four tiles, and a block's segments are summed one after the other: eight items per compute
+// unit (two or three run at once) in segments of 40 tiles and more, five in segments of 24 and more, else three, and none
+// shorter than eight tiles.  Whole backward, us, for three / five / eight items (in brackets, the tiles of a segment): L8192
+// 32/8 heads of 128 [170, 102, 64] 1204 / 1175 / 1153, L8192 16/2 of 64 [85, 51, 32] 454 / 407 and 396 with 40, L5000 32/4 of
+// 128 [65, 39, 24] 468 / 460 / 490, L4096 32/8 of 128 [42, 25, 16] 347 / 336, L4096 16/2 of 64 [21, 12, 8] 147 / 156 / 167,
+// B2 L2048 32/8 of 128 [21, 12, 8] 179 / 185 / 197; the other way only L8192 4/4 of 64 [21, 12, 8], 174 / 167.
 static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
   const int n_pair = (N + 1) / 2, QT = 64 / G, n_tiles = (L + QT - 1) / QT;
   long total = 0;
@@ -819,7 +823,13 @@ static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
     total += len;
   }
   const int longest = n_tiles - lz_tile0(0, W, QT);
-  long target = total * B * H / (5L * hils_device_cus());
+  auto tiles = [&](long items, long most) -> long {  // of a segment with that many items per compute unit
+    const long t = total * B * H / (items * hils_device_cus());
+    return t < most ? t : most;
+  };
+  const long three = tiles(3, 24), five = tiles(5, 40), eight = tiles(8, 1 << 30);
+  long target = three > five ? three : five;
+  target = target > eight ? target : eight;
   if (target < 8) target = 8;
   LzSeg sg{(int)(target < (1 << 30) ? target : (1 << 30)), 1 << 30};
   sg.max_seg = lz_nseg(longest, sg);

@@ -14,3 +14,13 @@ def test_backward_workspace_is_linear_in_the_length(pkg, B, L, HQ, H, D, K):
     # past 32K tokens a range's cells are too small for any of it
     if L >= 32768:
         assert got <= 4 * pairs + chunks * (64 * 3 * D * 2 + 64) + 2 * 2049 * partial + (1 << 20)
+
+
+# walks of dK: many segments only where they are long (a block's partial results are 128 D floats each)
+@pytest.mark.parametrize("B,L,HQ,H,D,most", [(1, 4096, 16, 2, 64, 25), (2, 2048, 32, 8, 128, 6), (1, 8192, 32, 8, 128, 8),
+                                             (1, 5000, 32, 4, 128, 16)])
+def test_log_z_segments(pkg, B, L, HQ, H, D, most):
+    from hils_attention_amd.ops import _cabi
+    got = _cabi.load().hils_chunk_logz_bwd_dk_workspace(B, L, HQ, H, D, 64, 64)
+    blocks = B * H * ((L // 64 + 2) // 2 if L % 128 else L // 128)
+    assert 1 < got // (blocks * 128 * D * 4) <= most
