@@ -2606,13 +2606,18 @@ static bool topk_use_split(int B, int L, int N, int h_kv) {
 // one-pass kernel reads the keys once per 4 to 16 queries; up to some thousand rows it takes one wavefront's time,
 // which grows with the chunks.  (us, row / one-pass, at 500 chunks: 1024 rows of 4 heads of 128 28 / 25, 4096 rows 85 / 30,
 // with a key for each of 8 heads 4096 rows of 128 470 / 52; at 1023 chunks 256 rows of 128 14 / 39, 4096 rows 107 / 49, with
-// a key for each of 8 heads 256 rows 54 / 104, 4096 rows 830 / 135.)
+// a key for each of 8 heads 256 rows 54 / 104, 4096 rows 830 / 135.  One head, whose kernel up to 256 chunks has the
+// queries as columns, heads of 64: 256 chunks, 512 rows 11.1 / 18.5, 1024 rows 19.2 / 18.7, 2048 rows 34.5 / 20.5, 4096 rows
+// 64 / 21; 320 chunks, 2048 rows 36.8 / 35.7; 512 chunks, 2048 rows 36 / 45, 4096 rows 68 / 46; 128 chunks - / 12.6.)
 static double topk_row_us(long rows, int N, int G, int D, int per_qhead) {
   const double key_bytes = (double)N * (per_qhead ? G : 1) * D * 2;
+  if (G == 1 && N <= 512) return 5.0 + rows * 0.015;
   return 8.0 + rows * (key_bytes > 180e3 ? key_bytes / 9.5e6 : 0.019);
 }
 static double topk_group_us(int N, int G, int per_qhead) {
-  return per_qhead ? (G > 4 && N > 512 ? 20.0 + N / 14.0 : 20.0 + N / 28.0) : (G == 1 ? 16.0 + N / 15.0 : 12.0 + N / 40.0);
+  if (per_qhead) return G > 4 && N > 512 ? 20.0 + N / 14.0 : 20.0 + N / 28.0;
+  if (G > 1) return 12.0 + N / 40.0;
+  return N <= 256 ? 10.0 + N / 25.0 : (N <= 512 ? 22.0 + N / 22.0 : 16.0 + N / 15.0);
 }
 static bool topk_group_ahead(long rows, int N, int G, int D, int per_qhead) {
   return topk_group_us(N, G, per_qhead) < topk_row_us(rows, N, G, D, per_qhead);

@@ -17,6 +17,11 @@ from util import note
     (1, 2048, 49200, 32, 4, 128, 32, 1, 1),   # more than 512 chunks, a key for each of eight heads
     (1, 128, 49200, 32, 4, 128, 32, 1, 0),
     (1, 63, 65536, 32, 8, 128, 32, 0, 0),     # the prefill kernels start at 64 queries
+    # one head per KV head on short caches
+    (1, 96, 8192, 16, 16, 64, 8, 0, 1),       # 56 / 50
+    (1, 64, 8192, 32, 32, 128, 16, 0, 1),     # 154 / 104
+    (1, 320, 8192, 4, 4, 64, 8, 0, 1),        # 46 / 43
+    (1, 256, 8192, 4, 4, 64, 8, 0, 0),        # 38 / 40
     # no prefill attention kernel for these groups: the shape-generic one is ten times as slow as the one-launch step
     (1, 512, 16400, 40, 8, 128, 32, 0, 0), (1, 2048, 65536, 12, 4, 64, 32, 0, 0), (1, 1024, 16400, 48, 8, 128, 8, 0, 0),
     (1, 1024, 16400, 28, 4, 64, 8, 0, 0),
