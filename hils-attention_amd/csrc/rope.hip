@@ -443,8 +443,9 @@ extern "C" int hils_norm_rope_pool_fwd(const void* x, const void* norm_weight, c
   return HILS_OK;
 }
 
-// (one block per compute unit: every block is a row of d_weight's sum)
-static int np_bwd_tokens(int B, int L, int H, int D) { return np_tokens(B, L, H, D, hils_device_cus()); }
+// One block per compute unit of the chip: every block is a row of d_weight's sum.  (Not of the device as it is partitioned:
+// the workspace and the order of the sum go by the shape alone.)
+static int np_bwd_tokens(int B, int L, int H, int D) { return np_tokens(B, L, H, D, 256); }
 
 static int np_bwd(const char* who, const void* x, const void* norm_weight, const void* cos_t, const void* sin_t,
                   const void* d_out, const void* d_lmk, void* dx, float* d_weight, float* part, int B, int L, int H,

@@ -443,7 +443,8 @@ int hils_norm_rope_pool_bwd(const void* x, const void* norm_weight, const void* 
                             const void* d_out, const void* d_lmk, void* dx, float* d_weight, int B, int L,
                             int H, int D, int S, int table_per_batch, float eps, void* stream);
 /* The same with the norm weight's gradient written (not added), bf16 or fp32, through a workspace of
- * hils_norm_rope_pool_bwd_workspace() bytes: one row of partial sums per workgroup, added in a fixed order. */
+ * hils_norm_rope_pool_bwd_workspace() bytes (a function of the shape alone): one row of partial sums per
+ * workgroup, added in a fixed order. */
 size_t hils_norm_rope_pool_bwd_workspace(int B, int L, int H, int D, int S);
 int hils_norm_rope_pool_bwd_ws(const void* x, const void* norm_weight, const void* cos_t, const void* sin_t,
                                const void* d_out, const void* d_lmk, void* dx, void* d_weight, int d_weight_bf16,

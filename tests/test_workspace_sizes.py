@@ -24,3 +24,11 @@ def test_log_z_segments(pkg, B, L, HQ, H, D, most):
     got = _cabi.load().hils_chunk_logz_bwd_dk_workspace(B, L, HQ, H, D, 64, 64)
     blocks = B * H * ((L // 64 + 2) // 2 if L % 128 else L // 128)
     assert 1 < got // (blocks * 128 * D * 4) <= most
+
+
+# a row of d_weight per workgroup: per chunk with a chunk mean, without one per 64 tokens or fewer up to 256 workgroups
+@pytest.mark.parametrize("B,L,H,D,S,rows", [(2, 1024, 16, 64, 64, 256), (2, 1024, 2, 64, 64, 128), (1, 300, 4, 128, 64, 75),
+                                            (8, 8192, 16, 64, 64, 2048), (1, 100, 2, 64, 8, 13)])
+def test_norm_rope_backward_workspace_goes_by_the_shape(pkg, B, L, H, D, S, rows):
+    from hils_attention_amd.ops import _cabi
+    assert _cabi.load().hils_norm_rope_pool_bwd_workspace(B, L, H, D, S) == rows * D * 4
