@@ -28,3 +28,31 @@ def test_nan_shows(pkg, dev, HQ, H, D, Dv, B, L, training):
     o, _ = pkg.flex_attn_tl(q, bad, v, 64, 64, training=training, mask_lmk=False)
     G = HQ // H
     assert o[0, L - 1, :G].isnan().all() and not o[0, L - 1, G:].isnan().any()
+
+
+# the window split between two wavefronts (few blocks, a long window): the share that has the key, or only one of the two
+# sees anything
+@pytest.mark.parametrize("B,L,HQ,H,D,Dv", [(1, 1999, 16, 2, 64, 64), (1, 1024, 32, 8, 128, 128), (1, 1203, 16, 16, 64, 64)])
+@pytest.mark.parametrize("t", [0, 70, 700, 1000])
+def test_nan_shows_in_a_split_window(pkg, dev, B, L, HQ, H, D, Dv, t):
+    note(f"split window with a NaN at {t}, L{L} heads {HQ}/{H} x {D}")
+    gen = torch.Generator(device=dev).manual_seed(t)
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev).bfloat16()
+    q, k, v = r(B, L, HQ, D), r(B, L, H, D), r(B, L, H, Dv)
+    o0, lse0 = pkg.flex_attn_tl(q, k, v, 512, 64, mask_lmk=False)
+    bad = q.clone()
+    bad[0, t, 1, 5] = float("nan")
+    o, lse = pkg.flex_attn_tl(bad, k, v, 512, 64, mask_lmk=False)
+    hit = torch.zeros(B, L, HQ, dtype=torch.bool, device=dev)
+    hit[0, t, 1] = True
+    assert o.isnan().all(-1).equal(hit) and o.isnan().any(-1).equal(hit)
+    assert torch.equal(o[~hit], o0[~hit]) and torch.equal(lse[~hit], lse0[~hit])
+    bad = k.clone()
+    bad[0, t, 0, 7] = float("nan")
+    o, _ = pkg.flex_attn_tl(q, bad, v, 512, 64, mask_lmk=False)
+    G = HQ // H
+    last = min(L - 1, t // 64 * 64 + 63 + 511)  # the window of 512 begins in t's chunk and grows to its start
+    sees = torch.zeros(L, dtype=torch.bool, device=dev)
+    sees[t:last + 1] = True
+    assert o[0, :, :G].isnan().any(-1).any(-1)[sees].all() and not o[0, :, G:].isnan().any()
+    assert not o[0, ~sees, :G].isnan().any()
