@@ -17,7 +17,8 @@
 // 16 queries.  Ties at the threshold go to the lower chunk indices.
 //
 // us, queries as rows / as columns, top-32, heads of 64: B8 L8192 16 heads 294 / 165; L16000 16 heads 62 + 87 / 35 + 60 (up to
-// 128 chunks + up to 256; 69 at two wavefronts per SIMD instead of three); B2 L3000 4 heads with a bias, top-16, 22.4 / 14.0.
+// 128 chunks + up to 256; held to the 168 registers of three wavefronts per SIMD the second spills four, 69 at two);
+// B2 L3000 4 heads with a bias, top-16, 22.4 / 14.0.
 #pragma once
 #include "topk_group_kernel.h"
 

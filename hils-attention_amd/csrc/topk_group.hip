@@ -94,10 +94,12 @@ int hils_topk_group_launch(const void* q, const void* lmk_packed, const float* l
       tg_dispatch(GM, D, bias != nullptr, per_qhead != 0, halves, [&](auto gm, auto ks, auto bi, auto pq, auto hf) {
 #define TG_NBS(NB_, EX_) tg_call<gm.value, ks.value, NB_, EX_, bi.value, pq.value, hf.value>(grid, st, a)
         if (exp) TG_NBS(32, true);
-        else if (gm.value > 1 && NB == 8) TG_NBS((gm.value > 1 ? 8 : 24), false);  // (one head: above)
-        else if (gm.value > 1 && NB == 16) TG_NBS((gm.value > 1 ? 16 : 24), false);
+        else if (NB == 32) TG_NBS(32, false);
         else if (NB == 24) TG_NBS(24, false);
-        else TG_NBS(32, false);
+        else if constexpr (gm.value > 1) {  // (one head: above)
+          if (NB == 16) TG_NBS(16, false);
+          else TG_NBS(8, false);
+        }
 #undef TG_NBS
       });
     }
