@@ -3,6 +3,7 @@
 #include "common.h"
 #include "stream_tiles.h"
 #include "../../include/hils_amd.h"
+#include <type_traits>
 
 #define LZ_THREADS 256
 
@@ -64,13 +65,7 @@ logz_fwd_simple(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
 }
 
-// Matrix-core forward for 64-token chunks.  A workgroup of four wavefronts owns 128/G consecutive
-// queries of one KV head (128 score rows: query x head of the group) and walks the chunks that are
-// remote for its last query.  The chunk's keys pass through LDS once per workgroup (double
-// buffered); each wavefront multiplies them with its 32 rows, computing the TRANSPOSED scores
-// K Q^T so that the 64 tokens of one row lie in 16 registers of 4 lanes: the log-sum-exp is an
-// in-lane reduction plus one row-swap reduction.
-#define LZM_RT 2  // 16-row tiles per wavefront
+#define LZ_ROWS 32  // score rows per wavefront
 
 // Workgroup order of the matrix-core kernels: one-dimensional grids in which the blocks of a
 // (batch, KV head) unit run on one XCD (the hardware hands consecutive workgroup ids to the 8 XCDs in
@@ -92,25 +87,77 @@ static dim3 lz_xcd_grid(int n_blk, int n_unit) {
   const int g = lz_units_apart(n_unit), m = 8 / g;
   return dim3((unsigned)(8l * (n_unit / g) * ((n_blk + m - 1) / m)));
 }
-// (the occupancy hint also keeps the score accumulators in ordinary registers: without it the
-// compiler, free to use 512 registers at this workgroup size, parks them in accumulation registers
-// and copies every score back for the softmax; its upper bound keeps the scheduler from saving registers for
-// wavefronts that do not fit anyway, one LDS read and its wait behind the other)
-// Bound by vector-ALU issue: 222 vector instructions (counted, beside 32 matrix ones) per 32 x 64 scores with a maximum
-// per chunk and addresses worked out per load, 197 with fixed addresses, 174 where the maximum is not taken; L 8192,
-// 32/8 heads of 128: 390, 366 and 350 us.
+// ---- streamed tiles of the matrix-core kernels: global memory -> LDS without registers in between -------
+// A wavefront's load brings 64 pieces of 16 bytes to consecutive LDS places; which piece a lane fetches is free, so the
+// tile's rows lie without padding and piece p of row r at p ^ lz_swz(r): conflict-free (4 cycles a wavefront instruction,
+// 8 with rows 16 bytes apart) for the 16-byte row reads of a 32x32 operand and for the transposing reads.
+// The loads are inline assembly that the compiler's wait counts do not know: the kernels wait by hand, for all but the
+// loads of the last step (vector-memory operations complete in order).
+template <int D>
+__device__ __forceinline__ int lz_swz(int r) {
+  return D == 128 ? (r & 3) << 2 | (r >> 2 & 3) : (r >> 1 & 1) << 2 | (r >> 2 & 3);
+}
+__device__ __forceinline__ unsigned long long lz_uniform(unsigned long long x) {
+  return (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)x) |
+         (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32;
+}
+__device__ __forceinline__ unsigned lz_lds_addr(const unsigned char* p) {
+  return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
+}
+// 64 pieces of 16 bytes, lane i's from base + off to lds + 16 i
+__device__ __forceinline__ void lz_dma16(unsigned lds, unsigned off, unsigned long long base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+// 64 words, lane i's from addr to lds + 4 i
+__device__ __forceinline__ void lz_dma4(unsigned lds, unsigned long long addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(addr) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void lz_landed() {  // all but the last N vector-memory operations
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ float lz_halves_sum(float x) {
+  const hils_uint2v y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(y.x) + __uint_as_float(y.y);
+}
+__device__ __forceinline__ float lz_halves_max(float x) {
+  const hils_uint2v y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(y.x), __uint_as_float(y.y));
+}
+// Steps 0 .. n-1, four a round: the buffers' numbers are constants, and so the LDS addresses fixed registers
+// and immediate offsets.
+template <typename F>
+__device__ __forceinline__ void lz_walk(int n, F&& step) {
+  for (int c = 0; c < n; c += 4) {
+    step(c, std::integral_constant<int, 0>{});
+    if (c + 1 < n) step(c + 1, std::integral_constant<int, 1>{});
+    if (c + 2 < n) step(c + 2, std::integral_constant<int, 2>{});
+    if (c + 3 < n) step(c + 3, std::integral_constant<int, 3>{});
+  }
+}
+
+// Matrix-core forward for 64-token chunks.  A workgroup of four wavefronts owns 128/G consecutive queries of one KV head
+// (a wavefront: 32 score rows, query x head of the group) and walks the chunks that are remote for its last query.  A
+// wavefront forms the TRANSPOSED scores K Q^T of 32 tokens at a time on 32x32x16 products, so that the 32 tokens of a row
+// lie in 16 registers of 2 lanes: the log-sum-exp is in-lane work and one half swap.  The products of the next 32 tokens
+// are issued between the exponentials of these (matrix and vector instructions of one wavefront overlap, those of two
+// that run in step hardly do), their operands read a stage before.
+// Bound by the chip's power: at L 8192, 32/8 heads of 128 it runs at 1.9 to 2.0 of 2.4 GHz, about 1000 cycles for the 32 x 64
+// scores of a wavefront against 1170 with 16x16x32 products that waited for their LDS reads and for each other; 325 -> 287 us
+// there, 136 -> 107 at 16/2 heads of 64, 75 -> 54 at L 4096 16/16 heads of 64, 26 -> 19 at L 1200 32/8 of 128 (64 rows a
+// wavefront, half the LDS reads: 285, 131, 57 and 29 us).
 template <int D, int G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
 logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
               float* __restrict__ log_z, LzDims dm, int n_qt, int n_unit) {
-  constexpr int KS = D / 32;
-  constexpr int QW = 16 * LZM_RT / G;  // queries per wavefront
-  constexpr int QB = 4 * QW;           // queries per workgroup
-  constexpr int PITCH = D * 2 + 16;    // bytes per staged key row
-  constexpr int NP = D / 32;           // 16-byte pieces of a chunk per thread
-  __shared__ __align__(16) unsigned char k_s[2][64 * PITCH];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, j = lane >> 4;
+  constexpr int KS = D / 16;
+  constexpr int QW = LZ_ROWS / G;       // queries per wavefront
+  constexpr int QB = 4 * QW;            // queries per workgroup
+  constexpr int NP = D / 32;            // loads of a chunk per wavefront
+  constexpr int NB = 4, TB = 64 * D * 2;
+  __shared__ __align__(16) unsigned char k_s[NB * TB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, h = lane >> 5;
   int unit, qt;
   if (!lz_xcd_unit(n_qt, n_unit, unit, qt)) return;
   qt = n_qt - 1 - qt;  // longest rows first
@@ -118,130 +165,143 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   const long b = unit / dm.H;
   const int t0 = qt * QB + wave * QW;
 
-  bf16x8_t qa[LZM_RT][KS];
-  int lim[LZM_RT];
-  long orow[LZM_RT];
-  bool live[LZM_RT];
+  bf16x8_t qa[KS];
+  const int t = t0 + col / G;
+  const bool live = t < dm.L;
+  const int lim = live ? lz_limit(dm, t) : 0;
+  const long orow = (b * dm.L + (live ? t : dm.L - 1)) * (long)dm.HQ + hk * G + col % G;
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt) {
-    const int row = rt * 16 + col;
-    const int t = t0 + row / G, g = row % G;
-    live[rt] = t < dm.L;
-    const int tc = live[rt] ? t : dm.L - 1;
-    lim[rt] = live[rt] ? lz_limit(dm, t) : 0;
-    orow[rt] = ((b * dm.L + tc) * (long)dm.HQ + hk * G + g);
-    const bf16_t* qp = q + orow[rt] * D + j * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qa[rt][ks] = *(const bf16x8_t*)(qp + ks * 32);
-  }
+  for (int ks = 0; ks < KS; ++ks) qa[ks] = *(const bf16x8_t*)(q + orow * D + h * 8 + ks * 16);
+  float* const z_row = log_z + orow * dm.N + h;
   int t_last = qt * QB + QB - 1;
   if (t_last > dm.L - 1) t_last = dm.L - 1;
-  const int nc = lz_limit(dm, t_last);  // chunks the workgroup walks
+  const int nc = __builtin_amdgcn_readfirstlane(lz_limit(dm, t_last));  // chunks the workgroup walks
   const float sc2 = dm.sm_scale * HILS_LOG2E;
 
-  // (a native vector type: an array of HIP's uint4 struct that lives across the loop's back edge
-  // is kept in scratch memory by the compiler)
-  typedef unsigned lz_u32x4 __attribute__((ext_vector_type(4)));
-  lz_u32x4 kr[NP];
-  // uniform base per chunk, lane offsets fixed: no address arithmetic per chunk (a quarter of the vector
-  // instructions of a chunk when it was worked out each time)
-  const bf16_t* const k_unit = k + (b * dm.L * (long)dm.H + hk) * D;
+  const unsigned long long k_unit = lz_uniform((unsigned long long)(k + (b * dm.L * (long)dm.H + hk) * D));
+  const unsigned k_step = 64u * dm.H * D * 2u;
   unsigned k_off[NP];
 #pragma unroll
-  for (int i = 0; i < NP; ++i) k_off[i] = (unsigned)((tid + 256 * i) / (D / 8) * (dm.H * D) + (tid + 256 * i) % (D / 8) * 8);
-  auto fetch = [&](int c) {
-    const bf16_t* kc = k_unit + (long)c * 64 * dm.H * D;
+  for (int i = 0; i < NP; ++i) {
+    const int x = (wave * NP + i) * 64 + lane, row = x / (D / 8), pc = x % (D / 8);
+    k_off[i] = (unsigned)(row * (dm.H * D) + (pc ^ lz_swz<D>(row)) * 8) * 2u;
+  }
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane(lz_lds_addr(k_s) + wave * (NP * 1024));
+  auto fetch = [&](int c, int buf) __attribute__((always_inline)) {  // (past the walk: its last chunk again)
+    const unsigned long long kc = lz_uniform(k_unit + (unsigned long long)(unsigned)(c < nc ? c : nc - 1) * k_step);
 #pragma unroll
-    for (int i = 0; i < NP; ++i) kr[i] = *(const lz_u32x4*)(kc + k_off[i]);
+    for (int i = 0; i < NP; ++i) lz_dma16(lds0 + buf * TB + i * 1024, k_off[i], kc);
   };
-  auto stash = [&](int buf) {
+  unsigned r_off[KS];
 #pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int p = tid + 256 * i;
-      const int tok = p / (D / 8), seg = p % (D / 8);
-      *(lz_u32x4*)(&k_s[buf][tok * PITCH + seg * 16]) = kr[i];
+  for (int ks = 0; ks < KS; ++ks) r_off[ks] = (unsigned)(col * (D * 2) + ((2 * ks + h) ^ lz_swz<D>(col)) * 16);
+  auto read_tile = [&](bf16x8_t (&x)[KS], int buf, int tt) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) x[ks] = *(const bf16x8_t*)(k_s + (r_off[ks] + buf * TB + tt * 32 * (D * 2)));
+  };
+  auto products = [&](const bf16x8_t (&x)[KS], f32x16_t& st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) st[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[ks], qa[ks], st, 0, 0, 0);
+  };
+  float keep = 0.f;
+  float ref = 0.f;   // reference point of the exponentials: the last chunk's log sum (log2 units)
+  bool far = true;   // (uniform) it was not near its predecessor: the next one's maximum is taken at once
+  const float last = dm.mask_lmk && h == 1 ? 0.f : 1.f;  // what token 63 (register 15 of the second tile) counts for
+  float s[2];
+  auto stage = [&](const bf16x8_t (&x)[KS], f32x16_t& nx, const f32x16_t& cu, bool second) __attribute__((always_inline)) {
+    products(x, nx);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = __builtin_amdgcn_exp2f(fmaf(cu[i], sc2, -ref));
+      if (second && i == 15) s[1] = fmaf(e, last, s[1]);
+      else s[i & 1] += e;
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {  // a product, the additions and fused ones of 16 / KS exponentials, those
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 32 / KS, 0);
+      __builtin_amdgcn_sched_group_barrier(0x400, 16 / KS, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto about_max = [&](const f32x16_t& y0, const f32x16_t& y1, float& m) __attribute__((always_inline)) {
+    const float x63 = last == 0.f ? HILS_NEG_INF : y1[15];
+    m = fmaxf(y0[15], x63);
+#pragma unroll
+    for (int i = 0; i < 15; ++i) m = fmaxf(fmaxf(m, y0[i]), y1[i]);
+    m = lz_halves_max(m) * sc2;  // in log2 units, as the sum below
+    float p0 = 0.f, p1 = __builtin_amdgcn_exp2f(fmaf(x63, sc2, -m));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      p0 += __builtin_amdgcn_exp2f(fmaf(y0[i], sc2, -m));
+      if (i < 15) p1 += __builtin_amdgcn_exp2f(fmaf(y1[i], sc2, -m));
+    }
+    return lz_halves_sum(p0 + p1);
+  };
+  bf16x8_t a0[KS], a1[KS];
+  f32x16_t xa, xb;  // scores of this chunk's first tile; second tile
+  auto step = [&](int c, auto bc) __attribute__((always_inline)) {
+    constexpr int B0 = decltype(bc)::value, B1 = (B0 + 1) % NB, B3 = (B0 + 3) % NB;
+    lz_landed<NP>();  // chunk c + 1
+    lds_barrier();    // ... of all wavefronts; chunk c - 1 has been read
+    fetch(c + 3, B3);
+    // The reference point need not be the maximum, only near it: the exponents of the terms that count and the log of
+    // the sum are rounded at the size of their distance from it.  The previous chunk's log sum serves while the
+    // sums of the whole wavefront stay within [1/8, 8] of it, which scores of a standard deviation of 1 do (the error
+    // against 64 bits is then a tenth below the maximum's; within 2^60 it was up to 1.2 times it with peaked
+    // scores); else the maximum is taken, at once where the last chunk's sum was not near its predecessor's, or going
+    // through the chunk again.  The scale is applied inside the exponent's fused multiply-add.
+    float m = ref, sum;
+    read_tile(a0, B1, 0);
+    if (!far) {
+      s[0] = s[1] = 0.f;
+      __builtin_amdgcn_sched_barrier(0);
+      stage(a1, xb, xa, false);
+      read_tile(a1, B1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(a0, xa, xb, true);
+      sum = lz_halves_sum(s[0] + s[1]);
+      far = __any(!(sum > 0.125f && sum < 8.f));
+      if (far) {
+        bf16x8_t x[KS];
+        f32x16_t y0, y1;
+        read_tile(x, B0, 0);
+        products(x, y0);
+        read_tile(x, B0, 1);
+        products(x, y1);
+        sum = about_max(y0, y1, m);
+      }
+    } else {
+      products(a1, xb);
+      read_tile(a1, B1, 1);
+      sum = about_max(xa, xb, m);
+      products(a0, xa);
+    }
+    const float lse2 = m + __builtin_amdgcn_logf(sum);
+    if (far) far = __any(!(fabsf(lse2 - ref) < 1.5f));  // (well inside: a chunk gone through twice costs 1.7 times)
+    ref = lse2;
+    const float val = (c < lim) ? lse2 * HILS_LN2 : HILS_NEG_INF;
+    if (h == (c & 1)) keep = val;
+    if ((c & 1) || c == nc - 1) {
+      if (live && (c & ~1) + h <= c) z_row[c & ~1] = keep;
     }
   };
   if (nc > 0) {
-    fetch(0);
-    stash(0);
-  }
-  __syncthreads();
-  float keep[LZM_RT];
-  float ref[LZM_RT];  // reference point of the exponentials: the last chunk's log sum (log2 units)
-  bool far[LZM_RT];   // (uniform) it was not near its predecessor: the next one's maximum is taken at once
-#pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt) {
-    keep[rt] = HILS_NEG_INF;
-    ref[rt] = 0.f;
-    far[rt] = true;
-  }
-  for (int c = 0; c < nc; ++c) {
-    fetch(c + 1 < nc ? c + 1 : c);
-    const unsigned char* kb = k_s[c & 1];
-    f32x4_t acc[LZM_RT][4];
-#pragma unroll
-    for (int rt = 0; rt < LZM_RT; ++rt)
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) acc[rt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8_t a = *(const bf16x8_t*)(kb + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
-#pragma unroll
-        for (int rt = 0; rt < LZM_RT; ++rt)
-          acc[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], acc[rt][tt], 0, 0, 0);
-      }
-#pragma unroll
-    for (int rt = 0; rt < LZM_RT; ++rt) {
-      // The reference point need not be the maximum, only near it: the exponents of the terms that count and the log of
-      // the sum are rounded at the size of their distance from it.  The previous chunk's log sum serves while the
-      // sums of the whole wavefront stay within [1/8, 8] of it, which scores of a standard deviation of 1 do (the error
-      // against 64 bits is then a tenth below the maximum's; within 2^60 it was up to 1.2 times it with peaked
-      // scores); else the maximum is taken.  The scale is applied inside the exponent's fused multiply-add.
-      float x[16];
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[tt * 4 + i] = acc[rt][tt][i];
-      if (dm.mask_lmk && j == 3) x[15] = HILS_NEG_INF;  // token 63 = tile 3, lane row 3, register 3
-      float s, m;
-      if (!far[rt]) {
-        m = ref[rt];
-        s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s += __builtin_amdgcn_exp2f(fmaf(x[i], sc2, -m));
-        s = rows_sum(s);
-        far[rt] = __any(!(s > 0.125f && s < 8.f));
-      }
-      if (far[rt]) {
-        m = fmaxf(x[0], x[1]);
-#pragma unroll
-        for (int i = 2; i < 16; i += 2) m = fmaxf(fmaxf(m, x[i]), x[i + 1]);
-        m = rows_max(m) * sc2;  // in log2 units, as the sum below
-        s = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s += __builtin_amdgcn_exp2f(fmaf(x[i], sc2, -m));
-        s = rows_sum(s);
-      }
-      const float lse2 = m + __builtin_amdgcn_logf(s);
-      if (far[rt]) far[rt] = __any(!(fabsf(lse2 - ref[rt]) < 3.f));
-      ref[rt] = lse2;
-      const float val = (c < lim[rt]) ? lse2 * HILS_LN2 : HILS_NEG_INF;
-      if (j == (c & 3)) keep[rt] = val;
-    }
-    if ((c & 3) == 3 || c == nc - 1) {
-      const int cc = (c & ~3) + j;
-#pragma unroll
-      for (int rt = 0; rt < LZM_RT; ++rt)
-        if (live[rt] && cc <= c) log_z[orow[rt] * dm.N + cc] = keep[rt];
-    }
-    stash((c + 1) & 1);
-    __syncthreads();
+    fetch(0, 0);
+    fetch(1, 1);
+    lz_landed<NP>();
+    lds_barrier();
+    fetch(2, 2);
+    read_tile(a0, 0, 0);
+    read_tile(a1, 0, 1);
+    products(a0, xa);
+    lz_walk(nc, step);
+    lz_landed<0>();
   }
   // chunks past the workgroup's walk are not remote for any of its rows
-  for (int r = 0; r < 16 * LZM_RT; ++r) {
+  for (int r = 0; r < LZ_ROWS; ++r) {
     const int t = t0 + r / G, g = r % G;
     if (t >= dm.L) break;
     float* out = log_z + ((b * dm.L + t) * (long)dm.HQ + hk * G + g) * dm.N;
@@ -255,144 +315,175 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 //   dQ = dS K,   dK = dS^T Q.
 // One side of the product is OWNED by a wavefront (32 rows, held in registers as matrix operands,
 // with the fp32 gradient accumulators), the other side STREAMS through LDS in 64-row tiles, stored
-// row-major and double-buffered: the operand of the score product is a row read, that of the gradient product
+// row-major: the operand of the score product is a row read, that of the gradient product
 // (whose contraction runs over the streamed rows) comes through the transposing LDS load.  With a second, transposed
 // copy in LDS a tile took 16 lane permutations, 8 more stores and two barriers; L 8192, 32/8 heads of 128: dQ
-// 715 -> 530 us, dK 840 -> 635 us; what is left is vector-ALU and matrix
-// issue, 150 to 160 vector instructions beside 64 matrix ones per tile.
-// The scores are computed with the
-// owned side as matrix columns, so their accumulator registers are already the left operand of
+// 715 -> 530 us, dK 840 -> 635 us.
+// The scores are computed with the owned side as matrix columns, so their accumulator registers are already an operand of
 // the gradient product.
-// dQ: a wavefront owns 32 score rows (query x head), the chunks' keys stream.
+// dQ: a wavefront owns 32 score rows (query x head), the chunks' keys stream 32 tokens at a time: the scores of the next
+// 32, the exponentials of these and the gradient product of the last ones are independent, and one wavefront's vector
+// instructions run beside its matrix ones.  32x32x16 products; four buffers, loaded two steps ahead without registers
+// between (also the rows' log_z and d_log_z).  Bound by the chip's power: L 8192, 32/8 heads of 128 in 2720 cycles a chunk and pair of
+// workgroups instead of 4010, but at 1.55 GHz instead of 2.1, 522 -> 471 us (1.16 PFLOP/s; a large plain product 1.39);
+// 180 -> 150 us at 16/2 heads of 64, 79 -> 61 at L 4096 16/16 of 64, 29 -> 22 at L 1200 32/8 of 128.  The same for dK, whose factors
+// differ by register instead of by lane, spilled and was slower.
 template <int D, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  const float* __restrict__ log_z, const float* __restrict__ d_log_z,
                  bf16_t* __restrict__ dq, LzDims dm, int n_qt, int n_unit) {
-  constexpr int KS = D / 32, DT = D / 16;
-  constexpr int QW = 16 * LZM_RT / G, QB = 4 * QW;
-  constexpr int PITCH = D * 2 + 16;
-  constexpr int NP = D / 32;  // 16-byte pieces of a chunk per thread
-  __shared__ __align__(16) unsigned char k_s[2][64 * PITCH];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 15, j = lane >> 4;
+  typedef short lz_s4 __attribute__((ext_vector_type(4)));
+  typedef short lz_s8 __attribute__((ext_vector_type(8)));
+  typedef unsigned lz_u4 __attribute__((ext_vector_type(4)));
+  constexpr int KS = D / 16, DT = D / 32;
+  constexpr int QW = LZ_ROWS / G, QB = 4 * QW;
+  constexpr int NP = D / 32;  // loads of a chunk per wavefront
+  constexpr int NB = 4, TB = 64 * D * 2;
+  __shared__ __align__(16) unsigned char k_s[NB * TB + 4 * NB * 256];  // keys; a wavefront's log_z and d_log_z of a chunk
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, h = lane >> 5;
   int unit, qt;
   if (!lz_xcd_unit(n_qt, n_unit, unit, qt)) return;
   qt = n_qt - 1 - qt;
   const int hk = unit % dm.H;
   const long b = unit / dm.H;
-  const int t0 = qt * QB + wave * QW;
-
-  bf16x8_t qa[LZM_RT][KS];
-  int lim[LZM_RT];
-  long orow[LZM_RT];
+  const int t = qt * QB + wave * QW + col / G;
+  const bool live = t < dm.L;
+  const int lim = live ? lz_limit(dm, t) : 0;
+  const long orow = ((b * dm.L + (live ? t : dm.L - 1)) * (long)dm.HQ + hk * G + col % G);
+  bf16x8_t qa[KS];
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt) {
-    const int row = rt * 16 + col;
-    const int t = t0 + row / G, g = row % G;
-    const int tc = t < dm.L ? t : dm.L - 1;
-    lim[rt] = t < dm.L ? lz_limit(dm, t) : 0;
-    orow[rt] = ((b * dm.L + tc) * (long)dm.HQ + hk * G + g);
-    const bf16_t* qp = q + orow[rt] * D + j * 8;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qa[rt][ks] = *(const bf16x8_t*)(qp + ks * 32);
-  }
+  for (int ks = 0; ks < KS; ++ks) qa[ks] = *(const bf16x8_t*)(q + orow * D + h * 8 + ks * 16);
   int t_last = qt * QB + QB - 1;
   if (t_last > dm.L - 1) t_last = dm.L - 1;
-  const int nc = lz_limit(dm, t_last);
+  const int nc = __builtin_amdgcn_readfirstlane(lz_limit(dm, t_last));
   const float sc2 = dm.sm_scale * HILS_LOG2E;
 
-  typedef unsigned lz_u32x4 __attribute__((ext_vector_type(4)));
-  lz_u32x4 kr[NP];
-  const bf16_t* const k_unit = k + (b * dm.L * (long)dm.H + hk) * D;
+  const unsigned long long k_unit = lz_uniform((unsigned long long)(k + (b * dm.L * (long)dm.H + hk) * D));
+  const unsigned k_step = 64u * dm.H * D * 2u;
   unsigned k_off[NP];
 #pragma unroll
-  for (int i = 0; i < NP; ++i) k_off[i] = (unsigned)((tid + 256 * i) / (D / 8) * (dm.H * D) + (tid + 256 * i) % (D / 8) * 8);
-  auto fetch = [&](int c) {
-    const bf16_t* kc = k_unit + (long)c * 64 * dm.H * D;
+  for (int i = 0; i < NP; ++i) {
+    const int x = (wave * NP + i) * 64 + lane, row = x / (D / 8), pc = x % (D / 8);
+    k_off[i] = (unsigned)(row * (dm.H * D) + (pc ^ lz_swz<D>(row)) * 8) * 2u;
+  }
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane(lz_lds_addr(k_s) + wave * (NP * 1024));
+  const unsigned z_lds = __builtin_amdgcn_readfirstlane(lz_lds_addr(k_s) + NB * TB + wave * (NB * 256));
+  // lanes 0..31 bring log_z of the wavefront's rows, the others d_log_z
+  const unsigned long long z_lane = (unsigned long long)((h ? d_log_z : log_z) + orow * dm.N);
+  auto fetch = [&](int c, int buf) __attribute__((always_inline)) {  // (past the walk: its last chunk again)
+    const unsigned long long kc = lz_uniform(k_unit + (unsigned long long)(unsigned)(c < nc ? c : nc - 1) * k_step);
 #pragma unroll
-    for (int i = 0; i < NP; ++i) kr[i] = *(const lz_u32x4*)(kc + k_off[i]);
+    for (int i = 0; i < NP; ++i) lz_dma16(lds0 + buf * TB + i * 1024, k_off[i], kc);
   };
-  auto stash = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NP; ++i)
-      *(lz_u32x4*)(&k_s[buf][(tid + 256 * i) / (D / 8) * PITCH + (tid + 256 * i) % (D / 8) * 16]) = kr[i];
+  auto fetch_z = [&](int c, int buf) __attribute__((always_inline)) {
+    lz_dma4(z_lds + buf * 256, z_lane + (unsigned)(c < nc ? c : nc - 1) * 4u);
   };
-  f32x4_t acc[LZM_RT][DT];
+  // LDS addresses: rows of a 32-token tile (operand of the scores), columns of 16 tokens (of the gradient)
+  unsigned r_off[KS], c_off[DT];
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt)
+  for (int ks = 0; ks < KS; ++ks) r_off[ks] = (unsigned)(col * (D * 2) + ((2 * ks + h) ^ lz_swz<D>(col)) * 16);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float lzn[LZM_RT], dln[LZM_RT];
-  unsigned z_off[LZM_RT];  // of the lane's row behind the first row of the workgroup's first query
-  const long z_first = (b * dm.L + qt * QB) * (long)dm.HQ * dm.N;
+  for (int dt = 0; dt < DT; ++dt) {
+    const int l = lane & 15, row = 4 * h + (l >> 2), pc = dt * 4 + (lane >> 4 & 1) * 2 + (l >> 1 & 1);
+    c_off[dt] = (unsigned)(row * (D * 2) + (pc ^ lz_swz<D>(row)) * 16 + (l & 1) * 8);
+  }
+  f32x16_t acc[DT], sa, sb;
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt) z_off[rt] = (unsigned)(orow[rt] * dm.N - z_first);
-  auto fetch_z = [&](int c) {
-    const float *zc = log_z + z_first + c, *dc = d_log_z + z_first + c;
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int rt = 0; rt < LZM_RT; ++rt) {
-      lzn[rt] = zc[z_off[rt]];
-      dln[rt] = dc[z_off[rt]];
+    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
+  bf16x8_t ra[KS], ca[2][DT], pp[2];
+  auto read_row = [&](int ks, int buf, int tt) __attribute__((always_inline)) {
+    ra[ks] = *(const bf16x8_t*)(k_s + (r_off[ks] + buf * TB + tt * 32 * (D * 2)));
+  };
+  auto read_col = [&](int s, int dt, int buf, int tt) __attribute__((always_inline)) {
+    const int imm = buf * TB + (tt * 32 + s * 16) * (D * 2);
+    unsigned down;  // the same piece eight rows further down: the swizzle's bit 1 (worked out here: four registers less)
+    asm volatile("v_xor_b32 %0, 32, %1" : "=v"(down) : "v"(c_off[dt]));
+    const lz_s4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lz_s4*)(k_s + (c_off[dt] + imm)));
+    const lz_s4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lz_s4*)(k_s + (down + (imm + 8 * (D * 2)))));
+    ca[s][dt] = __builtin_bit_cast(bf16x8_t, (lz_s8)__builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  float off = 0.f, coef = 0.f;
+  // One stage: scores of the next tile (nx), exponentials of this one's (cu), gradient product of the last one's (pp, ca).
+  // The next stage's operands are read behind the last use of these: rows of tile rtt of rbuf, columns of this tile.
+  auto stage = [&](f32x16_t& nx, const f32x16_t& cu, int rbuf, int rtt, int cbuf, int ctt) __attribute__((always_inline)) {
+    float p[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) nx[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      nx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ra[u], qa[u], nx, 0, 0, 0);
+      read_row(u, rbuf, rtt);
+      const int s = u / DT, dt = u % DT;
+      acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[s][dt], pp[s], acc[dt], 0, 0, 0);
+      read_col(s, dt, cbuf, ctt);
+#pragma unroll
+      for (int i = u * 16 / KS; i < (u + 1) * 16 / KS; ++i) p[i] = __builtin_amdgcn_exp2f(fmaf(cu[i], sc2, -off)) * coef;
     }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      lz_u4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = pack_bf2(p[s * 8 + 2 * e], p[s * 8 + 2 * e + 1]);
+      pp[s] = __builtin_bit_cast(bf16x8_t, x);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // (step c asks for the keys of chunk c + 3 and the row values of c + 2)
+  auto step = [&](int c, auto bc) __attribute__((always_inline)) {
+    constexpr int B0 = decltype(bc)::value, B1 = (B0 + 1) % NB, B2 = (B0 + 2) % NB, B3 = (B0 + 3) % NB;
+    lz_landed<NP + 1>();  // the keys of chunk c + 1, the row values of c
+    lds_barrier();        // ... of all wavefronts; chunk c - 1 has been read
+    const float* zs = (const float*)(k_s + (NB * TB + wave * (NB * 256) + B0 * 256 + col * 4));
+    const float lz = zs[0], dz = zs[32];
+    const bool ok = c < lim && lz > -1e30f;
+    off = ok ? lz * HILS_LOG2E : 0.f;
+    coef = ok ? dz * dm.sm_scale : 0.f;
+    fetch(c + 3, B3);
+    fetch_z(c + 2, B2);
+    __builtin_amdgcn_sched_barrier(0);
+    stage(sb, sa, B1, 0, B0, 0);
+    stage(sa, sb, B1, 1, B0, 1);
   };
   if (nc > 0) {
-    fetch(0);
-    fetch_z(0);
-    stash(0);
-  }
-  __syncthreads();
-  for (int c = 0; c < nc; ++c) {
-    const unsigned char* kb = k_s[c & 1];
-    float off[LZM_RT], coef[LZM_RT];
+    fetch(0, 0);
+    fetch_z(0, 0);
+    fetch(1, 1);
+    fetch_z(1, 1);
+    lz_landed<NP + 1>();
+    lds_barrier();
+    fetch(2, 2);
+    // the first tile's scores; the gradient product before it is one with zeros
 #pragma unroll
-    for (int rt = 0; rt < LZM_RT; ++rt) {
-      const bool ok = c < lim[rt] && lzn[rt] > -1e30f;
-      off[rt] = ok ? lzn[rt] * HILS_LOG2E : 0.f;
-      coef[rt] = ok ? dln[rt] * dm.sm_scale : 0.f;
+    for (int u = 0; u < KS; ++u) read_row(u, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sa[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ra[u], qa[u], sa, 0, 0, 0);
+      read_row(u, 0, 1);
+      read_col(u / DT, u % DT, 0, 0);
     }
-    const int cn = c + 1 < nc ? c + 1 : c;
-    fetch(cn);
-    fetch_z(cn);
-    __builtin_amdgcn_sched_barrier(0);  // (the loads would sink to their stores into LDS)
-    float p[LZM_RT][4][4];
-    {
-      f32x4_t st[LZM_RT][4];
+    pp[0] = pp[1] = __builtin_bit_cast(bf16x8_t, (lz_s8)(0));
+    lz_walk(nc, step);
 #pragma unroll
-      for (int rt = 0; rt < LZM_RT; ++rt)
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) st[rt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(kb + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
-#pragma unroll
-          for (int rt = 0; rt < LZM_RT; ++rt)
-            st[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], st[rt][tt], 0, 0, 0);
-        }
-#pragma unroll
-      for (int rt = 0; rt < LZM_RT; ++rt)
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            p[rt][tt][i] = __builtin_amdgcn_exp2f(st[rt][tt][i] * sc2 - off[rt]) * coef[rt];
-    }
-    lzm_grad_product_rows<D, LZM_RT, PITCH>(kb, p, acc, col, j);
-    stash((c + 1) & 1);
-    __syncthreads();
+    for (int u = 0; u < KS; ++u)  // of the last tile
+      acc[u % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[u / DT][u % DT], pp[u / DT], acc[u % DT], 0, 0, 0);
+    lz_landed<0>();
   }
+  if (!live) return;
+  bf16_t* out = dq + orow * D + 4 * h;  // a lane holds four neighbouring features of its row
 #pragma unroll
-  for (int rt = 0; rt < LZM_RT; ++rt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = rt * 16 + 4 * j + i;
-      const int t = t0 + row / G, g = row % G;
-      if (t >= dm.L) continue;
-      bf16_t* out = dq + ((b * dm.L + t) * (long)dm.HQ + hk * G + g) * D + col;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) out[dt * 16] = f2bf(acc[rt][dt][i]);
+    for (int e = 0; e < 4; ++e) {
+      uint2 x;
+      x.x = pack_bf2(acc[dt][4 * e], acc[dt][4 * e + 1]);
+      x.y = pack_bf2(acc[dt][4 * e + 2], acc[dt][4 * e + 3]);
+      *(uint2*)(out + dt * 32 + e * 8) = x;
     }
 }
 
@@ -421,7 +512,7 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  bf16_t* __restrict__ dk, LzDims dm, int n_pair, int n_unit, LzSeg sg, float* __restrict__ part) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int QT = 64 / G;  // queries per streamed tile
-  constexpr int PITCH = D * 2 + 16;
+  constexpr int PITCH = D * 2 + 32;  // (16-byte reads of 16 rows: 4 cycles; 8 at D * 2 + 16)
   constexpr int NP = D / 32;  // 16-byte pieces of a tile per thread
   __shared__ __align__(16) unsigned char q_s[2][64 * PITCH];
   __shared__ __align__(16) float off_s[2][2][64];
@@ -760,7 +851,7 @@ extern "C" int hils_chunk_logz_fwd(const void* q, const void* k, float* log_z, i
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, mask_lmk, sm_scale};
   const int G = HQ / H;
   if (lz_mfma_covers(G, D, S, H, B)) {
-    const int QB = 4 * 16 * LZM_RT / G;
+    const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;
     HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_fwd: B * H * L too large for the grid");
     const dim3 grid = lz_xcd_grid(n_qt, B * H);
@@ -788,7 +879,7 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, 0, sm_scale};
   if (lz_mfma_covers(HQ / H, D, S, H, B)) {
     const int G = HQ / H;
-    const int QB = 4 * 16 * LZM_RT / G;
+    const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;
     HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_bwd_dq: B * H * L too large for the grid");
     const dim3 grid = lz_xcd_grid(n_qt, B * H);

@@ -1,0 +1,35 @@
+"""Exact log Z and dQ: walks of one to nine chunks (the kernels take four steps a round and load three ahead), keys whose
+sums jump between neighbouring chunks, the landmark mask."""
+import pytest
+import torch
+
+from util import LSE_TOL, assert_close_bf16, assert_close_f32, note
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("HQ,H,D", [(2, 2, 64), (8, 2, 128), (16, 1, 64), (4, 4, 128)])
+@pytest.mark.parametrize("chunks,rest,mask_lmk", [(1, 0, False), (2, 1, True), (3, 63, False), (4, 0, True), (5, 17, False),
+                                                  (6, 40, True), (9, 5, False)])
+def test_walks(pkg, orc, dev, HQ, H, D, chunks, rest, mask_lmk):
+    note(f"log Z walks {chunks} chunks + {rest}, heads {HQ}/{H} x {D}, mask {mask_lmk}")
+    gen = torch.Generator().manual_seed(chunks * 100 + rest)
+    L, W = (chunks + 1) * 64 + rest, 64
+    q = torch.randn(2, L, HQ, D, generator=gen)
+    k = torch.randn(2, L, H, D, generator=gen)
+    k[:, 64:192] *= 5  # near its predecessor's sum, far, far and so on
+    k[1, 256:320] *= 0.1
+    q, k = q.bfloat16(), k.bfloat16()
+    qd, kd = q.to(dev).requires_grad_(not mask_lmk), k.to(dev).requires_grad_(not mask_lmk)
+    z = pkg.exact_chunk_log_z_tl(qd, kd, chunk_size=64, window_size=W, mask_lmk=mask_lmk)
+    qf, kf = q.float().requires_grad_(), k.float().requires_grad_()
+    ref = orc.exact_chunk_log_z(qf, kf, chunk_size=64, window_size=W, mask_lmk=mask_lmk)
+    assert_close_f32(z.detach(), ref.detach(), LSE_TOL, "log_z")
+    if mask_lmk:
+        return  # forward only
+    finite = torch.isfinite(ref)
+    g = torch.randn(ref.shape, generator=gen) * finite
+    z.backward(g.to(dev))
+    torch.where(finite, ref, torch.zeros(())).mul(g).sum().backward()
+    assert_close_bf16(qd.grad, qf.grad, "dq")
+    assert_close_bf16(kd.grad, kf.grad, "dk")
