@@ -512,7 +512,7 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                  bf16_t* __restrict__ dk, LzDims dm, int n_pair, int n_unit, LzSeg sg, float* __restrict__ part) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int QT = 64 / G;  // queries per streamed tile
-  constexpr int PITCH = D * 2 + 32;  // (16-byte reads of 16 rows: 4 cycles; 8 at D * 2 + 16)
+  constexpr int PITCH = D * 2 + 32;
   constexpr int NP = D / 32;  // 16-byte pieces of a tile per thread
   __shared__ __align__(16) unsigned char q_s[2][64 * PITCH];
   __shared__ __align__(16) float off_s[2][2][64];
@@ -645,26 +645,24 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     stash(buf ^ 1);
     __syncthreads();
   }
-  if (n_seg > 1) {
-    float* out = part + (((long)unit * n_pair + pair) * sg.max_seg + seg_i) * (128 * D);
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+  for (int tt = 0; tt < 2; ++tt) {  // (a lane holds four neighbouring features of its token)
+    const int t = tt * 16 + col, tok = tok0 + t;
+    if (n_seg > 1) {
+      float* out = part + (((long)unit * n_pair + pair) * sg.max_seg + seg_i) * (128 * D) + (wave * 32 + t) * D + 4 * j;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int dt = 0; dt < DT; ++dt) *(f32x4_t*)(out + dt * 16) = acc[tt][dt];
+    } else if (tok < dm.L) {
+      bf16_t* out = dk + ((b * dm.L + tok) * (long)dm.H + hk) * D + 4 * j;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) out[(wave * 32 + tt * 16 + 4 * j + i) * D + dt * 16 + col] = acc[tt][dt][i];
-    return;
-  }
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = tok0 + tt * 16 + 4 * j + i;
-      if (tok >= dm.L) continue;
-      bf16_t* out = dk + ((b * dm.L + tok) * (long)dm.H + hk) * D + col;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) out[dt * 16] = f2bf(acc[tt][dt][i]);
+      for (int dt = 0; dt < DT; ++dt) {
+        uint2 x;
+        x.x = pack_bf2(acc[tt][dt][0], acc[tt][dt][1]);
+        x.y = pack_bf2(acc[tt][dt][2], acc[tt][dt][3]);
+        *(uint2*)(out + dt * 16) = x;
+      }
     }
+  }
 }
 
 // the segments of the cut walks, in order; four features per thread

@@ -475,8 +475,11 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
 //   P = exp(s - lse),  dP = dO V^T,  delta = sum_d o*dO - d_lse,  dS = P (dP - delta) * scale
 //   dQ = dS K,  dK = dS^T Q,  dV = P^T dO.
 // Same split as the forward: one side owned by a wavefront in registers, the other streamed
-// through LDS in 64-row tiles (row-major for the score-like products, transposed for the
-// gradient products).
+// through LDS in 64-row tiles, row-major, which the gradient products read by the transposing LDS load.  Bound by vector
+// issue beside the matrix products.  With a second, transposed copy in LDS, rows 16 bytes apart (twice the cycles a read,
+// stream_tiles.h), masks in every tile and the results stored two bytes a lane, us, dQ + dK/dV then / now:
+// B2 L8192 32/4 heads of 64 window 512 400 / 340, L8192 32/8 of 128 window 512 503 / 371, L4096 32/4 of 128 282 / 191,
+// L8192 32/8 of 128 window 64 169 / 148, B8 L8192 16/16 of 64 window 64 432 / 429, B2 L1024 16/2 of 64 window 512 47 / 43.
 
 // visibility bits of this lane's landmark test for the 16 tokens tt*16 + 4j + i of a 64-token tile
 __device__ __forceinline__ unsigned swa_lmk_bits(const SwaDims& dm, int tok0) {
@@ -496,13 +499,13 @@ __device__ __forceinline__ unsigned swa_lmk_bits(const SwaDims& dm, int tok0) {
 // 16-row tiles per wavefront of the backward kernels: two for narrow heads; one for wide heads, whose two
 // tiles need more than 256 registers (one wavefront per SIMD, nothing to overlap a wait with)
 constexpr int swa_dq_rt(int D, int DV) { return (D <= 64 && DV <= 64) ? 2 : 1; }
+constexpr int swa_dkdv_buffers(int D, int DV) { return (D > 64 && DV > 64) ? 1 : 2; }
 
-// dQ (and delta): a wavefront owns 16 * RT score rows; K (row-major and transposed) and V stream.
+// dQ (and delta): a wavefront owns 16 * RT score rows; K and V stream.
 template <int D, int DV, int G>
-// (the hint keeps the accumulators out of accumulation registers; wide heads with their one tile per
-// wavefront are held to 168 registers, five spilled dwords, for three wavefronts per SIMD: 52 KiB of LDS
-// let three workgroups share a compute unit)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D > 64 && DV > 64) ? 3 : 2)))
+// (the hint keeps the accumulators out of accumulation registers; three wavefronts per SIMD of wide heads spilled: 222 us
+// instead of 191 at L4096 32/4 of 128 window 512)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                 const bf16_t* __restrict__ o, const float* __restrict__ lse,
                 const bf16_t* __restrict__ d_o, const float* __restrict__ d_lse,
@@ -510,12 +513,11 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
   constexpr int RT = swa_dq_rt(D, DV);
   constexpr int KS = D / 32, VS = DV / 32, DT = D / 16;
   constexpr int QW = 16 * RT / G > 0 ? 16 * RT / G : 1, QB = 4 * 16 * RT / G;
-  constexpr int PITCH = D * 2 + 16, VPITCH = DV * 2 + 16;
-  constexpr int KSEG = D / 8, KPPP = 256 / KSEG, KPASS = 32 / KPPP;
-  constexpr int VSEG = DV / 8, VPASS = 64 * VSEG / 256;
-  __shared__ __align__(16) unsigned char k_s[64 * PITCH];
-  __shared__ __align__(16) unsigned char kt_s[D * LZM_PT];
-  __shared__ __align__(16) unsigned char v_s[64 * VPITCH];
+  constexpr int PITCH = D * 2 + 32, VPITCH = DV * 2 + 32;
+  constexpr int KSEG = D / 8, KPASS = 64 * KSEG / 256, VSEG = DV / 8, VPASS = 64 * VSEG / 256;
+  constexpr int NB = (D > 64 && DV > 64) ? 1 : 2;  // buffers (two of wide heads: no faster)
+  __shared__ __align__(16) unsigned char k_s[NB][64 * PITCH];
+  __shared__ __align__(16) unsigned char v_s[NB][64 * VPITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   int qt, hk;
@@ -539,7 +541,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
     qabs[rt] = live ? t : -2147483647;
     const int left = tc - dm.window + 1;
     cstart[rt] = dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left;
-    lse2[rt] = live ? ls * HILS_LOG2E : 0.f;
+    lse2[rt] = live ? ls * HILS_LOG2E : INFINITY;  // (no probability but 0)
     const bf16_t* qp = q + rix * D + j * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qa[rt][ks] = *(const bf16x8_t*)(qp + ks * 32);
@@ -568,6 +570,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
     vspan[rt] = some ? (unsigned)(qabs[rt] - cstart[rt]) : 0u;
   }
   int tile_lo, tile_hi;
+  int full_lo, full_hi;  // tiles that all rows see whole
   {
     const int tq0 = qt * QB;
     int tq1 = tq0 + QB - 1;
@@ -577,23 +580,25 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
     lo = lo < 0 ? 0 : lo;
     tile_lo = lo / 64;
     tile_hi = tq1 / 64 + 1;
+    const int right_abs = tq1 - dm.window + 1;
+    const int first = dm.expand ? floordiv(right_abs, dm.chunk) * dm.chunk : right_abs;  // of the last row's window
+    full_lo = first > 0 ? (first + 63) / 64 : 0;
+    full_hi = dm.mask_lmk ? 0 : (tq0 + 1) / 64;
   }
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
   // prefetch registers as in the forward kernel: native vectors, loads without branches, tokens
   // past the end read the last row (their probabilities are masked to 0)
   typedef unsigned swa_u32x4 __attribute__((ext_vector_type(4)));
-  swa_u32x4 kr[KPASS][2], vr[VPASS];
-  auto as_uint4 = [](const swa_u32x4& x) { return make_uint4(x.x, x.y, x.z, x.w); };
+  swa_u32x4 kr[KPASS], vr[VPASS];
   auto fetch = [&](int tile) {
 #pragma unroll
-    for (int i = 0; i < KPASS; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        int tok = tile * 64 + 2 * (tid / KSEG + KPPP * i) + h;
-        tok = tok < L ? tok : L - 1;
-        kr[i][h] = *(const swa_u32x4*)(k + ((b * L + tok) * (long)dm.H + hk) * D + (tid % KSEG) * 8);
-      }
+    for (int i = 0; i < KPASS; ++i) {
+      const int p = tid + 256 * i;
+      int tok = tile * 64 + p / KSEG;
+      tok = tok < L ? tok : L - 1;
+      kr[i] = *(const swa_u32x4*)(k + ((b * L + tok) * (long)dm.H + hk) * D + (p % KSEG) * 8);
+    }
 #pragma unroll
     for (int i = 0; i < VPASS; ++i) {
       const int p = tid + 256 * i;
@@ -602,14 +607,16 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
       vr[i] = *(const swa_u32x4*)(v + ((b * L + tok) * (long)dm.H + hk) * DV + (p % VSEG) * 8);
     }
   };
-  auto stash = [&]() {
+  auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < KPASS; ++i)
-      lzm_stash_pair<PITCH>(k_s, kt_s, 2 * (tid / KSEG + KPPP * i), tid % KSEG, as_uint4(kr[i][0]), as_uint4(kr[i][1]));
+    for (int i = 0; i < KPASS; ++i) {
+      const int p = tid + 256 * i;
+      *(swa_u32x4*)(k_s[buf] + (p / KSEG) * PITCH + (p % KSEG) * 16) = kr[i];
+    }
 #pragma unroll
     for (int i = 0; i < VPASS; ++i) {
       const int p = tid + 256 * i;
-      *(swa_u32x4*)(v_s + (p / VSEG) * VPITCH + (p % VSEG) * 16) = vr[i];
+      *(swa_u32x4*)(v_s[buf] + (p / VSEG) * VPITCH + (p % VSEG) * 16) = vr[i];
     }
   };
   f32x4_t acc[RT][DT];
@@ -618,10 +625,12 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   fetch(tile_lo);
-  stash();
+  stash(0);
   __syncthreads();
-  for (int tile = tile_lo; tile < tile_hi; ++tile) {
+  for (int tile = tile_lo, buf = 0; tile < tile_hi; ++tile) {
     fetch(tile + 1 < tile_hi ? tile + 1 : tile);
+    const unsigned char *kb = k_s[buf], *vb = v_s[buf];
+    const bool full = tile >= full_lo && tile < full_hi;
     float ds[RT][4][4];
     {
       f32x4_t st[RT][4], dp[RT][4];
@@ -636,33 +645,43 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
       for (int tt = 0; tt < 4; ++tt) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(k_s + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(kb + (tt * 16 + col) * PITCH + ks * 64 + j * 16);
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
             st[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], st[rt][tt], 0, 0, 0);
         }
 #pragma unroll
         for (int vs = 0; vs < VS; ++vs) {
-          const bf16x8_t a = *(const bf16x8_t*)(v_s + (tt * 16 + col) * VPITCH + vs * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(vb + (tt * 16 + col) * VPITCH + vs * 64 + j * 16);
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
             dp[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, doa[rt][vs], dp[rt][tt], 0, 0, 0);
         }
       }
-      // token ta is visible to a row iff window start <= ta <= query: one unsigned compare of
-      // ta - start against query - start (a dead row has a start no token reaches)
       const int tok0 = tile * 64 + 4 * j;
+      if (full) {
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const unsigned base = (unsigned)(tok0 - vlo[rt]);
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
+          for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const bool vis = base + (unsigned)(tt * 16 + i) <= vspan[rt];
-            const float pv = vis ? __builtin_amdgcn_exp2f(st[rt][tt][i] * c2 - lse2[rt]) : 0.f;
-            ds[rt][tt][i] = pv * (dp[rt][tt][i] - delta[rt]) * dm.sm_scale;
-          }
+            for (int i = 0; i < 4; ++i)
+              ds[rt][tt][i] = __builtin_amdgcn_exp2f(st[rt][tt][i] * c2 - lse2[rt]) * (dp[rt][tt][i] - delta[rt]);
+      } else {
+        // token ta is visible to a row iff window start <= ta <= query: one unsigned compare of
+        // ta - start against query - start (a dead row has a start no token reaches)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const unsigned base = (unsigned)(tok0 - vlo[rt]);
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const bool vis = base + (unsigned)(tt * 16 + i) <= vspan[rt];
+              const float pv = vis ? __builtin_amdgcn_exp2f(st[rt][tt][i] * c2 - lse2[rt]) : 0.f;
+              ds[rt][tt][i] = pv * (dp[rt][tt][i] - delta[rt]);
+            }
+        }
       }
       if (dm.mask_lmk) {  // landmarks in a pass of their own behind a uniform branch (row-independent)
         const unsigned lmk_ok = swa_lmk_bits(dm, tok0);
@@ -676,28 +695,32 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
           }
       }
     }
-    lzm_grad_product<D, RT>(kt_s, ds, acc, col, j);
-    __syncthreads();
-    stash();
+    lzm_grad_product_rows<D, RT, PITCH>(kb, ds, acc, col, j);
+    if (NB == 1) __syncthreads();
+    else buf ^= 1;
+    stash(buf);
     __syncthreads();
   }
+  // (the scale of the scores last: a lane holds four neighbouring features of its rows)
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+  for (int rt = 0; rt < RT; ++rt) {
+    const int row = rt * 16 + col, t = t0 + row / G, g = row % G;
+    if (t >= L) continue;
+    bf16_t* out = dq + ((b * L + t) * (long)dm.HQ + hk * G + g) * D + 4 * j;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = rt * 16 + 4 * j + i;
-      const int t = t0 + row / G, g = row % G;
-      if (t >= L) continue;
-      bf16_t* out = dq + ((b * L + t) * (long)dm.HQ + hk * G + g) * D + col;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) out[dt * 16] = f2bf(acc[rt][dt][i]);
+    for (int dt = 0; dt < DT; ++dt) {
+      uint2 x;
+      x.x = pack_bf2(acc[rt][dt][0] * dm.sm_scale, acc[rt][dt][1] * dm.sm_scale);
+      x.y = pack_bf2(acc[rt][dt][2] * dm.sm_scale, acc[rt][dt][3] * dm.sm_scale);
+      *(uint2*)(out + dt * 16) = x;
     }
+  }
 }
 
 // dK, dV: a workgroup owns 64 * TT tokens of one KV head (TT 16-token tiles per wavefront, as matrix B
 // operands: two for narrow heads, one for wide heads, whose two tiles need more than 256 registers); the
-// score rows (query x head) that can see them stream in tiles of 64 rows, Q and dO both row-major
-// and transposed, with the rows' lse, delta and window start beside them.
+// score rows (query x head) that can see them stream in tiles of 64 rows of Q and dO,
+// with the rows' lse, delta and window start beside them.
 template <int D, int DV, int G>
 // (the hint gives two wavefronts per SIMD and keeps the accumulators out of accumulation registers)
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
@@ -709,17 +732,15 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   constexpr int TT = swa_dq_rt(D, DV);
   constexpr int KS = D / 32, VS = DV / 32, DT = D / 16, DVT = DV / 16;
   constexpr int QT = 64 / G;
-  constexpr int PITCH = D * 2 + 16, VPITCH = DV * 2 + 16;
-  constexpr int QSEG = D / 8, QPPP = 256 / QSEG, QPASS = 32 / QPPP;
-  constexpr int OSEG = DV / 8, OPPP = 256 / OSEG, OPASS = 32 / OPPP;
+  constexpr int PITCH = D * 2 + 32, VPITCH = DV * 2 + 32;
+  constexpr int QSEG = D / 8, QPASS = 64 * QSEG / 256, OSEG = DV / 8, OPASS = 64 * OSEG / 256;
+  constexpr int NB = swa_dkdv_buffers(D, DV);
   extern __shared__ __align__(16) unsigned char dyn[];
-  unsigned char* q_s = dyn;                       // 64 * PITCH
-  unsigned char* qt_s = q_s + 64 * PITCH;         // D * LZM_PT
-  unsigned char* do_s = qt_s + D * LZM_PT;        // 64 * VPITCH
-  unsigned char* dot_s = do_s + 64 * VPITCH;      // DV * LZM_PT
-  float* lse_s = (float*)(dot_s + DV * LZM_PT);   // 64
-  float* del_s = lse_s + 64;                      // 64
-  int* cs_s = (int*)(del_s + 64);                 // 64: window start of the row (INT_MAX: dead row)
+  unsigned char* const q_s = dyn;                               // [NB][64 * PITCH]
+  unsigned char* const do_s = q_s + NB * 64 * PITCH;            // [NB][64 * VPITCH]
+  float* const lse_s = (float*)(do_s + NB * 64 * VPITCH);       // [NB][64]
+  float* const del_s = lse_s + NB * 64;                         // [NB][64]
+  int* const cs_s = (int*)(del_s + NB * 64);                    // [NB][64]: window start of the row (INT_MAX: dead row)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   int kb, hk;
@@ -765,28 +786,25 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
-  uint4 qr[QPASS][2], dor[OPASS][2];
+  typedef unsigned swa_u32x4 __attribute__((ext_vector_type(4)));
+  swa_u32x4 qr[QPASS], dor[OPASS];
   float r_lse = 0.f, r_del = 0.f;
   int r_cs = 2147483647;
   auto fetch = [&](int tile) {
 #pragma unroll
-    for (int i = 0; i < QPASS; ++i)
+    for (int i = 0; i < QPASS; ++i) {
+      const int p = tid + 256 * i, row = p / QSEG;
+      int t = tile * QT + row / G;
+      if (t > L - 1) t = L - 1;
+      qr[i] = *(const swa_u32x4*)(q + ((b * L + t) * (long)dm.HQ + hk * G + row % G) * D + (p % QSEG) * 8);
+    }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 2 * (tid / QSEG + QPPP * i) + h;
-        int t = tile * QT + row / G;
-        if (t > L - 1) t = L - 1;
-        qr[i][h] = *(const uint4*)(q + ((b * L + t) * (long)dm.HQ + hk * G + row % G) * D + (tid % QSEG) * 8);
-      }
-#pragma unroll
-    for (int i = 0; i < OPASS; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int row = 2 * (tid / OSEG + OPPP * i) + h;
-        int t = tile * QT + row / G;
-        if (t > L - 1) t = L - 1;
-        dor[i][h] = *(const uint4*)(d_o + ((b * L + t) * (long)dm.HQ + hk * G + row % G) * DV + (tid % OSEG) * 8);
-      }
+    for (int i = 0; i < OPASS; ++i) {
+      const int p = tid + 256 * i, row = p / OSEG;
+      int t = tile * QT + row / G;
+      if (t > L - 1) t = L - 1;
+      dor[i] = *(const swa_u32x4*)(d_o + ((b * L + t) * (long)dm.HQ + hk * G + row % G) * DV + (p % OSEG) * 8);
+    }
     if (tid < 64) {
       const int t = tile * QT + tid / G;
       const int tc = t < L ? t : L - 1;
@@ -797,18 +815,22 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       r_cs = t < L ? (dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left) : 2147483647;
     }
   };
-  auto stash = [&]() {
+  auto stash = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < QPASS; ++i)
-      lzm_stash_pair<PITCH>(q_s, qt_s, 2 * (tid / QSEG + QPPP * i), tid % QSEG, qr[i][0], qr[i][1]);
+    for (int i = 0; i < QPASS; ++i) {
+      const int p = tid + 256 * i;
+      *(swa_u32x4*)(q_s + (buf * 64 + p / QSEG) * PITCH + (p % QSEG) * 16) = qr[i];
+    }
 #pragma unroll
-    for (int i = 0; i < OPASS; ++i)
-      lzm_stash_pair<VPITCH>(do_s, dot_s, 2 * (tid / OSEG + OPPP * i), tid % OSEG, dor[i][0], dor[i][1]);
+    for (int i = 0; i < OPASS; ++i) {
+      const int p = tid + 256 * i;
+      *(swa_u32x4*)(do_s + (buf * 64 + p / OSEG) * VPITCH + (p % OSEG) * 16) = dor[i];
+    }
     if (tid < 64) {
       const bool live = r_lse > -1e30f;  // rows with an empty window have lse = -inf
-      lse_s[tid] = live ? r_lse * HILS_LOG2E : 0.f;
-      del_s[tid] = r_del;
-      cs_s[tid] = live ? r_cs : 2147483647;
+      lse_s[buf * 64 + tid] = live && r_cs != 2147483647 ? r_lse * HILS_LOG2E : INFINITY;  // (dead: no probability but 0)
+      del_s[buf * 64 + tid] = r_del;
+      cs_s[buf * 64 + tid] = live ? r_cs : 2147483647;
     }
   };
   f32x4_t acck[TT][DT], accv[TT][DVT];
@@ -821,11 +843,12 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
   if (tile0 < n_tiles) {
     fetch(tile0);
-    stash();
+    stash(0);
   }
   __syncthreads();
-  for (int tile = tile0; tile < n_tiles; ++tile) {
+  for (int tile = tile0, buf = 0; tile < n_tiles; ++tile) {
     fetch(tile + 1 < n_tiles ? tile + 1 : tile);
+    const unsigned char *qb = q_s + buf * 64 * PITCH, *db = do_s + buf * 64 * VPITCH;
     float p[TT][4][4], ds[TT][4][4];  // [owned token tile][streamed row tile][row 4j+i]
     {
       f32x4_t st[TT][4], dp[TT][4];
@@ -840,26 +863,41 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       for (int rr = 0; rr < 4; ++rr) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(q_s + (rr * 16 + col) * PITCH + ks * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(qb + (rr * 16 + col) * PITCH + ks * 64 + j * 16);
 #pragma unroll
           for (int tt = 0; tt < TT; ++tt)
             st[tt][rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ka[tt][ks], st[tt][rr], 0, 0, 0);
         }
 #pragma unroll
         for (int vs = 0; vs < VS; ++vs) {
-          const bf16x8_t a = *(const bf16x8_t*)(do_s + (rr * 16 + col) * VPITCH + vs * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(db + (rr * 16 + col) * VPITCH + vs * 64 + j * 16);
 #pragma unroll
           for (int tt = 0; tt < TT; ++tt)
             dp[tt][rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, va[tt][vs], dp[tt][rr], 0, 0, 0);
         }
       }
       const int tq0 = tile * QT;
+      // do all rows of the tile see all tokens of the workgroup?  (wide heads: with two token tiles a wavefront the second
+      // copy of the loop cost more than the masks, 263 instead of 239 us at B8 L8192 16/16 of 64 window 64; rows and tokens past the end, whatever they see, count
+      // for nothing: such rows have no probability but 0, such tokens' sums are not written)
+      const int left = tq0 + QT - dm.window;
+      const bool full = TT == 1 && !dm.mask_lmk && tq0 >= j0 + 64 * TT - 1 && (dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left) <= j0;
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float4 l4 = *(const float4*)&lse_s[rr * 16 + 4 * j];
-        const float4 d4 = *(const float4*)&del_s[rr * 16 + 4 * j];
-        const int4 c4 = *(const int4*)&cs_s[rr * 16 + 4 * j];
+        const float4 l4 = *(const float4*)&lse_s[buf * 64 + rr * 16 + 4 * j];
+        const float4 d4 = *(const float4*)&del_s[buf * 64 + rr * 16 + 4 * j];
         const float ls[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+        if (full) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+              p[tt][rr][i] = __builtin_amdgcn_exp2f(st[tt][rr][i] * c2 - ls[i]);
+              ds[tt][rr][i] = p[tt][rr][i] * (dp[tt][rr][i] - dl[i]);
+            }
+          continue;
+        }
+        const int4 c4 = *(const int4*)&cs_s[buf * 64 + rr * 16 + 4 * j];
         const int cs[4] = {c4.x, c4.y, c4.z, c4.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -872,44 +910,53 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
             const bool vis = (unsigned)(t - tokv[tt]) < span1;
             const float pv = vis ? __builtin_amdgcn_exp2f(st[tt][rr][i] * c2 - ls[i]) : 0.f;
             p[tt][rr][i] = pv;
-            ds[tt][rr][i] = pv * (dp[tt][rr][i] - dl[i]) * dm.sm_scale;
+            ds[tt][rr][i] = pv * (dp[tt][rr][i] - dl[i]);
           }
         }
       }
     }
-    lzm_grad_product<DV, TT>(dot_s, p, accv, col, j);
-    lzm_grad_product<D, TT>(qt_s, ds, acck, col, j);
-    __syncthreads();
-    stash();
+    lzm_grad_product_rows<DV, TT, VPITCH>(db, p, accv, col, j);
+    lzm_grad_product_rows<D, TT, PITCH>(qb, ds, acck, col, j);
+    if (NB == 1) __syncthreads();
+    else buf ^= 1;
+    stash(buf);
     __syncthreads();
   }
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt)  // (the scale of the scores last)
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acck[tt][dt][i] *= dm.sm_scale;
+  // a lane holds four neighbouring features of its tokens
   if (n_split > 1) {
     float* out = part + (((b * dm.H + hk) * n_kb + kb) * (long)n_split + split) * (64 * TT * (D + DV));
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
+    for (int tt = 0; tt < TT; ++tt) {
+      float* row = out + (wave * (16 * TT) + tt * 16 + col) * (D + DV) + 4 * j;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float* row = out + (wave * (16 * TT) + tt * 16 + 4 * j + i) * (D + DV) + col;
+      for (int dt = 0; dt < DT; ++dt) *(f32x4_t*)(row + dt * 16) = acck[tt][dt];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) row[dt * 16] = acck[tt][dt][i];
-#pragma unroll
-        for (int dt = 0; dt < DVT; ++dt) row[D + dt * 16] = accv[tt][dt][i];
-      }
+      for (int dt = 0; dt < DVT; ++dt) *(f32x4_t*)(row + D + dt * 16) = accv[tt][dt];
+    }
     return;
   }
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt)
+  for (int tt = 0; tt < TT; ++tt) {
+    const int tok = tok_w + tt * 16 + col;
+    if (tok >= L) continue;
+    const long row = (b * L + tok) * (long)dm.H + hk;
+    auto put = [](bf16_t* at, const f32x4_t& x) {
+      uint2 y;
+      y.x = pack_bf2(x[0], x[1]);
+      y.y = pack_bf2(x[2], x[3]);
+      *(uint2*)at = y;
+    };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = tok_w + tt * 16 + 4 * j + i;
-      if (tok >= L) continue;
-      bf16_t* outk = dk + ((b * L + tok) * (long)dm.H + hk) * D + col;
-      bf16_t* outv = dv + ((b * L + tok) * (long)dm.H + hk) * DV + col;
+    for (int dt = 0; dt < DT; ++dt) put(dk + row * D + dt * 16 + 4 * j, acck[tt][dt]);
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) outk[dt * 16] = f2bf(acck[tt][dt][i]);
-#pragma unroll
-      for (int dt = 0; dt < DVT; ++dt) outv[dt * 16] = f2bf(accv[tt][dt][i]);
-    }
+    for (int dt = 0; dt < DVT; ++dt) put(dv + row * DV + dt * 16 + 4 * j, accv[tt][dt]);
+  }
 }
 
 // Sum of the shares of swa_bwd_dkdv_mfma, in order; four features per thread, a thread's loads eight at a time (B2 L1024
@@ -1078,8 +1125,7 @@ static int swa_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, con
   const int n_qt = (dm.Lq + QB - 1) / QB;
   hipLaunchKernelGGL((swa_bwd_dq_mfma<D, DV, G>), swa_xcd_grid(n_qt, dm.H, B),
                      dim3(256), 0, st, q, k, v, o, lse, d_o, d_lse, dq, delta, dm, n_qt, B);
-  const size_t smem = (size_t)64 * (D * 2 + 16) + (size_t)D * LZM_PT + (size_t)64 * (DV * 2 + 16) +
-                      (size_t)DV * LZM_PT + 3 * 64 * sizeof(float);
+  const size_t smem = (size_t)swa_dkdv_buffers(D, DV) * 64 * ((D * 2 + 32) + (DV * 2 + 32) + 3 * sizeof(float));
   auto kern = swa_bwd_dkdv_mfma<D, DV, G>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_swa_bwd")) return rc;
