@@ -32,15 +32,19 @@ static dim3 swa_xcd_grid(int n_blk, int H, int B) { return dim3((unsigned)(((lon
 // Forward.  A workgroup of NWV wavefronts owns NWV*32/G consecutive queries of one KV head: 32 score
 // rows (query x head of the group) per wavefront, held as matrix B operands.  The keys and values the
 // block can see (its queries' windows: two or three 64-token tiles at window 64) are loaded once, all
-// loads in flight together, and stay in LDS row-major (rows padded by 16 bytes); a longer window is
+// loads in flight together, and stay in LDS row-major, 16-byte piece p of row r at p ^ (r & pieces - 1), which no read
+// conflicts over (rows 16 bytes apart: 8 cycles a score operand instead of 4); a longer window is
 // worked through in phases of RES resident tiles.  S^T = K Q^T takes K rows as A operands, O += P V takes V
-// through the transposing LDS load, in the token order in which the S^T accumulators hold P.  A
+// through the transposing LDS load, in the token order in which the S^T accumulators hold P.
+// The outputs are formed transposed, O^T += V^T P^T, so that a row's factors, maximum and sum belong to its lanes (no way
+// through LDS) and a lane parks four neighbouring features at a time: with the reads above 64 -> 62 us at B4 L8192 16/16 heads of 64
+// window 64 (about the copy rate), 156 -> 148 at L32768 32/8 of 128, 140 -> 136 at B2 L8192 32/4 of 64 window 512, 13.7 -> 13.0 at L1999 16/2.  A
 // wavefront skips the tiles none of its rows can see and masks only the tiles that straddle a row's
 // window start, its diagonal, the end of the keys or a landmark; running max / sum per row as in
 // flash attention.
-// Two shapes of workgroup.  Wide: eight wavefronts, four resident tiles (139 KiB of LDS at D = Dv =
+// Two shapes of workgroup.  Wide: eight wavefronts, four resident tiles (128 KiB of LDS at D = Dv =
 // 128, one workgroup per compute unit: its load, compute and store phases follow each other with
-// nothing to overlap them).  Narrow: four wavefronts, two resident tiles (70 KiB), two workgroups per
+// nothing to overlap them).  Narrow: four wavefronts, two resident tiles (64 KiB), two workgroups per
 // compute unit, one loading while the other computes; taken when no block of 128/G queries needs more
 // than two tiles (window <= 64 at chunk 64), at the price of every tile being staged by twice as many
 // workgroups (L2 hits).
@@ -60,9 +64,9 @@ static dim3 swa_xcd_grid(int n_blk, int H, int B) { return dim3((unsigned)(((lon
 
 template <int D, int DV, int NWV, int RES>
 static size_t swa_fwd_smem() {
-  const size_t tiles = (size_t)RES * 64 * ((2 * D + 16) + (2 * DV + 16));
+  const size_t tiles = (size_t)RES * 64 * (2 * D + 2 * DV);
   const size_t outs = (size_t)NWV * 16 * SWA_FWD_RT * (2 * DV + 16);
-  return (tiles > outs ? tiles : outs) + (size_t)NWV * SWA_FWD_RT * 16 * sizeof(float);
+  return tiles > outs ? tiles : outs;
 }
 
 template <int D, int DV, int G, int NWV, int RES, int SPLIT>
@@ -75,7 +79,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
   constexpr int NRG = NWV / SPLIT;                       // wavefronts with rows of their own
   constexpr int QB = NRG * 16 * RT / G;                  // queries per workgroup
   static_assert(SPLIT == 1 || (SPLIT == 2 && RES == 4), "a phase's two tiles go to the two wavefronts with the same rows");
-  constexpr int KP = D * 2 + 16, VP = DV * 2 + 16;       // bytes per staged row
+  constexpr int KP = D * 2, VP = DV * 2;                 // bytes per staged row; piece p of row r lies at p ^ (r & SEG - 1)
   constexpr int KSEG = D / 8, VSEG = DV / 8;
   constexpr int KPT = 64 * KSEG / NT, VPT = 64 * VSEG / NT;  // 16-byte pieces per thread and tile
   static_assert(KPT >= 1 && VPT >= 1 && KPT * NT == 64 * KSEG && VPT * NT == 64 * VSEG,
@@ -87,14 +91,11 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
   typedef short swa_s8 __attribute__((ext_vector_type(8)));
   extern __shared__ __align__(16) unsigned char swa_dyn[];
   constexpr size_t TILES_B = (size_t)RES * TILE_B;
-  constexpr size_t OUTS_B = (size_t)NRG * 16 * RT * OP;
-  float* bc_all = (float*)(swa_dyn + (TILES_B > OUTS_B ? TILES_B : OUTS_B));  // [wave][rt][16] row factors
   const int tid = threadIdx.x, lane = tid & 63;
   // in a scalar register: what is derived from it (the wavefront's key range, "does this tile need
   // masks") then steers scalar branches instead of lane masks
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, j = lane >> 4;
-  float* bc_s = bc_all + wave * RT * 16;
   int qt, hk;
   long b;
   if (!swa_xcd_unit(n_qt, dm.H, n_b, qt, hk, b)) return;
@@ -171,10 +172,21 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
     l_run[rt] = 0.f;
   }
 
+  // this lane's places in a tile: a row's piece of the scores' k-step, a 4 x 4 block's share of V's columns
+  unsigned k_off[KS], v_off[DT];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) k_off[ks] = (unsigned)(col * KP + ((ks * 4 + j) ^ (col & (KSEG - 1))) * 16);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    const int row = 4 * j + (col >> 2);
+    v_off[dt] = (unsigned)(row * VP + ((dt * 2 + (col >> 1 & 1)) ^ (row & (VSEG - 1))) * 16 + (col & 1) * 8);
+  }
+
   // one resident tile: scores, masks where a row needs them, running softmax, O += P V
   auto tile_step = [&](int tile, const unsigned char* k_s, const unsigned char* v_s) __attribute__((always_inline)) {
     f32x4_t p[RT][4];  // scores, then probabilities: accumulator tiles (token tt*16 + 4j + i, row lane & 15)
     bool rescale = false;
+    float corr[RT];
     {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
@@ -184,7 +196,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(k_s + (tt * 16 + col) * KP + ks * 64 + j * 16);
+          const bf16x8_t a = *(const bf16x8_t*)(k_s + k_off[ks] + tt * 16 * KP);
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
             p[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], p[rt][tt], 0, 0, 0);
@@ -235,9 +247,9 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
         const bool move = fresh | ((mx - m_run[rt]) * c2 > SWA_LAZY);
         const float m_new = move ? fmaxf(m_run[rt], mx) : m_run[rt];
         const bool any = m_new > HILS_NEG_INF;
-        const float corr = (move & any & !fresh) ? __builtin_amdgcn_exp2f((m_run[rt] - m_new) * c2) : 1.f;
+        corr[rt] = (move & any & !fresh) ? __builtin_amdgcn_exp2f((m_run[rt] - m_new) * c2) : 1.f;
         const float mc = any ? m_new * c2 : 0.f;
-        rescale |= corr != 1.f;
+        rescale |= corr[rt] != 1.f;
         float sum = 0.f;
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
@@ -248,29 +260,21 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
             sum += e;
           }
         sum = rows_sum(sum);
-        l_run[rt] = l_run[rt] * corr + sum;
+        l_run[rt] = l_run[rt] * corr[rt] + sum;
         m_run[rt] = m_new;
-        if (j == 0) bc_s[rt * 16 + col] = corr;
       }
     }
-    __builtin_amdgcn_wave_barrier();
-    // rescale the output accumulators: their rows are 4j+i, the factors live per lane & 15
     if (__any(rescale)) {
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const float4 c4 = *(const float4*)&bc_s[rt * 16 + 4 * j];
-        const float cf[4] = {c4.x, c4.y, c4.z, c4.w};
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[rt][dt][i] *= cf[i];
-      }
+          for (int i = 0; i < 4; ++i) acc[rt][dt][i] *= corr[rt];
     }
-    __builtin_amdgcn_wave_barrier();
-    // O += P V: a lane's eight k-slots are tokens 4j..4j+3 of two neighbouring 16-token tiles; the
+    // O^T += V^T P^T (a lane's accumulators are its row's features 16 dt + 4j + i): a lane's eight k-slots are tokens 4j..4j+3 of two neighbouring 16-token tiles; the
     // transposing load (a 16-lane group addresses a 4 x 16 block, lane l row l/4 and columns 4(l%4)..,
     // and receives column l of it) delivers V in that order
-    const unsigned char* t_addr = v_s + (4 * j + (col >> 2)) * VP + (col & 3) * 8;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       bf16x8_t a[RT];
@@ -285,13 +289,13 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const unsigned char* p0 = t_addr + (2 * h * 16) * VP + dt * 32;
+        const unsigned char* p0 = v_s + v_off[dt] + (2 * h * 16) * VP;
         const swa_s4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) swa_s4*)p0);
         const swa_s4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) swa_s4*)(p0 + 16 * VP));
         const swa_s8 bb = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
-          acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], __builtin_bit_cast(bf16x8_t, bb), acc[rt][dt], 0, 0, 0);
+          acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bb), a[rt], acc[rt][dt], 0, 0, 0);
         if ((dt & 3) == 3) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -320,12 +324,12 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
       const int pc = tid + NT * i;
-      *(swa_u32x4*)(k_s + (pc / KSEG) * KP + (pc % KSEG) * 16) = kd[i];
+      *(swa_u32x4*)(k_s + (pc / KSEG) * KP + ((pc % KSEG) ^ (pc / KSEG & (KSEG - 1))) * 16) = kd[i];
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int pc = tid + NT * i;
-      *(swa_u32x4*)(v_s + (pc / VSEG) * VP + (pc % VSEG) * 16) = vd[i];
+      *(swa_u32x4*)(v_s + (pc / VSEG) * VP + ((pc % VSEG) ^ (pc / VSEG & (VSEG - 1))) * 16) = vd[i];
     }
   };
   swa_u32x4 kr[2][KPT], vr[2][VPT];  // two tiles' loads in flight
@@ -387,7 +391,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
     // barrier lies behind the tiles' last use)
     f32x4_t* xch = (f32x4_t*)swa_dyn;
     constexpr int XR = RT * DT + 1;
-    static_assert((size_t)NRG * XR * 64 * 16 <= TILES_B, "the exchange fits the tiles");
+    static_assert((size_t)NRG * XR * 64 * 16 <= (size_t)RES * TILE_B, "the exchange fits the tiles");
     if (share) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
@@ -409,35 +413,20 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
         fb[rt] = any ? __builtin_amdgcn_exp2f((m2 - M) * c2) : 1.f;
         m_run[rt] = M;
         l_run[rt] = l_run[rt] * fa[rt] + l2 * fb[rt];
-        if (j == 0) bc_s[rt * 16 + col] = fa[rt];
       }
-      __builtin_amdgcn_wave_barrier();
-      f32x4_t ca[RT], cb[RT];  // ... of the accumulators' rows 4j + i
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) ca[rt] = *(const f32x4_t*)&bc_s[rt * 16 + 4 * j];
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        if (j == 0) bc_s[rt * 16 + col] = fb[rt];
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) cb[rt] = *(const f32x4_t*)&bc_s[rt * 16 + 4 * j];
-      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const f32x4_t x = xch[(rg * XR + rt * DT + dt) * 64 + lane];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[rt][dt][i] = acc[rt][dt][i] * ca[rt][i] + x[i] * cb[rt][i];
+          for (int i = 0; i < 4; ++i) acc[rt][dt][i] = acc[rt][dt][i] * fa[rt] + x[i] * fb[rt];
         }
     }
   }
   // ---- finalize: o = acc / l, lse = ln(l) + max * scale ----
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    const float inv = l_run[rt] > 0.f ? 1.f / l_run[rt] : 0.f;
-    if (j == 0) bc_s[rt * 16 + col] = inv;
     const int row = rt * 16 + col;
     const int t = t0 + row / G, g = row % G;
     if (j == 0 && t < dm.Lq && share == 0)
@@ -451,13 +440,14 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
   unsigned char* ob = swa_dyn + (size_t)rg * (16 * RT) * OP;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    const float4 c4 = *(const float4*)&bc_s[rt * 16 + 4 * j];
-    const float cf[4] = {c4.x, c4.y, c4.z, c4.w};
+    const float inv = l_run[rt] > 0.f ? 1.f / l_run[rt] : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-        *(bf16_t*)(ob + (rt * 16 + 4 * j + i) * OP + (dt * 16 + col) * 2) = f2bf(acc[rt][dt][i] * cf[i]);
+    for (int dt = 0; dt < DT; ++dt) {
+      uint2 x;
+      x.x = pack_bf2(acc[rt][dt][0] * inv, acc[rt][dt][1] * inv);
+      x.y = pack_bf2(acc[rt][dt][2] * inv, acc[rt][dt][3] * inv);
+      *(uint2*)(ob + (rt * 16 + col) * OP + dt * 32 + j * 8) = x;
+    }
   }
   __builtin_amdgcn_wave_barrier();
   constexpr int OSEG = DV / 8;
