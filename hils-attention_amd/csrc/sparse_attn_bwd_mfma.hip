@@ -326,8 +326,10 @@ bw_dkdv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const
   constexpr int TT = bw_tt(D, DV);            // 16-token tiles of a wavefront
   constexpr int ROWS = 32 * TT;               // rows staged per round: 32 for each wavefront with the same tokens
   constexpr int PPR = ROWS / G;               // pairs per round
-  constexpr int QROW = D * 2 + 16;            // staging: padded row (bytes)
-  constexpr int OROW = DV * 2 + 16;
+  // staging: padded row (bytes).  32 bytes: the 16-byte reads of 16 rows take 4 cycles, 8 with 16 (dK/dV at L32768 32/8 heads
+  // of 128 4264 -> 3749 us, L8192 32/4 of 128 850 -> 768, B2 L8192 32/4 of 64 712 -> 688)
+  constexpr int QROW = D * 2 + 32;
+  constexpr int OROW = DV * 2 + 32;
   constexpr int BUF = ROWS * (QROW + OROW) + 3 * ROWS * 4;  // one staging buffer (bytes)
   extern __shared__ __attribute__((aligned(16))) char bw_smem[];  // two staging buffers
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1027,7 +1029,9 @@ bw_dq_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ d_o, const
 #pragma unroll
         for (int u = 0; u < 4 * VS; ++u) ya[u] = *(const bw_u4*)(va_c + u * 512);
       }
-      if (KEEP && p + QT < ve) load_rows(p + QT, nx);
+      // (with staged rows always, a visit's last tile its own again: behind a branch the wait for these loads is one for the
+      // next tile's too; B2 L8192 32/4 heads of 64 711 -> 664 us.  With gathered rows they cost more, 138 -> 144 at L8192 16/8)
+      if (KEEP && (STAGE || p + QT < ve)) load_rows(p + QT < ve ? p + QT : p, nx);
       if (STAGE) {
         const unsigned row_l = (x.pk >> 8) * G + g;
 #pragma unroll
@@ -1297,7 +1301,7 @@ static int bw_launch_dkdv(int G, dim3 grid, hipStream_t st, const bf16_t* q, con
     hipLaunchKernelGGL(kern, grid, dim3(256), smem, st, q, k, v, w, lse, delta, d_o, offsets, pairs, dk, dv, dm); \
   } while (0)
   constexpr size_t ROWS = 32 * bw_tt(D, DV);
-  const size_t smem = 2 * (ROWS * (D * 2 + 16) + ROWS * (DV * 2 + 16) + 3 * ROWS * sizeof(float));  // two staging buffers
+  const size_t smem = 2 * (ROWS * (D * 2 + 32) + ROWS * (DV * 2 + 32) + 3 * ROWS * sizeof(float));  // two staging buffers
   switch (G) {
     case 1: BW_CALL(1); break;
     case 2: BW_CALL(2); break;
