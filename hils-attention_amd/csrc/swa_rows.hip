@@ -2,7 +2,7 @@
 //
 // The tile kernel (swa.hip) gives a workgroup 128 or 256 score rows and walks the window tile by tile:
 // with a single query per sequence most of those rows are padding and the walk over a window of 512 is a
-// serial chain of phases (19 us for one sequence, 33 us for 64 (sequence, KV head) pairs of heads of 128).
+// serial chain of phases (13 us for one sequence of heads of 64, 18 us for 64 (sequence, KV head) pairs of heads of 128).
 // Here a workgroup owns 16 score rows (16/G queries times the G heads of a KV head: the 16 columns of the
 // matrix instructions) and its eight wavefronts share the WINDOW: units of 32 tokens go round-robin, the
 // next unit's K and V loads are in flight while one is worked on, and the eight partial results
@@ -12,6 +12,13 @@
 // row); V is staged row-major in the wavefront's own LDS area and read by the transposing LDS load as the
 // A operand of O^T += V^T P, in the token order in which the S^T accumulators hold P.  Rows are matrix
 // columns in both products, so maxima, sums and the rescaling of the accumulators stay in their lanes.
+//
+// With few rows a compute unit's share of the memory system bounds it: all of a row's keys and values are asked for at
+// once, 128 KB (heads of 64, window 512) arrive in about 3.5 us.  What a unit of 32 tokens computes comes on top, three
+// of them in series, so it must not branch: 0.4 us a unit, where masks tested score by score took 1.0 (the kernel in a
+// row of launches, 1 / 64 / 256 workgroups: heads of 64 6.2 / 6.8 / 7.5 -> 5.6 / 5.9 / 6.4 us, of 128 10.2 / 11.4 /
+// 14.3 -> 9.1 / 10.1 / 13.3).  Loads through buffer descriptors with the next unit asked for between its scores and its
+// softmax were slower (8.0 against 7.4 us at 64 workgroups): the loads past the end take their turn in the queue too.
 #include "stream_tiles.h"
 #include "swa_dims.h"
 
@@ -21,7 +28,7 @@
 template <int D, int DV>
 __global__ void __launch_bounds__(SR_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
-             bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int G, int n_rb) {
+             bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int g_bits) {
   constexpr int KS = D / 32, MT = DV / 16;
   constexpr int VL = DV / 8, TPI = 64 / VL, VI = SR_UNIT / TPI;  // lanes per V row, rows per load, loads per unit
   constexpr int VP = 2 * DV + 16;                                // bytes of a staged V row
@@ -35,15 +42,14 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, j = lane >> 4;
-  const int rb = blockIdx.x % n_rb;
-  const int hk = (blockIdx.x / n_rb) % dm.H;
-  const long b = blockIdx.x / n_rb / dm.H;
-  const int QB = 16 / G;
-  const int tq0 = rb * QB;
+  const int G = 1 << g_bits, QB = 16 >> g_bits;  // (no division: one is tens of instructions before the first load)
+  const int tq0 = blockIdx.x * QB;
+  const int hk = blockIdx.y;
+  const long b = blockIdx.z;
   const int q_off = dm.kv_start + dm.Lk - dm.Lq;  // absolute position of query 0
 
   // this lane's row and the key positions it sees, [vlo, vlo + vspan] (a start no position reaches: none)
-  const int t = tq0 + col / G, g = col % G;
+  const int t = tq0 + (col >> g_bits), g = col & (G - 1);
   const bool live = t < dm.Lq;
   const int tc = live ? t : dm.Lq - 1;
   bf16x8_t qb[KS];
@@ -54,7 +60,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   }
   auto win_start = [&](int tt) -> int {  // first absolute position query tt sees
     const int left = q_off + tt - dm.window + 1;
-    return dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left;
+    return !dm.expand ? left : dm.chunk_pow2 ? left & -dm.chunk : floordiv(left, dm.chunk) * dm.chunk;
   };
   int vlo;
   unsigned vspan;
@@ -116,19 +122,34 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
     }
     const int tok_raw0 = lo + u * SR_UNIT + 4 * j;
     const unsigned base = (unsigned)(dm.kv_start + tok_raw0 - vlo);
+    // (positions end at the last key's, so the end of the keys needs no test of its own; the options are decided once
+    // a unit: tested per element they made some twenty branches of it, 1.0 us against 0.5)
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[tt][i] = base + (unsigned)(tt * 16 + i) <= vspan ? S[tt][i] : HILS_NEG_INF;
+    if (dm.mask_lmk) {
+      const int ta = dm.kv_start + tok_raw0 + 1;
+      if (dm.chunk_pow2) {
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[tt][i] = ((ta + tt * 16 + i) & (dm.chunk - 1)) ? S[tt][i] : HILS_NEG_INF;
+      } else {
+#pragma unroll 1
+        for (int e = 0; e < 8; ++e) {  // (rolled: the divisions would be most of the kernel's code)
+          const int i = e & 3;
+          const bool lm = (ta + (e >> 2) * 16 + i) % dm.chunk == 0;
+#pragma unroll
+          for (int x = 0; x < 8; ++x) S[x >> 2][x & 3] = lm && x == e ? HILS_NEG_INF : S[x >> 2][x & 3];
+        }
+      }
+    }
     float mx = HILS_NEG_INF;
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bool see = base + (unsigned)(tt * 16 + i) <= vspan && tok_raw0 + tt * 16 + i < dm.Lk;
-        if (dm.mask_lmk) {  // uniform
-          const int ta = dm.kv_start + tok_raw0 + tt * 16 + i + 1;
-          see = see && (dm.chunk_pow2 ? (ta & (dm.chunk - 1)) : ta % dm.chunk) != 0;
-        }
-        S[tt][i] = see ? S[tt][i] : HILS_NEG_INF;
-        mx = fmaxf(mx, S[tt][i]);
-      }
+      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, S[tt][i]);
     mx = rows_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const bool any = m_new > HILS_NEG_INF;
@@ -191,7 +212,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   // 16 rows x DV/4 pieces of four features over the workgroup
   for (int p = tid; p < 16 * (DV / 4); p += SR_WAVES * 64) {
     const int row = p / (DV / 4), d4 = p % (DV / 4);
-    const int tr = tq0 + row / G;
+    const int tr = tq0 + (row >> g_bits);
     if (tr >= dm.Lq) continue;
     float M = HILS_NEG_INF;
 #pragma unroll
@@ -208,7 +229,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
       for (int i = 0; i < 4; ++i) x[i] = fmaf(f, ow[i], x[i]);
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    const long rix = (b * dm.Lq + tr) * (long)dm.HQ + hk * G + row % G;
+    const long rix = (b * dm.Lq + tr) * (long)dm.HQ + hk * G + (row & (G - 1));
     uint2 pk;
     pk.x = pack_bf2(x[0] * inv, x[1] * inv);
     pk.y = pack_bf2(x[2] * inv, x[3] * inv);
@@ -217,24 +238,32 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   }
 }
 
-// While the row kernel's workgroups fit two rounds of the chip it is ahead of the tile kernel, whose few
-// workgroups walk the window in series (window 512, row / tile kernel: heads of 64 7 / 19 us with one
-// workgroup, 8 / 25 us at 256, 12 / 25 at 512, 20 / 25 at 1024, 36 / 26 at 2048; heads of 128 10 / 24,
-// 12 / 31, 22 / 32, 41 / 32).  Window 64: 7 / 9 up to 512 workgroups, about even at 1024 with heads of 64.
+// The tile kernel gives a workgroup 128 or 256 score rows of a KV head, the row kernel 16.  With one or two row blocks
+// a (sequence, KV head) the tile kernel's workgroups are mostly padding and walk the window in series; with more,
+// every row block reads the window again.  Row / tile kernel in us, 256, 512, 1024, 2048 workgroups of the row kernel:
+//   one block:   heads of 64, window 512  6.8/14  13/38  25/73  67/149;  window 64  5.6/5.5  5.7/5.8  7.3/9.3  13/15
+//                heads of 128, 512  13/21  25/52  47/102  112/224;  256  9/12  17/30  31/57  71/125;
+//                128  5.6/7.7  11/10  20/22  38/38;  64  5.8/5.8  7.6/7.1  15/13  28/25
+//   two blocks:  heads of 64, 512  7.8/15  15/17  26/41  49/79;  256  5.4/11  9/11  17/25  31/49;  128  5.5/8.5  7/9  13/10  23/21
+//   eight:       heads of 64 (16 queries of eight heads), 512  -  15/15  27/16  48/18;  64  -  5.6/6.7  10/7  18/7
+//   four:        heads of 128 (16 queries of four heads), 512  15/21  27/23  52/25;  64  5.6/8.2  11/8  21/9
 bool hils_swa_rows_better(int B, int D, int Dv, const SwaDims& dm) {
+  if (B > 65535 || dm.H > 65535) return false;  // (dimensions of the row kernel's grid)
   const int QB = 16 / (dm.HQ / dm.H);
-  const long wgs = (long)((dm.Lq + QB - 1) / QB) * dm.H * B;
-  return wgs <= 512 || (wgs <= 1024 && D <= 64 && Dv <= 64 && dm.window >= 256);
+  const long n_rb = (dm.Lq + QB - 1) / QB, wgs = n_rb * dm.H * B;
+  const bool narrow = D <= 64 && Dv <= 64;
+  if (wgs <= (narrow ? 512 : 256)) return true;
+  return dm.window >= 256 ? n_rb <= (narrow ? 2 : 1) : narrow && n_rb == 1;
 }
 
 int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int D,
                       int Dv, const SwaDims& dm) {
   const int G = dm.HQ / dm.H;
-  const int n_rb = (dm.Lq + 16 / G - 1) / (16 / G);
-  const dim3 grid((unsigned)((long)n_rb * dm.H * B)), wg(SR_WAVES * 64);
+  const int n_rb = (dm.Lq + 16 / G - 1) / (16 / G), g_bits = __builtin_ctz(G);
+  const dim3 grid(n_rb, dm.H, B), wg(SR_WAVES * 64);
 #define SR_CALL(D_, V_)                                                                                     \
   hipLaunchKernelGGL((swa_fwd_rows<D_, V_>), grid, wg, 0, st, (const bf16_t*)q, (const bf16_t*)k,            \
-                     (const bf16_t*)v, (bf16_t*)o, lse, dm, G, n_rb)
+                     (const bf16_t*)v, (bf16_t*)o, lse, dm, g_bits)
   if (D == 64 && Dv == 64) SR_CALL(64, 64);
   else if (D == 128 && Dv == 128) SR_CALL(128, 128);
   else if (D == 64) SR_CALL(64, 128);

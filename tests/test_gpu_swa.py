@@ -46,6 +46,18 @@ def test_swa_few_blocks(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, kw):
     run(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, **kw)
 
 
+# few queries a sequence (the row kernel): chunks that are no power of two, cut caches, windows of one to three units a
+# wavefront, and counts of row blocks on either side of where the tile kernel takes over
+@pytest.mark.parametrize("B,Lq,Lk,HQ,H,D,Dv,W,S,kw", [
+    (1, 1, 700, 16, 2, 64, 64, 512, 48, {}), (2, 3, 200, 16, 2, 64, 128, 100, 20, {"expand": False, "kv_start": 37}),
+    (3, 1, 577, 32, 8, 128, 128, 512, 64, {"mask_lmk": False}), (1, 2, 40, 16, 1, 128, 64, 512, 64, {"kv_start": 1000}),
+    (66, 1, 130, 32, 16, 64, 64, 100, 64, {}), (65, 8, 300, 16, 8, 64, 64, 256, 64, {}),
+    (65, 9, 300, 16, 8, 64, 64, 256, 64, {}), (33, 1, 290, 32, 16, 128, 128, 256, 64, {}),
+    (33, 1, 290, 32, 16, 128, 128, 255, 64, {}), (17, 5, 90, 64, 16, 128, 64, 64, 16, {})])
+def test_swa_few_rows(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, kw):
+    run(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, **kw)
+
+
 def test_swa_mask_variants(pkg, orc, dev):
     for mask_lmk in (False, True):
         for expand in (False, True):
