@@ -1447,20 +1447,61 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
   TopkRowSharedT<GMAX>& sh = FUSED ? *sh_p : sh_own;  // FUSED: the caller's, which the attention reads after the return
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int piece = lane % LR, tsub = lane / LR;
-  const int hk = (int)(row % h_kv);
-  const long bt = row / h_kv;
-  const int t = (int)(bt % L);
-  const long b = bt / L;
+  const unsigned row_u = (unsigned)row;  // (below 2^31, a grid's dimension: the divisions are of 32 bits)
+  const int hk = (int)(row_u % (unsigned)h_kv);
+  const unsigned bt_u = row_u / (unsigned)h_kv;
+  const int t = (int)(bt_u % (unsigned)L);
+  const long b = bt_u / (unsigned)L;
   int lim = causal ? visible_limit(t + q_offset, window_size, block_size) : N;
   lim = lim < 0 ? 0 : (lim > N ? N : lim);
   float swa[GMAX];
 #pragma unroll
   for (int g = 0; g < GMAX; ++g) swa[g] = (g < G) ? lse_swa[row * G + g] : 0.f;
-  if (tid == 0) {
-    sh.next_group = 2 * NW;
-    if (FUSED) {
+  if (tid == 0) sh.next_group = 2 * NW;
+  typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
+  // key groups of the row: KG chunks each, times the G heads when every query head has its own keys
+  // (group number = chunk group * G + head: the heads of a chunk are neighbours in memory)
+  const int GK = perq ? G : 1;                  // key tensors of the row
+  const int h_lmk = h_kv * GK;                  // heads of the key tensor
+  const int ngroups = ((lim + KG - 1) / KG) * GK;
+  // dense chunk keys: (B, N, h_lmk, D), or head-major (B, h_lmk, lmk_cap, D) (a row's keys contiguous)
+  const bf16_t* base = lmks + (lmk_hm ? (b * h_lmk + hk * GK) * (long)lmk_cap * D : (b * N * (long)h_lmk + hk * GK) * D) + piece * 8;
+  const long cstride = (PAGED || !lmk_hm) ? (long)h_lmk * D : (long)D;
+  const long gstride = (!PAGED && lmk_hm) ? (long)lmk_cap * D : (long)D;  // from a head to the next of the group
+  const bf16_t* pbase = lmks + (long)hk * GK * D + piece * 8;  // paged: + page * h_lmk * D
+  auto fetch = [&](tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
+    const int grp = perq ? vg / G : vg;
+    const long goff = perq ? (vg - grp * G) * gstride : 0;
 #pragma unroll
-      for (int g = 0; g < GMAX; ++g) sh.swa[g] = swa[g];
+    for (int it = 0; it < GI; ++it) {
+      int c = grp * KG + it * TPI + tsub;
+      c = c < N ? c : N - 1;
+      if (PAGED) {
+        const int pg = page_s[c];  // an unmapped or invisible chunk reads page 0 and is masked below
+        kr[it] = *(const tr_u4*)(pbase + goff + (long)(pg < 0 ? 0 : pg) * cstride);
+      } else {
+        kr[it] = *(const tr_u4*)(base + goff + c * cstride);
+      }
+    }
+  };
+  // drawn group numbers only grow (the first two of a wavefront are wave and wave + NW), `last` stands in for one past the end
+  const int last = ngroups - 1;
+  tr_u4 ka[GI], kb[GI];
+  int ga = wave, gb = wave + NW;
+  // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
+  // features ks*32 + 8j ..
+  bf16x8_t qb[D / 32];
+  if constexpr (!PRE) {
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) {
+      tr_u4 t = {0u, 0u, 0u, 0u};
+      if ((lane & 15) < G) t = *(const tr_u4*)(q + (row * (long)G + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8);
+      qb[ks] = __builtin_bit_cast(bf16x8_t, t);
+    }
+    // the first keys are on their way before the bias is staged and the queries have arrived (page ids come first)
+    if (!PAGED && ngroups > 0) {
+      fetch(ka, ga < last ? ga : last);
+      fetch(kb, gb < last ? gb : last);
     }
   }
   // PRE: the wavefronts share out the heads' rows, four pieces a lane in flight at once (of up to NP / 4 a row), issued ahead
@@ -1520,6 +1561,10 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       for (int g = 0; g < GMAX; ++g) bias_s[g * NP + c] = bv[g];
     }
   }
+  if (FUSED && tid == 0) {  // (behind the other loads' issue: a store here waits for a latency of memory)
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g) sh.swa[g] = swa[g];
+  }
   if constexpr (PRE) {
     if (inplace) __syncthreads();  // the bias is in the logits' places
     const int ngroups = (lim + KG - 1) / KG;
@@ -1546,16 +1591,6 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       sh.grp_l[i / GMAX][i % GMAX] = i == tid ? pl : pre_l[i];
     }
   } else {
-  // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
-  // features ks*32 + 8j ..; loaded here so that the barrier below has waited for them
-  typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
-  bf16x8_t qb[D / 32];
-#pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    tr_u4 t = {0u, 0u, 0u, 0u};
-    if ((lane & 15) < G) t = *(const tr_u4*)(q + (row * (long)G + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8);
-    qb[ks] = __builtin_bit_cast(bf16x8_t, t);
-  }
   // have them arrive here: a load still pending at the streaming loop's first use would make the
   // compiler wait for every load in flight there, in every iteration
 #pragma unroll
@@ -1566,7 +1601,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       page_s[c] = (pg >= 0 && pg < num_pages) ? pg : -1;
     }
   }
-  __syncthreads();
+  lds_barrier();  // (no wait for the keys in flight)
 
   // ---- phase 1: logits of the visible chunks.  The chunk-key rows arrive by coalesced 16-byte lane
   // loads (LR lanes per row), are written row-major (rows padded by 16 bytes: no bank conflicts
@@ -1581,31 +1616,6 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     const int col = lane & 15, j = lane >> 4;
     char* const w_addr = stage_w + tsub * ROWB + piece * 16;
     const char* const k_addr = stage_w + col * ROWB + j * 16;
-    // key groups of the row: KG chunks each, times the G heads when every query head has its own keys
-    // (group number = chunk group * G + head: the heads of a chunk are neighbours in memory)
-    const int GK = perq ? G : 1;                  // key tensors of the row
-    const int h_lmk = h_kv * GK;                  // heads of the key tensor
-    const int ngroups = ((lim + KG - 1) / KG) * GK;
-    // dense chunk keys: (B, N, h_lmk, D), or head-major (B, h_lmk, lmk_cap, D) (a row's keys contiguous)
-    const bf16_t* base = lmks + (lmk_hm ? (b * h_lmk + hk * GK) * (long)lmk_cap * D : (b * N * (long)h_lmk + hk * GK) * D) + piece * 8;
-    const long cstride = (PAGED || !lmk_hm) ? (long)h_lmk * D : (long)D;
-    const long gstride = (!PAGED && lmk_hm) ? (long)lmk_cap * D : (long)D;  // from a head to the next of the group
-    const bf16_t* pbase = lmks + (long)hk * GK * D + piece * 8;  // paged: + page * h_lmk * D
-    auto fetch = [&](tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
-      const int grp = perq ? vg / G : vg;
-      const long goff = perq ? (vg - grp * G) * gstride : 0;
-#pragma unroll
-      for (int it = 0; it < GI; ++it) {
-        int c = grp * KG + it * TPI + tsub;
-        c = c < N ? c : N - 1;
-        if (PAGED) {
-          const int pg = page_s[c];  // an unmapped or invisible chunk reads page 0 and is masked below
-          kr[it] = *(const tr_u4*)(pbase + goff + (long)(pg < 0 ? 0 : pg) * cstride);
-        } else {
-          kr[it] = *(const tr_u4*)(base + goff + c * cstride);
-        }
-      }
-    };
     auto consume = [&](const tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
       const int grp = perq ? vg / G : vg;
       const int gh = perq ? vg - grp * G : -1;  // the head these keys belong to (-1: to all heads)
@@ -1673,10 +1683,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       return __builtin_amdgcn_readfirstlane(v);
     };
     // drawn group numbers only grow, so the first one past the end ends the wavefront's walk
-    const int last = ngroups - 1;
-    tr_u4 ka[GI], kb[GI];
-    int ga = wave, gb = wave + NW;
-    if (ngroups > 0) {
+    if (PAGED && ngroups > 0) {
       fetch(ka, ga < last ? ga : last);
       fetch(kb, gb < last ? gb : last);
     }
@@ -2043,8 +2050,8 @@ __device__ __forceinline__ void topk_step_weights(const DsArgs& a, TopkRowShared
   const bool has = lane < win.nc;
   if (wave == DS_WAVES - 1 && write_out && lane < topk) a.indices[row * topk + lane] = has ? widx : -1;
   if (wave >= G) return;
-  const int g = wave, hk = (int)(row % a.h_kv);
-  const long b = row / a.h_kv / a.L;
+  const int g = wave, hk = (int)((unsigned)row % (unsigned)a.h_kv);
+  const long b = (unsigned)row / (unsigned)a.h_kv / (unsigned)a.L;
   const float* logit_s = dyn;
   const int* page_s = (const int*)(dyn + (size_t)(GMAX + 1) * NP);
   float bw = 0.f;
@@ -2106,8 +2113,8 @@ template <int D, bool PAGED, int GMAX>
 __device__ __forceinline__ void decode_step_attend(const DsArgs& a, TopkRowSharedT<GMAX>& sh, float* dyn,
                                                    const long row, const TopkWinners& win, int split,
                                                    const bool write_out) {
-  const int hk = (int)(row % a.h_kv);
-  const long bt = row / a.h_kv;
+  const int hk = (int)((unsigned)row % (unsigned)a.h_kv);
+  const long bt = (unsigned)row / (unsigned)a.h_kv;
   const bf16_t* w_row = sh.win_w - (bt * a.dr.HQ + hk * a.G) * (long)a.dr.NW;
   const int32_t* i_row = sh.win_i - (bt * a.dr.H + hk) * (long)a.dr.K;
   decode_rows_body<D, DS_WAVES, true>(a.q, a.k, a.v, w_row, i_row, a.o, a.partial, a.dr, (char*)dyn, split, hk, bt,
@@ -2161,9 +2168,10 @@ __global__ void __launch_bounds__(256) decode_logits_kernel(DsArgs a) {
   const int col = lane & 15, j = lane >> 4, piece = lane % LR, tsub = lane / LR;
   const long row = blockIdx.y;
   if (blockIdx.x == 0 && threadIdx.x == 0) a.arrived[row] = 0;
-  const int hk = (int)(row % a.h_kv);
-  const long bt = row / a.h_kv, b = bt / a.L;
-  const int t = (int)(bt % a.L), G = a.G, N = a.N, NP = a.NP;
+  const int hk = (int)((unsigned)row % (unsigned)a.h_kv);
+  const unsigned bt = (unsigned)row / (unsigned)a.h_kv;
+  const long b = bt / (unsigned)a.L;
+  const int t = (int)(bt % (unsigned)a.L), G = a.G, N = a.N, NP = a.NP;
   int lim = visible_limit(t + a.q_offset, a.window_size, a.block_size);
   lim = lim < 0 ? 0 : (lim > N ? N : lim);
   const int GK = a.perq ? G : 1, h_lmk = a.h_kv * GK;
@@ -2193,17 +2201,26 @@ __global__ void __launch_bounds__(256) decode_logits_kernel(DsArgs a) {
   const char* const k_addr = stage_w + col * ROWB + j * 16;
   float* logits = a.pre_logits + row * (long)GMAX * NP;
   const bool mine = col < G && (gh < 0 || col == gh);
+  // the biases are asked for along with the keys (tile by tile each tile waited a latency of memory for its own)
+  constexpr int TT = GI / LPT;
+  f32x4_t bias_r[TT];
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) bias_r[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (a.bias) {
+    const float* bp = a.bias + (a.lmk_hm ? (b * a.h_kv + hk) * (long)a.lmk_cap : b * N * (long)a.h_kv + hk) * G + (mine ? col : 0);
+    const long bs = (a.lmk_hm ? 1L : (long)a.h_kv) * G;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = grp * KG + tt * 16 + 4 * j + i;
+        bias_r[tt][i] = bp[(c < lim ? c : lim - 1) * bs];
+      }
+  }
   float m_run = HILS_NEG_INF, l_run = 0.f;
 #pragma unroll
-  for (int tt = 0; tt < GI / LPT; ++tt) {
+  for (int tt = 0; tt < TT; ++tt) {
     const int c0 = grp * KG + tt * 16 + 4 * j;
-    f32x4_t bb = {0.f, 0.f, 0.f, 0.f};
-    if (a.bias && mine) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c0 + i < lim)
-          bb[i] = a.bias[(a.lmk_hm ? ((b * a.h_kv + hk) * (long)a.lmk_cap + c0 + i) : ((b * N + c0 + i) * (long)a.h_kv + hk)) * G + col];
-    }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int ii = 0; ii < LPT; ++ii) *(tr_u4*)(w_addr + ii * TPI * ROWB) = kr[tt * LPT + ii];
@@ -2221,7 +2238,7 @@ __global__ void __launch_bounds__(256) decode_logits_kernel(DsArgs a) {
       *(f32x4_t*)&logits[col * NP + c0] = out;
       if (a.bias) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = __fadd_rn(out[i], bb[i]);
+        for (int i = 0; i < 4; ++i) out[i] = __fadd_rn(out[i], bias_r[tt][i]);
       }
       const float mn = fmaxf(fmaxf(m_run, fmaxf(out[0], out[1])), fmaxf(out[2], out[3]));
       const float ms = (mn == HILS_NEG_INF) ? 0.f : mn * HILS_LOG2E;
@@ -2272,10 +2289,21 @@ __global__ void __launch_bounds__(DS_WAVES * 64) decode_attend_kernel(DsArgs a, 
   for (int i = threadIdx.x; i < a.G * (D / 4); i += DS_WAVES * 64) {
     const int g = i / (D / 4), d4 = i % (D / 4);
     f32x4_t x = {0.f, 0.f, 0.f, 0.f};
-    for (int sp = 0; sp < a.dr.nsplit; ++sp) {
+    for (int s0 = 0; s0 < a.dr.nsplit; s0 += 4) {  // four shares' loads in flight, added in their order
+      unsigned long long v[4][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        x[e] += __hip_atomic_load(&p[(g * (long)a.dr.nsplit + sp) * D + d4 * 4 + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < 4; ++u) {
+        const int sp = s0 + u < a.dr.nsplit ? s0 + u : a.dr.nsplit - 1;
+        const unsigned long long* src = (const unsigned long long*)&p[(g * (long)a.dr.nsplit + sp) * D + d4 * 4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) v[u][e] = __hip_atomic_load(src + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (s0 + u < a.dr.nsplit) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] += __uint_as_float((unsigned)(v[u][e >> 1] >> (32 * (e & 1))));
+        }
     }
     uint2 pk;
     pk.x = pack_bf2(x[0], x[1]);
