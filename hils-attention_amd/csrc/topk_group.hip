@@ -16,8 +16,8 @@
 //     keys, and the threshold is found on those by a bitwise search whose counts are 16-lane DPP
 //     reductions (no ballots, no scalar round trip) and which stops at the first probe that counts
 //     exactly K; ties at the threshold go to the lower chunk indices,
-//   * the ascending order of the winners from a 512-bit map of the winning chunks in LDS
-//     (rank = set bits below the chunk), and the winners' raw scores straight from the logits.
+//   * the ascending order of the winners from the votes of the blocks (rank = winners voted before and in
+//     lower columns), and the winners' raw scores straight from the logits.
 // Five to eight query heads per KV head (HALF below) take two wavefronts per four queries, one for the
 // heads 0..3 and one for the rest: each forms the partial selection scores of its heads, the two
 // trade them through LDS, and both then select on the same scores and write their own heads' outputs.

@@ -7,6 +7,7 @@
 
 #define TG_NB 64     // chunk blocks of 16 a lane row can hold (N <= 1024)
 #define TG_CAND 128  // compacted candidates per query (8 per lane)
+#define TG_REC_NB 32  // kernels of at least this many blocks keep the candidates as records
 
 // Order-preserving unsigned image of a finite score (larger score <-> larger key, -0 as +0) and its
 // inverse.  Every finite score has a key above 0x00800000, so 0 stands for "no key".
@@ -103,7 +104,13 @@ __device__ __forceinline__ uint32_t tg_kth_largest(const uint32_t (&k)[NE], uint
 // chunks and more than 16*NB/2 (NB = 8: any number), so only the blocks from NMASK on can hold
 // invisible chunks; t_base: first query.  Everything is unrolled over the NB blocks: register-resident
 // data has no other way of being indexed, and the host splits a call into launches by NB so that
-// early queries do not pay for 32.  (The 24-block instantiation pays through its occupancy: held to
+// early queries do not pay for 32.
+// What bounds it is the number of instructions, all the more with few wavefronts: a SIMD takes an instruction of one
+// wavefront in 4 to 5 cycles and those of two in the same time.  2048 queries x 8 KV heads of four 128-wide heads that see
+// 1024 chunks, one wavefront per SIMD: 133 -> 108 us (logits 8.2 us of a wavefront's 23, log-sum-exps 3.8, scores and
+// candidates 6, threshold and winners 3.5); 32K queries of the same, by blocks 8 / 16 / 24 / 32: 47.5 / 77 / 119 / 156 ->
+// 46 / 76 / 109 / 131 us.  (Keys through an LDS ring that four wavefronts share: logits as fast, kernel 147 us, since the
+// four wait for the slowest.)  (The 24-block instantiation pays through its occupancy: held to
 // 168 registers it runs three wavefronts per SIMD with ten spilled dwords, 114 us for the queries that
 // see 257..384 chunks against 133 us of the 32-block kernel; at two wavefronts per SIMD it was no
 // faster than 32 blocks.)
@@ -121,8 +128,8 @@ __device__ __forceinline__ uint32_t tg_kth_largest(const uint32_t (&k)[NE], uint
 // wavefront w) on 16 queries, otherwise one pair.
 template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF>
 __global__ void __launch_bounds__(64 * (PERQ ? (HALF ? 8 : 4) : TG_WAVES))
-    // (eight-wavefront workgroups: three per SIMD leave room for one workgroup only, i.e. two per SIMD)
-    __attribute__((amdgpu_waves_per_eu(NB <= 8 ? 5 : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1))))))
+    // (eight-wavefront workgroups are two per SIMD each: three per SIMD leave room for one only, six for three)
+    __attribute__((amdgpu_waves_per_eu(NB <= 8 ? (PERQ && HALF ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1))))))
 topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lmk_packed,
                       const float* __restrict__ lse_swa, const float* __restrict__ bias,
                       int32_t* __restrict__ indices,
@@ -138,6 +145,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   constexpr int QGROUPS = HALF ? TGW / 2 : TGW;              // ... and how many have queries of their own
   static_assert(!PERQ || GMAX == 4, "per-query-head keys: four heads, four wavefronts");
   static_assert(!HALF || (GMAX == 4 && TG_WAVES == 2), "halves: four heads each, a pair per workgroup");
+  constexpr bool ALONE = NB > 32;  // one wavefront per SIMD
   constexpr int PB = NB >= 32 ? 2 : 1;  // blocks per load group (two groups are live: 16 registers per block and group)
   // LDS that several wavefronts share.  PERQ: accumulators of a load group on their way between the
   // wavefronts, [buffer][block][from wavefront = head][register][lane]; two buffers take turns, so that
@@ -151,10 +159,14 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
                                             : (KX_F > TGW * SEL_B / 4 ? KX_F : TGW * SEL_B / 4))
                             : (XCH_F + KX_F > 0 ? XCH_F + KX_F : 1);
   __shared__ __align__(16) float xbuf[XB_F];
-  __shared__ uint32_t cand_w[OVER ? 1 : TGW][4][TG_CAND];          // compacted candidate keys, per lane row
-  constexpr int NW = NB > 32 ? 32 : 16;                          // words of the winner map
-  typedef typename std::conditional<(NB > 32), unsigned long long, uint32_t>::type mask_t;  // a bit per block
-  __shared__ uint32_t words_w[TGW][4][NW], wbase_w[TGW][4][NW];  // winner map of a query and its word prefix counts
+  // REC: candidates as records.  With 24 blocks and fewer walking all scores again is the cheaper way (24 blocks: 109 us
+  // against 124 with records, whose LDS and registers cost wavefronts; 32: 131 with, 156 without).
+  constexpr bool REC = NB >= TG_REC_NB && GMAX == 4 && !OVER;
+  constexpr int REC_N = NB > 32 ? 2 * TG_CAND : 3 * TG_CAND / 2;  // records of a lane row: one query in forty has more than 128
+  constexpr int NWORD = NB > 32 ? 32 : 16;  // words of the winner map
+  __shared__ __align__(16) uint4 rec_w[REC ? TGW : 1][REC ? 4 : 1][REC ? REC_N : 1];
+  __shared__ uint32_t cand_w[OVER || REC ? 1 : TGW][4][TG_CAND];  // (without records) compacted candidate keys, per lane row
+  __shared__ uint32_t words_w[REC ? TGW : 1][REC ? 4 : 1][REC ? NWORD : 1], wbase_w[REC ? TGW : 1][REC ? 4 : 1][REC ? NWORD : 1];
   __shared__ __align__(16) int stage_i_w[OVER ? 1 : TGW][NQ * 32];               // winners' chunk indices, [query][slot]
   __shared__ __align__(16) bf16_t stage_s_w[OVER ? 1 : TGW][NQ * GMAX * 32];  // their raw scores, [query][slot][head]
   // the bias of this (batch, KV head): [chunk][head, padded to 4] fp32, a copy per wavefront (they never
@@ -169,9 +181,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   const int pw = HALF ? (wave >> 1) : wave; // which of the workgroup's queries it has
   const int gofs = 4 * half;
   char* const sel_area = (char*)xbuf + (OVER ? wave * SEL_B : 0);
-  uint32_t (*cand)[TG_CAND] = OVER ? (uint32_t (*)[TG_CAND])sel_area : cand_w[OVER ? 0 : wave];
-  uint32_t (*words)[NW] = words_w[wave];
-  uint32_t (*wbase)[NW] = wbase_w[wave];
+  uint32_t (*cand)[TG_CAND] = OVER ? (uint32_t (*)[TG_CAND])sel_area : cand_w[OVER || REC ? 0 : wave];
   int* stage_i = OVER ? (int*)(sel_area + 4 * TG_CAND * 4) : stage_i_w[OVER ? 0 : wave];
   bf16_t* stage_s = OVER ? (bf16_t*)(sel_area + 4 * TG_CAND * 4 + NQ * 32 * 4) : stage_s_w[OVER ? 0 : wave];
   const int lane = threadIdx.x & 63, col = lane & 15, j = lane >> 4;
@@ -225,17 +235,14 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
     return lm < 0 ? 0 : (lm > N ? N : lm);
   };
   // accumulator row 4j+i <-> (query t0 + (4j+i)/GMAX, head (4j+i)%GMAX): a lane has QPL queries
-  int lim[4];
+  int lim[QPL];  // (one bound for a query's heads: the rows of heads past G, masked or not, end at their lse_tot below)
   bool rowok[4];
 #pragma unroll
   for (int u = 0; u < QPL; ++u) {
     const int tq = t0 + j * QPL + u;
-    const int lq = tq < t_end ? limit_of(tq) : 0;
+    lim[u] = tq < t_end ? limit_of(tq) : 0;
 #pragma unroll
-    for (int e = 0; e < GMAX; ++e) {
-      rowok[u * GMAX + e] = (tq < t_end) & (gofs + e < G);
-      lim[u * GMAX + e] = gofs + e < G ? lq : 0;
-    }
+    for (int e = 0; e < GMAX; ++e) rowok[u * GMAX + e] = (tq < t_end) & (gofs + e < G);
   }
   const int nb_real = (N + 15) / 16;  // blocks the packed chunk keys hold
 
@@ -291,6 +298,53 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   auto xch = [&](int buf, int p2, int w, int i, int l) -> float& {
     return xbuf[(((buf * PB + p2) * TGW + w) * 4 + i) * 64 + l];
   };
+  // the products of a group of blocks ...
+  auto mul_group = [&](const tg_u32x4 (&src)[PB][KS], f32x4_t (&acc)[PB]) {
+#pragma unroll
+    for (int p2 = 0; p2 < PB; ++p2) acc[p2] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int p2 = 0; p2 < PB; ++p2)
+        acc[p2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag[ks], __builtin_bit_cast(bf16x8_t, src[p2][ks]), acc[p2], 0, 0, 0);
+  };
+  // ... and its logits
+  auto put_group = [&](int g0, const f32x4_t (&acc)[PB]) {
+#pragma unroll
+    for (int p2 = 0; p2 < PB; ++p2) {
+      const int nt = g0 + p2, c = nt * 16 + col;
+      float bv[4];
+      if constexpr (BIAS && (!PERQ || HALF)) bias_of(nt * 16 + col, bv);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v;
+        if constexpr (PERQ) {
+          // row (query j of this wavefront, head i of its heads): that head's wavefront's register j of
+          // the lane that holds this chunk column for the queries 4 * pw .. 4 * pw + 3
+          v = xch((g0 / PB) & 1, p2, gofs + i, j, col + 16 * pw);
+          if constexpr (BIAS && HALF) v = __fadd_rn(v, bv[i]);
+        } else {
+          v = __fmul_rn(acc[p2][i], sm_scale);
+          if constexpr (BIAS) v = __fadd_rn(v, bv[i]);
+        }
+        if (nt >= NMASK) v = (c < lim[i / GMAX]) ? v : HILS_NEG_INF;
+        x[nt][i] = v;
+        // (pinned here: left alone the compiler forms some of these only where they are used and keeps
+        // product and bias, or the product and the mask, alive in their place, which this kernel has no registers for)
+        if constexpr ((BIAS && (!PERQ || HALF)) || ALONE) asm volatile("" : "+v"(x[nt][i]));
+      }
+      if (EXPORT) {
+        if (sel_logits_out && c < N) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (rowok[i]) {
+              const int r = 4 * j + i;
+              sel_logits_out[(((b * L + t0 + r / GMAX) * (long)h_kv + hk) * G + gofs + r % GMAX) * N + c] = x[nt][i];
+            }
+        }
+      }
+    }
+  };
   auto use_group = [&](int g0, const tg_u32x4 (&src)[PB][KS]) {
     const int buf = (g0 / PB) & 1;
     if constexpr (PERQ) {
@@ -313,49 +367,27 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
       }
       __syncthreads();
     }
-#pragma unroll
-    for (int p2 = 0; p2 < PB; ++p2) {
-      const int nt = g0 + p2;
-      float bv[4];
-      if constexpr (BIAS && (!PERQ || HALF)) bias_of(nt * 16 + col, bv);
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (!PERQ) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag[ks], __builtin_bit_cast(bf16x8_t, src[p2][ks]), acc, 0, 0, 0);
-      }
-      const int c = nt * 16 + col;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v;
-        if constexpr (PERQ) {
-          // row (query j of this wavefront, head i of its heads): that head's wavefront's register j of
-          // the lane that holds this chunk column for the queries 4 * pw .. 4 * pw + 3
-          v = xch(buf, p2, gofs + i, j, col + 16 * pw);
-          if constexpr (BIAS && HALF) v = __fadd_rn(v, bv[i]);
-        } else {
-          v = __fmul_rn(acc[i], sm_scale);
-          if constexpr (BIAS) v = __fadd_rn(v, bv[i]);
-        }
-        if (nt >= NMASK) v = (c < lim[i]) ? v : HILS_NEG_INF;
-        x[nt][i] = v;
-        // (pinned here: left alone the compiler forms some of these sums only where they are used and
-        // keeps product and bias alive in their place, which this kernel has no registers for)
-        if constexpr (BIAS && (!PERQ || HALF)) asm volatile("" : "+v"(x[nt][i]));
-      }
-      if (EXPORT) {
-        if (sel_logits_out && c < N) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (rowok[i]) {
-              const int r = 4 * j + i;
-              sel_logits_out[(((b * L + t0 + r / GMAX) * (long)h_kv + hk) * G + gofs + r % GMAX) * N + c] = x[nt][i];
-            }
-        }
-      }
-    }
+    f32x4_t acc[PB];
+    if constexpr (!PERQ) mul_group(src, acc);
+    put_group(g0, acc);
   };
-  {
+  if constexpr (ALONE && !PERQ) {
+    // nobody else's instructions to wait behind: the keys travel three groups ahead, and a group's products run while the
+    // logits of the one before are formed
+    constexpr int NG = NB / PB, AHEAD = 3;
+    tg_u32x4 keys[AHEAD + 1][PB][KS];
+    f32x4_t acc[2][PB];
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) load_group(g * PB, keys[g]);
+#pragma unroll
+    for (int g = 0; g <= NG; ++g) {
+      if (g + AHEAD < NG) load_group((g + AHEAD) * PB, keys[(g + AHEAD) % (AHEAD + 1)]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g < NG) mul_group(keys[g % (AHEAD + 1)], acc[g & 1]);
+      if (g > 0) put_group((g - 1) * PB, acc[(g - 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
     tg_u32x4 ba[PB][KS], bb2[PB][KS];
     load_group(0, ba);
 #pragma unroll
@@ -377,18 +409,37 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
 
   if (PERQ && !HALF && t0 >= t_end) return;  // no barrier behind this point
   // ---- lse_total per row = logaddexp(lse_swa, logsumexp of the visible logits) ----
-  float lse_tot[4];
+  // (ALONE: the four rows side by side.  One after the other every sum waited for its exponential, 9 instead of 5
+  // thousand cycles; with more wavefronts another one's instructions run meanwhile, and the registers are short.)
+  constexpr int RS = ALONE ? 4 : 1;
+  float lse_tot[4], m_row[4], l_row[4];
+#pragma unroll
+  for (int r0 = 0; r0 < 4; r0 += RS) {
+#pragma unroll
+    for (int i = r0; i < r0 + RS; ++i) {
+      float m = HILS_NEG_INF;
+#pragma unroll
+      for (int nt = 0; nt < NB; ++nt) m = fmaxf(m, x[nt][i]);
+      m = tg_row_max_f(m);
+      m_row[i] = (m > HILS_NEG_INF) ? m * HILS_LOG2E : 0.f;
+      l_row[i] = 0.f;
+    }
+#pragma unroll
+    for (int nt = 0; nt < NB; ++nt) {
+      float e4[4];
+#pragma unroll
+      for (int i = r0; i < r0 + RS; ++i) e4[i] = fmaf(x[nt][i], HILS_LOG2E, -m_row[i]);
+      if constexpr (ALONE) __builtin_amdgcn_sched_barrier(0);  // (the compiler would put the chains one after the other again)
+#pragma unroll
+      for (int i = r0; i < r0 + RS; ++i) e4[i] = __builtin_amdgcn_exp2f(e4[i]);
+      if constexpr (ALONE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = r0; i < r0 + RS; ++i) l_row[i] += e4[i];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float m = HILS_NEG_INF;
-#pragma unroll
-    for (int nt = 0; nt < NB; ++nt) m = fmaxf(m, x[nt][i]);
-    m = tg_row_max_f(m);
-    const float m2 = (m > HILS_NEG_INF) ? m * HILS_LOG2E : 0.f;
-    float l = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < NB; ++nt) l += __builtin_amdgcn_exp2f(fmaf(x[nt][i], HILS_LOG2E, -m2));
-    l = row_sum<16>(l);
+    const float m2 = m_row[i], l = row_sum<16>(l_row[i]);
     const float hils2 = (l > 0.f) ? m2 + __builtin_amdgcn_logf(l) : HILS_NEG_INF;  // log2 domain
     const float swa2 = swa[i] * HILS_LOG2E;
     const float mx = fmaxf(swa2, hils2), mn = fminf(swa2, hils2);
@@ -416,6 +467,11 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   if constexpr (!OVER) clear_stage();  // (OVER: once the memory is the stage's)
 
   // ---- selection, one query of every lane row at a time ----
+  // the lane row's bits of a vote, and those of its lower columns
+  const uint32_t row_bits = 0xffffu << (16 * (j & 1)), low_bits = ((1u << col) - 1u) << (16 * (j & 1));
+  const uint32_t row_lo = j < 2 ? row_bits : 0u, row_hi = j < 2 ? 0u : row_bits;
+  const uint32_t low_lo = j < 2 ? low_bits : 0u, low_hi = j < 2 ? 0u : low_bits;
+  constexpr int WB = BIAS ? (OVER ? 1 : 4) : 1;  // blocks whose biases are read together
 #pragma unroll
   for (int u = 0; u < QPL; ++u) {
     const int qi = j * QPL + u;  // query of the wavefront this lane row works on
@@ -471,6 +527,119 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
       nv += (kk > HILS_NEG_INF) ? 1 : 0;
     }
     const int nvalid = tg_row_sum_i(nv);
+    if constexpr (REC) {
+      // The candidates as records (score, chunk, raw scores), so that from here on a lane has at most eight of them to
+      // look at instead of NB: the threshold, the winners, their order (a map of the winning chunks and its prefix
+      // counts) and their raw scores all come from the records.  A query that keeps everything has all its valid scores
+      // (at most topk) as candidates.
+      const bool want = nvalid > topk;
+      const float hi = tg_row_max_f(m1), bound = tg_row_min_f(m2);  // >= 2 scores per lane reach it: >= 32 >= topk in all
+      const float cbound = want ? bound : -3.402823466e38f;
+      int nc = 0;
+#pragma unroll
+      for (int nt = 0; nt < NB; ++nt) nc += (key[nt] >= cbound) ? 1 : 0;
+      const int ntot = tg_row_sum_i(nc);
+      if (!__any(want & ((ntot > REC_N) | !(bound > HILS_NEG_INF)))) {  // (else: the search over all scores, below)
+        uint4* next = &rec_w[wave][j][tg_row_excl_scan(nc)];
+#pragma unroll
+        for (int n0 = 0; n0 < NB; n0 += WB) {
+          float bv[WB][4];
+          if constexpr (BIAS) {
+#pragma unroll
+            for (int n2 = 0; n2 < WB; ++n2) bias_of((n0 + n2) * 16 + col, bv[n2]);
+          }
+#pragma unroll
+          for (int n2 = 0; n2 < WB; ++n2) {
+            const int nt = n0 + n2;
+            if (key[nt] >= cbound) {
+              float raw[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) raw[i] = BIAS ? __fsub_rn(x[nt][i], bv[n2][i]) : x[nt][i];  // (the returned scores carry no bias)
+              *next++ = make_uint4(__float_as_uint(key[nt]), nt * 16 + col, pack_bf2(raw[0], raw[1]), pack_bf2(raw[2], raw[3]));
+            }
+          }
+        }
+        uint32_t (*words)[NWORD] = words_w[wave], (*wbase)[NWORD] = wbase_w[wave];
+#pragma unroll
+        for (int w = 0; w < NWORD; w += 16) words[j][w + col] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        auto pick = [&](auto ne) __attribute__((always_inline)) {  // at most ne records a lane
+          constexpr int NE = decltype(ne)::value;
+          uint4 rc[NE];
+          uint32_t ck[NE];
+#pragma unroll
+          for (int e = 0; e < NE; ++e) rc[e] = rec_w[wave][j][e * 16 + col];
+#pragma unroll
+          for (int e = 0; e < NE; ++e) ck[e] = (e * 16 + col < ntot) ? tg_score_key(__uint_as_float(rc[e].x)) : 0u;
+          const uint32_t lo_k = tg_score_key(want ? bound : 0.f), hi_k = tg_score_key(want ? hi : 0.f);
+          bool exact = false;
+          uint32_t T = tg_kth_largest(ck, lo_k, hi_k, topk, want & (ntot != topk), exact);
+          if (ntot == topk) {  // exactly the candidates win
+            T = lo_k;
+            exact = true;
+          }
+          if (!want) T = 1u;
+          // ties at the threshold (only where the search ran down to the last bit): the lowest chunk indices win
+          int cutoff = 1 << 30;
+          const bool loose = want & !exact;
+          if (__any(loose)) {
+            int ngt = 0, neq = 0;
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+              ngt += (ck[e] > T) ? 1 : 0;
+              neq += (ck[e] == T) ? 1 : 0;
+            }
+            ngt = tg_row_sum_i(ngt);
+            neq = tg_row_sum_i(neq);
+            const int need = topk - ngt;
+            if (__any(loose & (neq > need))) {
+              // smallest index C with count(score == T and chunk <= C) >= need, bit by bit
+              int C = 0;
+              for (int bit = 9; bit >= 0; --bit) {
+                const int c2 = C | (1 << bit);  // count the ties below c2
+                int cl = 0;
+#pragma unroll
+                for (int e = 0; e < NE; ++e) cl += ((ck[e] == T) & ((int)rc[e].y < c2)) ? 1 : 0;
+                if (tg_row_sum_i(cl) < need) C = c2;
+              }
+              if (loose & (neq > need)) cutoff = C;
+            }
+          }
+          bool win[NE];
+#pragma unroll
+          for (int e = 0; e < NE; ++e) {
+            win[e] = (ck[e] > T) | ((ck[e] == T) & ((int)rc[e].y <= cutoff));
+            if (win[e]) atomicOr(&words[j][rc[e].y >> 5], 1u << (rc[e].y & 31));
+          }
+          __builtin_amdgcn_wave_barrier();
+          if constexpr (NWORD > 16) {
+            const int p0 = __popc(words[j][2 * col]), p1 = __popc(words[j][2 * col + 1]);
+            const int base = tg_row_excl_scan(p0 + p1);
+            wbase[j][2 * col] = (uint32_t)base;
+            wbase[j][2 * col + 1] = (uint32_t)(base + p0);
+          } else {
+            wbase[j][col] = (uint32_t)tg_row_excl_scan(__popc(words[j][col]));
+          }
+          __builtin_amdgcn_wave_barrier();
+          int slot[NE];
+#pragma unroll
+          for (int e = 0; e < NE; ++e) {
+            const uint32_t c = win[e] ? rc[e].y : 0u;
+            slot[e] = (int)wbase[j][c >> 5] + __popc(words[j][c >> 5] & ((1u << (c & 31)) - 1u));
+          }
+#pragma unroll
+          for (int e = 0; e < NE; ++e)
+            if (win[e] & (slot[e] < topk)) {
+              stage_i[qi * 32 + slot[e]] = (int)rc[e].y;
+              *(uint2*)&stage_s[(qi * 32 + slot[e]) * GMAX] = make_uint2(rc[e].z, rc[e].w);
+            }
+        };
+        if (__any(ntot > TG_CAND)) pick(std::integral_constant<int, REC_N / 16>{});
+        else pick(std::integral_constant<int, TG_CAND / 16>{});
+        __builtin_amdgcn_wave_barrier();
+        continue;  // (the only query of the lane row)
+      }
+    }
     float Tf = HILS_NEG_INF;  // every valid score wins ...
     int cutoff = -1;          // ... and among the scores equal to Tf those with a chunk index <= cutoff
     bool cut = false;         // cutoff excludes some of them
@@ -487,16 +656,12 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
       const int ntot = tg_row_sum_i(nc);
       uint32_t T;
       bool exact = false;
-      if (!__any(want & ((ntot > TG_CAND) | !(bound > HILS_NEG_INF)))) {
+      if (!REC && !__any(want & ((ntot > TG_CAND) | !(bound > HILS_NEG_INF)))) {
         // compact the candidates of the lane row (any order) and take at most 8 per lane
-        int pos = tg_row_excl_scan(nc);
+        uint32_t* next = &cand[j][tg_row_excl_scan(nc)];
 #pragma unroll
-        for (int nt = 0; nt < NB; ++nt) {
-          if (key[nt] >= cbound) {
-            cand[j][pos] = __float_as_uint(key[nt]);
-            ++pos;
-          }
-        }
+        for (int nt = 0; nt < NB; ++nt)
+          if (key[nt] >= cbound) *next++ = __float_as_uint(key[nt]);
         __builtin_amdgcn_wave_barrier();
         uint32_t ck[TG_CAND / 16];
 #pragma unroll
@@ -557,59 +722,43 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
         }
       }
     }
-    // winners of this lane as a bit mask over its blocks
-    mask_t mask = 0u;
-    if (__any(cut)) {
+    if (__any(cut)) {  // the ties that lose leave the scores
 #pragma unroll
-      for (int nt = NB - 1; nt >= 0; --nt) {
-        const bool win = (key[nt] > Tf) | ((key[nt] == Tf) & (nt * 16 + col <= cutoff));
-        mask = (mask << 1) | (win ? 1u : 0u);
+      for (int nt = 0; nt < NB; ++nt)
+        if ((key[nt] == Tf) & (nt * 16 + col > cutoff)) key[nt] = HILS_NEG_INF;
+    }
+    // Everything from the threshold up wins (a query that keeps all its valid scores has Tf = -inf: the lowest finite
+    // float stands in for it).  A winner's slot is the number of winners with a lower chunk index: those of the blocks
+    // before (`before`, of this lane's row) and those of lower columns, both counted in the bits of the block's vote, so
+    // that nothing waits for LDS: with the winners' map and its prefix counts there, every block with a winner read them
+    // back and waited, 16 of the 36 thousand cycles that the selection of 1024 chunks took.
+    const float Tlow = fmaxf(Tf, -3.402823466e38f);
+    int before = 0;
+#pragma unroll
+    for (int n0 = 0; n0 < NB; n0 += WB) {
+      float bv[WB][4];
+      if constexpr (BIAS) {
+#pragma unroll
+        for (int n2 = 0; n2 < WB; ++n2) bias_of((n0 + n2) * 16 + col, bv[n2]);
       }
-    } else {
-      // no tie to break in this wavefront: everything from the threshold up wins (a query that keeps
-      // all its valid scores has Tf = -inf: the lowest finite float stands in for it)
-      const float Tlow = fmaxf(Tf, -3.402823466e38f);
 #pragma unroll
-      for (int nt = NB - 1; nt >= 0; --nt) mask = (mask << 1) | ((key[nt] >= Tlow) ? 1u : 0u);
-    }
-    // map of the winning chunks (chunk c = bit c): word w holds blocks 2w and 2w+1
-    words[j][col] = 0u;
-    if constexpr (NW > 16) words[j][16 + col] = 0u;
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int w = 0; w < (NB + 1) / 2; ++w) {
-      const uint32_t bits = ((uint32_t)((mask >> (2 * w)) & 1u) << col) | ((uint32_t)((mask >> (2 * w + 1)) & 1u) << (16 + col));
-      if (bits) atomicOr(&words[j][w], bits);
-    }
-    __builtin_amdgcn_wave_barrier();
-    if constexpr (NW > 16) {
-      const int p0 = __popc(words[j][2 * col]), p1 = __popc(words[j][2 * col + 1]);
-      const int base = tg_row_excl_scan(p0 + p1);
-      wbase[j][2 * col] = (uint32_t)base;
-      wbase[j][2 * col + 1] = (uint32_t)(base + p0);
-    } else {
-      const int pc = __popc(words[j][col]);
-      wbase[j][col] = (uint32_t)tg_row_excl_scan(pc);
-    }
-    __builtin_amdgcn_wave_barrier();
-    // every winner: its slot = winners with a lower chunk index; index and raw scores to the stage
-#pragma unroll
-    for (int nt = 0; nt < NB; ++nt) {
-      if ((mask >> nt) & 1u) {
-        const int c = nt * 16 + col, w = c >> 5;
-        const int slot = (int)wbase[j][w] + __popc(words[j][w] & ((1u << (c & 31)) - 1u));
-        if (slot < topk) {
-          stage_i[qi * 32 + slot] = c;
+      for (int n2 = 0; n2 < WB; ++n2) {
+        const int nt = n0 + n2;
+        const bool win = key[nt] >= Tlow;
+        const unsigned long long votes = __ballot(win);
+        const uint32_t v_lo = (uint32_t)votes, v_hi = (uint32_t)(votes >> 32);
+        const int slot = __popc(v_hi & low_hi) + (__popc(v_lo & low_lo) + before);
+        before = __popc(v_hi & row_hi) + (__popc(v_lo & row_lo) + before);
+        if (win & (slot < topk)) {  // its chunk and raw scores to the stage
+          stage_i[qi * 32 + slot] = nt * 16 + col;
           // the heads of the winner in one store (heads past G are never read back)
           bf16_t* dst = &stage_s[(qi * 32 + slot) * GMAX];
           float raw[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) raw[i] = x[nt][i];
           if constexpr (BIAS) {  // the returned scores carry no bias
-            float bv[4];
-            bias_of(c, bv);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) raw[i] = __fsub_rn(raw[i], bv[i]);
+            for (int i = 0; i < 4; ++i) raw[i] = __fsub_rn(raw[i], bv[n2][i]);
           }
           if constexpr (GMAX == 4) {
             *(uint2*)dst = make_uint2(pack_bf2(raw[0], raw[1]), pack_bf2(raw[2], raw[3]));
