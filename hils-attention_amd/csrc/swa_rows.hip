@@ -25,10 +25,11 @@
 #define SR_WAVES 8
 #define SR_UNIT 32  // tokens a wavefront works on at a time
 
-template <int D, int DV>
+template <int D, int DVF, int VS>
 __global__ void __launch_bounds__(SR_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
              bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int g_bits) {
+  constexpr int DV = DVF / VS;  // the value features of this workgroup, of DVF
   constexpr int KS = D / 32, MT = DV / 16;
   constexpr int VL = DV / 8, TPI = 64 / VL, VI = SR_UNIT / TPI;  // lanes per V row, rows per load, loads per unit
   constexpr int VP = 2 * DV + 16;                                // bytes of a staged V row
@@ -44,7 +45,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   const int col = lane & 15, j = lane >> 4;
   const int G = 1 << g_bits, QB = 16 >> g_bits;  // (no division: one is tens of instructions before the first load)
   const int tq0 = blockIdx.x * QB;
-  const int hk = blockIdx.y;
+  const int hk = VS > 1 ? blockIdx.y % dm.H : blockIdx.y, part = VS > 1 ? blockIdx.y / dm.H : 0;
   const long b = blockIdx.z;
   const int q_off = dm.kv_start + dm.Lk - dm.Lq;  // absolute position of query 0
 
@@ -81,7 +82,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
   const bf16_t* kb = k + b * dm.k_batch + (long)hk * D + j * 8;
-  const bf16_t* vb = v + b * dm.v_batch + (long)hk * DV + (lane % VL) * 8;
+  const bf16_t* vb = v + b * dm.v_batch + (long)hk * DVF + part * DV + (lane % VL) * 8;
   auto issue = [&](sr_u4 (&kd)[2][KS], sr_u4 (&vd)[VI], int u) __attribute__((always_inline)) {
     const int t0 = lo + u * SR_UNIT;  // tokens past the end read the last row: their scores are masked
 #pragma unroll
@@ -95,7 +96,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
     for (int i = 0; i < VI; ++i) {
       int tok = t0 + i * TPI + lane / VL;
       tok = tok < dm.Lk ? tok : dm.Lk - 1;
-      vd[i] = *(const sr_u4*)(vb + (long)tok * dm.H * DV);
+      vd[i] = *(const sr_u4*)(vb + (long)tok * dm.H * DVF);
     }
   };
 
@@ -233,8 +234,8 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
     uint2 pk;
     pk.x = pack_bf2(x[0] * inv, x[1] * inv);
     pk.y = pack_bf2(x[2] * inv, x[3] * inv);
-    *(uint2*)(o + rix * DV + d4 * 4) = pk;
-    if (d4 == 0) lse[rix] = L > 0.f ? (M * c2 + __builtin_amdgcn_logf(L)) * HILS_LN2 : HILS_NEG_INF;
+    *(uint2*)(o + rix * DVF + part * DV + d4 * 4) = pk;
+    if (d4 == 0 && part == 0) lse[rix] = L > 0.f ? (M * c2 + __builtin_amdgcn_logf(L)) * HILS_LN2 : HILS_NEG_INF;
   }
 }
 
@@ -260,14 +261,21 @@ int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const
                       int Dv, const SwaDims& dm) {
   const int G = dm.HQ / dm.H;
   const int n_rb = (dm.Lq + 16 / G - 1) / (16 / G), g_bits = __builtin_ctz(G);
-  const dim3 grid(n_rb, dm.H, B), wg(SR_WAVES * 64);
-#define SR_CALL(D_, V_)                                                                                     \
-  hipLaunchKernelGGL((swa_fwd_rows<D_, V_>), grid, wg, 0, st, (const bf16_t*)q, (const bf16_t*)k,            \
+  // While both fit the chip at once, two workgroups a row block, each with all keys and half of the value features: a
+  // compute unit's share of the memory system is the bound, and nothing has to be added up (one / two, window 512, us:
+  // heads of 64 5.5/5.3 with one row block, 6.0/5.8 with 128, 6.0/9.2 with 192; of 128 9.2/8.6, 10.0/9.3, 10.6/16.6;
+  // window 64: 3.6/3.5 and 4.5/4.2 with 128.  Four quarters: 8.8 against 9.2 on 64 blocks of heads of 128, else no faster).
+  const bool halves = 2l * n_rb * dm.H * B <= hils_device_cus();
+  const dim3 grid(n_rb, dm.H * (halves ? 2 : 1), B), wg(SR_WAVES * 64);
+#define SR_CALL(D_, V_, S_)                                                                                 \
+  hipLaunchKernelGGL((swa_fwd_rows<D_, V_, S_>), grid, wg, 0, st, (const bf16_t*)q, (const bf16_t*)k,        \
                      (const bf16_t*)v, (bf16_t*)o, lse, dm, g_bits)
-  if (D == 64 && Dv == 64) SR_CALL(64, 64);
-  else if (D == 128 && Dv == 128) SR_CALL(128, 128);
-  else if (D == 64) SR_CALL(64, 128);
-  else SR_CALL(128, 64);
+#define SR_CALL_S(D_, V_) do { if (halves) SR_CALL(D_, V_, 2); else SR_CALL(D_, V_, 1); } while (0)
+  if (D == 64 && Dv == 64) SR_CALL_S(64, 64);
+  else if (D == 128 && Dv == 128) SR_CALL_S(128, 128);
+  else if (D == 64) SR_CALL_S(64, 128);
+  else SR_CALL_S(128, 64);
+#undef SR_CALL_S
 #undef SR_CALL
   return HILS_OK;
 }
