@@ -1458,52 +1458,6 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
 #pragma unroll
   for (int g = 0; g < GMAX; ++g) swa[g] = (g < G) ? lse_swa[row * G + g] : 0.f;
   if (tid == 0) sh.next_group = 2 * NW;
-  typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
-  // key groups of the row: KG chunks each, times the G heads when every query head has its own keys
-  // (group number = chunk group * G + head: the heads of a chunk are neighbours in memory)
-  const int GK = perq ? G : 1;                  // key tensors of the row
-  const int h_lmk = h_kv * GK;                  // heads of the key tensor
-  const int ngroups = ((lim + KG - 1) / KG) * GK;
-  // dense chunk keys: (B, N, h_lmk, D), or head-major (B, h_lmk, lmk_cap, D) (a row's keys contiguous)
-  const bf16_t* base = lmks + (lmk_hm ? (b * h_lmk + hk * GK) * (long)lmk_cap * D : (b * N * (long)h_lmk + hk * GK) * D) + piece * 8;
-  const long cstride = (PAGED || !lmk_hm) ? (long)h_lmk * D : (long)D;
-  const long gstride = (!PAGED && lmk_hm) ? (long)lmk_cap * D : (long)D;  // from a head to the next of the group
-  const bf16_t* pbase = lmks + (long)hk * GK * D + piece * 8;  // paged: + page * h_lmk * D
-  auto fetch = [&](tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
-    const int grp = perq ? vg / G : vg;
-    const long goff = perq ? (vg - grp * G) * gstride : 0;
-#pragma unroll
-    for (int it = 0; it < GI; ++it) {
-      int c = grp * KG + it * TPI + tsub;
-      c = c < N ? c : N - 1;
-      if (PAGED) {
-        const int pg = page_s[c];  // an unmapped or invisible chunk reads page 0 and is masked below
-        kr[it] = *(const tr_u4*)(pbase + goff + (long)(pg < 0 ? 0 : pg) * cstride);
-      } else {
-        kr[it] = *(const tr_u4*)(base + goff + c * cstride);
-      }
-    }
-  };
-  // drawn group numbers only grow (the first two of a wavefront are wave and wave + NW), `last` stands in for one past the end
-  const int last = ngroups - 1;
-  tr_u4 ka[GI], kb[GI];
-  int ga = wave, gb = wave + NW;
-  // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
-  // features ks*32 + 8j ..
-  bf16x8_t qb[D / 32];
-  if constexpr (!PRE) {
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      tr_u4 t = {0u, 0u, 0u, 0u};
-      if ((lane & 15) < G) t = *(const tr_u4*)(q + (row * (long)G + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8);
-      qb[ks] = __builtin_bit_cast(bf16x8_t, t);
-    }
-    // the first keys are on their way before the bias is staged and the queries have arrived (page ids come first)
-    if (!PAGED && ngroups > 0) {
-      fetch(ka, ga < last ? ga : last);
-      fetch(kb, gb < last ? gb : last);
-    }
-  }
   // PRE: the wavefronts share out the heads' rows, four pieces a lane in flight at once (of up to NP / 4 a row), issued ahead
   // of the bias staging (as atomic loads, which the compiler leaves where they are written: one by one in a loop, three or
   // four latencies of memory were most of 2.7 us)
@@ -1561,7 +1515,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       for (int g = 0; g < GMAX; ++g) bias_s[g * NP + c] = bv[g];
     }
   }
-  if (FUSED && tid == 0) {  // (behind the other loads' issue: a store here waits for a latency of memory)
+  if (FUSED && tid == 0) {  // (behind the other loads' issue: a store ahead of them waits for a latency of memory first)
 #pragma unroll
     for (int g = 0; g < GMAX; ++g) sh.swa[g] = swa[g];
   }
@@ -1591,6 +1545,16 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       sh.grp_l[i / GMAX][i % GMAX] = i == tid ? pl : pre_l[i];
     }
   } else {
+  // the query heads as B operand of the logit products, lane (head = lane & 15, j = lane >> 4) holds
+  // features ks*32 + 8j ..; loaded here so that the barrier below has waited for them
+  typedef unsigned tr_u4 __attribute__((ext_vector_type(4)));
+  bf16x8_t qb[D / 32];
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) {
+    tr_u4 t = {0u, 0u, 0u, 0u};
+    if ((lane & 15) < G) t = *(const tr_u4*)(q + (row * (long)G + (lane & 15)) * D + ks * 32 + (lane >> 4) * 8);
+    qb[ks] = __builtin_bit_cast(bf16x8_t, t);
+  }
   // have them arrive here: a load still pending at the streaming loop's first use would make the
   // compiler wait for every load in flight there, in every iteration
 #pragma unroll
@@ -1601,7 +1565,7 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       page_s[c] = (pg >= 0 && pg < num_pages) ? pg : -1;
     }
   }
-  lds_barrier();  // (no wait for the keys in flight)
+  __syncthreads();
 
   // ---- phase 1: logits of the visible chunks.  The chunk-key rows arrive by coalesced 16-byte lane
   // loads (LR lanes per row), are written row-major (rows padded by 16 bytes: no bank conflicts
@@ -1616,6 +1580,31 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
     const int col = lane & 15, j = lane >> 4;
     char* const w_addr = stage_w + tsub * ROWB + piece * 16;
     const char* const k_addr = stage_w + col * ROWB + j * 16;
+    // key groups of the row: KG chunks each, times the G heads when every query head has its own keys
+    // (group number = chunk group * G + head: the heads of a chunk are neighbours in memory)
+    const int GK = perq ? G : 1;                  // key tensors of the row
+    const int h_lmk = h_kv * GK;                  // heads of the key tensor
+    const int ngroups = ((lim + KG - 1) / KG) * GK;
+    // dense chunk keys: (B, N, h_lmk, D), or head-major (B, h_lmk, lmk_cap, D) (a row's keys contiguous)
+    const bf16_t* base = lmks + (lmk_hm ? (b * h_lmk + hk * GK) * (long)lmk_cap * D : (b * N * (long)h_lmk + hk * GK) * D) + piece * 8;
+    const long cstride = (PAGED || !lmk_hm) ? (long)h_lmk * D : (long)D;
+    const long gstride = (!PAGED && lmk_hm) ? (long)lmk_cap * D : (long)D;  // from a head to the next of the group
+    const bf16_t* pbase = lmks + (long)hk * GK * D + piece * 8;  // paged: + page * h_lmk * D
+    auto fetch = [&](tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
+      const int grp = perq ? vg / G : vg;
+      const long goff = perq ? (vg - grp * G) * gstride : 0;
+#pragma unroll
+      for (int it = 0; it < GI; ++it) {
+        int c = grp * KG + it * TPI + tsub;
+        c = c < N ? c : N - 1;
+        if (PAGED) {
+          const int pg = page_s[c];  // an unmapped or invisible chunk reads page 0 and is masked below
+          kr[it] = *(const tr_u4*)(pbase + goff + (long)(pg < 0 ? 0 : pg) * cstride);
+        } else {
+          kr[it] = *(const tr_u4*)(base + goff + c * cstride);
+        }
+      }
+    };
     auto consume = [&](const tr_u4 (&kr)[GI], int vg) __attribute__((always_inline)) {
       const int grp = perq ? vg / G : vg;
       const int gh = perq ? vg - grp * G : -1;  // the head these keys belong to (-1: to all heads)
@@ -1683,7 +1672,10 @@ topk_row_body(const bf16_t* __restrict__ q, const bf16_t* __restrict__ lmks,
       return __builtin_amdgcn_readfirstlane(v);
     };
     // drawn group numbers only grow, so the first one past the end ends the wavefront's walk
-    if (PAGED && ngroups > 0) {
+    const int last = ngroups - 1;
+    tr_u4 ka[GI], kb[GI];
+    int ga = wave, gb = wave + NW;
+    if (ngroups > 0) {
       fetch(ka, ga < last ? ga : last);
       fetch(kb, gb < last ? gb : last);
     }
