@@ -5,6 +5,21 @@
 
 #define GL_MAXK 64
 
+// (batch element, token of the batch, query head) of a row.  With fewer than 2^31 rows the divisions are of 32 bits:
+// those of 64 bits were 200 of the forward's 390 instructions.
+__device__ __forceinline__ void gl_row_coords(long row, long rows, int L, int HQ, long& b, long& bt, int& hq) {
+  if (rows < (1L << 31)) {
+    const unsigned t = (unsigned)row / (unsigned)HQ;
+    hq = (int)((unsigned)row - t * (unsigned)HQ);
+    bt = t;
+    b = t / (unsigned)L;
+  } else {
+    bt = row / HQ;
+    hq = (int)(row - bt * HQ);
+    b = bt / L;
+  }
+}
+
 // One thread per (batch, query, query head) row.
 __global__ void __launch_bounds__(256)
 chunk_weights_kernel(const bf16_t* __restrict__ scores, const void* __restrict__ lse_ptr,
@@ -82,9 +97,9 @@ chunk_weights_rows_kernel(const bf16_t* __restrict__ scores, const void* __restr
     unpack8(v, x);
     lse = lse_bf16 ? bf2f(((const bf16_t*)lse_swa)[row]) : ((const float*)lse_swa)[row];
     if (prior_b) {
-      const int hq = (int)(row % HQ);
-      const long bt = row / HQ;
-      const long b = bt / L;
+      long b, bt;
+      int hq;
+      gl_row_coords(row, rows, L, HQ, b, bt, hq);
       const int G = HQ / H;
       const int32_t* ip = indices + (bt * H + hq / G) * (long)K + sub * 8;
 #pragma unroll
@@ -127,7 +142,13 @@ chunk_weights_rows_kernel(const bf16_t* __restrict__ scores, const void* __restr
   if (nrow <= 0) return;
   const int total = (int)nrow * NW;
   bf16_t* dst = weights + row0 * NW;
-  for (int i = lane; i < total; i += 64) dst[i] = stage[wave][i];
+  constexpr int PIECES = (RPW * (K + 2) + 63) / 64;
+  bf16_t w[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) w[p] = p * 64 + lane < total ? stage[wave][p * 64 + lane] : (bf16_t)0;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p)
+    if (p * 64 + lane < total) dst[p * 64 + lane] = w[p];
 }
 
 extern "C" int hils_chunk_weights(const void* scores, const void* lse_swa, int lse_bf16,
@@ -243,10 +264,12 @@ chunk_weights_bwd_kernel(const bf16_t* __restrict__ scores, const void* __restri
 // atomic per element has every query of a batch element adding into the same N x HQ words: 33 M adds into
 // 16 K words took 0.51 ms at B8 L8192 h16 K32.  The table is 64-bit fixed point (2^-40): integer LDS adds
 // run at several times the rate of float ones, and a run's sum does not depend on the order of its adds.
-// (TAB: 16 wavefronts a workgroup, two workgroups a compute unit: the rows of a run are walked one tile after
-// the other, and with four wavefronts a workgroup too few loads were in flight)
+// What bounds it are latencies of memory: a tile's loads are asked for together and, in a run, a tile ahead, before the
+// biases that hang on the indices (d_weights went to LDS one load a latency, nine a tile: 65.7 us at B2 L8192 32/4 heads
+// K32 with the bias, 40.2 now; without the bias 25.8 -> 18.5, B8 L8192 16 heads K32 49.1 -> 34.4).
+// TAB: one workgroup of 16 wavefronts a compute unit; with two the tables' own adds to memory are twice as many (48.8 us).
 template <int LPR, bool TAB>
-__global__ void __launch_bounds__(TAB ? 1024 : 256)
+__global__ void __launch_bounds__(TAB ? 1024 : 256) __attribute__((amdgpu_waves_per_eu(TAB ? 4 : 7)))
 chunk_weights_bwd_rows_kernel(const bf16_t* __restrict__ scores, const void* __restrict__ lse_swa,
                               int lse_bf16, const float* __restrict__ prior_b,
                               const int32_t* __restrict__ indices, const bf16_t* __restrict__ d_weights,
@@ -272,51 +295,80 @@ chunk_weights_bwd_rows_kernel(const bf16_t* __restrict__ scores, const void* __r
     for (int i = threadIdx.x; i < N * HQ; i += NWV * 64) cwb_tab[i] = 0ull;
     __syncthreads();
   }
-  for (int tile = 0; tile < ntile; ++tile) {
-    const long row0 = first + ((long)tile * NWV + wave) * RPW;
-    const long row = row0 + rl;
-    long nrow = last - row0;
-    if (nrow > RPW) nrow = RPW;
-    if (nrow <= 0) break;  // (the wavefront's rows only grow: nothing is left for it)
-    {
-      const int total = (int)nrow * NW;
-      const bf16_t* src = d_weights + row0 * NW;
-      for (int i = lane; i < total; i += 64) stage[wave][i] = src[i];
+  // Everything a tile reads but its biases is asked for a tile ahead (lanes past the last row read that row's)
+  constexpr int PIECES = (RPW * (K + 2) + 63) / 64;
+  const int G = HQ / H;
+  bf16_t dw[PIECES];  // the wavefront's rows of d_weights as they lie in memory
+  uint4 v;
+  float lse_n = 0.f;
+  int idx_n[8], hq_n = 0;
+  long b_n = 0;
+  auto rows_of = [&](int tile, long& row0, int& nrow) __attribute__((always_inline)) {
+    row0 = first + ((long)tile * NWV + wave) * RPW;
+    const long left = last - row0;
+    nrow = left > RPW ? RPW : (int)left;
+    return tile < ntile && left > 0;
+  };
+  auto ask = [&](long row0, int nrow) __attribute__((always_inline)) {
+    const long row = row0 + (rl < nrow ? rl : nrow - 1);
+    const int total = nrow * NW;
+    const bf16_t* src = d_weights + row0 * NW;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const int i = p * 64 + lane;
+      dw[p] = src[i < total ? i : total - 1];
     }
-    // same wavefront wrote the slice: stores and loads of one wavefront stay in program order
-    const bool valid = row < last;
-    float x[8], g[8];
+    v = *(const uint4*)(scores + row * K + sub * 8);
+    lse_n = lse_bf16 ? bf2f(((const bf16_t*)lse_swa)[row]) : ((const float*)lse_swa)[row];
+    if (prior_b) {
+      long bt;
+      gl_row_coords(row, rows, L, HQ, b_n, bt, hq_n);
+      const int32_t* ip = indices + (bt * H + hq_n / G) * (long)K + sub * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) idx_n[e] = ip[e];
+    }
+  };
+  long row0;
+  int nrow;
+  bool more = rows_of(0, row0, nrow);
+  if (more) ask(row0, nrow);
+  for (int tile = 0; more; ++tile) {
+    const bool valid = rl < nrow;
+    const long row = row0 + (valid ? rl : nrow - 1);
+    const int total = nrow * NW;
+    const long b = b_n;
+    const int hq = hq_n;
+    const float lse = lse_n;
+    float x[8], g[8], bias[8];
     int cidx[8];
-    float lse = HILS_NEG_INF, gl = 0.f, g0 = 0.f;
-    int hq = 0;
-    long b = 0;
-    if (valid) {
-      const uint4 v = *(const uint4*)(scores + row * K + sub * 8);
-      unpack8(v, x);
-      lse = lse_bf16 ? bf2f(((const bf16_t*)lse_swa)[row]) : ((const float*)lse_swa)[row];
-      const bf16_t* st = stage[wave] + rl * NW;
+    if (prior_b) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) g[e] = bf2f(st[sub * 8 + e]);
-      gl = bf2f(st[K]);
-      if (softmax1) g0 = bf2f(st[K + 1]);
-      if (prior_b) {
-        hq = (int)(row % HQ);
-        const long bt = row / HQ;
-        b = bt / L;
-        const int G = HQ / H;
-        const int32_t* ip = indices + (bt * H + hq / G) * (long)K + sub * 8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          int c = ip[e];
-          c = c < 0 ? 0 : c;
-          cidx[e] = c;
-          x[e] = bf2f(f2bf(x[e] + bf2f(f2bf(prior_b[(b * N + c) * (long)HQ + hq]))));
-        }
+      for (int e = 0; e < 8; ++e) {
+        cidx[e] = idx_n[e] < 0 ? 0 : idx_n[e];
+        bias[e] = prior_b[(b * N + cidx[e]) * (long)HQ + hq];
       }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { x[e] = HILS_NEG_INF; g[e] = 0.f; }
     }
+    unpack8(v, x);
+    // one wavefront writes and reads the slice: its stores and loads stay in program order
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+      if (p * 64 + lane < total) stage[wave][p * 64 + lane] = dw[p];
+    __builtin_amdgcn_wave_barrier();
+    const bf16_t* st = stage[wave] + (row - row0) * NW;
+    if (TAB) {
+      more = rows_of(tile + 1, row0, nrow);
+      if (more) ask(row0, nrow);
+    } else {
+      more = false;
+    }
+    if (prior_b) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = bf2f(f2bf(x[e] + bf2f(f2bf(bias[e]))));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = bf2f(st[sub * 8 + e]);
+    const float gl = bf2f(st[K]), g0 = softmax1 ? bf2f(st[K + 1]) : 0.f;
     float m = softmax1 ? fmaxf(lse, 0.f) : lse;
 #pragma unroll
     for (int e = 0; e < 8; ++e) m = fmaxf(m, x[e]);
@@ -388,12 +440,12 @@ extern "C" int hils_chunk_weights_bwd(const void* scores, const void* lse_swa, i
     const int rpw = 64 / (K / 8);
     const long nb = (rows + 4 * rpw - 1) / (4 * rpw);
     HILS_REQUIRE(nb <= 2147483647L, "hils_chunk_weights_bwd: grid too large");
-    // with a bias gradient whose table fits the LDS: runs of rows per workgroup, about two workgroups a
-    // compute unit, each run long enough that its adds outnumber the table it flushes
+    // with a bias gradient whose table fits the LDS: runs of rows per workgroup, one workgroup a
+    // compute unit (two: 48.8 us against 40.2 at B2 L8192 32 heads K32), each run long enough that its adds outnumber the table it flushes
     const size_t tab_b = (size_t)N * HQ * sizeof(unsigned long long);
     if (d_prior_b && tab_b <= 48 * 1024) {
       const long tiles_b = ((long)L * HQ + 16 * rpw - 1) / (16 * rpw);  // 16-wavefront tiles of a batch element
-      long segs = 2L * hils_device_cus() / B;
+      long segs = hils_device_cus() / B;
       if (segs < 1) segs = 1;
       if (segs > tiles_b) segs = tiles_b;
       const int tiles_per_wg = (int)((tiles_b + segs - 1) / segs);

@@ -49,6 +49,16 @@ def test_chunk_weights_kernel(pkg, orc, dev):
     _chunk_weights_case(pkg, orc, dev, 8, dims=(1, 9001, 6, 3, 141))
 
 
+@pytest.mark.parametrize("K,dims", [(8, (2, 33, 3, 3, 5)), (16, (2, 2777, 3, 3, 40)), (32, (3, 8001, 5, 1, 17)), (64, (1, 3001, 7, 7, 64)),
+                                    (32, (300, 7, 2, 1, 3))])
+def test_chunk_weights_runs_of_odd_rows(pkg, orc, dev, K, dims):
+    """Odd numbers of rows a batch element (slices of d_weights at odd elements), one to many tiles a run with a ragged
+    last one, wavefronts without rows, more batch elements than compute units."""
+    note(f"chunk_weights runs K={K} {dims}")
+    torch.manual_seed(5)
+    _chunk_weights_case(pkg, orc, dev, K, dims=dims)
+
+
 def _chunk_weights_case(pkg, orc, dev, K, dims=(2, 301, 8, 2, 40)):
     B, L, HQ, H, N = dims
     scores = torch.randn(B, L, HQ, K).bfloat16()
