@@ -3243,8 +3243,11 @@ topk_bwd_dlmk_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q
 // columns (A for A^T, chunk keys and query rows as right operands) comes by the transposing LDS load, in whose order of
 // rows the other operand is read too.  No inverse index, every input read once and coalesced.  (With A twice and keys
 // and rows feature-major, two-byte stores to a quarter of the banks were two thirds of the LDS time and 102 KiB allowed one
-// workgroup per compute unit; 71 KiB are two: B8 L8192 16 heads of 64, top-32: 294 -> 172 us.)  dlmk tiles of the query blocks are added with
-// float atomics (the summation order over query blocks is not fixed).  The chunk indices of one
+// workgroup per compute unit; 71 KiB are two: B8 L8192 16 heads of 64, top-32: 294 -> 172 us.)  Where the chunks fit one tile a
+// workgroup walks several query blocks and adds its dlmk up in registers, the next block's loads behind this block's
+// products; a block's 32 KB of atomics (D = 64), 268 MB in the call above, were a third of the time.  One block / a walk, us:
+// that call 180 / 151, B2 L8192 32 heads of 64 with a key each 76 / 65, L8192 32/8 heads of 128 82 / 57, L4001 of the
+// same top-8 36 / 29.  dlmk leaves by float atomics (the summation order over workgroups is not fixed).  The chunk indices of one
 // row must be distinct (they are when they come from the selection).
 #define TD_R 128        // rows per workgroup
 #define TD_NC 128       // chunks per tile (== TD_R: one thread-to-piece split serves rows and chunk keys)
@@ -3252,11 +3255,11 @@ topk_bwd_dlmk_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q
 #define TD_STRIDE 136   // elements per row of A: 128 + 8
 
 template <int D>
-__global__ void __launch_bounds__(TD_THREADS)
+__global__ void __launch_bounds__(TD_THREADS) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q,
                       const bf16_t* __restrict__ lmks, const int32_t* __restrict__ indices,
                       bf16_t* __restrict__ dq, float* __restrict__ dlmk, int L, int N, int h_kv, int G,
-                      int topk, int per_qhead, float sm_scale, uint32_t k_magic, int g_sh) {
+                      int topk, int per_qhead, float sm_scale, uint32_t k_magic, int g_sh, int walk) {
   constexpr int DT = D / 16, PPR = D / 8;
   constexpr int RS = D + 8;                   // elements per staged row
   extern __shared__ __align__(16) bf16_t td_sm[];
@@ -3264,7 +3267,8 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   bf16_t* L_s = A_s + TD_R * TD_STRIDE;       // [TD_NC][RS]  chunk keys of the tile
   bf16_t* Q_s = L_s + TD_NC * RS;             // [TD_R][RS]   query rows
   __shared__ int cmax_s;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   // grid order (chunk-key head, batch) fastest, query block slowest: the workgroups in flight at
   // one time add their dlmk tiles to different (batch, head) slices instead of all to the same one
@@ -3274,7 +3278,9 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   const int hk = per_qhead ? lh / G : lh;
   const int g_lo = per_qhead ? lh % G : 0, g_n = 1 << g_sh;  // (a divisor of TD_R)
   const int TQ = TD_R >> g_sh;
-  const int t0 = blockIdx.z * TQ;
+  int t0 = blockIdx.z * walk * TQ;
+  int n_blk = (L - t0 + TQ - 1) / TQ;  // query blocks of this workgroup (the host takes one where N > TD_NC)
+  n_blk = n_blk < walk ? n_blk : walk;
   auto row_rg = [&](int row) -> long {  // row of gs / q / dq of a block row (valid rows only)
     return ((b * L + t0 + (row >> g_sh)) * h_kv + hk) * (long)G + g_lo + (row & (g_n - 1));
   };
@@ -3286,15 +3292,15 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   constexpr int NI = 8;                        // (row, slot) entries per thread and batch
   const int n_item = TD_R * topk;              // entries of the block, row-major like gs
   uint4 qx[NP], lx[NP];
+  auto ask_rows = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < NP; ++u) {
-    const int i = tid + u * TD_THREADS;
-    const int row = i / PPR, pc = i % PPR;     // the pieces of a row sit in neighbouring lanes
-    const int rc = (t0 + (row >> g_sh) < L) ? row : 0;  // row 0 of a block always exists
-    qx[u] = *(const uint4*)(q + row_rg(rc) * D + pc * 8);
-    const int cc = row < N ? row : N - 1;      // TD_NC == TD_R: the same split serves the chunk keys
-    lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
-  }
+    for (int u = 0; u < NP; ++u) {
+      const int i = tid + u * TD_THREADS;
+      const int row = i / PPR, pc = i % PPR;   // the pieces of a row sit in neighbouring lanes
+      const int rc = (t0 + (row >> g_sh) < L) ? row : 0;  // row 0 of a block always exists
+      qx[u] = *(const uint4*)(q + row_rg(rc) * D + pc * 8);
+    }
+  };
   auto item_load = [&](int i, int& c, bf16_t& val) {  // entry i of the block (any i: clamped)
     const int ic = i < n_item ? i : 0;
     const int row = (int)hils_udiv((uint32_t)ic, (uint32_t)topk, k_magic), slot = ic - row * topk;
@@ -3306,15 +3312,19 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   };
   int ci[NI];
   bf16_t gv[NI];
+  auto ask_items = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < NI; ++u) item_load(tid + u * TD_THREADS, ci[u], gv[u]);
+    for (int u = 0; u < NI; ++u) item_load(i0 + tid + u * TD_THREADS, ci[u], gv[u]);
+  };
+  ask_rows();
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
     const int i = tid + u * TD_THREADS;
     const int row = i / PPR, pc = i % PPR;
-    const bool ok = t0 + (row >> g_sh) < L;
-    *(uint4*)(Q_s + row * RS + pc * 8) = ok ? qx[u] : make_uint4(0, 0, 0, 0);
+    const int cc = row < N ? row : N - 1;      // TD_NC == TD_R: the same split serves the chunk keys
+    lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
   }
+  ask_items(0);
   // Operand of columns c0 .. c0 + 15 over the rows r0 .. r0 + 31: a lane's eight values are column c0 + col of the rows
   // 4j .. 4j + 3 and 16 + 4j .. (transposing load: lane l of a 16-lane group addresses row l/4, columns 4*(l%4) .. +3)
   typedef short td_s4 __attribute__((ext_vector_type(4)));
@@ -3324,79 +3334,103 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
     const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) td_s4*)(p + 16 * stride)));
     return make_uint4(x.x, x.y, y.x, y.y);
   };
-  f32x4_t acc_q[DT];
-#pragma unroll
-  for (int t = 0; t < DT; ++t) acc_q[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  int cmax = 0;
-  for (int c0 = 0; c0 <= cmax; c0 += TD_NC) {
-    for (int i = tid; i < TD_R * TD_STRIDE / 8; i += TD_THREADS) ((uint4*)A_s)[i] = make_uint4(0, 0, 0, 0);
-    // chunk keys of the tile
+  f32x4_t acc_l[DT];  // dlmk of this wavefront's chunk tile
+  int c_seen = -1;    // largest chunk index of the blocks so far
+  for (int blk = 0; blk < n_blk; ++blk) {
+    // (hidden from the compiler, which would keep the addresses of all pieces and entries in registers: 190 of them,
+    // one workgroup per compute unit instead of two)
+    if constexpr (D == 64) asm volatile("" : "+v"(tid));
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
       const int i = tid + u * TD_THREADS;
-      const int cl = i / PPR, pc = i % PPR;
-      if (c0 > 0) {
-        const int cc = c0 + cl < N ? c0 + cl : N - 1;
-        lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
-      }
-      const bool ok = c0 + cl < N;
-      *(uint4*)(L_s + cl * RS + pc * 8) = ok ? lx[u] : make_uint4(0, 0, 0, 0);
+      const int row = i / PPR, pc = i % PPR;
+      const bool ok = t0 + (row >> g_sh) < L;
+      *(uint4*)(Q_s + row * RS + pc * 8) = ok ? qx[u] : make_uint4(0, 0, 0, 0);
     }
-    __syncthreads();
-    int my_max = -1;
-    for (int i0 = 0; i0 < n_item; i0 += NI * TD_THREADS) {
-      if (i0 > 0 || c0 > 0) {
+    f32x4_t acc_q[DT];
 #pragma unroll
-        for (int u = 0; u < NI; ++u) item_load(i0 + tid + u * TD_THREADS, ci[u], gv[u]);
-      }
+    for (int t = 0; t < DT; ++t) acc_q[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int t0_blk = t0;
+    int cmax = 0;
+    for (int c0 = 0; c0 <= cmax; c0 += TD_NC) {
+      for (int i = tid; i < TD_R * TD_STRIDE / 8; i += TD_THREADS) ((uint4*)A_s)[i] = make_uint4(0, 0, 0, 0);
+      if (blk == 0) {  // chunk keys of the tile (a workgroup of several blocks has one tile)
 #pragma unroll
-      for (int u = 0; u < NI; ++u) {
-        const int c = ci[u];
-        my_max = c > my_max ? c : my_max;
-        if (c >= c0 && c < c0 + TD_NC) {
-          const int row = (int)hils_udiv((uint32_t)(i0 + tid + u * TD_THREADS), (uint32_t)topk, k_magic);
-          A_s[row * TD_STRIDE + (c - c0)] = gv[u];
+        for (int u = 0; u < NP; ++u) {
+          const int i = tid + u * TD_THREADS;
+          const int cl = i / PPR, pc = i % PPR;
+          if (c0 > 0) {
+            const int cc = c0 + cl < N ? c0 + cl : N - 1;
+            lx[u] = *(const uint4*)(lmks + ((b * N + cc) * (long)lmk_h + lh) * D + pc * 8);
+          }
+          const bool ok = c0 + cl < N;
+          *(uint4*)(L_s + cl * RS + pc * 8) = ok ? lx[u] : make_uint4(0, 0, 0, 0);
         }
       }
-    }
-    if (c0 == 0) {  // largest chunk index of the block: how many tiles there are
+      __syncthreads();
+      int my_max = -1;
+      for (int i0 = 0; i0 < n_item; i0 += NI * TD_THREADS) {
+        if (i0 > 0 || c0 > 0) ask_items(i0);
 #pragma unroll
-      for (int o2 = 32; o2 >= 1; o2 >>= 1) {
-        const int y = __shfl_xor(my_max, o2, 64);
-        my_max = y > my_max ? y : my_max;
-      }
-      if (lane == 0 && my_max >= 0) atomicMax(&cmax_s, my_max);
-    }
-    __syncthreads();
-    cmax = cmax_s;
-    if (cmax >= c0) {  // (the first tile of a block with no valid entry has nothing to add)
-      // dq rows of this wavefront's row tile += A LMK
-#pragma unroll
-      for (int kc = 0; kc < TD_NC / 32; ++kc) {
-        const bf16_t* ap = A_s + (wave * 16 + col) * TD_STRIDE + kc * 32 + 4 * j;
-        const uint2 a0 = *(const uint2*)ap, a1 = *(const uint2*)(ap + 16);
-        const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
-#pragma unroll
-        for (int t = 0; t < DT; ++t) {
-          const uint4 bb = cols(L_s, RS, kc * 32, t * 16);
-          acc_q[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_q[t], 0, 0, 0);
-        }
-      }
-      // dlmk of this wavefront's chunk tile = A^T Q
-      const int c_tile = c0 + wave * 16;
-      if (c_tile <= cmax) {
-        f32x4_t acc_l[DT];
-#pragma unroll
-        for (int t = 0; t < DT; ++t) acc_l[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kr = 0; kr < TD_R / 32; ++kr) {
-          const uint4 a = cols(A_s, TD_STRIDE, kr * 32, wave * 16);
-#pragma unroll
-          for (int t = 0; t < DT; ++t) {
-            const uint4 bb = cols(Q_s, RS, kr * 32, t * 16);
-            acc_l[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_l[t], 0, 0, 0);
+        for (int u = 0; u < NI; ++u) {
+          const int c = ci[u];
+          my_max = c > my_max ? c : my_max;
+          if (c >= c0 && c < c0 + TD_NC) {
+            const int row = (int)hils_udiv((uint32_t)(i0 + tid + u * TD_THREADS), (uint32_t)topk, k_magic);
+            A_s[row * TD_STRIDE + (c - c0)] = gv[u];
           }
         }
+      }
+      if (c0 == 0) {  // largest chunk index of the block: how many tiles there are
+#pragma unroll
+        for (int o2 = 32; o2 >= 1; o2 >>= 1) {
+          const int y = __shfl_xor(my_max, o2, 64);
+          my_max = y > my_max ? y : my_max;
+        }
+        if (lane == 0 && my_max >= 0) atomicMax(&cmax_s, my_max);
+      }
+      __syncthreads();
+      cmax = cmax_s;
+      const bool last = blk + 1 == n_blk;
+      if (!last) {  // what the next block reads is asked for behind this block's products
+        t0 += TQ;
+        if constexpr (D == 64) asm volatile("" : "+v"(tid));
+        ask_rows();
+        ask_items(0);
+      }
+      const int c_tile = c0 + wave * 16;
+      if (blk == 0) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t) acc_l[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      }
+      if (cmax >= c0) {  // (the first tile of a block with no valid entry has nothing to add)
+        // dq rows of this wavefront's row tile += A LMK
+#pragma unroll
+        for (int kc = 0; kc < TD_NC / 32; ++kc) {
+          const bf16_t* ap = A_s + (wave * 16 + col) * TD_STRIDE + kc * 32 + 4 * j;
+          const uint2 a0 = *(const uint2*)ap, a1 = *(const uint2*)(ap + 16);
+          const uint4 a = make_uint4(a0.x, a0.y, a1.x, a1.y);
+#pragma unroll
+          for (int t = 0; t < DT; ++t) {
+            const uint4 bb = cols(L_s, RS, kc * 32, t * 16);
+            acc_q[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_q[t], 0, 0, 0);
+          }
+        }
+        // dlmk of this wavefront's chunk tile += A^T Q
+        if (c_tile <= cmax) {
+#pragma unroll
+          for (int kr = 0; kr < TD_R / 32; ++kr) {
+            const uint4 a = cols(A_s, TD_STRIDE, kr * 32, wave * 16);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+              const uint4 bb = cols(Q_s, RS, kr * 32, t * 16);
+              acc_l[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8_t*)&a, *(const bf16x8_t*)&bb, acc_l[t], 0, 0, 0);
+            }
+          }
+        }
+      }
+      c_seen = cmax > c_seen ? cmax : c_seen;
+      if (last && c_tile <= c_seen) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int c = c_tile + 4 * j + i;
@@ -3410,16 +3444,18 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
           }
         }
       }
+      __syncthreads();  // the tile is no longer read
     }
-    __syncthreads();  // the tile is no longer read
-  }
+    if (tid == 0) cmax_s = -1;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = wave * 16 + 4 * j + i;
-    if (t0 + (row >> g_sh) < L) {
-      bf16_t* dst = dq + row_rg(row) * D + col;
+    for (int i = 0; i < 4; ++i) {
+      const int row = wave * 16 + 4 * j + i;
+      const int t = t0_blk + (row >> g_sh);
+      if (t < L) {
+        bf16_t* dst = dq + (((b * L + t) * h_kv + hk) * (long)G + g_lo + (row & (g_n - 1))) * D + col;
 #pragma unroll
-      for (int t = 0; t < DT; ++t) dst[t * 16] = f2bf(acc_q[t][i] * sm_scale);
+        for (int d = 0; d < DT; ++d) dst[d * 16] = f2bf(acc_q[d][i] * sm_scale);
+      }
     }
   }
 }
@@ -3433,12 +3469,22 @@ template <int D>
 static int topk_bwd_dense_launch(dim3 grid, hipStream_t st, const bf16_t* gs, const bf16_t* q, const bf16_t* lmks,
                                  const int32_t* indices, bf16_t* dq, float* dlmk, int L, int N, int h_kv, int G,
                                  int topk, int per_qhead, float sm_scale) {
+  // As many query blocks a workgroup as let all workgroups fit the chip at once (by their LDS two per compute unit with
+  // heads of 64, one with 128), where the chunks fit one tile.  With twice / four times the workgroups: B8 L8192 16
+  // heads of 64 top-32 153 / 151 us, B2 L8192 32 heads of 64 65 / 66, L8192 32/8 heads of 128 63 -> 69 / 73.
+  int walk = 1;
+  if (N <= TD_NC) {
+    const long blocks = (long)grid.x * grid.y * grid.z, fit = (D == 64 ? 2 : 1) * (long)hils_device_cus();
+    const long w = (blocks + fit - 1) / fit;
+    walk = w < (long)grid.z ? (int)w : (int)grid.z;
+    grid.z = (grid.z + walk - 1) / walk;
+  }
   const size_t smem = ((size_t)TD_R * TD_STRIDE + (size_t)(TD_R + TD_NC) * (D + 8)) * sizeof(bf16_t);
   auto kern = topk_bwd_dense_kernel<D>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_topk_bwd")) return rc;
   hipLaunchKernelGGL(kern, grid, dim3(TD_THREADS), smem, st, gs, q, lmks, indices, dq, dlmk, L, N, h_kv, G, topk,
-                     per_qhead, sm_scale, hils_udiv_magic((uint32_t)topk), __builtin_ctz(per_qhead ? 1 : G));
+                     per_qhead, sm_scale, hils_udiv_magic((uint32_t)topk), __builtin_ctz(per_qhead ? 1 : G), walk);
   return HILS_OK;
 }
 

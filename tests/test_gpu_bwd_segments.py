@@ -148,3 +148,39 @@ def test_swa_backward_split(pkg, dev, B, L, HQ, H, D, W):
     for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), (o, lse, *got), (ro, rl, *ref)):
         err = (a.float() - b).norm() / b.norm()
         assert err < 1.5e-2, (name, err.item())
+
+
+# the score gather's backward by dense products: one query block a workgroup, walks of two to many with a ragged last one,
+# blocks without any entry, exactly one tile of chunks and one more (which is not walked)
+@pytest.mark.parametrize("B,L,N,H,G,D,K,per_qhead", [(1, 40, 3, 1, 1, 64, 2, 0), (2, 3001, 128, 16, 1, 64, 8, 0), (2, 3001, 129, 16, 1, 64, 8, 0),
+                                                     (3, 1037, 16, 2, 16, 64, 5, 1), (1, 2500, 40, 8, 4, 128, 16, 0),
+                                                     (9, 700, 11, 8, 4, 128, 33, 1), (4, 9001, 100, 4, 2, 64, 3, 0)])
+def test_dense_gather_backward_walks(pkg, dev, B, L, N, H, G, D, K, per_qhead):
+    from hils_attention_amd.ops import _cabi
+    lib, HK = _cabi.load(), H * G if per_qhead else H
+    gen = torch.Generator(device=dev).manual_seed(L + N)
+    q = torch.randn(B, L, H, G, D, device=dev, generator=gen).bfloat16()
+    lmks = torch.randn(B, N, HK, D, device=dev, generator=gen).bfloat16()
+    g = torch.randn(B, L, H, G, K, device=dev, generator=gen).bfloat16()
+    score = torch.rand(B, L, H, max(N, K), device=dev, generator=gen)
+    idx = score.topk(K, -1).indices
+    idx = idx.masked_fill(idx >= N, -1)
+    idx[:, 100:400] = -1
+    idx = idx.int().contiguous()
+    dq, dlmk = torch.empty_like(q), torch.zeros(B, N, HK, D, device=dev)
+    rc = lib.hils_topk_bwd(_cabi.ptr(g), _cabi.ptr(q), _cabi.ptr(lmks), _cabi.ptr(idx), _cabi.ptr(dq), _cabi.ptr(dlmk),
+                           None, 0, B, L, N, H, G, D, K, per_qhead, 0.125, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    live = (idx >= 0).unsqueeze(3)
+    a = torch.zeros(B, L, H, G, N, dtype=torch.float64, device=dev)
+    a.scatter_add_(4, idx.clamp(min=0).long().unsqueeze(3).expand(B, L, H, G, K), (g.double() * 0.125).masked_fill(~live, 0.))
+    a = a.permute(0, 2, 3, 1, 4).reshape(B, HK, -1, N)  # rows of a chunk-key head
+    rows = q.double().permute(0, 2, 3, 1, 4).reshape(B, HK, -1, D)
+    keys = lmks.double().permute(0, 2, 1, 3).contiguous()
+    want_q = (a @ keys).reshape(B, H, G, L, D).permute(0, 3, 1, 2, 4)
+    size_q = (a.abs() @ keys.abs()).reshape(B, H, G, L, D).permute(0, 3, 1, 2, 4)
+    at = a.transpose(2, 3).contiguous()
+    want_l, size_l = (at @ rows).permute(0, 2, 1, 3), (at.abs() @ rows.abs()).permute(0, 2, 1, 3)
+    # fp32 sums of n terms are within n 2^-24 of their terms' absolute sum; dq is then rounded to eight bits
+    assert bool(((dq.double() - want_q).abs() <= want_q.abs() * 2.0 ** -8 + (K + 1) * 2.0 ** -23 * size_q + 1e-30).all())
+    assert bool(((dlmk.double() - want_l).abs() <= (L * G + 1) * 2.0 ** -24 * size_l + 1e-30).all())
