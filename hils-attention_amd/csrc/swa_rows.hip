@@ -248,6 +248,8 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
 //   two blocks:  heads of 64, 512  7.8/15  15/17  26/41  49/79;  256  5.4/11  9/11  17/25  31/49;  128  5.5/8.5  7/9  13/10  23/21
 //   eight:       heads of 64 (16 queries of eight heads), 512  -  15/15  27/16  48/18;  64  -  5.6/6.7  10/7  18/7
 //   four:        heads of 128 (16 queries of four heads), 512  15/21  27/23  52/25;  64  5.6/8.2  11/8  21/9
+// Both round probabilities to bf16 and sum in fp32; outputs of 900 queries of eight heads of 64, window 512, are 1.94e-3 /
+// 2.04e-3 (relative) from 64 bits, of which their own rounding to bf16 is 1.7e-3.
 bool hils_swa_rows_better(int B, int D, int Dv, const SwaDims& dm) {
   if (B > 65535 || dm.H > 65535) return false;  // (dimensions of the row kernel's grid)
   const int QB = 16 / (dm.HQ / dm.H);
