@@ -248,15 +248,20 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
 //   two blocks:  heads of 64, 512  7.8/15  15/17  26/41  49/79;  256  5.4/11  9/11  17/25  31/49;  128  5.5/8.5  7/9  13/10  23/21
 //   eight:       heads of 64 (16 queries of eight heads), 512  -  15/15  27/16  48/18;  64  -  5.6/6.7  10/7  18/7
 //   four:        heads of 128 (16 queries of four heads), 512  15/21  27/23  52/25;  64  5.6/8.2  11/8  21/9
-// Both round probabilities to bf16 and sum in fp32; outputs of 900 queries of eight heads of 64, window 512, are 1.94e-3 /
-// 2.04e-3 (relative) from 64 bits, of which their own rounding to bf16 is 1.7e-3.
+// The line is not the times' alone.  Both round probabilities to bf16 and sum in fp32, but the row kernel takes them about
+// each wavefront's own maximum, whose probability is exactly 1, the tile kernel about a reference point that lags behind the
+// maximum: from 64 bits, relative, window 512, row / tile kernel 2.06e-3 / 2.28e-3 (32/8 heads of 128, 160 to 256
+// queries; 16/2 of 64, 900 queries: 2.05 / 2.27; about the maximum itself the tile kernel has 2.16), window 64 2.02 / 2.08,
+// 1.66 of each the output's own rounding.  So calls of up to 512 workgroups, and up to 1024 with narrow heads and a
+// long window, stay with the row kernel also where the tile kernel would be ahead (20 / 18 us and 19 / 13 us of the
+// two above).
 bool hils_swa_rows_better(int B, int D, int Dv, const SwaDims& dm) {
   if (B > 65535 || dm.H > 65535) return false;  // (dimensions of the row kernel's grid)
   const int QB = 16 / (dm.HQ / dm.H);
   const long n_rb = (dm.Lq + QB - 1) / QB, wgs = n_rb * dm.H * B;
-  const bool narrow = D <= 64 && Dv <= 64;
-  if (wgs <= (narrow ? 512 : 256)) return true;
-  return dm.window >= 256 ? n_rb <= (narrow ? 2 : 1) : narrow && n_rb == 1;
+  const bool narrow = D <= 64 && Dv <= 64, wide_window = dm.window >= 256;
+  if (wgs <= (narrow && wide_window ? 1024 : 512)) return true;
+  return wide_window ? n_rb <= (narrow ? 2 : 1) : narrow && n_rb == 1;
 }
 
 int hils_swa_fwd_rows(int B, hipStream_t st, const void* q, const void* k, const void* v, void* o, float* lse, int D,

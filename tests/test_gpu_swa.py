@@ -212,3 +212,29 @@ def test_local_and_remote_branch_sum_to_dense_attention(pkg, dev, L, HQ, H, D, W
     (1, 705, 16, 1, 128, 64, 320, 64, False, True), (1, 530, 2, 1, 64, 128, 500, 64, True, True)])
 def test_swa_backward_whole_tiles(pkg, orc, dev, B, L, HQ, H, D, Dv, W, S, mask_lmk, expand):
     _forward_backward(pkg, orc, dev, B, L, HQ, H, D, Dv, W, S, mask_lmk, expand)
+
+
+# A few hundred new tokens on a cache, or a few a sequence: the error is below that of probabilities rounded to bf16 once, about
+# their row's maximum, and an output rounded to bf16 (both formed here in 64 bits)
+@pytest.mark.parametrize("B,Lq,HQ,H,D,Dv,W", [(1, 160, 32, 8, 128, 128, 512), (20, 8, 32, 8, 128, 128, 512), (1, 700, 16, 16, 64, 64, 512),
+                                              (1, 900, 16, 2, 64, 64, 512), (24, 8, 32, 8, 64, 128, 512), (48, 4, 32, 8, 128, 64, 64)])
+def test_swa_few_rows_precision(pkg, dev, B, Lq, HQ, H, D, Dv, W):
+    Lk = Lq + 700
+    gen = torch.Generator(device=dev).manual_seed(5)
+    r = lambda *s: torch.randn(*s, device=dev, generator=gen).bfloat16()
+    q, k, v = r(B, Lq, HQ, D), r(B, Lk, H, D), r(B, Lk, H, Dv)
+    o, _ = pkg.flex_attn_tl(q, k, v, W, 64, training=False, mask_lmk=False)
+    t, j = torch.arange(Lq, device=dev) + Lk - Lq, torch.arange(Lk, device=dev)
+    start = (t - W + 1).div(64, rounding_mode="floor") * 64
+    hidden = (j > t[:, None]) | (j < start[:, None])
+    err = bound = 0.0
+    for b in range(min(B, 3)):
+        q6, k6, v6 = (x[b].double().repeat_interleave(HQ // x.shape[2], 1).transpose(0, 1).contiguous() for x in (q, k, v))
+        s = ((q6 @ k6.transpose(1, 2).contiguous()) * D ** -0.5).masked_fill(hidden, float("-inf"))
+        p = (s - s.amax(-1, keepdim=True)).exp()
+        total = p.sum(-1, keepdim=True)
+        ref = p @ v6 / total
+        once = (p.float().bfloat16().double() @ v6 / total).bfloat16().double()
+        err += (o[b].double().transpose(0, 1) - ref).square().sum().item()
+        bound += (once - ref).square().sum().item()
+    assert err <= bound, (err / bound) ** 0.5
