@@ -106,11 +106,11 @@ __device__ __forceinline__ unsigned lz_lds_addr(const unsigned char* p) {
 }
 // 64 pieces of 16 bytes, lane i's from base + off to lds + 16 i
 __device__ __forceinline__ void lz_dma16(unsigned lds, unsigned off, unsigned long long base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 // 64 words, lane i's from addr to lds + 4 i
 __device__ __forceinline__ void lz_dma4(unsigned lds, unsigned long long addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(addr) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(addr) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void lz_landed() {  // all but the last N vector-memory operations

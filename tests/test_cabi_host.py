@@ -227,3 +227,15 @@ def test_short_workspace_is_rejected_by_the_c_abi(pkg):
     assert need_tb > 0
     rc = lib.hils_topk_bwd(buf, buf, buf, buf, buf, buf, buf, need_tb - 1, B, L, N, h_kv, 3, D, K, 0, 0.088, None)
     assert rc == 1 and b"shorter" in lib.hils_last_error()
+
+
+def test_inline_assembly_declares_m0():
+    """A statement of inline assembly that writes M0 names it among the registers it changes."""
+    csrc = os.path.join(entry.PKG_DIR, "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        for stmt in re.findall(r"\basm\b[^;]*;", open(os.path.join(csrc, name)).read()):
+            if re.search(r"\bs_mov_b32 m0\b", stmt):
+                found += 1
+                assert '"m0"' in stmt.rsplit(":", 1)[1], f"{name}: {stmt}"
+    assert found
