@@ -816,9 +816,11 @@ logz_bwd_dk_simple(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   }
 }
 
-// shapes of the matrix-core kernels: 64-token chunks, head dim 64/128, group size dividing 16
-static bool lz_mfma_covers(int G, int D, int S, int H, int B) {
-  return S == 64 && (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) &&
+// shapes of the matrix-core kernels: 64-token chunks, head dim 64/128, group size dividing 16, and a window that is not
+// negative: with one a query's walk takes in chunks that end behind it, of which it sees a part, and the ragged last chunk,
+// whose rows the kernels would read past the end of the keys
+static bool lz_mfma_covers(int G, int D, int S, int H, int B, int W) {
+  return S == 64 && W >= 0 && (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) &&
          H <= 65535 && B <= 65535;
 }
 // expands LZ_LAUNCH(D, G) for the covered (D, G)
@@ -848,7 +850,7 @@ extern "C" int hils_chunk_logz_fwd(const void* q, const void* k, float* log_z, i
   if (int rc = lz_check("hils_chunk_logz_fwd", B, L, HQ, H, D, S)) return rc;
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, mask_lmk, sm_scale};
   const int G = HQ / H;
-  if (lz_mfma_covers(G, D, S, H, B)) {
+  if (lz_mfma_covers(G, D, S, H, B, window)) {
     const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;
     HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_fwd: B * H * L too large for the grid");
@@ -875,7 +877,7 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   if (int rc = lz_check("hils_chunk_logz_bwd_dq", B, L, HQ, H, D, S)) return rc;
   HILS_REQUIRE(D <= LZ_THREADS, "hils_chunk_logz_bwd_dq: D (%d) must be <= %d", D, LZ_THREADS);
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, 0, sm_scale};
-  if (lz_mfma_covers(HQ / H, D, S, H, B)) {
+  if (lz_mfma_covers(HQ / H, D, S, H, B, window)) {
     const int G = HQ / H;
     const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;
@@ -925,7 +927,7 @@ static LzSeg lz_segments(int B, int L, int G, int H, int N, int W) {
   return sg;
 }
 extern "C" size_t hils_chunk_logz_bwd_dk_workspace(int B, int L, int HQ, int H, int D, int S, int window) {
-  if (B <= 0 || L <= 0 || H <= 0 || HQ <= 0 || HQ % H != 0 || !lz_mfma_covers(HQ / H, D, S, H, B)) return 0;
+  if (B <= 0 || L <= 0 || H <= 0 || HQ <= 0 || HQ % H != 0 || !lz_mfma_covers(HQ / H, D, S, H, B, window)) return 0;
   const int N = (L + S - 1) / S;
   const LzSeg sg = lz_segments(B, L, HQ / H, H, N, window);
   return sg.max_seg == 1 ? 0 : (size_t)B * H * ((N + 1) / 2) * sg.max_seg * 128 * D * sizeof(float);
@@ -940,7 +942,7 @@ extern "C" int hils_chunk_logz_bwd_dk_ws(const void* q, const void* k, const flo
   const int G = HQ / H;
   HILS_REQUIRE(S * D <= LZ_MAX_ACC * LZ_THREADS, "hils_chunk_logz_bwd_dk: S*D (%d) too large", S * D);
   LzDims dm{L, HQ, H, G, D, S, window, (L + S - 1) / S, 0, sm_scale};
-  if (lz_mfma_covers(G, D, S, H, B)) {
+  if (lz_mfma_covers(G, D, S, H, B, window)) {
     const int n_pair = (dm.N + 1) / 2;
     HILS_REQUIRE(((long)B * H + 8) * (n_pair + 8) * 8 < (1L << 31), "hils_chunk_logz_bwd_dk: B * H * N too large for the grid");
     const int n_unit = B * H;

@@ -1,5 +1,5 @@
 """Exact log Z and dQ: walks of one to nine chunks (the kernels take four steps a round and load three ahead), keys whose
-sums jump between neighbouring chunks, the landmark mask."""
+sums jump between neighbouring chunks, the landmark mask, negative windows."""
 import pytest
 import torch
 
@@ -27,6 +27,26 @@ def test_walks(pkg, orc, dev, HQ, H, D, chunks, rest, mask_lmk):
     assert_close_f32(z.detach(), ref.detach(), LSE_TOL, "log_z")
     if mask_lmk:
         return  # forward only
+    finite = torch.isfinite(ref)
+    g = torch.randn(ref.shape, generator=gen) * finite
+    z.backward(g.to(dev))
+    torch.where(finite, ref, torch.zeros(())).mul(g).sum().backward()
+    assert_close_bf16(qd.grad, qf.grad, "dq")
+    assert_close_bf16(kd.grad, kf.grad, "dk")
+
+
+@pytest.mark.parametrize("HQ,H,D", [(4, 2, 64), (16, 1, 128)])
+@pytest.mark.parametrize("L,W", [(215, -1), (215, -40), (130, -63), (193, -200)])
+def test_negative_window(pkg, orc, dev, HQ, H, D, L, W):
+    """Chunks that end behind a query are visible to it up to the query itself, a ragged last one up to its end."""
+    note(f"log Z, window {W}, L{L} heads {HQ}/{H} x {D}")
+    gen = torch.Generator().manual_seed(L - W)
+    q, k = torch.randn(2, L, HQ, D, generator=gen).bfloat16(), torch.randn(2, L, H, D, generator=gen).bfloat16()
+    qd, kd = q.to(dev).requires_grad_(), k.to(dev).requires_grad_()
+    z = pkg.exact_chunk_log_z_tl(qd, kd, chunk_size=64, window_size=W)
+    qf, kf = q.float().requires_grad_(), k.float().requires_grad_()
+    ref = orc.exact_chunk_log_z(qf, kf, chunk_size=64, window_size=W)
+    assert_close_f32(z.detach(), ref.detach(), LSE_TOL, "log_z")
     finite = torch.isfinite(ref)
     g = torch.randn(ref.shape, generator=gen) * finite
     z.backward(g.to(dev))
