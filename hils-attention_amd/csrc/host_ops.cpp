@@ -853,8 +853,10 @@ Tensor chunk_log_z(const Tensor& q, const Tensor& k, int64_t chunk, int64_t wind
   HOST_ASSERT(k.size(0) == q.size(0) && k.size(1) == q.size(1) && k.size(3) == q.size(3),
               "q/k batch/seq/dim mismatch: q=", q.sizes(), ", k=", k.sizes());
   HOST_ASSERT(q.size(2) % k.size(2) == 0, "H_q (", q.size(2), ") must be a multiple of H_kv (", k.size(2), ") for GQA");
-  if (wants_grad({&q, &k})) return LogzFn::apply(q.contiguous(), k.contiguous(), chunk, window, scale, mask_lmk);
-  return LogzFn::forward(nullptr, q.contiguous(), k.contiguous(), chunk, window, scale, mask_lmk);
+  // (a view that begins between two multiples of 16 bytes is copied: the matrix kernels' direct loads want such keys)
+  const Tensor kc = (uintptr_t)k.const_data_ptr() % 16 ? k.clone(at::MemoryFormat::Contiguous) : k.contiguous();
+  if (wants_grad({&q, &k})) return LogzFn::apply(q.contiguous(), kc, chunk, window, scale, mask_lmk);
+  return LogzFn::forward(nullptr, q.contiguous(), kc, chunk, window, scale, mask_lmk);
 }
 
 }  // namespace

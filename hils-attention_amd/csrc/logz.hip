@@ -823,6 +823,9 @@ static bool lz_mfma_covers(int G, int D, int S, int H, int B, int W) {
   return S == 64 && W >= 0 && (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4 || G == 8 || G == 16) &&
          H <= 65535 && B <= 65535;
 }
+// ... the forward and dQ also need keys at a multiple of 16 bytes, which their direct loads to LDS want (loads to registers
+// take any address: the general kernels and dK)
+static bool lz_direct_loads(const void* k) { return (uintptr_t)k % 16 == 0; }
 // expands LZ_LAUNCH(D, G) for the covered (D, G)
 #define LZ_DISPATCH_G(DD, G_)                                                                  \
   switch (G_) {                                                                                \
@@ -850,7 +853,7 @@ extern "C" int hils_chunk_logz_fwd(const void* q, const void* k, float* log_z, i
   if (int rc = lz_check("hils_chunk_logz_fwd", B, L, HQ, H, D, S)) return rc;
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, mask_lmk, sm_scale};
   const int G = HQ / H;
-  if (lz_mfma_covers(G, D, S, H, B, window)) {
+  if (lz_mfma_covers(G, D, S, H, B, window) && lz_direct_loads(k)) {
     const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;
     HILS_REQUIRE(((long)B * H + 8) * (n_qt + 8) < (1L << 31), "hils_chunk_logz_fwd: B * H * L too large for the grid");
@@ -877,7 +880,7 @@ extern "C" int hils_chunk_logz_bwd_dq(const void* q, const void* k, const float*
   if (int rc = lz_check("hils_chunk_logz_bwd_dq", B, L, HQ, H, D, S)) return rc;
   HILS_REQUIRE(D <= LZ_THREADS, "hils_chunk_logz_bwd_dq: D (%d) must be <= %d", D, LZ_THREADS);
   LzDims dm{L, HQ, H, HQ / H, D, S, window, (L + S - 1) / S, 0, sm_scale};
-  if (lz_mfma_covers(HQ / H, D, S, H, B, window)) {
+  if (lz_mfma_covers(HQ / H, D, S, H, B, window) && lz_direct_loads(k)) {
     const int G = HQ / H;
     const int QB = 4 * LZ_ROWS / G;
     const int n_qt = (L + QB - 1) / QB;

@@ -355,7 +355,8 @@ int hils_decode_step_paged_ws(const void* q, const void* lmk_pages, const void* 
 
 /* Forward.  Replaces exact_chunk_log_z_fwd (ops/exact_chunk_log_z_tilelang.py:25-137).
  * q (B,L,HQ,D), k (B,L,H,D) bf16 -> log_z (B,L,HQ,ceil(L/S)) fp32, every element
- * written (-inf where the chunk is not fully remote). */
+ * written (-inf where the chunk is not fully remote).  k at a multiple of 16 bytes runs on the matrix kernels (here and in
+ * the backward w.r.t. q), elsewhere the general ones run.  A negative window runs on the general kernels. */
 int hils_chunk_logz_fwd(const void* q, const void* k, float* log_z, int B, int L, int HQ, int H,
                         int D, int S, int window, float sm_scale, int mask_lmk, void* stream);
 /* Backward w.r.t. q.  Replaces exact_chunk_log_z_bwd_dq (:148-262).  dq bf16 (written). */

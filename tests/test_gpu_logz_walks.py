@@ -1,5 +1,5 @@
 """Exact log Z and dQ: walks of one to nine chunks (the kernels take four steps a round and load three ahead), keys whose
-sums jump between neighbouring chunks, the landmark mask, negative windows."""
+sums jump between neighbouring chunks, the landmark mask, negative windows, keys at any address."""
 import pytest
 import torch
 
@@ -53,3 +53,35 @@ def test_negative_window(pkg, orc, dev, HQ, H, D, L, W):
     torch.where(finite, ref, torch.zeros(())).mul(g).sum().backward()
     assert_close_bf16(qd.grad, qf.grad, "dq")
     assert_close_bf16(kd.grad, kf.grad, "dk")
+
+
+@pytest.mark.parametrize("HQ,H,D", [(4, 2, 64), (8, 1, 128)])
+@pytest.mark.parametrize("at", [1, 4])
+def test_keys_at_any_address(pkg, dev, HQ, H, D, at):
+    """A contiguous view that begins 2 or 8 bytes behind a multiple of 16: the same as a copy of it, by the operator and by
+    the C entries."""
+    from hils_attention_amd.ops import _cabi
+    lib, B, L, W = _cabi.load(), 2, 470, 64
+    note(f"log Z, keys {2 * at} bytes off, heads {HQ}/{H} x {D}")
+    gen = torch.Generator(device=dev).manual_seed(at)
+    store = torch.randn(at + B * L * H * D, device=dev, generator=gen).bfloat16()
+    view = store[at:].view(B, L, H, D)
+    assert view.is_contiguous() and view.data_ptr() % 16
+    q = torch.randn(B, L, HQ, D, device=dev, generator=gen).bfloat16()
+    out = []
+    for k in (view, view.clone()):
+        a, b = q.clone().requires_grad_(), k.detach().requires_grad_()
+        z = pkg.exact_chunk_log_z_tl(a, b, chunk_size=64, window_size=W)
+        g = torch.ones_like(z).masked_fill(z == float("-inf"), 0.)
+        out.append([z.detach(), *torch.autograd.grad(z, [a, b], g)])
+    assert all(torch.equal(x, y) for x, y in zip(*out))
+    z, dq, dk = out[1]
+    cz, cq, ck = torch.empty_like(z), torch.empty_like(dq), torch.empty_like(dk)
+    p, s = _cabi.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.ones_like(z).masked_fill(z == float("-inf"), 0.)
+    assert lib.hils_chunk_logz_fwd(p(q), p(view), p(cz), B, L, HQ, H, D, 64, W, D ** -0.5, 0, s) == 0
+    assert lib.hils_chunk_logz_bwd_dq(p(q), p(view), p(z), p(g), p(cq), B, L, HQ, H, D, 64, W, D ** -0.5, s) == 0
+    assert lib.hils_chunk_logz_bwd_dk(p(q), p(view), p(z), p(g), p(ck), B, L, HQ, H, D, 64, W, D ** -0.5, s) == 0
+    assert_close_f32(cz, z, LSE_TOL, "log_z")
+    assert_close_bf16(cq, dq, "dq")
+    assert_close_bf16(ck, dk, "dk")
