@@ -263,10 +263,12 @@ chunk_weights_bwd_kernel(const bf16_t* __restrict__ scores, const void* __restri
 // gradients into a table (N x HQ) in LDS, which it adds to d_prior_b once at the end.  One global
 // atomic per element has every query of a batch element adding into the same N x HQ words: 33 M adds into
 // 16 K words took 0.51 ms at B8 L8192 h16 K32.  The table is 64-bit fixed point (2^-40): integer LDS adds
-// run at several times the rate of float ones, and a run's sum does not depend on the order of its adds.
+// run at several times the rate of float ones, and a run's sum does not depend on the order of its adds.  A wavefront with an
+// element so large that the run's sum could leave the range (tab_most: 2^23 over the most adds a word can get), or that is
+// no number, adds to memory instead (asked once a tile, 1 to 2 %; element by element 4 to 7 %).
 // What bounds it are latencies of memory: a tile's loads are asked for together and, in a run, a tile ahead, before the
 // biases that hang on the indices (d_weights went to LDS one load a latency, nine a tile: 65.7 us at B2 L8192 32/4 heads
-// K32 with the bias, 40.2 now; without the bias 25.8 -> 18.5, B8 L8192 16 heads K32 49.1 -> 34.4).
+// K32 with the bias, 41.2 now; without the bias 25.8 -> 18.5, B8 L8192 16 heads K32 49.1 -> 34.4).
 // TAB: one workgroup of 16 wavefronts a compute unit; with two the tables' own adds to memory are twice as many (48.8 us).
 template <int LPR, bool TAB>
 __global__ void __launch_bounds__(TAB ? 1024 : 256) __attribute__((amdgpu_waves_per_eu(TAB ? 4 : 7)))
@@ -275,12 +277,12 @@ chunk_weights_bwd_rows_kernel(const bf16_t* __restrict__ scores, const void* __r
                               const int32_t* __restrict__ indices, const bf16_t* __restrict__ d_weights,
                               bf16_t* __restrict__ d_scores, float* __restrict__ d_lse,
                               float* __restrict__ d_prior_b, long rows, int L, int HQ, int H, int N,
-                              int softmax1, int tiles_per_wg) {
+                              int softmax1, int tiles_per_wg, float tab_most) {
   constexpr int K = LPR * 8, RPW = 64 / LPR;
   constexpr int NWV = TAB ? 16 : 4;  // wavefronts of a workgroup
   __shared__ bf16_t stage[NWV][RPW * (K + 2)];
   extern __shared__ unsigned long long cwb_tab[];  // TAB: N x HQ, two's complement fixed point
-  constexpr float TAB_SCALE = 1099511627776.f;  // 2^40: |sums| below 2^23, steps far below an fp32 gradient's own
+  constexpr float TAB_SCALE = 1099511627776.f;  // 2^40: |sums| up to 2^23, steps far below an fp32 gradient's own
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane % LPR, rl = lane / LPR;
   const int NW = K + 1 + (softmax1 ? 1 : 0);
@@ -404,12 +406,20 @@ chunk_weights_bwd_rows_kernel(const bf16_t* __restrict__ scores, const void* __r
       out.w = pack_bf2(dl[6], dl[7]);
       *(uint4*)(d_scores + row * K + sub * 8) = out;
       if (d_prior_b && !dead) {
+        float most = 0.f;  // (a sum, which a NaN does not get lost in)
+        if (TAB) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (dl[e] != 0.f) {
-            if (TAB) atomicAdd(&cwb_tab[cidx[e] * HQ + hq], (unsigned long long)(long long)(dl[e] * TAB_SCALE));
-            else atomicAdd(d_prior_b + (b * N + cidx[e]) * (long)HQ + hq, dl[e]);
-          }
+          for (int e = 0; e < 8; ++e) most += fabsf(dl[e]);
+        }
+        if (TAB && !__any(!(most < tab_most))) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (dl[e] != 0.f) atomicAdd(&cwb_tab[cidx[e] * HQ + hq], (unsigned long long)(long long)(dl[e] * TAB_SCALE));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (dl[e] != 0.f) atomicAdd(d_prior_b + (b * N + cidx[e]) * (long)HQ + hq, dl[e]);
+        }
       }
       if (d_lse && sub == 0) d_lse[row] = dead ? nan : el * inv * (gl - dot);
     }
@@ -451,11 +461,14 @@ extern "C" int hils_chunk_weights_bwd(const void* scores, const void* lse_swa, i
       const int tiles_per_wg = (int)((tiles_b + segs - 1) / segs);
       const dim3 grid((unsigned)((tiles_b + tiles_per_wg - 1) / tiles_per_wg), (unsigned)B);
       HILS_REQUIRE(B <= 65535, "hils_chunk_weights_bwd: batch too large for the grid");
+      // a run has so many rows of a head, each with K indices, all of which may be the same
+      const long adds = (((long)tiles_per_wg * 16 * rpw + HQ - 1) / HQ) * K;
+      const float tab_most = 8388608.f / (float)adds;
 #define GL_CALL_T(LPR_)                                                                                \
   hipLaunchKernelGGL((chunk_weights_bwd_rows_kernel<LPR_, true>), grid, dim3(1024), tab_b,             \
                      (hipStream_t)stream, (const bf16_t*)scores, lse_swa, lse_bf16, prior_b, indices,  \
                      (const bf16_t*)d_weights, (bf16_t*)d_scores, d_lse, d_prior_b, rows, L, HQ, H, N, \
-                     softmax1, tiles_per_wg)
+                     softmax1, tiles_per_wg, tab_most)
       if (K == 8) GL_CALL_T(1); else if (K == 16) GL_CALL_T(2); else if (K == 32) GL_CALL_T(4); else GL_CALL_T(8);
 #undef GL_CALL_T
       HILS_CHECK_LAUNCH("hils_chunk_weights_bwd");
@@ -465,7 +478,7 @@ extern "C" int hils_chunk_weights_bwd(const void* scores, const void* lse_swa, i
   hipLaunchKernelGGL((chunk_weights_bwd_rows_kernel<LPR_, false>), dim3((unsigned)nb), dim3(256), 0,   \
                      (hipStream_t)stream, (const bf16_t*)scores, lse_swa, lse_bf16, prior_b, indices,  \
                      (const bf16_t*)d_weights, (bf16_t*)d_scores, d_lse, d_prior_b, rows, L, HQ, H, N, \
-                     softmax1, 1)
+                     softmax1, 1, 0.f)
     if (K == 8) GL_CALL(1); else if (K == 16) GL_CALL(2); else if (K == 32) GL_CALL(4); else GL_CALL(8);
 #undef GL_CALL
     HILS_CHECK_LAUNCH("hils_chunk_weights_bwd");

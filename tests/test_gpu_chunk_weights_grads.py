@@ -38,3 +38,36 @@ def test_only_what_is_asked_for(pkg, dev, want):
         assert (x.grad is not None) == w
         if w:
             assert_close_bf16(x.grad, r, name)
+
+
+@pytest.mark.parametrize("K,L,repeated", [(8, 4096, False), (32, 2500, False), (16, 700, True)])
+def test_prior_gradient_of_large_gradients(pkg, dev, K, L, repeated):
+    """Sums of a run of rows far past 2^23, small ones beside them, one index in all slots of a row, and a gradient that
+    is no number."""
+    note(f"chunk_weights, large gradients, K={K} L{L} repeated {repeated}")
+    gen = torch.Generator(device=dev).manual_seed(K)
+    B, HQ, H, N = 2, 2, 1, 64
+    sc = torch.randn(B, L, HQ, K, device=dev, generator=gen).bfloat16()
+    lse = torch.randn(B, L, HQ, device=dev, generator=gen) + 1
+    pb = torch.zeros(B, N, HQ, device=dev, requires_grad=True)
+    idx = torch.arange(K, device=dev, dtype=torch.int32).expand(B, L, H, K).contiguous()
+    if repeated:
+        idx.fill_(5)
+    g = torch.randn(B, L, HQ, K + 1, device=dev, generator=gen)
+    g[..., 0] += 2.0 ** 20
+    g[:, :, 1] *= 2.0 ** 12
+    g[1, 7, 0, 3] = float("nan")
+    g = g.bfloat16()
+    pkg.chunk_weights(sc, lse, pb, idx).backward(g)
+    x = torch.cat([sc.double(), lse.double().unsqueeze(-1)], -1)
+    y, g6 = torch.softmax(x, -1), g.double()
+    d = (y * (g6 - (y * g6).sum(-1, keepdim=True)))[..., :K]
+    size = (y * (g6.abs() + (y * g6).abs().sum(-1, keepdim=True)))[..., :K]
+    at = idx.long().view(B, L, 1, K).expand(B, L, HQ, K).permute(0, 1, 3, 2).reshape(B, L * K, HQ)
+    ref, most = (torch.zeros(B, N, HQ, dtype=torch.float64, device=dev).scatter_add_(1, at, t.permute(0, 1, 3, 2).reshape(B, L * K, HQ))
+                 for t in (d, size))
+    # an element is within some 16 roundings of its terms (exponentials, sum of K + 1, quotient), sums of n within n more
+    bad = ref.isnan()
+    assert bad[1, 5 if repeated else 3, 0] and pb.grad.isnan().equal(bad)
+    err = (pb.grad.double() - ref).abs()
+    assert bool((err <= (2 * K + 16 + L * K) * 2.0 ** -24 * most)[~bad].all())
