@@ -731,6 +731,7 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   float* const lse_s = (float*)(do_s + NB * 64 * VPITCH);       // [NB][64]
   float* const del_s = lse_s + NB * 64;                         // [NB][64]
   int* const cs_s = (int*)(del_s + NB * 64);                    // [NB][64]: window start of the row (INT_MAX: dead row)
+  int* const all_s = cs_s + NB * 64;                            // [NB]: no dead row
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, j = lane >> 4;
   int kb, hk;
@@ -817,10 +818,11 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       *(swa_u32x4*)(do_s + (buf * 64 + p / OSEG) * VPITCH + (p % OSEG) * 16) = dor[i];
     }
     if (tid < 64) {
-      const bool live = r_lse > -1e30f;  // rows with an empty window have lse = -inf
-      lse_s[buf * 64 + tid] = live && r_cs != 2147483647 ? r_lse * HILS_LOG2E : INFINITY;  // (dead: no probability but 0)
+      const bool live = r_lse > -1e30f;  // (no number, or -inf, as rows with an empty window have: no probability but 0)
+      lse_s[buf * 64 + tid] = live ? r_lse * HILS_LOG2E : 0.f;
       del_s[buf * 64 + tid] = r_del;
       cs_s[buf * 64 + tid] = live ? r_cs : 2147483647;
+      if (TT == 1) all_s[buf] = __all(live && r_cs != 2147483647);
     }
   };
   f32x4_t acck[TT][DT], accv[TT][DVT];
@@ -839,6 +841,13 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
   for (int tile = tile0, buf = 0; tile < n_tiles; ++tile) {
     fetch(tile + 1 < n_tiles ? tile + 1 : tile);
     const unsigned char *qb = q_s + buf * 64 * PITCH, *db = do_s + buf * 64 * VPITCH;
+    const int tq0 = tile * QT;
+    // do all rows of the tile see all tokens of the workgroup?  (wide heads: with two token tiles a wavefront the second
+    // copy of the loop cost more than the masks, 263 instead of 239 us at B8 L8192 16/16 of 64 window 64; tokens past the
+    // end may be seen, their sums are not written, but a dead row, whose scores may be no numbers, needs its mask)
+    const int left = tq0 + QT - dm.window;
+    const bool full = TT == 1 && !dm.mask_lmk && tq0 >= j0 + 64 * TT - 1 &&
+                      (dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left) <= j0 && __builtin_amdgcn_readfirstlane(all_s[buf]);
     float p[TT][4][4], ds[TT][4][4];  // [owned token tile][streamed row tile][row 4j+i]
     {
       f32x4_t st[TT][4], dp[TT][4];
@@ -866,12 +875,6 @@ swa_bwd_dkdv_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
             dp[tt][rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, va[tt][vs], dp[tt][rr], 0, 0, 0);
         }
       }
-      const int tq0 = tile * QT;
-      // do all rows of the tile see all tokens of the workgroup?  (wide heads: with two token tiles a wavefront the second
-      // copy of the loop cost more than the masks, 263 instead of 239 us at B8 L8192 16/16 of 64 window 64; rows and tokens past the end, whatever they see, count
-      // for nothing: such rows have no probability but 0, such tokens' sums are not written)
-      const int left = tq0 + QT - dm.window;
-      const bool full = TT == 1 && !dm.mask_lmk && tq0 >= j0 + 64 * TT - 1 && (dm.expand ? floordiv(left, dm.chunk) * dm.chunk : left) <= j0;
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         const float4 l4 = *(const float4*)&lse_s[buf * 64 + rr * 16 + 4 * j];
@@ -1115,7 +1118,7 @@ static int swa_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, con
   const int n_qt = (dm.Lq + QB - 1) / QB;
   hipLaunchKernelGGL((swa_bwd_dq_mfma<D, DV, G>), swa_xcd_grid(n_qt, dm.H, B),
                      dim3(256), 0, st, q, k, v, o, lse, d_o, d_lse, dq, delta, dm, n_qt, B);
-  const size_t smem = (size_t)swa_dkdv_buffers(D, DV) * 64 * ((D * 2 + 32) + (DV * 2 + 32) + 3 * sizeof(float));
+  const size_t smem = (size_t)swa_dkdv_buffers(D, DV) * (64 * ((D * 2 + 32) + (DV * 2 + 32) + 3 * sizeof(float)) + sizeof(int));
   auto kern = swa_bwd_dkdv_mfma<D, DV, G>;
   static HilsLdsReserve reserved;  // per instantiation
   if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_swa_bwd")) return rc;

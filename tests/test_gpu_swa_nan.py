@@ -1,4 +1,5 @@
-"""A query or key that is not a number shows in the local branch's output, whichever kernel the shape runs on."""
+"""A query or key that is not a number shows in the local branch's output, whichever kernel the shape runs on; a query's
+reaches its own gradient and those of the keys, not those of the values, whichever tile it lies in."""
 import pytest
 import torch
 
@@ -56,3 +57,30 @@ def test_nan_shows_in_a_split_window(pkg, dev, B, L, HQ, H, D, Dv, t):
     sees[t:last + 1] = True
     assert o[0, :, :G].isnan().any(-1).any(-1)[sees].all() and not o[0, :, G:].isnan().any()
     assert not o[0, ~sees, :G].isnan().any()
+
+
+@pytest.mark.parametrize("HQ,H,D,Dv", [(8, 2, 64, 64), (8, 2, 128, 128), (4, 4, 128, 128), (16, 1, 64, 128), (4, 2, 128, 64)])
+@pytest.mark.parametrize("W,mask_lmk", [(512, False), (300, True), (64, False)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_gradients_of_a_query_that_is_no_number(pkg, dev, HQ, H, D, Dv, W, mask_lmk, bad):
+    note(f"local branch backward, a query with {bad}, heads {HQ}/{H} x {D}/{Dv} window {W} mask {mask_lmk}")
+    gen = torch.Generator(device=dev).manual_seed(W + D)
+    B, L, t = 2, 901, 700
+    r = lambda *s: torch.randn(*s, generator=gen, device=dev).bfloat16()
+    q, k, v, d_o = r(B, L, HQ, D), r(B, L, H, D), r(B, L, H, Dv), r(B, L, HQ, Dv)
+
+    def grads(q, d_o):
+        ins = [x.clone().requires_grad_() for x in (q, k, v)]
+        o, _ = pkg.flex_attn_tl(*ins, W, 64, mask_lmk=mask_lmk)
+        return torch.autograd.grad(o, ins, d_o)
+
+    without = d_o.clone()
+    without[1, t, 1] = 0  # nothing but 0 comes from this row
+    q0, k0, v0 = grads(q, without)
+    q[1, t, 1, 5] = bad
+    q1, k1, v1 = grads(q, d_o)
+    assert torch.equal(v1, v0)
+    hit = torch.zeros(B, L, HQ, dtype=torch.bool, device=dev)
+    hit[1, t, 1] = True
+    assert q1.isnan().any(-1).equal(hit) and torch.equal(q1[~hit], q0[~hit])
+    assert torch.equal(k1[0], k0[0]) and k1[1, t, 1 // (HQ // H)].isnan().any()
