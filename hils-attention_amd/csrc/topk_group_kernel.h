@@ -126,10 +126,14 @@ __device__ __forceinline__ uint32_t tg_kth_largest(const uint32_t (&k)[NE], uint
 // HALF (G = 5..8): the wavefronts come in pairs on the same four queries, wavefront 2p takes the heads
 // 0..3 and 2p+1 the heads 4..G-1; with PERQ a workgroup is eight wavefronts (head w's keys in
 // wavefront w) on 16 queries, otherwise one pair.
+// Wavefronts per SIMD that the registers are held to.  (Eight-wavefront workgroups are two per SIMD each: three per SIMD
+// leave room for one only, six for three.)
+constexpr int tg_waves_per_eu(int NB, bool PERQ, bool HALF) {
+  return NB <= 8 ? (PERQ && HALF ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1)));
+}
 template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF>
 __global__ void __launch_bounds__(64 * (PERQ ? (HALF ? 8 : 4) : TG_WAVES))
-    // (eight-wavefront workgroups are two per SIMD each: three per SIMD leave room for one only, six for three)
-    __attribute__((amdgpu_waves_per_eu(NB <= 8 ? (PERQ && HALF ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1))))))
+    __attribute__((amdgpu_waves_per_eu(tg_waves_per_eu(NB, PERQ, HALF))))
 topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lmk_packed,
                       const float* __restrict__ lse_swa, const float* __restrict__ bias,
                       int32_t* __restrict__ indices,
@@ -160,8 +164,9 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
                             : (XCH_F + KX_F > 0 ? XCH_F + KX_F : 1);
   __shared__ __align__(16) float xbuf[XB_F];
   // REC: candidates as records.  With 24 blocks and fewer walking all scores again is the cheaper way (24 blocks: 109 us
-  // against 124 with records, whose LDS and registers cost wavefronts; 32: 131 with, 156 without).
-  constexpr bool REC = NB >= TG_REC_NB && GMAX == 4 && !OVER;
+  // against 124 with records, whose LDS and registers cost wavefronts; 32: 131 with, 156 without).  Not where the halves have
+  // a bias, whose copies and the records together leave room for one workgroup of two (64 blocks) or three of four.
+  constexpr bool REC = NB >= TG_REC_NB && GMAX == 4 && !OVER && !(HALF && BIAS);
   constexpr int REC_N = NB > 32 ? 2 * TG_CAND : 3 * TG_CAND / 2;  // records of a lane row: one query in forty has more than 128
   constexpr int NWORD = NB > 32 ? 32 : 16;  // words of the winner map
   __shared__ __align__(16) uint4 rec_w[REC ? TGW : 1][REC ? 4 : 1][REC ? REC_N : 1];
@@ -175,6 +180,10 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   // (One copy per workgroup, filled by its wavefronts together before they part; with HALF one per half of
   // the heads.)
   __shared__ __align__(16) float bias_w[BIAS ? (HALF ? (PERQ ? 2 : TGW) : 1) : 1][BIAS ? NB * 16 : 1][4];
+  constexpr size_t LDS_B = sizeof(xbuf) + (REC ? sizeof(rec_w) + sizeof(words_w) + sizeof(wbase_w) : OVER ? 0 : sizeof(cand_w)) +
+                           (OVER ? 0 : sizeof(stage_i_w) + sizeof(stage_s_w)) + (BIAS ? sizeof(bias_w) : 0);
+  static_assert(LDS_B * (4 * tg_waves_per_eu(NB, PERQ, HALF) / TGW) <= 160 * 1024,
+                "the LDS holds as many workgroups as the registers");
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = HALF ? (wave & 1) : 0;   // this wavefront's heads are 4 * half ..

@@ -63,6 +63,18 @@ def test_equal_scores_past_512_chunks(pkg, dev):
 def test_selection_by_candidate_count(pkg, dev, G, perq, lim, topk, kind):
     """Exact scores whose candidates (those above the weakest lane's second largest score) are few, more than 128, or more
     than the kernel keeps, and ties at the threshold: the best scores win, of equal ones the lowest chunks."""
+    _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, False)
+
+
+@pytest.mark.parametrize("G,perq", [(4, False), (4, True), (8, False), (8, True)])
+@pytest.mark.parametrize("lim,topk", [(40, 32), (512, 32), (1024, 32)])
+@pytest.mark.parametrize("kind", ["shuffled", "column", "far column", "ties"])
+def test_selection_by_candidate_count_with_a_bias(pkg, dev, G, perq, lim, topk, kind):
+    """The same scores, their last three bits in the prior bias: the scores that come back carry none of it."""
+    _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, True)
+
+
+def _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased):
     L, S, D = 640, 64, 64
     N = min(1024, lim + 4)
     gen = torch.Generator().manual_seed(lim)
@@ -79,13 +91,17 @@ def test_selection_by_candidate_count(pkg, dev, G, perq, lim, topk, kind):
     lmk = torch.zeros(1, N, G if perq else 1, D)
     lmk[..., 0], lmk[..., 1] = (v // 8 * 8).view(1, N, 1), (v % 8).view(1, N, 1)  # (each exact in bf16, so is their sum)
     q = torch.zeros(1, L, G, D)
-    q[..., :2] = 1
+    q[..., :1 if biased else 2] = 1
+    bias = (v % 8 / 8).view(1, N, 1).expand(1, N, G).contiguous().to(dev) if biased else None  # (logits are sums / 8)
     off = lim * S - L  # the last query's window of one token begins in chunk lim
-    idx, _, _ = pkg.topk_chunk_weights(q.bfloat16().to(dev), lmk.bfloat16().to(dev), torch.zeros(1, L, G, device=dev), topk, S, 1,
-                                       q_offset=off, num_kv_heads=1)
+    idx, scores, _ = pkg.topk_chunk_weights(q.bfloat16().to(dev), lmk.bfloat16().to(dev), torch.zeros(1, L, G, device=dev), topk, S, 1,
+                                            q_offset=off, num_kv_heads=1, prior_b=bias)
     seen = ((torch.arange(L) + off) // S).clamp(0, N)
     order = (v * 2048 - torch.arange(N)).expand(L, N).masked_fill(torch.arange(N) >= seen.view(L, 1), -(1 << 30))
     best = order.topk(topk, -1)
     want = torch.where(best.values > -(1 << 30), best.indices, torch.full_like(best.indices, 1 << 20)).sort(-1).values
     want = torch.where(want == 1 << 20, torch.full_like(want, -1), want)
     assert torch.equal(idx[0, :, 0].cpu().long(), want)
+    raw = (v // 8 * 8 if biased else v).to(torch.float32)[want.clamp(min=0)] / 8
+    raw = raw.masked_fill(want < 0, float("-inf")).bfloat16()
+    assert torch.equal(scores[0].cpu(), raw.unsqueeze(1).expand(L, G, topk))
