@@ -149,7 +149,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   constexpr int QGROUPS = HALF ? TGW / 2 : TGW;              // ... and how many have queries of their own
   static_assert(!PERQ || GMAX == 4, "per-query-head keys: four heads, four wavefronts");
   static_assert(!HALF || (GMAX == 4 && TG_WAVES == 2), "halves: four heads each, a pair per workgroup");
-  constexpr bool ALONE = NB > 32;  // one wavefront per SIMD
+  constexpr bool ALONE = tg_waves_per_eu(NB, PERQ, HALF) == 1 && TGW <= 4;  // one wavefront per SIMD (eight-wavefront workgroups: two)
   constexpr int PB = NB >= 32 ? 2 : 1;  // blocks per load group (two groups are live: 16 registers per block and group)
   // LDS that several wavefronts share.  PERQ: accumulators of a load group on their way between the
   // wavefronts, [buffer][block][from wavefront = head][register][lane]; two buffers take turns, so that
@@ -171,7 +171,12 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   constexpr int NWORD = NB > 32 ? 32 : 16;  // words of the winner map
   __shared__ __align__(16) uint4 rec_w[REC ? TGW : 1][REC ? 4 : 1][REC ? REC_N : 1];
   __shared__ uint32_t cand_w[OVER || REC ? 1 : TGW][4][TG_CAND];  // (without records) compacted candidate keys, per lane row
-  __shared__ uint32_t words_w[REC ? TGW : 1][REC ? 4 : 1][REC ? NWORD : 1], wbase_w[REC ? TGW : 1][REC ? 4 : 1][REC ? NWORD : 1];
+  // MAP: the eight-wavefront 64-block kernel, whose 64 logits a lane of four heads lie in scratch memory for the most part, keeps a
+  // bit per block of the winners and takes their order from a map of the winning chunks, like the records.  With votes, which
+  // need all scores until the end, it read them from scratch once more, and side by side its log-sum-exps (ALONE) spilled
+  // more (B1 L4096 32/4 heads of 64, a key per head, 1000 chunks, top-32: 524 -> 348 us, with a bias 562 -> 362).
+  constexpr bool MAP = OVER && NB > 32, WORDS = REC || MAP;
+  __shared__ uint32_t words_w[WORDS ? TGW : 1][WORDS ? 4 : 1][WORDS ? NWORD : 1], wbase_w[WORDS ? TGW : 1][WORDS ? 4 : 1][WORDS ? NWORD : 1];
   __shared__ __align__(16) int stage_i_w[OVER ? 1 : TGW][NQ * 32];               // winners' chunk indices, [query][slot]
   __shared__ __align__(16) bf16_t stage_s_w[OVER ? 1 : TGW][NQ * GMAX * 32];  // their raw scores, [query][slot][head]
   // the bias of this (batch, KV head): [chunk][head, padded to 4] fp32, a copy per wavefront (they never
@@ -180,8 +185,8 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   // (One copy per workgroup, filled by its wavefronts together before they part; with HALF one per half of
   // the heads.)
   __shared__ __align__(16) float bias_w[BIAS ? (HALF ? (PERQ ? 2 : TGW) : 1) : 1][BIAS ? NB * 16 : 1][4];
-  constexpr size_t LDS_B = sizeof(xbuf) + (REC ? sizeof(rec_w) + sizeof(words_w) + sizeof(wbase_w) : OVER ? 0 : sizeof(cand_w)) +
-                           (OVER ? 0 : sizeof(stage_i_w) + sizeof(stage_s_w)) + (BIAS ? sizeof(bias_w) : 0);
+  constexpr size_t LDS_B = sizeof(xbuf) + (REC ? sizeof(rec_w) : OVER ? 0 : sizeof(cand_w)) +
+                           (WORDS ? sizeof(words_w) + sizeof(wbase_w) : 0) + (OVER ? 0 : sizeof(stage_i_w) + sizeof(stage_s_w)) + (BIAS ? sizeof(bias_w) : 0);
   static_assert(LDS_B * (4 * tg_waves_per_eu(NB, PERQ, HALF) / TGW) <= 160 * 1024,
                 "the LDS holds as many workgroups as the registers");
 
@@ -421,9 +426,12 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   // (ALONE: the four rows side by side.  One after the other every sum waited for its exponential, 9 instead of 5
   // thousand cycles; with more wavefronts another one's instructions run meanwhile, and the registers are short.)
   constexpr int RS = ALONE ? 4 : 1;
+  // (MAP, heads of 64, a bias: written as one loop over the rows the kernel spills 206 registers instead of 251, 362 us
+  // against 426 in the call above; heads of 128 are faster this way)
+  constexpr bool SERIAL = MAP && BIAS && KS == 2;
   float lse_tot[4], m_row[4], l_row[4];
 #pragma unroll
-  for (int r0 = 0; r0 < 4; r0 += RS) {
+  for (int r0 = 0; r0 < (SERIAL ? 0 : 4); r0 += RS) {
 #pragma unroll
     for (int i = r0; i < r0 + RS; ++i) {
       float m = HILS_NEG_INF;
@@ -448,6 +456,16 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
+    if constexpr (SERIAL) {
+      float m = HILS_NEG_INF;
+#pragma unroll
+      for (int nt = 0; nt < NB; ++nt) m = fmaxf(m, x[nt][i]);
+      m = tg_row_max_f(m);
+      m_row[i] = (m > HILS_NEG_INF) ? m * HILS_LOG2E : 0.f;
+      l_row[i] = 0.f;
+#pragma unroll
+      for (int nt = 0; nt < NB; ++nt) l_row[i] += __builtin_amdgcn_exp2f(fmaf(x[nt][i], HILS_LOG2E, -m_row[i]));
+    }
     const float m2 = m_row[i], l = row_sum<16>(l_row[i]);
     const float hils2 = (l > 0.f) ? m2 + __builtin_amdgcn_logf(l) : HILS_NEG_INF;  // log2 domain
     const float swa2 = swa[i] * HILS_LOG2E;
@@ -731,50 +749,103 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
         }
       }
     }
-    if (__any(cut)) {  // the ties that lose leave the scores
+    if constexpr (MAP) {
+      // winners of this lane as a bit mask over its blocks
+      unsigned long long mask = 0u;
+      if (__any(cut)) {
 #pragma unroll
-      for (int nt = 0; nt < NB; ++nt)
-        if ((key[nt] == Tf) & (nt * 16 + col > cutoff)) key[nt] = HILS_NEG_INF;
-    }
-    // Everything from the threshold up wins (a query that keeps all its valid scores has Tf = -inf: the lowest finite
-    // float stands in for it).  A winner's slot is the number of winners with a lower chunk index: those of the blocks
-    // before (`before`, of this lane's row) and those of lower columns, both counted in the bits of the block's vote, so
-    // that nothing waits for LDS: with the winners' map and its prefix counts there, every block with a winner read them
-    // back and waited, 16 of the 36 thousand cycles that the selection of 1024 chunks took.
-    const float Tlow = fmaxf(Tf, -3.402823466e38f);
-    int before = 0;
+        for (int nt = NB - 1; nt >= 0; --nt) {
+          const bool win = (key[nt] > Tf) | ((key[nt] == Tf) & (nt * 16 + col <= cutoff));
+          mask = (mask << 1) | (win ? 1u : 0u);
+        }
+      } else {
+        const float Tlow = fmaxf(Tf, -3.402823466e38f);  // (as below)
 #pragma unroll
-    for (int n0 = 0; n0 < NB; n0 += WB) {
-      float bv[WB][4];
-      if constexpr (BIAS) {
-#pragma unroll
-        for (int n2 = 0; n2 < WB; ++n2) bias_of((n0 + n2) * 16 + col, bv[n2]);
+        for (int nt = NB - 1; nt >= 0; --nt) mask = (mask << 1) | ((key[nt] >= Tlow) ? 1u : 0u);
       }
+      // map of the winning chunks (chunk c = bit c): word w holds blocks 2w and 2w+1
+      uint32_t (*words)[NWORD] = words_w[wave], (*wbase)[NWORD] = wbase_w[wave];
+      words[j][col] = 0u;
+      words[j][16 + col] = 0u;
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int n2 = 0; n2 < WB; ++n2) {
-        const int nt = n0 + n2;
-        const bool win = key[nt] >= Tlow;
-        const unsigned long long votes = __ballot(win);
-        const uint32_t v_lo = (uint32_t)votes, v_hi = (uint32_t)(votes >> 32);
-        const int slot = __popc(v_hi & low_hi) + (__popc(v_lo & low_lo) + before);
-        before = __popc(v_hi & row_hi) + (__popc(v_lo & row_lo) + before);
-        if (win & (slot < topk)) {  // its chunk and raw scores to the stage
-          stage_i[qi * 32 + slot] = nt * 16 + col;
-          // the heads of the winner in one store (heads past G are never read back)
-          bf16_t* dst = &stage_s[(qi * 32 + slot) * GMAX];
-          float raw[4];
+      for (int w = 0; w < NB / 2; ++w) {
+        const uint32_t bits = ((uint32_t)((mask >> (2 * w)) & 1u) << col) | ((uint32_t)((mask >> (2 * w + 1)) & 1u) << (16 + col));
+        if (bits) atomicOr(&words[j][w], bits);
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int p0 = __popc(words[j][2 * col]), p1 = __popc(words[j][2 * col + 1]);
+      const int base = tg_row_excl_scan(p0 + p1);
+      wbase[j][2 * col] = (uint32_t)base;
+      wbase[j][2 * col + 1] = (uint32_t)(base + p0);
+      __builtin_amdgcn_wave_barrier();
+      // every winner: its slot = winners with a lower chunk index; index and raw scores to the stage
 #pragma unroll
-          for (int i = 0; i < 4; ++i) raw[i] = x[nt][i];
-          if constexpr (BIAS) {  // the returned scores carry no bias
+      for (int nt = 0; nt < NB; ++nt) {
+        if ((mask >> nt) & 1u) {
+          const int c = nt * 16 + col, w = c >> 5;
+          const int slot = (int)wbase[j][w] + __popc(words[j][w] & ((1u << (c & 31)) - 1u));
+          if (slot < topk) {
+            stage_i[qi * 32 + slot] = c;
+            float raw[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) raw[i] = __fsub_rn(raw[i], bv[n2][i]);
+            for (int i = 0; i < 4; ++i) raw[i] = x[nt][i];
+            if constexpr (BIAS) {  // the returned scores carry no bias
+              float bv[4];
+              bias_of(c, bv);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) raw[i] = __fsub_rn(raw[i], bv[i]);
+            }
+            *(uint2*)&stage_s[(qi * 32 + slot) * GMAX] = make_uint2(pack_bf2(raw[0], raw[1]), pack_bf2(raw[2], raw[3]));
           }
-          if constexpr (GMAX == 4) {
-            *(uint2*)dst = make_uint2(pack_bf2(raw[0], raw[1]), pack_bf2(raw[2], raw[3]));
-          } else if constexpr (GMAX == 2) {
-            *(uint32_t*)dst = pack_bf2(raw[u * 2], raw[u * 2 + 1]);
-          } else {
-            *dst = f2bf(raw[u]);
+        }
+      }
+    } else {
+      if (__any(cut)) {  // the ties that lose leave the scores
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt)
+          if ((key[nt] == Tf) & (nt * 16 + col > cutoff)) key[nt] = HILS_NEG_INF;
+      }
+      // Everything from the threshold up wins (a query that keeps all its valid scores has Tf = -inf: the lowest finite
+      // float stands in for it).  A winner's slot is the number of winners with a lower chunk index: those of the blocks
+      // before (`before`, of this lane's row) and those of lower columns, both counted in the bits of the block's vote, so
+      // that nothing waits for LDS: with the winners' map and its prefix counts there, every block with a winner read them
+      // back and waited, 16 of the 36 thousand cycles that the selection of 1024 chunks took.
+      const float Tlow = fmaxf(Tf, -3.402823466e38f);
+      int before = 0;
+#pragma unroll
+      for (int n0 = 0; n0 < NB; n0 += WB) {
+        float bv[WB][4];
+        if constexpr (BIAS) {
+#pragma unroll
+          for (int n2 = 0; n2 < WB; ++n2) bias_of((n0 + n2) * 16 + col, bv[n2]);
+        }
+#pragma unroll
+        for (int n2 = 0; n2 < WB; ++n2) {
+          const int nt = n0 + n2;
+          const bool win = key[nt] >= Tlow;
+          const unsigned long long votes = __ballot(win);
+          const uint32_t v_lo = (uint32_t)votes, v_hi = (uint32_t)(votes >> 32);
+          const int slot = __popc(v_hi & low_hi) + (__popc(v_lo & low_lo) + before);
+          before = __popc(v_hi & row_hi) + (__popc(v_lo & row_lo) + before);
+          if (win & (slot < topk)) {  // its chunk and raw scores to the stage
+            stage_i[qi * 32 + slot] = nt * 16 + col;
+            // the heads of the winner in one store (heads past G are never read back)
+            bf16_t* dst = &stage_s[(qi * 32 + slot) * GMAX];
+            float raw[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[i] = x[nt][i];
+            if constexpr (BIAS) {  // the returned scores carry no bias
+#pragma unroll
+              for (int i = 0; i < 4; ++i) raw[i] = __fsub_rn(raw[i], bv[n2][i]);
+            }
+            if constexpr (GMAX == 4) {
+              *(uint2*)dst = make_uint2(pack_bf2(raw[0], raw[1]), pack_bf2(raw[2], raw[3]));
+            } else if constexpr (GMAX == 2) {
+              *(uint32_t*)dst = pack_bf2(raw[u * 2], raw[u * 2 + 1]);
+            } else {
+              *dst = f2bf(raw[u]);
+            }
           }
         }
       }
