@@ -127,13 +127,14 @@ __device__ __forceinline__ uint32_t tg_kth_largest(const uint32_t (&k)[NE], uint
 // 0..3 and 2p+1 the heads 4..G-1; with PERQ a workgroup is eight wavefronts (head w's keys in
 // wavefront w) on 16 queries, otherwise one pair.
 // Wavefronts per SIMD that the registers are held to.  (Eight-wavefront workgroups are two per SIMD each: three per SIMD
-// leave room for one only, six for three.)
-constexpr int tg_waves_per_eu(int NB, bool PERQ, bool HALF) {
-  return NB <= 8 ? (PERQ && HALF ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1)));
+// leave room for one only, six for three.  Six spill 16 registers with heads of 128: B1 L4096 32/4 heads of 128, 100 chunks, 48.8
+// us against 44.6; of 64 they spill none, L4096 64/8 66 -> 58 us.)
+constexpr int tg_waves_per_eu(int KS, int NB, bool PERQ, bool HALF) {
+  return NB <= 8 ? (PERQ && HALF && KS == 2 ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1)));
 }
 template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF>
 __global__ void __launch_bounds__(64 * (PERQ ? (HALF ? 8 : 4) : TG_WAVES))
-    __attribute__((amdgpu_waves_per_eu(tg_waves_per_eu(NB, PERQ, HALF))))
+    __attribute__((amdgpu_waves_per_eu(tg_waves_per_eu(KS, NB, PERQ, HALF))))
 topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lmk_packed,
                       const float* __restrict__ lse_swa, const float* __restrict__ bias,
                       int32_t* __restrict__ indices,
@@ -149,7 +150,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   constexpr int QGROUPS = HALF ? TGW / 2 : TGW;              // ... and how many have queries of their own
   static_assert(!PERQ || GMAX == 4, "per-query-head keys: four heads, four wavefronts");
   static_assert(!HALF || (GMAX == 4 && TG_WAVES == 2), "halves: four heads each, a pair per workgroup");
-  constexpr bool ALONE = tg_waves_per_eu(NB, PERQ, HALF) == 1 && TGW <= 4;  // one wavefront per SIMD (eight-wavefront workgroups: two)
+  constexpr bool ALONE = tg_waves_per_eu(KS, NB, PERQ, HALF) == 1 && TGW <= 4;  // one wavefront per SIMD (eight-wavefront workgroups: two)
   constexpr int PB = NB >= 32 ? 2 : 1;  // blocks per load group (two groups are live: 16 registers per block and group)
   // LDS that several wavefronts share.  PERQ: accumulators of a load group on their way between the
   // wavefronts, [buffer][block][from wavefront = head][register][lane]; two buffers take turns, so that
@@ -187,7 +188,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   __shared__ __align__(16) float bias_w[BIAS ? (HALF ? (PERQ ? 2 : TGW) : 1) : 1][BIAS ? NB * 16 : 1][4];
   constexpr size_t LDS_B = sizeof(xbuf) + (REC ? sizeof(rec_w) : OVER ? 0 : sizeof(cand_w)) +
                            (WORDS ? sizeof(words_w) + sizeof(wbase_w) : 0) + (OVER ? 0 : sizeof(stage_i_w) + sizeof(stage_s_w)) + (BIAS ? sizeof(bias_w) : 0);
-  static_assert(LDS_B * (4 * tg_waves_per_eu(NB, PERQ, HALF) / TGW) <= 160 * 1024,
+  static_assert(LDS_B * (4 * tg_waves_per_eu(KS, NB, PERQ, HALF) / TGW) <= 160 * 1024,
                 "the LDS holds as many workgroups as the registers");
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
