@@ -641,28 +641,32 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
             p[tt][rr][i] = __builtin_amdgcn_exp2f(st[tt][rr][i] * sc2 - o[i]) * cf[i];
       }
     }
-    lzm_grad_product_rows<D, 2, PITCH>(qb, p, acc, col, j);
+    lzm_grad_product_rows<D, 2, PITCH, true>(qb, p, acc, col, j);
     stash(buf ^ 1);
     __syncthreads();
   }
+  // (a lane holds a feature of four tokens.  With four features of a token, and 16-byte stores, the whole kernel was 1 to 7 %
+  // slower at 54 of 60 lengths and head shapes: L2048 32/8 heads of 128 67.9 us against 64.0, L8192 582 against 573)
+  if (n_seg > 1) {
+    float* out = part + (((long)unit * n_pair + pair) * sg.max_seg + seg_i) * (128 * D);
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {  // (a lane holds four neighbouring features of its token)
-    const int t = tt * 16 + col, tok = tok0 + t;
-    if (n_seg > 1) {
-      float* out = part + (((long)unit * n_pair + pair) * sg.max_seg + seg_i) * (128 * D) + (wave * 32 + t) * D + 4 * j;
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) *(f32x4_t*)(out + dt * 16) = acc[tt][dt];
-    } else if (tok < dm.L) {
-      bf16_t* out = dk + ((b * dm.L + tok) * (long)dm.H + hk) * D + 4 * j;
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        uint2 x;
-        x.x = pack_bf2(acc[tt][dt][0], acc[tt][dt][1]);
-        x.y = pack_bf2(acc[tt][dt][2], acc[tt][dt][3]);
-        *(uint2*)(out + dt * 16) = x;
-      }
-    }
+        for (int dt = 0; dt < DT; ++dt) out[(wave * 32 + tt * 16 + 4 * j + i) * D + dt * 16 + col] = acc[tt][dt][i];
+    return;
   }
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tok = tok0 + tt * 16 + 4 * j + i;
+      if (tok >= dm.L) continue;
+      bf16_t* out = dk + ((b * dm.L + tok) * (long)dm.H + hk) * D + col;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) out[dt * 16] = f2bf(acc[tt][dt][i]);
+    }
 }
 
 // the segments of the cut walks, in order; four features per thread

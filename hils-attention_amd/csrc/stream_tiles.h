@@ -7,8 +7,9 @@
 // the features by the transposing LDS load: a 16-lane group addresses a
 // 4 x 16 block, lane l row l/4 and columns 4(l%4).., and receives column l of it; with rows 4j.. of two neighbouring
 // 16-row tiles that is the order in which the score accumulators hold p (lane: owned row = lane & 15, streamed rows
-// 4*(lane>>4)+i of tile tt).  A lane's accumulators are features 16 dt + 4*(lane>>4)+i of its owned row.
-template <int D, int NT, int PITCH>
+// 4*(lane>>4)+i of tile tt).  A lane's accumulators are features 16 dt + 4*(lane>>4)+i of its owned row or, with COLS, the
+// product taken the other way round, feature 16 dt + (lane & 15) of the owned rows 4*(lane>>4)+i.
+template <int D, int NT, int PITCH, bool COLS = false>
 __device__ __forceinline__ void lzm_grad_product_rows(const unsigned char* rows, const float (&p)[NT][4][4],
                                                       f32x4_t (&acc)[NT][D / 16], int col, int j) {
   typedef short lz_s4 __attribute__((ext_vector_type(4)));
@@ -34,7 +35,8 @@ __device__ __forceinline__ void lzm_grad_product_rows(const unsigned char* rows,
       const lz_s4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lz_s4*)(p0 + 16 * PITCH));
       const bf16x8_t b = __builtin_bit_cast(bf16x8_t, (lz_s8)__builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-      for (int rt = 0; rt < NT; ++rt) acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[rt], acc[rt][dt], 0, 0, 0);
+      for (int rt = 0; rt < NT; ++rt)
+        acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(COLS ? a[rt] : b, COLS ? b : a[rt], acc[rt][dt], 0, 0, 0);
     }
   }
 }
