@@ -94,7 +94,19 @@ int hils_topk_group_launch(const void* q, const void* lmk_packed, const float* l
       tg_dispatch(GM, D, bias != nullptr, per_qhead != 0, halves, [&](auto gm, auto ks, auto bi, auto pq, auto hf) {
 #define TG_NBS(NB_, EX_) tg_call<gm.value, ks.value, NB_, EX_, bi.value, pq.value, hf.value>(grid, st, a)
         if (exp) TG_NBS(32, true);
-        else if (NB == 32) TG_NBS(32, false);
+        else if (NB == 32) {
+          // Records shorten a wavefront's serial chain, but with a bias and wide heads they spill: past one round of
+          // wavefronts (two per SIMD, four workgroups a compute unit), where the instructions count, votes are ahead
+          // (records / votes, 32/8 heads of 128, 512 chunks, top-8: 1024 queries 28.5 / 31.8 us, 1536 48.5 / 46.6,
+          // 4096 94 / 91, 8192 168 / 159)
+          if constexpr (gm.value == 4 && ks.value == 4 && bi.value && !pq.value && !hf.value) {
+            if ((long)grid.x * grid.y * grid.z > 4L * hils_device_cus()) {
+              tg_call<4, 4, 32, false, true, false, false, false>(grid, st, a);
+              return;
+            }
+          }
+          TG_NBS(32, false);
+        }
         else if (NB == 24) TG_NBS(24, false);
         else if constexpr (gm.value > 1) {  // (one head: above)
           if (NB == 16) TG_NBS(16, false);

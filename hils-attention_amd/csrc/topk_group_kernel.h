@@ -132,7 +132,7 @@ __device__ __forceinline__ uint32_t tg_kth_largest(const uint32_t (&k)[NE], uint
 constexpr int tg_waves_per_eu(int KS, int NB, bool PERQ, bool HALF) {
   return NB <= 8 ? (PERQ && HALF && KS == 2 ? 6 : 5) : (NB <= 16 ? 4 : (NB <= 24 && !(PERQ && HALF) ? 3 : (NB <= 32 ? 2 : 1)));
 }
-template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF>
+template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF, bool RECORDS>
 __global__ void __launch_bounds__(64 * (PERQ ? (HALF ? 8 : 4) : TG_WAVES))
     __attribute__((amdgpu_waves_per_eu(tg_waves_per_eu(KS, NB, PERQ, HALF))))
 topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lmk_packed,
@@ -164,10 +164,10 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
                                             : (KX_F > TGW * SEL_B / 4 ? KX_F : TGW * SEL_B / 4))
                             : (XCH_F + KX_F > 0 ? XCH_F + KX_F : 1);
   __shared__ __align__(16) float xbuf[XB_F];
-  // REC: candidates as records.  With 24 blocks and fewer walking all scores again is the cheaper way (24 blocks: 109 us
+  // REC (RECORDS false: the host wants none): candidates as records.  With 24 blocks and fewer walking all scores again is the cheaper way (24 blocks: 109 us
   // against 124 with records, whose LDS and registers cost wavefronts; 32: 131 with, 156 without).  Not where the halves have
   // a bias, whose copies and the records together leave room for one workgroup of two (64 blocks) or three of four.
-  constexpr bool REC = NB >= TG_REC_NB && GMAX == 4 && !OVER && !(HALF && BIAS);
+  constexpr bool REC = RECORDS && NB >= TG_REC_NB && GMAX == 4 && !OVER && !(HALF && BIAS);
   constexpr int REC_N = NB > 32 ? 2 * TG_CAND : 3 * TG_CAND / 2;  // records of a lane row: one query in forty has more than 128
   constexpr int NWORD = NB > 32 ? 32 : 16;  // words of the winner map
   __shared__ __align__(16) uint4 rec_w[REC ? TGW : 1][REC ? 4 : 1][REC ? REC_N : 1];
@@ -499,7 +499,7 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
   const uint32_t row_bits = 0xffffu << (16 * (j & 1)), low_bits = ((1u << col) - 1u) << (16 * (j & 1));
   const uint32_t row_lo = j < 2 ? row_bits : 0u, row_hi = j < 2 ? 0u : row_bits;
   const uint32_t low_lo = j < 2 ? low_bits : 0u, low_hi = j < 2 ? 0u : low_bits;
-  constexpr int WB = BIAS ? (OVER ? 1 : 4) : 1;  // blocks whose biases are read together
+  constexpr int WB = BIAS ? (OVER || (REC && KS == 4) ? 1 : 4) : 1;  // blocks whose biases are read together (wide heads' records: four spill 16 registers, one 7)
 #pragma unroll
   for (int u = 0; u < QPL; ++u) {
     const int qi = j * QPL + u;  // query of the wavefront this lane row works on
@@ -885,10 +885,10 @@ struct TgArgs {
   int t_base, t_end, lse_bf16;
 };
 
-template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF>
+template <int GMAX, int KS, int NB, bool EXPORT, bool BIAS, bool PERQ, bool HALF, bool RECORDS = true>
 static void tg_call(dim3 grid, hipStream_t st, const TgArgs& a) {
   const int bs_shift = (a.block_size > 0 && (a.block_size & (a.block_size - 1)) == 0) ? __builtin_ctz(a.block_size) : -1;
-  hipLaunchKernelGGL((topk_fwd_group_kernel<GMAX, KS, NB, EXPORT, BIAS, PERQ, HALF>), grid,
+  hipLaunchKernelGGL((topk_fwd_group_kernel<GMAX, KS, NB, EXPORT, BIAS, PERQ, HALF, RECORDS>), grid,
                      dim3(64 * (PERQ ? (HALF ? 8 : 4) : TG_WAVES)), 0, st, a.q, a.pk, a.lse_swa, a.bias, a.indices, a.scores,
                      a.lse_total, a.sel_logits, a.L, a.N, a.h_kv, a.G, a.topk, a.block_size, a.window_size, a.causal,
                      a.q_offset, a.sm_scale, a.t_base, a.t_end, bs_shift, a.lse_bf16);

@@ -74,8 +74,16 @@ def test_selection_by_candidate_count_with_a_bias(pkg, dev, G, perq, lim, topk, 
     _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, True)
 
 
-def _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased):
-    L, S, D = 640, 64, 64
+@pytest.mark.parametrize("G", [3, 4])
+@pytest.mark.parametrize("L", [8300, 4000])
+@pytest.mark.parametrize("kind", ["shuffled", "column", "far column", "ties"])
+def test_selection_by_candidate_count_wide_heads(pkg, dev, G, L, kind):
+    """Heads of 128 with a bias and 385 to 512 chunks: more than one round of wavefronts and less."""
+    _by_candidate_count(pkg, dev, G, False, 512, 16, kind, True, L, 128, 2)
+
+
+def _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased, L=640, D=64, B=1):
+    S = 64
     N = min(1024, lim + 4)
     gen = torch.Generator().manual_seed(lim)
     v = torch.randperm(N, generator=gen)
@@ -88,20 +96,20 @@ def _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased):
         v[col], v[torch.arange(N) % 16 != 5] = weak, rest[torch.randperm(len(rest), generator=gen)]
     elif kind == "ties":
         v = v // 3
-    lmk = torch.zeros(1, N, G if perq else 1, D)
+    lmk = torch.zeros(B, N, G if perq else 1, D)
     lmk[..., 0], lmk[..., 1] = (v // 8 * 8).view(1, N, 1), (v % 8).view(1, N, 1)  # (each exact in bf16, so is their sum)
-    q = torch.zeros(1, L, G, D)
+    q = torch.zeros(B, L, G, D)
     q[..., :1 if biased else 2] = 1
-    bias = (v % 8 / 8).view(1, N, 1).expand(1, N, G).contiguous().to(dev) if biased else None  # (logits are sums / 8)
+    bias = (v % 8 / 8).view(1, N, 1).expand(B, N, G).contiguous().to(dev) if biased else None  # (logits are sums / 8)
     off = lim * S - L  # the last query's window of one token begins in chunk lim
-    idx, scores, _ = pkg.topk_chunk_weights(q.bfloat16().to(dev), lmk.bfloat16().to(dev), torch.zeros(1, L, G, device=dev), topk, S, 1,
-                                            q_offset=off, num_kv_heads=1, prior_b=bias)
+    idx, scores, _ = pkg.topk_chunk_weights(q.bfloat16().to(dev), lmk.bfloat16().to(dev), torch.zeros(B, L, G, device=dev), topk, S, 1,
+                                            q_offset=off, num_kv_heads=1, prior_b=bias, sm_scale=1 / 8)
     seen = ((torch.arange(L) + off) // S).clamp(0, N)
     order = (v * 2048 - torch.arange(N)).expand(L, N).masked_fill(torch.arange(N) >= seen.view(L, 1), -(1 << 30))
     best = order.topk(topk, -1)
     want = torch.where(best.values > -(1 << 30), best.indices, torch.full_like(best.indices, 1 << 20)).sort(-1).values
     want = torch.where(want == 1 << 20, torch.full_like(want, -1), want)
-    assert torch.equal(idx[0, :, 0].cpu().long(), want)
+    assert torch.equal(idx[:, :, 0].cpu().long(), want.expand(B, L, topk))
     raw = (v // 8 * 8 if biased else v).to(torch.float32)[want.clamp(min=0)] / 8
     raw = raw.masked_fill(want < 0, float("-inf")).bfloat16()
-    assert torch.equal(scores[0].cpu(), raw.unsqueeze(1).expand(L, G, topk))
+    assert torch.equal(scores.cpu(), raw.unsqueeze(1).expand(B, L, G, topk))
