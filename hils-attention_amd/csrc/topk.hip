@@ -3247,15 +3247,16 @@ topk_bwd_dlmk_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q
 // workgroup walks several query blocks and adds its dlmk up in registers, the next block's loads behind this block's
 // products; a block's 32 KB of atomics (D = 64), 268 MB in the call above, were a third of the time.  One block / a walk, us:
 // that call 180 / 151, B2 L8192 32 heads of 64 with a key each 76 / 65, L8192 32/8 heads of 128 82 / 57, L4001 of the
-// same top-8 36 / 29.  dlmk leaves by float atomics (the summation order over workgroups is not fixed).  The chunk indices of one
+// same top-8 36 / 29.  (A single block is a kernel without WALK: the walk's registers, 248 with heads of 128 instead of 164, cost it a
+// wavefront per SIMD, 16384 tokens of 32/4 such heads 198 us instead of 186.)  dlmk leaves by float atomics (the summation order over workgroups is not fixed).  The chunk indices of one
 // row must be distinct (they are when they come from the selection).
 #define TD_R 128        // rows per workgroup
 #define TD_NC 128       // chunks per tile (== TD_R: one thread-to-piece split serves rows and chunk keys)
 #define TD_THREADS 512
 #define TD_STRIDE 136   // elements per row of A: 128 + 8
 
-template <int D>
-__global__ void __launch_bounds__(TD_THREADS) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
+template <int D, bool WALK>
+__global__ void __launch_bounds__(TD_THREADS) __attribute__((amdgpu_waves_per_eu(WALK && D == 64 ? 4 : 2)))
 topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ q,
                       const bf16_t* __restrict__ lmks, const int32_t* __restrict__ indices,
                       bf16_t* __restrict__ dq, float* __restrict__ dlmk, int L, int N, int h_kv, int G,
@@ -3278,9 +3279,12 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   const int hk = per_qhead ? lh / G : lh;
   const int g_lo = per_qhead ? lh % G : 0, g_n = 1 << g_sh;  // (a divisor of TD_R)
   const int TQ = TD_R >> g_sh;
-  int t0 = blockIdx.z * walk * TQ;
-  int n_blk = (L - t0 + TQ - 1) / TQ;  // query blocks of this workgroup (the host takes one where N > TD_NC)
-  n_blk = n_blk < walk ? n_blk : walk;
+  int t0 = blockIdx.z * (WALK ? walk * TQ : TQ);
+  int n_blk = 1;  // query blocks of this workgroup
+  if (WALK) {
+    n_blk = (L - t0 + TQ - 1) / TQ;
+    n_blk = n_blk < walk ? n_blk : walk;
+  }
   auto row_rg = [&](int row) -> long {  // row of gs / q / dq of a block row (valid rows only)
     return ((b * L + t0 + (row >> g_sh)) * h_kv + hk) * (long)G + g_lo + (row & (g_n - 1));
   };
@@ -3339,7 +3343,7 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
   for (int blk = 0; blk < n_blk; ++blk) {
     // (hidden from the compiler, which would keep the addresses of all pieces and entries in registers: 190 of them,
     // one workgroup per compute unit instead of two)
-    if constexpr (D == 64) asm volatile("" : "+v"(tid));
+    if constexpr (WALK && D == 64) asm volatile("" : "+v"(tid));
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
       const int i = tid + u * TD_THREADS;
@@ -3391,7 +3395,7 @@ topk_bwd_dense_kernel(const bf16_t* __restrict__ gs, const bf16_t* __restrict__ 
       }
       __syncthreads();
       cmax = cmax_s;
-      const bool last = blk + 1 == n_blk;
+      const bool last = !WALK || blk + 1 == n_blk;
       if (!last) {  // what the next block reads is asked for behind this block's products
         t0 += TQ;
         if constexpr (D == 64) asm volatile("" : "+v"(tid));
@@ -3480,9 +3484,9 @@ static int topk_bwd_dense_launch(dim3 grid, hipStream_t st, const bf16_t* gs, co
     grid.z = (grid.z + walk - 1) / walk;
   }
   const size_t smem = ((size_t)TD_R * TD_STRIDE + (size_t)(TD_R + TD_NC) * (D + 8)) * sizeof(bf16_t);
-  auto kern = topk_bwd_dense_kernel<D>;
-  static HilsLdsReserve reserved;  // per instantiation
-  if (int rc = hils_reserve_lds(&reserved, (const void*)kern, smem, "hils_topk_bwd")) return rc;
+  auto kern = walk > 1 ? topk_bwd_dense_kernel<D, true> : topk_bwd_dense_kernel<D, false>;
+  static HilsLdsReserve reserved[2];  // per instantiation
+  if (int rc = hils_reserve_lds(&reserved[walk > 1], (const void*)kern, smem, "hils_topk_bwd")) return rc;
   hipLaunchKernelGGL(kern, grid, dim3(TD_THREADS), smem, st, gs, q, lmks, indices, dq, dlmk, L, N, h_kv, G, topk,
                      per_qhead, sm_scale, hils_udiv_magic((uint32_t)topk), __builtin_ctz(per_qhead ? 1 : G), walk);
   return HILS_OK;

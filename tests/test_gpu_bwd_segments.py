@@ -154,7 +154,8 @@ def test_swa_backward_split(pkg, dev, B, L, HQ, H, D, W):
 # blocks without any entry, exactly one tile of chunks and one more (which is not walked)
 @pytest.mark.parametrize("B,L,N,H,G,D,K,per_qhead", [(1, 40, 3, 1, 1, 64, 2, 0), (2, 3001, 128, 16, 1, 64, 8, 0), (2, 3001, 129, 16, 1, 64, 8, 0),
                                                      (3, 1037, 16, 2, 16, 64, 5, 1), (1, 2500, 40, 8, 4, 128, 16, 0),
-                                                     (9, 700, 11, 8, 4, 128, 33, 1), (4, 9001, 100, 4, 2, 64, 3, 0)])
+                                                     (9, 700, 11, 8, 4, 128, 33, 1), (4, 9001, 100, 4, 2, 64, 3, 0),
+                                                     (1, 300, 20, 2, 4, 128, 6, 0), (2, 901, 140, 2, 4, 128, 9, 1)])
 def test_dense_gather_backward_walks(pkg, dev, B, L, N, H, G, D, K, per_qhead):
     from hils_attention_amd.ops import _cabi
     lib, HK = _cabi.load(), H * G if per_qhead else H
