@@ -451,14 +451,25 @@ extern "C" int hils_chunk_weights_bwd(const void* scores, const void* lse_swa, i
     const long nb = (rows + 4 * rpw - 1) / (4 * rpw);
     HILS_REQUIRE(nb <= 2147483647L, "hils_chunk_weights_bwd: grid too large");
     // with a bias gradient whose table fits the LDS: runs of rows per workgroup, one workgroup a
-    // compute unit (two: 48.8 us against 40.2 at B2 L8192 32 heads K32), each run long enough that its adds outnumber the table it flushes
+    // compute unit (two: 48.8 us against 40.2 at B2 L8192 32 heads K32), each run long enough that its adds outnumber the table it flushes.
+    // Where a round of such runs leaves much of the chip idle (129 batch elements on 256 compute units) shorter runs in up to two
+    // rounds more, by the tiles a compute unit goes through, a table's adds to memory counted as one.  One round / so, us, N 64: B129
+    // L1024 16/16 heads K32 266 / 185, 16/2 heads K8 64 / 52; B192 L256 16/16 K32 68 / 62; B300 of it 144 / 117; B129 L256 16/2 K8
+    // stays (18.9 / 20.5 in two rounds).
     const size_t tab_b = (size_t)N * HQ * sizeof(unsigned long long);
     if (d_prior_b && tab_b <= 48 * 1024) {
       const long tiles_b = ((long)L * HQ + 16 * rpw - 1) / (16 * rpw);  // 16-wavefront tiles of a batch element
-      long segs = hils_device_cus() / B;
-      if (segs < 1) segs = 1;
-      if (segs > tiles_b) segs = tiles_b;
-      const int tiles_per_wg = (int)((tiles_b + segs - 1) / segs);
+      const long cus = hils_device_cus(), first = (B + cus - 1) / cus;  // rounds of one run a batch element
+      long tiles_per_wg_l = 0, best = 0;
+      for (long r = first; r <= first + 2; ++r) {
+        const long per = (tiles_b - 1) / (r * cus / B) + 1, runs = (tiles_b + per - 1) / per;
+        const long cost = (B * runs + cus - 1) / cus * (per + 1);
+        if (r == first || cost < best) {
+          best = cost;
+          tiles_per_wg_l = per;
+        }
+      }
+      const int tiles_per_wg = (int)tiles_per_wg_l;
       const dim3 grid((unsigned)((tiles_b + tiles_per_wg - 1) / tiles_per_wg), (unsigned)B);
       HILS_REQUIRE(B <= 65535, "hils_chunk_weights_bwd: batch too large for the grid");
       // a run has so many rows of a head, each with K indices, all of which may be the same

@@ -40,13 +40,13 @@ def test_only_what_is_asked_for(pkg, dev, want):
             assert_close_bf16(x.grad, r, name)
 
 
-@pytest.mark.parametrize("K,L,repeated", [(8, 4096, False), (32, 2500, False), (16, 700, True)])
-def test_prior_gradient_of_large_gradients(pkg, dev, K, L, repeated):
+@pytest.mark.parametrize("B,K,L,repeated", [(2, 8, 4096, False), (2, 32, 2500, False), (2, 16, 700, True), (129, 32, 1001, False), (300, 16, 1801, False)])
+def test_prior_gradient_of_large_gradients(pkg, dev, B, K, L, repeated):
     """Sums of a run of rows far past 2^23, small ones beside them, one index in all slots of a row, and a gradient that
-    is no number."""
-    note(f"chunk_weights, large gradients, K={K} L{L} repeated {repeated}")
+    is no number; one round of runs of rows, two and three."""
+    note(f"chunk_weights, large gradients, B{B} K={K} L{L} repeated {repeated}")
     gen = torch.Generator(device=dev).manual_seed(K)
-    B, HQ, H, N = 2, 2, 1, 64
+    HQ, H, N = 2, 1, 64
     sc = torch.randn(B, L, HQ, K, device=dev, generator=gen).bfloat16()
     lse = torch.randn(B, L, HQ, device=dev, generator=gen) + 1
     pb = torch.zeros(B, N, HQ, device=dev, requires_grad=True)
