@@ -440,7 +440,7 @@ logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     const float* zs = (const float*)(k_s + (NB * TB + wave * (NB * 256) + B0 * 256 + col * 4));
     const float lz = zs[0], dz = zs[32];
     const bool ok = c < lim && lz > -1e30f;
-    off = ok ? lz * HILS_LOG2E : 0.f;
+    off = ok ? lz * HILS_LOG2E : INFINITY;  // (no probability but 0, however large the score)
     coef = ok ? dz * dm.sm_scale : 0.f;
     fetch(c + 3, B3);
     fetch_z(c + 2, B2);
@@ -595,7 +595,7 @@ logz_bwd_dk_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
       *(lz_u32x4*)(&q_s[buf][(tid + 256 * i) / (D / 8) * PITCH + (tid + 256 * i) % (D / 8) * 16]) = qr[i];
     if (tid < 128) {
       const bool ok = zin && zo > -1e30f;
-      off_s[buf][tid >> 6][tid & 63] = ok ? zo * HILS_LOG2E : 0.f;
+      off_s[buf][tid >> 6][tid & 63] = ok ? zo * HILS_LOG2E : INFINITY;  // (no probability but 0, however large the score)
       coef_s[buf][tid >> 6][tid & 63] = ok ? zc * dm.sm_scale : 0.f;
     }
   };

@@ -55,6 +55,29 @@ def test_negative_window(pkg, orc, dev, HQ, H, D, L, W):
     assert_close_bf16(kd.grad, kf.grad, "dk")
 
 
+@pytest.mark.parametrize("HQ,H,D", [(4, 2, 64), (2, 2, 64), (8, 1, 128), (4, 1, 128)])
+def test_gradients_beside_large_scores(pkg, orc, dev, HQ, H, D):
+    """Scores past the exponential's range in chunks that a query does not see, but its workgroup walks."""
+    L, W = 470, 64
+    note(f"log Z, large scores, heads {HQ}/{H} x {D}")
+    gen = torch.Generator().manual_seed(D + HQ)
+    q, k = 8 * torch.randn(1, L, HQ, D, generator=gen), 8 * torch.randn(1, L, H, D, generator=gen)
+    q, k = q.bfloat16(), k.bfloat16()
+    qd, kd = q.to(dev).requires_grad_(), k.to(dev).requires_grad_()
+    z = pkg.exact_chunk_log_z_tl(qd, kd, chunk_size=64, window_size=W)
+    qf, kf = q.double().requires_grad_(), k.double().requires_grad_()
+    s = torch.einsum("blhd,bjhd->blhj", qf, kf.repeat_interleave(HQ // H, 2)) * D ** -0.5
+    n = z.shape[-1]
+    s = torch.nn.functional.pad(s, (0, 64 * n - L), value=float("-inf")).unflatten(-1, (n, 64))
+    seen = (torch.arange(1, n + 1) * 64 <= torch.arange(L).view(-1, 1) - W + 1).view(1, L, 1, n)
+    assert s.detach().masked_fill(seen.unsqueeze(-1), 0)[0, :-64].amax() > 89  # (the exponential's range ends at 88.7)
+    g = torch.randn(z.shape, generator=gen) * seen
+    z.backward(g.to(dev))
+    s.masked_fill(~seen.unsqueeze(-1), 0).logsumexp(-1).mul(g * seen).sum().backward()
+    assert_close_bf16(qd.grad, qf.grad.float(), "dq")
+    assert_close_bf16(kd.grad, kf.grad.float(), "dk")
+
+
 @pytest.mark.parametrize("HQ,H,D", [(4, 2, 64), (8, 1, 128)])
 @pytest.mark.parametrize("at", [1, 4])
 def test_keys_at_any_address(pkg, dev, HQ, H, D, at):
