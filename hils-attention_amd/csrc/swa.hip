@@ -69,8 +69,18 @@ static size_t swa_fwd_smem() {
   return tiles > outs ? tiles : outs;
 }
 
+// Wavefronts per SIMD that the registers are held to: as many as the LDS holds workgroups for, where the kernel by itself is
+// only a few registers above (16 heads a KV head 135 of 128 and 187 of 168, heads of 128 with values of 64 170 to 174 of 168) and
+// the workgroups that go with them cost more than what brings the registers down.  Two / three or four, us: B2 L4096 32/2 heads
+// of 64 window 512 97 / 77, B4 L8192 of it window 64 95 / 86; with values of 128 140 / 125; 16/4 heads of 128 with values of 64 66 / 59.
+// (Others need spills: 2 to 8 heads of 64 a KV head, held to four, 44 us instead of 49 at L4096 window 512, but 29.6 instead of 26.9 with 8/4.)
+constexpr int swa_fwd_waves(int D, int DV, int G, int NWV, int RES, int SPLIT) {
+  if (D == 64 && DV == 64) return G == 16 && SPLIT == 1 && (NWV == 8 || RES == 2) ? 4 : 2;
+  return RES == 2 && (D == 64 ? G == 16 : DV == 64 && G < 16) ? 3 : 2;
+}
+
 template <int D, int DV, int G, int NWV, int RES, int SPLIT>
-__global__ void __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(swa_fwd_waves(D, DV, G, NWV, RES, SPLIT))))
 swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
             bf16_t* __restrict__ o, float* __restrict__ lse, SwaDims dm, int n_qt, int n_b) {
   constexpr int RT = SWA_FWD_RT, NT = NWV * 64;
@@ -172,15 +182,22 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
     l_run[rt] = 0.f;
   }
 
-  // this lane's places in a tile: a row's piece of the scores' k-step, a 4 x 4 block's share of V's columns
-  unsigned k_off[KS], v_off[DT];
+  // this lane's places in a tile: a row's piece of the scores' k-step, a 4 x 4 block's share of V's columns.  Those of the
+  // other steps and columns differ in a few bits: a register each or, held to more wavefronts, worked out where they are used
+  constexpr bool TIGHT = swa_fwd_waves(D, DV, G, NWV, RES, SPLIT) > 2;
+  constexpr int KN = TIGHT && D == 128 ? 1 : KS, VN = TIGHT && D == 64 ? 2 : DT;
+  unsigned k_off[KN], v_off[VN];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) k_off[ks] = (unsigned)(col * KP + ((ks * 4 + j) ^ (col & (KSEG - 1))) * 16);
+  for (int ks = 0; ks < KN; ++ks) k_off[ks] = (unsigned)(col * KP + ((ks * 4 + j) ^ (col & (KSEG - 1))) * 16);
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
+  for (int dt = 0; dt < VN; ++dt) {
     const int row = 4 * j + (col >> 2);
     v_off[dt] = (unsigned)(row * VP + ((dt * 2 + (col >> 1 & 1)) ^ (row & (VSEG - 1))) * 16 + (col & 1) * 8);
   }
+  auto other = [](unsigned first, unsigned bits) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(first));
+    return first ^ bits;
+  };
 
   // one resident tile: scores, masks where a row needs them, running softmax, O += P V
   auto tile_step = [&](int tile, const unsigned char* k_s, const unsigned char* v_s) __attribute__((always_inline)) {
@@ -196,7 +213,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8_t a = *(const bf16x8_t*)(k_s + k_off[ks] + tt * 16 * KP);
+          const bf16x8_t a = *(const bf16x8_t*)(k_s + (ks < KN ? k_off[ks % KN] : other(k_off[0], ks * 64)) + tt * 16 * KP);
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
             p[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qa[rt][ks], p[rt][tt], 0, 0, 0);
@@ -289,7 +306,7 @@ swa_fwd_blk(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const unsigned char* p0 = v_s + v_off[dt] + (2 * h * 16) * VP;
+        const unsigned char* p0 = v_s + (dt < VN ? v_off[dt % VN] : other(v_off[dt % VN], dt / VN * VN * 32)) + (2 * h * 16) * VP;
         const swa_s4 b0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) swa_s4*)p0);
         const swa_s4 b1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) swa_s4*)(p0 + 16 * VP));
         const swa_s8 bb = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);

@@ -46,6 +46,14 @@ def test_swa_few_blocks(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, kw):
     run(pkg, orc, dev, B, Lq, Lk, HQ, H, D, Dv, W, S, **kw)
 
 
+# tile kernels that work out where their operands lie
+@pytest.mark.parametrize("B,L,HQ,H,D,Dv,W,S,kw", [
+    (1, 2111, 16, 1, 64, 64, 512, 64, {"mask_lmk": False}), (1, 1300, 16, 1, 64, 64, 64, 64, {}), (2, 1100, 16, 1, 64, 128, 64, 64, {}),
+    (1, 1500, 8, 2, 128, 64, 64, 64, {"mask_lmk": True}), (1, 1201, 8, 8, 128, 64, 50, 16, {"expand": False})])
+def test_swa_tiles_of_few_registers(pkg, orc, dev, B, L, HQ, H, D, Dv, W, S, kw):
+    run(pkg, orc, dev, B, L, L, HQ, H, D, Dv, W, S, **kw)
+
+
 # few queries a sequence (the row kernel): chunks that are no power of two, cut caches, windows of one to three units a
 # wavefront, and counts of row blocks on either side of where the tile kernel takes over
 @pytest.mark.parametrize("B,Lq,Lk,HQ,H,D,Dv,W,S,kw", [
