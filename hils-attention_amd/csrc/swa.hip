@@ -511,8 +511,10 @@ constexpr int swa_dkdv_buffers(int D, int DV) { return (D > 64 && DV > 64) ? 1 :
 // dQ (and delta): a wavefront owns 16 * RT score rows; K and V stream.
 template <int D, int DV, int G>
 // (the hint keeps the accumulators out of accumulation registers; three wavefronts per SIMD of wide heads spilled: 222 us
-// instead of 191 at L4096 32/4 of 128 window 512)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+// instead of 191 at L4096 32/4 of 128 window 512.  Unequal widths have three: one buffer and, where it would spill 7 registers,
+// with values of 64, masks in all tiles.  Two / three, us: B4 L8192 16/4 heads window 64 146 / 127 with values of 64, 133 / 119 of 128;
+// B2 L4096 window 512 97 / 82, 92 / 79)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D != DV ? 3 : 2)))
 swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                 const bf16_t* __restrict__ o, const float* __restrict__ lse,
                 const bf16_t* __restrict__ d_o, const float* __restrict__ d_lse,
@@ -522,7 +524,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
   constexpr int QW = 16 * RT / G > 0 ? 16 * RT / G : 1, QB = 4 * 16 * RT / G;
   constexpr int PITCH = D * 2 + 32, VPITCH = DV * 2 + 32;
   constexpr int KSEG = D / 8, KPASS = 64 * KSEG / 256, VSEG = DV / 8, VPASS = 64 * VSEG / 256;
-  constexpr int NB = (D > 64 && DV > 64) ? 1 : 2;  // buffers (two of wide heads: no faster)
+  constexpr int NB = (D > 64 || DV > 64) ? 1 : 2;  // buffers (two of equally wide heads: no faster)
   __shared__ __align__(16) unsigned char k_s[NB][64 * PITCH];
   __shared__ __align__(16) unsigned char v_s[NB][64 * VPITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -577,7 +579,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
     vspan[rt] = some ? (unsigned)(qabs[rt] - cstart[rt]) : 0u;
   }
   int tile_lo, tile_hi;
-  int full_lo, full_hi;  // tiles that all rows see whole
+  int full_lo, full_hi;  // tiles that all rows see whole, of which the masks are left out
   {
     const int tq0 = qt * QB;
     int tq1 = tq0 + QB - 1;
@@ -590,7 +592,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
     const int right_abs = tq1 - dm.window + 1;
     const int first = dm.expand ? floordiv(right_abs, dm.chunk) * dm.chunk : right_abs;  // of the last row's window
     full_lo = first > 0 ? (first + 63) / 64 : 0;
-    full_hi = dm.mask_lmk ? 0 : (tq0 + 1) / 64;
+    full_hi = dm.mask_lmk || D > DV ? 0 : (tq0 + 1) / 64;
   }
   const float c2 = dm.sm_scale * HILS_LOG2E;
 
@@ -637,7 +639,7 @@ swa_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, cons
   for (int tile = tile_lo, buf = 0; tile < tile_hi; ++tile) {
     fetch(tile + 1 < tile_hi ? tile + 1 : tile);
     const unsigned char *kb = k_s[buf], *vb = v_s[buf];
-    const bool full = tile >= full_lo && tile < full_hi;
+    const bool full = D <= DV && tile >= full_lo && tile < full_hi;
     float ds[RT][4][4];
     {
       f32x4_t st[RT][4], dp[RT][4];

@@ -217,7 +217,8 @@ def test_local_and_remote_branch_sum_to_dense_attention(pkg, dev, L, HQ, H, D, W
 @pytest.mark.parametrize("B,L,HQ,H,D,Dv,W,S,mask_lmk,expand", [
     (1, 833, 8, 1, 64, 64, 512, 64, False, True), (1, 640, 4, 4, 64, 64, 300, 64, False, False),
     (2, 577, 8, 2, 128, 128, 385, 64, False, True), (1, 900, 4, 4, 128, 128, 449, 48, False, False),
-    (1, 705, 16, 1, 128, 64, 320, 64, False, True), (1, 530, 2, 1, 64, 128, 500, 64, True, True)])
+    (1, 705, 16, 1, 128, 64, 320, 64, False, True), (1, 530, 2, 1, 64, 128, 500, 64, True, True),
+    (2, 641, 8, 2, 64, 128, 320, 64, False, True), (1, 770, 4, 4, 128, 64, 64, 64, False, False)])
 def test_swa_backward_whole_tiles(pkg, orc, dev, B, L, HQ, H, D, Dv, W, S, mask_lmk, expand):
     _forward_backward(pkg, orc, dev, B, L, HQ, H, D, Dv, W, S, mask_lmk, expand)
 
