@@ -323,8 +323,8 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 // the gradient product.
 // dQ: a wavefront owns 32 score rows (query x head), the chunks' keys stream 32 tokens at a time: the scores of the next
 // 32, the exponentials of these and the gradient product of the last ones are independent, and one wavefront's vector
-// instructions run beside its matrix ones.  32x32x16 products; four buffers, loaded two steps ahead without registers
-// between (also the rows' log_z and d_log_z).  Bound by the chip's power: L 8192, 32/8 heads of 128 in 2720 cycles a chunk and pair of
+// instructions run beside its matrix ones.  32x32x16 products; four buffers, loaded without registers between, the keys three
+// chunks ahead and the rows' log_z and d_log_z two.  Bound by the chip's power: L 8192, 32/8 heads of 128 in 2720 cycles a chunk and pair of
 // workgroups instead of 4010, but at 1.55 GHz instead of 2.1, 522 -> 471 us (1.16 PFLOP/s; a large plain product 1.39);
 // 180 -> 150 us at 16/2 heads of 64, 79 -> 61 at L 4096 16/16 of 64, 29 -> 22 at L 1200 32/8 of 128.  The same for dK, whose factors
 // differ by register instead of by lane, spilled and was slower.

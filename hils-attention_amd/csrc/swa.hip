@@ -3,10 +3,10 @@
 // exactly), optionally without the landmark key of every chunk; outputs o and the natural-log LSE.
 //
 // A wavefront owns 32 score rows (query x head of the group), held as matrix B operands; the keys
-// and values of the window pass through LDS in 64-token tiles: K row-major (A operand of the
-// transposed scores K Q^T), V as the B operand of O += P V, whose contraction runs over the tokens.
+// and values of the window pass through LDS in 64-token tiles, both row-major: K rows are the A operand of
+// the transposed scores K Q^T, V's columns that of O^T += V^T P^T, whose contraction runs over the tokens.
 // With the rows as matrix columns a row's 64 scores lie in 16 registers of 4 lanes (in-lane softmax
-// plus one row-swap reduction) and the probabilities are already the A operand of the second product.
+// plus one row-swap reduction) and the probabilities are already the B operand of the second product.
 #include <type_traits>
 #include "stream_tiles.h"
 #include "swa_dims.h"
@@ -34,7 +34,7 @@ static dim3 swa_xcd_grid(int n_blk, int H, int B) { return dim3((unsigned)(((lon
 // block can see (its queries' windows: two or three 64-token tiles at window 64) are loaded once, all
 // loads in flight together, and stay in LDS row-major, 16-byte piece p of row r at p ^ (r & pieces - 1), which no read
 // conflicts over (rows 16 bytes apart: 8 cycles a score operand instead of 4); a longer window is
-// worked through in phases of RES resident tiles.  S^T = K Q^T takes K rows as A operands, O += P V takes V
+// worked through in phases of RES resident tiles.  S^T = K Q^T takes K rows as A operands, the outputs V
 // through the transposing LDS load, in the token order in which the S^T accumulators hold P.
 // The outputs are formed transposed, O^T += V^T P^T, so that a row's factors, maximum and sum belong to its lanes (no way
 // through LDS) and a lane parks four neighbouring features at a time: with the reads above 64 -> 62 us at B4 L8192 16/16 heads of 64
@@ -1062,7 +1062,7 @@ static int swa_fwd_launch(int B, hipStream_t st, const bf16_t* q, const bf16_t* 
                           bf16_t* o, float* lse, const SwaDims& dm) {
   const int tiles = swa_fwd_block_tiles(dm, 4 * 16 * SWA_FWD_RT / G);
   if (tiles <= 2) return swa_fwd_launch_shape<D, DV, G, 4, 2>(B, st, q, k, v, o, lse, dm);
-  // narrow heads: four resident tiles are 72 KiB, and two 4-wavefront workgroups fit a compute unit
+  // narrow heads: four resident tiles are 64 KiB, and two 4-wavefront workgroups fit a compute unit
   // where one 8-wavefront workgroup does (150 registers: three wavefronts per SIMD)
   if constexpr (D <= 64 && DV <= 64)
     if (tiles <= 4) return swa_fwd_launch_shape<D, DV, G, 4, 4>(B, st, q, k, v, o, lse, dm);

@@ -12,12 +12,13 @@
 //   * the top-K per query, the four lane rows working on four queries at once: the K-th largest
 //     score is bracketed from the two largest scores of every lane (their minimum over the lanes is
 //     a lower bound with at least 32 scores above it), the scores above the bound (about 1.5 K of
-//     512) are compacted through LDS to at most 8 per lane, turned into order-preserving unsigned
+//     512) are compacted through LDS to at most 8 per lane (12 or 16 as records, from 32 blocks on), turned into order-preserving unsigned
 //     keys, and the threshold is found on those by a bitwise search whose counts are 16-lane DPP
 //     reductions (no ballots, no scalar round trip) and which stops at the first probe that counts
 //     exactly K; ties at the threshold go to the lower chunk indices,
 //   * the ascending order of the winners from the votes of the blocks (rank = winners voted before and in
-//     lower columns), and the winners' raw scores straight from the logits.
+//     lower columns) and their raw scores straight from the logits; with records (most kernels of 32 and 64 blocks) from a
+//     map of the winning chunks in LDS and from the records.
 // Five to eight query heads per KV head (HALF below) take two wavefronts per four queries, one for the
 // heads 0..3 and one for the rest: each forms the partial selection scores of its heads, the two
 // trade them through LDS, and both then select on the same scores and write their own heads' outputs.

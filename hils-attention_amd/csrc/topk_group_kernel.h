@@ -556,9 +556,9 @@ topk_fwd_group_kernel(const bf16_t* __restrict__ q, const uint4* __restrict__ lm
     }
     const int nvalid = tg_row_sum_i(nv);
     if constexpr (REC) {
-      // The candidates as records (score, chunk, raw scores), so that from here on a lane has at most eight of them to
-      // look at instead of NB: the threshold, the winners, their order (a map of the winning chunks and its prefix
-      // counts) and their raw scores all come from the records.  A query that keeps everything has all its valid scores
+      // The candidates as records (score, chunk, raw scores), so that from here on a lane has at most REC_N / 16 of them
+      // to look at (eight while TG_CAND do) instead of NB: the threshold, the winners, their order (a map of the winning
+      // chunks and its prefix counts) and their raw scores all come from the records.  A query that keeps everything has all its valid scores
       // (at most topk) as candidates.
       const bool want = nvalid > topk;
       const float hi = tg_row_max_f(m1), bound = tg_row_min_f(m2);  // >= 2 scores per lane reach it: >= 32 >= topk in all
