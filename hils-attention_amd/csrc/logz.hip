@@ -104,6 +104,10 @@ __device__ __forceinline__ unsigned long long lz_uniform(unsigned long long x) {
 __device__ __forceinline__ unsigned lz_lds_addr(const unsigned char* p) {
   return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
 }
+// (M0, which both statements set, is a register that the compiler never holds a variable in: it warns that naming it cannot
+// preserve it.  Named, its own settings of M0 are not taken to last over the statement, which is what is wanted.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 // 64 pieces of 16 bytes, lane i's from base + off to lds + 16 i
 __device__ __forceinline__ void lz_dma16(unsigned lds, unsigned off, unsigned long long base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
@@ -112,6 +116,7 @@ __device__ __forceinline__ void lz_dma16(unsigned lds, unsigned off, unsigned lo
 __device__ __forceinline__ void lz_dma4(unsigned lds, unsigned long long addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(addr) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 template <int N>
 __device__ __forceinline__ void lz_landed() {  // all but the last N vector-memory operations
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
