@@ -150,7 +150,8 @@ __device__ __forceinline__ void lz_walk(int n, F&& step) {
 // Bound by the chip's power: at L 8192, 32/8 heads of 128 it runs at 1.9 to 2.0 of 2.4 GHz, about 1000 cycles for the 32 x 64
 // scores of a wavefront against 1170 with 16x16x32 products that waited for their LDS reads and for each other; 325 -> 287 us
 // there, 136 -> 107 at 16/2 heads of 64, 75 -> 54 at L 4096 16/16 heads of 64, 26 -> 19 at L 1200 32/8 of 128 (64 rows a
-// wavefront, half the LDS reads: 285, 131, 57 and 29 us).
+// wavefront, half the LDS reads: 285, 131, 57 and 29 us).  Times at the power limit are the card's: two others took 314 and
+// 322 us for the first.
 template <int D, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
 logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
@@ -332,7 +333,7 @@ logz_fwd_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
 // chunks ahead and the rows' log_z and d_log_z two.  Bound by the chip's power: L 8192, 32/8 heads of 128 in 2720 cycles a chunk and pair of
 // workgroups instead of 4010, but at 1.55 GHz instead of 2.1, 522 -> 471 us (1.16 PFLOP/s; a large plain product 1.39);
 // 180 -> 150 us at 16/2 heads of 64, 79 -> 61 at L 4096 16/16 of 64, 29 -> 22 at L 1200 32/8 of 128.  The same for dK, whose factors
-// differ by register instead of by lane, spilled and was slower.
+// differ by register instead of by lane, spilled and was slower.  (Two other cards: 495 and 528 us.)
 template <int D, int G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 logz_bwd_dq_mfma(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,

@@ -245,6 +245,7 @@ swa_fwd_rows(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const b
 //   one block:   heads of 64, window 512  6.8/14  13/38  25/73  67/149;  window 64  5.6/5.5  5.7/5.8  7.3/9.3  13/15
 //                heads of 128, 512  13/21  25/52  47/102  112/224;  256  9/12  17/30  31/57  71/125;
 //                128  5.6/7.7  11/10  20/22  38/38;  64  5.8/5.8  7.6/7.1  15/13  28/25
+//                keys of 64 and values of 128, 512  24/51 (640 workgroups), 256  27/52 (1280); the reverse 27/51 and 30/51
 //   two blocks:  heads of 64, 512  7.8/15  15/17  26/41  49/79;  256  5.4/11  9/11  17/25  31/49;  128  5.5/8.5  7/9  13/10  23/21
 //   eight:       heads of 64 (16 queries of eight heads), 512  -  15/15  27/16  48/18;  64  -  5.6/6.7  10/7  18/7
 //   four:        heads of 128 (16 queries of four heads), 512  15/21  27/23  52/25;  64  5.6/8.2  11/8  21/9
