@@ -63,15 +63,41 @@ def test_equal_scores_past_512_chunks(pkg, dev):
 def test_selection_by_candidate_count(pkg, dev, G, perq, lim, topk, kind):
     """Exact scores whose candidates (those above the weakest lane's second largest score) are few, more than 128, or more
     than the kernel keeps, and ties at the threshold: the best scores win, of equal ones the lowest chunks."""
-    _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, False)
+    L, S, D = 640, 64, 64
+    N = min(1024, lim + 4)
+    gen = torch.Generator().manual_seed(lim)
+    v = torch.randperm(N, generator=gen)
+    if kind.endswith("column"):  # the chunks of one lane hold nothing above the given rank
+        low = N - 1 - (N // 2 if kind.startswith("far") else min(150, N // 4))
+        col = (torch.arange(N) % 16 == 5).nonzero().view(-1)
+        weak = torch.randperm(low, generator=gen)[: len(col)]
+        rest = torch.ones(N, dtype=torch.bool).index_fill(0, weak, False).nonzero().view(-1)
+        v = torch.empty(N, dtype=torch.long)
+        v[col], v[torch.arange(N) % 16 != 5] = weak, rest[torch.randperm(len(rest), generator=gen)]
+    elif kind == "ties":
+        v = v // 3
+    lmk = torch.zeros(1, N, G if perq else 1, D)
+    lmk[..., 0], lmk[..., 1] = (v // 8 * 8).view(1, N, 1), (v % 8).view(1, N, 1)  # (each exact in bf16, so is their sum)
+    q = torch.zeros(1, L, G, D)
+    q[..., :2] = 1
+    off = lim * S - L  # the last query's window of one token begins in chunk lim
+    idx, _, _ = pkg.topk_chunk_weights(q.bfloat16().to(dev), lmk.bfloat16().to(dev), torch.zeros(1, L, G, device=dev), topk, S, 1,
+                                       q_offset=off, num_kv_heads=1)
+    seen = ((torch.arange(L) + off) // S).clamp(0, N)
+    order = (v * 2048 - torch.arange(N)).expand(L, N).masked_fill(torch.arange(N) >= seen.view(L, 1), -(1 << 30))
+    best = order.topk(topk, -1)
+    want = torch.where(best.values > -(1 << 30), best.indices, torch.full_like(best.indices, 1 << 20)).sort(-1).values
+    want = torch.where(want == 1 << 20, torch.full_like(want, -1), want)
+    assert torch.equal(idx[0, :, 0].cpu().long(), want)
 
 
 @pytest.mark.parametrize("G,perq", [(4, False), (4, True), (8, False), (8, True)])
 @pytest.mark.parametrize("lim,topk", [(40, 32), (512, 32), (1024, 32)])
 @pytest.mark.parametrize("kind", ["shuffled", "column", "far column", "ties"])
-def test_selection_by_candidate_count_with_a_bias(pkg, dev, G, perq, lim, topk, kind):
-    """The same scores, their last three bits in the prior bias: the scores that come back carry none of it."""
-    _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, True)
+@pytest.mark.parametrize("biased", [False, True])
+def test_selected_scores_by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased):
+    """The scores that come back, also with the last three bits of the logits in the prior bias, of which they carry none."""
+    _by_candidate_count(pkg, dev, G, perq, lim, topk, kind, biased)
 
 
 @pytest.mark.parametrize("G", [3, 4])
